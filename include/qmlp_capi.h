@@ -206,14 +206,25 @@ int qmlp_activation_precompile(qmlp_activation_t activation);
 /* ---- qmlp::Utils (src_cpp/include/qmlp/utils.h:50-85; bound for torch as utils.pullpush_forward
  * and utils.pullpush_backward in src_cpp/pytorch-bindings/src/bind_utils.cpp:9-40) ---- */
 /* fractionalPullpush, utils.h:65: mask (B,H,W), data and output (B,C,H,W), C < 16, all float
- * or all double. Returns after the work on 'stream' has finished (the image pyramid is
- * temporary device memory of the call). */
+ * or all double. The image pyramid is temporary device memory of the call, allocated and released
+ * in the order of the stream. */
 int qmlp_utils_pullpush_forward(const qmlp_tensor* mask, const qmlp_tensor* data, const qmlp_tensor* output,
                                 void* stream);
 /* adjointFractionalPullpush, utils.h:80: adds into adj_mask (B,H,W) and adj_data (B,C,H,W),
  * which the caller zeroes first (bind_utils.cpp:26-27). */
 int qmlp_utils_pullpush_adjoint(const qmlp_tensor* mask, const qmlp_tensor* data, const qmlp_tensor* adj_output,
                                 const qmlp_tensor* adj_mask, const qmlp_tensor* adj_data, void* stream);
+/* The same with device memory of the caller, aligned to 16 bytes, of the sizes that the first call
+ * reports for images like 'data': 'pyramid' receives the image pyramid of the forward pass, and an
+ * adjoint call on the same mask and data reads it if 'pyramid_ready' is not 0 (otherwise it computes
+ * it); 'gradients' is scratch memory of the adjoint call. 'accumulate' 0: adj_mask and adj_data are
+ * overwritten instead of added to. These calls allocate nothing and do not synchronise. */
+int qmlp_utils_pullpush_memory(const qmlp_tensor* data, size_t* pyramid_bytes, size_t* gradient_bytes);
+int qmlp_utils_pullpush_forward_in(const qmlp_tensor* mask, const qmlp_tensor* data, const qmlp_tensor* output,
+                                   void* pyramid, void* stream);
+int qmlp_utils_pullpush_adjoint_in(const qmlp_tensor* mask, const qmlp_tensor* data, const qmlp_tensor* adj_output,
+                                   const qmlp_tensor* adj_mask, const qmlp_tensor* adj_data, int accumulate,
+                                   void* pyramid, int pyramid_ready, void* gradients, void* stream);
 /* Compiles the pull-push kernels for QMLP_FLOAT or QMLP_DOUBLE into the kernel cache without a
  * device (the reference compiles them on first use, src_cpp/src/utils.cpp:12-35 and :145-180). */
 int qmlp_utils_pullpush_precompile(int precision);

@@ -49,6 +49,11 @@ int qmlp_hip_get_device_props(int device, qmlp_hip_device_props* props);
  * (src_cpp/src/tensor.cpp:41-44,68-98, include/qmlp/tmp_memory.h:14-36). */
 int qmlp_hip_malloc(void** ptr, size_t bytes);
 int qmlp_hip_free(void* ptr);
+/* Device memory in the order of a stream (hipMallocAsync / hipFreeAsync on the device's default pool, which gives
+ * back what is unused when the stream is synchronised): temporary memory of a call that does not wait for its own
+ * kernels. No counterpart in the reference, which allocates and frees such memory around a synchronisation. */
+int qmlp_hip_malloc_async(void** ptr, size_t bytes, qmlp_hip_stream stream);
+int qmlp_hip_free_async(void* ptr, qmlp_hip_stream stream);
 int qmlp_hip_memset_async(void* ptr, int value, size_t bytes, qmlp_hip_stream stream);
 int qmlp_hip_memcpy_h2d(void* dst, const void* src, size_t bytes, qmlp_hip_stream stream);
 int qmlp_hip_memcpy_d2h(void* dst, const void* src, size_t bytes, qmlp_hip_stream stream);

@@ -1,315 +1,695 @@
 #pragma once
-// Differentiable pull-push inpainting on an image pyramid (fractional masks): one kernel per
-// pyramid level and direction; every kernel is a grid-stride loop with one thread per pixel
-// and is bound by HBM bandwidth.
+// Differentiable pull-push inpainting on an image pyramid (fractional masks).
 //
 //   down:  low-res pixel = mask-weighted mean of its window of high-res pixels, low-res mask =
-//          maximum of the window (windows as in adaptive pooling: [floor(i*H/oH), ceil((i+1)*H/oH)),
-//          evaluated in fp32 like the reference; they overlap when a size is odd)
+//          maximum of the window (windows as in adaptive pooling, [floor(i*H/oH), ceil((i+1)*H/oH))
+//          with oH = H/2: rows 2i, 2i+1 of an even height, 2i .. 2i+2 of an odd one, where
+//          neighbouring windows share a row)
 //   up:    high-res pixel = m*data + (1-m)*(bilinear mix of the 4 nearest low-res pixels,
 //          weights 9/16, 3/16, 3/16, 1/16, renormalised by the low-res masks)
 //
+// The coarsest level (a row or a column of pixels) is its own inpainting. Every step is bound by HBM traffic
+// on the fine levels and by latency on the coarse ones (a launch for a level of 64 x 64 pixels takes 5 to 10 us, most of it
+// instructions and operands that arrive for the first time). Hence one launch per level while a level is large, and one
+// launch with a workgroup per image for all levels below, which then fit into LDS (4 channels of float: below 32 x 32).
+//
+// The unit of work is the quad: the 2 x 2 high-res pixels of one low-res pixel. Its pixels are moved in pairs
+// (8 or 16 bytes per lane) and share their 3 x 3 low-res neighbours (9 loads instead of 16).
+//
+// The adjoint walks the pyramid twice and keeps no per-pixel intermediates:
+//   A, fine to coarse: the gradient of the inpainted low-res level from that of the inpainted high-res level
+//      (adjoint of up with respect to the low-res level; the terms that high-res pixels pass down stay in LDS)
+//   B, coarse to fine: the gradient of a level before inpainting = adjoint of up with respect to the high-res
+//      level + adjoint of down, both formed per quad by gathering, without atomics
+// so a level of P pixels and C channels moves 2C+1 + (2C+2)/4 planes in A and 3C+2 + (5C+6)/4 planes in B.
+// 1 x 4 x 2048 x 2048 floats, finest level: down 21, up 37, A 49, B 68 us (4.9, 4.6, 2.6, 4.1 TB/s of the planes above; a
+// large copy reaches 5.2); the whole forward and adjoint call 435 us, of which 175 are levels of 1024 x 1024 and larger
+// (9.4 ms with four passes per level through memory, atomics for odd sizes, and memory allocated and released by every call).
+//
 // Follows src_cpp/include/qmlp/kernels/pullpush.cuh:22-303 of the reference. Differences on
-// purpose: no per-thread channel arrays (the channels are looped and the few mask values
-// re-read from cache), the adjoint of `down` adds with atomics when the windows of
-// neighbouring low-res pixels overlap (odd sizes; the reference adds without), and the adjoint
-// of `up` gathers per low-res pixel in a second pass instead of scattering with atomics.
+// purpose: no per-thread channel arrays, no atomics (the reference scatters the adjoint of up with atomics and adds
+// the adjoint of down without them, a race between overlapping windows), window limits in integers (the reference's
+// fp32 quotient is exact only while the products stay below 2^24), the pyramid of the forward pass is kept for the
+// adjoint pass.
 
 #include <qmlp/kernels/common.h>
 
 QUICKMLP_KERNEL_NAMESPACE_BEGIN
 
-template <typename T> using Tensor3Read = TensorAccessor<const T, 3>;
-template <typename T> using Tensor4Read = TensorAccessor<const T, 4>;
-template <typename T> using Tensor3RW = TensorAccessor<T, 3>;
-template <typename T> using Tensor4RW = TensorAccessor<T, 4>;
+/**
+ * A stack of images: entry (b, c, y, x); p == nullptr: absent. As built by the host (src/utils.cpp), which makes sure
+ * that the entries of a plane lie within 2^32 of each other: the same plane for a whole workgroup (scalar registers) and
+ * one 32-bit offset per lane.
+ */
+template <typename T>
+struct PullPushView
+{
+    T* p;
+    long long b, c;   // strides in entries
+    unsigned y, x;
+};
+
+/** One level of the pyramid. The views of the coarsest level alias (post = pre, its gradients too). */
+template <typename T>
+struct PullPushLevel
+{
+    int H, W;
+    PullPushView<T> maskPre, dataPre;     // before inpainting
+    PullPushView<T> maskPost, dataPost;   // inpainted; the mask of the finest level is absent
+    PullPushView<T> maskSum;              // sum of the masks of the window of this pixel in the finer level
+    PullPushView<T> gradMaskPost, gradDataPost, gradMaskPre, gradDataPre;   // adjoint; the first is absent on the finest level (zero)
+};
+
+constexpr int PULLPUSH_TAIL_BLOCK = 512;
+/** The levels that the kernels for all coarse levels keep in LDS: levels[0] is the one above them. */
+struct PullPushTail
+{
+    int numLevels;
+    int offsets[31];   // of level k in entries
+};
+/** Channels that are in flight together: their loads are issued before the first of them is used. */
+template <typename T> constexpr int pullpushChunk() { return sizeof(T) == 4 ? 4 : 2; }
 
 namespace pullpush
 {
-// clamped to [0, c]: the fp32 quotient is only exact while the products stay below 2^24
-__device__ __forceinline__ int windowStart(int a, int b, int c) { return max(0, static_cast<int>(floorf(static_cast<float>(a * c) / b))); }
-__device__ __forceinline__ int windowEnd(int a, int b, int c) { return min(c, static_cast<int>(ceilf(static_cast<float>((a + 1) * c) / b))); }
+template <typename T> struct Pair;
+template <> struct Pair<float> { typedef float type __attribute__((ext_vector_type(2))); };
+template <> struct Pair<double> { typedef double type __attribute__((ext_vector_type(2))); };
 
-template <typename A>
-__device__ __forceinline__ long long at3(const A& t, int b, int y, int x)
+template <typename T>
+__device__ __forceinline__ T* at(const PullPushView<T>& v, int b, int c, int y, int x)
 {
-    return static_cast<long long>(b) * t.strides_[0] + static_cast<long long>(y) * t.strides_[1]
-         + static_cast<long long>(x) * t.strides_[2];
-}
-template <typename A>
-__device__ __forceinline__ long long at4(const A& t, int b, int c, int y, int x)
-{
-    return static_cast<long long>(b) * t.strides_[0] + static_cast<long long>(c) * t.strides_[1]
-         + static_cast<long long>(y) * t.strides_[2] + static_cast<long long>(x) * t.strides_[3];
+    return v.p + (b * v.b + c * v.c) + (static_cast<unsigned>(y) * v.y + static_cast<unsigned>(x) * v.x);
 }
 
-__device__ __forceinline__ void atomicAccumulate(float* p, float v) { unsafeAtomicAdd(p, v); }
-__device__ __forceinline__ void atomicAccumulate(double* p, double v) { unsafeAtomicAdd(p, v); }
-
-/** Pixel (b, i, j) of the idx-th entry of a (B, h, w) image stack; 32-bit divisions whenever they suffice. */
-__device__ __forceinline__ void pixelOf(long long idx, int h, int w, int& b, int& i, int& j)
+/**
+ * Two neighbours in a row. PAIRS: the host found the images aligned for it, they are moved as one, and what lies behind
+ * an odd row is padding that belongs to the image. Otherwise the second is only touched if it exists (v[1] stays as it is).
+ */
+template <bool PAIRS, typename T>
+__device__ __forceinline__ void loadPair(const T* p, unsigned stride, bool second, T (&v)[2])
 {
-    if (idx <= 0x7fffffffLL) {
-        const unsigned u = static_cast<unsigned>(idx), uw = static_cast<unsigned>(w), uh = static_cast<unsigned>(h);
-        const unsigned row = u / uw;
-        j = static_cast<int>(u - row * uw);
-        b = static_cast<int>(row / uh);
-        i = static_cast<int>(row - static_cast<unsigned>(b) * uh);
+    if constexpr (PAIRS) {
+        const typename Pair<T>::type w = *reinterpret_cast<const typename Pair<T>::type*>(p);
+        v[0] = w[0];
+        v[1] = w[1];
     } else {
-        const long long row = idx / w;
-        j = static_cast<int>(idx - row * w);
-        b = static_cast<int>(row / h);
-        i = static_cast<int>(row - static_cast<long long>(b) * h);
+        v[0] = p[0];
+        if (second) v[1] = p[stride];
+    }
+}
+template <bool PAIRS, typename T>
+__device__ __forceinline__ void storePair(T* p, unsigned stride, bool second, const T (&v)[2])
+{
+    if constexpr (PAIRS) {
+        typename Pair<T>::type w;
+        w[0] = v[0];
+        w[1] = v[1];
+        *reinterpret_cast<typename Pair<T>::type*>(p) = w;
+    } else {
+        p[0] = v[0];
+        if (second) p[stride] = v[1];
     }
 }
 
-/** The 4 low-res neighbours of high-res pixel (i, j) and their bilinear weights. A neighbour
- *  outside the image has weight 0 and the coordinates of the pixel's own low-res cell clamped
- *  into the image, so that it can be loaded without a branch. */
-struct Neighbours
+/** down for the low-res pixel (a, e). */
+template <bool PAIRS, typename T>
+__device__ __forceinline__ void downPixel(const PullPushLevel<T>& high, const PullPushLevel<T>& low, int C, int b, int a, int e)
 {
-    int ii[4], jj[4];
-    float w[4];
-};
-__device__ __forceinline__ Neighbours neighbours(int i, int j, int oH, int oW)
-{
-    const int io = (i % 2 == 0) ? -1 : +1;
-    const int jo = (j % 2 == 0) ? -1 : +1;
-    Neighbours n;
-    n.ii[0] = i / 2;      n.jj[0] = j / 2;      n.w[0] = 0.75f * 0.75f;
-    n.ii[1] = i / 2 + io; n.jj[1] = j / 2;      n.w[1] = 0.25f * 0.75f;
-    n.ii[2] = i / 2;      n.jj[2] = j / 2 + jo; n.w[2] = 0.25f * 0.75f;
-    n.ii[3] = i / 2 + io; n.jj[3] = j / 2 + jo; n.w[3] = 0.25f * 0.25f;
+    const int rows = 2 + (high.H & 1), columns = 2 + (high.W & 1);
+    T m[3][3];
+    T sum = 0, most = 0;
+    auto window = [&](const PullPushView<T>& v, int c, T (&out)[3][3]) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const bool inside = n.ii[k] >= 0 && n.jj[k] >= 0 && n.ii[k] < oH && n.jj[k] < oW;
-        n.w[k] = inside ? n.w[k] : 0.f;
-        n.ii[k] = min(max(n.ii[k], 0), oH - 1);
-        n.jj[k] = min(max(n.jj[k], 0), oW - 1);
+        for (int i = 0; i < 3; ++i) {
+            out[i][0] = out[i][1] = out[i][2] = T(0);
+            if (i >= rows) continue;
+            const T* p = at(v, b, c, 2 * a + i, 2 * e);
+            T pair[2];
+            loadPair<PAIRS>(p, v.x, true, pair);
+            out[i][0] = pair[0];
+            out[i][1] = pair[1];
+            if (columns > 2) out[i][2] = p[2 * v.x];
+        }
+    };
+    window(high.maskPre, 0, m);
+    // column by column, as the sums of the whole pyramid have always been taken
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            sum += m[i][j];             // (entries beyond the window are zero)
+            most = max(most, m[i][j]);
+        }
+    *at(low.maskPre, b, 0, a, e) = most;
+    *at(low.maskSum, b, 0, a, e) = sum;
+    const T inverse = sum > 0 ? T(1) / sum : T(0);
+    constexpr int CHUNK = pullpushChunk<T>();
+    for (int c0 = 0; c0 < C; c0 += CHUNK) {
+        T d[CHUNK];
+#pragma unroll
+        for (int k = 0; k < CHUNK; ++k) {
+            T v[3][3];
+            d[k] = T(0);
+            if (c0 + k >= C) continue;
+            window(high.dataPre, c0 + k, v);
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                    if (i < rows && j < columns) d[k] += m[i][j] * v[i][j];
+        }
+#pragma unroll
+        for (int k = 0; k < CHUNK; ++k)
+            if (c0 + k < C) *at(low.dataPre, b, c0 + k, a, e) = d[k] * inverse;
     }
-    return n;
+}
+
+/** The low-res neighbourhood of a quad (a, e): rows a-1 .. a+1, columns e-1 .. e+1, clamped into the image;
+ *  validity as factors of the bilinear weights. */
+struct Neighbourhood
+{
+    int row[3], column[3];
+    float rowIn[3], columnIn[3];
+    __device__ __forceinline__ Neighbourhood(int a, int e, int oH, int oW)
+    {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int y = a - 1 + k, x = e - 1 + k;
+            rowIn[k] = y >= 0 && y < oH ? 1.f : 0.f;
+            columnIn[k] = x >= 0 && x < oW ? 1.f : 0.f;
+            row[k] = min(max(y, 0), oH - 1);
+            column[k] = min(max(x, 0), oW - 1);
+        }
+    }
+    template <typename T>
+    __device__ __forceinline__ void load(const PullPushView<T>& v, int b, int c, T (&out)[3][3]) const
+    {
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) out[i][j] = *at(v, b, c, row[i], column[j]);
+    }
+    /** Weights of the own cell, the neighbour in the other row, in the other column, and the diagonal one, for pixel (di, dj) of the quad. */
+    __device__ __forceinline__ void weights(int di, int dj, float (&w)[4]) const
+    {
+        const float own = 0.75f * rowIn[1], other = 0.25f * rowIn[2 * di];
+        const float ownColumn = 0.75f * columnIn[1], otherColumn = 0.25f * columnIn[2 * dj];
+        w[0] = own * ownColumn;
+        w[1] = other * ownColumn;
+        w[2] = own * otherColumn;
+        w[3] = other * otherColumn;
+    }
+    template <typename T>
+    __device__ __forceinline__ static void pick(const T (&v)[3][3], int di, int dj, T (&out)[4])
+    {
+        out[0] = v[1][1];
+        out[1] = v[2 * di][1];
+        out[2] = v[1][2 * dj];
+        out[3] = v[2 * di][2 * dj];
+    }
+};
+
+/** Masks and weights of the low-res neighbours of the four pixels of a quad: wm[k] = weight * mask, their sum n. */
+template <typename T>
+struct QuadMix
+{
+    T wm[2][2][4], n[2][2], inverse[2][2], weight[2][2];   // (inverse: 1 / n, or zero)
+    __device__ __forceinline__ QuadMix(const Neighbourhood& nb, const T (&maskLow)[3][3])
+    {
+#pragma unroll
+        for (int di = 0; di < 2; ++di)
+#pragma unroll
+            for (int dj = 0; dj < 2; ++dj) {
+                float w[4];
+                T ml[4];
+                nb.weights(di, dj, w);
+                nb.pick(maskLow, di, dj, ml);
+                weight[di][dj] = 0;
+                n[di][dj] = 0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    wm[di][dj][k] = w[k] * ml[k];
+                    weight[di][dj] += w[k];
+                    n[di][dj] += wm[di][dj][k];
+                }
+                inverse[di][dj] = n[di][dj] > 0 ? T(1) / n[di][dj] : T(0);
+            }
+    }
+    /** The weighted sum of a channel for pixel (di, dj). */
+    __device__ __forceinline__ T sum(const T (&low)[3][3], int di, int dj) const
+    {
+        T v[4];
+        Neighbourhood::pick(low, di, dj, v);
+        T d = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) d += wm[di][dj][k] * v[k];
+        return d;
+    }
+};
+
+/** up for the quad (a, e) of the high-res level. */
+template <bool PAIRS, typename T>
+__device__ __forceinline__ void upQuad(const PullPushLevel<T>& high, const PullPushLevel<T>& low, int C, int b, int a, int e)
+{
+    const Neighbourhood nb(a, e, low.H, low.W);
+    T lowMask[3][3];
+    nb.load(low.maskPost, b, 0, lowMask);
+    const QuadMix<T> mix(nb, lowMask);
+    const bool second = 2 * e + 1 < high.W;
+    T m[2][2];
+#pragma unroll
+    for (int di = 0; di < 2; ++di) {
+        m[di][0] = m[di][1] = T(0);
+        if (2 * a + di >= high.H) continue;
+        loadPair<PAIRS>(at(high.maskPre, b, 0, 2 * a + di, 2 * e), high.maskPre.x, second, m[di]);
+        if (!high.maskPost.p) continue;
+        T out[2];
+#pragma unroll
+        for (int dj = 0; dj < 2; ++dj)
+            out[dj] = m[di][dj] + (mix.n[di][dj] > 0 ? (1 - m[di][dj]) * (mix.n[di][dj] / mix.weight[di][dj]) : T(0));
+        storePair<PAIRS>(at(high.maskPost, b, 0, 2 * a + di, 2 * e), high.maskPost.x, second, out);
+    }
+    constexpr int CHUNK = pullpushChunk<T>();
+    for (int c0 = 0; c0 < C; c0 += CHUNK) {
+        T lowData[CHUNK][3][3], v[CHUNK][2][2];
+#pragma unroll
+        for (int k = 0; k < CHUNK; ++k) {
+            if (c0 + k >= C) continue;
+            nb.load(low.dataPost, b, c0 + k, lowData[k]);
+#pragma unroll
+            for (int di = 0; di < 2; ++di)
+                if (2 * a + di < high.H) loadPair<PAIRS>(at(high.dataPre, b, c0 + k, 2 * a + di, 2 * e), high.dataPre.x, second, v[k][di]);
+        }
+#pragma unroll
+        for (int k = 0; k < CHUNK; ++k) {
+            if (c0 + k >= C) continue;
+#pragma unroll
+            for (int di = 0; di < 2; ++di) {
+                if (2 * a + di >= high.H) continue;
+                T out[2];
+#pragma unroll
+                for (int dj = 0; dj < 2; ++dj)
+                    out[dj] = m[di][dj] * v[k][di][dj] + (1 - m[di][dj]) * (mix.sum(lowData[k], di, dj) * mix.inverse[di][dj]);
+                storePair<PAIRS>(at(high.dataPost, b, c0 + k, 2 * a + di, 2 * e), high.dataPost.x, second, out);
+            }
+        }
+    }
+}
+
+constexpr int pullpushTileEntries(int tw, int th) { return 2 * (th + 2) * (2 * (tw + 2) + 1); }   // high-res pixels of a tile with its border
+
+/**
+ * Step A for the TW x TH low-res pixels from (a0, e0) on, by a workgroup of TW * TH threads (all of them call this):
+ *   gradDataPost_c of the low-res pixel = mask * sum over the 4 x 4 high-res pixels p that interpolate from it of w_p fill_c(p)
+ *   gradMaskPost                        = sum of w_p (fillN(p) + sum_c fill_c(p) data_c)
+ * with fill_c(p) the gradient of the weighted low-res sum d_c of p and fillN(p) that of its mask sum n. A thread forms these
+ * terms for the quads of the tile and a border of one quad (34 x 10 quads for 32 x 8 pixels) and they wait in LDS, a
+ * few channels at a time, until the low-res pixels gather them; fillN (the last plane) is summed over the channels there.
+ */
+template <bool PAIRS, int TW, int TH, typename T>
+__device__ __forceinline__ void gradientUpTile(const PullPushLevel<T>& high, const PullPushLevel<T>& low, int C, int b, int a0, int e0,
+                                               T (&sFill)[pullpushChunk<T>() + 1][pullpushTileEntries(TW, TH)])
+{
+    constexpr int THREADS = TW * TH, QW = TW + 2, QH = TH + 2, QUADS = QW * QH, CHUNK = pullpushChunk<T>();
+    constexpr int STRIDE = 2 * QW + 1;   // entries per row of high-res pixels
+    const int la = threadIdx.x / TW, le = threadIdx.x % TW;
+    const int a = a0 + la, e = e0 + le;
+    const bool mine = a < low.H && e < low.W;
+    auto gather = [&](const T* plane) {
+        T sum = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const T* row = plane + (2 * la + 1 + i) * STRIDE + 2 * le + 1;
+            const float wr = (i == 1 || i == 2) ? 0.75f : 0.25f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sum += (wr * ((j == 1 || j == 2) ? 0.75f : 0.25f)) * row[j];
+        }
+        return sum;
+    };
+    T lowMask = 0, gradMask = 0;
+    if (mine) lowMask = *at(low.maskPost, b, 0, a, e);
+    for (int c0 = 0; c0 < C; c0 += CHUNK) {
+        __syncthreads();   // what the previous channels (or tile) left has been gathered
+#pragma unroll 1
+        for (int quad = threadIdx.x; quad < QUADS; quad += THREADS) {
+            const int qa = a0 - 1 + quad / QW, qe = e0 - 1 + quad % QW;
+            const int at0 = 2 * (quad / QW) * STRIDE + 2 * (quad % QW);
+            T fill[CHUNK][2][2], fillN[2][2];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                fillN[i >> 1][i & 1] = T(0);
+#pragma unroll
+                for (int k = 0; k < CHUNK; ++k) fill[k][i >> 1][i & 1] = T(0);
+            }
+            if (qa >= 0 && qe >= 0 && 2 * qa < high.H && 2 * qe < high.W) {
+                const Neighbourhood nb(qa, qe, low.H, low.W);
+                const bool second = 2 * qe + 1 < high.W;
+                T masks[3][3], lowData[CHUNK][3][3], m[2][2], gm[2][2];
+                nb.load(low.maskPost, b, 0, masks);
+#pragma unroll
+                for (int di = 0; di < 2; ++di) {
+                    m[di][0] = m[di][1] = T(0);
+                    gm[di][0] = gm[di][1] = T(0);
+                    if (2 * qa + di >= high.H) continue;
+                    loadPair<PAIRS>(at(high.maskPre, b, 0, 2 * qa + di, 2 * qe), high.maskPre.x, second, m[di]);
+                    if (c0 == 0 && high.gradMaskPost.p)
+                        loadPair<PAIRS>(at(high.gradMaskPost, b, 0, 2 * qa + di, 2 * qe), high.gradMaskPost.x, second, gm[di]);
+                }
+#pragma unroll
+                for (int k = 0; k < CHUNK; ++k) {
+                    if (c0 + k >= C) continue;
+                    nb.load(low.dataPost, b, c0 + k, lowData[k]);
+#pragma unroll
+                    for (int di = 0; di < 2; ++di)
+                        if (2 * qa + di < high.H)   // (the gradient: turned into the fill below)
+                            loadPair<PAIRS>(at(high.gradDataPost, b, c0 + k, 2 * qa + di, 2 * qe), high.gradDataPost.x, second, fill[k][di]);
+                }
+                const QuadMix<T> mix(nb, masks);
+#pragma unroll
+                for (int di = 0; di < 2; ++di)
+#pragma unroll
+                    for (int dj = 0; dj < 2; ++dj) {
+                        if (2 * qa + di >= high.H || (dj == 1 && !second)) {
+                            // outside: passes nothing down
+#pragma unroll
+                            for (int k = 0; k < CHUNK; ++k) fill[k][di][dj] = T(0);
+                            continue;
+                        }
+                        const T passed = (1 - m[di][dj]) * mix.inverse[di][dj];
+                        if (c0 == 0) fillN[di][dj] = gm[di][dj] * ((1 - m[di][dj]) / mix.weight[di][dj]);
+#pragma unroll
+                        for (int k = 0; k < CHUNK; ++k) {
+                            if (c0 + k >= C) continue;
+                            fill[k][di][dj] *= passed;
+                            fillN[di][dj] -= fill[k][di][dj] * (mix.sum(lowData[k], di, dj) * mix.inverse[di][dj]);
+                        }
+                    }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int entry = at0 + (i >> 1) * STRIDE + (i & 1);
+#pragma unroll
+                for (int k = 0; k < CHUNK; ++k)
+                    if (c0 + k < C) sFill[k][entry] = fill[k][i >> 1][i & 1];
+                sFill[CHUNK][entry] = (c0 == 0 ? T(0) : sFill[CHUNK][entry]) + fillN[i >> 1][i & 1];
+            }
+        }
+        __syncthreads();
+        if (!mine) continue;
+#pragma unroll
+        for (int k = 0; k < CHUNK; ++k) {
+            if (c0 + k >= C) continue;
+            const T sum = gather(sFill[k]);
+            gradMask += sum * *at(low.dataPost, b, c0 + k, a, e);
+            *at(low.gradDataPost, b, c0 + k, a, e) = sum * lowMask;
+        }
+    }
+    if (mine) *at(low.gradMaskPost, b, 0, a, e) = gradMask + gather(sFill[CHUNK]);
+}
+
+/**
+ * Step B for the quad (a, e) of the high-res level: the gradients of its pixels before inpainting.
+ * \tparam ACCUMULATE add to what is there
+ */
+template <bool PAIRS, bool ACCUMULATE, typename T>
+__device__ __forceinline__ void gradientQuad(const PullPushLevel<T>& high, const PullPushLevel<T>& low, int C, int b, int a, int e)
+{
+    const Neighbourhood nb(a, e, low.H, low.W);
+    T lowMask[3][3];
+    nb.load(low.maskPost, b, 0, lowMask);
+    const QuadMix<T> mix(nb, lowMask);
+    const bool second = 2 * e + 1 < high.W;
+    // the low-res windows the pixels lie in: (a, e), and of odd sizes also those of the row above and the column to the
+    // left, which reach into the first row and column of the quad
+    const bool oddH = high.H & 1, oddW = high.W & 1;
+    bool in[2][2];
+    T inverse[2][2], most[2][2], gradMost[2][2];
+#pragma unroll
+    for (int wa = 0; wa < 2; ++wa)
+#pragma unroll
+        for (int we = 0; we < 2; ++we) {
+            const int y = a - wa, x = e - we;
+            in[wa][we] = (wa == 0 || oddH) && (we == 0 || oddW) && y >= 0 && x >= 0 && y < low.H && x < low.W;
+            inverse[wa][we] = most[wa][we] = gradMost[wa][we] = T(0);
+            if (!in[wa][we]) continue;
+            const T sum = *at(low.maskSum, b, 0, y, x);
+            inverse[wa][we] = sum > 0 ? T(1) / sum : T(0);
+            most[wa][we] = *at(low.maskPre, b, 0, y, x);
+            gradMost[wa][we] = *at(low.gradMaskPre, b, 0, y, x);
+        }
+    T m[2][2], gradMask[2][2];
+#pragma unroll
+    for (int di = 0; di < 2; ++di) {
+        m[di][0] = m[di][1] = gradMask[di][0] = gradMask[di][1] = T(0);
+        if (2 * a + di >= high.H) continue;
+        loadPair<PAIRS>(at(high.maskPre, b, 0, 2 * a + di, 2 * e), high.maskPre.x, second, m[di]);
+        T gm[2] = {T(0), T(0)};
+        if (high.gradMaskPost.p)
+            loadPair<PAIRS>(at(high.gradMaskPost, b, 0, 2 * a + di, 2 * e), high.gradMaskPost.x, second, gm);
+#pragma unroll
+        for (int dj = 0; dj < 2; ++dj) {
+            if (dj == 1 && !second) continue;
+            // maskHigh = m + (n > 0 ? (1 - m) * n / weight : 0)
+            gradMask[di][dj] = high.gradMaskPost.p ? gm[dj] * (1 - mix.n[di][dj] / mix.weight[di][dj]) : T(0);
+            // the maximum of a window passes its gradient to every pixel that attains it
+#pragma unroll
+            for (int wa = 0; wa <= 1 - di; ++wa)
+#pragma unroll
+                for (int we = 0; we <= 1 - dj; ++we)
+                    if (in[wa][we] && most[wa][we] == m[di][dj]) gradMask[di][dj] += gradMost[wa][we];
+        }
+    }
+    constexpr int CHUNK = 1;   // (more of them in flight cost more wavefronts than they hide: 2048 x 2048 floats 70 us with one, 98 us with two)
+    for (int c0 = 0; c0 < C; c0 += CHUNK) {
+        T lowData[CHUNK][3][3], v[CHUNK][2][2], g[CHUNK][2][2], before[CHUNK][2][2];
+        T mean[CHUNK][2][2], grad[CHUNK][2][2];   // of the windows
+#pragma unroll
+        for (int k = 0; k < CHUNK; ++k) {
+            if (c0 + k >= C) continue;
+            nb.load(low.dataPost, b, c0 + k, lowData[k]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int wa = i >> 1, we = i & 1;
+                mean[k][wa][we] = grad[k][wa][we] = T(0);
+                if (!in[wa][we]) continue;
+                mean[k][wa][we] = *at(low.dataPre, b, c0 + k, a - wa, e - we);
+                grad[k][wa][we] = *at(low.gradDataPre, b, c0 + k, a - wa, e - we) * inverse[wa][we];
+            }
+#pragma unroll
+            for (int di = 0; di < 2; ++di) {
+                before[k][di][0] = before[k][di][1] = T(0);
+                if (2 * a + di >= high.H) continue;
+                loadPair<PAIRS>(at(high.dataPre, b, c0 + k, 2 * a + di, 2 * e), high.dataPre.x, second, v[k][di]);
+                loadPair<PAIRS>(at(high.gradDataPost, b, c0 + k, 2 * a + di, 2 * e), high.gradDataPost.x, second, g[k][di]);
+                if (ACCUMULATE) loadPair<PAIRS>(at(high.gradDataPre, b, c0 + k, 2 * a + di, 2 * e), high.gradDataPre.x, second, before[k][di]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < CHUNK; ++k) {
+            if (c0 + k >= C) continue;
+#pragma unroll
+            for (int di = 0; di < 2; ++di) {
+                if (2 * a + di >= high.H) continue;
+                T out[2];
+#pragma unroll
+                for (int dj = 0; dj < 2; ++dj) {
+                    // dataHigh = m * data + (1 - m) * (n > 0 ? d / n : 0)
+                    gradMask[di][dj] += g[k][di][dj] * (v[k][di][dj] - mix.sum(lowData[k], di, dj) * mix.inverse[di][dj]);
+                    T sum = g[k][di][dj];
+#pragma unroll
+                    for (int wa = 0; wa <= 1 - di; ++wa)
+#pragma unroll
+                        for (int we = 0; we <= 1 - dj; ++we) {
+                            // dataLow = sum m * data / sum m
+                            if (!in[wa][we]) continue;
+                            sum += grad[k][wa][we];
+                            gradMask[di][dj] += grad[k][wa][we] * (v[k][di][dj] - mean[k][wa][we]);
+                        }
+                    out[dj] = before[k][di][dj] + m[di][dj] * sum;
+                }
+                storePair<PAIRS>(at(high.gradDataPre, b, c0 + k, 2 * a + di, 2 * e), high.gradDataPre.x, second, out);
+            }
+        }
+    }
+#pragma unroll
+    for (int di = 0; di < 2; ++di) {
+        if (2 * a + di >= high.H) continue;
+        T* target = at(high.gradMaskPre, b, 0, 2 * a + di, 2 * e);
+        if (ACCUMULATE) {
+            T before[2];
+            loadPair<PAIRS>(target, high.gradMaskPre.x, second, before);
+            gradMask[di][0] += before[0];
+            gradMask[di][1] += before[1];
+        }
+        storePair<PAIRS>(target, high.gradMaskPre.x, second, gradMask[di]);
+    }
+}
+
+constexpr int TILE_W = 32, TILE_H = 8;   // of the kernels with a launch per level: 256 threads
+
+/**
+ * Tile of this workgroup: a stack of B images of width x height items in tiles of TILE_W x TILE_H. Workgroups go to the 8 XCDs
+ * in turn; every XCD gets a run of consecutive tiles, whose borders then meet in its own L2.
+ */
+__device__ __forceinline__ void tileOf(int width, int height, int& b, int& a0, int& e0)
+{
+    constexpr unsigned XCDS = 8;
+    const unsigned xcd = blockIdx.x % XCDS, perXcd = gridDim.x / XCDS, more = gridDim.x % XCDS;
+    const unsigned tile = xcd * perXcd + min(xcd, more) + blockIdx.x / XCDS;
+    const unsigned tilesX = (width + TILE_W - 1) / TILE_W, tilesY = (height + TILE_H - 1) / TILE_H;
+    const unsigned row = tile / tilesX;
+    e0 = static_cast<int>(tile - row * tilesX) * TILE_W;
+    b = static_cast<int>(row / tilesY);
+    a0 = static_cast<int>(row - b * tilesY) * TILE_H;
+}
+
+/**
+ * Level k (> 0) of the coarse levels that one workgroup keeps in LDS, below a level of H x W pixels (sizes are halved, rounding
+ * down, and rows start at even entries). The views have no image stride: a workgroup has one image.
+ */
+template <typename T, bool GRADIENTS>
+__device__ __forceinline__ PullPushLevel<T> ldsLevel(T* sLevels, const PullPushTail& tail, int H, int W, int C, int k)
+{
+    T* next = sLevels + tail.offsets[k];
+    PullPushLevel<T> l;
+    l.H = H >> k;
+    l.W = W >> k;
+    const unsigned pitch = (l.W + 1) & ~1, plane = l.H * pitch;
+    auto take = [&](int channels) {
+        PullPushView<T> v{next, 0, plane, pitch, 1};
+        next += channels * plane;
+        return v;
+    };
+    l.maskPre = take(1);
+    l.dataPre = take(C);
+    l.maskSum = take(1);
+    const bool coarsest = k == tail.numLevels - 1;   // its own inpainting: nothing changes from before to after
+    l.maskPost = coarsest ? l.maskPre : take(1);
+    l.dataPost = coarsest ? l.dataPre : take(C);
+    if (GRADIENTS) {
+        l.gradMaskPost = take(1);
+        l.gradDataPost = take(C);
+        l.gradMaskPre = coarsest ? l.gradMaskPost : take(1);
+        l.gradDataPre = coarsest ? l.gradDataPost : take(C);
+    }
+    return l;
 }
 } // namespace pullpush
 
-/** One thread per low-res pixel (b, i, j). */
 template <typename T>
-__global__ void __launch_bounds__(256) PullPushDownKernel(
-    long long numel, const Tensor3Read<T> mask, const Tensor4Read<T> data, Tensor3RW<T> maskLow, Tensor4RW<T> dataLow)
+__global__ void __launch_bounds__(256) PullPushDownKernel(const PullPushLevel<T> high, const PullPushLevel<T> low, int C, int pairs)
 {
     using namespace pullpush;
-    const int H = mask.sizes_[1], W = mask.sizes_[2], oH = H / 2, oW = W / 2, C = data.sizes_[1];
-    for (long long idx = blockIdx.x * static_cast<long long>(blockDim.x) + threadIdx.x; idx < numel;
-         idx += static_cast<long long>(blockDim.x) * gridDim.x)
-    {
-        int b, i, j;
-        pixelOf(idx, oH, oW, b, i, j);
-        const int i0 = windowStart(i, oH, H), i1 = windowEnd(i, oH, H), j0 = windowStart(j, oW, W), j1 = windowEnd(j, oW, W);
-        T n1 = 0, n2 = 0;
-        for (int jj = j0; jj < j1; ++jj)
-            for (int ii = i0; ii < i1; ++ii) {
-                const T m = mask.data_[at3(mask, b, ii, jj)];
-                n1 += m;
-                n2 = max(n2, m);
-            }
-        maskLow.data_[at3(maskLow, b, i, j)] = n2;
-        for (int c = 0; c < C; ++c) {
-            T d = 0;
-            for (int jj = j0; jj < j1; ++jj)
-                for (int ii = i0; ii < i1; ++ii) d += mask.data_[at3(mask, b, ii, jj)] * data.data_[at4(data, b, c, ii, jj)];
-            dataLow.data_[at4(dataLow, b, c, i, j)] = n1 > 0 ? d / n1 : T(0);
-        }
-    }
+    int b, a, e;
+    tileOf(low.W, low.H, b, a, e);
+    a += threadIdx.x / TILE_W;
+    e += threadIdx.x % TILE_W;
+    if (a >= low.H || e >= low.W) return;
+    if (pairs) downPixel<true>(high, low, C, b, a, e);
+    else downPixel<false>(high, low, C, b, a, e);
 }
 
-/** One thread per high-res pixel (b, i, j). */
 template <typename T>
-__global__ void __launch_bounds__(256) PullPushUpKernel(
-    long long numel, const Tensor3Read<T> mask, const Tensor4Read<T> data, const Tensor3Read<T> maskLow,
-    const Tensor4Read<T> dataLow, Tensor3RW<T> maskHigh, Tensor4RW<T> dataHigh)
+__global__ void __launch_bounds__(256) PullPushUpKernel(const PullPushLevel<T> high, const PullPushLevel<T> low, int C, int pairs)
 {
     using namespace pullpush;
-    const int H = mask.sizes_[1], W = mask.sizes_[2], oH = H / 2, oW = W / 2, C = data.sizes_[1];
-    for (long long idx = blockIdx.x * static_cast<long long>(blockDim.x) + threadIdx.x; idx < numel;
-         idx += static_cast<long long>(blockDim.x) * gridDim.x)
-    {
-        int b, i, j;
-        pixelOf(idx, H, W, b, i, j);
-        const Neighbours nb = neighbours(i, j, oH, oW);
-        T weight = 0, n = 0, ml[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            ml[k] = maskLow.data_[at3(maskLow, b, nb.ii[k], nb.jj[k])];
-            weight += nb.w[k];
-            n += nb.w[k] * ml[k];
-        }
-        const T m = mask.data_[at3(mask, b, i, j)];
-        maskHigh.data_[at3(maskHigh, b, i, j)] = m + (n > 0 ? (1 - m) * (n / weight) : T(0));
-        for (int c = 0; c < C; ++c) {
-            T d = 0;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                d += nb.w[k] * ml[k] * dataLow.data_[at4(dataLow, b, c, nb.ii[k], nb.jj[k])];
-            dataHigh.data_[at4(dataHigh, b, c, i, j)] = m * data.data_[at4(data, b, c, i, j)] + (1 - m) * (n > 0 ? d / n : T(0));
-        }
-    }
+    int b, a, e;
+    const int height = (high.H + 1) / 2, width = (high.W + 1) / 2;
+    tileOf(width, height, b, a, e);
+    a += threadIdx.x / TILE_W;
+    e += threadIdx.x % TILE_W;
+    if (a >= height || e >= width) return;
+    if (pairs) upQuad<true>(high, low, C, b, a, e);
+    else upQuad<false>(high, low, C, b, a, e);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) PullPushGradientUpKernel(const PullPushLevel<T> high, const PullPushLevel<T> low, int C, int pairs)
+{
+    using namespace pullpush;
+    __shared__ T sFill[pullpushChunk<T>() + 1][pullpushTileEntries(TILE_W, TILE_H)];
+    int b, a0, e0;
+    tileOf(low.W, low.H, b, a0, e0);
+    if (pairs) gradientUpTile<true, TILE_W, TILE_H>(high, low, C, b, a0, e0, sFill);
+    else gradientUpTile<false, TILE_W, TILE_H>(high, low, C, b, a0, e0, sFill);
+}
+
+template <typename T, bool ACCUMULATE>
+__global__ void __launch_bounds__(256) PullPushGradientKernel(const PullPushLevel<T> high, const PullPushLevel<T> low, int C, int pairs)
+{
+    using namespace pullpush;
+    int b, a, e;
+    const int height = (high.H + 1) / 2, width = (high.W + 1) / 2;
+    tileOf(width, height, b, a, e);
+    a += threadIdx.x / TILE_W;
+    e += threadIdx.x % TILE_W;
+    if (a >= height || e >= width) return;
+    if (pairs) gradientQuad<true, ACCUMULATE>(high, low, C, b, a, e);
+    else gradientQuad<false, ACCUMULATE>(high, low, C, b, a, e);
 }
 
 /**
- * Adjoint of PullPushDownKernel; one thread per low-res pixel, gradients accumulated.
- * \tparam OVERLAP the windows of neighbouring low-res pixels share high-res pixels (an odd
- *   height or width): accumulate with atomics. Otherwise every high-res pixel has one owner.
+ * All coarse levels, one workgroup per image: from 'finest' down to the coarsest level and up again. The levels
+ * below 'finest' live in LDS (dynamic, sized by the host) and are not kept: the adjoint forms them again.
  */
-template <typename T, bool OVERLAP>
-__global__ void __launch_bounds__(256) PullPushAdjointDownKernel(
-    long long numel, const Tensor3Read<T> mask, const Tensor4Read<T> data, const Tensor3Read<T> gradMaskLow,
-    const Tensor4Read<T> gradDataLow, Tensor3RW<T> gradMask, Tensor4RW<T> gradData)
+template <typename T>
+__global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushTailKernel(const PullPushLevel<T> finest, int C, const PullPushTail tail)
 {
     using namespace pullpush;
-    const int H = mask.sizes_[1], W = mask.sizes_[2], oH = H / 2, oW = W / 2, C = data.sizes_[1];
-    for (long long idx = blockIdx.x * static_cast<long long>(blockDim.x) + threadIdx.x; idx < numel;
-         idx += static_cast<long long>(blockDim.x) * gridDim.x)
-    {
-        int b, i, j;
-        pixelOf(idx, oH, oW, b, i, j);
-        const int i0 = windowStart(i, oH, H), i1 = windowEnd(i, oH, H), j0 = windowStart(j, oW, W), j1 = windowEnd(j, oW, W);
-        T n1 = 0, n2 = 0;
-        for (int jj = j0; jj < j1; ++jj)
-            for (int ii = i0; ii < i1; ++ii) {
-                const T m = mask.data_[at3(mask, b, ii, jj)];
-                n1 += m;
-                n2 = max(n2, m);
-            }
-        // dataLow_c = d_c / n1: adjoint of n1 collects all channels
-        T adjN1 = 0;
-        for (int c = 0; c < C; ++c) {
-            T d = 0;
-            for (int jj = j0; jj < j1; ++jj)
-                for (int ii = i0; ii < i1; ++ii) d += mask.data_[at3(mask, b, ii, jj)] * data.data_[at4(data, b, c, ii, jj)];
-            if (n1 > 0) adjN1 -= gradDataLow.data_[at4(gradDataLow, b, c, i, j)] * d / (n1 * n1);
-        }
-        const T adjN2 = gradMaskLow.data_[at3(gradMaskLow, b, i, j)];
-        for (int jj = j0; jj < j1; ++jj)
-            for (int ii = i0; ii < i1; ++ii) {
-                const T m = mask.data_[at3(mask, b, ii, jj)];
-                T adjMask = adjN1;
-                for (int c = 0; c < C; ++c) {
-                    const T adjD = n1 > 0 ? gradDataLow.data_[at4(gradDataLow, b, c, i, j)] / n1 : T(0);
-                    T* target = gradData.data_ + at4(gradData, b, c, ii, jj);
-                    if (OVERLAP) atomicAccumulate(target, adjD * m);
-                    else *target += adjD * m;
-                    adjMask += adjD * data.data_[at4(data, b, c, ii, jj)];
-                }
-                if (n2 == m) adjMask += adjN2;   // the maximum passes its gradient to every pixel that attains it
-                T* target = gradMask.data_ + at3(gradMask, b, ii, jj);
-                if (OVERLAP) atomicAccumulate(target, adjMask);
-                else *target += adjMask;
-            }
+    extern __shared__ __align__(16) unsigned char sMemory[];
+    T* sLevels = reinterpret_cast<T*>(sMemory);
+    const int b = blockIdx.x;
+    auto level = [&](int k) { return k == 0 ? finest : ldsLevel<T, false>(sLevels, tail, finest.H, finest.W, C, k); };
+    for (int k = 0; k + 1 < tail.numLevels; ++k) {
+        const auto high = level(k), low = level(k + 1);
+        for (int i = threadIdx.x; i < low.H * low.W; i += PULLPUSH_TAIL_BLOCK) downPixel<false>(high, low, C, b, i / low.W, i % low.W);
+        __syncthreads();
+    }
+    for (int k = tail.numLevels - 2; k >= 0; --k) {
+        const auto high = level(k), low = level(k + 1);
+        const int height = (high.H + 1) / 2, width = (high.W + 1) / 2;
+        for (int i = threadIdx.x; i < height * width; i += PULLPUSH_TAIL_BLOCK) upQuad<false>(high, low, C, b, i / width, i % width);
+        __syncthreads();
     }
 }
 
-/**
- * Adjoint of PullPushUpKernel, first pass; one thread per high-res pixel. Adds the gradients of
- * this level's inputs into gradMask / gradData and stores what the low-res level needs from
- * this pixel: adjFill(b, c, i, j) = gradient of the channel's weighted low-res sum d_c,
- * adjFill(b, C, i, j) = gradient of the low-res mask sum n.
- */
-template <typename T>
-__global__ void __launch_bounds__(256) PullPushAdjointUpKernel(
-    long long numel, const Tensor3Read<T> mask, const Tensor4Read<T> data, const Tensor3Read<T> maskLow,
-    const Tensor4Read<T> dataLow, const Tensor3Read<T> gradMaskHigh, const Tensor4Read<T> gradDataHigh,
-    Tensor3RW<T> gradMask, Tensor4RW<T> gradData, Tensor4RW<T> adjFill)
+/** The adjoint of all coarse levels, one workgroup per image. ACCUMULATE: 'finest' is the image itself and its gradients are added to. */
+template <typename T, bool ACCUMULATE>
+__global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushGradientTailKernel(const PullPushLevel<T> finest, int C, const PullPushTail tail)
 {
     using namespace pullpush;
-    const int H = mask.sizes_[1], W = mask.sizes_[2], oH = H / 2, oW = W / 2, C = data.sizes_[1];
-    for (long long idx = blockIdx.x * static_cast<long long>(blockDim.x) + threadIdx.x; idx < numel;
-         idx += static_cast<long long>(blockDim.x) * gridDim.x)
-    {
-        int b, i, j;
-        pixelOf(idx, H, W, b, i, j);
-        const Neighbours nb = neighbours(i, j, oH, oW);
-        T weight = 0, n = 0, ml[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            ml[k] = maskLow.data_[at3(maskLow, b, nb.ii[k], nb.jj[k])];
-            weight += nb.w[k];
-            n += nb.w[k] * ml[k];
-        }
-        const T m = mask.data_[at3(mask, b, i, j)];
-        T adjMask = 0, adjN = 0;
-        for (int c = 0; c < C; ++c) {
-            T d = 0;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                d += nb.w[k] * ml[k] * dataLow.data_[at4(dataLow, b, c, nb.ii[k], nb.jj[k])];
-            const T g = gradDataHigh.data_[at4(gradDataHigh, b, c, i, j)];
-            // dataHigh = m * data + (1 - m) * (n > 0 ? d / n : 0)
-            adjMask += g * (data.data_[at4(data, b, c, i, j)] - (n > 0 ? d / n : T(0)));
-            gradData.data_[at4(gradData, b, c, i, j)] += g * m;
-            if (n > 0) adjN -= g * (1 - m) * d / (n * n);
-            adjFill.data_[at4(adjFill, b, c, i, j)] = n > 0 ? g * (1 - m) / n : T(0);
-        }
-        // maskHigh = m + (n > 0 ? (1 - m) * n / weight : 0)
-        const T gm = gradMaskHigh.data_[at3(gradMaskHigh, b, i, j)];
-        adjMask += gm * (1 - (n / weight));
-        adjN += gm * ((1 - m) / weight);
-        gradMask.data_[at3(gradMask, b, i, j)] += adjMask;
-        adjFill.data_[at4(adjFill, b, C, i, j)] = adjN;
+    constexpr int TW = 32, TH = PULLPUSH_TAIL_BLOCK / TW;
+    extern __shared__ __align__(16) unsigned char sMemory[];
+    auto& sFill = *reinterpret_cast<T (*)[pullpushChunk<T>() + 1][pullpushTileEntries(TW, TH)]>(sMemory);
+    T* sLevels = reinterpret_cast<T*>(sMemory + sizeof(sFill));
+    const int b = blockIdx.x;
+    auto level = [&](int k) { return k == 0 ? finest : ldsLevel<T, true>(sLevels, tail, finest.H, finest.W, C, k); };
+    for (int k = 0; k + 1 < tail.numLevels; ++k) {
+        const auto high = level(k), low = level(k + 1);
+        for (int i = threadIdx.x; i < low.H * low.W; i += PULLPUSH_TAIL_BLOCK) downPixel<false>(high, low, C, b, i / low.W, i % low.W);
+        __syncthreads();
     }
-}
-
-/**
- * Adjoint of PullPushUpKernel, second pass; one thread per low-res pixel (b, ii, jj). Gathers
- * from the up to 4 x 4 high-res pixels that interpolate from it (rows 2ii-1 .. 2ii+2: the two
- * inner ones with weight 3/4, the outer ones with 1/4; columns alike), so no atomics are
- * needed (the reference scatters with atomicAdd, pullpush.cuh:256-273):
- *   gradDataLow_c += maskLow * sum_p w_p adjFill_c(p)
- *   gradMaskLow   += sum_p w_p (adjFill_C(p) + sum_c adjFill_c(p) dataLow_c)
- */
-template <typename T>
-__global__ void __launch_bounds__(256) PullPushAdjointUpGatherKernel(
-    long long numel, const Tensor3Read<T> maskLow, const Tensor4Read<T> dataLow, const Tensor4Read<T> adjFill,
-    Tensor3RW<T> gradMaskLow, Tensor4RW<T> gradDataLow)
-{
-    using namespace pullpush;
-    const int oH = maskLow.sizes_[1], oW = maskLow.sizes_[2], C = dataLow.sizes_[1];
-    const int H = adjFill.sizes_[2], W = adjFill.sizes_[3];
-    for (long long idx = blockIdx.x * static_cast<long long>(blockDim.x) + threadIdx.x; idx < numel;
-         idx += static_cast<long long>(blockDim.x) * gridDim.x)
-    {
-        int b, ii, jj;
-        pixelOf(idx, oH, oW, b, ii, jj);
-        const T ml = maskLow.data_[at3(maskLow, b, ii, jj)];
-        T sumN = 0, adjMaskLow = 0;
-#pragma unroll
-        for (int di = -1; di <= 2; ++di) {
-            const int i = 2 * ii + di;
-            if (i < 0 || i >= H) continue;
-#pragma unroll
-            for (int dj = -1; dj <= 2; ++dj) {
-                const int j = 2 * jj + dj;
-                if (j < 0 || j >= W) continue;
-                const float w = ((di == 0 || di == 1) ? 0.75f : 0.25f) * ((dj == 0 || dj == 1) ? 0.75f : 0.25f);
-                sumN += w * adjFill.data_[at4(adjFill, b, C, i, j)];
-            }
+    for (int k = tail.numLevels - 2; k >= 1; --k) {
+        const auto high = level(k), low = level(k + 1);
+        const int height = (high.H + 1) / 2, width = (high.W + 1) / 2;
+        for (int i = threadIdx.x; i < height * width; i += PULLPUSH_TAIL_BLOCK) upQuad<false>(high, low, C, b, i / width, i % width);
+        __syncthreads();
+    }
+    for (int k = 0; k + 1 < tail.numLevels; ++k) {
+        const auto high = level(k), low = level(k + 1);
+        for (int a0 = 0; a0 < low.H; a0 += TH)
+            for (int e0 = 0; e0 < low.W; e0 += TW) gradientUpTile<false, TW, TH>(high, low, C, b, a0, e0, sFill);
+        __syncthreads();
+    }
+    for (int k = tail.numLevels - 2; k >= 0; --k) {
+        const auto high = level(k), low = level(k + 1);
+        const int height = (high.H + 1) / 2, width = (high.W + 1) / 2;
+        for (int i = threadIdx.x; i < height * width; i += PULLPUSH_TAIL_BLOCK) {
+            if (ACCUMULATE && k == 0) gradientQuad<false, true>(high, low, C, b, i / width, i % width);
+            else gradientQuad<false, false>(high, low, C, b, i / width, i % width);
         }
-        for (int c = 0; c < C; ++c) {
-            T sumD = 0;
-#pragma unroll
-            for (int di = -1; di <= 2; ++di) {
-                const int i = 2 * ii + di;
-                if (i < 0 || i >= H) continue;
-#pragma unroll
-                for (int dj = -1; dj <= 2; ++dj) {
-                    const int j = 2 * jj + dj;
-                    if (j < 0 || j >= W) continue;
-                    const float w = ((di == 0 || di == 1) ? 0.75f : 0.25f) * ((dj == 0 || dj == 1) ? 0.75f : 0.25f);
-                    sumD += w * adjFill.data_[at4(adjFill, b, c, i, j)];
-                }
-            }
-            gradDataLow.data_[at4(gradDataLow, b, c, ii, jj)] += sumD * ml;
-            adjMaskLow += sumD * dataLow.data_[at4(dataLow, b, c, ii, jj)];
-        }
-        gradMaskLow.data_[at3(gradMaskLow, b, ii, jj)] += adjMaskLow + sumN;
+        __syncthreads();
     }
 }
 
@@ -345,7 +725,7 @@ __global__ void __launch_bounds__(256) PullPushAddKernel(long long numel, Tensor
     }
 }
 
-/** dst = src for tensors of any strides (an image of one row or column is its own inpainting). */
+/** dst = src (zero if src has no data) for tensors of any strides (an image of one row or column is its own inpainting). */
 template <typename T, int N>
 __global__ void __launch_bounds__(256) PullPushCopyKernel(long long numel, TensorAccessor<T, N> dst, const TensorAccessor<const T, N> src)
 {
@@ -354,7 +734,7 @@ __global__ void __launch_bounds__(256) PullPushCopyKernel(long long numel, Tenso
     {
         long long od, os;
         pullpush::offsetsOf(idx, dst, src, od, os);
-        dst.data_[od] = src.data_[os];
+        dst.data_[od] = src.data_ ? src.data_[os] : T(0);
     }
 }
 

@@ -573,6 +573,32 @@ int qmlp_utils_pullpush_adjoint(const qmlp_tensor* mask, const qmlp_tensor* data
     QMLP_API_END
 }
 
+int qmlp_utils_pullpush_memory(const qmlp_tensor* data, size_t* pyramid_bytes, size_t* gradient_bytes)
+{
+    QMLP_API_BEGIN
+    Utils::pullpushMemory(wrap(data), *pyramid_bytes, *gradient_bytes);
+    QMLP_API_END
+}
+
+int qmlp_utils_pullpush_forward_in(const qmlp_tensor* mask, const qmlp_tensor* data, const qmlp_tensor* output, void* pyramid, void* stream)
+{
+    QMLP_API_BEGIN
+    Tensor out = wrap(output);
+    Utils::fractionalPullpush(wrap(mask), wrap(data), out, pyramid, static_cast<stream_t>(stream));
+    QMLP_API_END
+}
+
+int qmlp_utils_pullpush_adjoint_in(const qmlp_tensor* mask, const qmlp_tensor* data, const qmlp_tensor* adj_output,
+                                   const qmlp_tensor* adj_mask, const qmlp_tensor* adj_data, int accumulate, void* pyramid,
+                                   int pyramid_ready, void* gradients, void* stream)
+{
+    QMLP_API_BEGIN
+    Tensor adjMask = wrap(adj_mask), adjData = wrap(adj_data);
+    Utils::adjointFractionalPullpush(wrap(mask), wrap(data), wrap(adj_output), adjMask, adjData, accumulate != 0, pyramid,
+                                     pyramid_ready != 0, gradients, static_cast<stream_t>(stream));
+    QMLP_API_END
+}
+
 int qmlp_utils_pullpush_precompile(int precision)
 {
     QMLP_API_BEGIN

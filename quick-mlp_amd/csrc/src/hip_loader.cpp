@@ -101,6 +101,19 @@ int qmlp_hip_free(void* ptr)
     return check(hipFree(ptr), "hipFree");
 }
 
+int qmlp_hip_malloc_async(void** ptr, size_t bytes, qmlp_hip_stream stream)
+{
+    *ptr = nullptr;
+    if (bytes == 0) return 0;
+    return check(hipMallocAsync(ptr, bytes, static_cast<hipStream_t>(stream)), "hipMallocAsync");
+}
+
+int qmlp_hip_free_async(void* ptr, qmlp_hip_stream stream)
+{
+    if (!ptr) return 0;
+    return check(hipFreeAsync(ptr, static_cast<hipStream_t>(stream)), "hipFreeAsync");
+}
+
 int qmlp_hip_memset_async(void* ptr, int value, size_t bytes, qmlp_hip_stream stream)
 {
     // a kernel, not hipMemsetAsync: memset nodes in a captured HIP graph have given wrong

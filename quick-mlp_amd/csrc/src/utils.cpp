@@ -1,12 +1,12 @@
 #include <qmlp/utils.h>
 
 #include <qmlp/errors.h>
+#include <qmlp/fused_network.h>
 #include <qmlp/qmlp.h>
 
 #include "qmlp_hip.h"
 
 #include <algorithm>
-#include <map>
 #include <mutex>
 #include <vector>
 
@@ -21,174 +21,277 @@ const char* scalarName(Tensor::Precision p)
     throw std::runtime_error("fractionalPullpush works on float or double tensors");
 }
 
-const char* const KERNEL_NAMES[] = {"PullPushDownKernel<$T>", "PullPushUpKernel<$T>", "PullPushAdjointUpKernel<$T>",
-                                    "PullPushAdjointUpGatherKernel<$T>", "PullPushAdjointDownKernel<$T, true>",
-                                    "PullPushAdjointDownKernel<$T, false>", "PullPushAddKernel<$T, 3>",
-                                    "PullPushAddKernel<$T, 4>", "PullPushCopyKernel<$T, 3>",
+const char* const KERNEL_NAMES[] = {"PullPushDownKernel<$T>", "PullPushUpKernel<$T>", "PullPushTailKernel<$T>",
+                                    "PullPushGradientUpKernel<$T>", "PullPushGradientKernel<$T, false>",
+                                    "PullPushGradientKernel<$T, true>", "PullPushGradientTailKernel<$T, false>",
+                                    "PullPushGradientTailKernel<$T, true>", "PullPushAddKernel<$T, 4>",
                                     "PullPushCopyKernel<$T, 4>"};
+enum KernelIndex { DOWN, UP, TAIL, GRADIENT_UP, GRADIENT, GRADIENT_ADD, GRADIENT_TAIL, GRADIENT_TAIL_ADD, ADD_4, COPY_4 };
+
+// as in kernels/pullpush.h
+constexpr int TAIL_BLOCK = 512, TILE_W = 32, TILE_H = 8, BLOCK = 256;
+template <typename T>
+constexpr int tailFillBytes()
+{
+    constexpr int TH = TAIL_BLOCK / TILE_W, planes = (sizeof(T) == 4 ? 4 : 2) + 1;
+    return planes * (2 * (TH + 2) * (2 * (TILE_W + 2) + 1)) * static_cast<int>(sizeof(T));
+}
 
 std::string pullpushSource() { return KernelLoader::MainFile("qmlp/kernels/pullpush.h"); }
 
+std::string kernelName(int index, const std::string& scalar)
+{
+    std::string name = KERNEL_NAMES[index];
+    name.replace(name.find("$T"), 2, scalar);
+    return "qmlp::kernel::" + name;
+}
+
 /** The compiled kernels stay loaded for the life of the process, like the reference's static kernels. */
-KernelFunction pullpushKernel(const std::string& name)
+template <typename T>
+KernelFunction& pullpushKernel(KernelIndex index)
 {
     static std::mutex mutex;
-    static std::map<std::string, KernelFunction> kernels;
+    static KernelFunction kernels[sizeof(KERNEL_NAMES) / sizeof(KERNEL_NAMES[0])];
     std::lock_guard<std::mutex> lock(mutex);
-    auto it = kernels.find(name);
-    if (it == kernels.end()) {
-        auto kl = QuickMLP::Instance().kernelLoader();
-        auto fun = kl->getKernel("qmlp::kernel::" + name, pullpushSource(), QuickMLP::Instance().getCompileFlags());
-        it = kernels.emplace(name, fun.value()).first;
-    }
-    return it->second;
+    auto& fun = kernels[index];
+    if (!fun.defined())
+        fun = QuickMLP::Instance().kernelLoader()->getKernel(kernelName(index, sizeof(T) == 4 ? "float" : "double"), pullpushSource(),
+                                                             QuickMLP::Instance().getCompileFlags()).value();
+    return fun;
 }
 
-template <typename T, int N>
-kernel::TensorAccessor<T, N> accessorOf(const Tensor& t)
+/** PullPushView of kernels/pullpush.h */
+template <typename T>
+struct View
 {
-    return t.accessor<kernel::TensorAccessor<T, N>>();
-}
-
-void launch(KernelFunction& fun, long long numel, stream_t stream, std::vector<void*> args)
-{
-    if (numel == 0) return;
-    const int block = 256;
-    const int grid = static_cast<int>(std::min<long long>(divUp<long long>(numel, block), fun.fullGridSize(block, 0)));
-    std::vector<void*> all = {&numel};
-    all.insert(all.end(), args.begin(), args.end());
-    fun.launch(grid, block, 0, stream, all.data());
-}
-
-/** One pyramid level: the down-sampled inputs and the inpainted low-res result. */
+    T* p = nullptr;
+    long long b = 0, c = 0;
+    unsigned y = 0, x = 0;
+};
+/** PullPushLevel of kernels/pullpush.h */
+template <typename T>
 struct Level
 {
-    Tensor maskLowPre, dataLowPre, maskLowPost, dataLowPost;
+    int H, W;
+    View<T> maskPre, dataPre, maskPost, dataPost, maskSum, gradMaskPost, gradDataPost, gradMaskPre, gradDataPre;
+};
+template <typename T>
+View<T> viewOf(const Tensor& t)
+{
+    View<T> v;
+    v.p = static_cast<T*>(const_cast<void*>(t.rawPtr()));
+    const int n = t.ndim();
+    v.b = t.stride(0);
+    v.c = n == 4 ? t.stride(1) : 0;
+    v.y = static_cast<unsigned>(t.stride(n - 2));
+    v.x = static_cast<unsigned>(t.stride(n - 1));
+    CHECK_ERROR(t.stride(n - 2) >= 0 && t.stride(n - 1) >= 0
+                    && (t.size(n - 2) - 1ll) * t.stride(n - 2) + (t.size(n - 1) - 1ll) * t.stride(n - 1) < (1ll << 32),
+                "fractionalPullpush: the entries of an image plane must lie within 2^32 of each other");
+    return v;
+}
+
+bool isCoarsest(int H, int W) { return H <= 1 || W <= 1; }
+
+/** Hands out the image stacks of a workspace one after the other; rows start at even entries, stacks at multiples of 16. */
+template <typename T>
+struct Workspace
+{
+    T* base;
+    size_t entries = 0;
+    View<T> take(int B, int C, int H, int W)
+    {
+        View<T> v;
+        v.p = base ? base + entries : nullptr;
+        v.x = 1;
+        v.y = static_cast<unsigned>(roundUp(W, 2));
+        v.c = static_cast<long long>(H) * v.y;
+        v.b = C * v.c;
+        entries += roundUp(static_cast<size_t>(B) * static_cast<size_t>(v.b), size_t(16));
+        return v;
+    }
 };
 
-template <typename T>
-void forwardRecursion(const Tensor& maskInput, const Tensor& dataInput, Tensor& maskOutput, Tensor& dataOutput,
-                      std::vector<Level>* saved, stream_t stream)
+/** PullPushTail of kernels/pullpush.h */
+struct Tail
 {
-    const int B = dataInput.size(0), C = dataInput.size(1), H = dataInput.size(2), W = dataInput.size(3);
-    const auto dtype = dataInput.precision();
-    if (H <= 1 || W <= 1) {
-        // end of the recursion: nothing coarser to fill from
-        const std::string t = scalarName(dtype);
-        auto copy3 = pullpushKernel("PullPushCopyKernel<" + t + ", 3>");
-        auto copy4 = pullpushKernel("PullPushCopyKernel<" + t + ", 4>");
-        auto dstM = accessorOf<T, 3>(maskOutput);
-        auto srcM = accessorOf<const T, 3>(maskInput);
-        launch(copy3, maskOutput.numel(), stream, {&dstM, &srcM});
-        auto dstD = accessorOf<T, 4>(dataOutput);
-        auto srcD = accessorOf<const T, 4>(dataInput);
-        launch(copy4, dataOutput.numel(), stream, {&dstD, &srcD});
-        return;
-    }
-    const int oH = H / 2, oW = W / 2;
-    const std::string t = scalarName(dtype);
+    int numLevels;
+    int offsets[31];
+};
 
-    Level level;
-    level.maskLowPre = Tensor(dtype, {B, oH, oW});
-    level.dataLowPre = Tensor(dtype, {B, C, oH, oW});
-    {
-        auto fun = pullpushKernel("PullPushDownKernel<" + t + ">");
-        auto mask = accessorOf<const T, 3>(maskInput);
-        auto data = accessorOf<const T, 4>(dataInput);
-        auto maskLow = accessorOf<T, 3>(level.maskLowPre);
-        auto dataLow = accessorOf<T, 4>(level.dataLowPre);
-        launch(fun, static_cast<long long>(B) * oH * oW, stream, {&mask, &data, &maskLow, &dataLow});
+/** LDS bytes of the kernel that takes over the coarse levels below an (H, W) level: with the gradients, which need more. */
+template <typename T>
+size_t tailLdsBytes(int C, int H, int W, bool gradients, Tail* tail = nullptr)
+{
+    size_t entries = 0;
+    int level = 0;
+    while (!isCoarsest(H, W)) {
+        H /= 2;
+        W /= 2;
+        ++level;
+        if (tail) tail->offsets[level] = static_cast<int>(entries);
+        const size_t plane = static_cast<size_t>(H) * roundUp(W, 2);
+        const bool coarsest = isCoarsest(H, W);
+        entries += plane * (coarsest ? 2 + C : 3 + 2 * C);
+        if (gradients) entries += plane * (coarsest ? 1 + C : 2 + 2 * C);
     }
-    level.maskLowPost = Tensor(dtype, {B, oH, oW});
-    level.dataLowPost = Tensor(dtype, {B, C, oH, oW});
-    forwardRecursion<T>(level.maskLowPre, level.dataLowPre, level.maskLowPost, level.dataLowPost, saved, stream);
-    {
-        auto fun = pullpushKernel("PullPushUpKernel<" + t + ">");
-        auto mask = accessorOf<const T, 3>(maskInput);
-        auto data = accessorOf<const T, 4>(dataInput);
-        auto maskLow = accessorOf<const T, 3>(level.maskLowPost);
-        auto dataLow = accessorOf<const T, 4>(level.dataLowPost);
-        auto maskHigh = accessorOf<T, 3>(maskOutput);
-        auto dataHigh = accessorOf<T, 4>(dataOutput);
-        launch(fun, static_cast<long long>(B) * H * W, stream, {&mask, &data, &maskLow, &dataLow, &maskHigh, &dataHigh});
+    if (tail) tail->numLevels = level + 1;
+    return entries * sizeof(T) + (gradients ? tailFillBytes<T>() : 0);
+}
+
+/**
+ * The levels of the pyramid of a (B, C, H, W) image that have kernel launches of their own, finest first, with the views of
+ * the low-res ones in the given workspaces (null: only the sizes are wanted, in 'bytes' and 'gradientBytes'). The levels
+ * below the last one are left to the kernels that keep them in LDS: from there on where all of them fit (1 x 4 float:
+ * from 32 x 32 pixels on), as a step inside such a workgroup takes less than the 3 us of a launch.
+ */
+template <typename T>
+std::vector<Level<T>> layout(int B, int C, int H, int W, void* pyramid, void* gradients, size_t* bytes = nullptr, size_t* gradientBytes = nullptr)
+{
+    std::vector<Level<T>> levels(1);
+    levels[0] = {};
+    levels[0].H = H;
+    levels[0].W = W;
+    Workspace<T> forward{static_cast<T*>(pyramid)}, adjoint{static_cast<T*>(gradients)};
+    const size_t lds = FusedNetwork::MaxSharedMemoryBytes();
+    while (!isCoarsest(H, W) && tailLdsBytes<T>(C, H, W, true) > lds) {
+        H /= 2;
+        W /= 2;
+        Level<T> l = {};
+        l.H = H;
+        l.W = W;
+        l.maskPre = forward.take(B, 1, H, W);
+        l.dataPre = forward.take(B, C, H, W);
+        l.maskSum = forward.take(B, 1, H, W);
+        l.gradMaskPost = adjoint.take(B, 1, H, W);
+        l.gradDataPost = adjoint.take(B, C, H, W);
+        if (isCoarsest(H, W)) {   // its own inpainting: nothing changes from before to after
+            l.maskPost = l.maskPre;
+            l.dataPost = l.dataPre;
+            l.gradMaskPre = l.gradMaskPost;
+            l.gradDataPre = l.gradDataPost;
+        } else {
+            l.maskPost = forward.take(B, 1, H, W);
+            l.dataPost = forward.take(B, C, H, W);
+            l.gradMaskPre = adjoint.take(B, 1, H, W);
+            l.gradDataPre = adjoint.take(B, C, H, W);
+        }
+        levels.push_back(l);
     }
-    // The temporaries of this level are freed when 'level' goes out of scope, which may be
-    // before the kernels have run: keep them until the caller has synchronised.
-    saved->push_back(std::move(level));
+    if (bytes) *bytes = forward.entries * sizeof(T);
+    if (gradientBytes) *gradientBytes = adjoint.entries * sizeof(T);
+    return levels;
+}
+
+/** The levels below the last one with launches of its own, one workgroup per image. */
+template <typename T>
+void launchTail(KernelIndex kernel, int B, int C, Level<T> finest, bool gradients, stream_t stream)
+{
+    if (isCoarsest(finest.H, finest.W)) return;
+    Tail tail = {};
+    const size_t lds = tailLdsBytes<T>(C, finest.H, finest.W, gradients, &tail);
+    void* args[] = {&finest, &C, &tail};
+    pullpushKernel<T>(kernel).launch(static_cast<unsigned>(B), TAIL_BLOCK, static_cast<unsigned>(lds), stream, args);
+}
+
+/** Whether the pixels (y, 2k) and (y, 2k + 1) of all images of a level can be moved as one aligned pair. */
+template <typename T>
+bool movesPairs(const Level<T>& level, bool padded)
+{
+    for (const View<T>* v : {&level.maskPre, &level.dataPre, &level.maskPost, &level.dataPost, &level.gradMaskPost, &level.gradDataPost,
+                             &level.gradMaskPre, &level.gradDataPre})
+        if (v->p && !(v->x == 1 && v->y % 2 == 0 && v->b % 2 == 0 && v->c % 2 == 0 && reinterpret_cast<uintptr_t>(v->p) % (2 * sizeof(T)) == 0))
+            return false;
+    return padded || level.W % 2 == 0;   // the rows of the workspaces end at even entries, the caller's where they end
+}
+
+/** One launch for one level: a workgroup per tile of 32 x 8 items. */
+template <typename T>
+void launchLevel(KernelIndex kernel, int B, int C, int height, int width, const std::vector<Level<T>>& levels, int l, stream_t stream)
+{
+    Level<T> high = levels[l], low = levels[l + 1];
+    int pairs = movesPairs(high, l > 0) ? 1 : 0;
+    const long long grid = static_cast<long long>(B) * divUp(height, TILE_H) * divUp(width, TILE_W);
+    void* args[] = {&high, &low, &C, &pairs};
+    pullpushKernel<T>(kernel).launch(static_cast<unsigned>(grid), BLOCK, 0, stream, args);
+}
+
+/** The pyramid down to the coarsest level and the inpainted levels up to levels[1]; with 'finest' up to levels[0]. */
+template <typename T>
+void runForward(const std::vector<Level<T>>& levels, int B, int C, bool finest, stream_t stream)
+{
+    const int last = static_cast<int>(levels.size()) - 1;
+    for (int l = 0; l < last; ++l) launchLevel(DOWN, B, C, levels[l + 1].H, levels[l + 1].W, levels, l, stream);
+    if (last > 0 || finest) launchTail(TAIL, B, C, levels[last], false, stream);
+    for (int l = last - 1; l >= (finest ? 0 : 1); --l)
+        launchLevel(UP, B, C, divUp(levels[l].H, 2), divUp(levels[l].W, 2), levels, l, stream);
 }
 
 template <typename T>
-void adjointRecursion(const Tensor& maskInput, const Tensor& dataInput, const Tensor& gradMaskOutput,
-                      const Tensor& gradDataOutput, Tensor& gradMaskInput, Tensor& gradDataInput,
-                      std::vector<Level>& saved, std::vector<Tensor>& keepAlive, stream_t stream)
+void runAdjoint(const std::vector<Level<T>>& levels, int B, int C, bool accumulate, stream_t stream)
 {
-    const int B = dataInput.size(0), C = dataInput.size(1), H = dataInput.size(2), W = dataInput.size(3);
-    const auto dtype = dataInput.precision();
-    const std::string t = scalarName(dtype);
-    if (H <= 1 || W <= 1) {
-        auto add3 = pullpushKernel("PullPushAddKernel<" + t + ", 3>");
-        auto add4 = pullpushKernel("PullPushAddKernel<" + t + ", 4>");
-        auto dstM = accessorOf<T, 3>(gradMaskInput);
-        auto srcM = accessorOf<const T, 3>(gradMaskOutput);
-        launch(add3, gradMaskInput.numel(), stream, {&dstM, &srcM});
-        auto dstD = accessorOf<T, 4>(gradDataInput);
-        auto srcD = accessorOf<const T, 4>(gradDataOutput);
-        launch(add4, gradDataInput.numel(), stream, {&dstD, &srcD});
+    const int last = static_cast<int>(levels.size()) - 1;
+    for (int l = 0; l < last; ++l) launchLevel(GRADIENT_UP, B, C, levels[l + 1].H, levels[l + 1].W, levels, l, stream);
+    launchTail(last == 0 && accumulate ? GRADIENT_TAIL_ADD : GRADIENT_TAIL, B, C, levels[last], true, stream);
+    for (int l = last - 1; l >= 0; --l)
+        launchLevel(l == 0 && accumulate ? GRADIENT_ADD : GRADIENT, B, C, divUp(levels[l].H, 2), divUp(levels[l].W, 2), levels, l, stream);
+}
+
+/** dst = src or dst += src for image stacks of any strides; without src: zero. */
+template <typename T>
+void elementwise(KernelIndex kernel, const Tensor& dst, const Tensor* src, stream_t stream)
+{
+    auto accessor = [](const Tensor& t) {   // a mask is an image of one channel
+        kernel::TensorAccessor<T, 4> a;
+        const bool mask = t.ndim() == 3;
+        a.data_ = static_cast<T*>(const_cast<void*>(t.rawPtr()));
+        for (int d = 0; d < 4; ++d) {
+            a.sizes_[d] = mask && d == 1 ? 1 : t.size(mask && d > 1 ? d - 1 : d);
+            a.strides_[d] = mask && d == 1 ? 0 : t.stride(mask && d > 1 ? d - 1 : d);
+        }
+        return a;
+    };
+    long long numel = dst.numel();
+    auto d = accessor(dst);
+    kernel::TensorAccessor<T, 4> s = {};
+    if (src) s = accessor(*src);
+    void* args[] = {&numel, &d, &s};
+    pullpushKernel<T>(kernel).launch(static_cast<unsigned>(std::min<long long>(divUp<long long>(numel, BLOCK), 1 << 16)), BLOCK, 0, stream, args);
+}
+
+template <typename T>
+void forward(const Tensor& mask, const Tensor& data, Tensor& output, void* pyramid, stream_t stream)
+{
+    const int B = data.size(0), C = data.size(1), H = data.size(2), W = data.size(3);
+    if (isCoarsest(H, W)) {   // nothing coarser to fill from
+        elementwise<T>(COPY_4, output, &data, stream);
         return;
     }
-    const int oH = H / 2, oW = W / 2;
-    // the levels were saved coarsest first: the finest one is at the back
-    Level level = std::move(saved.back());
-    saved.pop_back();
+    auto levels = layout<T>(B, C, H, W, pyramid, nullptr);
+    levels[0].maskPre = viewOf<T>(mask);
+    levels[0].dataPre = viewOf<T>(data);
+    levels[0].dataPost = viewOf<T>(output);
+    runForward(levels, B, C, true, stream);
+}
 
-    Tensor gradMaskLowPost(dtype, {B, oH, oW}), gradDataLowPost(dtype, {B, C, oH, oW});
-    gradMaskLowPost.zeroAsync_(stream);
-    gradDataLowPost.zeroAsync_(stream);
-    // what every high-res pixel passes down: C channel terms and one mask term
-    Tensor adjFill(dtype, {B, C + 1, H, W});
-    {
-        auto fun = pullpushKernel("PullPushAdjointUpKernel<" + t + ">");
-        auto mask = accessorOf<const T, 3>(maskInput);
-        auto data = accessorOf<const T, 4>(dataInput);
-        auto maskLow = accessorOf<const T, 3>(level.maskLowPost);
-        auto dataLow = accessorOf<const T, 4>(level.dataLowPost);
-        auto gMaskHigh = accessorOf<const T, 3>(gradMaskOutput);
-        auto gDataHigh = accessorOf<const T, 4>(gradDataOutput);
-        auto gMask = accessorOf<T, 3>(gradMaskInput);
-        auto gData = accessorOf<T, 4>(gradDataInput);
-        auto fill = accessorOf<T, 4>(adjFill);
-        launch(fun, static_cast<long long>(B) * H * W, stream,
-               {&mask, &data, &maskLow, &dataLow, &gMaskHigh, &gDataHigh, &gMask, &gData, &fill});
+template <typename T>
+void adjoint(const Tensor& mask, const Tensor& data, const Tensor& adjOutput, Tensor& adjMask, Tensor& adjData, bool accumulate,
+             void* pyramid, bool pyramidReady, void* gradients, stream_t stream)
+{
+    const int B = data.size(0), C = data.size(1), H = data.size(2), W = data.size(3);
+    if (isCoarsest(H, W)) {
+        elementwise<T>(accumulate ? ADD_4 : COPY_4, adjData, &adjOutput, stream);
+        if (!accumulate) elementwise<T>(COPY_4, adjMask, nullptr, stream);   // the mask of a row or a column has no influence
+        return;
     }
-    {
-        auto fun = pullpushKernel("PullPushAdjointUpGatherKernel<" + t + ">");
-        auto maskLow = accessorOf<const T, 3>(level.maskLowPost);
-        auto dataLow = accessorOf<const T, 4>(level.dataLowPost);
-        auto fill = accessorOf<const T, 4>(adjFill);
-        auto gMaskLow = accessorOf<T, 3>(gradMaskLowPost);
-        auto gDataLow = accessorOf<T, 4>(gradDataLowPost);
-        launch(fun, static_cast<long long>(B) * oH * oW, stream, {&maskLow, &dataLow, &fill, &gMaskLow, &gDataLow});
-    }
-    Tensor gradMaskLowPre(dtype, {B, oH, oW}), gradDataLowPre(dtype, {B, C, oH, oW});
-    gradMaskLowPre.zeroAsync_(stream);
-    gradDataLowPre.zeroAsync_(stream);
-    adjointRecursion<T>(level.maskLowPre, level.dataLowPre, gradMaskLowPost, gradDataLowPost, gradMaskLowPre,
-                        gradDataLowPre, saved, keepAlive, stream);
-    {
-        // windows of neighbouring low-res pixels overlap when a size is odd
-        const bool overlap = (H % 2 != 0) || (W % 2 != 0);
-        auto fun = pullpushKernel("PullPushAdjointDownKernel<" + t + (overlap ? ", true>" : ", false>"));
-        auto mask = accessorOf<const T, 3>(maskInput);
-        auto data = accessorOf<const T, 4>(dataInput);
-        auto gMaskLow = accessorOf<const T, 3>(gradMaskLowPre);
-        auto gDataLow = accessorOf<const T, 4>(gradDataLowPre);
-        auto gMask = accessorOf<T, 3>(gradMaskInput);
-        auto gData = accessorOf<T, 4>(gradDataInput);
-        launch(fun, static_cast<long long>(B) * oH * oW, stream, {&mask, &data, &gMaskLow, &gDataLow, &gMask, &gData});
-    }
-    for (Tensor* x : {&level.maskLowPre, &level.dataLowPre, &level.maskLowPost, &level.dataLowPost, &gradMaskLowPost,
-                      &gradDataLowPost, &gradMaskLowPre, &gradDataLowPre, &adjFill})
-        keepAlive.push_back(std::move(*x));
+    auto levels = layout<T>(B, C, H, W, pyramid, gradients);
+    levels[0].maskPre = viewOf<T>(mask);
+    levels[0].dataPre = viewOf<T>(data);
+    if (!pyramidReady) runForward(levels, B, C, false, stream);
+    levels[0].gradDataPost = viewOf<T>(adjOutput);
+    levels[0].gradMaskPre = viewOf<T>(adjMask);
+    levels[0].gradDataPre = viewOf<T>(adjData);
+    runAdjoint(levels, B, C, accumulate, stream);
 }
 
 void checkShapes(const Tensor& mask, const Tensor& data)
@@ -211,10 +314,16 @@ void checkLike(const Tensor& x, const Tensor& like, const char* what)
     CHECK_DTYPE(x, like.precision());
 }
 
-void synchronize(stream_t stream)
+/** Device memory of one call, in the order of the stream. */
+struct CallMemory
 {
-    QMLP_HIP_CALL(qmlp_hip_stream_synchronize(stream));
-}
+    void* p = nullptr;
+    stream_t stream;
+    CallMemory(size_t bytes, stream_t s) : stream(s) { if (bytes > 0) QMLP_HIP_CALL(qmlp_hip_malloc_async(&p, bytes, s)); }
+    ~CallMemory() { if (p) qmlp_hip_free_async(p, stream); }
+    CallMemory(const CallMemory&) = delete;
+    CallMemory& operator=(const CallMemory&) = delete;
+};
 
 } // namespace
 
@@ -223,26 +332,37 @@ void Utils::precompile(Tensor::Precision precision)
     const std::string t = scalarName(precision);
     auto kl = QuickMLP::Instance().kernelLoader();
     const int flags = QuickMLP::Instance().getCompileFlags() | KernelLoader::CompileOnly;
-    for (const char* pattern : KERNEL_NAMES) {
-        std::string name = pattern;
-        name.replace(name.find("$T"), 2, t);
-        kl->getKernel("qmlp::kernel::" + name, pullpushSource(), flags);
-    }
+    for (size_t i = 0; i < sizeof(KERNEL_NAMES) / sizeof(KERNEL_NAMES[0]); ++i)
+        kl->getKernel(kernelName(static_cast<int>(i), t), pullpushSource(), flags);
+}
+
+void Utils::pullpushMemory(const Tensor& data, size_t& pyramidBytes, size_t& gradientBytes)
+{
+    CHECK_DIM(data, 4);
+    pyramidBytes = gradientBytes = 0;
+    if (data.numel() == 0) return;
+    const int B = data.size(0), C = data.size(1), H = data.size(2), W = data.size(3);
+    if (data.precision() == Tensor::FLOAT) layout<float>(B, C, H, W, nullptr, nullptr, &pyramidBytes, &gradientBytes);
+    else layout<double>(B, C, H, W, nullptr, nullptr, &pyramidBytes, &gradientBytes);
 }
 
 void Utils::fractionalPullpush(const Tensor& mask, const Tensor& data, Tensor& output, stream_t stream)
 {
     checkShapes(mask, data);
     checkLike(output, data, "output");
+    size_t pyramidBytes = 0, gradientBytes = 0;
+    pullpushMemory(data, pyramidBytes, gradientBytes);
+    CallMemory pyramid(pyramidBytes, stream);
+    fractionalPullpush(mask, data, output, pyramid.p, stream);
+}
+
+void Utils::fractionalPullpush(const Tensor& mask, const Tensor& data, Tensor& output, void* pyramid, stream_t stream)
+{
+    checkShapes(mask, data);
+    checkLike(output, data, "output");
     if (data.numel() == 0) return;
-    std::vector<Level> levels;
-    Tensor maskOutput(data.precision(), mask.sizes());
-    if (data.precision() == Tensor::FLOAT)
-        forwardRecursion<float>(mask, data, maskOutput, output, &levels, stream);
-    else
-        forwardRecursion<double>(mask, data, maskOutput, output, &levels, stream);
-    // the pyramid is temporary device memory of this call: wait before it is released
-    synchronize(stream);
+    if (data.precision() == Tensor::FLOAT) forward<float>(mask, data, output, pyramid, stream);
+    else forward<double>(mask, data, output, pyramid, stream);
 }
 
 void Utils::adjointFractionalPullpush(const Tensor& mask, const Tensor& data, const Tensor& adjOutput, Tensor& adjMask,
@@ -252,20 +372,24 @@ void Utils::adjointFractionalPullpush(const Tensor& mask, const Tensor& data, co
     checkLike(adjOutput, data, "adjOutput");
     checkLike(adjData, data, "adjData");
     checkLike(adjMask, mask, "adjMask");
+    size_t pyramidBytes = 0, gradientBytes = 0;
+    pullpushMemory(data, pyramidBytes, gradientBytes);
+    CallMemory pyramid(pyramidBytes, stream), gradients(gradientBytes, stream);
+    adjointFractionalPullpush(mask, data, adjOutput, adjMask, adjData, true, pyramid.p, false, gradients.p, stream);
+}
+
+void Utils::adjointFractionalPullpush(const Tensor& mask, const Tensor& data, const Tensor& adjOutput, Tensor& adjMask, Tensor& adjData,
+                                      bool accumulate, void* pyramid, bool pyramidReady, void* gradients, stream_t stream)
+{
+    checkShapes(mask, data);
+    checkLike(adjOutput, data, "adjOutput");
+    checkLike(adjData, data, "adjData");
+    checkLike(adjMask, mask, "adjMask");
     if (data.numel() == 0) return;
-    const auto dtype = data.precision();
-    std::vector<Level> levels;
-    std::vector<Tensor> keepAlive;
-    Tensor maskOutput(dtype, mask.sizes()), output(dtype, data.sizes()), gradMaskOutput(dtype, mask.sizes());
-    gradMaskOutput.zeroAsync_(stream);   // only the data output has a gradient
-    if (dtype == Tensor::FLOAT) {
-        forwardRecursion<float>(mask, data, maskOutput, output, &levels, stream);
-        adjointRecursion<float>(mask, data, gradMaskOutput, adjOutput, adjMask, adjData, levels, keepAlive, stream);
-    } else {
-        forwardRecursion<double>(mask, data, maskOutput, output, &levels, stream);
-        adjointRecursion<double>(mask, data, gradMaskOutput, adjOutput, adjMask, adjData, levels, keepAlive, stream);
-    }
-    synchronize(stream);
+    if (data.precision() == Tensor::FLOAT)
+        adjoint<float>(mask, data, adjOutput, adjMask, adjData, accumulate, pyramid, pyramidReady, gradients, stream);
+    else
+        adjoint<double>(mask, data, adjOutput, adjMask, adjData, accumulate, pyramid, pyramidReady, gradients, stream);
 }
 
 QUICKMLP_NAMESPACE_END

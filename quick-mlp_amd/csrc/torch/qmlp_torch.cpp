@@ -516,21 +516,42 @@ torch::Tensor NetworkBindings::forward(const NetworkBindings_ptr& self, const to
 // ------------------------------------------------------------------------------------- utils
 struct UtilsBindings : torch::CustomClassHolder
 {
-    static torch::Tensor pullpushForward(const torch::Tensor& mask, const torch::Tensor& data)
+    // device memory of the image pyramid (first) and of its gradients (second) for images like data
+    static torch::Tensor memory(const torch::Tensor& data, const qmlp_tensor& d, bool gradients)
+    {
+        size_t bytes[2] = {0, 0};
+        QMLP_CHECK(qmlp_utils_pullpush_memory(&d, &bytes[0], &bytes[1]));
+        return torch::empty({static_cast<int64_t>(std::max<size_t>(bytes[gradients ? 1 : 0], 16))}, data.options().dtype(torch::kUInt8));
+    }
+    static std::tuple<torch::Tensor, torch::Tensor> forwardKeepingPyramid(const torch::Tensor& mask, const torch::Tensor& data)
     {
         auto output = torch::empty_like(data);
         const qmlp_tensor m = wrap(mask), d = wrap(data), o = wrap(output);
-        QMLP_CHECK(qmlp_utils_pullpush_forward(&m, &d, &o, currentStream()));
-        return output;
+        auto pyramid = memory(data, d, false);
+        QMLP_CHECK(qmlp_utils_pullpush_forward_in(&m, &d, &o, pyramid.data_ptr(), currentStream()));
+        return {output, pyramid};
+    }
+    static torch::Tensor pullpushForward(const torch::Tensor& mask, const torch::Tensor& data)
+    {
+        return std::get<0>(forwardKeepingPyramid(mask, data));
+    }
+    static std::tuple<torch::Tensor, torch::Tensor> adjointFrom(const torch::Tensor& mask, const torch::Tensor& data,
+                                                                const torch::Tensor& adjOutput, torch::Tensor pyramid)
+    {
+        auto gradMask = torch::empty_like(mask);
+        auto gradData = torch::empty_like(data);
+        const qmlp_tensor m = wrap(mask), d = wrap(data), a = wrap(adjOutput), gm = wrap(gradMask), gd = wrap(gradData);
+        const bool ready = pyramid.defined();
+        if (!ready) pyramid = memory(data, d, false);
+        auto gradients = memory(data, d, true);
+        QMLP_CHECK(qmlp_utils_pullpush_adjoint_in(&m, &d, &a, &gm, &gd, 0, pyramid.data_ptr(), ready ? 1 : 0, gradients.data_ptr(),
+                                                  currentStream()));
+        return {gradMask, gradData};
     }
     static std::tuple<torch::Tensor, torch::Tensor> pullpushAdjoint(const torch::Tensor& mask, const torch::Tensor& data,
                                                                     const torch::Tensor& adjOutput)
     {
-        auto gradMask = torch::zeros_like(mask);
-        auto gradData = torch::zeros_like(data);
-        const qmlp_tensor m = wrap(mask), d = wrap(data), a = wrap(adjOutput), gm = wrap(gradMask), gd = wrap(gradData);
-        QMLP_CHECK(qmlp_utils_pullpush_adjoint(&m, &d, &a, &gm, &gd, currentStream()));
-        return {gradMask, gradData};
+        return adjointFrom(mask, data, adjOutput, {});
     }
     static torch::Tensor pullpush(const torch::Tensor& mask, const torch::Tensor& data);
 };
@@ -539,13 +560,14 @@ struct PushPullFunction : torch::autograd::Function<PushPullFunction>
 {
     static torch::Tensor forward(torch::autograd::AutogradContext* ctx, const torch::Tensor& mask, const torch::Tensor& data)
     {
-        ctx->save_for_backward({mask, data});
-        return UtilsBindings::pullpushForward(mask, data);
+        auto [output, pyramid] = UtilsBindings::forwardKeepingPyramid(mask, data);
+        ctx->save_for_backward({mask, data, pyramid});
+        return output;
     }
     static torch::autograd::tensor_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::tensor_list gradOutputs)
     {
         const auto saved = ctx->get_saved_variables();
-        auto grads = UtilsBindings::pullpushAdjoint(saved[0], saved[1], gradOutputs[0].contiguous());
+        auto grads = UtilsBindings::adjointFrom(saved[0], saved[1], gradOutputs[0], saved[2]);
         return {std::get<0>(grads), std::get<1>(grads)};
     }
 };

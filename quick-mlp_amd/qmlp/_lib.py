@@ -107,6 +107,9 @@ _SIGNATURES = {
     "qmlp_activation_precompile": [_vp],
     "qmlp_utils_pullpush_forward": [_TD, _TD, _TD, _vp],
     "qmlp_utils_pullpush_adjoint": [_TD, _TD, _TD, _TD, _TD, _vp],
+    "qmlp_utils_pullpush_memory": [_TD, _P(ctypes.c_size_t), _P(ctypes.c_size_t)],
+    "qmlp_utils_pullpush_forward_in": [_TD, _TD, _TD, _vp, _vp],
+    "qmlp_utils_pullpush_adjoint_in": [_TD, _TD, _TD, _TD, _TD, _ci, _vp, _ci, _vp, _vp],
     "qmlp_utils_pullpush_precompile": [_ci],
 }
 for _name, _args in _SIGNATURES.items():

@@ -191,3 +191,48 @@ def test_errors():
     # empty batch: nothing to do
     out = pullpush(torch.zeros((0, 4, 4), device="cuda"), torch.zeros((0, 2, 4, 4), device="cuda"))
     assert out.shape == (0, 2, 4, 4)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("shape", [(1, 1, 129, 130), (2, 4, 33, 34), (1, 4, 65, 64), (2, 5, 66, 257), (1, 15, 40, 31), (1, 2, 3, 700),
+                                   (1, 9, 96, 96)])
+def test_levels_with_launches_of_their_own_and_levels_in_lds(shape, dtype):
+    """Around the size from which the coarse levels run inside one workgroup (it depends on channels and type), even and
+    odd sizes at every level, more channels than are in flight together; the adjoint from the pyramid that the forward
+    pass kept, from one of its own, and added to what is there."""
+    mask, data, adj = make_case(sum(shape) + 2, *shape, dtype)
+    print("pullpush levels", shape, dtype, flush=True)
+    m64, d64, a64 = (x.astype(np.float64) for x in (mask, data, adj))
+    tm, td, ta = gpu(mask, dtype).requires_grad_(True), gpu(data, dtype).requires_grad_(True), gpu(adj, dtype)
+    out = pullpush(tm, td)
+    np.testing.assert_allclose(out.detach().cpu().numpy().astype(np.float64), ppo.pullpush(m64, d64), **FWD_TOL[dtype])
+    gm, gd = torch.autograd.grad(out, [tm, td], ta)
+    wm, wd = ppo.pullpush_adjoint(m64, d64, a64)
+    np.testing.assert_allclose(gd.cpu().numpy().astype(np.float64), wd, **ADJ_TOL[dtype])
+    np.testing.assert_allclose(gm.cpu().numpy().astype(np.float64), wm, **ADJ_TOL[dtype])
+    gm2, gd2 = qpp.pullpush_backward(tm.detach(), td.detach(), ta)
+    assert torch.equal(gm, gm2) and torch.equal(gd, gd2)
+    lib = qpp.lib
+    gm3, gd3 = torch.ones_like(gm), torch.full_like(gd, -2.0)
+    qpp.check(lib.qmlp_utils_pullpush_adjoint(qpp.desc(tm), qpp.desc(td), qpp.desc(ta), qpp.desc(gm3), qpp.desc(gd3),
+                                              qpp.current_stream(td.device)))
+    torch.testing.assert_close(gm3 - 1, gm, **ADJ_TOL[dtype])
+    torch.testing.assert_close(gd3 + 2, gd, **ADJ_TOL[dtype])
+
+
+def test_rows_with_room_behind_an_odd_width():
+    """An odd width inside rows of even length: what lies behind the row belongs to the caller and stays untouched."""
+    rng = np.random.default_rng(8)
+    print("pullpush odd width in even rows", flush=True)
+    big = torch.from_numpy(rng.uniform(0.1, 1, (4, 1, 3, 70, 102))).cuda()
+    m, d, a = big[0, :, 0, :, :101], big[1, :, :, :, :101], big[2, :, :, :, :101]
+    gd = torch.full((1, 3, 70, 102), 7.0, dtype=torch.float64, device="cuda")
+    gm = torch.full((1, 70, 102), 7.0, dtype=torch.float64, device="cuda")
+    view_d, view_m = gd[:, :, :, :101], gm[:, :, :101]
+    view_d.zero_(), view_m.zero_()
+    qpp.check(qpp.lib.qmlp_utils_pullpush_adjoint(qpp.desc(m), qpp.desc(d), qpp.desc(a), qpp.desc(view_m), qpp.desc(view_d),
+                                                  qpp.current_stream(d.device)))
+    wm, wd = ppo.pullpush_adjoint(m.cpu().numpy(), d.cpu().numpy(), a.cpu().numpy())
+    np.testing.assert_allclose(view_d.cpu().numpy(), wd, **ADJ_TOL[torch.float64])
+    np.testing.assert_allclose(view_m.cpu().numpy(), wm, **ADJ_TOL[torch.float64])
+    assert (gd[..., 101] == 7).all() and (gm[..., 101] == 7).all()
