@@ -7,11 +7,11 @@ device memory, the current stream and autograd bookkeeping here.
 """
 import ctypes
 import json
-import threading
 
 import torch
 
 from . import _lib
+from . import _native   # the per-batch calls in C++; like libqmlp.so there is no fallback
 from ._lib import (GRADIENTS_INPUT, GRADIENTS_INPUT_ENCODINGS, GRADIENTS_NETWORK_WEIGHTS,
                    QMLP_GRADIENTS, QMLP_INFERENCE, check, current_stream, desc, lib)
 
@@ -200,9 +200,10 @@ class Encoding:
 
     def set_parameter(self, tensor, gradients=False):
         if not gradients:
-            # binding the same memory again changes nothing: skipped, this sits on every call of a network
+            # binding the same memory again changes nothing: skipped, unless the encoding belongs to a network,
+            # whose own calls bind it as well
             key = None if tensor is None else (tensor.data_ptr(), tensor.numel(), tensor.dtype)
-            if key is not None and key == getattr(self, "_bound_inference", None):
+            if key is not None and not self._borrowed and key == getattr(self, "_bound_inference", None):
                 return
             self._bound_inference = key
         check(lib.qmlp_encoding_set_parameter(self._handle, desc(tensor),
@@ -299,79 +300,17 @@ class Encoding:
 
 
 # ---------------------------------------------------------------------------- network
-class _NetworkFunction(torch.autograd.Function):
-    """Differentiable fused forward (bind_network.cpp:189-319)."""
-
-    @staticmethod
-    def forward(ctx, net, flags, input, network_parameters, *encoding_parameters):
-        ctx.net = net
-        ctx.flags = flags
-        ctx.param_dtype = network_parameters.dtype
-        np16 = network_parameters if network_parameters.dtype == torch.float16 else network_parameters.to(torch.float16)
-        nbytes = net.forward_memory(input.shape[0], flags)
-        tmp_forward = torch.empty((max(nbytes, 16),), dtype=torch.uint8, device=input.device)
-        output = _create_output(input, net.channels_out())
-        with net._mutex:
-            net._set_network_parameters(np16, encoding_parameters)
-            check(lib.qmlp_network_forward(net._handle, desc(input), desc(output),
-                                           ctypes.c_void_p(tmp_forward.data_ptr()), current_stream(input.device)))
-        ctx.save_for_backward(input, np16, tmp_forward, *encoding_parameters)
-        return output
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        net, flags = ctx.net, ctx.flags
-        input, np16, tmp_forward = ctx.saved_tensors[:3]
-        encoding_parameters = ctx.saved_tensors[3:]
-        grad_output = grad_output.contiguous()
-        adj_input = torch.zeros_like(input) if flags & GRADIENTS_INPUT else None
-        adj_network = None
-        adj_encodings = [None] * len(encoding_parameters)
-        with net._mutex:
-            net._set_network_parameters(np16, encoding_parameters)
-            if flags & GRADIENTS_NETWORK_WEIGHTS:
-                adj_network = torch.zeros(np16.shape, dtype=torch.float32, device=np16.device)
-                check(lib.qmlp_network_set_parameter(net._handle, desc(adj_network), QMLP_GRADIENTS))
-            if flags & GRADIENTS_INPUT_ENCODINGS:
-                for i, p in enumerate(encoding_parameters):
-                    enc = net.encoding(i)
-                    # the kernel adds the gradients of every encoding with parameters: a frozen one
-                    # gets a zero tensor as well, which is dropped below (bind_network.cpp:277-290)
-                    if enc.has_parameters():
-                        adj_encodings[i] = torch.zeros(p.shape, dtype=enc.parameter_dtype(True), device=p.device)
-                        enc.set_parameter(adj_encodings[i], gradients=True)
-            nbytes = net.adjoint_memory(input.shape[0], flags)
-            tmp_adjoint = torch.empty((max(nbytes, 16),), dtype=torch.uint8, device=input.device)
-            check(lib.qmlp_network_adjoint(net._handle, desc(input), desc(grad_output), flags, desc(adj_input),
-                                           ctypes.c_void_p(tmp_forward.data_ptr()),
-                                           ctypes.c_void_p(tmp_adjoint.data_ptr()), current_stream(input.device)))
-            # do not leave dangling gradient bindings behind
-            check(lib.qmlp_network_set_parameter(net._handle, None, QMLP_GRADIENTS))
-            for i, g in enumerate(adj_encodings):
-                if g is not None:
-                    net.encoding(i).set_parameter(None, gradients=True)
-        if adj_network is not None:
-            adj_network = adj_network.to(ctx.param_dtype)
-        adj_encodings = [g.to(p.dtype) if g is not None and ctx.needs_input_grad[4 + i] else None
-                         for i, (g, p) in enumerate(zip(adj_encodings, encoding_parameters))]
-        return (None, None, adj_input, adj_network, *adj_encodings)
-
-
 class Network:
     """The fused network of a JSON configuration (bind_network.h:16-95)."""
 
     def __init__(self, cfg, parent="."):
         self._cfg = cfg
         self._parent = parent
-        self._mutex = threading.Lock()
         self._handle = ctypes.c_void_p()
         check(lib.qmlp_network_create(cfg.encode(), parent.encode(), ctypes.byref(self._handle)))
+        self._native = _native.Network(self._handle.value)   # owns the handle, together with the autograd graphs of its calls
+        self._mutex = self._native    # (one call of the native network at a time)
         self._encodings = {}
-
-    def __del__(self):
-        if getattr(self, "_handle", None):
-            lib.qmlp_network_destroy(self._handle)
-            self._handle = None
 
     def cfg(self):
         return self._cfg
@@ -431,7 +370,6 @@ class Network:
         """Default (torch.nn.Linear style) initialization of the fp16 tensor 'dst'."""
         with self._mutex:
             check(lib.qmlp_network_set_parameter(self._handle, desc(dst), QMLP_INFERENCE))
-            self._bound_inference = (dst.data_ptr(), dst.numel(), dst.dtype)
             seed = int(torch.randint(2 ** 31 - 1, (1,)).item())
             check(lib.qmlp_network_initialize_inference_parameters(self._handle, seed))
 
@@ -474,26 +412,10 @@ class Network:
         return _lib.get_string(lib.qmlp_network_generated_source, self._handle, kind.encode(), int(adjoint_flags))
 
     def _set_network_parameters(self, network_parameters, encoding_parameters):
-        if network_parameters is not None:
-            key = (network_parameters.data_ptr(), network_parameters.numel(), network_parameters.dtype)
-            if key != getattr(self, "_bound_inference", None):
-                check(lib.qmlp_network_set_parameter(self._handle, desc(network_parameters), QMLP_INFERENCE))
-                self._bound_inference = key
-        m = min(len(encoding_parameters), self.num_encodings())
-        for i in range(m):
-            p = encoding_parameters[i]
-            enc = self.encoding(i)
-            if p is not None and enc.has_parameters():
-                enc.set_parameter(p, gradients=False)
+        self._native.bind(network_parameters, list(encoding_parameters))
 
     def inference(self, input, network_parameters, encoding_parameters=()):
-        _device_of(input)
-        output = _create_output(input, self.channels_out())
-        np16 = network_parameters if network_parameters.dtype == torch.float16 else network_parameters.to(torch.float16)
-        with self._mutex:
-            self._set_network_parameters(np16, list(encoding_parameters))
-            check(lib.qmlp_network_inference(self._handle, desc(input), desc(output), current_stream(input.device)))
-        return output
+        return self._native.inference(input, network_parameters, list(encoding_parameters))
 
     def inference_noalloc(self, input, output, network_parameters, encoding_parameters=()):
         """inference() into a tensor of the caller through the entry point of the C ABI that
@@ -561,25 +483,7 @@ class Network:
 
     def forward(self, input, network_parameters, encoding_parameters=()):
         """Differentiable forward pass; gradients flow to every argument that requires them."""
-        encoding_parameters = list(encoding_parameters)
-        flags = 0
-        if input.requires_grad:
-            flags |= GRADIENTS_INPUT
-        if network_parameters is not None and network_parameters.requires_grad:
-            flags |= GRADIENTS_NETWORK_WEIGHTS
-        for i, t in enumerate(encoding_parameters):
-            if t is not None and t.requires_grad and i < self.num_encodings() and self.encoding(i).has_parameters():
-                flags |= GRADIENTS_INPUT_ENCODINGS
-        if flags == 0 or not torch.is_grad_enabled():
-            return self.inference(input, network_parameters, encoding_parameters)
-        # encodings without parameters get a placeholder so that positions line up
-        filled = []
-        for i in range(self.num_encodings()):
-            p = encoding_parameters[i] if i < len(encoding_parameters) else None
-            if p is None or not self.encoding(i).has_parameters():
-                p = torch.zeros((1,), device=input.device)
-            filled.append(p)
-        return _NetworkFunction.apply(self, flags, input, network_parameters, *filled)
+        return self._native.forward(input, network_parameters, list(encoding_parameters))
 
     def __getstate__(self):
         return (self._cfg, self._parent)

@@ -122,7 +122,14 @@ class FusedNetwork(torch.nn.Module):
         if self.weights.requires_grad and self.weights.dtype == torch.float16 and torch.is_grad_enabled():
             warnings.warn("Training a network with 16-bit master weights: the gradient tensor is 16-bit as well, "
                           "which most optimizers cannot handle. Pass weight_dtype=torch.float32 to the constructor.")
-        return self._network.forward(x, self.weights, list(self.encoding_parameters))
+        if self._scriptable:
+            return self._network.forward(x, self.weights, list(self.encoding_parameters))
+        encodings = self.encoding_parameters
+        # (from the list's own dict: its iterator looks every parameter up by name again)
+        tables = list(encodings._parameters.values())
+        if len(tables) != self._num_encodings:
+            tables = list(encodings)
+        return self._network._native.forward(x, self.weights, tables)
 
     def __getstate__(self):
         state = super().__getstate__() if hasattr(super(), "__getstate__") else self.__dict__.copy()
