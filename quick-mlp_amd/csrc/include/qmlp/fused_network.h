@@ -106,6 +106,12 @@ public:
         // registers of a wavefront), in networks whose weights all stay in LDS; 0: never; >0: up to 32 tiles.
         int fusedWeightUpdate = -1;
 
+        // Backward kernel whose workgroups run the layers again and share the gradient tiles of all layers between their
+        // wavefronts (kernels/network_backward_cooperative.h). <0 (default): where the network allows it, for batches of
+        // COOPERATIVE_MIN_BATCH points or more, of networks that would need weight-update kernels otherwise for every
+        // batch; 0: never; >0: for every batch.
+        int cooperativeBackward = -1;
+
         // Accepted for compatibility; the LDS layouts of this implementation are
         // bank-conflict free for 64 lanes by construction and need no skew.
         bool skewSharedMemory = false;
@@ -250,8 +256,36 @@ private:
         bool fusedWeightUpdate = false;   // any of them
         bool outputOrder = false;         // the kernel takes the order of a sorted batch for its rows of dL/dy
     };
-    // [adjoint flags][grid gradients by slices instead of atomics][the layers run again instead of reading their intermediates]
-    std::optional<AdjointKernel> backwardKernel_[ADJOINT_MODE_MAX_COMBINATIONS][2][2];
+    // How the backward kernel gets at the pre-activations. STORED: from the forward memory. RECOMPUTED: it runs the layers
+    // again, every wavefront by itself. COOPERATIVE: it runs them again, and the wavefronts of a workgroup share the
+    // gradient tiles of all layers.
+    enum BackwardMode { BACKWARD_STORED = 0, BACKWARD_RECOMPUTED = 1, BACKWARD_COOPERATIVE = 2 };
+    // [adjoint flags][grid gradients by slices instead of atomics][BackwardMode]
+    std::optional<AdjointKernel> backwardKernel_[ADJOINT_MODE_MAX_COMBINATIONS][2][3];
+    // Smaller batches go to the kernel whose wavefronts sum all gradient tiles by themselves, where the network has one.
+    static constexpr int COOPERATIVE_MIN_BATCH = 1 << 13;
+    /** Whether the cooperative kernel exists for this network and flags and a batch of numel points takes it, registers aside. */
+    bool cooperatesFor(int numel, int flags) const;
+    /** The cooperative kernel of this network: workgroup size (0: none fits), LDS bytes, offsets in halves. */
+    struct CooperativeLayout
+    {
+        int blockSize = 0, ldsBytes = 0;
+        std::vector<int> weightOffsets, biasOffsets;
+        int paramHalves = 0, rowsPerWave = 0;
+        int registerWeight = 0;   // how the wavefronts share the gradient tiles, TileShare of kernels/layer_cooperative.h
+        std::string attributes;
+        bool opaqueLanes = false;   // addresses in LDS are computed where they are used
+    };
+    const CooperativeLayout& cooperativeLayout() const;
+    CooperativeLayout findCooperativeLayout() const;
+    mutable std::optional<CooperativeLayout> cooperativeLayout_;
+    /** Registers of a lane for what the cooperative kernel holds across a tile: gradient tiles, pre-activations, one layer's work. */
+    int cooperativeRegisters(int waves, int registerWeight) const;
+    /** Slices of partial weight gradients that a batch leaves room for: one per workgroup of the cooperative kernel. */
+    int cooperativeSlices(int numTiles) const;
+    std::string cooperativeBackwardSource(int flags, bool sliceGradients) const;
+    /** True if the training pass in front of a cooperative backward kernel stores nothing (the encoded input is the input). */
+    bool cooperativeReadsInputRows() const { return directInputStart() >= 0; }
     // Below this the two slice kernels cost more than the atomics they save (their work items zero and write
     // back whole slices whatever the batch): a train step of a 16-level hash grid at 2^14 / 2^15 / 2^16 / 2^17
     // points 0.18 / 0.24 / 0.37 / 0.63 ms with atomics, 0.18 / 0.19 / 0.22 / 0.30 ms by slices; of one dense
@@ -284,20 +318,26 @@ private:
     {
         int numel = 0;
         bool derivatives = false;   // position derivatives of the grids
-        bool inputOnly = false;     // of the intermediates only the encoded input
+        BackwardMode mode = BACKWARD_STORED;   // else: what the backward kernel of this mode reads, the encoded input at most
     };
     std::unordered_map<const void*, ForwardRecord> forwardRecords_;
     /** Whether adjoint(flags) over numel points runs the layers again in its backward kernel instead of reading
      *  their intermediates: a training pass that is followed by it keeps the encoded input only. */
     bool recomputesFor(int numel, int flags) const;
+    bool canRecompute(int flags, bool sliceGradients) const;
+    mutable int recomputesKnown_[ADJOINT_MODE_MAX_COMBINATIONS][2];   // canRecompute(), -1: not known yet
     /**
      * recomputesFor(), and the backward kernel that runs the layers again holds its registers: loaded on the first
      * call for these flags (it is the kernel that adjoint() will run), and not used if it spills more than a few
      * words (16 -> 64 -> 64 -> 16 with biases: 27 gradient tiles and 72 registers of pre-activations, 316 bytes).
      */
     bool recomputes(int numel, int flags);
-    int recomputeVerdict_[ADJOINT_MODE_MAX_COMBINATIONS][2];   // -1: not known yet
+    /** The mode of the backward kernel of a batch: cooperative where it holds its registers, else as recomputes() says. */
+    BackwardMode backwardMode(int numel, int flags);
+    int recomputeVerdict_[ADJOINT_MODE_MAX_COMBINATIONS][2][3];   // [..][..][mode], -1: not known yet
     static constexpr int MAX_RECOMPUTE_SCRATCH = 64;
+    // (4 -> 128 -> 64 -> 48 -> 4 with sines spills 124 bytes and still takes half the time of the kernels it replaces)
+    static constexpr int MAX_COOPERATIVE_SCRATCH = 256;
     /** Bytes per point of the forward memory: intermediates and, where kept, position derivatives. */
     size_t forwardBytesPerPoint() const { return static_cast<size_t>(perEntryForwardMemoryBytes_) + static_cast<size_t>(derivativeBytesPerPoint_); }
     /** Whether a training pass over numel points that is followed by adjoint(flags) stores position derivatives. */
@@ -457,7 +497,7 @@ private:
     /** Throws unless every encoding with parameters has a tensor bound for 'usage'. */
     void checkEncodingParameters(Tensor::Usage usage) const;
     void launchForward(bool store, const Tensor& input, Tensor& output, half* tmpMemory, stream_t stream, bool noAlloc = false, bool derivatives = false, bool inputOnly = false);
-    void compileBackwardKernel(int flags, bool sliceGradients = false, bool compileOnly = false, bool recompute = false);
+    void compileBackwardKernel(int flags, bool sliceGradients = false, bool compileOnly = false, BackwardMode mode = BACKWARD_STORED);
     /** The records kernel of a batch of numel points (compiled on first use; compileOnly: all of them into the cache). */
     const CompiledKernel& recordsKernelFor(SliceGradientKernel& sk, int flags, int numel, bool fromDerivatives = false);
     /** Compiles (compileOnly: into the cache) or loads the two kernels of kernels/grid_gradient_columns.h for sk. */
@@ -483,6 +523,13 @@ private:
      *  wideRegisters: receives whether that kernel runs one wavefront per SIMD with 512 registers (the gradient
      *  tiles of all layers in its accumulation registers). */
     std::vector<bool> fusedWeightUpdateLayers(int adjointFlags, bool sliceGradients, bool* wideRegisters = nullptr) const;
+    std::vector<bool> findFusedWeightUpdateLayers(int adjointFlags, bool sliceGradients, bool* wideRegisters) const;
+    struct FusedLayers
+    {
+        std::vector<bool> layers;
+        bool all = false, wideRegisters = false;
+    };
+    mutable std::optional<FusedLayers> fusedLayers_[ADJOINT_MODE_MAX_COMBINATIONS][2];
     /** LDS halves per wavefront of the backward kernel for the tile that Layer::weightGradient transposes. */
     int fusedWeightUpdateTransposeHalves(bool recompute = false) const;
     /** Channels of adjoint pre-activations that the backward kernel stores per point for the weight-update kernels. */

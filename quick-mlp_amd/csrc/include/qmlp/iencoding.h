@@ -7,6 +7,7 @@
 #include <qmlp/kernels/point_order_key.h>
 
 #include <functional>
+#include <mutex>
 #include <optional>
 #include <sstream>
 #include <unordered_map>
@@ -191,6 +192,16 @@ public:
         return false;
     }
 
+    /** gradientSlices(), worked out once (asked on every call of a network): nullptr where there are none. */
+    [[nodiscard]] const GradientSliceLayout* sliceLayout() const
+    {
+        std::call_once(sliceLayoutOnce_, [this] {
+            GradientSliceLayout layout;
+            if (gradientSlices(layout)) sliceLayout_ = std::move(layout);
+        });
+        return sliceLayout_.has_value() ? &sliceLayout_.value() : nullptr;
+    }
+
     [[nodiscard]] virtual int ldsGradientFloats(int maxBytes, int& levels) const
     {
         levels = 0;
@@ -232,6 +243,8 @@ private:
     std::string adjointKernelSource(int adjointMode) const;
     std::optional<KernelFunction> forwardKernel_;
     std::optional<KernelFunction> adjointKernel_[AdjointMode::ALL_GRADIENTS + 1];
+    mutable std::once_flag sliceLayoutOnce_;
+    mutable std::optional<GradientSliceLayout> sliceLayout_;
 };
 typedef std::shared_ptr<IEncoding> IEncoding_ptr;
 

@@ -149,6 +149,18 @@ struct HasPackedForward<Act, decltype(void(Act::forward4(f16x4{})))>
     static constexpr bool value = true;
 };
 
+/** Detects the optional packed form `static f16x4 adjoint4(f16x4 x, f16x4 adjz)` of an activation. */
+template <typename Act, typename = void>
+struct HasPackedAdjoint
+{
+    static constexpr bool value = false;
+};
+template <typename Act>
+struct HasPackedAdjoint<Act, decltype(void(Act::adjoint4(f16x4{}, f16x4{})))>
+{
+    static constexpr bool value = true;
+};
+
 /** Detects composites with one activation per channel (forwardAt / adjointAt with a channel). */
 template <typename Act, typename = void>
 struct IsPerChannel
@@ -174,6 +186,20 @@ __device__ __forceinline__ half activationAdjointChannel(half x, half adjz, int 
 {
     if constexpr (IsPerChannel<Act>::value) return Act::adjointAt(x, adjz, channel);
     else return Act::adjoint(x, adjz);
+}
+
+/** Adjoint of 4 values that belong to the consecutive channels channel0 .. channel0+3. */
+template <typename Act>
+__device__ __forceinline__ f16x4 activationAdjointChannels(f16x4 x, f16x4 adjz, int channel0)
+{
+    if constexpr (HasPackedAdjoint<Act>::value) {
+        return Act::adjoint4(x, adjz);
+    } else {
+        f16x4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = fromHalf(activationAdjointChannel<Act>(toHalf(x[i]), toHalf(adjz[i]), channel0 + i));
+        return o;
+    }
 }
 
 template <typename Act>

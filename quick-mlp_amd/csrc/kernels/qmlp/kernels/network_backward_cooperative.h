@@ -1,0 +1,220 @@
+// Template of the adjoint kernel that runs the layers again and sums all weight gradients, workgroup by workgroup.
+// The host code generator replaces everything in $$..$$ before the source is handed to the compiler.
+//
+// A workgroup of 4 or 8 wavefronts takes tiles of 32 points per wavefront. From the encoded input (read from the
+// forward memory, or, where the only encoding is an identity, straight from the input rows: the training pass then
+// stores nothing at all) a wavefront runs the layers forward, keeps the pre-activations in registers, and goes back
+// layer by layer; the weight gradients of a layer are formed by the workgroup from rows in LDS
+// (layer_cooperative.h), two workgroup barriers per layer. For the adjoint of the encoded input: the input gradients
+// of identity encodings are added here, those of grids are left to the kernels behind this one.
+//
+// Replaces, like network_backward.h, NetworkKernelBackward of the reference
+// (src_cpp/include/qmlp/kernels/network_backward.cuh:33-114) and its weight update
+// (network_weight_update_block.cuh:356-494).
+
+#include <qmlp/kernels/common.h>
+#include <qmlp/kernels/arrays.h>
+#include <qmlp/kernels/layer_cooperative.h>
+
+$$INCLUDES$$
+
+QUICKMLP_KERNEL_NAMESPACE_BEGIN
+
+namespace activations
+{
+$$DEFINE_ACTIVATIONS$$
+    // stands for "no activation": the input of the first layer
+    struct passthrough_
+    {
+        static __device__ __forceinline__ half forward(half x) { return x; }
+        static __device__ __forceinline__ f16x4 forward4(f16x4 x) { return x; }
+    };
+}
+
+__global__ void __launch_bounds__($$BLOCK_SIZE$$) $$KERNEL_ATTRIBUTES$$ NetworkKernelBackwardCooperative(
+    int numel,
+    const Tensor2Read<float> inputs,      //shape (numel, Cin)
+    const Tensor2Read<float> adjOutputs,  //shape (numel, Cout)
+    Tensor2RW<float> adjInputs,           //shape (numel, Cin), accumulated; unused without input gradients
+    const half* __restrict__ networkParametersH,
+    const half* __restrict__ forwardTmpMemoryH,  //the encoded input, 64-point tiles (unused with DIRECT_INPUT)
+    half* __restrict__ adjointTmpMemoryH,        //receives the adjoint of the encoded input (STORE_ENCODED_ADJOINT)
+    float* __restrict__ partialGradients,        //partialSlices x the layout of the parameters; workgroup b stores the sums of
+    int partialSlices,                           //its tiles into slice b (and zeroes slices b + k * gridDim.x)
+    const int* __restrict__ adjOutputOrder       //nullptr, or (numel) the row of adjOutputs that belongs to point p
+    $$ENCODING_PARAMETERS$$)
+{
+    constexpr int NUM_INPUTS = $$NUM_INPUTS$$;
+    constexpr int ENCODED_CHANNELS = $$ENCODED_CHANNELS$$;
+    constexpr int CHANNELS_IN = $$CHANNELS_IN$$;
+    constexpr int CHANNELS_OUT = $$CHANNELS_OUT$$;
+    constexpr int KT0 = CHANNELS_IN / 16;
+    constexpr int MTL = CHANNELS_OUT / 16;
+    constexpr int WAVES = $$BLOCK_SIZE$$ / WAVE_SIZE;
+    constexpr int NUM_PARAMETERS = $$NUM_PARAMETERS$$;
+    constexpr int ROWS_PER_WAVE = $$ROWS_PER_WAVE$$;   // halves
+    constexpr bool HAS_INPUT_GRADIENTS = $$HAS_INPUT_GRADIENTS$$;         // of encodings that are differentiated here
+    constexpr bool NEEDS_ENCODING_ADJOINT = $$NEEDS_ENCODING_ADJOINT$$;   // here or in the kernels behind this one
+    constexpr bool STORE_ENCODED_ADJOINT = $$STORE_ENCODED_ADJOINT$$;
+    // >= 0: the only encoding is an identity encoding of the input channels from this one on
+    constexpr int DIRECT_INPUT_START = $$DIRECT_INPUT_START$$;
+    constexpr bool DIRECT_INPUT = DIRECT_INPUT_START >= 0;
+    (void)ENCODED_CHANNELS; (void)NUM_INPUTS;
+
+    const f16* __restrict__ networkParameters = reinterpret_cast<const f16*>(networkParametersH);
+    const f16* __restrict__ forwardTmpMemory = reinterpret_cast<const f16*>(forwardTmpMemoryH);
+    f16* __restrict__ adjointTmpMemory = reinterpret_cast<f16*>(adjointTmpMemoryH);
+    (void)forwardTmpMemory; (void)adjointTmpMemory;
+
+    extern __shared__ __align__(16) unsigned char sMemory[];
+    f16* sParams = reinterpret_cast<f16*>(sMemory);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+    const int lane = threadIdx.x % WAVE_SIZE;
+    const int g = lane >> 4, r = lane & 15;
+    f16* sRowsAll = sParams + $$LDS_PARAM_HALVES$$;
+    f16* sRows = sRowsAll + wave * ROWS_PER_WAVE;
+
+$$STAGE_PARAMETERS$$
+$$DECLARE_WEIGHT_GRADIENTS$$
+    __syncthreads();
+
+    const int numTiles = (numel + TILE_POINTS - 1) / TILE_POINTS;
+    const int actualChannelsOut = adjOutputs.sizes_[1];
+    const bool adjOutputRowsOfFloat4 = actualChannelsOut % 4 == 0 && adjOutputs.strides_[1] == 1 && adjOutputs.strides_[0] % 4 == 0
+        && reinterpret_cast<unsigned long long>(adjOutputs.data_) % 16 == 0;
+    const bool inputRowsOfFloat4 = DIRECT_INPUT && DIRECT_INPUT_START % 4 == 0 && inputs.strides_[1] == 1 && inputs.strides_[0] % 4 == 0
+        && reinterpret_cast<unsigned long long>(inputs.data_) % 16 == 0;
+    (void)inputRowsOfFloat4;
+    const int numGroups = (numel + WAVES * COOP_POINTS - 1) / (WAVES * COOP_POINTS);
+    for (int group = blockIdx.x; group < numGroups; group += gridDim.x)
+    {
+        const int half32 = group * WAVES + wave;               // this wavefront's 32 points
+        const int point0 = half32 * COOP_POINTS + 2 * r;       // points 2r and 2r + 1 of them
+        const int tile = half32 >> 1;
+        unsigned valid[COOP_NT];
+        f16x4 dyOut[COOP_NT][MTL];
+        f16x4 x0[COOP_NT][KT0];
+#pragma unroll
+        for (int nt = 0; nt < COOP_NT; ++nt) {
+            const int p = point0 + nt;
+            const bool pv = p < numel;
+            valid[nt] = pv ? ~0u : 0u;
+            // dL/dy -> accumulator layout (fp32 -> fp16), zero outside batch / real channels
+            const long long adjRow = pv ? (adjOutputOrder ? adjOutputOrder[p] : p) : 0;
+            const float* row = adjOutputs.data_ + adjRow * adjOutputs.strides_[0];
+#pragma unroll
+            for (int m = 0; m < MTL; ++m) {
+                const int c = 16 * m + 4 * g;
+                f32x4 v = {0.f, 0.f, 0.f, 0.f};
+                if (adjOutputRowsOfFloat4) {
+                    if (pv && c < actualChannelsOut) v = *reinterpret_cast<const f32x4*>(row + c);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (pv && c + i < actualChannelsOut) v[i] = row[static_cast<long long>(c + i) * adjOutputs.strides_[1]];
+                }
+                dyOut[nt][m] = toF16(v);
+            }
+            if constexpr (DIRECT_INPUT) {
+                const float* in = inputs.data_ + static_cast<long long>(pv ? p : 0) * inputs.strides_[0]
+                    + static_cast<long long>(DIRECT_INPUT_START) * inputs.strides_[1];
+#pragma unroll
+                for (int t = 0; t < KT0; ++t) {
+                    const int c = 16 * t + 4 * g;
+                    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+                    if (16 * t + 15 < ENCODED_CHANNELS && inputRowsOfFloat4) {
+                        if (pv) v = *reinterpret_cast<const f32x4*>(in + c);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (pv && c + i < ENCODED_CHANNELS) v[i] = in[static_cast<long long>(c + i) * inputs.strides_[1]];
+                    }
+                    x0[nt][t] = toF16(v);
+                }
+            }
+        }
+        if constexpr (!DIRECT_INPUT) {
+            // as the forward kernel stored it: channel-major tiles of 64 points, zero outside the batch
+            const f16* encTile = forwardTmpMemory + static_cast<long long>(tile < numTiles ? tile : numTiles - 1) * (CHANNELS_IN * TILE_POINTS)
+                + (half32 & 1) * COOP_POINTS + 2 * r;
+#pragma unroll
+            for (int t = 0; t < KT0; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const f16x2 v = *reinterpret_cast<const f16x2*>(encTile + (16 * t + 4 * g + i) * TILE_POINTS);
+                    x0[0][t][i] = v[0];
+                    x0[1][t][i] = v[1];
+                }
+        }
+
+        // the layers forward, pre-activations kept; then last to first
+$$CALL_NETWORK_LAYERS$$
+
+        if constexpr (STORE_ENCODED_ADJOINT) {
+            if (tile < numTiles) {
+                f16* adjTile = adjointTmpMemory + static_cast<long long>(tile) * (CHANNELS_IN * TILE_POINTS) + (half32 & 1) * COOP_POINTS + 2 * r;
+#pragma unroll
+                for (int t = 0; t < KT0; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const f16x2 v = {dxIn[0][t][i], dxIn[1][t][i]};
+                        *reinterpret_cast<f16x2*>(adjTile + (16 * t + 4 * g + i) * TILE_POINTS) = v;
+                    }
+            }
+        }
+        if constexpr (HAS_INPUT_GRADIENTS && DIRECT_INPUT) {
+            // a lane holds the gradients of 4 channels side by side
+            const bool rowsOfFloat4 = DIRECT_INPUT_START % 4 == 0 && adjInputs.strides_[1] == 1 && adjInputs.strides_[0] % 4 == 0
+                && reinterpret_cast<unsigned long long>(adjInputs.data_) % 16 == 0;
+#pragma unroll
+            for (int nt = 0; nt < COOP_NT; ++nt) {
+                if (point0 + nt >= numel) continue;
+                float* row = adjInputs.data_ + static_cast<long long>(point0 + nt) * adjInputs.strides_[0]
+                    + static_cast<long long>(DIRECT_INPUT_START) * adjInputs.strides_[1];
+#pragma unroll
+                for (int t = 0; t < KT0; ++t) {
+                    const int c = 16 * t + 4 * g;
+                    if (16 * t + 15 < ENCODED_CHANNELS && rowsOfFloat4) {
+                        f32x4* target = reinterpret_cast<f32x4*>(row + c);
+                        *target = *target + __builtin_convertvector(dxIn[nt][t], f32x4);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (c + i < ENCODED_CHANNELS) row[static_cast<long long>(c + i) * adjInputs.strides_[1]] += static_cast<float>(dxIn[nt][t][i]);
+                    }
+                }
+            }
+        }
+        if constexpr (HAS_INPUT_GRADIENTS && !DIRECT_INPUT) {
+            // the adjoint of the encoded input: registers -> a row per point (the rows of this wavefront are free: the last
+            // barrier of layer 0 is behind) -> one lane per point
+            constexpr int STAGE_STRIDE = CHANNELS_IN + 8;
+#pragma unroll
+            for (int nt = 0; nt < COOP_NT; ++nt)
+#pragma unroll
+                for (int t = 0; t < KT0; ++t)
+                    *reinterpret_cast<f16x4*>(sRows + (2 * r + nt) * STAGE_STRIDE + 16 * t + 4 * g) = dxIn[nt][t];
+            waveLdsSync();
+            const int index = half32 * COOP_POINTS + lane;
+            if (lane < COOP_POINTS && index < numel) {
+                StaticArray<float, NUM_INPUTS> encodingInput;
+#pragma unroll
+                for (int i = 0; i < NUM_INPUTS; ++i)
+                    encodingInput[i] = inputs.data_[static_cast<long long>(index) * inputs.strides_[0]
+                                                    + static_cast<long long>(i) * inputs.strides_[1]];
+                StaticArray<float, NUM_INPUTS> adjEncodingInput;
+#pragma unroll
+                for (int i = 0; i < NUM_INPUTS; ++i) adjEncodingInput[i] = 0.f;
+                WrappedArray<const f16> adjEncodingOutput{sRows + lane * STAGE_STRIDE};
+$$CALL_ENCODINGS$$
+                float* adjRow = adjInputs.data_ + static_cast<long long>(index) * adjInputs.strides_[0];
+#pragma unroll
+                for (int i = 0; i < NUM_INPUTS; ++i) adjRow[static_cast<long long>(i) * adjInputs.strides_[1]] += adjEncodingInput[i];
+            }
+            waveLdsSync();
+        }
+    }
+$$STORE_WEIGHT_GRADIENTS$$
+}
+
+QUICKMLP_KERNEL_NAMESPACE_END

@@ -32,6 +32,20 @@ static std::string packedForward(const std::string& forward)
     return "";
 }
 
+/** The same for adjoint snippets. */
+static std::string packedAdjoint(const std::string& adjoint)
+{
+    const std::string a = withoutSpaces(adjoint);
+    if (a == "adjx=__hgt(x,hZERO())?adjz:hZERO()")
+        // ReLU: one where x is positive (as integers: neither NaN, which the maximum removed, nor -0), times the bits of adjz
+        return "        typedef short s16x4 __attribute__((ext_vector_type(4)));\n"
+               "        const s16x4 p = __builtin_bit_cast(s16x4, __builtin_elementwise_max(x, f16x4{0, 0, 0, 0}));\n"
+               "        const s16x4 one = __builtin_elementwise_min(__builtin_elementwise_max(p, s16x4{0, 0, 0, 0}), s16x4{1, 1, 1, 1});\n"
+               "        return __builtin_bit_cast(f16x4, __builtin_bit_cast(s16x4, adjz) * one);\n";
+    if (a == "adjx=adjz") return "        return adjz;\n";
+    return "";
+}
+
 static std::string generateCode(const std::string& id, const std::string& forward, const std::string& adjoint)
 {
     static const char* TEMPLATE = R"code(
@@ -56,6 +70,9 @@ struct %s
     std::string packed = packedForward(forward);
     if (!packed.empty())
         packed = "    static __device__ __forceinline__ f16x4 forward4(f16x4 x) {\n" + packed + "    }\n";
+    const std::string packedAdj = packedAdjoint(adjoint);
+    if (!packedAdj.empty())
+        packed += "    static __device__ __forceinline__ f16x4 adjoint4(f16x4 x, f16x4 adjz) {\n" + packedAdj + "    }\n";
     return format(TEMPLATE, id.c_str(), forward.c_str(), adjoint.c_str(), packed.c_str());
 }
 

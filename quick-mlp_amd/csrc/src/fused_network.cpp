@@ -43,11 +43,9 @@ int FusedNetwork::MaxSharedMemoryBytes()
     return value;
 }
 
-static bool offersSlices(const IEncoding& e, IEncoding::GradientSliceLayout* layout = nullptr)
-{
-    IEncoding::GradientSliceLayout local;
-    return e.hasParameters() && e.gradientSlices(layout ? *layout : local);
-}
+/** The gradient slices of an encoding, nullptr if it has none. */
+static const IEncoding::GradientSliceLayout* slicesOf(const IEncoding& e) { return e.hasParameters() ? e.sliceLayout() : nullptr; }
+static bool offersSlices(const IEncoding& e) { return slicesOf(e) != nullptr; }
 
 FusedNetwork::FusedNetwork(const json& cfg, const std::filesystem::path& parent)
     : channelsIn_(cfg.at("num_inputs").get<int>())
@@ -88,6 +86,7 @@ FusedNetwork::FusedNetwork(const json& cfg, const std::filesystem::path& parent)
         compileOptions_.columnGradients = options.value("column_gradients", compileOptions_.columnGradients);
         compileOptions_.recomputeIntermediates = options.value("recompute_intermediates", compileOptions_.recomputeIntermediates);
         compileOptions_.fusedWeightUpdate = options.value("fused_weight_update", compileOptions_.fusedWeightUpdate);
+        compileOptions_.cooperativeBackward = options.value("cooperative_backward", compileOptions_.cooperativeBackward);
         compileOptions_.skewSharedMemory = options.value("skew_shared_memory", compileOptions_.skewSharedMemory);
         compileOptions_.parallelWeightUpdate =
             options.value("parallel_weight_update", compileOptions_.parallelWeightUpdate);
@@ -220,16 +219,18 @@ FusedNetwork::FusedNetwork(const json& cfg, const std::filesystem::path& parent)
     }
     perEntryForwardMemoryBytes_ = offsetFwd * static_cast<int>(sizeof(half));
 
-    for (auto& perFlags : recomputeVerdict_) perFlags[0] = perFlags[1] = -1;
+    for (auto& perFlags : recomputesKnown_) perFlags[0] = perFlags[1] = -1;
+    for (auto& perFlags : recomputeVerdict_)
+        for (auto& perSlices : perFlags) std::fill(std::begin(perSlices), std::end(perSlices), -1);
     // behind the intermediates: the position derivatives of the grids whose gradients take the slice kernels
     derivativeOffsets_.assign(encodings_.size(), -1);
     derivativeBytesPerPoint_ = 0;
     if (compileOptions_.inputDerivatives != 0 && hasSliceGradients()) {
         for (size_t i = 0; i < encodings_.size(); ++i) {
-            IEncoding::GradientSliceLayout layout;
-            if (!offersSlices(*encodings_[i], &layout) || layout.derivativeBytesPerPoint <= 0) continue;
+            const auto* layout = slicesOf(*encodings_[i]);
+            if (!layout || layout->derivativeBytesPerPoint <= 0) continue;
             derivativeOffsets_[i] = derivativeBytesPerPoint_;
-            derivativeBytesPerPoint_ += layout.derivativeBytesPerPoint;
+            derivativeBytesPerPoint_ += layout->derivativeBytesPerPoint;
         }
     }
 }
@@ -238,8 +239,15 @@ bool FusedNetwork::recomputesFor(int numel, int flags) const
 {
     if (compileOptions_.recomputeIntermediates == 0 || flags <= 0 || flags >= ADJOINT_MODE_MAX_COMBINATIONS) return false;
     if (!(flags & GRADIENTS_NETWORK_WEIGHTS)) return false;
-    // the backward kernel of these flags sums the weight gradients of every layer itself ...
     const bool sliceGradients = useSliceGradients(numel, flags);
+    int& known = recomputesKnown_[flags][sliceGradients ? 1 : 0];
+    if (known < 0) known = canRecompute(flags, sliceGradients) ? 1 : 0;
+    return known == 1;
+}
+
+bool FusedNetwork::canRecompute(int flags, bool sliceGradients) const
+{
+    // the backward kernel of these flags sums the weight gradients of every layer itself ...
     for (bool fused : fusedWeightUpdateLayers(flags, sliceGradients))
         if (!fused) return false;
     // ... and has room for the weights in both operand orders and for a second tile per wavefront
@@ -252,20 +260,135 @@ bool FusedNetwork::recomputesFor(int numel, int flags) const
     return lds <= MaxSharedMemoryBytes();
 }
 
-bool FusedNetwork::recomputes(int numel, int flags)
+bool FusedNetwork::recomputes(int numel, int flags) { return backwardMode(numel, flags) != BACKWARD_STORED; }
+
+FusedNetwork::BackwardMode FusedNetwork::backwardMode(int numel, int flags)
 {
-    if (!recomputesFor(numel, flags)) return false;
-    const bool sliceGradients = useSliceGradients(numel, flags);
-    int& verdict = recomputeVerdict_[flags][sliceGradients ? 1 : 0];
-    if (verdict < 0) {
-        compileBackwardKernel(flags, sliceGradients, false, true);
-        const auto& kernel = backwardKernel_[flags][sliceGradients ? 1 : 0][1].value().adjoint;
-        verdict = kernel.fun.scratchBytes() <= MAX_RECOMPUTE_SCRATCH ? 1 : 0;
-        if (!verdict)
-            QuickMLP::Instance().getLogger()->debug("the backward kernel that runs the layers again (flags %d) spills %d bytes per lane, not used",
-                                                    flags, kernel.fun.scratchBytes());
+    if (flags <= 0 || flags >= ADJOINT_MODE_MAX_COMBINATIONS) return BACKWARD_STORED;
+    for (BackwardMode mode : {BACKWARD_COOPERATIVE, BACKWARD_RECOMPUTED}) {
+        if (!(mode == BACKWARD_COOPERATIVE ? cooperatesFor(numel, flags) : recomputesFor(numel, flags))) continue;
+        const int slices = useSliceGradients(numel, flags) ? 1 : 0;
+        int& verdict = recomputeVerdict_[flags][slices][mode];
+        if (verdict < 0) {
+            compileBackwardKernel(flags, slices != 0, false, mode);
+            const auto& kernel = backwardKernel_[flags][slices][mode].value().adjoint;
+            verdict = kernel.fun.scratchBytes() <= (mode == BACKWARD_COOPERATIVE ? MAX_COOPERATIVE_SCRATCH : MAX_RECOMPUTE_SCRATCH) ? 1 : 0;
+            if (!verdict)
+                QuickMLP::Instance().getLogger()->debug("the %s backward kernel (flags %d) spills %d bytes per lane, not used",
+                                                        mode == BACKWARD_COOPERATIVE ? "cooperative" : "recomputing", flags,
+                                                        kernel.fun.scratchBytes());
+        }
+        if (verdict == 1) return mode;
     }
-    return verdict == 1;
+    return BACKWARD_STORED;
+}
+
+bool FusedNetwork::cooperatesFor(int numel, int flags) const
+{
+    if (compileOptions_.cooperativeBackward == 0 || compileOptions_.recomputeIntermediates == 0 || compileOptions_.fusedWeightUpdate >= 0
+        || compileOptions_.overwriteBlocksizeBackward > 0)
+        return false;
+    if (!(flags & GRADIENTS_NETWORK_WEIGHTS)) return false;
+    if (compileOptions_.cooperativeBackward < 0) {
+        // The kernel whose wavefronts sum all gradient tiles by themselves starts more workgroups; one that leaves some of
+        // them to kernels of their own is behind at every size (64 x 4 hidden layers, 2048 points: 58 against 29 us). With an
+        // encoded input to be stored and read, two wavefronts per SIMD that hold all tiles are as fast as the shared
+        // ones (16 -> 32 x 3 -> 16 behind a dense 4-D grid, 2^21 points: 568 us both).
+        bool wideRegisters = false;
+        (void)fusedWeightUpdateLayers(flags, useSliceGradients(numel, flags), &wideRegisters);
+        if (fusedLayers_[flags][useSliceGradients(numel, flags) ? 1 : 0]->all && (numel < COOPERATIVE_MIN_BATCH || (!wideRegisters && !cooperativeReadsInputRows()))) return false;
+    }
+    // grids are left to the kernels of the gradient slices, which also differentiate them with respect to the position
+    const bool sliceGradients = useSliceGradients(numel, flags);
+    for (const auto& e : encodings_) {
+        if (!(flags & (GRADIENTS_INPUT | GRADIENTS_INPUT_ENCODINGS))) continue;
+        if (dynamic_cast<const EncodingIdentity*>(e.get())) continue;
+        if (!(sliceGradients && (flags & GRADIENTS_INPUT_ENCODINGS) && offersSlices(*e))) return false;
+    }
+    return cooperativeLayout().blockSize > 0;
+}
+
+const FusedNetwork::CooperativeLayout& FusedNetwork::cooperativeLayout() const
+{
+    if (!cooperativeLayout_.has_value()) cooperativeLayout_ = findCooperativeLayout();
+    return cooperativeLayout_.value();
+}
+
+FusedNetwork::CooperativeLayout FusedNetwork::findCooperativeLayout() const
+{
+    // as kernels/layer_cooperative.h: weights row-major with 4 halves of padding per row, then the biases, then per
+    // wavefront 32 rows of the widest layer's adjoint pre-activations and input
+    constexpr int PAD = 4, POINTS = 32;
+    CooperativeLayout c;
+    c.biasOffsets.assign(layers_.size(), 0);
+    int sums = 0;
+    for (const auto& l : layers_) {
+        c.weightOffsets.push_back(c.paramHalves);
+        c.paramHalves += l.channelsOut * (l.channelsIn + PAD);
+        c.rowsPerWave = std::max(c.rowsPerWave, POINTS * (l.channelsOut + PAD + l.channelsIn + PAD));
+        sums = std::max(sums, l.channelsOut * (l.channelsIn + 1) * static_cast<int>(sizeof(float)));
+    }
+    for (size_t i = 0; i < layers_.size(); ++i) {
+        if (!layers_[i].useBias) continue;
+        c.biasOffsets[i] = c.paramHalves;
+        c.paramHalves += layers_[i].channelsOut;
+    }
+    c.paramHalves = roundUp(c.paramHalves, 8);
+    // Workgroups of 4 wavefronts, two or more per compute unit, where LDS and registers allow it (at the barriers of one the
+    // other goes on: 64 -> 64 x 4 -> 4 on 10^6 points, forward and backward, 207 -> 176 us); else one of 8, whose wavefronts
+    // hold half as many gradient tiles (the 256 registers of two wavefronts per SIMD both); else one of 4 with 512 registers.
+    // (4 -> 128 -> 64 -> 48 -> 4, 10^6 points: 348, 365 and 421 us; 96 x 3 hidden layers, where the first does not fit into
+    // the LDS: 288 and 302 us.) The limits leave room for addresses and operands in flight.
+    const int lds = MaxSharedMemoryBytes();
+    struct Candidate { int waves, ldsLimit, registers; const char* attributes; };
+    const Candidate candidates[] = {{4, lds / 2, 225, "__attribute__((amdgpu_waves_per_eu(2)))"},
+                                    {8, lds, 225, ""},
+                                    {4, lds, 420, "__attribute__((amdgpu_waves_per_eu(1, 1)))"}};
+    for (const auto& candidate : candidates) {
+        const int bytes = std::max(sums, (c.paramHalves + candidate.waves * c.rowsPerWave) * static_cast<int>(sizeof(half)));
+        if (bytes > candidate.ldsLimit) continue;
+        for (int weight : {8, 16}) {
+            const int registers = cooperativeRegisters(candidate.waves, weight);
+            if (c.blockSize > 0 || registers > (weight == 16 ? candidate.registers : 200)) continue;
+            // Addresses of all layers held over the loop cost up to 40 registers, computed where they are used 5 % of the
+            // time of a kernel that has them to spare (64 x 4: 173 against 181 us; 4 -> 128 -> 64 -> 48 -> 4: 442 against 348).
+            c.opaqueLanes = registers > 180;
+            c.blockSize = candidate.waves * WARP_SIZE;
+            c.ldsBytes = bytes;
+            c.registerWeight = weight;
+            c.attributes = candidate.attributes;
+        }
+    }
+    return c;
+}
+
+int FusedNetwork::cooperativeRegisters(int waves, int registerWeight) const
+{
+    int tiles = 0, kept = layers_[0].channelsIn / MATRIX_SIZE, work = 0;
+    for (const auto& l : layers_) {
+        const int mt = l.channelsOut / MATRIX_SIZE, kt = l.channelsIn / MATRIX_SIZE;
+        int best = std::numeric_limits<int>::max(), own = 0;
+        for (int m = 1; m <= waves; m *= 2)   // TileShare::split
+            for (int k = 1; m * k <= waves; k *= 2) {
+                const int mo = divUp(mt, m), ki = divUp(kt, k);
+                const int cost = 8 * m * k * (mo * ki + mo + ki) + registerWeight * 4 * mo * ki;
+                if (cost < best) {
+                    best = cost;
+                    own = mo * ki;
+                }
+            }
+        tiles += own + (l.useBias ? 1 : 0);
+        kept += mt;
+        work = std::max(work, mt + 2 * kt);   // adjoint, input and its adjoint of a layer
+    }
+    return 4 * (tiles + kept + work);   // a tile of sums: 4 registers; 16 channels of 2 x 16 points in half precision: 4
+}
+
+int FusedNetwork::cooperativeSlices(int numTiles) const
+{
+    // one per workgroup, four workgroups per compute unit at most
+    const CooperativeLayout& layout = cooperativeLayout();
+    return std::max(1, std::min(divUp(2 * numTiles, layout.blockSize / WARP_SIZE), 2 * MAX_WEIGHT_UPDATE_SLICES));
 }
 
 bool FusedNetwork::storesDerivatives(int numel, int flags) const
@@ -663,6 +786,19 @@ int FusedNetwork::weightUpdateSlices(int numTiles) const
 
 std::vector<bool> FusedNetwork::fusedWeightUpdateLayers(int adjointFlags, bool sliceGradients, bool* wideRegisters) const
 {
+    // (a function of the specification: worked out once, the calls of a training loop ask several times each)
+    auto& known = fusedLayers_[adjointFlags & (ADJOINT_MODE_MAX_COMBINATIONS - 1)][sliceGradients ? 1 : 0];
+    if (!known.has_value()) {
+        known.emplace();
+        known->layers = findFusedWeightUpdateLayers(adjointFlags, sliceGradients, &known->wideRegisters);
+        known->all = std::find(known->layers.begin(), known->layers.end(), false) == known->layers.end();
+    }
+    if (wideRegisters) *wideRegisters = known->wideRegisters;
+    return known->layers;
+}
+
+std::vector<bool> FusedNetwork::findFusedWeightUpdateLayers(int adjointFlags, bool sliceGradients, bool* wideRegisters) const
+{
     std::vector<bool> fused(layers_.size(), false);
     if (wideRegisters) *wideRegisters = false;
     if (compileOptions_.fusedWeightUpdate == 0 || !(adjointFlags & GRADIENTS_NETWORK_WEIGHTS)) return fused;
@@ -811,8 +947,9 @@ std::string FusedNetwork::forwardSource(int blockSize, int pointsPerLane, bool r
             callEncodings << "            {\n                StageRowArray<f16, CHANNELS_IN> encodingOutputK[PPL];\n"
                           << "#pragma unroll\n                for (int q = 0; q < PPL; ++q) encodingOutputK[q] = encodingOutput[q] + "
                           << encodingOffset << ";\n                ";
-        IEncoding::GradientSliceLayout sliceLayout;
-        if (derivatives && derivativeOffsets_[encodingIdx] >= 0 && offersSlices(*e, &sliceLayout)) {
+        const auto* slices = slicesOf(*e);
+        if (derivatives && derivativeOffsets_[encodingIdx] >= 0 && slices) {
+            const auto& sliceLayout = *slices;
             // the lane's chunks of its first tile; the tiles of a wave follow one another
             callEncodings << "static_assert(STORE && DERIVATIVES, \"this source is that of the training pass that keeps position derivatives\");\n"
                           << "                typedef PositionDerivativeLayout<" << sliceLayout.configType << "> DerivativeLayout;\n"
@@ -879,8 +1016,9 @@ size_t FusedNetwork::sliceGradientWorkspaceBytes(long long numel) const
     if (!hasSliceGradients()) return 0;
     size_t bytes = 0;
     for (const auto& e : encodings_) {
-        IEncoding::GradientSliceLayout layout;
-        if (!offersSlices(*e, &layout)) continue;
+        const auto* slices = slicesOf(*e);
+        if (!slices) continue;
+        const auto& layout = *slices;
         bytes += roundUp(static_cast<size_t>(layout.numBuckets() + 1) * sizeof(int), size_t(256));   // cursors, largest adjoint
         bytes += roundUp(static_cast<size_t>(layout.totalRecords(numel)) * layout.recordWords * sizeof(uint32_t), size_t(256));
     }
@@ -893,8 +1031,8 @@ bool FusedNetwork::useSliceGradients(int numel, int flags) const
     if (compileOptions_.sliceGradients > 0 || numel >= SLICE_GRADIENTS_MIN_BATCH) return true;
     if (numel < SLICE_GRADIENTS_MIN_BATCH_MANY_LEVELS) return false;
     for (const auto& e : encodings_) {
-        IEncoding::GradientSliceLayout layout;
-        if (offersSlices(*e, &layout) && layout.slicesPerLevel.size() >= 8) return true;
+        const auto* layout = slicesOf(*e);
+        if (layout && layout->slicesPerLevel.size() >= 8) return true;
     }
     return false;
 }
@@ -1146,6 +1284,82 @@ std::string FusedNetwork::backwardSource(int flags, int blockSize, bool sliceGra
     return code;
 }
 
+std::string FusedNetwork::cooperativeBackwardSource(int flags, bool sliceGradients) const
+{
+    const bool hasInputGradients = flags & GRADIENTS_INPUT;
+    const bool hasEncodingGradients = flags & GRADIENTS_INPUT_ENCODINGS;
+    auto kl = QuickMLP::Instance().kernelLoader();
+    std::string code = kl->findFile("qmlp/kernels/network_backward_cooperative.h").value();
+    fillEncodingsAndActivations(code);
+    const CooperativeLayout& layout = cooperativeLayout();
+    const std::vector<int>&ldsW = layout.weightOffsets, &ldsB = layout.biasOffsets;
+    const int L = static_cast<int>(layers_.size());
+    const int weight = layout.registerWeight;
+    const std::string lane = layout.opaqueLanes ? "opaqueLane(lane)" : "lane";
+    std::stringstream stage, declare, call, store;
+    for (int i = 0; i < L; ++i) {
+        const auto& l = layers_[i];
+        stage << "    typedef CooperativeLayer<" << l.channelsIn << ", " << l.channelsOut << ", " << (l.useBias ? "true" : "false")
+              << ", activations::" << activationTypeName(i) << ", WAVES, " << weight << "> Layer" << i << ";\n";
+        stage << "    Layer" << i << "::stageWeights(networkParameters + " << l.weightsStart << ", sParams + " << ldsW[i] << ", threadIdx.x, blockDim.x);\n";
+        if (l.useBias)
+            stage << "    for (int i = threadIdx.x; i < " << l.channelsOut << "; i += blockDim.x) sParams[" << ldsB[i] << " + i] = networkParameters["
+                  << l.biasStart << " + i];\n";
+        declare << "    Layer" << i << "::Sums sums" << i << ";\n    sums" << i << ".zero();\n";
+        call << "        Layer" << i << "::output_t pre" << i << ";\n        Layer" << i << "::forward(sParams + " << ldsW[i] << ", "
+             << (l.useBias ? "sParams + " + std::to_string(ldsB[i]) : std::string("nullptr")) << ", " << (i == 0 ? std::string("x0") : "act" + std::to_string(i))
+             << ", pre" << i << ", " << lane << ");\n";
+        if (i + 1 < L) call << "        Layer" << i << "::output_t act" << (i + 1) << ";\n        Layer" << i << "::activate(pre" << i << ", act" << (i + 1) << ", lane);\n";
+        store << "    Layer" << i << "::storeWeightGradient(sums" << i << ", reinterpret_cast<float*>(sMemory),\n        partialGradients + (static_cast<long long>(blockIdx.x) * NUM_PARAMETERS + "
+              << l.weightsStart << "), partialGradients + (static_cast<long long>(blockIdx.x) * NUM_PARAMETERS + " << (l.useBias ? l.biasStart : 0)
+              << "), partialSlices, NUM_PARAMETERS, wave, lane);\n";
+    }
+    const bool needsEncodingAdjoint = hasInputGradients || hasEncodingGradients;
+    for (int i = L - 1; i >= 0; --i) {
+        const std::string dy = i == L - 1 ? std::string("dyOut") : "dx" + std::to_string(i + 1);
+        call << "        Layer" << i << "::adjointActivation(pre" << i << ", " << dy << ", sRows, valid, " << lane << ");\n";
+        if (i > 0)
+            // (from the pre-activations again: held from the forward pass on, the inputs of all layers would not fit into the registers)
+            call << "        materialize(pre" << (i - 1) << ");\n        Layer" << i << "::template stageInput<activations::" << activationTypeName(i - 1)
+                 << ">(pre" << (i - 1) << ", sRows, " << lane << ");\n";
+        else
+            call << "        Layer0::template stageInput<activations::passthrough_>(x0, sRows, " << lane << ");\n";
+        call << "        workgroupLdsBarrier();\n        Layer" << i << "::input_t dx" << i << ";\n";
+        if (i > 0 || needsEncodingAdjoint) call << "        Layer" << i << "::adjointInput(sParams + " << ldsW[i] << ", " << dy << ", dx" << i << ", " << lane << ");\n";
+        call << "        Layer" << i << "::weightGradient(sRowsAll, ROWS_PER_WAVE, sums" << i << ", wave, " << lane << ");\n        workgroupLdsBarrier();\n";
+    }
+    call << "        auto& dxIn = dx0;\n        (void)dxIn;\n";
+
+    std::stringstream callEncodings;
+    int encodingOffset = 0;
+    bool storeEncodedAdjoint = false, inputGradientsHere = false;
+    for (const auto& e : encodings_) {
+        const bool slices = hasEncodingGradients && sliceGradients && offersSlices(*e);
+        storeEncodedAdjoint = storeEncodedAdjoint || slices;
+        if (hasInputGradients && !slices) {
+            inputGradientsHere = true;
+            callEncodings << "                {\n                    auto adjEncodingOutputK = adjEncodingOutput + " << encodingOffset << ";\n                    "
+                          << e->qualifiedName() << "::template adjoint<true, false>(encodingInput, adjEncodingOutputK, adjEncodingInput);\n                }\n";
+        }
+        encodingOffset += e->numOutputChannels();
+    }
+    replaceAll(code, "$$CALL_ENCODINGS$$", callEncodings.str());
+    replaceAll(code, "$$STORE_ENCODED_ADJOINT$$", storeEncodedAdjoint ? "true" : "false");
+    replaceAll(code, "$$HAS_INPUT_GRADIENTS$$", inputGradientsHere ? "true" : "false");
+    replaceAll(code, "$$NEEDS_ENCODING_ADJOINT$$", needsEncodingAdjoint ? "true" : "false");
+    replaceAll(code, "$$DIRECT_INPUT_START$$", std::to_string(directInputStart()));
+    replaceAll(code, "$$BLOCK_SIZE$$", std::to_string(layout.blockSize));
+    replaceAll(code, "$$KERNEL_ATTRIBUTES$$", layout.attributes);
+    replaceAll(code, "$$LDS_PARAM_HALVES$$", std::to_string(layout.paramHalves));
+    replaceAll(code, "$$ROWS_PER_WAVE$$", std::to_string(layout.rowsPerWave));
+    replaceAll(code, "$$NUM_PARAMETERS$$", std::to_string(numParameters_));
+    replaceAll(code, "$$STAGE_PARAMETERS$$", stage.str());
+    replaceAll(code, "$$DECLARE_WEIGHT_GRADIENTS$$", declare.str());
+    replaceAll(code, "$$CALL_NETWORK_LAYERS$$", call.str());
+    replaceAll(code, "$$STORE_WEIGHT_GRADIENTS$$", store.str());
+    return code;
+}
+
 std::string FusedNetwork::weightUpdateSource(int blockSize) const
 {
     auto kl = QuickMLP::Instance().kernelLoader();
@@ -1226,14 +1440,20 @@ std::string FusedNetwork::generatedSource(const std::string& kind, int adjointFl
     if (kind == "backward_recompute")   // the variant that runs the layers again, for networks that have one at these flags
         return backwardSource(adjointFlags, forwardBlockSize(compileOptions_.overwriteBlocksizeBackward, true),
                               useSliceGradients(1 << 30, adjointFlags), true);
+    if (kind == "backward_cooperative")   // for networks that have one at these flags
+        return cooperativeBackwardSource(adjointFlags, useSliceGradients(1 << 30, adjointFlags));
     if (kind == "weight_update") return weightUpdateSource(weightUpdateBlockSize());
     if (kind == "backward_resources" || kind == "backward_slices_resources") {
         // what the loaded backward kernel takes (needs a device): for tests of the register budget
         const bool slices = kind == "backward_slices_resources";
         // ("recompute": the kernel of a batch of that kind runs the layers again instead of reading their intermediates)
-        const bool recompute = useSliceGradients(slices ? (1 << 30) : 1, adjointFlags) == slices && recomputes(slices ? (1 << 30) : 1, adjointFlags);
-        compileBackwardKernel(adjointFlags, slices, false, recompute);
-        const auto& ak = backwardKernel_[adjointFlags][slices ? 1 : 0][recompute ? 1 : 0].value();
+        // (of batches below COOPERATIVE_MIN_BATCH points)
+        const int numel = slices ? COOPERATIVE_MIN_BATCH - 1 : 1;
+        BackwardMode mode = BACKWARD_STORED;
+        if (useSliceGradients(slices ? (1 << 30) : 1, adjointFlags) == slices) mode = backwardMode(numel, adjointFlags);
+        const bool recompute = mode == BACKWARD_RECOMPUTED;
+        compileBackwardKernel(adjointFlags, slices, false, mode);
+        const auto& ak = backwardKernel_[adjointFlags][slices ? 1 : 0][mode].value();
         return format("{\"block\": %d, \"lds_bytes\": %d, \"registers\": %d, \"scratch_bytes\": %d, \"full_grid\": %d, \"recompute\": %s}",
                       ak.adjoint.blockSize, ak.adjoint.sharedMemorySize, ak.adjoint.fun.numVgprs(), ak.adjoint.fun.scratchBytes(),
                       ak.adjoint.fullGrid, recompute ? "true" : "false");
@@ -1417,16 +1637,28 @@ const FusedNetwork::CompiledKernel& FusedNetwork::forwardKernelFor(bool store, i
     return forwardKernels_[s][best].value();
 }
 
-void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool compileOnly, bool recompute)
+void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool compileOnly, BackwardMode mode)
 {
     if (flags <= 0 || flags >= ADJOINT_MODE_MAX_COMBINATIONS) throw std::runtime_error("At least one derivative must be enabled");
     const int variant = sliceGradients ? 1 : 0;
-    if (backwardKernel_[flags][variant][recompute ? 1 : 0].has_value() && !compileOnly) return;
+    if (backwardKernel_[flags][variant][mode].has_value() && !compileOnly) return;
+    const bool recompute = mode == BACKWARD_RECOMPUTED, cooperative = mode == BACKWARD_COOPERATIVE;
     const bool hasNetworkGradients = flags & GRADIENTS_NETWORK_WEIGHTS;
     auto kl = QuickMLP::Instance().kernelLoader();
     auto logger = QuickMLP::Instance().getLogger();
 
     AdjointKernel ak;
+    if (cooperative) {
+        const CooperativeLayout& layout = cooperativeLayout();
+        ak.adjoint.blockSize = layout.blockSize;
+        ak.adjoint.sharedMemorySize = layout.ldsBytes;
+        ak.outputOrder = true;
+        ak.fusedLayers.assign(layers_.size(), true);
+        ak.fusedWeightUpdate = true;
+        // a kernel of many registers like those below: left to the offline compiler where there is one
+        const int offlineFlags = loaderFlags(compileOnly) | KernelLoader::CompileOffline;
+        ak.adjoint.fun = kl->getKernel("qmlp::kernel::NetworkKernelBackwardCooperative", cooperativeBackwardSource(flags, sliceGradients), offlineFlags).value();
+    } else {
     ak.adjoint.blockSize = forwardBlockSize(compileOptions_.overwriteBlocksizeBackward, true);
     {
         std::vector<LdsGradients> ldsGradients;
@@ -1494,14 +1726,15 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
                 kl->getKernel("qmlp::kernel::TransposeWeightsKernel", adjointSource, adjointLoaderFlags, offlineOptions).value();
         }
     }
+    }
     if (!compileOnly) {
         ak.adjoint.fullGrid = ak.adjoint.fun.fullGridSize(ak.adjoint.blockSize, ak.adjoint.sharedMemorySize);
         logger->debug("backward kernel (flags %d%s): block %d, LDS %d bytes, %d VGPRs, %d bytes scratch, full grid %d", flags,
-                      recompute ? ", the layers run again" : "",
+                      recompute ? ", the layers run again" : cooperative ? ", cooperative" : "",
                       ak.adjoint.blockSize, ak.adjoint.sharedMemorySize, ak.adjoint.fun.numVgprs(),
                       ak.adjoint.fun.scratchBytes(), ak.adjoint.fullGrid);
     }
-    ak.perEntryAdjointMemoryBytes = storedAdjointChannels(flags, sliceGradients) * static_cast<int>(sizeof(half));
+    ak.perEntryAdjointMemoryBytes = cooperative ? 0 : storedAdjointChannels(flags, sliceGradients) * static_cast<int>(sizeof(half));
     // behind the adjoint pre-activations: the adjoint of the encoded rows for the records kernels
     if (sliceGradients && (flags & GRADIENTS_INPUT_ENCODINGS)) ak.perEntryAdjointMemoryBytes += sliceGradientBytesPerPoint();
 
@@ -1512,7 +1745,8 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
             const int offset = channelOffset;
             channelOffset += e->numOutputChannels();
             SliceGradientKernel sk;
-            if (!offersSlices(*e, &sk.layout)) continue;
+            if (!offersSlices(*e)) continue;
+            sk.layout = *slicesOf(*e);
             const auto& layout = sk.layout;
             sk.encoding = static_cast<int>(i);
             std::stringstream source;
@@ -1579,7 +1813,7 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
             }
         }
     }
-    if (!compileOnly) backwardKernel_[flags][variant][recompute ? 1 : 0] = std::move(ak);
+    if (!compileOnly) backwardKernel_[flags][variant][mode] = std::move(ak);
 }
 
 void FusedNetwork::compileRecordsKernel(SliceGradientKernel& sk, int flags, size_t variant, bool compileOnly, bool fromDerivatives)
@@ -1669,7 +1903,11 @@ void FusedNetwork::precompile(int adjointFlags)
         for (int numel : {1, 1 << 30}) {
             if (!recomputesFor(numel, adjointFlags)) continue;
             any = true;
-            compileBackwardKernel(adjointFlags, useSliceGradients(numel, adjointFlags), true, true);
+            compileBackwardKernel(adjointFlags, useSliceGradients(numel, adjointFlags), true, BACKWARD_RECOMPUTED);
+        }
+        if (cooperatesFor(1 << 30, adjointFlags)) {
+            any = any || !cooperativeReadsInputRows();   // (otherwise the inference kernel is the training pass)
+            compileBackwardKernel(adjointFlags, useSliceGradients(1 << 30, adjointFlags), true, BACKWARD_COOPERATIVE);
         }
         if (any)
             for (int derivatives = 0; derivatives <= (storesDerivatives(1 << 30, adjointFlags) ? 1 : 0); ++derivatives) {
@@ -1859,8 +2097,10 @@ void FusedNetwork::prepare(int numel, int adjointFlags)
     for (int store = 0; store <= (adjointFlags > 0 ? 1 : 0); ++store)
         for (long long start = 0; start < numel;) {
             int launchTiles = 0;
-            const auto& ck = forwardKernelFor(store != 0, static_cast<int>(divUp<long long>(numel - start, TILE_POINTS)), &launchTiles, false,
-                                              store != 0 && storesDerivatives(numel, adjointFlags), store != 0 && recomputes(numel, adjointFlags));
+            const BackwardMode mode = store ? backwardMode(numel, adjointFlags) : BACKWARD_STORED;
+            const bool stores = store != 0 && !(mode == BACKWARD_COOPERATIVE && cooperativeReadsInputRows());
+            const auto& ck = forwardKernelFor(stores, static_cast<int>(divUp<long long>(numel - start, TILE_POINTS)), &launchTiles, false,
+                                              stores && storesDerivatives(numel, adjointFlags), stores && mode != BACKWARD_STORED);
             start += std::min<long long>({static_cast<long long>(gatherChunkPoints(ck)), static_cast<long long>(launchTiles) * TILE_POINTS,
                                           numel - start});
         }
@@ -1881,9 +2121,9 @@ void FusedNetwork::prepare(int numel, int adjointFlags)
     }
     if (adjointFlags > 0) {
         const bool sliceGradients = useSliceGradients(numel, adjointFlags);
-        const bool recompute = recomputes(numel, adjointFlags);
-        compileBackwardKernel(adjointFlags, sliceGradients, false, recompute);
-        for (auto& sk : backwardKernel_[adjointFlags][sliceGradients ? 1 : 0][recompute ? 1 : 0].value().sliceGradients)
+        const BackwardMode mode = backwardMode(numel, adjointFlags);
+        compileBackwardKernel(adjointFlags, sliceGradients, false, mode);
+        for (auto& sk : backwardKernel_[adjointFlags][sliceGradients ? 1 : 0][mode].value().sliceGradients)
         {
             (void)recordsKernelFor(sk, adjointFlags, numel, storesDerivatives(numel, adjointFlags) && sk.derivativeOffset >= 0);
             if (sk.columnsOffered && sortsTraining(numel))
@@ -2042,10 +2282,11 @@ void FusedNetwork::forward(const Tensor& input, Tensor& output, void* tmpMemory,
     CHECK_ERROR(reinterpret_cast<uintptr_t>(tmpMemory) % 16 == 0, "The temporary memory must be aligned to 16 bytes");
 
     const bool derivatives = storesDerivatives(numel, announcedFlags_);
-    const bool inputOnly = recomputes(numel, announcedFlags_);
-    if (derivatives || inputOnly) forwardRecords_[tmpMemory] = ForwardRecord{numel, derivatives, inputOnly};
+    const BackwardMode mode = backwardMode(numel, announcedFlags_);
+    if (derivatives || mode != BACKWARD_STORED) forwardRecords_[tmpMemory] = ForwardRecord{numel, derivatives, mode};
     else forwardRecords_.erase(tmpMemory);
-    launchForward(true, input, output, static_cast<half*>(tmpMemory), stream, false, derivatives, inputOnly);
+    if (mode == BACKWARD_COOPERATIVE && cooperativeReadsInputRows()) launchForward(false, input, output, nullptr, stream);
+    else launchForward(true, input, output, static_cast<half*>(tmpMemory), stream, false, derivatives, mode != BACKWARD_STORED);
 }
 
 void FusedNetwork::zeroGradients()
@@ -2068,11 +2309,14 @@ size_t FusedNetwork::adjointMemoryAsGiven(int numElements, AdjointModeFlags adjo
     const bool sliceGradients = useSliceGradients(numElements, adjointFlags);
     int perEntry = storedAdjointChannels(adjointFlags, sliceGradients) * static_cast<int>(sizeof(half));
     if (sliceGradients) perEntry += sliceGradientBytesPerPoint();
+    const int batch = numElements;
     numElements = roundUp(numElements, WARP_SIZE);
     size_t bytes = static_cast<size_t>(perEntry) * static_cast<size_t>(numElements);
     // behind the adjoint pre-activations: the partial weight gradients of the batch slices
     if (adjointFlags & GRADIENTS_NETWORK_WEIGHTS)
-        bytes += static_cast<size_t>(weightUpdateSlices(numElements / TILE_POINTS)) * numParameters_ * sizeof(float);
+        bytes += static_cast<size_t>(std::max(weightUpdateSlices(numElements / TILE_POINTS),
+                                              cooperatesFor(batch, adjointFlags) ? cooperativeSlices(numElements / TILE_POINTS) : 0))
+            * numParameters_ * sizeof(float);
     // last: transposed copies of the weights the adjoint kernel cannot keep in LDS
     std::vector<long long> transposed;
     bytes += roundUp(transposedWeightLayout(adjointFlags, transposed) * sizeof(half), size_t(16));
@@ -2144,14 +2388,15 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
     announcedFlags_ = adjointFlags;
     // what the forward pass that wrote this forward memory left there: the position derivatives of the grids? Of the
     // intermediates the encoded input only?
-    bool derivativesStored = false, recompute = false;
+    bool derivativesStored = false;
+    BackwardMode mode = BACKWARD_STORED;
     {
         const auto it = forwardRecords_.find(tmpMemoryForward);
         if (it != forwardRecords_.end() && it->second.numel == numel) {
             derivativesStored = hasInputGradients && sliceGradients && it->second.derivatives;
-            if (it->second.inputOnly) {
-                if (recomputes(numel, adjointFlags)) {
-                    recompute = true;
+            if (it->second.mode != BACKWARD_STORED) {
+                if (backwardMode(numel, adjointFlags) == it->second.mode) {
+                    mode = it->second.mode;
                 } else {
                     // Announced otherwise: the kernels of these flags read intermediates that the training pass did not
                     // keep. The forward pass runs again into the same memory, this time storing them (a batch that
@@ -2159,17 +2404,20 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
                     QuickMLP::Instance().getLogger()->debug("adjoint(flags %d): the forward pass kept the encoded input only; it runs again", adjointFlags);
                     Tensor scratchOutput(precisionOut(), {numel, channelsOut()});
                     const bool derivatives = it->second.derivatives;
-                    it->second.inputOnly = false;
+                    it->second.mode = BACKWARD_STORED;
                     launchForward(true, input, scratchOutput, static_cast<half*>(const_cast<void*>(tmpMemoryForward)), stream, false, derivatives, false);
                 }
             }
         }
     }
     const bool sortedPoints = sortsTraining(numel);
-    compileBackwardKernel(adjointFlags, sliceGradients, false, recompute);
-    auto& ak = backwardKernel_[adjointFlags][sliceGradients ? 1 : 0][recompute ? 1 : 0].value();
+    compileBackwardKernel(adjointFlags, sliceGradients, false, mode);
+    auto& ak = backwardKernel_[adjointFlags][sliceGradients ? 1 : 0][mode].value();
+    const bool cooperative = mode == BACKWARD_COOPERATIVE;
 
     const int numTiles = divUp(numel, TILE_POINTS);
+    // (of the cooperative kernel no more than it has workgroups)
+    const int partialSliceCount = cooperative ? std::min(cooperativeSlices(numTiles), ak.adjoint.fullGrid) : weightUpdateSlices(numTiles);
     const long long numel64 = static_cast<long long>(numTiles) * TILE_POINTS;
     // a batch that the forward pass evaluated in sorted order: the rows as it sorted them, and for every row its
     // place in the caller's batch (rows of dL/dy are read, rows of the input gradients written through it)
@@ -2202,9 +2450,9 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
         }
     }
     const half* transposedWeights = nullptr;
-    if (transposedHalves > 0) {
+    if (transposedHalves > 0 && !cooperative) {
         size_t offset = static_cast<size_t>(ak.perEntryAdjointMemoryBytes) * static_cast<size_t>(numel64);
-        if (hasNetworkGradients) offset += static_cast<size_t>(weightUpdateSlices(numTiles)) * numParameters_ * sizeof(float);
+        if (hasNetworkGradients) offset += static_cast<size_t>(partialSliceCount) * numParameters_ * sizeof(float);
         half* dstBase = reinterpret_cast<half*>(static_cast<char*>(tmpMemoryAdjoint) + offset);
         transposedWeights = dstBase;
         for (size_t layer = 0; layer < layers_.size(); ++layer) {
@@ -2221,10 +2469,11 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
     {
         const auto& ck = ak.adjoint;
         const int waves = ck.blockSize / WARP_SIZE;
-        int grid = std::min(divUp(numTiles, waves), ck.fullGrid);
+        // (a wavefront of the cooperative kernel takes half a tile)
+        int grid = std::min(cooperative ? divUp(2 * numTiles, waves) : divUp(numTiles, waves), ck.fullGrid);
         // every workgroup stores its sums of the weight gradients as one of the slices of the batch that the
         // reduction adds up (and zeroes its share of the slices beyond the grid)
-        int partialSlices = weightUpdateSlices(numTiles);
+        int partialSlices = partialSliceCount;
         if (ak.fusedWeightUpdate) grid = std::min(grid, partialSlices);
         auto inputAcc = sortedInput;
         auto adjOutputAcc = sortedAdjOutput;
@@ -2234,8 +2483,9 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
         half* adjointTmpMemory = static_cast<half*>(tmpMemoryAdjoint);
         float* partialGradients = reinterpret_cast<float*>(static_cast<char*>(tmpMemoryAdjoint)
                                                            + static_cast<size_t>(ak.perEntryAdjointMemoryBytes) * static_cast<size_t>(numel64));
-        std::vector<void*> args = {&numel, &inputAcc, &adjOutputAcc, &adjInputAcc, &networkParams,
-                                   &forwardTmpMemory, &adjointTmpMemory, &transposedWeights, &partialGradients, &partialSlices};
+        std::vector<void*> args = {&numel, &inputAcc, &adjOutputAcc, &adjInputAcc, &networkParams, &forwardTmpMemory, &adjointTmpMemory};
+        if (!cooperative) args.push_back(&transposedWeights);
+        args.insert(args.end(), {&partialGradients, &partialSlices});
         CHECK_ERROR(ak.outputOrder || adjOutputOrder == nullptr, "a batch trains in sorted order but the backward kernel does not take the order");
         if (ak.outputOrder) args.push_back(&adjOutputOrder);
         std::vector<std::vector<char>> storage;
@@ -2244,10 +2494,11 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
     }
     // parameter gradients of the grids, slice by slice, from the adjoint of the encoded rows the kernel above stored
     if (!ak.sliceGradients.empty()) {
-        const half* adjEncoded = static_cast<const half*>(tmpMemoryAdjoint) + static_cast<ptrdiff_t>(storedAdjointChannels(adjointFlags, true)) * numel64;
+        const half* adjEncoded = static_cast<const half*>(tmpMemoryAdjoint)
+            + (cooperative ? 0 : static_cast<ptrdiff_t>(storedAdjointChannels(adjointFlags, true)) * numel64);
         // the workspace is the last part of the adjoint memory: everything in front of it
         size_t offset = static_cast<size_t>(ak.perEntryAdjointMemoryBytes) * static_cast<size_t>(numel64);
-        if (hasNetworkGradients) offset += static_cast<size_t>(weightUpdateSlices(numTiles)) * numParameters_ * sizeof(float);
+        if (hasNetworkGradients) offset += static_cast<size_t>(partialSliceCount) * numParameters_ * sizeof(float);
         offset += roundUp(transposedHalves * sizeof(half), size_t(16));
         char* workspace = static_cast<char*>(tmpMemoryAdjoint) + roundUp(offset, size_t(256));
         auto inputAcc = sortedInput;
@@ -2341,7 +2592,7 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
         ensureStreams();
         QMLP_HIP_CALL(qmlp_hip_event_record(adjointEvent_, stream));
     }
-    const int slices = weightUpdateSlices(numTiles);
+    const int slices = partialSliceCount;
     float* partial = reinterpret_cast<float*>(static_cast<char*>(tmpMemoryAdjoint)
                                               + static_cast<size_t>(ak.perEntryAdjointMemoryBytes) * static_cast<size_t>(numel64));
     for (size_t layer = 0; layer < layers_.size(); ++layer) {
@@ -2385,7 +2636,8 @@ void FusedNetwork::clearCachedKernels()
     for (int i = 0; i < ADJOINT_MODE_MAX_COMBINATIONS; ++i)
         for (auto& perSlices : backwardKernel_[i])
             for (auto& k : perSlices) k = {};
-    for (auto& perFlags : recomputeVerdict_) perFlags[0] = perFlags[1] = -1;
+    for (auto& perFlags : recomputeVerdict_)
+        for (auto& perSlices : perFlags) std::fill(std::begin(perSlices), std::end(perSlices), -1);
     pointOrder_.scan = {};
     pointOrder_.count = {};
     pointOrder_.scatter = {};
