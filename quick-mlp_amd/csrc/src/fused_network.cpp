@@ -386,9 +386,11 @@ int FusedNetwork::cooperativeRegisters(int waves, int registerWeight) const
 
 int FusedNetwork::cooperativeSlices(int numTiles) const
 {
-    // one per workgroup, four workgroups per compute unit at most
+    // One per workgroup: two of them per compute unit, up to four where a lane holds so little that more wavefronts find room.
     const CooperativeLayout& layout = cooperativeLayout();
-    return std::max(1, std::min(divUp(2 * numTiles, layout.blockSize / WARP_SIZE), 2 * MAX_WEIGHT_UPDATE_SLICES));
+    const int waves = layout.blockSize / WARP_SIZE;
+    const int perComputeUnit = cooperativeRegisters(waves, layout.registerWeight) <= 100 ? 4 : 2;
+    return std::max(1, std::min(divUp(2 * numTiles, waves), perComputeUnit * (MAX_WEIGHT_UPDATE_SLICES / 2)));
 }
 
 bool FusedNetwork::storesDerivatives(int numel, int flags) const
