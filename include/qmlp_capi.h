@@ -160,6 +160,12 @@ int qmlp_encoding_forward(qmlp_encoding_t encoding, const qmlp_tensor* input, co
 int qmlp_encoding_adjoint(qmlp_encoding_t encoding, const qmlp_tensor* input, const qmlp_tensor* adj_output,
                           const qmlp_tensor* adj_input, void* stream, const qmlp_tensor* parameters_forward,
                           const qmlp_tensor* parameters_gradients, int adjoint_mode);
+/* Temporary device memory with which an adjoint pass of so many points is fastest (0: it needs none), and the adjoint
+ * pass with it (at a multiple of 256 bytes, the call's own until its kernels have run; NULL: as qmlp_encoding_adjoint). */
+int qmlp_encoding_adjoint_memory(qmlp_encoding_t encoding, long long points, int adjoint_mode, size_t* bytes);
+int qmlp_encoding_adjoint_in(qmlp_encoding_t encoding, const qmlp_tensor* input, const qmlp_tensor* adj_output,
+                             const qmlp_tensor* adj_input, void* stream, const qmlp_tensor* parameters_forward,
+                             const qmlp_tensor* parameters_gradients, int adjoint_mode, void* memory);
 /* Compiles the standalone kernels (forward, and the adjoint of adjoint_mode if > 0) into the
  * kernel cache without a GPU. No counterpart in the reference, which compiles lazily inside
  * forward()/adjoint() (src_cpp/src/iencoding.cpp:30-43,98-112). */

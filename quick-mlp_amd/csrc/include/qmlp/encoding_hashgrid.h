@@ -72,8 +72,9 @@ public:
     [[nodiscard]] Tensor::Precision parameterPrecision(Tensor::Usage usage) const override;
     [[nodiscard]] int parameterCount() const override;
     [[nodiscard]] int ldsGradientFloats(int maxBytes, int& levels) const override;
-    [[nodiscard]] bool gradientSlices(GradientSliceLayout& layout) const override;
+    [[nodiscard]] bool gradientSlices(GradientSliceLayout& layout, bool floatAdjoints) const override;
     [[nodiscard]] bool gradientColumns(const kernel::PointOrderKey& key, GradientColumnLayout& layout) const override;
+    [[nodiscard]] int levelGroups() const override;
     [[nodiscard]] int numSweptTables() const override { return numLevels_; }
     [[nodiscard]] int gatherRegistersPerPoint() const override;
     [[nodiscard]] bool pointOrderKey(kernel::PointOrderKey& key, long long numPoints = 0) const override;

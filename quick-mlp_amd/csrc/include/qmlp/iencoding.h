@@ -121,6 +121,9 @@ public:
     /** Output channels that the device code writes together (the features of a grid entry). */
     [[nodiscard]] virtual int channelsWrittenTogether() const { return 1; }
 
+    /** Workgroups of the standalone forward kernel that may share out the levels of a point (device function forwardGroup; 1: forward). */
+    [[nodiscard]] virtual int levelGroups() const { return 1; }
+
     /** One work item of GridGradientSlicesKernel (mirrors kernel::GridGradientSlice). */
     struct GradientSlice
     {
@@ -161,6 +164,23 @@ public:
             for (int s : slicesPerLevel) n += s;
             return n;
         }
+        /**
+         * Workgroups of the records kernel over which the levels of a point are shared out. The levels of a batch
+         * without input gradients have nothing in common: eight times as many workgroups, each with an eighth of the
+         * chain of sorts (16 levels, records and slices of 2^14 / 2^15 / 2^16 / 2^17 points with 1 group 87 / 99 / 106 / 126 us,
+         * with 4 groups 55 / 61 / 88 / 125 us, with 8 groups 51 / 66 / 89 / 128 us; no difference from there on).
+         */
+        int levelGroups(bool inputGradients) const { return inputGradients ? 1 : std::min(8, static_cast<int>(slicesPerLevel.size())); }
+        static int recordsGrid(int numel, int points, int groups, int fullGrid)
+        {
+            return groups * std::min(divUp(numel, points), std::max(1, fullGrid / groups));
+        }
+        /** What the records kernel and the slice kernel share: first the fill of the buckets and the largest adjoint, then the records. */
+        size_t cursorBytes() const { return roundUp(static_cast<size_t>(numBuckets() + 1) * sizeof(int), size_t(256)); }
+        size_t workspaceBytes(long long numel) const
+        {
+            return cursorBytes() + roundUp(static_cast<size_t>(totalRecords(numel)) * recordWords * sizeof(uint32_t), size_t(256));
+        }
     };
     /** What the host needs to run the kernels of kernels/grid_gradient_columns.h for an encoding. */
     struct GradientColumnLayout
@@ -185,21 +205,45 @@ public:
     /**
      * Encodings whose parameter gradients can be summed slice by slice in LDS instead of being
      * scattered with global atomics (see kernels/grid_gradient.h) return true and fill in the layout.
+     * \param floatAdjoints the adjoint of the encoded rows is given in floats (standalone), else in halves (fused)
      */
-    [[nodiscard]] virtual bool gradientSlices(GradientSliceLayout& layout) const
+    [[nodiscard]] virtual bool gradientSlices(GradientSliceLayout& layout, bool floatAdjoints = false) const
     {
         (void)layout;
+        (void)floatAdjoints;
         return false;
     }
 
-    /** gradientSlices(), worked out once (asked on every call of a network): nullptr where there are none. */
-    [[nodiscard]] const GradientSliceLayout* sliceLayout() const
+    /** gradientSlices(), worked out once (asked on every call): nullptr where there are none. */
+    [[nodiscard]] const GradientSliceLayout* sliceLayout(bool floatAdjoints = false) const
     {
-        std::call_once(sliceLayoutOnce_, [this] {
+        const int k = floatAdjoints ? 1 : 0;
+        std::call_once(sliceLayoutOnce_[k], [this, k] {
             GradientSliceLayout layout;
-            if (gradientSlices(layout)) sliceLayout_ = std::move(layout);
+            if (gradientSlices(layout, k == 1)) sliceLayout_[k] = std::move(layout);
         });
-        return sliceLayout_.has_value() ? &sliceLayout_.value() : nullptr;
+        return sliceLayout_[k].has_value() ? &sliceLayout_[k].value() : nullptr;
+    }
+
+    /**
+     * Whether the parameter gradients of a batch go through the slice kernels rather than through float atomics.
+     * Below these sizes the two slice kernels cost more than the atomics they save (their work items zero and write
+     * back whole slices whatever the batch). A train step of one dense 4-D level with 8 features at 2^14 / 2^15 / 2^16 /
+     * 2^17 points 0.08 / 0.09 / 0.12 / 0.19 ms with atomics, 0.10 / 0.11 / 0.12 / 0.23 ms by slices. The atomics of a
+     * point grow with the number of levels, the fixed work of the slice kernels with the size of the table: a train
+     * step of a network behind a 16-level hash grid of floats at 2^13 / 2^14 / 2^15 points 111 / 134 / 190 us with atomics,
+     * 103 / 106 / 117 us by slices (with input gradients 157 / 180 / 238 and 146 / 151 / 166 us); the adjoint pass of
+     * that grid alone 38 / 61 / 117 and 46 / 51 / 67 us (with input gradients 76 / 98 / 155 and 91 / 98 / 112 us).
+     * \param manyLevelsMinBatch from which size on grids of 8 levels or more take the slices
+     */
+    static constexpr int SLICE_GRADIENTS_MIN_BATCH = 1 << 16;
+    static constexpr int SLICE_GRADIENTS_MIN_BATCH_STANDALONE = 1 << 14;
+    static constexpr int SLICE_GRADIENTS_MIN_BATCH_TRAIN_STEP = 1 << 13;
+    // (a pass without weight gradients needs no temporary memory for batches below)
+    static constexpr int SLICE_GRADIENTS_MIN_BATCH_NO_WEIGHTS = 1 << 15;
+    [[nodiscard]] static bool slicesPay(const GradientSliceLayout& layout, long long numel, int manyLevelsMinBatch)
+    {
+        return numel >= SLICE_GRADIENTS_MIN_BATCH || (numel >= manyLevelsMinBatch && layout.slicesPerLevel.size() >= 8);
     }
 
     [[nodiscard]] virtual int ldsGradientFloats(int maxBytes, int& levels) const
@@ -224,27 +268,49 @@ public:
         ALL_GRADIENTS = INPUT_GRADIENTS | PARAM_GRADIENTS
     };
 
+    /** Bytes of temporary device memory with which adjoint() is fastest for such a batch (0: it needs none). */
+    [[nodiscard]] size_t adjointMemory(long long numel, int adjointMode) const;
+
     /**
      * Standalone adjoint pass; adjInput (B, Cin) and the parameter gradients are accumulated.
+     * \param tmpMemory adjointMemory() bytes at a multiple of 256, which belong to this call until its kernels have
+     *    run; without them the parameter gradients are scattered with atomics
      */
     virtual void adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& adjInput, stream_t stream,
                          const std::optional<const Tensor>& parametersForward,
                          const std::optional<const Tensor>& parametersGradients,
-                         int adjointMode = AdjointMode::ALL_GRADIENTS);
+                         int adjointMode = AdjointMode::ALL_GRADIENTS, void* tmpMemory = nullptr);
 
     /**
-     * Compiles the standalone forward kernel and, for adjointMode > 0, the adjoint kernel of
+     * Compiles the standalone forward kernel and, for adjointMode > 0, the adjoint kernels of
      * that mode into the kernel cache without loading them; needs no GPU.
      */
     void precompile(int adjointMode = AdjointMode::ALL_GRADIENTS);
 
 private:
-    std::string forwardKernelSource() const;
+    std::string forwardKernelSource(int groups) const;
     std::string adjointKernelSource(int adjointMode) const;
-    std::optional<KernelFunction> forwardKernel_;
+    std::optional<KernelFunction> forwardKernel_[2];   // [1]: by groups of levels
+    // Where the kernel without groups is the faster one, see EncodingForwardKernel.
+    static constexpr long long FORWARD_WHOLE_ROWS_MIN_BATCH = 3 << 14;
     std::optional<KernelFunction> adjointKernel_[AdjointMode::ALL_GRADIENTS + 1];
-    mutable std::once_flag sliceLayoutOnce_;
-    mutable std::optional<GradientSliceLayout> sliceLayout_;
+    mutable std::once_flag sliceLayoutOnce_[2];
+    mutable std::optional<GradientSliceLayout> sliceLayout_[2];
+
+    /** The kernels of kernels/grid_gradient.h for adjoints given in floats. */
+    struct SliceKernels
+    {
+        // GridGradientRecordsKernel without / with input gradients, with pointsPerWorkgroup >> i lanes per workgroup
+        std::vector<std::optional<KernelFunction>> records[2];
+        std::optional<KernelFunction> clear, slices;
+        Tensor items;
+    };
+    SliceKernels sliceKernels_;
+    static int recordsVariants(const GradientSliceLayout& layout);
+    std::optional<KernelFunction> compileRecords(const GradientSliceLayout& layout, bool inputGradients, int variant, int flags) const;
+    std::optional<KernelFunction> compileSlices(const GradientSliceLayout& layout, bool clear, int flags) const;
+    void adjointBySlices(const GradientSliceLayout& layout, const Tensor& input, const Tensor& adjOutput, Tensor& adjInput, stream_t stream,
+                         int adjointMode, void* tmpMemory, char* parameters);
 };
 typedef std::shared_ptr<IEncoding> IEncoding_ptr;
 

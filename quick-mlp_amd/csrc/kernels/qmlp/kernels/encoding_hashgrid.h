@@ -551,6 +551,27 @@ struct EncodingHashGrid
         }
     }
 
+    /** The features of the levels of one of GROUPS groups (concatenated levels), from the group's first feature on. */
+    template <int G, int GROUPS, typename I, typename O>
+    __device__ __forceinline__ static void forwardGroup(int group, const I& input, O& output, const param_t& params)
+    {
+        typedef typename O::ValueType O_t;
+        if (G + 1 == GROUPS || group == G) {
+            float pos[D];
+            unitPosition(input, params, pos);
+            constexpr int FIRST = L * G / GROUPS, END = L * (G + 1) / GROUPS;
+#pragma unroll
+            for (int l = FIRST; l < END; ++l) {
+                float feat[F];
+                gatherLevel(l, pos, params.parametersForward, feat);
+#pragma unroll
+                for (int i = 0; i < F; ++i) output[(l - FIRST) * F + i] = fcast<O_t>(feat[i]);
+            }
+        } else if constexpr (G + 1 < GROUPS) {
+            forwardGroup<G + 1, GROUPS>(group, input, output, params);
+        }
+    }
+
     /**
      * Adjoint: scatters w * adjFeature into the gradient table with hardware fp32
      * atomics and accumulates the analytic multilinear derivative into adjInput.

@@ -9,18 +9,48 @@ $$INCLUDES$$
 
 QUICKMLP_KERNEL_NAMESPACE_BEGIN
 
-__global__ void EncodingForwardKernel(
+/**
+ * One lane per point. The rows of a wavefront's 64 points are put together in LDS and written side by side (a lane that
+ * writes its own row touches one line per value and point; 16 levels of 2 floats, 2^17 points 80 -> 70 us, where the
+ * lines of the gathers bound it).
+ * A grid whose levels stand next to each other in the output may be evaluated by GROUPS times as many workgroups, each
+ * of them a few of the levels: a small batch leaves few wavefronts, each of which waits for one level's entries after the
+ * other's (2^10 / 2^14 / 2^15 / 2^16 / 2^17 points 21 / 30 / 32 / 42 / 70 us, with 8 groups 6.5 / 13 / 23 / 48 / 91 us; the
+ * same with half tables 17 / 30 / 30 / 35 / 49 and 6.4 / 10 / 17 / 33 / 62 us: the rows are then written in pieces).
+ */
+__global__ void __launch_bounds__(256) EncodingForwardKernel(
     long long numel,
     const Tensor2Read<float> inputs,  //shape (numel, Cin)
     Tensor2RW<float> outputs          //shape (numel, Cout), unit stride along the channels
     $$ENCODING_PARAMETERS$$)
 {
-    for (long long index = blockIdx.x * static_cast<long long>(blockDim.x) + threadIdx.x; index < numel;
-         index += static_cast<long long>(blockDim.x) * gridDim.x)
+    constexpr int GROUPS = $$LEVEL_GROUPS$$;
+    constexpr int CHANNELS = $$GROUP_CHANNELS$$;   // of the widest group
+    constexpr bool STAGED = CHANNELS > 1 && CHANNELS <= 62;
+    constexpr int PITCH = CHANNELS | 1;
+    __shared__ float sRows[256 / WAVE_SIZE][STAGED ? TILE_POINTS * PITCH : 1];
+    const int lane = threadIdx.x % WAVE_SIZE;
+    float* rows = sRows[threadIdx.x / WAVE_SIZE];
+    const int group = blockIdx.x % GROUPS;
+    const int firstChannel = $$FIRST_CHANNEL$$, channels = $$CHANNELS$$;   // of this group
+    for (long long tileBase = (blockIdx.x / GROUPS * static_cast<long long>(blockDim.x / WAVE_SIZE) + threadIdx.x / WAVE_SIZE) * TILE_POINTS;
+         tileBase < numel; tileBase += static_cast<long long>(blockDim.x) * (gridDim.x / GROUPS))
     {
-        const StridedArray<const float> encodingInput{inputs.data_ + index * inputs.strides_[0], inputs.strides_[1]};
-        WrappedArray<float> encodingOutput{outputs.data_ + index * outputs.strides_[0]};
-        $$CALL_ENCODINGS_FORWARD$$
+        const long long index = tileBase + lane;
+        if (index < numel) {
+            const StridedArray<const float> encodingInput{inputs.data_ + index * inputs.strides_[0], inputs.strides_[1]};
+            WrappedArray<float> encodingOutput{STAGED ? rows + lane * PITCH : outputs.data_ + index * outputs.strides_[0] + firstChannel};
+            $$CALL_ENCODINGS_FORWARD$$
+        }
+        if constexpr (STAGED) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const int points = static_cast<int>(min(numel - tileBase, static_cast<long long>(TILE_POINTS)));
+            for (int i = lane; i < points * CHANNELS; i += WAVE_SIZE) {
+                const int row = i / CHANNELS, channel = i % CHANNELS;
+                if (channel < channels) outputs.data_[(tileBase + row) * outputs.strides_[0] + firstChannel + channel] = rows[row * PITCH + channel];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
     }
 }
 

@@ -36,6 +36,10 @@
 // records, such that no sum can overflow: at least 37 bits remain below the largest possible
 // contribution at 2^24 records, and the sums do not depend on the order of the additions. Batches whose
 // adjoints are not finite take the float additions, so that NaN and infinity reach the gradients. Weights
+// The adjoint pass of a standalone encoding gives its adjoints in floats. Its records hold floats (GridGradientLayout),
+// the scale of a sum goes by the records of its work item, and a value that would still lose bits in it (floats span
+// more than 64 bits) goes to the gradient tensor with an atomic: 3 of 10^5 in a batch of normally distributed adjoints
+// (16 levels of 2^19 entries of 2 floats, 2^17 points: 458 us with atomics, 81 + 53 us; 2^14 points 61 -> 51 us). Weights
 // are at most one for points inside the box; the records of points outside of it (extrapolated with weights
 // beyond one, or NaN for a NaN coordinate) are added to the gradient tensor by the records kernel itself.
 // Two forms that were measured and dropped: a workgroup per slice that tests every point of
@@ -67,7 +71,33 @@ struct GridGradientSlice
     int reserved1;
 };
 
-template <typename Cfg, int SLICE_FLOATS>
+/**
+ * Where the records kernel finds the adjoints of the encoded rows. The fused backward kernels leave them as halves, tile
+ * by tile of 64 points with the ROW_CHANNELS values of a row 64 apart; the adjoint pass of a standalone encoding is
+ * given rows of floats with strides (ROW_CHANNELS == 0), and its records then hold floats.
+ */
+template <int ROW_CHANNELS>
+struct GridGradientAdjoints
+{
+    const half* __restrict__ data;   //(tiles, ROW_CHANNELS, 64)
+    __device__ __forceinline__ f16 operator()(int p, int channel) const
+    {
+        return reinterpret_cast<const f16*>(data)[static_cast<long long>(p / TILE_POINTS) * (ROW_CHANNELS * TILE_POINTS)
+                                                  + channel * TILE_POINTS + p % TILE_POINTS];
+    }
+};
+template <>
+struct GridGradientAdjoints<0>
+{
+    Tensor2Read<float> rows;         //(points, channels)
+    __device__ __forceinline__ float operator()(int p, int channel) const
+    {
+        return rows.data_[static_cast<long long>(p) * rows.strides_[0] + static_cast<long long>(channel) * rows.strides_[1]];
+    }
+};
+
+/** \tparam FLOATS the adjoints are floats, else halves */
+template <typename Cfg, int SLICE_FLOATS, bool FLOATS = false>
 struct GridGradientLayout
 {
     typedef EncodingHashGrid<Cfg> Grid;
@@ -77,10 +107,32 @@ struct GridGradientLayout
     static constexpr int PAIRS = Grid::NC / 2 > 0 ? Grid::NC / 2 : 1;
     /** A record in 32-bit words: the offsets of the lower and of the upper entry within the slice (16 bits
      *  each), their two weights, F halves of adjoint; one word of padding where that makes it a multiple of
-     *  16 bytes (records of 16 or 32 bytes move as whole vector loads and stores). */
-    static constexpr int RECORD_WORDS_USED = 3 + (F + 1) / 2;
+     *  16 bytes (records of 16 or 32 bytes move as whole vector loads and stores). With adjoints that are floats:
+     *  the offsets, the share of the upper entry, F products of adjoint and weight of the pair, so that the
+     *  records of 2 features take 16 bytes as well. */
+    static constexpr int ADJOINT_WORDS = FLOATS ? F : (F + 1) / 2;
+    static constexpr int FIRST_ADJOINT = FLOATS ? 2 : 3;
+    static constexpr int RECORD_WORDS_USED = FIRST_ADJOINT + ADJOINT_WORDS;
     static constexpr int RECORD_WORDS = RECORD_WORDS_USED % 4 == 3 ? RECORD_WORDS_USED + 1 : RECORD_WORDS_USED;
     static_assert(SLICE_FLOATS <= 65536, "offsets within a slice are stored in 16 bits");
+
+    /** Value i among the adjoint words. */
+    __device__ __forceinline__ static float adjoint(const unsigned* words, int i)
+    {
+        if constexpr (FLOATS) return __builtin_bit_cast(float, words[i]);
+        else return static_cast<float>(__builtin_bit_cast(f16, static_cast<unsigned short>(words[i / 2] >> (16 * (i % 2)))));
+    }
+    /** What a record adds to its lower and to its upper entry, as a multiple of its adjoint values. */
+    __device__ __forceinline__ static void weights(const unsigned* record, float& wL, float& wH)
+    {
+        if constexpr (FLOATS) {
+            wH = __builtin_bit_cast(float, record[1]);
+            wL = 1.f - wH;
+        } else {
+            wL = __builtin_bit_cast(float, record[1]);
+            wH = __builtin_bit_cast(float, record[2]);
+        }
+    }
 
     /** Records start at multiples of their size from a 16-byte aligned base (LDS or global memory). */
     template <typename Pointer>
@@ -149,9 +201,12 @@ __device__ __forceinline__ void ldsBarrier()
 template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS, int POINTS>
 struct GridGradientRecords
 {
-    typedef GridGradientLayout<Cfg, SLICE_FLOATS> Layout;
+    static constexpr bool FLOATS = ROW_CHANNELS == 0;
+    typedef GridGradientLayout<Cfg, SLICE_FLOATS, FLOATS> Layout;
+    typedef GridGradientAdjoints<ROW_CHANNELS> Adjoints;
     typedef EncodingHashGrid<Cfg> Grid;
     typedef typename Grid::param_t param_t;
+    static constexpr int AW = Layout::ADJOINT_WORDS;
     static constexpr int D = Grid::D;
     static constexpr int F = Grid::F;
     static constexpr int PAIRS = Layout::PAIRS;
@@ -270,13 +325,10 @@ struct GridGradientRecords
     struct AddToTensor
     {
         float* __restrict__ gradients;
-        __device__ __forceinline__ void operator()(unsigned element, float weight, const unsigned (&adjWords)[(F + 1) / 2]) const
+        __device__ __forceinline__ void operator()(unsigned element, float weight, const unsigned (&adjWords)[AW]) const
         {
 #pragma unroll
-            for (int i = 0; i < F; ++i) {
-                const unsigned short bits = static_cast<unsigned short>(adjWords[i / 2] >> (16 * (i % 2)));
-                unsafeAtomicAdd(gradients + element + i, weight * static_cast<float>(__builtin_bit_cast(f16, bits)));
-            }
+            for (int i = 0; i < F; ++i) unsafeAtomicAdd(gradients + element + i, weight * Layout::adjoint(adjWords, i));
         }
     };
 
@@ -289,7 +341,7 @@ struct GridGradientRecords
      */
     template <int LEVEL, typename OtherSlice>
     __device__ __forceinline__ static int buildRecord(const typename Grid::LevelSetup& s, int c,
-                                                      const unsigned (&adjWords)[(F + 1) / 2], unsigned (&rec)[RW],
+                                                      const unsigned (&adjWords)[AW], unsigned (&rec)[RW],
                                                       const OtherSlice& otherSlice)
     {
         constexpr int PD = Cfg::hashed[LEVEL] ? 0 : D - 1;
@@ -309,10 +361,19 @@ struct GridGradientRecords
             wH = 0.f;
         }
         rec[0] = eL | (eH << 16);
-        rec[1] = __builtin_bit_cast(unsigned, wL);
-        rec[2] = __builtin_bit_cast(unsigned, wH);
+        if constexpr (FLOATS) {
+            // (without an upper entry the lower one takes all of it: its own weight then goes into the products)
+            const bool lowerOnly = eH == eL && wH == 0.f;
+            rec[1] = lowerOnly ? 0u : __builtin_bit_cast(unsigned, s.f[PD]);
 #pragma unroll
-        for (int i = 0; i < (F + 1) / 2; ++i) rec[3 + i] = adjWords[i];
+            for (int i = 0; i < F; ++i)
+                rec[2 + i] = __builtin_bit_cast(unsigned, (lowerOnly ? wL : w) * Layout::adjoint(adjWords, i));
+        } else {
+            rec[1] = __builtin_bit_cast(unsigned, wL);
+            rec[2] = __builtin_bit_cast(unsigned, wH);
+#pragma unroll
+            for (int i = 0; i < AW; ++i) rec[3 + i] = adjWords[i];
+        }
 #pragma unroll
         for (int v = Layout::RECORD_WORDS_USED; v < RW; ++v) rec[v] = 0u;
         return bucket;
@@ -321,20 +382,24 @@ struct GridGradientRecords
     /** Adds a record to the gradient tensor itself (its bucket was full); grad: element 0 of the record's slice. */
     __device__ __forceinline__ static void addToTensor(const unsigned (&rec)[RW], float* __restrict__ grad)
     {
-        const float wL = __builtin_bit_cast(float, rec[1]), wH = __builtin_bit_cast(float, rec[2]);
+        float wL, wH;
+        Layout::weights(rec, wL, wH);
         const unsigned eL = rec[0] & 0xffffu, eH = rec[0] >> 16;
 #pragma unroll
         for (int i = 0; i < F; ++i) {
-            const unsigned short bits = static_cast<unsigned short>(rec[3 + i / 2] >> (16 * (i % 2)));
-            const float adj = static_cast<float>(__builtin_bit_cast(f16, bits));
+            const float adj = Layout::adjoint(rec + Layout::FIRST_ADJOINT, i);
             unsafeAtomicAdd(grad + eL + i, wL * adj);
             if (wH != 0.f) unsafeAtomicAdd(grad + eH + i, wH * adj);
         }
     }
 
+    /** Feature i of a level among the channels of the encoded rows. */
+    template <int LEVEL>
+    __device__ __forceinline__ static constexpr int channel(int i) { return CHANNEL_OFFSET + (Cfg::Concat ? LEVEL * F : 0) + i; }
+
     template <int LEVEL, int INPUT_GRADIENTS>
     __device__ __forceinline__ static void runLevel(int p, bool valid, long long numel, const float (&pos)[D],
-                                                    const f16* __restrict__ adjEncoded, const param_t& params,
+                                                    const Adjoints& adjEncoded, const param_t& params,
                                                     unsigned* __restrict__ records, int* __restrict__ cursors,
                                                     unsigned* sStage, unsigned short* sBucketOf, int* sHist,
                                                     int* sLocalBase, long long* sGlobalBase, unsigned& maxAdjBits,
@@ -356,17 +421,20 @@ struct GridGradientRecords
         detail::HeldFeatures<F, typename Cfg::table_t> held[Grid::NC];
         (void)held;
         if (valid) {
-            const f16* adjRow = adjEncoded + static_cast<long long>(p / TILE_POINTS) * (ROW_CHANNELS * TILE_POINTS)
-                + (CHANNEL_OFFSET + (Cfg::Concat ? LEVEL * F : 0)) * TILE_POINTS + (p % TILE_POINTS);
-            unsigned adjWords[(F + 1) / 2];
+            unsigned adjWords[AW];
 #pragma unroll
-            for (int i = 0; i < (F + 1) / 2; ++i) adjWords[i] = 0u;
+            for (int i = 0; i < AW; ++i) adjWords[i] = 0u;
 #pragma unroll
             for (int i = 0; i < F; ++i) {
-                const unsigned bits = __builtin_bit_cast(unsigned short, adjRow[i * TILE_POINTS]);
-                adjWords[i / 2] |= bits << (16 * (i % 2));
-                // largest magnitude seen (as fp16 bits without the sign: ordered like the values, NaN above infinity)
-                maxAdjBits = max(maxAdjBits, bits & 0x7fffu);
+                // largest magnitude seen (as bits without the sign: ordered like the values, NaN above infinity)
+                if constexpr (FLOATS) {
+                    adjWords[i] = __builtin_bit_cast(unsigned, adjEncoded(p, channel<LEVEL>(i)));
+                    maxAdjBits = max(maxAdjBits, adjWords[i] & 0x7fffffffu);
+                } else {
+                    const unsigned bits = __builtin_bit_cast(unsigned short, adjEncoded(p, channel<LEVEL>(i)));
+                    adjWords[i / 2] |= bits << (16 * (i % 2));
+                    maxAdjBits = max(maxAdjBits, bits & 0x7fffu);
+                }
             }
             if constexpr (INPUT_GRADIENTS == 1 && !DEFER_ENTRIES) {
                 // the entries of all corners, for this grid's share of dL/dinput (a dense 4-D grid with 8 features
@@ -403,15 +471,15 @@ struct GridGradientRecords
                     const bool upperAdded = idxH * F - sliceStart >= static_cast<unsigned>(SLICE_FLOATS);
 #pragma unroll 1
                     for (int i = 0; i < F; ++i) {
-                        const float adj = static_cast<float>(adjRow[i * TILE_POINTS]);
+                        const float adj = static_cast<float>(adjEncoded(p, channel<LEVEL>(i)));
                         unsafeAtomicAdd(grad + idxL * F + i, wL * adj);
                         if (!upperAdded) unsafeAtomicAdd(grad + idxH * F + i, wH * adj);
                     }
                 }
 #pragma unroll
                 for (int c = 0; c < PAIRS; ++c) {
-                    rec[c][1] = 0u;
-                    rec[c][2] = 0u;
+#pragma unroll
+                    for (int v = 1; v < (FLOATS ? 2 + F : 3); ++v) rec[c][v] = 0u;
                 }
             }
         } else {
@@ -497,10 +565,8 @@ struct GridGradientRecords
      */
     template <int LEVEL>
     __device__ __forceinline__ static void positionGradientFromDerivatives(int p, const DerivativeChunk* __restrict__ derivatives,
-                                                                           const f16* __restrict__ adjEncoded, float (&adjPos)[D])
+                                                                           const Adjoints& adjEncoded, float (&adjPos)[D])
     {
-        const f16* adjRow = adjEncoded + static_cast<long long>(p / TILE_POINTS) * (ROW_CHANNELS * TILE_POINTS)
-            + (CHANNEL_OFFSET + (Cfg::Concat ? LEVEL * F : 0)) * TILE_POINTS + (p % TILE_POINTS);
         float values[DerivativeLayout::VALUES];
         DerivativeLayout::load(derivatives + DerivativeLayout::chunkIndex(p / TILE_POINTS, 0, 0, p % TILE_POINTS), LEVEL, values);
         float lvl[D];
@@ -508,7 +574,7 @@ struct GridGradientRecords
         for (int d = 0; d < D; ++d) lvl[d] = 0.f;
 #pragma unroll
         for (int i = 0; i < F; ++i) {
-            const float adj = static_cast<float>(adjRow[i * TILE_POINTS]);
+            const float adj = static_cast<float>(adjEncoded(p, channel<LEVEL>(i)));
 #pragma unroll
             for (int d = 0; d < D; ++d) lvl[d] += adj * values[i * D + d];
         }
@@ -527,13 +593,11 @@ struct GridGradientRecords
     template <int LEVEL>
     __device__ __forceinline__ static void positionGradient(int p, const typename Grid::LevelSetup& s,
                                                             const detail::HeldFeatures<F, typename Cfg::table_t> (&held)[Grid::NC],
-                                                            const f16* __restrict__ adjEncoded, float (&adjPos)[D])
+                                                            const Adjoints& adjEncoded, float (&adjPos)[D])
     {
-        const f16* adjRow = adjEncoded + static_cast<long long>(p / TILE_POINTS) * (ROW_CHANNELS * TILE_POINTS)
-            + (CHANNEL_OFFSET + (Cfg::Concat ? LEVEL * F : 0)) * TILE_POINTS + (p % TILE_POINTS);
         float adjFeat[F];
 #pragma unroll
-        for (int i = 0; i < F; ++i) adjFeat[i] = static_cast<float>(adjRow[i * TILE_POINTS]);
+        for (int i = 0; i < F; ++i) adjFeat[i] = static_cast<float>(adjEncoded(p, channel<LEVEL>(i)));
         positionGradient<LEVEL>(s, held, adjFeat, adjPos);
     }
 
@@ -567,34 +631,50 @@ struct GridGradientRecords
         for (int d = 0; d < D; ++d) adjPos[d] += scale * lvl[d];
     }
 
-    template <int LEVEL, int INPUT_GRADIENTS>
+    /** The levels from LEVEL to END - 1. */
+    template <int LEVEL, int END, int INPUT_GRADIENTS>
     __device__ __forceinline__ static void runLevels(int p, bool valid, long long numel, const float (&pos)[D],
-                                                     const f16* __restrict__ adjEncoded, const param_t& params,
+                                                     const Adjoints& adjEncoded, const param_t& params,
                                                      unsigned* __restrict__ records, int* __restrict__ cursors,
                                                      unsigned* sStage, unsigned short* sBucketOf, int* sHist,
                                                      int* sLocalBase, long long* sGlobalBase, unsigned& maxAdjBits,
                                                      float (&adjPos)[D], const DerivativeChunk* __restrict__ derivatives)
     {
-        if constexpr (LEVEL < Cfg::Levels) {
+        if constexpr (LEVEL < END) {
             runLevel<LEVEL, INPUT_GRADIENTS>(p, valid, numel, pos, adjEncoded, params, records, cursors, sStage, sBucketOf, sHist,
                                              sLocalBase, sGlobalBase, maxAdjBits, adjPos, derivatives);
-            runLevels<LEVEL + 1, INPUT_GRADIENTS>(p, valid, numel, pos, adjEncoded, params, records, cursors, sStage, sBucketOf,
+            runLevels<LEVEL + 1, END, INPUT_GRADIENTS>(p, valid, numel, pos, adjEncoded, params, records, cursors, sStage, sBucketOf,
                                                   sHist, sLocalBase, sGlobalBase, maxAdjBits, adjPos, derivatives);
+        }
+    }
+
+    /** The levels of one of GROUPS groups. */
+    template <int G, int GROUPS, int INPUT_GRADIENTS, typename... Args>
+    __device__ __forceinline__ static void runGroup(int group, Args&&... args)
+    {
+        if constexpr (G + 1 < GROUPS) {
+            if (group == G) runLevels<Cfg::Levels * G / GROUPS, Cfg::Levels * (G + 1) / GROUPS, INPUT_GRADIENTS>(args...);
+            else runGroup<G + 1, GROUPS, INPUT_GRADIENTS>(group, args...);
+        } else {
+            runLevels<Cfg::Levels * G / GROUPS, Cfg::Levels, INPUT_GRADIENTS>(args...);
         }
     }
 };
 
 /**
+ * \tparam GROUPS the levels are shared out over so many workgroups (the grid is a multiple of it) where each of them
+ *    needs nothing of the others (no input gradients)
  * \tparam POINTS points (= lanes) of a workgroup; its records of one level are staged in LDS
  * records: room for levelOffset(Levels, layoutNumel) records; cursors: one int per bucket, then one word that
- * receives the largest magnitude among the adjoints (fp16 bits without the sign); all zeroed by the caller.
+ * receives the largest magnitude among the adjoints (bits without the sign); all zeroed by the caller.
+ * \tparam ROW_CHANNELS, CHANNEL_OFFSET where the adjoints of this grid lie, see GridGradientAdjoints
  */
-template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS, int POINTS, int INPUT_GRADIENTS>
+template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS, int POINTS, int INPUT_GRADIENTS, int GROUPS>
 __global__ void __launch_bounds__(POINTS) GridGradientRecordsKernel(
     int numel,
     int layoutNumel,                          //points the buckets are laid out for (numel rounded up to whole tiles)
     const Tensor2Read<float> inputs,          //shape (numel, Cin)
-    const half* __restrict__ adjEncodedH,     //adjoint of the encoded rows: (tiles, ROW_CHANNELS, 64)
+    const GridGradientAdjoints<ROW_CHANNELS> adjEncoded,
     const HashGridParams<typename Cfg::table_t, Cfg::Dim> params,
     unsigned* __restrict__ records, int* __restrict__ cursors,
     Tensor2RW<float> adjInputs,               //INPUT_GRADIENTS: shape (numel, Cin), this grid's share of dL/dinput is added
@@ -609,7 +689,8 @@ __global__ void __launch_bounds__(POINTS) GridGradientRecordsKernel(
     int* sLocalBase = sHist + Impl::MAX_SLICES;
     unsigned short* sBucketOf = reinterpret_cast<unsigned short*>(sLocalBase + Impl::MAX_SLICES + 1);
     unsigned maxAdjBits = 0u;
-    for (int chunk = blockIdx.x * POINTS; chunk < numel; chunk += gridDim.x * POINTS) {
+    const int group = blockIdx.x % GROUPS;
+    for (int chunk = blockIdx.x / GROUPS * POINTS; chunk < numel; chunk += gridDim.x / GROUPS * POINTS) {
         const int p = chunk + threadIdx.x;
         const bool valid = p < numel;
         float pos[D];
@@ -625,7 +706,7 @@ __global__ void __launch_bounds__(POINTS) GridGradientRecordsKernel(
         float adjPos[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) adjPos[d] = 0.f;
-        Impl::template runLevels<0, INPUT_GRADIENTS>(p, valid, layoutNumel, pos, reinterpret_cast<const f16*>(adjEncodedH), params,
+        Impl::template runGroup<0, GROUPS, INPUT_GRADIENTS>(group, p, valid, layoutNumel, pos, adjEncoded, params,
                                                      records, cursors, sStage, sBucketOf, sHist, sLocalBase, sGlobalBase, maxAdjBits,
                                                      adjPos, static_cast<const typename Impl::DerivativeChunk*>(derivativesV));
         if constexpr (INPUT_GRADIENTS != 0) {
@@ -645,7 +726,14 @@ __global__ void __launch_bounds__(POINTS) GridGradientRecordsKernel(
     if (maxAdjBits != 0u) atomicMax(sHist, static_cast<int>(maxAdjBits));
     __syncthreads();
     if (threadIdx.x == 0 && sHist[0] != 0)
-        atomicMax(cursors + GridGradientLayout<Cfg, SLICE_FLOATS>::firstBucket(Cfg::Levels), sHist[0]);
+        atomicMax(cursors + Impl::Layout::firstBucket(Cfg::Levels), sHist[0]);
+}
+
+/** Zeroes the fill of the buckets and the largest adjoint. */
+__global__ void __launch_bounds__(256) GridGradientClearKernel(int* __restrict__ words, int count)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < count) words[i] = 0;
 }
 
 template <typename Cfg, int SLICE_FLOATS, int LEVEL>
@@ -715,10 +803,10 @@ __global__ void __launch_bounds__(256) GridGradientTraceKernel(
     }
 }
 
-template <typename Cfg, int SLICE_FLOATS>
+template <typename Cfg, int SLICE_FLOATS, bool FLOATS>
 struct GridGradientSlices
 {
-    typedef GridGradientLayout<Cfg, SLICE_FLOATS> Layout;
+    typedef GridGradientLayout<Cfg, SLICE_FLOATS, FLOATS> Layout;
     typedef EncodingHashGrid<Cfg> Grid;
     static constexpr int F = Grid::F;
     static constexpr int RW = Layout::RECORD_WORDS;
@@ -727,6 +815,14 @@ struct GridGradientSlices
     /** v * 2^scaleExponent as a 64-bit integer, rounded towards minus infinity in the low word (|v * 2^scaleExponent| < 2^62). */
     __device__ __forceinline__ static long long toFixed(float v, int scaleExponent)
     {
+        if constexpr (FLOATS) {
+            // by magnitude: no bit of a float of 2^23 units or more is lost
+            const float magnitude = ldexpf(fabsf(v), scaleExponent - 32);
+            const float whole = floorf(magnitude);
+            const long long fixed = (static_cast<long long>(static_cast<int>(whole)) << 32)
+                + static_cast<long long>(static_cast<unsigned>(ldexpf(magnitude - whole, 32)));
+            return v < 0.f ? -fixed : fixed;
+        }
         const float x = ldexpf(v, scaleExponent - 32);             // in units of 2^32
         const float hi = floorf(x);
         // the low bits of a 24-bit mantissa: exact, in [0, 2^32) (a tiny negative x gives hi = -1 and x - hi = 1 after rounding)
@@ -738,6 +834,13 @@ struct GridGradientSlices
     {
         typedef __attribute__((address_space(3))) unsigned long long lds_u64;
         __hip_atomic_fetch_add((lds_u64*)p, static_cast<unsigned long long>(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+
+    /** Floats span more than the 64 bits of a sum: a value of which the sum would lose bits goes to the gradient tensor. */
+    __device__ __forceinline__ static void addFixedOrSmall(long long* sum, float* __restrict__ gradient, float v, int scaleExponent, float smallest)
+    {
+        if (fabsf(v) >= smallest) ldsAddFixed(sum, toFixed(v, scaleExponent));
+        else if (v != 0.f) unsafeAtomicAdd(gradient, v);
     }
 
     /** FIXED: 64-bit fixed-point sums (the slice is SLICE_FLOATS long long); else float sums. */
@@ -753,6 +856,9 @@ struct GridGradientSlices
         const long long begin = filled * item.part / item.parts, end = filled * (item.part + 1) / item.parts;
         const unsigned* bucket = records + (Layout::levelOffset(LEVEL, numel) + static_cast<long long>(item.slice) * capacity) * RW;
         constexpr int UNROLL = 4;
+        // (the smallest magnitude of which the fixed-point sums keep all bits of a float)
+        const float smallest = ldexpf(1.f, 23 - scaleExponent);
+        (void)smallest;
         for (long long j0 = begin + tid; j0 < end; j0 += UNROLL * BLOCK) {
             unsigned rec[UNROLL][RW];
 #pragma unroll
@@ -769,19 +875,24 @@ struct GridGradientSlices
             for (int u = 0; u < UNROLL; ++u) {
                 if (j0 + u * BLOCK >= end) continue;
                 const unsigned eL = rec[u][0] & 0xffffu, eH = rec[u][0] >> 16;   // both inside this slice
-                const float wL = __builtin_bit_cast(float, rec[u][1]), wH = __builtin_bit_cast(float, rec[u][2]);
+                float wL, wH;
+                Layout::weights(rec[u], wL, wH);
 #pragma unroll
                 for (int step = 0; step < F; ++step) {
                     // Neighbouring lanes take the features in rotated order: an entry starts at a multiple of
                     // 8 * F bytes, so lanes that all add feature `step` meet on a few LDS banks (measured on a
                     // dense grid with 8 features: conflicts 90 % of the LDS cycles of this kernel).
                     const int i = (F & (F - 1)) == 0 ? ((step + tid) & (F - 1)) : ((step + tid % F) % F);
-                    unsigned word = rec[u][3];
+                    unsigned word = rec[u][Layout::FIRST_ADJOINT];
+                    const int at = FLOATS ? i : i >> 1;
 #pragma unroll
-                    for (int w = 1; w < (F + 1) / 2; ++w) word = (i >> 1) == w ? rec[u][3 + w] : word;
-                    const unsigned short bits = static_cast<unsigned short>(word >> (16 * (i & 1)));
-                    const float adj = static_cast<float>(__builtin_bit_cast(f16, bits));
-                    if constexpr (FIXED) {
+                    for (int w = 1; w < Layout::ADJOINT_WORDS; ++w) word = at == w ? rec[u][Layout::FIRST_ADJOINT + w] : word;
+                    const float adj = FLOATS ? __builtin_bit_cast(float, word)
+                        : static_cast<float>(__builtin_bit_cast(f16, static_cast<unsigned short>(word >> (16 * (i & 1)))));
+                    if constexpr (FIXED && FLOATS) {
+                        addFixedOrSmall(sFixed + eL + i, gradients + item.first + eL + i, wL * adj, scaleExponent, smallest);
+                        addFixedOrSmall(sFixed + eH + i, gradients + item.first + eH + i, wH * adj, scaleExponent, smallest);
+                    } else if constexpr (FIXED) {
                         ldsAddFixed(sFixed + eL + i, toFixed(wL * adj, scaleExponent));
                         ldsAddFixed(sFixed + eH + i, toFixed(wH * adj, scaleExponent));
                     } else {
@@ -791,6 +902,20 @@ struct GridGradientSlices
                 }
             }
         }
+    }
+
+    /**
+     * Terms of at most the largest adjoint that one sum may take. Halves: those of the whole batch, so that a slice
+     * gives the same bits however its bucket is split. Floats need the bits below more: the records of this work item
+     * (the two weights of a record make at most one).
+     */
+    template <int LEVEL>
+    __device__ __forceinline__ static unsigned long long termsOf(long long numel, const int* __restrict__ cursors, const GridGradientSlice item)
+    {
+        if constexpr (FLOATS)
+            return static_cast<unsigned long long>(min(static_cast<long long>(cursors[Layout::firstBucket(LEVEL) + item.slice]),
+                                                       Layout::capacity(LEVEL, numel)) / item.parts + 1);
+        else return static_cast<unsigned long long>(2 * Layout::PAIRS) * static_cast<unsigned long long>(numel);
     }
 
     template <int LEVEL>
@@ -804,13 +929,15 @@ struct GridGradientSlices
         // |adjoint| < 2^maxExponent; a sum has at most 2 * PAIRS * numel terms, each at most that large (weights <= 1)
         const unsigned maxBits = static_cast<unsigned>(cursors[Layout::firstBucket(Cfg::Levels)]);
         if (maxBits == 0u) return;   // all adjoints are zero: nothing to add
-        const bool finite = maxBits < 0x7c00u;
-        const int maxExponent = static_cast<int>(maxBits >> 10) - 14;          // fp16: value < 2^(biased exponent - 14), subnormals included
-        const int termsLog2 = 64 - __builtin_clzll(static_cast<unsigned long long>(2 * Layout::PAIRS) * static_cast<unsigned long long>(numel));
+        const bool finite = maxBits < (FLOATS ? 0x7f800000u : 0x7c00u);
+        // value < 2^(biased exponent - 14) of halves, 2^(biased exponent - 126) of floats, subnormals included
+        const int maxExponent = FLOATS ? static_cast<int>(maxBits >> 23) - 126 : static_cast<int>(maxBits >> 10) - 14;
+        const int termsLog2 = 64 - __builtin_clzll(termsOf<LEVEL>(numel, cursors, item));
         const int scaleExponent = 61 - maxExponent - termsLog2;
         float* sFloat = reinterpret_cast<float*>(sSlice);
         if (finite) sumRecords<LEVEL, true>(numel, records, cursors, gradients, item, sSlice, sFloat, scaleExponent);
         else sumRecords<LEVEL, false>(numel, records, cursors, gradients, item, sSlice, sFloat, 0);
+        if constexpr (FLOATS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's atomics have been carried out
         __syncthreads();
         // Added to the gradient tensor: with atomics (16 neighbouring floats per request) where other work
         // items hold sums for the same slice (parts > 1), else this workgroup is the only writer of its
@@ -825,8 +952,14 @@ struct GridGradientSlices
                 v = sFloat[i];
             }
             if (v != 0.f) {
-                if (item.parts > 1) unsafeAtomicAdd(grad + i, v);
-                else grad[i] += v;
+                if (item.parts > 1) {
+                    unsafeAtomicAdd(grad + i, v);
+                } else if constexpr (FLOATS) {
+                    // (read behind this workgroup's own atomics: they have ended, but the L1 does not know of them)
+                    grad[i] = __hip_atomic_load(grad + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + v;
+                } else {
+                    grad[i] += v;
+                }
             }
         }
     }
@@ -844,13 +977,13 @@ struct GridGradientSlices
 };
 
 /** One workgroup of 1024 lanes per work item; `items` is indexed by the workgroup; SLICE_FLOATS * 8 bytes of dynamic LDS. */
-template <typename Cfg, int SLICE_FLOATS>
+template <typename Cfg, int SLICE_FLOATS, bool FLOATS>
 __global__ void __launch_bounds__(1024) GridGradientSlicesKernel(
     int numel, const unsigned* __restrict__ records, const int* __restrict__ cursors, float* __restrict__ gradients,
     const GridGradientSlice* __restrict__ items)
 {
     extern __shared__ __align__(16) unsigned char sMemory[];
-    GridGradientSlices<Cfg, SLICE_FLOATS>::template dispatch<0>(numel, records, cursors, gradients, items[blockIdx.x],
+    GridGradientSlices<Cfg, SLICE_FLOATS, FLOATS>::template dispatch<0>(numel, records, cursors, gradients, items[blockIdx.x],
                                                                 reinterpret_cast<long long*>(sMemory));
 }
 

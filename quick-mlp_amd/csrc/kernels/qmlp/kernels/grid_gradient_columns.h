@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(BLOCK) GridGradientColumnsKernel(
     typedef GridGradientColumns<Cfg, CPS> Impl;
     typedef EncodingHashGrid<Cfg> Grid;
     typedef GridGradientRecords<Cfg, ROW_CHANNELS, CHANNEL_OFFSET, 8192, 256> Records;   // its gathers for the input gradients
-    typedef GridGradientSlices<Cfg, 8192> Fixed;                                         // its fixed-point arithmetic
+    typedef GridGradientSlices<Cfg, 8192, false> Fixed;                                         // its fixed-point arithmetic
     constexpr int D = Cfg::Dim, F = Cfg::Features, NC = Grid::NC;
     extern __shared__ __align__(16) unsigned char sMemory[];
     long long* sSums = reinterpret_cast<long long*>(sMemory);
@@ -440,7 +440,7 @@ __global__ void __launch_bounds__(BLOCK) GridGradientColumnsKernel(
             for (int d = 0; d < D; ++d) adjPos[d] = 0.f;
             if constexpr (INPUT_GRADIENTS == 2) {
                 Records::template positionGradientFromDerivatives<0>(
-                    p, static_cast<const typename Records::DerivativeChunk*>(derivativesV), adjEncoded, adjPos);
+                    p, static_cast<const typename Records::DerivativeChunk*>(derivativesV), typename Records::Adjoints{adjEncodedH}, adjPos);
             } else {
                 const typename Grid::LevelSetup s = Grid::setupLevel(0, pos);
                 detail::HeldFeatures<F, table_t> held[NC];
@@ -463,7 +463,7 @@ __global__ void __launch_bounds__(BLOCK) GridGradientColumnsKernel(
                 } else {
                     Records::template loadHeld<0>(s, params, held);
                 }
-                Records::template positionGradient<0>(p, s, held, adjEncoded, adjPos);
+                Records::template positionGradient<0>(p, s, held, typename Records::Adjoints{adjEncodedH}, adjPos);
             }
 #pragma unroll
             for (int d = 0; d < D; ++d)

@@ -452,11 +452,24 @@ int qmlp_encoding_adjoint(qmlp_encoding_t encoding, const qmlp_tensor* input, co
                           const qmlp_tensor* adj_input, void* stream, const qmlp_tensor* parameters_forward,
                           const qmlp_tensor* parameters_gradients, int adjoint_mode)
 {
+    return qmlp_encoding_adjoint_in(encoding, input, adj_output, adj_input, stream, parameters_forward, parameters_gradients,
+                                    adjoint_mode, nullptr);
+}
+int qmlp_encoding_adjoint_memory(qmlp_encoding_t encoding, long long points, int adjoint_mode, size_t* bytes)
+{
+    QMLP_API_BEGIN
+    *bytes = encoding->encoding->adjointMemory(points, adjoint_mode);
+    QMLP_API_END
+}
+int qmlp_encoding_adjoint_in(qmlp_encoding_t encoding, const qmlp_tensor* input, const qmlp_tensor* adj_output,
+                             const qmlp_tensor* adj_input, void* stream, const qmlp_tensor* parameters_forward,
+                             const qmlp_tensor* parameters_gradients, int adjoint_mode, void* memory)
+{
     QMLP_API_BEGIN
     Tensor adjIn = wrap(adj_input);
     encoding->encoding->adjoint(wrap(input), wrap(adj_output), adjIn, static_cast<stream_t>(stream),
                                 optionalTensor(parameters_forward), optionalTensor(parameters_gradients),
-                                adjoint_mode);
+                                adjoint_mode, memory);
     QMLP_API_END
 }
 

@@ -297,6 +297,12 @@ bool EncodingHashGrid::hashedPointOrderKey(kernel::PointOrderKey& key, long long
     return true;
 }
 
+int EncodingHashGrid::levelGroups() const
+{
+    // one group per die; levels that are added up stay together
+    return combinationMode_ == LayerCombinationMode::CONCAT ? std::min(8, numLevels_) : 1;
+}
+
 int EncodingHashGrid::ldsGradientFloats(int maxBytes, int& levels) const
 {
     levels = 0;
@@ -314,7 +320,7 @@ int EncodingHashGrid::ldsGradientFloats(int maxBytes, int& levels) const
     return floats;
 }
 
-bool EncodingHashGrid::gradientSlices(GradientSliceLayout& layout) const
+bool EncodingHashGrid::gradientSlices(GradientSliceLayout& layout, bool floatAdjoints) const
 {
     if (dimension_ > 4 || numParameters_ >= (1 << 30)) return false;   // up to 8 records per point and level in registers
     const int lds = FusedNetwork::MaxSharedMemoryBytes();
@@ -333,8 +339,9 @@ bool EncodingHashGrid::gradientSlices(GradientSliceLayout& layout) const
     layout.sliceFloats = entries * numFeaturesPerLevel_;
     layout.configType = "qmlp::kernel::" + configName();
     layout.pairs = std::max(1, (1 << dimension_) / 2);
-    // as GridGradientLayout::RECORD_WORDS: two 16-bit offsets, two weights, the adjoint halves, padded to 16 / 32 bytes
-    const int usedWords = 3 + (numFeaturesPerLevel_ + 1) / 2;
+    // as GridGradientLayout::RECORD_WORDS: two 16-bit offsets, two weights, the adjoint halves (or: one weight, products in float),
+    // padded to 16 / 32 bytes
+    const int usedWords = floatAdjoints ? 2 + numFeaturesPerLevel_ : 3 + (numFeaturesPerLevel_ + 1) / 2;
     layout.recordWords = usedWords % 4 == 3 ? usedWords + 1 : usedWords;
     // the records of a workgroup and level are sorted in LDS: 96 KiB for them, the rest for the book-keeping
     int points = 1024;

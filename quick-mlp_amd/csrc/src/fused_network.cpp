@@ -1021,8 +1021,7 @@ size_t FusedNetwork::sliceGradientWorkspaceBytes(long long numel) const
         const auto* slices = slicesOf(*e);
         if (!slices) continue;
         const auto& layout = *slices;
-        bytes += roundUp(static_cast<size_t>(layout.numBuckets() + 1) * sizeof(int), size_t(256));   // cursors, largest adjoint
-        bytes += roundUp(static_cast<size_t>(layout.totalRecords(numel)) * layout.recordWords * sizeof(uint32_t), size_t(256));
+        bytes += layout.workspaceBytes(numel);
     }
     return bytes;
 }
@@ -1030,11 +1029,11 @@ size_t FusedNetwork::sliceGradientWorkspaceBytes(long long numel) const
 bool FusedNetwork::useSliceGradients(int numel, int flags) const
 {
     if (!(flags & GRADIENTS_INPUT_ENCODINGS) || !hasSliceGradients()) return false;
-    if (compileOptions_.sliceGradients > 0 || numel >= SLICE_GRADIENTS_MIN_BATCH) return true;
-    if (numel < SLICE_GRADIENTS_MIN_BATCH_MANY_LEVELS) return false;
+    if (compileOptions_.sliceGradients > 0) return true;
     for (const auto& e : encodings_) {
         const auto* layout = slicesOf(*e);
-        if (layout && layout->slicesPerLevel.size() >= 8) return true;
+        if (layout && IEncoding::slicesPay(*layout, numel, flags & GRADIENTS_NETWORK_WEIGHTS ? IEncoding::SLICE_GRADIENTS_MIN_BATCH_TRAIN_STEP
+                                                                                             : IEncoding::SLICE_GRADIENTS_MIN_BATCH_NO_WEIGHTS)) return true;
     }
     return false;
 }
@@ -1778,7 +1777,7 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
                 }
             sk.kernel.blockSize = 1024;
             sk.kernel.sharedMemorySize = layout.sliceFloats * static_cast<int>(sizeof(long long));
-            sk.kernel.fun = kl->getKernel(format("qmlp::kernel::GridGradientSlicesKernel<%s, %d>", layout.configType.c_str(), layout.sliceFloats),
+            sk.kernel.fun = kl->getKernel(format("qmlp::kernel::GridGradientSlicesKernel<%s, %d, false>", layout.configType.c_str(), layout.sliceFloats),
                                           source.str(), loaderFlags(compileOnly)).value();
             if (!compileOnly) {
                 static_assert(sizeof(IEncoding::GradientSlice) == 32, "eight 32-bit words, as in kernels/grid_gradient.h");
@@ -1827,8 +1826,9 @@ void FusedNetwork::compileRecordsKernel(SliceGradientKernel& sk, int flags, size
     ck.sharedMemorySize = layout.recordsLdsBytes(points);
     ck.fun = QuickMLP::Instance().kernelLoader()->getKernel(
         // (last argument: no input gradients | from gathers of all corners | from the position derivatives of the forward pass)
-        format("qmlp::kernel::GridGradientRecordsKernel<%s, %d, %d, %d, %d, %d>", layout.configType.c_str(), layers_[0].channelsIn,
-               sk.channelOffset, layout.sliceFloats, points, !(flags & GRADIENTS_INPUT) ? 0 : fromDerivatives ? 2 : 1),
+        format("qmlp::kernel::GridGradientRecordsKernel<%s, %d, %d, %d, %d, %d, %d>", layout.configType.c_str(), layers_[0].channelsIn,
+               sk.channelOffset, layout.sliceFloats, points, !(flags & GRADIENTS_INPUT) ? 0 : fromDerivatives ? 2 : 1,
+               layout.levelGroups(flags & GRADIENTS_INPUT)),
         sk.recordsSource, loaderFlags(compileOnly)).value();
     if (compileOnly) return;
     ck.fullGrid = ck.fun.fullGridSize(ck.blockSize, ck.sharedMemorySize);
@@ -1883,7 +1883,8 @@ const FusedNetwork::CompiledKernel& FusedNetwork::recordsKernelFor(SliceGradient
     // 2^17 points 0.414 / 0.302 / 0.319 / 0.371, 2^16 points 0.290 / 0.233 / 0.215 / 0.244.
     const int computeUnits = KernelFunction::computeUnits();
     size_t variant = 0;
-    while (variant + 1 < sk.records.size() && divUp(numel, sk.layout.pointsPerWorkgroup >> variant) < computeUnits) ++variant;
+    const int groups = sk.layout.levelGroups(flags & GRADIENTS_INPUT);
+    while (variant + 1 < sk.records.size() && groups * divUp(numel, sk.layout.pointsPerWorkgroup >> variant) < computeUnits) ++variant;
     auto& kernels = fromDerivatives ? sk.recordsFromDerivatives : sk.records;
     if (!kernels[variant].has_value()) compileRecordsKernel(sk, flags, variant, false, fromDerivatives);
     return kernels[variant].value();
@@ -2541,15 +2542,14 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
                         ck.fun.launch(maxItems, ck.blockSize, ck.sharedMemorySize, stream, args);
                     }
                     // (the room of this encoding's cursors and records stays where it is for the encodings behind it)
-                    workspace += roundUp(static_cast<size_t>(layout.numBuckets() + 1) * sizeof(int), size_t(256))
-                        + roundUp(static_cast<size_t>(layout.totalRecords(numel64)) * layout.recordWords * sizeof(uint32_t), size_t(256));
+                    workspace += layout.workspaceBytes(numel64);
                     continue;
                 }
             }
             int* cursors = reinterpret_cast<int*>(workspace);
-            const size_t cursorBytes = roundUp(static_cast<size_t>(layout.numBuckets() + 1) * sizeof(int), size_t(256));
+            const size_t cursorBytes = layout.cursorBytes();
             uint32_t* records = reinterpret_cast<uint32_t*>(workspace + cursorBytes);
-            workspace += cursorBytes + roundUp(static_cast<size_t>(layout.totalRecords(numel64)) * layout.recordWords * sizeof(uint32_t), size_t(256));
+            workspace += layout.workspaceBytes(numel64);
             QMLP_HIP_CALL(qmlp_hip_memset_async(cursors, 0, cursorBytes, stream));
             std::vector<char> params(1024);
             int n = encodings_[sk.encoding]->fillParameterMemory(params.data(), static_cast<int>(params.size()));
@@ -2563,7 +2563,7 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
                     + (static_cast<long long>(perEntryForwardMemoryBytes_) + std::max(0ll, sk.derivativeOffset)) * numel64;
                 void* args[] = {&numel, &numelPadded, &inputAcc, &adjEncoded, params.data(), &records, &cursors, &adjInputAcc, &derivatives};
                 const CompiledKernel& rk = recordsKernelFor(sk, adjointFlags, numel, fromDerivatives);
-                rk.fun.launch(std::min(divUp(numel, rk.blockSize), rk.fullGrid), rk.blockSize, rk.sharedMemorySize, stream, args);
+                rk.fun.launch(layout.recordsGrid(numel, rk.blockSize, layout.levelGroups(adjointFlags & GRADIENTS_INPUT), rk.fullGrid), rk.blockSize, rk.sharedMemorySize, stream, args);
             }
             const uint32_t* recordsRead = records;
             const int* cursorsRead = cursors;

@@ -4,6 +4,7 @@
 #include <qmlp/encoding_line_integration.h>
 #include <qmlp/encoding_identity.h>
 #include <qmlp/qmlp.h>
+#include <qmlp_hip.h>
 
 #include <cctype>
 #include <cstring>
@@ -21,7 +22,7 @@ struct ArgPack
 
 std::string standaloneSource(const IEncoding& e, const std::string& callForward, const std::string& callAdjoint,
                              const std::string& callCorners = "", const std::string& callScatter = "",
-                             const std::string& callTraceGather = "", const std::string& callTraceScatter = "")
+                             const std::string& callTraceGather = "", const std::string& callTraceScatter = "", int groups = 1)
 {
     auto kl = QuickMLP::Instance().kernelLoader();
     std::string codeTemplate = kl->findFile("qmlp/kernels/encoding_kernels.h").value();
@@ -31,6 +32,14 @@ std::string standaloneSource(const IEncoding& e, const std::string& callForward,
     replaceAll(codeTemplate, "$$INCLUDES$$", includes.str());
     replaceAll(codeTemplate, "$$ENCODING_PARAMETERS$$",
                e.hasParameters() ? ", const " + e.parameterName() + " cEncoding" : std::string());
+    // the channels of a group of levels (EncodingForwardKernel)
+    const std::string levels = std::to_string(e.numOutputChannels() / e.channelsWrittenTogether());
+    const std::string features = std::to_string(e.channelsWrittenTogether());
+    replaceAll(codeTemplate, "$$LEVEL_GROUPS$$", std::to_string(groups));
+    replaceAll(codeTemplate, "$$GROUP_CHANNELS$$", groups == 1 ? std::to_string(e.numOutputChannels())
+                                                               : "(" + levels + " + GROUPS - 1) / GROUPS * " + features);
+    replaceAll(codeTemplate, "$$FIRST_CHANNEL$$", groups == 1 ? "0" : levels + " * group / GROUPS * " + features);
+    replaceAll(codeTemplate, "$$CHANNELS$$", groups == 1 ? "CHANNELS" : levels + " * (group + 1) / GROUPS * " + features + " - firstChannel");
     replaceAll(codeTemplate, "$$CALL_ENCODINGS_FORWARD$$", callForward);
     replaceAll(codeTemplate, "$$CALL_ENCODINGS_ADJOINT$$", callAdjoint);
     replaceAll(codeTemplate, "$$CALL_ENCODINGS_CORNERS$$", callCorners);
@@ -42,13 +51,14 @@ std::string standaloneSource(const IEncoding& e, const std::string& callForward,
 
 } // namespace
 
-std::string IEncoding::forwardKernelSource() const
+std::string IEncoding::forwardKernelSource(int groups) const
 {
     std::stringstream call;
-    call << qualifiedName() << "::forward(encodingInput, encodingOutput";
+    if (groups > 1) call << qualifiedName() << "::forwardGroup<0, GROUPS>(group, encodingInput, encodingOutput";
+    else call << qualifiedName() << "::forward(encodingInput, encodingOutput";
     if (hasParameters()) call << ", cEncoding";
     call << ");\n";
-    return standaloneSource(*this, call.str(), "");
+    return standaloneSource(*this, call.str(), "", "", "", "", "", groups);
 }
 
 std::string IEncoding::adjointKernelSource(int adjointMode) const
@@ -73,10 +83,16 @@ void IEncoding::precompile(int adjointMode)
 {
     auto kl = QuickMLP::Instance().kernelLoader();
     const int flags = QuickMLP::Instance().getCompileFlags() | KernelLoader::CompileOnly;
-    kl->getKernel("qmlp::kernel::EncodingForwardKernel", forwardKernelSource(), flags);
+    kl->getKernel("qmlp::kernel::EncodingForwardKernel", forwardKernelSource(1), flags);
+    if (levelGroups() > 1) kl->getKernel("qmlp::kernel::EncodingForwardKernel", forwardKernelSource(levelGroups()), flags);
     if (adjointMode > 0) {
         CHECK_ERROR(adjointMode <= ALL_GRADIENTS, "Illegal adjoint mode");
         kl->getKernel("qmlp::kernel::EncodingAdjointKernel", adjointKernelSource(adjointMode), flags);
+        if (const auto* layout = (adjointMode & PARAM_GRADIENTS) && hasParameters() ? sliceLayout(true) : nullptr) {
+            for (int v = 0; v < recordsVariants(*layout); ++v) compileRecords(*layout, adjointMode & INPUT_GRADIENTS, v, flags);
+            compileSlices(*layout, true, flags);
+            compileSlices(*layout, false, flags);
+        }
     }
 }
 
@@ -97,10 +113,12 @@ void IEncoding::forward(const Tensor& input, Tensor& output, stream_t stream,
                     "The encoding has parameters, but no inference tensor is bound or passed");
     if (numel == 0) return;
 
-    if (!forwardKernel_.has_value())
-        forwardKernel_ = QuickMLP::Instance().kernelLoader()->getKernel(
-            "qmlp::kernel::EncodingForwardKernel", forwardKernelSource(), QuickMLP::Instance().getCompileFlags()).value();
-    auto& fun = forwardKernel_.value();
+    const int groups = numel < FORWARD_WHOLE_ROWS_MIN_BATCH ? levelGroups() : 1;
+    auto& kernel = forwardKernel_[groups > 1 ? 1 : 0];
+    if (!kernel.has_value())
+        kernel = QuickMLP::Instance().kernelLoader()->getKernel(
+            "qmlp::kernel::EncodingForwardKernel", forwardKernelSource(groups), QuickMLP::Instance().getCompileFlags()).value();
+    auto& fun = kernel.value();
 
     std::vector<char> paramBytes(4096);
     if (hasParameters()) {
@@ -110,7 +128,7 @@ void IEncoding::forward(const Tensor& input, Tensor& output, stream_t stream,
     }
 
     const int block = 256;
-    const int grid = static_cast<int>(std::min<long long>(divUp<long long>(numel, block), fun.fullGridSize(block, 0)));
+    const int grid = groups * static_cast<int>(std::min<long long>(divUp<long long>(numel, block), std::max(1, fun.fullGridSize(block, 0) / groups)));
     auto inputAcc = input.accessor<kernel::Tensor2Read<float>>();
     auto outputAcc = output.accessor<kernel::Tensor2RW<float>>();
     std::vector<void*> args = {&numel, &inputAcc, &outputAcc};
@@ -122,7 +140,7 @@ void IEncoding::forward(const Tensor& input, Tensor& output, stream_t stream,
 
 void IEncoding::adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& adjInput, stream_t stream,
                         const std::optional<const Tensor>& parametersForward,
-                        const std::optional<const Tensor>& parametersGradients, int adjointMode)
+                        const std::optional<const Tensor>& parametersGradients, int adjointMode, void* tmpMemory)
 {
     CHECK_DIM(input, 2);
     CHECK_DIM(adjOutput, 2);
@@ -145,12 +163,12 @@ void IEncoding::adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& ad
                     "Parameter gradients requested, but no gradient tensor is bound or passed");
     }
     if (numel == 0) return;
+    const bool bySlices = tmpMemory != nullptr && adjointMemory(numel, adjointMode) > 0;
 
-    if (!adjointKernel_[adjointMode].has_value())
+    if (!bySlices && !adjointKernel_[adjointMode].has_value())
         adjointKernel_[adjointMode] = QuickMLP::Instance().kernelLoader()->getKernel(
             "qmlp::kernel::EncodingAdjointKernel", adjointKernelSource(adjointMode),
             QuickMLP::Instance().getCompileFlags()).value();
-    auto& fun = adjointKernel_[adjointMode].value();
 
     std::vector<char> paramBytes(4096);
     if (hasParameters()) {
@@ -160,17 +178,107 @@ void IEncoding::adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& ad
         (void)n;
     }
 
-    const int block = 256;
-    const int grid = static_cast<int>(std::min<long long>(divUp<long long>(numel, block), fun.fullGridSize(block, 0)));
-    auto inputAcc = input.accessor<kernel::Tensor2Read<float>>();
-    auto adjOutputAcc = adjOutput.accessor<kernel::Tensor2Read<float>>();
-    auto adjInputAcc = adjInput.accessor<kernel::Tensor2RW<float>>();
-    std::vector<void*> args = {&numel, &inputAcc, &adjOutputAcc, &adjInputAcc};
-    if (hasParameters()) args.push_back(paramBytes.data());
-    fun.launch(grid, block, 0, stream, args.data());
+    if (bySlices) {
+        adjointBySlices(*sliceLayout(true), input, adjOutput, adjInput, stream, adjointMode, tmpMemory, paramBytes.data());
+    } else {
+        auto& fun = adjointKernel_[adjointMode].value();
+        const int block = 256;
+        const int grid = static_cast<int>(std::min<long long>(divUp<long long>(numel, block), fun.fullGridSize(block, 0)));
+        auto inputAcc = input.accessor<kernel::Tensor2Read<float>>();
+        auto adjOutputAcc = adjOutput.accessor<kernel::Tensor2Read<float>>();
+        auto adjInputAcc = adjInput.accessor<kernel::Tensor2RW<float>>();
+        std::vector<void*> args = {&numel, &inputAcc, &adjOutputAcc, &adjInputAcc};
+        if (hasParameters()) args.push_back(paramBytes.data());
+        fun.launch(grid, block, 0, stream, args.data());
+    }
 
     if (hasParameters() && parametersForward.has_value()) setParameter({}, Tensor::INFERENCE);
     if (hasParameters() && parametersGradients.has_value()) setParameter({}, Tensor::GRADIENTS);
+}
+
+size_t IEncoding::adjointMemory(long long numel, int adjointMode) const
+{
+    if (!(adjointMode & PARAM_GRADIENTS) || !hasParameters() || numel >= (1 << 27)) return 0;
+    const auto* layout = sliceLayout(true);
+    return layout && slicesPay(*layout, numel, SLICE_GRADIENTS_MIN_BATCH_STANDALONE) ? layout->workspaceBytes(numel) : 0;
+}
+
+int IEncoding::recordsVariants(const GradientSliceLayout& layout)
+{
+    int n = 1;
+    while ((layout.pointsPerWorkgroup >> n) >= 128) ++n;
+    return n;
+}
+
+std::optional<KernelFunction> IEncoding::compileRecords(const GradientSliceLayout& layout, bool inputGradients, int variant, int flags) const
+{
+    std::stringstream source;
+    fillCode(source);
+    source << "\n" << KernelLoader::MainFile("qmlp/kernels/grid_gradient.h");
+    return QuickMLP::Instance().kernelLoader()->getKernel(
+        format("qmlp::kernel::GridGradientRecordsKernel<%s, 0, 0, %d, %d, %d, %d>", layout.configType.c_str(), layout.sliceFloats,
+               layout.pointsPerWorkgroup >> variant, inputGradients ? 1 : 0, layout.levelGroups(inputGradients)), source.str(), flags);
+}
+
+std::optional<KernelFunction> IEncoding::compileSlices(const GradientSliceLayout& layout, bool clear, int flags) const
+{
+    std::stringstream source;
+    fillCode(source);
+    source << "\n" << KernelLoader::MainFile("qmlp/kernels/grid_gradient.h");
+    return QuickMLP::Instance().kernelLoader()->getKernel(
+        clear ? std::string("qmlp::kernel::GridGradientClearKernel")
+              : format("qmlp::kernel::GridGradientSlicesKernel<%s, %d, true>", layout.configType.c_str(), layout.sliceFloats),
+        source.str(), flags);
+}
+
+void IEncoding::adjointBySlices(const GradientSliceLayout& layout, const Tensor& input, const Tensor& adjOutput, Tensor& adjInput, stream_t stream,
+                                int adjointMode, void* tmpMemory, char* parameters)
+{
+    CHECK_ERROR(reinterpret_cast<uintptr_t>(tmpMemory) % 256 == 0, "The temporary memory must be aligned to 256 bytes");
+    auto& sk = sliceKernels_;
+    const int flags = QuickMLP::Instance().getCompileFlags();
+    int numel = static_cast<int>(input.size(0));
+    const bool inputGradients = adjointMode & INPUT_GRADIENTS;
+    const int groups = layout.levelGroups(inputGradients);
+    // as for the fused networks: as many points per workgroup as keep every compute unit busy
+    int variant = 0;
+    while (variant + 1 < recordsVariants(layout) && groups * divUp(numel, layout.pointsPerWorkgroup >> variant) < KernelFunction::computeUnits()) ++variant;
+    auto& variants = sk.records[inputGradients ? 1 : 0];
+    if (variants.empty()) variants.resize(recordsVariants(layout));
+    if (!variants[variant].has_value()) variants[variant] = compileRecords(layout, inputGradients, variant, flags).value();
+    if (!sk.clear.has_value()) sk.clear = compileSlices(layout, true, flags).value();
+    if (!sk.slices.has_value()) {
+        sk.slices = compileSlices(layout, false, flags).value();
+        sk.items = Tensor(Tensor::FLOAT, {static_cast<int32_t>(layout.items.size() * (sizeof(GradientSlice) / sizeof(float)))});
+        QMLP_HIP_CALL(qmlp_hip_memcpy_h2d(sk.items.rawPtr(), layout.items.data(), layout.items.size() * sizeof(layout.items[0]), nullptr));
+    }
+
+    int* cursors = static_cast<int*>(tmpMemory);
+    uint32_t* records = reinterpret_cast<uint32_t*>(static_cast<char*>(tmpMemory) + layout.cursorBytes());
+    {
+        // (a kernel and not a memset, which calls that are captured into a graph would not repeat reliably)
+        int words = layout.numBuckets() + 1;
+        void* args[] = {&cursors, &words};
+        sk.clear.value().launch(divUp(words, 256), 256, 0, stream, args);
+    }
+    {
+        auto inputAcc = input.accessor<kernel::Tensor2Read<float>>();
+        auto adjOutputAcc = adjOutput.accessor<kernel::Tensor2Read<float>>();
+        auto adjInputAcc = adjInput.accessor<kernel::Tensor2RW<float>>();
+        const void* derivatives = nullptr;
+        void* args[] = {&numel, &numel, &inputAcc, &adjOutputAcc, parameters, &records, &cursors, &adjInputAcc, &derivatives};
+        const int points = layout.pointsPerWorkgroup >> variant;
+        auto& fun = variants[variant].value();
+        const int lds = layout.recordsLdsBytes(points);
+        fun.launch(layout.recordsGrid(numel, points, groups, fun.fullGridSize(points, lds)), points, lds, stream, args);
+    }
+    const uint32_t* recordsRead = records;
+    const int* cursorsRead = cursors;
+    float* gradients = nullptr;
+    std::memcpy(&gradients, parameters + sizeof(void*), sizeof(void*));   // HashGridParams: forward table, gradient table, ...
+    const void* items = sk.items.rawPtr();
+    void* args[] = {&numel, &recordsRead, &cursorsRead, &gradients, &items};
+    sk.slices.value().launch(static_cast<int>(layout.items.size()), 1024, layout.sliceFloats * static_cast<int>(sizeof(long long)), stream, args);
 }
 
 void EncodingHashGrid::corners(const Tensor& input, unsigned* indices, float* weights, stream_t stream, int mode)
@@ -211,7 +319,7 @@ void EncodingHashGrid::precompileCorners(int mode, bool compileOnly)
     if (mode == 3) {
         // the record building of kernels/grid_gradient.h with the slice size the fused network uses for this grid
         GradientSliceLayout layout;
-        CHECK_ERROR(gradientSlices(layout), "this grid has no gradient slices");
+        CHECK_ERROR(gradientSlices(layout, false), "this grid has no gradient slices");
         std::stringstream source;
         fillCode(source);
         source << "\n" << KernelLoader::MainFile("qmlp/kernels/grid_gradient.h");

@@ -220,7 +220,12 @@ struct EncodingBindings : torch::CustomClassHolder
         auto adjParameter = torch::zeros(parameter.sizes(), parameter.options().dtype(parameterDtype(true)));
         const qmlp_tensor in = wrap(input), adjOut = wrap(adjOutput), adjIn = wrap(adjInput), par = wrap(parameter),
                           adjPar = wrap(adjParameter);
-        QMLP_CHECK(qmlp_encoding_adjoint(handle_, &in, &adjOut, &adjIn, currentStream(), &par, &adjPar, static_cast<int>(flags)));
+        size_t bytes = 0;
+        QMLP_CHECK(qmlp_encoding_adjoint_memory(handle_, input.size(0), static_cast<int>(flags), &bytes));
+        torch::Tensor memory;
+        if (bytes > 0) memory = torch::empty({static_cast<int64_t>(bytes)}, input.options().dtype(torch::kUInt8));
+        QMLP_CHECK(qmlp_encoding_adjoint_in(handle_, &in, &adjOut, &adjIn, currentStream(), &par, &adjPar, static_cast<int>(flags),
+                                            bytes > 0 ? memory.data_ptr() : nullptr));
         return {adjInput, adjParameter.to(parameter.scalar_type())};
     }
     std::tuple<torch::Tensor, torch::Tensor> adjointWithParameter(const torch::Tensor& input, const torch::Tensor& parameter,

@@ -95,6 +95,8 @@ _SIGNATURES = {
     "qmlp_encoding_zero_gradients": [_vp],
     "qmlp_encoding_forward": [_vp, _TD, _TD, _vp, _TD],
     "qmlp_encoding_adjoint": [_vp, _TD, _TD, _TD, _vp, _TD, _TD, _ci],
+    "qmlp_encoding_adjoint_memory": [_vp, ctypes.c_longlong, _ci, _P(ctypes.c_size_t)],
+    "qmlp_encoding_adjoint_in": [_vp, _TD, _TD, _TD, _vp, _TD, _TD, _ci, _vp],
     "qmlp_encoding_hashgrid_levels": [_vp, _ci, _pi, _pi, _pi, _pi, _pi],
     "qmlp_encoding_hashgrid_corners": [_vp, _TD, _vp, _vp, _vp],
     "qmlp_encoding_hashgrid_trace": [_vp, _TD, _ci, _vp, _vp, _vp],

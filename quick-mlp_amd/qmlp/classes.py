@@ -276,9 +276,12 @@ class Encoding:
         adj_input = torch.zeros_like(input)
         adj_param = torch.zeros(parameter_forward.shape, dtype=self.parameter_dtype(True),
                                 device=parameter_forward.device)
-        check(lib.qmlp_encoding_adjoint(self._handle, desc(input), desc(adj_output), desc(adj_input),
-                                        current_stream(input.device), desc(parameter_forward), desc(adj_param),
-                                        int(flags)))
+        size = ctypes.c_size_t()
+        check(lib.qmlp_encoding_adjoint_memory(self._handle, input.shape[0], int(flags), ctypes.byref(size)))
+        memory = torch.empty((size.value,), dtype=torch.uint8, device=input.device) if size.value else None
+        check(lib.qmlp_encoding_adjoint_in(self._handle, desc(input), desc(adj_output), desc(adj_input),
+                                           current_stream(input.device), desc(parameter_forward), desc(adj_param),
+                                           int(flags), memory.data_ptr() if size.value else None))
         self._bound_inference = None   # as in inference_with_parameter
         return adj_input, adj_param.to(parameter_forward.dtype)
 
