@@ -1,5 +1,5 @@
-// qmlp._native: the calls that a training or rendering loop makes once per batch (FusedNetwork.forward and its
-// backward pass), from Python straight into C++. A call on a small batch is bound by the host: through ctypes and a
+// qmlp._native: the calls that a training or rendering loop makes once per batch (FusedNetwork.forward, a standalone
+// encoding, and their backward passes), from Python straight into C++. A call on a small batch is bound by the host: through ctypes and a
 // Python autograd function, inference on 1000 points took 13 us beside a kernel of 3.6 us, and a train step on 513
 // points 148 us beside kernels of 25 us. Everything else of the Python package stays on ctypes.
 //
@@ -13,6 +13,7 @@
 
 #include "qmlp_capi.h"
 
+#include <atomic>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -277,6 +278,117 @@ at::Tensor forward(const Network_ptr& net, const at::Tensor& input, const at::Te
     return output;
 }
 
+// ------------------------------------------------------------------------------------------------ standalone encodings
+/** An encoding of the C ABI, of its own or of a network (which it keeps alive), one call at a time. */
+struct Encoding
+{
+    qmlp_encoding_t handle;
+    Network_ptr network;
+    std::mutex ownMutex;
+    std::mutex& mutex;
+    int channelsOut = 0;
+    std::atomic<long long> calls{0};   // each leaves the native encoding without a bound table
+
+    Encoding(uintptr_t h, Network_ptr net)
+        : handle(reinterpret_cast<qmlp_encoding_t>(h)), network(std::move(net)), mutex(network ? network->mutex : ownMutex)
+    {
+        check(qmlp_encoding_num_output_channels(handle, &channelsOut));
+    }
+    ~Encoding() { if (!network) qmlp_encoding_destroy(handle); }
+};
+using Encoding_ptr = std::shared_ptr<Encoding>;
+
+/** parameter: undefined for encodings without parameters */
+at::Tensor encode(const Encoding_ptr& enc, const at::Tensor& input, const at::Tensor& parameter)
+{
+    try {
+        at::AutoDispatchBelowADInplaceOrView guard;
+        auto output = createOutput(input, enc->channelsOut);
+        const qmlp_tensor in = wrap(input), out = wrap(output), par = wrap(parameter);
+        void* stream = currentStream(input);
+        {
+            py::gil_scoped_release release;
+            std::lock_guard<std::mutex> lock(enc->mutex);
+            ++enc->calls;
+            check(qmlp_encoding_forward(enc->handle, &in, &out, stream, parameter.defined() ? &par : nullptr));
+        }
+        return output;
+    } catch (const Failure& f) {
+        raise(f);
+    }
+}
+
+/** Gradients of input and parameter (in float); undefined where they were not asked for or there are none. */
+std::pair<at::Tensor, at::Tensor> encodeAdjoint(Encoding& enc, const at::Tensor& input, const at::Tensor& parameter, const at::Tensor& adjOutput, int flags)
+{
+    at::AutoDispatchBelowADInplaceOrView guard;
+    // (the native call wants the tensor in any case: without input gradients it is not written)
+    at::Tensor adjInput = flags & QMLP_ENCODING_INPUT_GRADIENTS ? at::zeros_like(input) : at::Tensor();
+    at::Tensor adjParameter;
+    if (parameter.defined() && (flags & QMLP_ENCODING_PARAM_GRADIENTS))
+        adjParameter = at::zeros(parameter.sizes(), parameter.options().dtype(at::kFloat));
+    const qmlp_tensor in = wrap(input), adjOut = wrap(adjOutput), adjIn = adjInput.defined() ? wrap(adjInput) : in, par = wrap(parameter),
+                      adjPar = wrap(adjParameter);
+    std::lock_guard<std::mutex> lock(enc.mutex);
+    ++enc.calls;
+    size_t bytes = 0;
+    check(qmlp_encoding_adjoint_memory(enc.handle, in.sizes[0], flags, &bytes));
+    at::Tensor memory;
+    if (bytes > 0) memory = bytesOn(input, bytes);
+    check(qmlp_encoding_adjoint_in(enc.handle, &in, &adjOut, &adjIn, currentStream(input), parameter.defined() ? &par : nullptr,
+                                   adjParameter.defined() ? &adjPar : nullptr, flags, bytes > 0 ? memory.data_ptr() : nullptr));
+    return {adjInput, adjParameter};
+}
+
+struct EncodingBackward : torch::autograd::Node
+{
+    Encoding_ptr enc;
+    int flags = 0;
+    SavedVariable input, parameter;
+
+    std::string name() const override { return "QmlpEncodingBackward"; }
+    void release_variables() override
+    {
+        input.reset_data();
+        parameter.reset_data();
+    }
+    variable_list apply(variable_list&& gradOutputs) override
+    {
+        variable_list grads(2);
+        if (!gradOutputs[0].defined()) return grads;
+        const at::Tensor x = input.unpack(), table = parameter.unpack();
+        try {
+            auto [adjInput, adjParameter] = encodeAdjoint(*enc, x, table, gradOutputs[0].contiguous(), flags);
+            if (adjInput.defined() && task_should_compute_output(0)) grads[0] = adjInput;
+            if (adjParameter.defined() && task_should_compute_output(1)) grads[1] = adjParameter.to(table.scalar_type());
+        } catch (const Failure& f) {
+            throw std::runtime_error(f.message);
+        }
+        return grads;
+    }
+};
+
+at::Tensor encodeForward(const Encoding_ptr& enc, const at::Tensor& input, const at::Tensor& parameter)
+{
+    int flags = 0;
+    if (at::GradMode::is_enabled()) {
+        if (input.requires_grad()) flags |= QMLP_ENCODING_INPUT_GRADIENTS;
+        if (parameter.defined() && parameter.requires_grad()) flags |= QMLP_ENCODING_PARAM_GRADIENTS;
+    }
+    auto output = encode(enc, input, parameter);
+    if (flags == 0) return output;
+    auto node = std::shared_ptr<EncodingBackward>(new EncodingBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(input, parameter));
+    node->enc = enc;
+    node->flags = flags;
+    node->input = SavedVariable(input, false);
+    node->parameter = SavedVariable(parameter, false);
+    torch::autograd::set_history(output, node);
+    return output;
+}
+
+at::Tensor tensorOrNone(const py::object& o) { return o.is_none() ? at::Tensor() : o.cast<at::Tensor>(); }
+
 } // namespace
 
 PYBIND11_MODULE(_native, m)
@@ -303,4 +415,13 @@ PYBIND11_MODULE(_native, m)
                              const py::list& tables) { return inference(net, input, parameters, tensorsOf(tables)); })
         .def("forward", [](const Network_ptr& net, const at::Tensor& input, const at::Tensor& parameters,
                            const py::list& tables) { return forward(net, input, parameters, tensorsOf(tables)); });
+    py::class_<Encoding, Encoding_ptr>(m, "Encoding")
+        .def(py::init<uintptr_t, Network_ptr>())   // handle, the network it belongs to (None: it is taken over)
+        .def_property_readonly("calls", [](const Encoding_ptr& enc) { return enc->calls.load(); })
+        .def("inference", [](const Encoding_ptr& enc, const at::Tensor& input, const py::object& parameter) {
+            return encode(enc, input, tensorOrNone(parameter));
+        })
+        .def("forward", [](const Encoding_ptr& enc, const at::Tensor& input, const py::object& parameter) {
+            return encodeForward(enc, input, tensorOrNone(parameter));
+        });
 }

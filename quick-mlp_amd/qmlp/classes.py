@@ -110,36 +110,6 @@ class Activation:
 
 
 # ---------------------------------------------------------------------------- encoding
-class _EncodingFunction(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, input, enc):
-        ctx.save_for_backward(input)
-        ctx.enc = enc
-        return enc.inference(input)
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        (input,) = ctx.saved_tensors
-        return ctx.enc.adjoint(input, grad_output.contiguous()), None
-
-
-class _EncodingFunctionWithParameter(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, input, parameter, enc):
-        ctx.save_for_backward(input, parameter)
-        ctx.enc = enc
-        ctx.flags = (1 if input.requires_grad else 0) | (2 if parameter.requires_grad else 0)
-        return enc.inference_with_parameter(input, parameter)
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        input, parameter = ctx.saved_tensors
-        if ctx.flags == 0:
-            return None, None, None
-        gi, gp = ctx.enc.adjoint_with_parameter_and_flags(input, parameter, grad_output.contiguous(), ctx.flags)
-        return (gi if ctx.flags & 1 else None), (gp if ctx.flags & 2 else None), None
-
-
 class Encoding:
     """One input encoding, standalone (fp32 in, fp32 out)."""
 
@@ -153,11 +123,8 @@ class Encoding:
             self._cfg = cfg
             self._handle = ctypes.c_void_p()
             check(lib.qmlp_encoding_create(cfg.encode(), ctypes.byref(self._handle)))
-
-    def __del__(self):
-        if getattr(self, "_handle", None) and not self._borrowed:
-            lib.qmlp_encoding_destroy(self._handle)
-        self._handle = None
+        # owns the handle, unless a network does, together with the autograd graphs of its calls
+        self._native = _native.Encoding(self._handle.value, _owner._native if self._borrowed else None)
 
     def cfg(self):
         return self._cfg
@@ -202,7 +169,8 @@ class Encoding:
         if not gradients:
             # binding the same memory again changes nothing: skipped, unless the encoding belongs to a network,
             # whose own calls bind it as well
-            key = None if tensor is None else (tensor.data_ptr(), tensor.numel(), tensor.dtype)
+            # (a native call on a table of its own leaves the encoding without one)
+            key = None if tensor is None else (tensor.data_ptr(), tensor.numel(), tensor.dtype, self._native.calls)
             if key is not None and not self._borrowed and key == getattr(self, "_bound_inference", None):
                 return
             self._bound_inference = key
@@ -243,21 +211,14 @@ class Encoding:
     def inference(self, input):
         if self.has_parameters():
             raise RuntimeError("Encoding has parameters, call the variation of 'inference' with parameters")
-        _device_of(input)
-        output = _create_output(input, self.num_output_channels())
-        check(lib.qmlp_encoding_forward(self._handle, desc(input), desc(output), current_stream(input.device), None))
-        return output
+        return self._native.inference(input, None)
 
     def inference_with_parameter(self, input, parameter_forward):
         if not self.has_parameters():
             raise RuntimeError("Encoding doesn't have parameters, call the variation of 'inference' without parameters")
-        _device_of(input)
-        output = _create_output(input, self.num_output_channels())
-        check(lib.qmlp_encoding_forward(self._handle, desc(input), desc(output), current_stream(input.device),
-                                        desc(parameter_forward)))
         # the native call binds the table for its own duration and leaves the encoding unbound
         self._bound_inference = None
-        return output
+        return self._native.inference(input, parameter_forward)
 
     def adjoint(self, input, adj_output):
         if self.has_parameters():
@@ -288,12 +249,12 @@ class Encoding:
     def forward(self, input):
         if self.has_parameters():
             raise RuntimeError("Encoding has parameters, call the variation of 'forward' with parameters")
-        return _EncodingFunction.apply(input, self)
+        return self._native.forward(input, None)
 
     def forward_with_parameter(self, input, parameter):
         if not self.has_parameters():
             raise RuntimeError("Encoding doesn't have parameters, call the variation of 'forward' without parameters")
-        return _EncodingFunctionWithParameter.apply(input, parameter, self)
+        return self._native.forward(input, parameter)
 
     def __getstate__(self):
         return self._cfg
