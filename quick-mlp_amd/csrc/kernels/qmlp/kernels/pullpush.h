@@ -23,7 +23,7 @@
 //      level + adjoint of down, both formed per quad by gathering, without atomics
 // so a level of P pixels and C channels moves 2C+1 + (2C+2)/4 planes in A and 3C+2 + (5C+6)/4 planes in B.
 // 1 x 4 x 2048 x 2048 floats, finest level: down 21, up 37, A 49, B 68 us (4.9, 4.6, 2.6, 4.1 TB/s of the planes above; a
-// large copy reaches 5.2); the whole forward and adjoint call 435 us, of which 175 are levels of 1024 x 1024 and larger
+// large copy reaches 5.2); the whole forward and adjoint call 428 us (438 with the coarse levels formed again by the adjoint), of which 175 are levels of 1024 x 1024 and larger
 // (9.4 ms with four passes per level through memory, atomics for odd sizes, and memory allocated and released by every call).
 //
 // Follows src_cpp/include/qmlp/kernels/pullpush.cuh:22-303 of the reference. Differences on
@@ -630,11 +630,13 @@ __global__ void __launch_bounds__(256) PullPushGradientKernel(const PullPushLeve
 }
 
 /**
- * All coarse levels, one workgroup per image: from 'finest' down to the coarsest level and up again. The levels
- * below 'finest' live in LDS (dynamic, sized by the host) and are not kept: the adjoint forms them again.
+ * All coarse levels, one workgroup per image: from 'finest' down to the coarsest level and up again (without an output
+ * for 'finest' up to the level below it). The levels below 'finest' live in LDS (dynamic, sized by the host); a copy goes
+ * to kept, keptEntries per image, for the adjoint.
  */
 template <typename T>
-__global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushTailKernel(const PullPushLevel<T> finest, int C, const PullPushTail tail)
+__global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushTailKernel(const PullPushLevel<T> finest, int C, const PullPushTail tail,
+                                                                           T* __restrict__ kept, int keptEntries)
 {
     using namespace pullpush;
     extern __shared__ __align__(16) unsigned char sMemory[];
@@ -646,17 +648,20 @@ __global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushTailKernel(const 
         for (int i = threadIdx.x; i < low.H * low.W; i += PULLPUSH_TAIL_BLOCK) downPixel<false>(high, low, C, b, i / low.W, i % low.W);
         __syncthreads();
     }
-    for (int k = tail.numLevels - 2; k >= 0; --k) {
+    for (int k = tail.numLevels - 2; k >= (finest.dataPost.p ? 0 : 1); --k) {
         const auto high = level(k), low = level(k + 1);
         const int height = (high.H + 1) / 2, width = (high.W + 1) / 2;
         for (int i = threadIdx.x; i < height * width; i += PULLPUSH_TAIL_BLOCK) upQuad<false>(high, low, C, b, i / width, i % width);
         __syncthreads();
     }
+    for (int i = threadIdx.x; i < keptEntries; i += PULLPUSH_TAIL_BLOCK) kept[static_cast<long long>(b) * keptEntries + i] = sLevels[i];
 }
 
 /** The adjoint of all coarse levels, one workgroup per image. ACCUMULATE: 'finest' is the image itself and its gradients are added to. */
 template <typename T, bool ACCUMULATE>
-__global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushGradientTailKernel(const PullPushLevel<T> finest, int C, const PullPushTail tail)
+__global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushGradientTailKernel(const PullPushLevel<T> finest, int C, const PullPushTail tail,
+                                                                                   const T* __restrict__ kept, int keptEntries,
+                                                                                   const PullPushTail keptTail)
 {
     using namespace pullpush;
     constexpr int TW = 32, TH = PULLPUSH_TAIL_BLOCK / TW;
@@ -665,17 +670,13 @@ __global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushGradientTailKerne
     T* sLevels = reinterpret_cast<T*>(sMemory + sizeof(sFill));
     const int b = blockIdx.x;
     auto level = [&](int k) { return k == 0 ? finest : ldsLevel<T, true>(sLevels, tail, finest.H, finest.W, C, k); };
-    for (int k = 0; k + 1 < tail.numLevels; ++k) {
-        const auto high = level(k), low = level(k + 1);
-        for (int i = threadIdx.x; i < low.H * low.W; i += PULLPUSH_TAIL_BLOCK) downPixel<false>(high, low, C, b, i / low.W, i % low.W);
-        __syncthreads();
+    // the levels of the forward pass; here the gradients of a level follow behind it
+    for (int k = 1; k < tail.numLevels; ++k) {
+        const T* from = kept + (static_cast<long long>(b) * keptEntries + keptTail.offsets[k]);
+        const int entries = (k + 1 < tail.numLevels ? keptTail.offsets[k + 1] : keptEntries) - keptTail.offsets[k];
+        for (int i = threadIdx.x; i < entries; i += PULLPUSH_TAIL_BLOCK) sLevels[tail.offsets[k] + i] = from[i];
     }
-    for (int k = tail.numLevels - 2; k >= 1; --k) {
-        const auto high = level(k), low = level(k + 1);
-        const int height = (high.H + 1) / 2, width = (high.W + 1) / 2;
-        for (int i = threadIdx.x; i < height * width; i += PULLPUSH_TAIL_BLOCK) upQuad<false>(high, low, C, b, i / width, i % width);
-        __syncthreads();
-    }
+    __syncthreads();
     for (int k = 0; k + 1 < tail.numLevels; ++k) {
         const auto high = level(k), low = level(k + 1);
         for (int a0 = 0; a0 < low.H; a0 += TH)

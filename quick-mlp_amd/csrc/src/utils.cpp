@@ -142,11 +142,12 @@ size_t tailLdsBytes(int C, int H, int W, bool gradients, Tail* tail = nullptr)
 /**
  * The levels of the pyramid of a (B, C, H, W) image that have kernel launches of their own, finest first, with the views of
  * the low-res ones in the given workspaces (null: only the sizes are wanted, in 'bytes' and 'gradientBytes'). The levels
- * below the last one are left to the kernels that keep them in LDS: from there on where all of them fit (1 x 4 float:
+ * below the last one (their copy behind the forward pass: keptTail) are left to the kernels that keep them in LDS: from there on where all of them fit (1 x 4 float:
  * from 32 x 32 pixels on), as a step inside such a workgroup takes less than the 3 us of a launch.
  */
 template <typename T>
-std::vector<Level<T>> layout(int B, int C, int H, int W, void* pyramid, void* gradients, size_t* bytes = nullptr, size_t* gradientBytes = nullptr)
+std::vector<Level<T>> layout(int B, int C, int H, int W, void* pyramid, void* gradients, T*& keptTail, size_t* bytes = nullptr,
+                             size_t* gradientBytes = nullptr)
 {
     std::vector<Level<T>> levels(1);
     levels[0] = {};
@@ -178,6 +179,8 @@ std::vector<Level<T>> layout(int B, int C, int H, int W, void* pyramid, void* gr
         }
         levels.push_back(l);
     }
+    keptTail = forward.base ? forward.base + forward.entries : nullptr;
+    forward.entries += static_cast<size_t>(B) * (tailLdsBytes<T>(C, H, W, false) / sizeof(T));
     if (bytes) *bytes = forward.entries * sizeof(T);
     if (gradientBytes) *gradientBytes = adjoint.entries * sizeof(T);
     return levels;
@@ -185,12 +188,13 @@ std::vector<Level<T>> layout(int B, int C, int H, int W, void* pyramid, void* gr
 
 /** The levels below the last one with launches of its own, one workgroup per image. */
 template <typename T>
-void launchTail(KernelIndex kernel, int B, int C, Level<T> finest, bool gradients, stream_t stream)
+void launchTail(KernelIndex kernel, int B, int C, Level<T> finest, bool gradients, T* kept, stream_t stream)
 {
     if (isCoarsest(finest.H, finest.W)) return;
-    Tail tail = {};
+    Tail tail = {}, keptTail = {};
     const size_t lds = tailLdsBytes<T>(C, finest.H, finest.W, gradients, &tail);
-    void* args[] = {&finest, &C, &tail};
+    int keptEntries = static_cast<int>(tailLdsBytes<T>(C, finest.H, finest.W, false, &keptTail) / sizeof(T));
+    void* args[] = {&finest, &C, &tail, &kept, &keptEntries, &keptTail};   // (the last one for the gradients only)
     pullpushKernel<T>(kernel).launch(static_cast<unsigned>(B), TAIL_BLOCK, static_cast<unsigned>(lds), stream, args);
 }
 
@@ -218,21 +222,21 @@ void launchLevel(KernelIndex kernel, int B, int C, int height, int width, const 
 
 /** The pyramid down to the coarsest level and the inpainted levels up to levels[1]; with 'finest' up to levels[0]. */
 template <typename T>
-void runForward(const std::vector<Level<T>>& levels, int B, int C, bool finest, stream_t stream)
+void runForward(const std::vector<Level<T>>& levels, int B, int C, bool finest, T* keptTail, stream_t stream)
 {
     const int last = static_cast<int>(levels.size()) - 1;
     for (int l = 0; l < last; ++l) launchLevel(DOWN, B, C, levels[l + 1].H, levels[l + 1].W, levels, l, stream);
-    if (last > 0 || finest) launchTail(TAIL, B, C, levels[last], false, stream);
+    launchTail(TAIL, B, C, levels[last], false, keptTail, stream);
     for (int l = last - 1; l >= (finest ? 0 : 1); --l)
         launchLevel(UP, B, C, divUp(levels[l].H, 2), divUp(levels[l].W, 2), levels, l, stream);
 }
 
 template <typename T>
-void runAdjoint(const std::vector<Level<T>>& levels, int B, int C, bool accumulate, stream_t stream)
+void runAdjoint(const std::vector<Level<T>>& levels, int B, int C, bool accumulate, T* keptTail, stream_t stream)
 {
     const int last = static_cast<int>(levels.size()) - 1;
     for (int l = 0; l < last; ++l) launchLevel(GRADIENT_UP, B, C, levels[l + 1].H, levels[l + 1].W, levels, l, stream);
-    launchTail(last == 0 && accumulate ? GRADIENT_TAIL_ADD : GRADIENT_TAIL, B, C, levels[last], true, stream);
+    launchTail(last == 0 && accumulate ? GRADIENT_TAIL_ADD : GRADIENT_TAIL, B, C, levels[last], true, keptTail, stream);
     for (int l = last - 1; l >= 0; --l)
         launchLevel(l == 0 && accumulate ? GRADIENT_ADD : GRADIENT, B, C, divUp(levels[l].H, 2), divUp(levels[l].W, 2), levels, l, stream);
 }
@@ -267,11 +271,12 @@ void forward(const Tensor& mask, const Tensor& data, Tensor& output, void* pyram
         elementwise<T>(COPY_4, output, &data, stream);
         return;
     }
-    auto levels = layout<T>(B, C, H, W, pyramid, nullptr);
+    T* keptTail = nullptr;
+    auto levels = layout<T>(B, C, H, W, pyramid, nullptr, keptTail);
     levels[0].maskPre = viewOf<T>(mask);
     levels[0].dataPre = viewOf<T>(data);
     levels[0].dataPost = viewOf<T>(output);
-    runForward(levels, B, C, true, stream);
+    runForward(levels, B, C, true, keptTail, stream);
 }
 
 template <typename T>
@@ -284,14 +289,15 @@ void adjoint(const Tensor& mask, const Tensor& data, const Tensor& adjOutput, Te
         if (!accumulate) elementwise<T>(COPY_4, adjMask, nullptr, stream);   // the mask of a row or a column has no influence
         return;
     }
-    auto levels = layout<T>(B, C, H, W, pyramid, gradients);
+    T* keptTail = nullptr;
+    auto levels = layout<T>(B, C, H, W, pyramid, gradients, keptTail);
     levels[0].maskPre = viewOf<T>(mask);
     levels[0].dataPre = viewOf<T>(data);
-    if (!pyramidReady) runForward(levels, B, C, false, stream);
+    if (!pyramidReady) runForward(levels, B, C, false, keptTail, stream);
     levels[0].gradDataPost = viewOf<T>(adjOutput);
     levels[0].gradMaskPre = viewOf<T>(adjMask);
     levels[0].gradDataPre = viewOf<T>(adjData);
-    runAdjoint(levels, B, C, accumulate, stream);
+    runAdjoint(levels, B, C, accumulate, keptTail, stream);
 }
 
 void checkShapes(const Tensor& mask, const Tensor& data)
@@ -342,8 +348,13 @@ void Utils::pullpushMemory(const Tensor& data, size_t& pyramidBytes, size_t& gra
     pyramidBytes = gradientBytes = 0;
     if (data.numel() == 0) return;
     const int B = data.size(0), C = data.size(1), H = data.size(2), W = data.size(3);
-    if (data.precision() == Tensor::FLOAT) layout<float>(B, C, H, W, nullptr, nullptr, &pyramidBytes, &gradientBytes);
-    else layout<double>(B, C, H, W, nullptr, nullptr, &pyramidBytes, &gradientBytes);
+    if (data.precision() == Tensor::FLOAT) {
+        float* keptTail = nullptr;
+        layout<float>(B, C, H, W, nullptr, nullptr, keptTail, &pyramidBytes, &gradientBytes);
+    } else {
+        double* keptTail = nullptr;
+        layout<double>(B, C, H, W, nullptr, nullptr, keptTail, &pyramidBytes, &gradientBytes);
+    }
 }
 
 void Utils::fractionalPullpush(const Tensor& mask, const Tensor& data, Tensor& output, stream_t stream)
