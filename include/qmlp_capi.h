@@ -123,6 +123,14 @@ int qmlp_network_adjoint_memory(qmlp_network_t network, int num_elements, int ad
 int qmlp_network_adjoint(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* adj_output,
                          int adjoint_flags, const qmlp_tensor* adj_input, const void* tmp_memory_forward,
                          void* tmp_memory_adjoint, void* stream);
+/* Which of QMLP_GRADIENTS_INPUT and QMLP_GRADIENTS_NETWORK_WEIGHTS an adjoint pass on what the forward pass left in
+ * tmp_memory_forward can write, every element, instead of adding to them; and an adjoint pass that does so for the
+ * `overwrite` among them: those gradients need not be zeroed. */
+int qmlp_network_overwritable_gradients(qmlp_network_t network, int num_elements, int adjoint_flags,
+                                        const void* tmp_memory_forward, int* flags);
+int qmlp_network_adjoint_overwriting(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* adj_output,
+                                     int adjoint_flags, int overwrite, const qmlp_tensor* adj_input,
+                                     const void* tmp_memory_forward, void* tmp_memory_adjoint, void* stream);
 /* clearCachedKernels(), :319 */
 int qmlp_network_clear_cached_kernels(qmlp_network_t network);
 /* Generates and compiles all kernels of the network without touching a GPU

@@ -317,6 +317,8 @@ private:
      *  their intermediates: a training pass that is followed by it keeps the encoded input only. */
     bool recomputesFor(int numel, int flags) const;
     bool canRecompute(int flags, bool sliceGradients) const;
+    /** Whether the backward kernel itself adds input gradients of an encoding (those of sliced grids come from the kernels behind it). */
+    bool differentiatesEncodings(int flags, bool sliceGradients) const;
     mutable int recomputesKnown_[ADJOINT_MODE_MAX_COMBINATIONS][2];   // canRecompute(), -1: not known yet
     /**
      * recomputesFor(), and the backward kernel that runs the layers again holds its registers: loaded on the first
@@ -436,6 +438,19 @@ public:
      */
     void adjoint(const Tensor& input, const Tensor& adjOutput, AdjointModeFlags adjointFlags, Tensor& adjInput,
                  const void* tmpMemoryForward, void* tmpMemoryAdjoint, stream_t stream);
+    /**
+     * \param overwrite of GRADIENTS_INPUT and GRADIENTS_NETWORK_WEIGHTS those whose tensor holds nothing yet; only those that
+     *    overwritableGradients() names
+     */
+    void adjoint(const Tensor& input, const Tensor& adjOutput, AdjointModeFlags adjointFlags, Tensor& adjInput,
+                 const void* tmpMemoryForward, void* tmpMemoryAdjoint, stream_t stream, AdjointModeFlags overwrite);
+
+    /**
+     * Which of the gradients of the input and of the network weights adjoint() on what forward() left in tmpMemoryForward
+     * can write, every element, instead of adding to them: the caller need not zero them then, nor a kernel read them
+     * (2^20 points of 16 channels: 64 MB each; a fill kernel of 4 us in front of a small batch).
+     */
+    [[nodiscard]] AdjointModeFlags overwritableGradients(int numel, AdjointModeFlags adjointFlags, const void* tmpMemoryForward);
 
     /** For debugging, clears all cached kernels. */
     void clearCachedKernels();

@@ -273,13 +273,18 @@ public:
 
     /**
      * Standalone adjoint pass; adjInput (B, Cin) and the parameter gradients are accumulated.
-     * \param tmpMemory adjointMemory() bytes at a multiple of 256, which belong to this call until its kernels have
-     *    run; without them the parameter gradients are scattered with atomics
      */
     virtual void adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& adjInput, stream_t stream,
                          const std::optional<const Tensor>& parametersForward,
                          const std::optional<const Tensor>& parametersGradients,
-                         int adjointMode = AdjointMode::ALL_GRADIENTS, void* tmpMemory = nullptr);
+                         int adjointMode = AdjointMode::ALL_GRADIENTS);
+    /**
+     * \param tmpMemory adjointMemory() bytes at a multiple of 256, which belong to this call until its kernels have
+     *    run; without them the parameter gradients are scattered with atomics
+     */
+    void adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& adjInput, stream_t stream,
+                 const std::optional<const Tensor>& parametersForward,
+                 const std::optional<const Tensor>& parametersGradients, int adjointMode, void* tmpMemory);
 
     /**
      * Compiles the standalone forward kernel and, for adjointMode > 0, the adjoint kernels of

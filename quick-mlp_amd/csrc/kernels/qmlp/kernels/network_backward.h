@@ -144,15 +144,71 @@ $$ZERO_LDS_GRADIENTS$$
         && reinterpret_cast<unsigned long long>(adjOutputs.data_) % 8 == 0;
     const bool adjOutputRowsOfFloat4 = actualChannelsOut % 4 == 0 && adjOutputs.strides_[1] == 1 && adjOutputs.strides_[0] % 4 == 0
         && reinterpret_cast<unsigned long long>(adjOutputs.data_) % 16 == 0;
+    // Kernels that run the layers again read little per tile: dL/dy and the encoded input of this wavefront's next tile
+    // are asked for one tile ahead, behind the order of a sorted batch (the row of dL/dy) that is asked for two ahead. A
+    // wavefront's tiles follow each other with nothing else to hide the latency of three dependent loads (12 -> 16 -> 32 x 3
+    // -> 2 with a grid, 2^21 points: 154 -> 131 us).
+    constexpr bool LOADS_AHEAD = $$RECOMPUTES$$ && MTL == 1 && KT0 <= 2 && !HAS_STREAMED_LAYERS;
+    const int firstTile = static_cast<int>(blockIdx.x) * WAVES + wave, tileStep = static_cast<int>(gridDim.x) * WAVES;
+    (void)firstTile; (void)tileStep;
 #if $$HAS_OUTPUT_ORDER$$
     // a batch that trains in sorted order: the rows of dL/dy of this wavefront's next tile, asked for one tile ahead
     int adjRowAhead[NT];
+    auto loadRows = [&](int tile) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        const int p = (static_cast<int>(blockIdx.x) * WAVES + wave) * TILE_POINTS + 4 * r + nt;
-        adjRowAhead[nt] = (adjOutputOrder && p < numel) ? adjOutputOrder[p] : p;
-    }
+        for (int nt = 0; nt < NT; ++nt) {
+            const int p = tile * TILE_POINTS + 4 * r + nt;
+            adjRowAhead[nt] = p < numel ? (adjOutputOrder ? adjOutputOrder[p] : p) : 0;
+        }
+    };
+    loadRows(firstTile < numTiles ? firstTile : numTiles - 1);
 #endif
+    float4 dyAhead[NT];
+    f16x4 encodedAhead[LOADS_AHEAD ? KT0 : 1][4];
+    (void)dyAhead; (void)encodedAhead;
+    auto loadAhead = [&](int tile) {
+        const int last = numTiles - 1;
+        const int t0 = tile < last ? tile : last;   // (behind the last tile nobody looks at what is loaded)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const int p = t0 * TILE_POINTS + 4 * r + nt;
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (p < numel) {
+#if $$HAS_OUTPUT_ORDER$$
+                const long long adjRow = adjRowAhead[nt];
+#else
+                const long long adjRow = p;
+#endif
+                const float* row = adjOutputs.data_ + adjRow * adjOutputs.strides_[0];
+                if (adjOutputRowsOfFloat4) {
+                    if (4 * g < actualChannelsOut) v = *reinterpret_cast<const float4*>(row + 4 * g);
+                } else if (adjOutputRowsOfFloat2) {
+                    if (g == 0) {
+                        const float2 two = *reinterpret_cast<const float2*>(row);
+                        v.x = two.x, v.y = two.y;
+                    }
+                } else {
+                    const int c = 4 * g;
+                    const long long stride = adjOutputs.strides_[1];
+                    if (c < actualChannelsOut) v.x = row[c * stride];
+                    if (c + 1 < actualChannelsOut) v.y = row[(c + 1) * stride];
+                    if (c + 2 < actualChannelsOut) v.z = row[(c + 2) * stride];
+                    if (c + 3 < actualChannelsOut) v.w = row[(c + 3) * stride];
+                }
+            }
+            dyAhead[nt] = v;
+        }
+#if $$HAS_OUTPUT_ORDER$$
+        loadRows(t0 + tileStep < last ? t0 + tileStep : last);
+#endif
+        const f16* encTile = forwardTmpMemory + static_cast<long long>(t0) * (CHANNELS_IN * TILE_POINTS);
+#pragma unroll
+        for (int t = 0; t < KT0; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                encodedAhead[LOADS_AHEAD ? t : 0][i] = *reinterpret_cast<const f16x4*>(encTile + (16 * t + 4 * g + i) * TILE_POINTS + 4 * r);
+    };
+    if constexpr (LOADS_AHEAD) loadAhead(firstTile);
     for (int tileBase = blockIdx.x * WAVES; tileBase < numTiles; tileBase += gridDim.x * WAVES)
     {
         const int tile = tileBase + wave;
@@ -168,6 +224,13 @@ $$ZERO_LDS_GRADIENTS$$
             const int p = tile * TILE_POINTS + 4 * r + nt;
             const bool pv = p < numel;
             validMask |= pv ? (1 << nt) : 0;
+            if constexpr (LOADS_AHEAD) {
+                dyOut[nt][0][0] = static_cast<f16>(dyAhead[nt].x);
+                dyOut[nt][0][1] = static_cast<f16>(dyAhead[nt].y);
+                dyOut[nt][0][2] = static_cast<f16>(dyAhead[nt].z);
+                dyOut[nt][0][3] = static_cast<f16>(dyAhead[nt].w);
+                continue;
+            }
 #if $$HAS_OUTPUT_ORDER$$
             const long long adjRow = adjRowAhead[nt];
             {
@@ -257,6 +320,21 @@ $$CALL_ENCODINGS$$
 
                 if constexpr (HAS_INPUT_GRADIENTS) {
                     float* adjRow = adjInputs.data_ + static_cast<long long>(index) * adjInputs.strides_[0];
+#if $$HAS_OUTPUT_ORDER$$
+                    // (the rows of a sorted batch are the host's own, this kernel is the first to write them)
+                    if (adjOutputOrder) {
+                        if (NUM_INPUTS % 4 == 0 && adjInputs.strides_[1] == 1 && adjInputs.strides_[0] % 4 == 0
+                            && reinterpret_cast<unsigned long long>(adjInputs.data_) % 16 == 0) {
+#pragma unroll
+                            for (int i = 0; i + 3 < NUM_INPUTS; i += 4)
+                                *reinterpret_cast<float4*>(adjRow + i) = make_float4(adjEncodingInput[i], adjEncodingInput[i + 1],
+                                                                                    adjEncodingInput[i + 2], adjEncodingInput[i + 3]);
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < NUM_INPUTS; ++i) adjRow[static_cast<long long>(i) * adjInputs.strides_[1]] = adjEncodingInput[i];
+                        }
+                    } else
+#endif
                     if (!HAS_ENCODING_GRADIENTS && NUM_INPUTS % 4 == 0 && adjInputs.strides_[1] == 1 && adjInputs.strides_[0] % 4 == 0
                         && reinterpret_cast<unsigned long long>(adjInputs.data_) % 16 == 0) {
                         // the channels of a row side by side: four per load and store. Kept to

@@ -41,7 +41,8 @@ __global__ void __launch_bounds__($$BLOCK_SIZE$$) $$KERNEL_ATTRIBUTES$$ NetworkK
     half* __restrict__ adjointTmpMemoryH,        //receives the adjoint of the encoded input (STORE_ENCODED_ADJOINT)
     float* __restrict__ partialGradients,        //partialSlices x the layout of the parameters; workgroup b stores the sums of
     int partialSlices,                           //its tiles into slice b (and zeroes slices b + k * gridDim.x)
-    const int* __restrict__ adjOutputOrder       //nullptr, or (numel) the row of adjOutputs that belongs to point p
+    const int* __restrict__ adjOutputOrder,      //nullptr, or (numel) the row of adjOutputs that belongs to point p
+    int overwriteInputs                          //adjInputs holds nothing yet: written, not added to
     $$ENCODING_PARAMETERS$$)
 {
     constexpr int NUM_INPUTS = $$NUM_INPUTS$$;
@@ -176,11 +177,17 @@ $$CALL_NETWORK_LAYERS$$
                     const int c = 16 * t + 4 * g;
                     if (16 * t + 15 < ENCODED_CHANNELS && rowsOfFloat4) {
                         f32x4* target = reinterpret_cast<f32x4*>(row + c);
-                        *target = *target + __builtin_convertvector(dxIn[nt][t], f32x4);
+                        f32x4 v = __builtin_convertvector(dxIn[nt][t], f32x4);
+                        if (!overwriteInputs) v = *target + v;
+                        *target = v;
                     } else {
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
-                            if (c + i < ENCODED_CHANNELS) row[static_cast<long long>(c + i) * adjInputs.strides_[1]] += static_cast<float>(dxIn[nt][t][i]);
+                            if (c + i < ENCODED_CHANNELS) {
+                                float* target = row + static_cast<long long>(c + i) * adjInputs.strides_[1];
+                                const float v = static_cast<float>(dxIn[nt][t][i]);
+                                *target = overwriteInputs ? v : *target + v;
+                            }
                     }
                 }
             }
@@ -209,7 +216,10 @@ $$CALL_NETWORK_LAYERS$$
 $$CALL_ENCODINGS$$
                 float* adjRow = adjInputs.data_ + static_cast<long long>(index) * adjInputs.strides_[0];
 #pragma unroll
-                for (int i = 0; i < NUM_INPUTS; ++i) adjRow[static_cast<long long>(i) * adjInputs.strides_[1]] += adjEncodingInput[i];
+                for (int i = 0; i < NUM_INPUTS; ++i) {
+                    float* target = adjRow + static_cast<long long>(i) * adjInputs.strides_[1];
+                    *target = overwriteInputs ? adjEncodingInput[i] : *target + adjEncodingInput[i];
+                }
             }
             waveLdsSync();
         }

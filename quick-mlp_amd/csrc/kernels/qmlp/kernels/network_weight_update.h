@@ -162,11 +162,11 @@ __global__ void __launch_bounds__($$BLOCK_SIZE$$) WeightUpdateKernel(
 }
 
 /**
- * gradients[i] += sum over the slices of partial[slice * count + i]. One workgroup of
+ * gradients[i] += (overwrite: =) sum over the slices of partial[slice * count + i]. One workgroup of
  * 1024 threads per 64 parameters: 16 wavefronts each sum every 16th slice, LDS combines them.
  */
 __global__ void __launch_bounds__(1024) WeightUpdateReduceKernel(
-    int count, int numSlices, const float* __restrict__ partial, float* __restrict__ gradients)
+    int count, int numSlices, const float* __restrict__ partial, float* __restrict__ gradients, int overwrite)
 {
     __shared__ float sSum[16][WAVE_SIZE];
     const int lane = threadIdx.x % WAVE_SIZE;
@@ -190,7 +190,7 @@ __global__ void __launch_bounds__(1024) WeightUpdateReduceKernel(
         float total = 0.f;
 #pragma unroll
         for (int w = 0; w < 16; ++w) total += sSum[w][lane];
-        gradients[i] += total;
+        gradients[i] = overwrite ? total : gradients[i] + total;
     }
 }
 

@@ -344,6 +344,25 @@ int qmlp_network_adjoint(qmlp_network_t network, const qmlp_tensor* input, const
     QMLP_API_END
 }
 
+int qmlp_network_overwritable_gradients(qmlp_network_t network, int num_elements, int adjoint_flags,
+                                        const void* tmp_memory_forward, int* flags)
+{
+    QMLP_API_BEGIN
+    *flags = network->network->overwritableGradients(num_elements, adjoint_flags, tmp_memory_forward);
+    QMLP_API_END
+}
+
+int qmlp_network_adjoint_overwriting(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* adj_output,
+                                     int adjoint_flags, int overwrite, const qmlp_tensor* adj_input,
+                                     const void* tmp_memory_forward, void* tmp_memory_adjoint, void* stream)
+{
+    QMLP_API_BEGIN
+    Tensor adjIn = wrap(adj_input);
+    network->network->adjoint(wrap(input), wrap(adj_output), adjoint_flags, adjIn, tmp_memory_forward,
+                              tmp_memory_adjoint, static_cast<stream_t>(stream), overwrite);
+    QMLP_API_END
+}
+
 int qmlp_network_clear_cached_kernels(qmlp_network_t network)
 {
     QMLP_API_BEGIN

@@ -1074,6 +1074,7 @@ std::string FusedNetwork::backwardSource(int flags, int blockSize, bool sliceGra
     fillEncodingsAndActivations(code);
     replaceAll(code, "$$BLOCK_SIZE$$", std::to_string(blockSize));
     replaceAll(code, "$$HAS_OUTPUT_ORDER$$", trainsSortedBatches() ? "1" : "0");
+    replaceAll(code, "$$RECOMPUTES$$", recompute ? "true" : "false");
     bool wideRegisters = false;
     (void)fusedWeightUpdateLayers(flags, sliceGradients, &wideRegisters);
     // (the pre-activations of all layers stay in registers beside the gradient tiles: 256 registers spilled 404 bytes
@@ -1204,8 +1205,10 @@ std::string FusedNetwork::backwardSource(int flags, int blockSize, bool sliceGra
             forward << "        f16x4 x0Kept[NT][Layer0::KT];\n        {\n"
                     << "            const f16* encTile = forwardTmpMemory + static_cast<long long>(tileRead) * (CHANNELS_IN * TILE_POINTS);\n"
                     << "#pragma unroll\n            for (int t = 0; t < KT0; ++t)\n#pragma unroll\n                for (int i = 0; i < 4; ++i) {\n"
-                    << "                    const f16x4 v = *reinterpret_cast<const f16x4*>(encTile + (16 * t + 4 * g + i) * TILE_POINTS + 4 * r);\n"
-                    << "#pragma unroll\n                    for (int nt = 0; nt < NT; ++nt) x0Kept[nt][t][i] = v[nt];\n                }\n        }\n";
+                    << "                    const f16x4 v = LOADS_AHEAD ? encodedAhead[LOADS_AHEAD ? t : 0][i]\n"
+                    << "                        : *reinterpret_cast<const f16x4*>(encTile + (16 * t + 4 * g + i) * TILE_POINTS + 4 * r);\n"
+                    << "#pragma unroll\n                    for (int nt = 0; nt < NT; ++nt) x0Kept[nt][t][i] = v[nt];\n                }\n        }\n"
+                    << "        if constexpr (LOADS_AHEAD) loadAhead(tile + tileStep);\n";
             for (int i = 0; i < L; ++i) {
                 const auto& l = layers_[i];
                 const std::string in = i == 0 ? std::string("x0Kept") : "act" + std::to_string(i);
@@ -2345,8 +2348,40 @@ size_t FusedNetwork::adjointMemory(const Tensor& input, AdjointModeFlags adjoint
     return adjointMemory(input.size(0), adjointFlags);
 }
 
+bool FusedNetwork::differentiatesEncodings(int flags, bool sliceGradients) const
+{
+    if (!(flags & GRADIENTS_INPUT)) return false;
+    for (const auto& e : encodings_)
+        if (!((flags & GRADIENTS_INPUT_ENCODINGS) && sliceGradients && offersSlices(*e))) return true;
+    return false;
+}
+
+FusedNetwork::AdjointModeFlags FusedNetwork::overwritableGradients(int numel, AdjointModeFlags adjointFlags, const void* tmpMemoryForward)
+{
+    if (numel <= 0) return 0;
+    // the sums of the weight gradients, all of them, are written at the end
+    const int weights = adjointFlags & GRADIENTS_NETWORK_WEIGHTS;
+    if (!(adjointFlags & GRADIENTS_INPUT)) return weights;
+    // the rows of a batch that trained in sorted order are moved to the caller's tensor, all of them, at the end
+    if (sortsTraining(numel)) return weights | GRADIENTS_INPUT;
+    const auto it = forwardRecords_.find(tmpMemoryForward);
+    if (it == forwardRecords_.end() || it->second.numel != numel || it->second.mode != BACKWARD_COOPERATIVE
+        || backwardMode(numel, adjointFlags) != BACKWARD_COOPERATIVE)
+        return weights;
+    // the cooperative kernel: one that reads the input rows writes the channels of its encoding, else all of them
+    const bool all = differentiatesEncodings(adjointFlags, useSliceGradients(numel, adjointFlags))
+        && (directInputStart() < 0 || (directInputStart() == 0 && encodings_[0]->numOutputChannels() == channelsIn()));
+    return all ? weights | GRADIENTS_INPUT : weights;
+}
+
 void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, AdjointModeFlags adjointFlags,
                            Tensor& adjInput, const void* tmpMemoryForward, void* tmpMemoryAdjoint, stream_t stream)
+{
+    adjoint(input, adjOutput, adjointFlags, adjInput, tmpMemoryForward, tmpMemoryAdjoint, stream, 0);
+}
+
+void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, AdjointModeFlags adjointFlags,
+                           Tensor& adjInput, const void* tmpMemoryForward, void* tmpMemoryAdjoint, stream_t stream, AdjointModeFlags overwrite)
 {
     CHECK_DIM(input, 2);
     CHECK_DIM(adjOutput, 2);
@@ -2389,6 +2424,9 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
     const bool sliceGradients = useSliceGradients(numel, adjointFlags);
     CHECK_ERROR(!sliceGradients || numel < (1 << 27), "batches of 2^27 points or more: set options.slice_gradients to 0");
     announcedFlags_ = adjointFlags;
+    CHECK_ERROR((overwrite & ~overwritableGradients(numel, adjointFlags, tmpMemoryForward)) == 0,
+                "adjoint() adds to gradients of this batch that it was asked to overwrite");
+    const bool overwriteInputGradients = overwrite & GRADIENTS_INPUT;
     // what the forward pass that wrote this forward memory left there: the position derivatives of the grids? Of the
     // intermediates the encoded input only?
     bool derivativesStored = false;
@@ -2446,7 +2484,9 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
         char* staging = static_cast<char*>(tmpMemoryAdjoint) + roundUp(adjointMemoryAsGiven(numel, adjointFlags), size_t(256));
         if (hasInputGradients) {
             float* adjInputRows = reinterpret_cast<float*>(staging);
-            QMLP_HIP_CALL(qmlp_hip_memset_async(adjInputRows, 0, static_cast<size_t>(numel) * channelsIn() * sizeof(float), stream));
+            // (where an encoding is differentiated by the backward kernel, that writes all rows)
+            if (!differentiatesEncodings(adjointFlags, sliceGradients))
+                QMLP_HIP_CALL(qmlp_hip_memset_async(adjInputRows, 0, static_cast<size_t>(numel) * channelsIn() * sizeof(float), stream));
             sortedAdjInput.data_ = adjInputRows;
             sortedAdjInput.strides_[0] = channelsIn();
             sortedAdjInput.strides_[1] = 1;
@@ -2491,6 +2531,8 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
         args.insert(args.end(), {&partialGradients, &partialSlices});
         CHECK_ERROR(ak.outputOrder || adjOutputOrder == nullptr, "a batch trains in sorted order but the backward kernel does not take the order");
         if (ak.outputOrder) args.push_back(&adjOutputOrder);
+        int overwriteRows = sortedPoints || overwriteInputGradients ? 1 : 0;
+        if (cooperative) args.push_back(&overwriteRows);
         std::vector<std::vector<char>> storage;
         encodingArguments(args, storage);
         ck.fun.launch(grid, ck.blockSize, ck.sharedMemorySize, stream, args.data());
@@ -2582,9 +2624,11 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
         const float* src = sortedAdjInput.data_;
         auto dst = adjInput.accessor<kernel::Tensor2RW<float>>();
         const int* placement = reinterpret_cast<const int*>(static_cast<const char*>(tmpMemoryForward) + sortedPlacementOffset(numel));
-        void* args[] = {&elements, &channels, &src, &placement, &dst};
-        pointOrder_.gatherAddRows.value().launch(static_cast<int>(std::min<long long>(divUp<long long>(elements, 1024), 1 << 16)), 1024, 0,
-                                                  stream, args);
+        int overwriteRows = overwriteInputGradients ? 1 : 0;
+        void* args[] = {&elements, &channels, &src, &placement, &dst, &overwriteRows};
+        // (a lane moves an element, or four rows of four)
+        pointOrder_.gatherAddRows.value().launch(static_cast<int>(std::min<long long>(divUp<long long>(elements, channels == 4 ? 16 * 1024 : 1024), 1 << 16)),
+                                                  1024, 0, stream, args);
     }
 
     if (!hasNetworkGradients) return;
@@ -2626,7 +2670,8 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
         int count = numParameters_, numSlices = slices;
         const float* partialArg = partial;
         float* gradBase = parametersGradients_.dataPtr<float>();
-        void* args[] = {&count, &numSlices, &partialArg, &gradBase};
+        int overwriteWeights = overwrite & GRADIENTS_NETWORK_WEIGHTS ? 1 : 0;
+        void* args[] = {&count, &numSlices, &partialArg, &gradBase, &overwriteWeights};
         ak.reduce.fun.launch(divUp(numParameters_, WARP_SIZE), ak.reduce.blockSize, 0, stream, args);
     }
 }

@@ -140,6 +140,13 @@ void IEncoding::forward(const Tensor& input, Tensor& output, stream_t stream,
 
 void IEncoding::adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& adjInput, stream_t stream,
                         const std::optional<const Tensor>& parametersForward,
+                        const std::optional<const Tensor>& parametersGradients, int adjointMode)
+{
+    adjoint(input, adjOutput, adjInput, stream, parametersForward, parametersGradients, adjointMode, nullptr);
+}
+
+void IEncoding::adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& adjInput, stream_t stream,
+                        const std::optional<const Tensor>& parametersForward,
                         const std::optional<const Tensor>& parametersGradients, int adjointMode, void* tmpMemory)
 {
     CHECK_DIM(input, 2);

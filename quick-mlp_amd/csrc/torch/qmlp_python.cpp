@@ -192,15 +192,13 @@ struct FusedBackward : torch::autograd::Node
         at::AutoDispatchBelowADInplaceOrView guard;
         const at::Tensor gradOutput = gradOutputs[0].contiguous();
         at::Tensor adjInput, adjNetwork;
-        if (flags & QMLP_GRADIENTS_INPUT) adjInput = at::zeros_like(x);
-        if (flags & QMLP_GRADIENTS_NETWORK_WEIGHTS) adjNetwork = at::zeros(parameters.sizes(), parameters.options().dtype(at::kFloat));
         if (flags & QMLP_GRADIENTS_INPUT_ENCODINGS)
             // the kernel adds the gradients of every encoding with parameters: a frozen one gets a zero tensor as
             // well, which is dropped below (bind_network.cpp:277-290)
             for (size_t i = 0; i < n; ++i)
                 if (net->encodings[i].hasParameters) adjTables[i] = at::zeros(unpacked[i].sizes(), unpacked[i].options().dtype(at::kFloat));
         const auto wrappedTables = wrapAll(*net, unpacked);
-        const qmlp_tensor p = wrap(parameters), in = wrap(x), adjOut = wrap(gradOutput), adjIn = wrap(adjInput), adjNet = wrap(adjNetwork);
+        const qmlp_tensor p = wrap(parameters), in = wrap(x), adjOut = wrap(gradOutput);
         std::vector<qmlp_tensor> adjEnc(n);
         for (size_t i = 0; i < n; ++i) adjEnc[i] = wrap(adjTables[i]);
         void* stream = currentStream(x);
@@ -210,10 +208,20 @@ struct FusedBackward : torch::autograd::Node
             check(qmlp_network_adjoint_memory(net->handle, in.sizes[0], flags, &bytes));
             const at::Tensor scratch = bytesOn(x, bytes);
             net->bind(p, wrappedTables);
+            // zeroed only where the kernels add to them
+            int overwrite = 0;
+            check(qmlp_network_overwritable_gradients(net->handle, in.sizes[0], flags, memory.data_ptr(), &overwrite));
+            if (flags & QMLP_GRADIENTS_INPUT) adjInput = overwrite & QMLP_GRADIENTS_INPUT ? at::empty_like(x) : at::zeros_like(x);
+            if (flags & QMLP_GRADIENTS_NETWORK_WEIGHTS) {
+                const auto options = parameters.options().dtype(at::kFloat);
+                adjNetwork = overwrite & QMLP_GRADIENTS_NETWORK_WEIGHTS ? at::empty(parameters.sizes(), options) : at::zeros(parameters.sizes(), options);
+            }
+            const qmlp_tensor adjIn = wrap(adjInput), adjNet = wrap(adjNetwork);
             if (adjNetwork.defined()) check(qmlp_network_set_parameter(net->handle, &adjNet, QMLP_GRADIENTS));
             for (size_t i = 0; i < n; ++i)
                 if (adjTables[i].defined()) check(qmlp_encoding_set_parameter(net->encodings[i].handle, &adjEnc[i], QMLP_GRADIENTS));
-            const int rc = qmlp_network_adjoint(net->handle, &in, &adjOut, flags, &adjIn, memory.data_ptr(), scratch.data_ptr(), stream);
+            const int rc = qmlp_network_adjoint_overwriting(net->handle, &in, &adjOut, flags, overwrite, &adjIn, memory.data_ptr(),
+                                                            scratch.data_ptr(), stream);
             const std::string message = rc != 0 ? qmlp_last_error() : "";
             // no dangling gradient bindings, whatever happened
             qmlp_network_set_parameter(net->handle, nullptr, QMLP_GRADIENTS);

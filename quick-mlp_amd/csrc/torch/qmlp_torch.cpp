@@ -453,12 +453,16 @@ struct NetworkFunction : torch::autograd::Function<NetworkFunction>
 
         torch::Tensor adjInput, adjNetwork;
         std::vector<torch::Tensor> adjEncodings(encodingParameters.size());
-        if (flags & QMLP_GRADIENTS_INPUT) adjInput = torch::zeros_like(input);
         {
             std::lock_guard<std::mutex> lock(net->mutex_);
             net->bindParameters(p16, encodingParameters);
+            // zeroed only where the kernels add to them
+            int overwrite = 0;
+            QMLP_CHECK(qmlp_network_overwritable_gradients(net->handle_, static_cast<int>(input.size(0)), flags, tmpForward.data_ptr(), &overwrite));
+            if (flags & QMLP_GRADIENTS_INPUT) adjInput = overwrite & QMLP_GRADIENTS_INPUT ? torch::empty_like(input) : torch::zeros_like(input);
             if (flags & QMLP_GRADIENTS_NETWORK_WEIGHTS) {
-                adjNetwork = torch::zeros(p16.sizes(), p16.options().dtype(torch::kFloat32));
+                const auto options = p16.options().dtype(torch::kFloat32);
+                adjNetwork = overwrite & QMLP_GRADIENTS_NETWORK_WEIGHTS ? torch::empty(p16.sizes(), options) : torch::zeros(p16.sizes(), options);
                 const qmlp_tensor g = wrap(adjNetwork);
                 QMLP_CHECK(qmlp_network_set_parameter(net->handle_, &g, QMLP_GRADIENTS));
             }
@@ -479,8 +483,8 @@ struct NetworkFunction : torch::autograd::Function<NetworkFunction>
             auto tmpAdjoint = torch::empty({static_cast<int64_t>(std::max<size_t>(bytes, 16))},
                                            torch::TensorOptions().dtype(torch::kUInt8).device(input.device()));
             const qmlp_tensor in = wrap(input), adjOut = wrap(gradOutput), adjIn = wrap(adjInput);
-            const int rc = qmlp_network_adjoint(net->handle_, &in, &adjOut, flags, &adjIn, tmpForward.data_ptr(),
-                                                tmpAdjoint.data_ptr(), currentStream());
+            const int rc = qmlp_network_adjoint_overwriting(net->handle_, &in, &adjOut, flags, overwrite, &adjIn, tmpForward.data_ptr(),
+                                                            tmpAdjoint.data_ptr(), currentStream());
             // no dangling gradient bindings, whatever happened
             qmlp_network_set_parameter(net->handle_, nullptr, QMLP_GRADIENTS);
             for (size_t i = 0; i < adjEncodings.size(); ++i)
