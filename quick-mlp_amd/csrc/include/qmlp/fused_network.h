@@ -159,11 +159,12 @@ private:
         int pointsPerLane = 1;
         int sharedMemorySize = 0;
         int fullGrid = 0;
+        int tilesPerWorkgroup = 1;   // of the forward kernels
     };
     // [store intermediates][variant], see ForwardVariant
     // [0]: inference, [1]: forward (stores the intermediates), [2]: forward that also stores position derivatives
     // ([3], [4]: as [1], [2], but of the intermediates only the encoded input is stored)
-    std::optional<CompiledKernel> forwardKernels_[5][4];
+    std::optional<CompiledKernel> forwardKernels_[5][5];
     // set once the compiled REGISTERS shape turned out to spill heavily: it is not used then
     bool registerShapeSpills_[5] = {false, false, false, false, false};
 
@@ -480,10 +481,15 @@ private:
     // wavefront for small batches.
     // REGISTERS: 8 wavefronts whose encoded rows wait in registers (up to 8 tiles each) and pass
     // through one LDS staging tile per wavefront: one sweep over the level tables per 2^20 points.
-    enum ForwardVariant { VARIANT_DEFAULT = 0, VARIANT_NARROW = 1, VARIANT_LARGE = 2, VARIANT_REGISTERS = 3 };
+    // SHARED: wavefronts that share the levels of a tile, for small batches of networks with grids of many levels.
+    enum ForwardVariant { VARIANT_DEFAULT = 0, VARIANT_NARROW = 1, VARIANT_LARGE = 2, VARIANT_REGISTERS = 3, VARIANT_SHARED = 4 };
     bool hasLargeVariant(bool store) const;
     /** Tiles per wavefront of the REGISTERS shape, 0 if the network has none. */
     int registerVariantTiles(bool store) const;
+    /** Wavefronts per workgroup of the SHARED shape, 0 if the network has none. */
+    int sharedTileWaves(bool store) const;
+    mutable int sharedTileWaves_[2] = {-1, -1};
+    static constexpr int SHARED_TILE_MAX_TILES = 448;   // from about 500 on the other shapes are faster, see kernels/network_forward.h
     /** Workgroup size and tiles per wavefront of a shape of the forward kernel. */
     void forwardShape(bool store, int variant, int& blockSize, int& pointsPerLane) const;
     void compileForwardKernel(bool store, int variant, bool compileOnly = false, bool derivatives = false, bool inputOnly = false);
@@ -517,7 +523,7 @@ private:
     size_t sortedPlacementOffset(int numel) const;
     void compileRecordsKernel(SliceGradientKernel& sk, int flags, size_t variant, bool compileOnly, bool fromDerivatives = false);
 
-    std::string forwardSource(int blockSize, int pointsPerLane, bool registerStaging = false, bool derivatives = false, bool inputOnly = false) const;
+    std::string forwardSource(int blockSize, int pointsPerLane, bool registerStaging = false, bool derivatives = false, bool inputOnly = false, bool sharedTile = false) const;
     std::string backwardSource(int flags, int blockSize, bool sliceGradients = false, bool recompute = false, bool twoWavefrontsPerSimd = false) const;
     std::string weightUpdateSource(int blockSize) const;
     std::string weightUpdateKernelName(int layer, int& numChunks, int& tilesPerBlock) const;

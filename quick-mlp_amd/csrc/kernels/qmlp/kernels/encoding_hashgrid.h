@@ -470,8 +470,9 @@ struct EncodingHashGrid
      * Level-major evaluation of PPL points of one lane: all points finish level l before
      * any starts level l+1, so that the workgroups of the device sweep through the level
      * tables together and a level's table stays in L2 while it is in use.
+     * \tparam FIRST, END the levels from FIRST to END - 1 only (of levels that are concatenated)
      */
-    template <int PPL, typename I, typename Os, typename Derivatives = NoPositionDerivatives>
+    template <int PPL, int FIRST = 0, int END = L, typename I, typename Os, typename Derivatives = NoPositionDerivatives>
     __device__ __forceinline__ static void forwardBatch(const I (&inputs)[PPL], Os& outputs, const param_t& params,
                                                         const Derivatives& derivatives = Derivatives{})
     {
@@ -485,7 +486,7 @@ struct EncodingHashGrid
 #pragma unroll
             for (int i = 0; i < F; ++i) sum[q][i] = 0.f;
 #pragma unroll
-        for (int l = 0; l < L; ++l) {
+        for (int l = FIRST; l < END; ++l) {
             float feat[PPL][F];
 #pragma unroll
             for (int q = 0; q < PPL; ++q) {
@@ -549,6 +550,15 @@ struct EncodingHashGrid
 #pragma unroll
             for (int i = 0; i < F; ++i) output[i] = fcast<O_t>(sum[i]);
         }
+    }
+
+    /** The share of wavefront `wave` of WAVES in forwardBatch() of one tile: some of the levels (concatenated levels). */
+    template <int WAVES, int WAVE = 0, typename I, typename Os, typename Derivatives = NoPositionDerivatives>
+    __device__ __forceinline__ static void forwardBatchShared(int wave, const I (&inputs)[1], Os& outputs, const param_t& params,
+                                                              const Derivatives& derivatives = Derivatives{})
+    {
+        if (wave == WAVE) forwardBatch<1, L * WAVE / WAVES, L * (WAVE + 1) / WAVES>(inputs, outputs, params, derivatives);
+        else if constexpr (WAVE + 1 < WAVES) forwardBatchShared<WAVES, WAVE + 1>(wave, inputs, outputs, params, derivatives);
     }
 
     /** The features of the levels of one of GROUPS groups (concatenated levels), from the group's first feature on. */

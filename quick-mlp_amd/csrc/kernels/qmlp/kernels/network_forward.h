@@ -84,6 +84,13 @@ __global__ void __launch_bounds__($$BLOCK_SIZE$$) $$KERNEL_ATTRIBUTES$$ NetworkK
     constexpr int DIRECT_INPUT_START = $$DIRECT_INPUT_START$$;
     constexpr bool DIRECT_INPUT = DIRECT_INPUT_START >= 0;
     static_assert(!DIRECT_INPUT || PPL == 1, "direct input rows: one tile per wave");
+    // For small batches of networks with grids of many levels: the wavefronts of the workgroup share the levels of one tile,
+    // whose rows they write to the same staging rows, and the first of them runs the layers. A batch that leaves most of the
+    // device idle waits for the entries of one level after the other (16 levels of 2 halves, inference of 64 / 2000 / 8000 /
+    // 20 011 / 32 768 points 16 / 20 / 29 / 30 / 31 us with a tile per wavefront, 9 / 9 / 12 / 24 / 29 us so).
+    constexpr bool SHARED_TILE = $$SHARED_TILE$$;
+    static_assert(!SHARED_TILE || (PPL == 1 && !REGISTER_STAGING && !HAS_STREAMED_LAYERS && !DIRECT_INPUT), "a tile of the workgroup");
+    constexpr int GROUP_TILES = SHARED_TILE ? 1 : WAVES * PPL;
 
     const f16* __restrict__ networkParameters = reinterpret_cast<const f16*>(networkParametersH);
     f16* __restrict__ forwardTmpMemory = reinterpret_cast<f16*>(forwardTmpMemoryH);
@@ -93,7 +100,7 @@ __global__ void __launch_bounds__($$BLOCK_SIZE$$) $$KERNEL_ATTRIBUTES$$ NetworkK
     const int wave = threadIdx.x / WAVE_SIZE;
     const int lane = threadIdx.x % WAVE_SIZE;
     const int g = lane >> 4, r = lane & 15;
-    f16* sStage = sParams + LDS_PARAM_HALVES + wave * (STAGED_TILES * TILE_POINTS * STAGE_STRIDE);
+    f16* sStage = sParams + LDS_PARAM_HALVES + (SHARED_TILE ? 0 : wave) * (STAGED_TILES * TILE_POINTS * STAGE_STRIDE);
     (void)sStage;
 
     // stage the weights in operand order, then the biases
@@ -108,9 +115,9 @@ $$STAGE_PARAMETERS$$
     // the regions of the temporary memory are laid out for the whole batch
     const long long numel64 = static_cast<long long>(tmpNumTiles) * TILE_POINTS;
     (void)numel64;
-    for (int tileBase = blockIdx.x * WAVES * PPL; tileBase < numTiles; tileBase += gridDim.x * WAVES * PPL)
+    for (int tileBase = blockIdx.x * GROUP_TILES; tileBase < numTiles; tileBase += gridDim.x * GROUP_TILES)
     {
-        const int tile0 = tileBase + wave * PPL;
+        const int tile0 = SHARED_TILE ? tileBase : tileBase + wave * PPL;
         if (!HAS_STREAMED_LAYERS && tile0 >= numTiles) continue;
 
         // encodings: PPL points per lane (one of each tile), each into its staging row.
@@ -151,8 +158,10 @@ $$STAGE_PARAMETERS$$
                 }
             }
 $$CALL_ENCODINGS$$
+            if constexpr (SHARED_TILE) __syncthreads();
 #pragma unroll
             for (int q = 0; q < PPL; ++q) {
+                if (SHARED_TILE && wave != 0) break;
 #pragma unroll
                 for (int c = ENCODED_CHANNELS; c < CHANNELS_IN; ++c) encodingOutput[q][c] = static_cast<f16>(0);
                 if (!valid[q]) {
@@ -168,6 +177,7 @@ $$TILE_LOOP_PRAGMA$$
         {
         const int tile = tile0 + q;
         if (!HAS_STREAMED_LAYERS && tile >= numTiles) break;
+        if (SHARED_TILE && wave != 0) break;
         const bool tileValid = tile < numTiles;
         const int tmpTile = tile + tmpTileOffset;
         (void)tmpTile;
@@ -308,7 +318,8 @@ $$CALL_NETWORK_LAYERS$$
                 }
         }
         }
-        if constexpr (!DIRECT_INPUT) waveLdsSync();   // the staging rows are overwritten by the next group of tiles
+        if constexpr (SHARED_TILE) __syncthreads();
+        else if constexpr (!DIRECT_INPUT) waveLdsSync();   // the staging rows are overwritten by the next group of tiles
     }
 }
 

@@ -897,7 +897,7 @@ static std::string layerTypedefs(const std::vector<std::string>& layerTypes)
     return ss.str();
 }
 
-std::string FusedNetwork::forwardSource(int blockSize, int pointsPerLane, bool registerStaging, bool derivatives, bool inputOnly) const
+std::string FusedNetwork::forwardSource(int blockSize, int pointsPerLane, bool registerStaging, bool derivatives, bool inputOnly, bool sharedTile) const
 {
     auto kl = QuickMLP::Instance().kernelLoader();
     std::string code = kl->findFile("qmlp/kernels/network_forward.h").value();
@@ -905,6 +905,7 @@ std::string FusedNetwork::forwardSource(int blockSize, int pointsPerLane, bool r
     replaceAll(code, "$$BLOCK_SIZE$$", std::to_string(blockSize));
     replaceAll(code, "$$POINTS_PER_LANE$$", std::to_string(pointsPerLane));
     replaceAll(code, "$$REGISTER_STAGING$$", registerStaging ? "true" : "false");
+    replaceAll(code, "$$SHARED_TILE$$", sharedTile ? "true" : "false");
     replaceAll(code, "$$DIRECT_INPUT_START$$", std::to_string(directInputStart()));
     replaceAll(code, "$$KERNEL_ATTRIBUTES$$", kernelAttributes(blockSize));
     // rows in registers are indexed by the tile: that loop has to be unrolled
@@ -950,6 +951,13 @@ std::string FusedNetwork::forwardSource(int blockSize, int pointsPerLane, bool r
                           << "#pragma unroll\n                for (int q = 0; q < PPL; ++q) encodingOutputK[q] = encodingOutput[q] + "
                           << encodingOffset << ";\n                ";
         const auto* slices = slicesOf(*e);
+        // (sharedTile: grids by level, other encodings by one of the wavefronts)
+        const int waves = blockSize / WARP_SIZE;
+        std::string callForward = e->qualifiedName() + "::template forwardBatch<PPL>(";
+        if (sharedTile && e->levelGroups() > 1)
+            callForward = e->qualifiedName() + "::template forwardBatchShared<WAVES>(__builtin_amdgcn_readfirstlane(wave), ";
+        else if (sharedTile)
+            callForward = "if (wave == " + std::to_string(waves - 1 - static_cast<int>(encodingIdx) % waves) + ") " + callForward;
         if (derivatives && derivativeOffsets_[encodingIdx] >= 0 && slices) {
             const auto& sliceLayout = *slices;
             // the lane's chunks of its first tile; the tiles of a wave follow one another
@@ -960,10 +968,10 @@ std::string FusedNetwork::forwardSource(int blockSize, int pointsPerLane, bool r
                           << (static_cast<long long>(perEntryForwardMemoryBytes_) + derivativeOffsets_[encodingIdx]) << "ll * numel64)\n"
                           << "                        + DerivativeLayout::chunkIndex(tile0 + tmpTileOffset, 0, 0, lane),\n"
                           << "                    numTiles - tile0};\n                ";
-            callEncodings << e->qualifiedName() << "::template forwardBatch<PPL>(encodingInput, encodingOutputK, cEncoding" << encodingIdx
+            callEncodings << callForward << "encodingInput, encodingOutputK, cEncoding" << encodingIdx
                           << ", derivatives);\n            }\n";
         } else {
-            callEncodings << e->qualifiedName() << "::template forwardBatch<PPL>(encodingInput, encodingOutputK";
+            callEncodings << callForward << "encodingInput, encodingOutputK";
             if (e->hasParameters()) callEncodings << ", cEncoding" << encodingIdx;
             callEncodings << ");\n            }\n";
         }
@@ -1434,6 +1442,7 @@ std::string FusedNetwork::generatedSource(const std::string& kind, int adjointFl
             if (ppl > 1) add("narrow", VARIANT_NARROW);
             if (hasLargeVariant(store != 0)) add("large", VARIANT_LARGE);
             if (registerVariantTiles(store != 0) > 0) add("registers", VARIANT_REGISTERS);
+            if (sharedTileWaves(store != 0) > 0) add("shared", VARIANT_SHARED);
         }
         ss << "]";
         return ss.str();
@@ -1533,6 +1542,27 @@ void FusedNetwork::forwardShape(bool store, int variant, int& blockSize, int& po
         blockSize = 2 * DEFAULT_BLOCK_SIZE;
         pointsPerLane = registerVariantTiles(store);
     }
+    if (variant == VARIANT_SHARED) {
+        blockSize = sharedTileWaves(store) * WARP_SIZE;
+        pointsPerLane = 1;
+    }
+}
+
+int FusedNetwork::sharedTileWaves(bool store) const
+{
+    int& known = sharedTileWaves_[store ? 1 : 0];   // (fixed by the specification, asked on every call)
+    if (known >= 0) return known;
+    known = 0;
+    if ((store ? compileOptions_.overwriteBlocksizeForward : compileOptions_.overwriteBlocksizeInference) > 0) return known;   // a pinned shape
+    std::vector<int> ldsW, ldsB;
+    int streamOffset = -1;
+    const int params = ldsLayout(false, ldsW, ldsB, &streamOffset);
+    if (streamOffset >= 0 || params * static_cast<int>(sizeof(half)) + stageBytesPerWave(false) > MaxSharedMemoryBytes()) return known;
+    int levels = 0;
+    for (const auto& e : encodings_)
+        if (e->levelGroups() > 1) levels = std::max(levels, e->numSweptTables());
+    known = levels >= 8 ? 8 : levels >= 4 ? 4 : 0;
+    return known;
 }
 
 void FusedNetwork::compileForwardKernel(bool store, int variant, bool compileOnly, bool derivatives, bool inputOnly)
@@ -1545,12 +1575,14 @@ void FusedNetwork::compileForwardKernel(bool store, int variant, bool compileOnl
     CompiledKernel ck;
     forwardShape(store, variant, ck.blockSize, ck.pointsPerLane);
     const bool registerStaging = variant == VARIANT_REGISTERS;
+    const bool sharedTile = variant == VARIANT_SHARED;
+    ck.tilesPerWorkgroup = sharedTile ? 1 : (ck.blockSize / WARP_SIZE) * ck.pointsPerLane;
     ck.sharedMemorySize = ldsParamHalves(false) * static_cast<int>(sizeof(half))
-        + (ck.blockSize / WARP_SIZE) * (registerStaging ? 1 : ck.pointsPerLane) * stageBytesPerWave(false);
+        + (sharedTile ? 1 : (ck.blockSize / WARP_SIZE) * (registerStaging ? 1 : ck.pointsPerLane)) * stageBytesPerWave(false);
     ck.fun = kl->getKernel(derivatives ? "qmlp::kernel::NetworkKernelInferenceAndForward<true, true>"
                            : store     ? "qmlp::kernel::NetworkKernelInferenceAndForward<true>"
                                        : "qmlp::kernel::NetworkKernelInferenceAndForward<false>",
-                           forwardSource(ck.blockSize, ck.pointsPerLane, registerStaging, derivatives, inputOnly), loaderFlags(compileOnly)).value();
+                           forwardSource(ck.blockSize, ck.pointsPerLane, registerStaging, derivatives, inputOnly, sharedTile), loaderFlags(compileOnly)).value();
     if (compileOnly) return;
     ck.fullGrid = ck.fun.fullGridSize(ck.blockSize, ck.sharedMemorySize);
     QuickMLP::Instance().getLogger()->debug(
@@ -1576,6 +1608,7 @@ const FusedNetwork::CompiledKernel& FusedNetwork::forwardKernelFor(bool store, i
         return forwardKernels_[s][variant].value();
     };
     if (launchTiles) *launchTiles = numTiles;
+    if (numTiles <= SHARED_TILE_MAX_TILES && sharedTileWaves(store) > 0) return loaded(VARIANT_SHARED);
     {
         int blockSize = 0, pointsPerLane = 1;
         forwardShape(store, VARIANT_DEFAULT, blockSize, pointsPerLane);
@@ -1901,6 +1934,7 @@ void FusedNetwork::precompile(int adjointFlags)
         forwardBlockSize(-1, false, &ppl);
         if (ppl > 1) compileForwardKernel(store, VARIANT_NARROW, true);
         if (hasLargeVariant(store)) compileForwardKernel(store, VARIANT_LARGE, true);
+        if (sharedTileWaves(store) > 0) compileForwardKernel(store, VARIANT_SHARED, true);
         if (registerVariantTiles(store) > 0) compileForwardKernel(store, VARIANT_REGISTERS, true);
     }
     if (adjointFlags > 0) {
@@ -1922,6 +1956,7 @@ void FusedNetwork::precompile(int adjointFlags)
                 forwardBlockSize(-1, false, &ppl);
                 if (ppl > 1) compileForwardKernel(true, VARIANT_NARROW, true, derivatives != 0, true);
                 if (hasLargeVariant(true)) compileForwardKernel(true, VARIANT_LARGE, true, derivatives != 0, true);
+                if (sharedTileWaves(true) > 0) compileForwardKernel(true, VARIANT_SHARED, true, derivatives != 0, true);
                 if (registerVariantTiles(true) > 0) compileForwardKernel(true, VARIANT_REGISTERS, true, derivatives != 0, true);
             }
     }
@@ -1932,6 +1967,7 @@ void FusedNetwork::precompile(int adjointFlags)
         forwardBlockSize(-1, false, &ppl);
         if (ppl > 1) compileForwardKernel(true, VARIANT_NARROW, true, true);
         if (hasLargeVariant(true)) compileForwardKernel(true, VARIANT_LARGE, true, true);
+        if (sharedTileWaves(true) > 0) compileForwardKernel(true, VARIANT_SHARED, true, true);
         if (registerVariantTiles(true) > 0) compileForwardKernel(true, VARIANT_REGISTERS, true, true);
     }
     if (adjointFlags > 0) {
@@ -2059,8 +2095,7 @@ void FusedNetwork::launchForward(bool store, const Tensor& input, Tensor& output
         inputAcc.sizes_[0] = outputAcc.sizes_[0] = count;
         const int* order = sorted ? orderAll + start : nullptr;
         int tmpTileOffset = static_cast<int>(start / TILE_POINTS);
-        const int waves = ck.blockSize / WARP_SIZE;
-        const int grid = std::min(divUp(divUp(count, TILE_POINTS), waves * ck.pointsPerLane), ck.fullGrid);
+        const int grid = std::min(divUp(divUp(count, TILE_POINTS), ck.tilesPerWorkgroup), ck.fullGrid);
         std::vector<void*> args = {&count, &inputAcc, &outputAcc, &networkParams, &tmpMemory, &tmpTileOffset, &tmpNumTiles, &order};
         std::vector<std::vector<char>> storage;
         encodingArguments(args, storage);

@@ -1,0 +1,53 @@
+"""The forward kernel for small batches, whose wavefronts share the levels of a tile: the same bits as the shapes with a
+tile per wavefront, for the results and for what the training pass leaves to the adjoint pass."""
+import json
+
+import pytest
+import torch
+
+import qmlp
+from helpers import warm_cache
+
+pytestmark = pytest.mark.gpu
+
+
+def grid(levels, features, start, mode="concat", precision="half"):
+    return {"id": "HashGrid", "start_in": start, "n_in": 2, "n_levels": levels, "n_features_per_level": features,
+            "log2_hashmap_size": 10, "min_resolution": 4, "max_resolution": 100, "combination_mode": mode,
+            "bounding_box_min": [0.0, 0.0], "bounding_box_size": [1.0, 1.0], "parameter_precision": precision}
+
+
+def spec(*encodings):
+    return {"num_inputs": 3, "num_outputs": 3, "activation_specification": ["qmlp/builtin-activations.json"],
+            "encodings": list(encodings), "options": {"slice_gradients": 1},
+            "network": [{"n_out": 32, "bias": True, "activation": "relu"}, {"n_out": 3, "bias": False, "activation": "identity"}]}
+
+
+IDENTITY = {"id": "Identity", "start_in": 1, "n_in": 2}
+# 8 wavefronts (levels that do not divide among them), 4 wavefronts, grids without levels of their own beside them
+SPECS = [spec(IDENTITY, grid(9, 2, 0)), spec(grid(5, 1, 1, precision="float"), grid(6, 2, 0, "add")), spec(grid(12, 4, 0))]
+
+
+@pytest.mark.parametrize("cfg", SPECS)
+def test_small_batches_give_the_bits_of_large_ones(cfg):
+    warm_cache(cfg)
+    net = qmlp.Network(json.dumps(cfg))
+    assert any(s["shape"] == "shared" for s in json.loads(net.generated_source("shapes")))
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    rand = lambda *shape: torch.rand(shape, device="cuda", generator=gen)  # noqa: E731
+    x, g = rand(40000, 3) * 1.2 - 0.1, rand(40000, 3) - 0.5
+    params = (rand(net.num_network_parameters()) - 0.5).half()
+    tables = [(rand(net.encoding(i).num_parameters()) - 0.5).to(net.encoding(i).parameter_dtype())
+              if net.encoding(i).has_parameters() else None for i in range(len(cfg["encodings"]))]
+
+    def train(n):
+        out, memory = net.forward_raw(x[:n], params, tables, 7)
+        adj_x, _, _ = net.adjoint_raw(x[:n], g[:n], 7, memory, params, tables)
+        return out, adj_x
+
+    large = net.inference(x, params, tables)
+    large_out, large_adj = train(len(x))
+    for n in (1, 63, 65, 1000, 448 * 64, 448 * 64 + 1):
+        assert torch.equal(net.inference(x[:n], params, tables), large[:n]), n
+        out, adj_x = train(n)
+        assert torch.equal(out, large_out[:n]) and torch.equal(adj_x, large_adj[:n]), n
