@@ -159,7 +159,7 @@ private:
         int pointsPerLane = 1;
         int sharedMemorySize = 0;
         int fullGrid = 0;
-        int tilesPerWorkgroup = 1;   // of the forward kernels
+        int tilesPerWorkgroup = 1;   // of the forward and backward kernels
     };
     // [store intermediates][variant], see ForwardVariant
     // [0]: inference, [1]: forward (stores the intermediates), [2]: forward that also stores position derivatives
@@ -260,9 +260,10 @@ private:
     // How the backward kernel gets at the pre-activations. STORED: from the forward memory. RECOMPUTED: it runs the layers
     // again, every wavefront by itself. COOPERATIVE: it runs them again, and the wavefronts of a workgroup share the
     // gradient tiles of all layers.
-    enum BackwardMode { BACKWARD_STORED = 0, BACKWARD_RECOMPUTED = 1, BACKWARD_COOPERATIVE = 2 };
+    // SHARED_TILE: as STORED, the wavefronts of a workgroup share the grid levels of one tile (small batches).
+    enum BackwardMode { BACKWARD_STORED = 0, BACKWARD_RECOMPUTED = 1, BACKWARD_COOPERATIVE = 2, BACKWARD_SHARED_TILE = 3 };
     // [adjoint flags][grid gradients by slices instead of atomics][BackwardMode]
-    std::optional<AdjointKernel> backwardKernel_[ADJOINT_MODE_MAX_COMBINATIONS][2][3];
+    std::optional<AdjointKernel> backwardKernel_[ADJOINT_MODE_MAX_COMBINATIONS][2][4];
     // Smaller batches go to the kernel whose wavefronts sum all gradient tiles by themselves, where the network has one.
     static constexpr int COOPERATIVE_MIN_BATCH = 1 << 13;
     /** Whether the cooperative kernel exists for this network and flags and a batch of numel points takes it, registers aside. */
@@ -318,6 +319,15 @@ private:
      *  their intermediates: a training pass that is followed by it keeps the encoded input only. */
     bool recomputesFor(int numel, int flags) const;
     bool canRecompute(int flags, bool sliceGradients) const;
+    /** Whether the wavefronts of a workgroup can share the levels of this encoding, and whether a batch is differentiated that way. */
+    bool sharesLevels(const IEncoding& e) const;
+    bool sharesBackwardTile(int numel, int flags);
+    int sharesBackwardTile_[ADJOINT_MODE_MAX_COMBINATIONS] = {-1, -1, -1, -1, -1, -1, -1, -1};
+    static constexpr int SHARED_BACKWARD_MAX_TILES = 256;   // a workgroup per compute unit
+    static constexpr int NUM_SHARED_DIMENSIONS = 6;         // of a grid, at most
+    /** LDS of such a kernel, and where in it the derivatives of the levels begin. */
+    int sharedTileLdsBytes(int flags, int blockSize) const;
+    int sharedTileLdsOffset(int blockSize) const;
     /** Whether the backward kernel itself adds input gradients of an encoding (those of sliced grids come from the kernels behind it). */
     bool differentiatesEncodings(int flags, bool sliceGradients) const;
     mutable int recomputesKnown_[ADJOINT_MODE_MAX_COMBINATIONS][2];   // canRecompute(), -1: not known yet
@@ -524,7 +534,7 @@ private:
     void compileRecordsKernel(SliceGradientKernel& sk, int flags, size_t variant, bool compileOnly, bool fromDerivatives = false);
 
     std::string forwardSource(int blockSize, int pointsPerLane, bool registerStaging = false, bool derivatives = false, bool inputOnly = false, bool sharedTile = false) const;
-    std::string backwardSource(int flags, int blockSize, bool sliceGradients = false, bool recompute = false, bool twoWavefrontsPerSimd = false) const;
+    std::string backwardSource(int flags, int blockSize, bool sliceGradients = false, bool recompute = false, bool twoWavefrontsPerSimd = false, bool sharedTile = false) const;
     std::string weightUpdateSource(int blockSize) const;
     std::string weightUpdateKernelName(int layer, int& numChunks, int& tilesPerBlock) const;
     void fillEncodingsAndActivations(std::string& codeTemplate) const;

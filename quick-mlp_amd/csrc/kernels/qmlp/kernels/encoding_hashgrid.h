@@ -582,6 +582,25 @@ struct EncodingHashGrid
         }
     }
 
+    /** What corner c of a level adds to the derivative of the loss with respect to the position in cells. */
+    __device__ __forceinline__ static void addCornerDerivative(int l, const LevelSetup& s, int c, const float (&adjFeat)[F],
+                                                               const param_t& params, float (&lvl)[D])
+    {
+        float v[F];
+        detail::loadFeatures<F>(params.parametersForward + cornerOffset(l, s, c), v);
+        float dot = 0.f;
+#pragma unroll
+        for (int i = 0; i < F; ++i) dot += adjFeat[i] * v[i];
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            float prod = 1.f;
+#pragma unroll
+            for (int e = D - 1; e >= 0; --e)
+                if (e != d) prod *= ((c >> e) & 1) ? s.f[e] : (1.f - s.f[e]);
+            lvl[d] += (((c >> d) & 1) ? prod : -prod) * dot;
+        }
+    }
+
     /**
      * Adjoint: scatters w * adjFeature into the gradient table with hardware fp32
      * atomics and accumulates the analytic multilinear derivative into adjInput.
@@ -615,21 +634,7 @@ struct EncodingHashGrid
                     for (int i = 0; i < F; ++i)
                         unsafeAtomicAdd(params.parametersBackward + (off + i), w * adjFeat[i]);
                 }
-                if constexpr (EvaluateInputGradients) {
-                    float v[F];
-                    detail::loadFeatures<F>(params.parametersForward + off, v);
-                    float dot = 0.f;
-#pragma unroll
-                    for (int i = 0; i < F; ++i) dot += adjFeat[i] * v[i];
-#pragma unroll
-                    for (int d = 0; d < D; ++d) {
-                        float prod = 1.f;
-#pragma unroll
-                        for (int e = D - 1; e >= 0; --e)
-                            if (e != d) prod *= ((c >> e) & 1) ? s.f[e] : (1.f - s.f[e]);
-                        lvl[d] += (((c >> d) & 1) ? prod : -prod) * dot;
-                    }
-                }
+                if constexpr (EvaluateInputGradients) addCornerDerivative(l, s, c, adjFeat, params, lvl);
             }
             if constexpr (EvaluateInputGradients) {
                 const float scale = Cfg::ResolutionFactor ? static_cast<float>(Cfg::resolution[l] - 1) : 1.f;
@@ -688,11 +693,12 @@ struct EncodingHashGrid
      *    (ldsGradients, leadingElements<LDS_LEVELS>() floats, zeroed by the workgroup) and reach
      *    global memory once per workgroup through flushLdsGradients: a coarse level receives
      *    many points per cell, so this saves its share of the atomic requests
+     * \tparam FIRST, END the levels from FIRST to END - 1 only
      * \param index0 index of the first point of the tile
      * \param adjOutput callable (point of the tile 0..63, output channel of this encoding) ->
      *    adjoint of that output as float
      */
-    template <int LDS_LEVELS = 0, typename AdjFn, typename Trace = NoCornerTrace>
+    template <int LDS_LEVELS = 0, int FIRST = 0, int END = L, typename AdjFn, typename Trace = NoCornerTrace>
     __device__ __forceinline__ static void scatterTile(int lane, long long index0, long long numel,
                                                        const Tensor2Read<float>& inputs, const AdjFn& adjOutput,
                                                        const param_t& params, float* ldsGradients = nullptr,
@@ -721,7 +727,7 @@ struct EncodingHashGrid
                 for (int d = 0; d < D; ++d) pos[d] = (in[d] - params.boundingBoxMin[d]) * params.boundingBoxInvSize[d];
             }
 #pragma unroll
-            for (int l = 0; l < L; ++l) {
+            for (int l = FIRST; l < END; ++l) {
                 const LevelSetup s = setupLevel(l, pos);
                 const bool hashed = Cfg::hashed[l];
                 const unsigned base = static_cast<unsigned>(Cfg::memoryOffset[l]);
@@ -759,6 +765,59 @@ struct EncodingHashGrid
                 }
             }
         }
+    }
+
+    /**
+     * The share of wavefront `wave` of WAVES in the adjoint of a tile (with HasTileScatter): the parameter gradients of some
+     * of the levels, and the derivatives of these levels with respect to the position for finishShared().
+     * \param input, adjOutput rows of the point of this lane, adjFn as adjOutput of scatterTile()
+     * \param sLevels L * D * 64 floats in LDS, shared by the wavefronts
+     */
+    template <int WAVES, bool EvaluateInputGradients, bool EvaluateParameterGradients, int WAVE = 0, typename I, typename O, typename AdjFn>
+    __device__ __forceinline__ static void adjointShared(int wave, int lane, long long index0, long long numel, const Tensor2Read<float>& inputs,
+                                                         const I& input, const O& adjOutput, const AdjFn& adjFn, const param_t& params, float* sLevels)
+    {
+        constexpr int FIRST = L * WAVE / WAVES, END = L * (WAVE + 1) / WAVES;
+        if (wave == WAVE) {
+            if constexpr (EvaluateInputGradients) {
+                float pos[D];
+                unitPosition(input, params, pos);
+#pragma unroll
+                for (int l = FIRST; l < END; ++l) {
+                    const LevelSetup s = setupLevel(l, pos);
+                    float adjFeat[F], lvl[D];
+#pragma unroll
+                    for (int i = 0; i < F; ++i) adjFeat[i] = fcast<float>(adjOutput[(Cfg::Concat ? l * F : 0) + i]);
+#pragma unroll
+                    for (int d = 0; d < D; ++d) lvl[d] = 0.f;
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) addCornerDerivative(l, s, c, adjFeat, params, lvl);
+#pragma unroll
+                    for (int d = 0; d < D; ++d) sLevels[(l * D + d) * TILE_POINTS + lane] = lvl[d];
+                }
+            }
+            if constexpr (EvaluateParameterGradients) scatterTile<0, FIRST, END>(lane, index0, numel, inputs, adjFn, params);
+        } else if constexpr (WAVE + 1 < WAVES) {
+            adjointShared<WAVES, EvaluateInputGradients, EvaluateParameterGradients, WAVE + 1>(wave, lane, index0, numel, inputs, input, adjOutput,
+                                                                                              adjFn, params, sLevels);
+        }
+    }
+
+    /** The input gradients of the point of this lane from the derivatives of its levels, in the order of adjoint(). */
+    template <typename AdjI>
+    __device__ __forceinline__ static void finishShared(AdjI& adjInput, const param_t& params, const float* sLevels, int lane)
+    {
+        float adjPos[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) adjPos[d] = 0.f;
+#pragma unroll
+        for (int l = 0; l < L; ++l) {
+            const float scale = Cfg::ResolutionFactor ? static_cast<float>(Cfg::resolution[l] - 1) : 1.f;
+#pragma unroll
+            for (int d = 0; d < D; ++d) adjPos[d] += scale * sLevels[(l * D + d) * TILE_POINTS + lane];
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d) adjInput[d + Cfg::Start] += adjPos[d] * params.boundingBoxInvSize[d];
     }
 
     /** Test aid: what the gathers of the fused forward kernels (gatherLevel) read for this point:

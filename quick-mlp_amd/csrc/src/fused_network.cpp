@@ -1071,7 +1071,7 @@ int FusedNetwork::ldsGradientLayout(int adjointFlags, int blockSize, std::vector
     return bytes;
 }
 
-std::string FusedNetwork::backwardSource(int flags, int blockSize, bool sliceGradients, bool recompute, bool twoWavefrontsPerSimd) const
+std::string FusedNetwork::backwardSource(int flags, int blockSize, bool sliceGradients, bool recompute, bool twoWavefrontsPerSimd, bool sharedTile) const
 {
     const bool hasInputGradients = flags & GRADIENTS_INPUT;
     const bool hasNetworkGradients = flags & GRADIENTS_NETWORK_WEIGHTS;
@@ -1083,6 +1083,7 @@ std::string FusedNetwork::backwardSource(int flags, int blockSize, bool sliceGra
     replaceAll(code, "$$BLOCK_SIZE$$", std::to_string(blockSize));
     replaceAll(code, "$$HAS_OUTPUT_ORDER$$", trainsSortedBatches() ? "1" : "0");
     replaceAll(code, "$$RECOMPUTES$$", recompute ? "true" : "false");
+    replaceAll(code, "$$SHARED_TILE$$", sharedTile ? "true" : "false");
     bool wideRegisters = false;
     (void)fusedWeightUpdateLayers(flags, sliceGradients, &wideRegisters);
     // (the pre-activations of all layers stay in registers beside the gradient tiles: 256 registers spilled 404 bytes
@@ -1233,9 +1234,14 @@ std::string FusedNetwork::backwardSource(int flags, int blockSize, bool sliceGra
     replaceAll(code, "$$CALL_NETWORK_LAYERS$$", callLayers.str());
     replaceAll(code, "$$HAS_STREAMED_LAYERS$$", anyStreamed ? "true" : "false");
 
-    std::stringstream callEncodings, callScatter, zeroLds, flushLds;
+    std::stringstream callEncodings, callScatter, callShared, zeroLds, flushLds;
     std::vector<LdsGradients> ldsGradients;
-    ldsGradientLayout(flags, blockSize, ldsGradients, sliceGradients);
+    int sharedOffset = ldsGradientLayout(flags, blockSize, ldsGradients, sliceGradients);
+    if (sharedTile) {
+        // (a workgroup has one tile: nothing to sum in LDS first)
+        sharedOffset = roundUp(sharedTileLdsOffset(blockSize), 16);
+        ldsGradients.assign(encodings_.size(), LdsGradients{});
+    }
     int encodingOffset = 0;
     bool storeEncodedAdjoint = false, gradientsInKernel = false, inputGradientsInKernel = false;
     for (size_t encodingIdx = 0; encodingIdx < encodings_.size(); ++encodingIdx) {
@@ -1264,6 +1270,22 @@ std::string FusedNetwork::backwardSource(int flags, int blockSize, bool sliceGra
         // encodings with a tile-wide scatter take their parameter gradients out of the per-point call
         const std::string perPointParameterGradients =
             parameterGradients ? "!" + name + "::HasTileScatter" : std::string("false");
+        if (sharedTile && sharesLevels(*e)) {
+            callShared << "                {\n                    StaticArray<float, NUM_INPUTS> sharedInput;\n                    const long long point = min(static_cast<long long>(tile) * TILE_POINTS + lane, static_cast<long long>(numel - 1));\n"
+                       << "#pragma unroll\n                    for (int i = 0; i < NUM_INPUTS; ++i) sharedInput[i] = inputs.data_[point * inputs.strides_[0] + i * inputs.strides_[1]];\n"
+                       << "                    const WrappedArray<const f16> sharedAdjoint{sStage + stageRow(lane) * STAGE_STRIDE + " << encodingOffset << "};\n"
+                       << "                    " << name << "::template adjointShared<WAVES, " << (inputGradients ? "true" : "false") << ", "
+                       << (parameterGradients ? "true" : "false") << ">(__builtin_amdgcn_readfirstlane(wave), lane, static_cast<long long>(tile) * TILE_POINTS, numel, inputs,\n"
+                       << "                        sharedInput, sharedAdjoint, [&](int pt, int c) { return static_cast<float>(sStage[stageRow(pt) * STAGE_STRIDE + "
+                       << encodingOffset << " + c]); },\n                        cEncoding" << encodingIdx << ", reinterpret_cast<float*>(sMemory + " << sharedOffset << "));\n                }\n";
+            if (inputGradients) {
+                callEncodings << "                " << name << "::finishShared(adjEncodingInput, cEncoding" << encodingIdx
+                              << ", reinterpret_cast<const float*>(sMemory + " << sharedOffset << "), lane);\n";
+                sharedOffset += e->numSweptTables() * NUM_SHARED_DIMENSIONS * TILE_POINTS * static_cast<int>(sizeof(float));
+            }
+            encodingOffset += e->numOutputChannels();
+            continue;
+        }
         callEncodings << "                {\n                    auto adjEncodingOutputK = adjEncodingOutput + "
                       << encodingOffset << ";\n                    " << name << "::template adjoint<"
                       << (inputGradients ? "true" : "false") << ", " << perPointParameterGradients
@@ -1291,9 +1313,48 @@ std::string FusedNetwork::backwardSource(int flags, int blockSize, bool sliceGra
     // layer 0 still has to produce the adjoint of the encoded rows for the kernels behind this one
     replaceAll(code, "$$NEEDS_ENCODING_ADJOINT$$", (hasInputGradients || hasEncodingGradients) ? "true" : "false");
     replaceAll(code, "$$CALL_ENCODING_SCATTER$$", callScatter.str());
+    replaceAll(code, "$$CALL_SHARED_ENCODINGS$$", callShared.str());
     replaceAll(code, "$$ZERO_LDS_GRADIENTS$$", zeroLds.str());
     replaceAll(code, "$$FLUSH_LDS_GRADIENTS$$", flushLds.str().empty() ? std::string() : "    __syncthreads();\n" + flushLds.str());
     return code;
+}
+
+int FusedNetwork::sharedTileLdsOffset(int blockSize) const
+{
+    return ldsParamHalves(true) * static_cast<int>(sizeof(half)) + (blockSize / WARP_SIZE) * stageBytesPerWave(true);
+}
+
+int FusedNetwork::sharedTileLdsBytes(int flags, int blockSize) const
+{
+    int bytes = roundUp(sharedTileLdsOffset(blockSize), 16);
+    if (flags & GRADIENTS_INPUT)
+        for (const auto& e : encodings_)
+            if (sharesLevels(*e)) bytes += e->numSweptTables() * NUM_SHARED_DIMENSIONS * TILE_POINTS * static_cast<int>(sizeof(float));
+    return bytes;
+}
+
+bool FusedNetwork::sharesLevels(const IEncoding& e) const
+{
+    // (as many features as scatterTile() takes)
+    const int features = e.channelsWrittenTogether();
+    return e.hasParameters() && e.levelGroups() > 1 && e.numSweptTables() >= 4 && (features & (features - 1)) == 0 && 2 * features <= WARP_SIZE;
+}
+
+bool FusedNetwork::sharesBackwardTile(int numel, int flags)
+{
+    if (divUp(numel, TILE_POINTS) > SHARED_BACKWARD_MAX_TILES || !(flags & (GRADIENTS_INPUT | GRADIENTS_INPUT_ENCODINGS)) || useSliceGradients(numel, flags)) return false;
+    int& known = sharesBackwardTile_[flags];   // (but for the size fixed by the specification)
+    if (known < 0) {
+        known = 0;
+        for (const auto& e : encodings_) known = known || sharesLevels(*e) ? 1 : 0;
+        if (trainsSortedBatches() || compileOptions_.overwriteBlocksizeBackward > 0) known = 0;
+        for (bool fused : fusedWeightUpdateLayers(flags, false))
+            if (fused) known = 0;   // (as many workgroups as slices of partial sums: a fourth of the tiles)
+        for (auto placement : weightPlacement(true))
+            if (placement == WEIGHTS_STREAMED) known = 0;
+        if (sharedTileLdsBytes(flags, forwardBlockSize(compileOptions_.overwriteBlocksizeBackward, true)) > MaxSharedMemoryBytes()) known = 0;
+    }
+    return known != 0;
 }
 
 std::string FusedNetwork::cooperativeBackwardSource(int flags, bool sliceGradients) const
@@ -1679,7 +1740,7 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
     if (flags <= 0 || flags >= ADJOINT_MODE_MAX_COMBINATIONS) throw std::runtime_error("At least one derivative must be enabled");
     const int variant = sliceGradients ? 1 : 0;
     if (backwardKernel_[flags][variant][mode].has_value() && !compileOnly) return;
-    const bool recompute = mode == BACKWARD_RECOMPUTED, cooperative = mode == BACKWARD_COOPERATIVE;
+    const bool recompute = mode == BACKWARD_RECOMPUTED, cooperative = mode == BACKWARD_COOPERATIVE, sharedTile = mode == BACKWARD_SHARED_TILE;
     const bool hasNetworkGradients = flags & GRADIENTS_NETWORK_WEIGHTS;
     auto kl = QuickMLP::Instance().kernelLoader();
     auto logger = QuickMLP::Instance().getLogger();
@@ -1699,8 +1760,10 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
     ak.adjoint.blockSize = forwardBlockSize(compileOptions_.overwriteBlocksizeBackward, true);
     {
         std::vector<LdsGradients> ldsGradients;
-        ak.adjoint.sharedMemorySize = ldsGradientLayout(flags, ak.adjoint.blockSize, ldsGradients, sliceGradients, recompute);
+        ak.adjoint.sharedMemorySize = sharedTile ? sharedTileLdsBytes(flags, ak.adjoint.blockSize)
+                                                 : ldsGradientLayout(flags, ak.adjoint.blockSize, ldsGradients, sliceGradients, recompute);
     }
+    ak.adjoint.tilesPerWorkgroup = sharedTile ? 1 : ak.adjoint.blockSize / WARP_SIZE;
     ak.fusedLayers = fusedWeightUpdateLayers(flags, sliceGradients);
     ak.outputOrder = trainsSortedBatches();
     ak.fusedWeightUpdate = false;
@@ -1748,7 +1811,7 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
         }
     }
     if (!chosen) {
-        adjointSource = backwardSource(flags, ak.adjoint.blockSize, sliceGradients, recompute);
+        adjointSource = backwardSource(flags, ak.adjoint.blockSize, sliceGradients, recompute, false, sharedTile);
         if (offlineCompiler) {
             adjointLoaderFlags |= KernelLoader::CompileOffline;
             offlineOptions = {"-mllvm", "-amdgpu-mfma-vgpr-form"};
@@ -1767,7 +1830,7 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
     if (!compileOnly) {
         ak.adjoint.fullGrid = ak.adjoint.fun.fullGridSize(ak.adjoint.blockSize, ak.adjoint.sharedMemorySize);
         logger->debug("backward kernel (flags %d%s): block %d, LDS %d bytes, %d VGPRs, %d bytes scratch, full grid %d", flags,
-                      recompute ? ", the layers run again" : cooperative ? ", cooperative" : "",
+                      recompute ? ", the layers run again" : cooperative ? ", cooperative" : sharedTile ? ", shared tiles" : "",
                       ak.adjoint.blockSize, ak.adjoint.sharedMemorySize, ak.adjoint.fun.numVgprs(),
                       ak.adjoint.fun.scratchBytes(), ak.adjoint.fullGrid);
     }
@@ -1973,6 +2036,7 @@ void FusedNetwork::precompile(int adjointFlags)
     if (adjointFlags > 0) {
         if (compileOptions_.sliceGradients <= 0 || !hasSliceGradients() || !(adjointFlags & GRADIENTS_INPUT_ENCODINGS))
             compileBackwardKernel(adjointFlags, false, true);
+        if (sharesBackwardTile(1, adjointFlags)) compileBackwardKernel(adjointFlags, false, true, BACKWARD_SHARED_TILE);
         if ((adjointFlags & GRADIENTS_INPUT_ENCODINGS) && hasSliceGradients()) compileBackwardKernel(adjointFlags, true, true);
     }
     kernel::PointOrderKey key{};
@@ -2162,7 +2226,8 @@ void FusedNetwork::prepare(int numel, int adjointFlags)
     }
     if (adjointFlags > 0) {
         const bool sliceGradients = useSliceGradients(numel, adjointFlags);
-        const BackwardMode mode = backwardMode(numel, adjointFlags);
+        BackwardMode mode = backwardMode(numel, adjointFlags);
+        if (mode == BACKWARD_STORED && sharesBackwardTile(numel, adjointFlags)) mode = BACKWARD_SHARED_TILE;
         compileBackwardKernel(adjointFlags, sliceGradients, false, mode);
         for (auto& sk : backwardKernel_[adjointFlags][sliceGradients ? 1 : 0][mode].value().sliceGradients)
         {
@@ -2487,6 +2552,7 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
         }
     }
     const bool sortedPoints = sortsTraining(numel);
+    if (mode == BACKWARD_STORED && sharesBackwardTile(numel, adjointFlags)) mode = BACKWARD_SHARED_TILE;
     compileBackwardKernel(adjointFlags, sliceGradients, false, mode);
     auto& ak = backwardKernel_[adjointFlags][sliceGradients ? 1 : 0][mode].value();
     const bool cooperative = mode == BACKWARD_COOPERATIVE;
@@ -2548,7 +2614,7 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
         const auto& ck = ak.adjoint;
         const int waves = ck.blockSize / WARP_SIZE;
         // (a wavefront of the cooperative kernel takes half a tile)
-        int grid = std::min(cooperative ? divUp(2 * numTiles, waves) : divUp(numTiles, waves), ck.fullGrid);
+        int grid = std::min(cooperative ? divUp(2 * numTiles, waves) : divUp(numTiles, ck.tilesPerWorkgroup), ck.fullGrid);
         // every workgroup stores its sums of the weight gradients as one of the slices of the batch that the
         // reduction adds up (and zeroes its share of the slices beyond the grid)
         int partialSlices = partialSliceCount;

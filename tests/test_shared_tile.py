@@ -1,5 +1,6 @@
-"""The forward kernel for small batches, whose wavefronts share the levels of a tile: the same bits as the shapes with a
-tile per wavefront, for the results and for what the training pass leaves to the adjoint pass."""
+"""The kernels for small batches, whose wavefronts share the grid levels of a tile. Forward: the same bits as the shapes with
+a tile per wavefront, for the results and for what the training pass leaves to the adjoint pass. Backward: the same
+gradients but for rounding."""
 import json
 
 import pytest
@@ -17,9 +18,9 @@ def grid(levels, features, start, mode="concat", precision="half"):
             "bounding_box_min": [0.0, 0.0], "bounding_box_size": [1.0, 1.0], "parameter_precision": precision}
 
 
-def spec(*encodings):
+def spec(*encodings, slices=1):
     return {"num_inputs": 3, "num_outputs": 3, "activation_specification": ["qmlp/builtin-activations.json"],
-            "encodings": list(encodings), "options": {"slice_gradients": 1},
+            "encodings": list(encodings), "options": {"slice_gradients": slices},
             "network": [{"n_out": 32, "bias": True, "activation": "relu"}, {"n_out": 3, "bias": False, "activation": "identity"}]}
 
 
@@ -51,3 +52,38 @@ def test_small_batches_give_the_bits_of_large_ones(cfg):
         assert torch.equal(net.inference(x[:n], params, tables), large[:n]), n
         out, adj_x = train(n)
         assert torch.equal(out, large_out[:n]) and torch.equal(adj_x, large_adj[:n]), n
+
+
+# three levels in no wavefront, levels added up and many features stay with the first wavefront
+BACKWARD = [(IDENTITY, grid(9, 2, 0)), (grid(5, 1, 1, precision="float"), grid(6, 2, 0, "add")), (grid(4, 4, 0), grid(4, 3, 1))]
+
+
+@pytest.mark.parametrize("encodings", BACKWARD)
+@pytest.mark.parametrize("flags", [1, 4, 6, 7])
+def test_small_batches_are_differentiated_like_large_ones(encodings, flags):
+    cfg, sliced = spec(*encodings, slices=0), spec(*encodings, slices=1)
+    warm_cache(cfg, sliced)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    rand = lambda *shape: torch.rand(shape, device="cuda", generator=gen)  # noqa: E731
+    x, g = rand(20000, 3) * 1.2 - 0.1, rand(20000, 3) - 0.5
+    nets = [qmlp.Network(json.dumps(c)) for c in (cfg, sliced)]
+    params = (rand(nets[0].num_network_parameters()) - 0.5).half()
+    tables = [(rand(nets[0].encoding(i).num_parameters()) - 0.5).to(nets[0].encoding(i).parameter_dtype())
+              if nets[0].encoding(i).has_parameters() else None for i in range(len(encodings))]
+
+    def train(net, n):
+        _, memory = net.forward_raw(x[:n], params, tables, flags)
+        return net.adjoint_raw(x[:n], g[:n], flags, memory, params, tables)
+
+    large, _, _ = train(nets[0], len(x))
+    for n in (1, 63, 65, 1000, 256 * 64, 256 * 64 + 1):
+        adj_x, weights, adj_tables = train(nets[0], n)
+        if flags & 1:
+            # (the same operations, multiplications and additions contracted differently here and there)
+            torch.testing.assert_close(adj_x, large[:n], rtol=1e-5, atol=1e-6 * float(large.abs().max()))
+        _, expected_weights, expected_tables = train(nets[1], n)
+        pairs = [(weights, expected_weights)] if flags & 2 else []
+        pairs += [(a, b) for a, b in zip(adj_tables, expected_tables) if a is not None] if flags & 4 else []
+        for a, b in pairs:
+            assert float(b.abs().max()) > 0
+            torch.testing.assert_close(a, b, rtol=1e-3, atol=1e-4 * float(b.abs().max()))
