@@ -319,8 +319,7 @@ private:
      *  their intermediates: a training pass that is followed by it keeps the encoded input only. */
     bool recomputesFor(int numel, int flags) const;
     bool canRecompute(int flags, bool sliceGradients) const;
-    /** Whether the wavefronts of a workgroup can share the levels of this encoding, and whether a batch is differentiated that way. */
-    bool sharesLevels(const IEncoding& e) const;
+    /** Whether the wavefronts of a workgroup share the grid levels of a tile in the backward kernel for this batch. */
     bool sharesBackwardTile(int numel, int flags);
     int sharesBackwardTile_[ADJOINT_MODE_MAX_COMBINATIONS] = {-1, -1, -1, -1, -1, -1, -1, -1};
     static constexpr int SHARED_BACKWARD_MAX_TILES = 256;   // a workgroup per compute unit

@@ -124,6 +124,16 @@ public:
     /** Workgroups of the standalone forward kernel that may share out the levels of a point (device function forwardGroup; 1: forward). */
     [[nodiscard]] virtual int levelGroups() const { return 1; }
 
+    /** Grids of many levels whose tile-wide adjoint the wavefronts of a workgroup may share by levels (device function
+     *  adjointShared, for as many features as scatterTile() takes); 0 or the number of wavefronts. */
+    [[nodiscard]] int sharedAdjointWaves() const
+    {
+        const int features = channelsWrittenTogether(), levels = numSweptTables();
+        if (!hasParameters() || levelGroups() <= 1 || levels < 4 || (features & (features - 1)) != 0 || features > 32) return 0;
+        return levels >= 8 ? 8 : 4;
+    }
+    static constexpr int SHARED_ADJOINT_MAX_BATCH = 256 * 64;   // a workgroup per compute unit
+
     /** One work item of GridGradientSlicesKernel (mirrors kernel::GridGradientSlice). */
     struct GradientSlice
     {
@@ -231,14 +241,14 @@ public:
      * back whole slices whatever the batch). A train step of one dense 4-D level with 8 features at 2^14 / 2^15 / 2^16 /
      * 2^17 points 0.08 / 0.09 / 0.12 / 0.19 ms with atomics, 0.10 / 0.11 / 0.12 / 0.23 ms by slices. The atomics of a
      * point grow with the number of levels, the fixed work of the slice kernels with the size of the table: a train
-     * step of a network behind a 16-level hash grid of floats at 2^13 / 2^14 / 2^15 points 111 / 134 / 190 us with atomics,
-     * 103 / 106 / 117 us by slices (with input gradients 157 / 180 / 238 and 146 / 151 / 166 us); the adjoint pass of
-     * that grid alone 38 / 61 / 117 and 46 / 51 / 67 us (with input gradients 76 / 98 / 155 and 91 / 98 / 112 us).
+     * step of a network behind a 16-level hash grid of halves at 2^13 / 2^14 / 2^15 points 96 / 128 / 201 us with atomics,
+     * 96 / 102 / 126 us by slices (with input gradients 111 / 148 / 244 and 137 / 146 / 176 us); the adjoint pass of
+     * that grid alone 32 / 60 / 117 and 46 / 51 / 66 us (with input gradients 41 / 72 / 152 and 91 / 96 / 112 us).
      * \param manyLevelsMinBatch from which size on grids of 8 levels or more take the slices
      */
     static constexpr int SLICE_GRADIENTS_MIN_BATCH = 1 << 16;
-    static constexpr int SLICE_GRADIENTS_MIN_BATCH_STANDALONE = 1 << 14;
-    static constexpr int SLICE_GRADIENTS_MIN_BATCH_TRAIN_STEP = 1 << 13;
+    static constexpr int SLICE_GRADIENTS_MIN_BATCH_STANDALONE = 1 << 14, SLICE_GRADIENTS_MIN_BATCH_STANDALONE_INPUT = (1 << 14) + 1;
+    static constexpr int SLICE_GRADIENTS_MIN_BATCH_TRAIN_STEP = 1 << 13, SLICE_GRADIENTS_MIN_BATCH_TRAIN_STEP_INPUT = 1 << 14;
     // (a pass without weight gradients needs no temporary memory for batches below)
     static constexpr int SLICE_GRADIENTS_MIN_BATCH_NO_WEIGHTS = 1 << 15;
     [[nodiscard]] static bool slicesPay(const GradientSliceLayout& layout, long long numel, int manyLevelsMinBatch)
@@ -294,7 +304,8 @@ public:
 
 private:
     std::string forwardKernelSource(int groups) const;
-    std::string adjointKernelSource(int adjointMode) const;
+    std::string adjointKernelSource(int adjointMode, bool sharedTile = false) const;
+    std::optional<KernelFunction> adjointSharedKernel_[AdjointMode::ALL_GRADIENTS + 1];
     std::optional<KernelFunction> forwardKernel_[2];   // [1]: by groups of levels
     // Where the kernel without groups is the faster one, see EncodingForwardKernel.
     static constexpr long long FORWARD_WHOLE_ROWS_MIN_BATCH = 3 << 14;

@@ -1040,8 +1040,10 @@ bool FusedNetwork::useSliceGradients(int numel, int flags) const
     if (compileOptions_.sliceGradients > 0) return true;
     for (const auto& e : encodings_) {
         const auto* layout = slicesOf(*e);
-        if (layout && IEncoding::slicesPay(*layout, numel, flags & GRADIENTS_NETWORK_WEIGHTS ? IEncoding::SLICE_GRADIENTS_MIN_BATCH_TRAIN_STEP
-                                                                                             : IEncoding::SLICE_GRADIENTS_MIN_BATCH_NO_WEIGHTS)) return true;
+        const int manyLevels = !(flags & GRADIENTS_NETWORK_WEIGHTS) ? IEncoding::SLICE_GRADIENTS_MIN_BATCH_NO_WEIGHTS
+            : flags & GRADIENTS_INPUT                               ? IEncoding::SLICE_GRADIENTS_MIN_BATCH_TRAIN_STEP_INPUT
+                                                                    : IEncoding::SLICE_GRADIENTS_MIN_BATCH_TRAIN_STEP;
+        if (layout && IEncoding::slicesPay(*layout, numel, manyLevels)) return true;
     }
     return false;
 }
@@ -1270,7 +1272,7 @@ std::string FusedNetwork::backwardSource(int flags, int blockSize, bool sliceGra
         // encodings with a tile-wide scatter take their parameter gradients out of the per-point call
         const std::string perPointParameterGradients =
             parameterGradients ? "!" + name + "::HasTileScatter" : std::string("false");
-        if (sharedTile && sharesLevels(*e)) {
+        if (sharedTile && e->sharedAdjointWaves() > 0) {
             callShared << "                {\n                    StaticArray<float, NUM_INPUTS> sharedInput;\n                    const long long point = min(static_cast<long long>(tile) * TILE_POINTS + lane, static_cast<long long>(numel - 1));\n"
                        << "#pragma unroll\n                    for (int i = 0; i < NUM_INPUTS; ++i) sharedInput[i] = inputs.data_[point * inputs.strides_[0] + i * inputs.strides_[1]];\n"
                        << "                    const WrappedArray<const f16> sharedAdjoint{sStage + stageRow(lane) * STAGE_STRIDE + " << encodingOffset << "};\n"
@@ -1329,15 +1331,8 @@ int FusedNetwork::sharedTileLdsBytes(int flags, int blockSize) const
     int bytes = roundUp(sharedTileLdsOffset(blockSize), 16);
     if (flags & GRADIENTS_INPUT)
         for (const auto& e : encodings_)
-            if (sharesLevels(*e)) bytes += e->numSweptTables() * NUM_SHARED_DIMENSIONS * TILE_POINTS * static_cast<int>(sizeof(float));
+            if (e->sharedAdjointWaves() > 0) bytes += e->numSweptTables() * NUM_SHARED_DIMENSIONS * TILE_POINTS * static_cast<int>(sizeof(float));
     return bytes;
-}
-
-bool FusedNetwork::sharesLevels(const IEncoding& e) const
-{
-    // (as many features as scatterTile() takes)
-    const int features = e.channelsWrittenTogether();
-    return e.hasParameters() && e.levelGroups() > 1 && e.numSweptTables() >= 4 && (features & (features - 1)) == 0 && 2 * features <= WARP_SIZE;
 }
 
 bool FusedNetwork::sharesBackwardTile(int numel, int flags)
@@ -1346,7 +1341,7 @@ bool FusedNetwork::sharesBackwardTile(int numel, int flags)
     int& known = sharesBackwardTile_[flags];   // (but for the size fixed by the specification)
     if (known < 0) {
         known = 0;
-        for (const auto& e : encodings_) known = known || sharesLevels(*e) ? 1 : 0;
+        for (const auto& e : encodings_) known = known || e->sharedAdjointWaves() > 0 ? 1 : 0;
         if (trainsSortedBatches() || compileOptions_.overwriteBlocksizeBackward > 0) known = 0;
         for (bool fused : fusedWeightUpdateLayers(flags, false))
             if (fused) known = 0;   // (as many workgroups as slices of partial sums: a fourth of the tiles)

@@ -22,7 +22,7 @@ struct ArgPack
 
 std::string standaloneSource(const IEncoding& e, const std::string& callForward, const std::string& callAdjoint,
                              const std::string& callCorners = "", const std::string& callScatter = "",
-                             const std::string& callTraceGather = "", const std::string& callTraceScatter = "", int groups = 1)
+                             const std::string& callTraceGather = "", const std::string& callTraceScatter = "", int groups = 1, bool sharedTile = false)
 {
     auto kl = QuickMLP::Instance().kernelLoader();
     std::string codeTemplate = kl->findFile("qmlp/kernels/encoding_kernels.h").value();
@@ -32,6 +32,7 @@ std::string standaloneSource(const IEncoding& e, const std::string& callForward,
     replaceAll(codeTemplate, "$$INCLUDES$$", includes.str());
     replaceAll(codeTemplate, "$$ENCODING_PARAMETERS$$",
                e.hasParameters() ? ", const " + e.parameterName() + " cEncoding" : std::string());
+    replaceAll(codeTemplate, "$$SHARED_TILE$$", sharedTile ? "1" : "0");
     // the channels of a group of levels (EncodingForwardKernel)
     const std::string levels = std::to_string(e.numOutputChannels() / e.channelsWrittenTogether());
     const std::string features = std::to_string(e.channelsWrittenTogether());
@@ -61,10 +62,18 @@ std::string IEncoding::forwardKernelSource(int groups) const
     return standaloneSource(*this, call.str(), "", "", "", "", "", groups);
 }
 
-std::string IEncoding::adjointKernelSource(int adjointMode) const
+std::string IEncoding::adjointKernelSource(int adjointMode, bool sharedTile) const
 {
     const bool hasInputGradients = adjointMode & INPUT_GRADIENTS;
     const bool hasParamGradients = (adjointMode & PARAM_GRADIENTS) && hasParameters();
+    if (sharedTile) {
+        std::string source = standaloneSource(*this, "", "", "", "", "", "", 1, true);
+        replaceAll(source, "$$ENCODING$$", qualifiedName());
+        replaceAll(source, "$$SHARED_WAVES$$", std::to_string(sharedAdjointWaves()));
+        replaceAll(source, "$$INPUT_GRADIENTS$$", hasInputGradients ? "true" : "false");
+        replaceAll(source, "$$PARAMETER_GRADIENTS$$", hasParamGradients ? "true" : "false");
+        return source;
+    }
     // encodings with a tile-wide scatter take their parameter gradients out of the per-point call
     std::stringstream call, scatter;
     call << qualifiedName() << "::template adjoint<" << (hasInputGradients ? "true" : "false") << ", "
@@ -88,6 +97,7 @@ void IEncoding::precompile(int adjointMode)
     if (adjointMode > 0) {
         CHECK_ERROR(adjointMode <= ALL_GRADIENTS, "Illegal adjoint mode");
         kl->getKernel("qmlp::kernel::EncodingAdjointKernel", adjointKernelSource(adjointMode), flags);
+        if (sharedAdjointWaves() > 0) kl->getKernel("qmlp::kernel::EncodingAdjointSharedKernel", adjointKernelSource(adjointMode, true), flags);
         if (const auto* layout = (adjointMode & PARAM_GRADIENTS) && hasParameters() ? sliceLayout(true) : nullptr) {
             for (int v = 0; v < recordsVariants(*layout); ++v) compileRecords(*layout, adjointMode & INPUT_GRADIENTS, v, flags);
             compileSlices(*layout, true, flags);
@@ -172,10 +182,12 @@ void IEncoding::adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& ad
     if (numel == 0) return;
     const bool bySlices = tmpMemory != nullptr && adjointMemory(numel, adjointMode) > 0;
 
-    if (!bySlices && !adjointKernel_[adjointMode].has_value())
-        adjointKernel_[adjointMode] = QuickMLP::Instance().kernelLoader()->getKernel(
-            "qmlp::kernel::EncodingAdjointKernel", adjointKernelSource(adjointMode),
-            QuickMLP::Instance().getCompileFlags()).value();
+    const bool sharedTile = !bySlices && sharedAdjointWaves() > 0 && numel <= SHARED_ADJOINT_MAX_BATCH;
+    auto& kernel = sharedTile ? adjointSharedKernel_[adjointMode] : adjointKernel_[adjointMode];
+    if (!bySlices && !kernel.has_value())
+        kernel = QuickMLP::Instance().kernelLoader()->getKernel(
+            sharedTile ? "qmlp::kernel::EncodingAdjointSharedKernel" : "qmlp::kernel::EncodingAdjointKernel",
+            adjointKernelSource(adjointMode, sharedTile), QuickMLP::Instance().getCompileFlags()).value();
 
     std::vector<char> paramBytes(4096);
     if (hasParameters()) {
@@ -188,9 +200,9 @@ void IEncoding::adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& ad
     if (bySlices) {
         adjointBySlices(*sliceLayout(true), input, adjOutput, adjInput, stream, adjointMode, tmpMemory, paramBytes.data());
     } else {
-        auto& fun = adjointKernel_[adjointMode].value();
-        const int block = 256;
-        const int grid = static_cast<int>(std::min<long long>(divUp<long long>(numel, block), fun.fullGridSize(block, 0)));
+        auto& fun = kernel.value();
+        const int block = sharedTile ? sharedAdjointWaves() * 64 : 256;
+        const int grid = static_cast<int>(std::min<long long>(divUp<long long>(numel, sharedTile ? 64 : block), fun.fullGridSize(block, 0)));
         auto inputAcc = input.accessor<kernel::Tensor2Read<float>>();
         auto adjOutputAcc = adjOutput.accessor<kernel::Tensor2Read<float>>();
         auto adjInputAcc = adjInput.accessor<kernel::Tensor2RW<float>>();
@@ -207,7 +219,8 @@ size_t IEncoding::adjointMemory(long long numel, int adjointMode) const
 {
     if (!(adjointMode & PARAM_GRADIENTS) || !hasParameters() || numel >= (1 << 27)) return 0;
     const auto* layout = sliceLayout(true);
-    return layout && slicesPay(*layout, numel, SLICE_GRADIENTS_MIN_BATCH_STANDALONE) ? layout->workspaceBytes(numel) : 0;
+    return layout && slicesPay(*layout, numel, adjointMode & INPUT_GRADIENTS ? SLICE_GRADIENTS_MIN_BATCH_STANDALONE_INPUT
+                                                                               : SLICE_GRADIENTS_MIN_BATCH_STANDALONE) ? layout->workspaceBytes(numel) : 0;
 }
 
 int IEncoding::recordsVariants(const GradientSliceLayout& layout)

@@ -26,7 +26,7 @@ GRIDS = [grid(8, 2, 13, "float"), grid(9, 1, 14, "half"), grid(11, 4, 12, "float
 def adjoint(enc, x, table, g, flags, with_memory):
     size = ctypes.c_size_t()
     check(lib.qmlp_encoding_adjoint_memory(enc._handle, x.shape[0], flags, ctypes.byref(size)))
-    assert (size.value > 0) == (x.shape[0] >= 1 << 14)
+    assert (size.value > 0) == (x.shape[0] >= (1 << 14) + (flags & 1))
     memory = torch.empty(max(size.value, 256), dtype=torch.uint8, device="cuda")
     adj_x, adj_table = torch.zeros_like(x), torch.zeros(table.shape, device="cuda")
     check(lib.qmlp_encoding_adjoint_in(enc._handle, desc(x), desc(g), desc(adj_x), current_stream(x.device), desc(table),

@@ -7,7 +7,9 @@ import pytest
 import torch
 
 import qmlp
-from helpers import warm_cache
+from helpers import require_gpu, warm_cache
+from qmlp._lib import check, lib
+from qmlp.classes import current_stream, desc
 
 pytestmark = pytest.mark.gpu
 
@@ -87,3 +89,28 @@ def test_small_batches_are_differentiated_like_large_ones(encodings, flags):
         for a, b in pairs:
             assert float(b.abs().max()) > 0
             torch.testing.assert_close(a, b, rtol=1e-3, atol=1e-4 * float(b.abs().max()))
+
+
+@pytest.mark.parametrize("encoding", [grid(9, 2, 0), grid(5, 1, 1, precision="float"), grid(4, 4, 0)])
+def test_standalone_adjoint_of_small_batches(encoding):
+    """Against a batch that is too large for the kernel, whose further rows have no adjoint."""
+    require_gpu(encoding, (1, 2, 3))
+    enc = qmlp.Encoding(json.dumps(encoding))
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.rand((20000, 3), device="cuda", generator=gen) * 1.02 - 0.01
+    g = torch.rand((20000, enc.num_output_channels()), device="cuda", generator=gen) - 0.5
+    table = (torch.rand(enc.num_parameters(), device="cuda", generator=gen) - 0.5).to(enc.parameter_dtype())
+
+    def adjoint(x, g, flags):
+        adj_x, adj_table = torch.ones_like(x), torch.zeros(table.shape, device="cuda")
+        check(lib.qmlp_encoding_adjoint(enc._handle, desc(x), desc(g), desc(adj_x), current_stream(x.device), desc(table),
+                                        desc(adj_table), flags))
+        return adj_x, adj_table
+
+    for n in (1, 63, 65, 1000, 256 * 64):
+        front = g.clone()
+        front[n:] = 0
+        for flags in (1, 2, 3):
+            for a, b in zip(adjoint(x[:n], g[:n], flags), adjoint(x, front, flags)):
+                b = b[:n] if b.dim() == 2 else b
+                torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5 * float(b.abs().max()))
