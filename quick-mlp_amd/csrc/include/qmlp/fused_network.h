@@ -250,6 +250,9 @@ private:
         CompiledKernel adjoint;
         std::vector<SliceGradientKernel> sliceGradients;
         std::vector<WeightUpdateKernel> layers;
+        CompiledKernel allLayers;         // WeightUpdateLayersKernel (updatesAllLayers), with updateWorkgroups per slice of the batch
+        bool updatesAllLayers = false;
+        int updateWorkgroups = 0;
         CompiledKernel reduce;
         CompiledKernel transpose;
         int perEntryAdjointMemoryBytes = 0;
@@ -534,7 +537,8 @@ private:
 
     std::string forwardSource(int blockSize, int pointsPerLane, bool registerStaging = false, bool derivatives = false, bool inputOnly = false, bool sharedTile = false) const;
     std::string backwardSource(int flags, int blockSize, bool sliceGradients = false, bool recompute = false, bool twoWavefrontsPerSimd = false, bool sharedTile = false) const;
-    std::string weightUpdateSource(int blockSize) const;
+    /** \param fusedLayers also the kernel that updates all layers but these in one launch */
+    std::string weightUpdateSource(int blockSize, const std::vector<bool>* fusedLayers = nullptr) const;
     std::string weightUpdateKernelName(int layer, int& numChunks, int& tilesPerBlock) const;
     void fillEncodingsAndActivations(std::string& codeTemplate) const;
     int forwardBlockSize(int overwrite, bool adjoint, int* pointsPerLane = nullptr, int fixedPointsPerLane = 0) const;

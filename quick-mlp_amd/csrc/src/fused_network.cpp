@@ -1428,10 +1428,24 @@ std::string FusedNetwork::cooperativeBackwardSource(int flags, bool sliceGradien
     return code;
 }
 
-std::string FusedNetwork::weightUpdateSource(int blockSize) const
+std::string FusedNetwork::weightUpdateSource(int blockSize, const std::vector<bool>* fusedLayers) const
 {
     auto kl = QuickMLP::Instance().kernelLoader();
     std::string code = kl->findFile("qmlp/kernels/network_weight_update.h").value();
+    std::stringstream call;
+    for (size_t layer = 0; fusedLayers && layer < layers_.size(); ++layer) {
+        if ((*fusedLayers)[layer]) continue;
+        const auto& l = layers_[layer];
+        const auto& info = backwardInfo_[layer];
+        int chunks = 0, tiles = 0;
+        std::string name = weightUpdateKernelName(static_cast<int>(layer), chunks, tiles);
+        replaceAll(name, "WeightUpdateKernel", "weightUpdateBlock");
+        call << "    if (block < " << chunks << " * numSlices) {\n        " << name << "(block, " << chunks << " * numSlices, numTiles, partial + " << l.weightsStart << ", "
+             << (l.useBias ? "partial + " + std::to_string(l.biasStart) : std::string("nullptr")) << ", sliceStride,\n            adjointTmpMemory + "
+             << info.offsetAdjOut << "ll * numel64, forwardTmpMemory + " << info.offsetIn << "ll * numel64);\n        return;\n    }\n    block -= " << chunks << " * numSlices;\n";
+    }
+    replaceAll(code, "$$ALL_LAYERS$$", fusedLayers ? "1" : "0");
+    replaceAll(code, "$$CALL_LAYERS$$", call.str());
     replaceAll(code, "$$DEFINE_ACTIVATIONS$$", activationDefinitions());
     replaceAll(code, "$$BLOCK_SIZE$$", std::to_string(blockSize));
     return code;
@@ -1899,6 +1913,8 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
             wk.kernel.sharedMemorySize = tiles * 256 * static_cast<int>(sizeof(float));
             if (wk.kernel.sharedMemorySize > MaxSharedMemoryBytes())
                 throw configuration_error("Layer %d too large for block-wise weight update!", static_cast<int>(layer));
+            ak.updateWorkgroups += wk.numChunks;
+            ak.allLayers.sharedMemorySize = std::max(ak.allLayers.sharedMemorySize, wk.kernel.sharedMemorySize);
             wk.kernel.fun = kl->getKernel(name, source, loaderFlags(compileOnly)).value();
             if (!compileOnly) {
                 wk.kernel.fullGrid = wk.kernel.fun.fullGridSize(blockSize, wk.kernel.sharedMemorySize);
@@ -1907,6 +1923,12 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
                               wk.kernel.fun.numVgprs(), wk.kernel.fullGrid);
             }
         }
+    }
+    if (hasNetworkGradients && std::count(ak.fusedLayers.begin(), ak.fusedLayers.end(), false) >= 2) {
+        ak.allLayers.blockSize = weightUpdateBlockSize();
+        ak.allLayers.fun = kl->getKernel("qmlp::kernel::WeightUpdateLayersKernel", weightUpdateSource(ak.allLayers.blockSize, &ak.fusedLayers),
+                                         loaderFlags(compileOnly)).value();
+        ak.updatesAllLayers = true;
     }
     if (!compileOnly) backwardKernel_[flags][variant][mode] = std::move(ak);
 }
@@ -2737,8 +2759,17 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
     const int slices = partialSliceCount;
     float* partial = reinterpret_cast<float*>(static_cast<char*>(tmpMemoryAdjoint)
                                               + static_cast<size_t>(ak.perEntryAdjointMemoryBytes) * static_cast<size_t>(numel64));
+    // one launch for all layers where they fit onto the device side by side
+    const bool together = ak.updatesAllLayers && !parallel && slices * ak.updateWorkgroups <= 2 * KernelFunction::computeUnits();
+    if (together) {
+        int numTilesArg = numTiles, numSlices = slices, sliceStride = numParameters_;
+        const half* adjointTmpMemory = static_cast<const half*>(tmpMemoryAdjoint);
+        const half* forwardTmpMemory = static_cast<const half*>(tmpMemoryForward);
+        void* args[] = {&numTilesArg, &numSlices, &partial, &sliceStride, &adjointTmpMemory, &forwardTmpMemory};
+        ak.allLayers.fun.launch(slices * ak.updateWorkgroups, ak.allLayers.blockSize, ak.allLayers.sharedMemorySize, stream, args);
+    }
     for (size_t layer = 0; layer < layers_.size(); ++layer) {
-        if (ak.fusedLayers[layer]) continue;
+        if (ak.fusedLayers[layer] || together) continue;
         const auto& ls = layers_[layer];
         const auto& ali = backwardInfo_[layer];
         const auto& wk = ak.layers[layer];
