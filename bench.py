@@ -196,13 +196,13 @@ def run_train(case, steps, warmup, input_gradients=True, warmup_seconds=0.0):
         for g in grad_enc:
             if g is not None:
                 g.zero_()
-        out, tmp = net.forward_raw(x, params, enc, flags)
+        out, tmp, contents = net.forward_raw(x, params, enc, flags, contents=True)
         # (mean squared error with the loss scaled by 2^16, as fp16 training does: 2 / numel alone is 5e-7 for 2^21
         # points with two outputs, and the adjoints of the layers, which are halves, underflow to zero -- a step whose
         # gradients vanish is not the work of a train step: kernels that skip zeros would look faster than they are)
         adj_out = (out - target) * (2.0 * LOSS_SCALE / out.numel())
         net.adjoint_raw(x, adj_out, flags, tmp, params, enc, grad_network=grad_net, grad_encodings=grad_enc,
-                        adj_input=adj_in if input_gradients else None)
+                        adj_input=adj_in if input_gradients else None, contents=contents)
 
     step()
     torch.cuda.synchronize()
@@ -282,8 +282,8 @@ def run_mlp(n_in, widths, n, device, steps, warmup, cached_input=False, train=Fa
 
         def step():
             # the reference's "forward + backward": gradients for the input and the weights
-            out, tmp = net.forward_raw(x, params, [], 3)
-            net.adjoint_raw(x, adj, 3, tmp, params, [], grad_network=grad_net, adj_input=adj_in)
+            out, tmp, contents = net.forward_raw(x, params, [], 3, contents=True)
+            net.adjoint_raw(x, adj, 3, tmp, params, [], grad_network=grad_net, adj_input=adj_in, contents=contents)
     step()
     torch.cuda.synchronize()
     elapsed, launch_ms = time_steps(step, steps, warmup)

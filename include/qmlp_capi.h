@@ -114,23 +114,33 @@ int qmlp_network_forward_memory(qmlp_network_t network, int num_elements, int ad
 /* forward(input, output, tmpMemory, stream), :263 */
 int qmlp_network_forward(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* output,
                          void* tmp_memory, void* stream);
+/* The same for an adjoint pass with these flags: stores no more than that one reads, and sets `contents` to what
+ * qmlp_network_adjoint_for has to be told of the memory (which may be moved in between). */
+int qmlp_network_forward_for(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* output,
+                             int adjoint_flags, void* tmp_memory, int* contents, void* stream);
 /* zeroGradients(), :269 */
 int qmlp_network_zero_gradients(qmlp_network_t network);
 /* adjointMemory(numElements, flags), :280 */
 int qmlp_network_adjoint_memory(qmlp_network_t network, int num_elements, int adjoint_flags, size_t* bytes);
 /* adjoint(input, adjOutput, flags, adjInput, tmpFwd, tmpAdj, stream), :313.
- * adj_input may be NULL / undefined unless QMLP_GRADIENTS_INPUT is set. */
+ * adj_input may be NULL / undefined unless QMLP_GRADIENTS_INPUT is set. `input` still holds the values that the
+ * forward pass saw: they are read again. tmp_memory_forward: as qmlp_network_forward left it. */
 int qmlp_network_adjoint(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* adj_output,
                          int adjoint_flags, const qmlp_tensor* adj_input, const void* tmp_memory_forward,
                          void* tmp_memory_adjoint, void* stream);
-/* Which of QMLP_GRADIENTS_INPUT and QMLP_GRADIENTS_NETWORK_WEIGHTS an adjoint pass on what the forward pass left in
- * tmp_memory_forward can write, every element, instead of adding to them; and an adjoint pass that does so for the
- * `overwrite` among them: those gradients need not be zeroed. */
+/* Which of QMLP_GRADIENTS_INPUT and QMLP_GRADIENTS_NETWORK_WEIGHTS an adjoint pass can write, every element, instead of
+ * adding to them (tmp_memory_forward: not looked at, may be NULL); and an adjoint pass that does so for the `overwrite`
+ * among them: those gradients need not be zeroed. */
 int qmlp_network_overwritable_gradients(qmlp_network_t network, int num_elements, int adjoint_flags,
                                         const void* tmp_memory_forward, int* flags);
 int qmlp_network_adjoint_overwriting(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* adj_output,
                                      int adjoint_flags, int overwrite, const qmlp_tensor* adj_input,
                                      const void* tmp_memory_forward, void* tmp_memory_adjoint, void* stream);
+/* qmlp_network_adjoint_overwriting on what qmlp_network_forward_for left, with the `contents` that it reported. Where
+ * adjoint_flags need more than that, the forward pass runs again into tmp_memory_forward. */
+int qmlp_network_adjoint_for(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* adj_output,
+                             int adjoint_flags, int overwrite, const qmlp_tensor* adj_input,
+                             void* tmp_memory_forward, int contents, void* tmp_memory_adjoint, void* stream);
 /* clearCachedKernels(), :319 */
 int qmlp_network_clear_cached_kernels(qmlp_network_t network);
 /* Generates and compiles all kernels of the network without touching a GPU

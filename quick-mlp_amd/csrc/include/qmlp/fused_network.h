@@ -308,16 +308,19 @@ private:
      */
     std::vector<long long> derivativeOffsets_;
     int derivativeBytesPerPoint_ = 0;
-    /** The adjoint flags that the caller announced last: forwardMemory(n, flags), adjoint(..., flags, ...). */
+    /**
+     * For the forward passes that are not told what follows them: the adjoint flags that the caller announced last
+     * (forwardMemory(n, flags), adjoint(..., flags, ...)) decide whether position derivatives are stored beside the
+     * intermediates, and here stands which memory holds those of how many points. Only a hint: memory that is not listed
+     * (moved, or pushed out of the list) has all that an adjoint pass needs, and the grids are gathered from again.
+     */
     int announcedFlags_ = 0;
-    /** What the last training pass left in a forward memory. */
-    struct ForwardRecord
-    {
-        int numel = 0;
-        bool derivatives = false;   // position derivatives of the grids
-        BackwardMode mode = BACKWARD_STORED;   // else: what the backward kernel of this mode reads, the encoded input at most
-    };
-    std::unordered_map<const void*, ForwardRecord> forwardRecords_;
+    std::unordered_map<const void*, int> derivativeMemories_;
+    static constexpr size_t MAX_DERIVATIVE_MEMORIES = 256;
+    /** What of the intermediates the backward kernel of this mode reads (ForwardContents). */
+    int contentsFor(BackwardMode mode) const;
+    /** forward() whose memory receives the given contents. */
+    void launchTraining(const Tensor& input, Tensor& output, void* tmpMemory, stream_t stream, int contents);
     /** Whether adjoint(flags) over numel points runs the layers again in its backward kernel instead of reading
      *  their intermediates: a training pass that is followed by it keeps the encoded input only. */
     bool recomputesFor(int numel, int flags) const;
@@ -334,12 +337,11 @@ private:
     bool differentiatesEncodings(int flags, bool sliceGradients) const;
     mutable int recomputesKnown_[ADJOINT_MODE_MAX_COMBINATIONS][2];   // canRecompute(), -1: not known yet
     /**
-     * recomputesFor(), and the backward kernel that runs the layers again holds its registers: loaded on the first
-     * call for these flags (it is the kernel that adjoint() will run), and not used if it spills more than a few
-     * words (16 -> 64 -> 64 -> 16 with biases: 27 gradient tiles and 72 registers of pre-activations, 316 bytes).
+     * The mode of the backward kernel of a batch: cooperatesFor(), else recomputesFor(), where that kernel also holds its
+     * registers: it is loaded on the first call for these flags (it is the kernel that adjoint() will run), and not used
+     * if it spills more than a few words (16 -> 64 -> 64 -> 16 with biases: 27 gradient tiles and 72 registers of
+     * pre-activations, 316 bytes).
      */
-    bool recomputes(int numel, int flags);
-    /** The mode of the backward kernel of a batch: cooperative where it holds its registers, else as recomputes() says. */
     BackwardMode backwardMode(int numel, int flags);
     int recomputeVerdict_[ADJOINT_MODE_MAX_COMBINATIONS][2][3];   // [..][..][mode], -1: not known yet
     static constexpr int MAX_RECOMPUTE_SCRATCH = 64;
@@ -433,9 +435,27 @@ public:
 
     /**
      * Forward pass that stores intermediate results in 'tmpMemory' (forwardMemory() bytes,
-     * 16-byte aligned) for a following adjoint().
+     * 16-byte aligned) for a following adjoint(): all that any of them reads.
      */
     void forward(const Tensor& input, Tensor& output, void* tmpMemory, stream_t stream);
+
+    /**
+     * What a forward pass left in its memory, as the caller hands it on to adjoint() together with that memory, which may
+     * have been moved in between: how much of the intermediates, and whether the position derivatives of the grids.
+     */
+    enum ForwardContents
+    {
+        CONTENTS_INTERMEDIATES = 0,   // all of them
+        CONTENTS_ENCODED_INPUT = 1,   // the encoded input only
+        CONTENTS_NOTHING = 2,         // nothing: the adjoint pass starts from the input rows
+        CONTENTS_AMOUNT = 3,          // (mask of the three above)
+        CONTENTS_DERIVATIVES = 4
+    };
+    /**
+     * forward() that stores no more than adjoint(adjointFlags) reads.
+     * \return ForwardContents
+     */
+    int forward(const Tensor& input, Tensor& output, void* tmpMemory, stream_t stream, AdjointModeFlags adjointFlags);
 
     /** Zeros the gradients of the network weights and of the encodings. */
     void zeroGradients();
@@ -448,6 +468,7 @@ public:
      * Adjoint pass following forward(). Weight and encoding gradients are added to the
      * gradient tensors set via setNetworkParameter / IEncoding::setParameter with
      * Usage::GRADIENTS; input gradients are added to 'adjInput'.
+     * \param input the input of the forward pass, with the values it had there: they are read again
      */
     void adjoint(const Tensor& input, const Tensor& adjOutput, AdjointModeFlags adjointFlags, Tensor& adjInput,
                  const void* tmpMemoryForward, void* tmpMemoryAdjoint, stream_t stream);
@@ -457,13 +478,19 @@ public:
      */
     void adjoint(const Tensor& input, const Tensor& adjOutput, AdjointModeFlags adjointFlags, Tensor& adjInput,
                  const void* tmpMemoryForward, void* tmpMemoryAdjoint, stream_t stream, AdjointModeFlags overwrite);
+    /**
+     * \param contents what the forward pass returned that left tmpMemoryForward. Where these flags need more than that,
+     *    the forward pass runs again into the same memory.
+     */
+    void adjoint(const Tensor& input, const Tensor& adjOutput, AdjointModeFlags adjointFlags, Tensor& adjInput,
+                 const void* tmpMemoryForward, void* tmpMemoryAdjoint, stream_t stream, AdjointModeFlags overwrite, int contents);
 
     /**
-     * Which of the gradients of the input and of the network weights adjoint() on what forward() left in tmpMemoryForward
-     * can write, every element, instead of adding to them: the caller need not zero them then, nor a kernel read them
-     * (2^20 points of 16 channels: 64 MB each; a fill kernel of 4 us in front of a small batch).
+     * Which of the gradients of the input and of the network weights adjoint() can write, every element, instead of adding
+     * to them: the caller need not zero them then, nor a kernel read them (2^20 points of 16 channels: 64 MB each; a fill
+     * kernel of 4 us in front of a small batch). Depends on neither the memory of the forward pass nor what it holds.
      */
-    [[nodiscard]] AdjointModeFlags overwritableGradients(int numel, AdjointModeFlags adjointFlags, const void* tmpMemoryForward);
+    [[nodiscard]] AdjointModeFlags overwritableGradients(int numel, AdjointModeFlags adjointFlags, const void* tmpMemoryForward = nullptr);
 
     /** For debugging, clears all cached kernels. */
     void clearCachedKernels();

@@ -319,6 +319,15 @@ int qmlp_network_forward(qmlp_network_t network, const qmlp_tensor* input, const
     QMLP_API_END
 }
 
+int qmlp_network_forward_for(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* output,
+                             int adjoint_flags, void* tmp_memory, int* contents, void* stream)
+{
+    QMLP_API_BEGIN
+    Tensor out = wrap(output);
+    *contents = network->network->forward(wrap(input), out, tmp_memory, static_cast<stream_t>(stream), adjoint_flags);
+    QMLP_API_END
+}
+
 int qmlp_network_zero_gradients(qmlp_network_t network)
 {
     QMLP_API_BEGIN
@@ -360,6 +369,17 @@ int qmlp_network_adjoint_overwriting(qmlp_network_t network, const qmlp_tensor* 
     Tensor adjIn = wrap(adj_input);
     network->network->adjoint(wrap(input), wrap(adj_output), adjoint_flags, adjIn, tmp_memory_forward,
                               tmp_memory_adjoint, static_cast<stream_t>(stream), overwrite);
+    QMLP_API_END
+}
+
+int qmlp_network_adjoint_for(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* adj_output,
+                             int adjoint_flags, int overwrite, const qmlp_tensor* adj_input,
+                             void* tmp_memory_forward, int contents, void* tmp_memory_adjoint, void* stream)
+{
+    QMLP_API_BEGIN
+    Tensor adjIn = wrap(adj_input);
+    network->network->adjoint(wrap(input), wrap(adj_output), adjoint_flags, adjIn, tmp_memory_forward,
+                              tmp_memory_adjoint, static_cast<stream_t>(stream), overwrite, contents);
     QMLP_API_END
 }
 

@@ -260,8 +260,6 @@ bool FusedNetwork::canRecompute(int flags, bool sliceGradients) const
     return lds <= MaxSharedMemoryBytes();
 }
 
-bool FusedNetwork::recomputes(int numel, int flags) { return backwardMode(numel, flags) != BACKWARD_STORED; }
-
 FusedNetwork::BackwardMode FusedNetwork::backwardMode(int numel, int flags)
 {
     if (flags <= 0 || flags >= ADJOINT_MODE_MAX_COMBINATIONS) return BACKWARD_STORED;
@@ -2215,14 +2213,14 @@ void FusedNetwork::prepare(int numel, int adjointFlags)
     CHECK_ERROR(adjointFlags >= 0 && adjointFlags < ADJOINT_MODE_MAX_COMBINATIONS, "prepare(): unknown adjoint flags ", adjointFlags);
     if (numel == 0) return;
     // the forward kernels that launchForward() takes for the pieces of a batch of this size
+    // ([0]: inference, [1]: forward passes that store all intermediates, [2]: that store the encoded input only)
     if (adjointFlags > 0) announcedFlags_ = adjointFlags;
-    for (int store = 0; store <= (adjointFlags > 0 ? 1 : 0); ++store)
+    const int forwardKinds = adjointFlags <= 0 ? 1 : contentsFor(backwardMode(numel, adjointFlags)) == CONTENTS_ENCODED_INPUT ? 3 : 2;
+    for (int store = 0; store < forwardKinds; ++store)
         for (long long start = 0; start < numel;) {
             int launchTiles = 0;
-            const BackwardMode mode = store ? backwardMode(numel, adjointFlags) : BACKWARD_STORED;
-            const bool stores = store != 0 && !(mode == BACKWARD_COOPERATIVE && cooperativeReadsInputRows());
-            const auto& ck = forwardKernelFor(stores, static_cast<int>(divUp<long long>(numel - start, TILE_POINTS)), &launchTiles, false,
-                                              stores && storesDerivatives(numel, adjointFlags), stores && mode != BACKWARD_STORED);
+            const auto& ck = forwardKernelFor(store > 0, static_cast<int>(divUp<long long>(numel - start, TILE_POINTS)), &launchTiles, false,
+                                              store > 0 && storesDerivatives(numel, adjointFlags), store > 1);
             start += std::min<long long>({static_cast<long long>(gatherChunkPoints(ck)), static_cast<long long>(launchTiles) * TILE_POINTS,
                                           numel - start});
         }
@@ -2390,6 +2388,36 @@ size_t FusedNetwork::forwardMemory(const Tensor& input, AdjointModeFlags adjoint
 
 void FusedNetwork::forward(const Tensor& input, Tensor& output, void* tmpMemory, stream_t stream)
 {
+    const int numel = input.ndim() > 0 ? input.size(0) : 0;
+    const int contents = CONTENTS_INTERMEDIATES | (storesDerivatives(numel, announcedFlags_) ? CONTENTS_DERIVATIVES : 0);
+    derivativeMemories_.erase(tmpMemory);
+    launchTraining(input, output, tmpMemory, stream, contents);
+    if (numel == 0 || !(contents & CONTENTS_DERIVATIVES)) return;
+    if (derivativeMemories_.size() >= MAX_DERIVATIVE_MEMORIES) derivativeMemories_.clear();
+    derivativeMemories_[tmpMemory] = numel;
+}
+
+int FusedNetwork::forward(const Tensor& input, Tensor& output, void* tmpMemory, stream_t stream, AdjointModeFlags adjointFlags)
+{
+    if (adjointFlags <= 0 || adjointFlags >= ADJOINT_MODE_MAX_COMBINATIONS)
+        throw std::runtime_error("At least one derivative must be enabled");
+    CHECK_DIM(input, 2);
+    const int numel = input.size(0);
+    const int contents = numel > 0 ? contentsFor(backwardMode(numel, adjointFlags)) | (storesDerivatives(numel, adjointFlags) ? CONTENTS_DERIVATIVES : 0)
+                                   : static_cast<int>(CONTENTS_INTERMEDIATES);
+    derivativeMemories_.erase(tmpMemory);
+    launchTraining(input, output, tmpMemory, stream, contents);
+    return contents;
+}
+
+int FusedNetwork::contentsFor(BackwardMode mode) const
+{
+    if (mode == BACKWARD_COOPERATIVE && cooperativeReadsInputRows()) return CONTENTS_NOTHING;
+    return mode == BACKWARD_COOPERATIVE || mode == BACKWARD_RECOMPUTED ? CONTENTS_ENCODED_INPUT : CONTENTS_INTERMEDIATES;
+}
+
+void FusedNetwork::launchTraining(const Tensor& input, Tensor& output, void* tmpMemory, stream_t stream, int contents)
+{
     CHECK_DIM(input, 2);
     CHECK_DIM(output, 2);
     CHECK_SIZE(input, 1, channelsIn());
@@ -2404,12 +2432,9 @@ void FusedNetwork::forward(const Tensor& input, Tensor& output, void* tmpMemory,
     CHECK_ERROR(tmpMemory != nullptr, "forward() needs temporary memory of forwardMemory() bytes");
     CHECK_ERROR(reinterpret_cast<uintptr_t>(tmpMemory) % 16 == 0, "The temporary memory must be aligned to 16 bytes");
 
-    const bool derivatives = storesDerivatives(numel, announcedFlags_);
-    const BackwardMode mode = backwardMode(numel, announcedFlags_);
-    if (derivatives || mode != BACKWARD_STORED) forwardRecords_[tmpMemory] = ForwardRecord{numel, derivatives, mode};
-    else forwardRecords_.erase(tmpMemory);
-    if (mode == BACKWARD_COOPERATIVE && cooperativeReadsInputRows()) launchForward(false, input, output, nullptr, stream);
-    else launchForward(true, input, output, static_cast<half*>(tmpMemory), stream, false, derivatives, mode != BACKWARD_STORED);
+    const int amount = contents & CONTENTS_AMOUNT;
+    if (amount == CONTENTS_NOTHING) launchForward(false, input, output, nullptr, stream);
+    else launchForward(true, input, output, static_cast<half*>(tmpMemory), stream, false, (contents & CONTENTS_DERIVATIVES) != 0, amount == CONTENTS_ENCODED_INPUT);
 }
 
 void FusedNetwork::zeroGradients()
@@ -2473,7 +2498,7 @@ bool FusedNetwork::differentiatesEncodings(int flags, bool sliceGradients) const
     return false;
 }
 
-FusedNetwork::AdjointModeFlags FusedNetwork::overwritableGradients(int numel, AdjointModeFlags adjointFlags, const void* tmpMemoryForward)
+FusedNetwork::AdjointModeFlags FusedNetwork::overwritableGradients(int numel, AdjointModeFlags adjointFlags, const void*)
 {
     if (numel <= 0) return 0;
     // the sums of the weight gradients, all of them, are written at the end
@@ -2481,10 +2506,7 @@ FusedNetwork::AdjointModeFlags FusedNetwork::overwritableGradients(int numel, Ad
     if (!(adjointFlags & GRADIENTS_INPUT)) return weights;
     // the rows of a batch that trained in sorted order are moved to the caller's tensor, all of them, at the end
     if (sortsTraining(numel)) return weights | GRADIENTS_INPUT;
-    const auto it = forwardRecords_.find(tmpMemoryForward);
-    if (it == forwardRecords_.end() || it->second.numel != numel || it->second.mode != BACKWARD_COOPERATIVE
-        || backwardMode(numel, adjointFlags) != BACKWARD_COOPERATIVE)
-        return weights;
+    if (backwardMode(numel, adjointFlags) != BACKWARD_COOPERATIVE) return weights;
     // the cooperative kernel: one that reads the input rows writes the channels of its encoding, else all of them
     const bool all = differentiatesEncodings(adjointFlags, useSliceGradients(numel, adjointFlags))
         && (directInputStart() < 0 || (directInputStart() == 0 && encodings_[0]->numOutputChannels() == channelsIn()));
@@ -2499,6 +2521,16 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
 
 void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, AdjointModeFlags adjointFlags,
                            Tensor& adjInput, const void* tmpMemoryForward, void* tmpMemoryAdjoint, stream_t stream, AdjointModeFlags overwrite)
+{
+    const auto it = derivativeMemories_.find(tmpMemoryForward);
+    const bool derivatives = it != derivativeMemories_.end() && input.ndim() > 0 && it->second == input.size(0);
+    if (adjointFlags > 0 && adjointFlags < ADJOINT_MODE_MAX_COMBINATIONS) announcedFlags_ = adjointFlags;
+    adjoint(input, adjOutput, adjointFlags, adjInput, tmpMemoryForward, tmpMemoryAdjoint, stream, overwrite,
+            CONTENTS_INTERMEDIATES | (derivatives ? CONTENTS_DERIVATIVES : 0));
+}
+
+void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, AdjointModeFlags adjointFlags, Tensor& adjInput,
+                           const void* tmpMemoryForward, void* tmpMemoryAdjoint, stream_t stream, AdjointModeFlags overwrite, int contents)
 {
     CHECK_DIM(input, 2);
     CHECK_DIM(adjOutput, 2);
@@ -2540,33 +2572,21 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
 
     const bool sliceGradients = useSliceGradients(numel, adjointFlags);
     CHECK_ERROR(!sliceGradients || numel < (1 << 27), "batches of 2^27 points or more: set options.slice_gradients to 0");
-    announcedFlags_ = adjointFlags;
-    CHECK_ERROR((overwrite & ~overwritableGradients(numel, adjointFlags, tmpMemoryForward)) == 0,
+    CHECK_ERROR((overwrite & ~overwritableGradients(numel, adjointFlags)) == 0,
                 "adjoint() adds to gradients of this batch that it was asked to overwrite");
     const bool overwriteInputGradients = overwrite & GRADIENTS_INPUT;
-    // what the forward pass that wrote this forward memory left there: the position derivatives of the grids? Of the
-    // intermediates the encoded input only?
-    bool derivativesStored = false;
-    BackwardMode mode = BACKWARD_STORED;
-    {
-        const auto it = forwardRecords_.find(tmpMemoryForward);
-        if (it != forwardRecords_.end() && it->second.numel == numel) {
-            derivativesStored = hasInputGradients && sliceGradients && it->second.derivatives;
-            if (it->second.mode != BACKWARD_STORED) {
-                if (backwardMode(numel, adjointFlags) == it->second.mode) {
-                    mode = it->second.mode;
-                } else {
-                    // Announced otherwise: the kernels of these flags read intermediates that the training pass did not
-                    // keep. The forward pass runs again into the same memory, this time storing them (a batch that
-                    // trains in sorted order is sorted again: rows, order and slab totals are rewritten together).
-                    QuickMLP::Instance().getLogger()->debug("adjoint(flags %d): the forward pass kept the encoded input only; it runs again", adjointFlags);
-                    Tensor scratchOutput(precisionOut(), {numel, channelsOut()});
-                    const bool derivatives = it->second.derivatives;
-                    it->second.mode = BACKWARD_STORED;
-                    launchForward(true, input, scratchOutput, static_cast<half*>(const_cast<void*>(tmpMemoryForward)), stream, false, derivatives, false);
-                }
-            }
-        }
+    CHECK_ERROR(contents >= 0 && contents <= (CONTENTS_DERIVATIVES | CONTENTS_NOTHING) && (contents & CONTENTS_AMOUNT) != CONTENTS_AMOUNT,
+                "adjoint(): unknown contents of the forward memory ", contents);
+    const bool derivativesInMemory = (contents & CONTENTS_DERIVATIVES) && derivativeBytesPerPoint_ > 0;
+    const bool derivativesStored = hasInputGradients && sliceGradients && derivativesInMemory;
+    BackwardMode mode = backwardMode(numel, adjointFlags);
+    if ((contents & CONTENTS_AMOUNT) > contentsFor(mode)) {
+        // The backward kernel of these flags reads intermediates that the forward pass did not keep for those that it was
+        // told of: it runs again into the same memory (a batch that trains in sorted order is sorted again: rows, order
+        // and slab totals are rewritten together).
+        QuickMLP::Instance().getLogger()->debug("adjoint(flags %d): the forward pass kept too little for it and runs again", adjointFlags);
+        Tensor scratchOutput(precisionOut(), {numel, channelsOut()});
+        launchTraining(input, scratchOutput, const_cast<void*>(tmpMemoryForward), stream, contentsFor(mode) | (derivativesInMemory ? CONTENTS_DERIVATIVES : 0));
     }
     const bool sortedPoints = sortsTraining(numel);
     if (mode == BACKWARD_STORED && sharesBackwardTile(numel, adjointFlags)) mode = BACKWARD_SHARED_TILE;

@@ -168,7 +168,8 @@ struct FusedBackward : torch::autograd::Node
     int flags = 0;
     SavedVariable input, p16;
     std::vector<SavedVariable> tables;
-    at::Tensor memory;   // what the forward pass left for the adjoint pass
+    SavedVariable memory;   // what the forward pass left for the adjoint pass (may come back at another address: saved-tensor hooks)
+    int contents = 0;       // of it
     at::ScalarType parameterType = at::kHalf;
 
     std::string name() const override { return "QmlpFusedBackward"; }
@@ -177,7 +178,7 @@ struct FusedBackward : torch::autograd::Node
         input.reset_data();
         p16.reset_data();
         for (auto& t : tables) t.reset_data();
-        memory.reset();
+        memory.reset_data();
     }
 
     variable_list apply(variable_list&& gradOutputs) override
@@ -185,7 +186,8 @@ struct FusedBackward : torch::autograd::Node
         const size_t n = net->encodings.size();
         variable_list grads(2 + n);
         if (!gradOutputs[0].defined()) return grads;
-        const at::Tensor x = input.unpack(), parameters = p16.unpack();
+        const at::Tensor x = input.unpack(), parameters = p16.unpack(), forwardMemory = memory.unpack();
+        TORCH_CHECK(x.is_cuda() && forwardMemory.device() == x.device() && forwardMemory.is_contiguous(), "saved tensors came back on another device");
         std::vector<at::Tensor> unpacked(n), adjTables(n);
         for (size_t i = 0; i < n; ++i)
             if (net->encodings[i].hasParameters) unpacked[i] = tables[i].unpack();
@@ -210,7 +212,7 @@ struct FusedBackward : torch::autograd::Node
             net->bind(p, wrappedTables);
             // zeroed only where the kernels add to them
             int overwrite = 0;
-            check(qmlp_network_overwritable_gradients(net->handle, in.sizes[0], flags, memory.data_ptr(), &overwrite));
+            check(qmlp_network_overwritable_gradients(net->handle, in.sizes[0], flags, nullptr, &overwrite));
             if (flags & QMLP_GRADIENTS_INPUT) adjInput = overwrite & QMLP_GRADIENTS_INPUT ? at::empty_like(x) : at::zeros_like(x);
             if (flags & QMLP_GRADIENTS_NETWORK_WEIGHTS) {
                 const auto options = parameters.options().dtype(at::kFloat);
@@ -220,8 +222,8 @@ struct FusedBackward : torch::autograd::Node
             if (adjNetwork.defined()) check(qmlp_network_set_parameter(net->handle, &adjNet, QMLP_GRADIENTS));
             for (size_t i = 0; i < n; ++i)
                 if (adjTables[i].defined()) check(qmlp_encoding_set_parameter(net->encodings[i].handle, &adjEnc[i], QMLP_GRADIENTS));
-            const int rc = qmlp_network_adjoint_overwriting(net->handle, &in, &adjOut, flags, overwrite, &adjIn, memory.data_ptr(),
-                                                            scratch.data_ptr(), stream);
+            const int rc = qmlp_network_adjoint_for(net->handle, &in, &adjOut, flags, overwrite, &adjIn, forwardMemory.data_ptr(), contents,
+                                                    scratch.data_ptr(), stream);
             const std::string message = rc != 0 ? qmlp_last_error() : "";
             // no dangling gradient bindings, whatever happened
             qmlp_network_set_parameter(net->handle, nullptr, QMLP_GRADIENTS);
@@ -256,6 +258,7 @@ at::Tensor forward(const Network_ptr& net, const at::Tensor& input, const at::Te
         if (net->encodings[i].hasParameters) positions[i] = tables[i];
     auto output = createOutput(input, net->channelsOut);
     at::Tensor p16, memory;
+    int contents = 0;
     try {
         at::AutoDispatchBelowADInplaceOrView guard;
         p16 = parameters.scalar_type() == at::kHalf ? parameters : parameters.to(at::kHalf);
@@ -268,7 +271,7 @@ at::Tensor forward(const Network_ptr& net, const at::Tensor& input, const at::Te
         check(qmlp_network_forward_memory(net->handle, in.sizes[0], flags, &bytes));
         memory = bytesOn(input, bytes);
         net->bind(p, wrappedTables);
-        check(qmlp_network_forward(net->handle, &in, &out, memory.data_ptr(), stream));
+        check(qmlp_network_forward_for(net->handle, &in, &out, flags, memory.data_ptr(), &contents, stream));
     } catch (const Failure& f) {
         raise(f);
     }
@@ -280,7 +283,8 @@ at::Tensor forward(const Network_ptr& net, const at::Tensor& input, const at::Te
     node->p16 = SavedVariable(p16, false);
     node->tables.reserve(n);
     for (const auto& t : positions) node->tables.emplace_back(t, false);
-    node->memory = memory;
+    node->memory = SavedVariable(memory, false);
+    node->contents = contents;
     node->parameterType = parameters.scalar_type();
     torch::autograd::set_history(output, node);
     return output;

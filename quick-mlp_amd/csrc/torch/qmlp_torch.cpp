@@ -420,17 +420,19 @@ struct NetworkFunction : torch::autograd::Function<NetworkFunction>
         auto tmpForward = torch::empty({static_cast<int64_t>(std::max<size_t>(bytes, 16))},
                                        torch::TensorOptions().dtype(torch::kUInt8).device(input.device()));
         auto output = createOutput(input, static_cast<int>(net->channelsOut()));
+        int contents = 0;   // of tmpForward, which may come back at another address (saved-tensor hooks)
         {
             std::lock_guard<std::mutex> lock(net->mutex_);
             net->bindParameters(p16, encodingParameters);
             const qmlp_tensor in = wrap(input), out = wrap(output);
-            QMLP_CHECK(qmlp_network_forward(net->handle_, &in, &out, tmpForward.data_ptr(), currentStream()));
+            QMLP_CHECK(qmlp_network_forward_for(net->handle_, &in, &out, static_cast<int>(flags), tmpForward.data_ptr(), &contents, currentStream()));
         }
         torch::autograd::variable_list saved = {input, p16, tmpForward};
         saved.insert(saved.end(), encodingParameters.begin(), encodingParameters.end());
         ctx->save_for_backward(saved);
         ctx->saved_data["net"] = net;
         ctx->saved_data["flags"] = flags;
+        ctx->saved_data["contents"] = static_cast<int64_t>(contents);
         ctx->saved_data["param_dtype"] = static_cast<int64_t>(networkParameters.scalar_type());
         std::vector<int64_t> needs;
         for (const auto& t : encodingParameters) needs.push_back(t.defined() && t.requires_grad() ? 1 : 0);
@@ -442,6 +444,7 @@ struct NetworkFunction : torch::autograd::Function<NetworkFunction>
     {
         auto net = ctx->saved_data["net"].toCustomClass<NetworkBindings>();
         const int flags = static_cast<int>(ctx->saved_data["flags"].toInt());
+        const int contents = static_cast<int>(ctx->saved_data["contents"].toInt());
         const auto paramDtype = static_cast<torch::ScalarType>(ctx->saved_data["param_dtype"].toInt());
         const auto needs = ctx->saved_data["enc_needs_grad"].toIntVector();
         const auto saved = ctx->get_saved_variables();
@@ -458,7 +461,7 @@ struct NetworkFunction : torch::autograd::Function<NetworkFunction>
             net->bindParameters(p16, encodingParameters);
             // zeroed only where the kernels add to them
             int overwrite = 0;
-            QMLP_CHECK(qmlp_network_overwritable_gradients(net->handle_, static_cast<int>(input.size(0)), flags, tmpForward.data_ptr(), &overwrite));
+            QMLP_CHECK(qmlp_network_overwritable_gradients(net->handle_, static_cast<int>(input.size(0)), flags, nullptr, &overwrite));
             if (flags & QMLP_GRADIENTS_INPUT) adjInput = overwrite & QMLP_GRADIENTS_INPUT ? torch::empty_like(input) : torch::zeros_like(input);
             if (flags & QMLP_GRADIENTS_NETWORK_WEIGHTS) {
                 const auto options = p16.options().dtype(torch::kFloat32);
@@ -483,8 +486,8 @@ struct NetworkFunction : torch::autograd::Function<NetworkFunction>
             auto tmpAdjoint = torch::empty({static_cast<int64_t>(std::max<size_t>(bytes, 16))},
                                            torch::TensorOptions().dtype(torch::kUInt8).device(input.device()));
             const qmlp_tensor in = wrap(input), adjOut = wrap(gradOutput), adjIn = wrap(adjInput);
-            const int rc = qmlp_network_adjoint_overwriting(net->handle_, &in, &adjOut, flags, overwrite, &adjIn, tmpForward.data_ptr(),
-                                                            tmpAdjoint.data_ptr(), currentStream());
+            const int rc = qmlp_network_adjoint_for(net->handle_, &in, &adjOut, flags, overwrite, &adjIn, tmpForward.data_ptr(), contents,
+                                                    tmpAdjoint.data_ptr(), currentStream());
             // no dangling gradient bindings, whatever happened
             qmlp_network_set_parameter(net->handle_, nullptr, QMLP_GRADIENTS);
             for (size_t i = 0; i < adjEncodings.size(); ++i)

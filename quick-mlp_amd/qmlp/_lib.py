@@ -75,11 +75,13 @@ _SIGNATURES = {
     "qmlp_network_inference_noalloc": [_vp, _TD, _TD, _vp],
     "qmlp_network_forward_memory": [_vp, _ci, _ci, _P(ctypes.c_size_t)],
     "qmlp_network_forward": [_vp, _TD, _TD, _vp, _vp],
+    "qmlp_network_forward_for": [_vp, _TD, _TD, _ci, _vp, _pi, _vp],
     "qmlp_network_zero_gradients": [_vp],
     "qmlp_network_adjoint_memory": [_vp, _ci, _ci, _P(ctypes.c_size_t)],
     "qmlp_network_adjoint": [_vp, _TD, _TD, _ci, _TD, _vp, _vp, _vp],
     "qmlp_network_overwritable_gradients": [_vp, _ci, _ci, _vp, _pi],
     "qmlp_network_adjoint_overwriting": [_vp, _TD, _TD, _ci, _ci, _TD, _vp, _vp, _vp],
+    "qmlp_network_adjoint_for": [_vp, _TD, _TD, _ci, _ci, _TD, _vp, _ci, _vp, _vp],
     "qmlp_network_clear_cached_kernels": [_vp],
     "qmlp_network_precompile": [_vp, _ci],
     "qmlp_network_prepare": [_vp, _ci, _ci],

@@ -395,22 +395,31 @@ class Network:
             check(lib.qmlp_network_inference_noalloc(self._handle, desc(input), desc(output), current_stream(input.device)))
         return output
 
-    def forward_raw(self, input, network_parameters, encoding_parameters=(), flags=7):
-        """forward() of the C ABI without autograd: returns (output, tmp_forward)."""
+    def forward_raw(self, input, network_parameters, encoding_parameters=(), flags=7, contents=False):
+        """forward() of the C ABI without autograd: returns (output, tmp_forward). With contents=True the pass leaves no
+        more in tmp_forward than an adjoint pass with these flags reads, and what it left is the third value returned:
+        the 'contents' of adjoint_raw."""
         _device_of(input)
         output = _create_output(input, self.channels_out())
         nbytes = self.forward_memory(input.shape[0], flags)
         tmp_forward = torch.empty((max(nbytes, 16),), dtype=torch.uint8, device=input.device)
+        left = ctypes.c_int()
         with self._mutex:
             self._set_network_parameters(network_parameters, list(encoding_parameters))
-            check(lib.qmlp_network_forward(self._handle, desc(input), desc(output),
-                                           ctypes.c_void_p(tmp_forward.data_ptr()), current_stream(input.device)))
-        return output, tmp_forward
+            if contents:
+                check(lib.qmlp_network_forward_for(self._handle, desc(input), desc(output), int(flags),
+                                                   ctypes.c_void_p(tmp_forward.data_ptr()), ctypes.byref(left),
+                                                   current_stream(input.device)))
+            else:
+                check(lib.qmlp_network_forward(self._handle, desc(input), desc(output),
+                                               ctypes.c_void_p(tmp_forward.data_ptr()), current_stream(input.device)))
+        return (output, tmp_forward, left.value) if contents else (output, tmp_forward)
 
     def adjoint_raw(self, input, adj_output, flags, tmp_forward, network_parameters, encoding_parameters=(),
-                    grad_network=None, grad_encodings=None, adj_input=None):
+                    grad_network=None, grad_encodings=None, adj_input=None, contents=None):
         """adjoint() of the C ABI without autograd. Gradient tensors that are passed in are
-        accumulated into (+=); missing ones are created zero-filled.
+        accumulated into (+=); missing ones are created zero-filled. contents: what forward_raw
+        reported of tmp_forward, if it was asked to.
         Returns (adj_input, grad_network, grad_encodings)."""
         encoding_parameters = list(encoding_parameters)
         if flags & GRADIENTS_INPUT and adj_input is None:
@@ -435,10 +444,15 @@ class Network:
                 for i, g in enumerate(grad_encodings):
                     if g is not None:
                         self.encoding(i).set_parameter(g, gradients=True)
-            check(lib.qmlp_network_adjoint(self._handle, desc(input), desc(adj_output), int(flags),
-                                           desc(adj_input if flags & GRADIENTS_INPUT else None),
-                                           ctypes.c_void_p(tmp_forward.data_ptr()),
-                                           ctypes.c_void_p(tmp_adjoint.data_ptr()), current_stream(input.device)))
+            adj = desc(adj_input if flags & GRADIENTS_INPUT else None)
+            if contents is None:
+                check(lib.qmlp_network_adjoint(self._handle, desc(input), desc(adj_output), int(flags), adj,
+                                               ctypes.c_void_p(tmp_forward.data_ptr()),
+                                               ctypes.c_void_p(tmp_adjoint.data_ptr()), current_stream(input.device)))
+            else:
+                check(lib.qmlp_network_adjoint_for(self._handle, desc(input), desc(adj_output), int(flags), 0, adj,
+                                                   ctypes.c_void_p(tmp_forward.data_ptr()), int(contents),
+                                                   ctypes.c_void_p(tmp_adjoint.data_ptr()), current_stream(input.device)))
             check(lib.qmlp_network_set_parameter(self._handle, None, QMLP_GRADIENTS))
             for i, g in enumerate(grad_encodings):
                 if g is not None and self.encoding(i).has_parameters():
