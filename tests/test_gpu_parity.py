@@ -550,13 +550,19 @@ def test_grid_gradients_summed_by_slices_match_the_atomic_scatter_and_the_oracle
             got = {mode: c.gpu_train(X, adj, flags) for mode, c in cases.items() if mode < 2 or flags & FLAG_INPUT}
             a, b = got[0]["table_grads"][1], got[1]["table_grads"][1]
             scale = max(1.0, float(np.abs(a).max()))
-            assert np.allclose(a / scale, b / scale, rtol=1e-4, atol=2e-6), "N=%d flags=%d: %g" % (N, flags, np.abs(a - b).max())
+            # A clustered batch adds up to N floats to one entry, in any order: each addition rounds with a standard
+            # deviation of at most 2^-24 / sqrt(3) of the running sum, which is a random walk (adjoints of both signs) that
+            # ends within the largest sum of the table. Two such sums differ by sqrt(2 N / 3) 2^-24 of that; six of these
+            # (replayed on the CPU with 70 001 random terms: 1.3e-5 by this formula, 6.7e-6 in the median of the largest of 24
+            # entries and 1.4e-5 at most in 60 repetitions; 2e-6 is passed in one of twelve).
+            order = 6 * np.sqrt(2 * N / 3) * 2.0 ** -24 if clustered else 2e-6
+            assert np.allclose(a / scale, b / scale, rtol=1e-4, atol=order), "N=%d flags=%d: %g" % (N, flags, np.abs(a - b).max())
             if flags & FLAG_WEIGHTS:
                 assert np.array_equal(got[0]["grads"], got[1]["grads"]) and np.array_equal(got[0]["grads"], got[2]["grads"])
                 # gathered a second time, in the same order of operations: the bits of the atomic path
                 assert np.array_equal(got[0]["adj_x"], got[2]["adj_x"])
                 # (fixed-point sums, but entries next to a slice boundary and coarse levels also receive float atomics)
-                assert np.allclose(got[1]["table_grads"][1] / scale, got[2]["table_grads"][1] / scale, rtol=1e-4, atol=2e-6)
+                assert np.allclose(got[1]["table_grads"][1] / scale, got[2]["table_grads"][1] / scale, rtol=1e-4, atol=order)
                 # from the stored derivatives (kept in the precision of the table: relative 2^-11 each for half)
                 sx = float(np.abs(got[0]["adj_x"]).max())
                 assert np.allclose(got[1]["adj_x"] / sx, got[0]["adj_x"] / sx, rtol=2e-3, atol=1e-3 if precision == "half" else 1e-5)
