@@ -104,6 +104,9 @@ public:
      */
     std::optional<KernelFunction> getKernel(const std::string& kernelName, const std::string& source, int flags,
                                             const std::vector<std::string>& offlineOptions = {});
+    /** getKernel() for several functions of 'source' in one code object; empty where that returns an empty optional. */
+    std::vector<KernelFunction> getKernels(const std::vector<std::string>& kernelNames, const std::string& source, int flags,
+                                           const std::vector<std::string>& offlineOptions = {});
 
     /**
      * True if kernels can be compiled by the offline compiler of the installed ROCm (`<ROCM_PATH>/bin/hipcc`, run as

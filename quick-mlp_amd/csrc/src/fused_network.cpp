@@ -1902,6 +1902,9 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
         ak.reduce.blockSize = 1024;
         ak.reduce.fun = kl->getKernel("qmlp::kernel::WeightUpdateReduceKernel", source, loaderFlags(compileOnly)).value();
         ak.layers.resize(layers_.size());
+        // the kernel of all layers shares the code object of the last one's: no look-up of its own when a network is built
+        ak.updatesAllLayers = std::count(ak.fusedLayers.begin(), ak.fusedLayers.end(), false) >= 2;
+        const size_t last = std::find(ak.fusedLayers.rbegin(), ak.fusedLayers.rend(), false).base() - ak.fusedLayers.begin();
         for (size_t layer = 0; layer < ak.layers.size(); ++layer) {
             if (ak.fusedLayers[layer]) continue;   // summed by the adjoint kernel
             auto& wk = ak.layers[layer];
@@ -1913,7 +1916,15 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
                 throw configuration_error("Layer %d too large for block-wise weight update!", static_cast<int>(layer));
             ak.updateWorkgroups += wk.numChunks;
             ak.allLayers.sharedMemorySize = std::max(ak.allLayers.sharedMemorySize, wk.kernel.sharedMemorySize);
-            wk.kernel.fun = kl->getKernel(name, source, loaderFlags(compileOnly)).value();
+            if (ak.updatesAllLayers && layer + 1 == last) {
+                auto functions = kl->getKernels({name, "qmlp::kernel::WeightUpdateLayersKernel"}, weightUpdateSource(blockSize, &ak.fusedLayers),
+                                                loaderFlags(compileOnly));
+                ak.allLayers.blockSize = blockSize;
+                wk.kernel.fun = functions.at(0);
+                ak.allLayers.fun = functions.at(1);
+            } else {
+                wk.kernel.fun = kl->getKernel(name, source, loaderFlags(compileOnly)).value();
+            }
             if (!compileOnly) {
                 wk.kernel.fullGrid = wk.kernel.fun.fullGridSize(blockSize, wk.kernel.sharedMemorySize);
                 logger->debug("weight update kernel layer %d: %s, LDS %d bytes, %d VGPRs, full grid %d",
@@ -1921,12 +1932,6 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
                               wk.kernel.fun.numVgprs(), wk.kernel.fullGrid);
             }
         }
-    }
-    if (hasNetworkGradients && std::count(ak.fusedLayers.begin(), ak.fusedLayers.end(), false) >= 2) {
-        ak.allLayers.blockSize = weightUpdateBlockSize();
-        ak.allLayers.fun = kl->getKernel("qmlp::kernel::WeightUpdateLayersKernel", weightUpdateSource(ak.allLayers.blockSize, &ak.fusedLayers),
-                                         loaderFlags(compileOnly)).value();
-        ak.updatesAllLayers = true;
     }
     if (!compileOnly) backwardKernel_[flags][variant][mode] = std::move(ak);
 }

@@ -394,6 +394,17 @@ void KernelLoader::saveToDisk(const std::string& key, const Entry& entry)
 std::optional<KernelFunction> KernelLoader::getKernel(const std::string& kernelName, const std::string& source,
                                                       int flags, const std::vector<std::string>& offlineOptions)
 {
+    auto functions = getKernels({kernelName}, source, flags, offlineOptions);
+    if (functions.empty()) return {};
+    return std::move(functions.front());
+}
+
+std::vector<KernelFunction> KernelLoader::getKernels(const std::vector<std::string>& kernelNames, const std::string& source,
+                                                     int flags, const std::vector<std::string>& offlineOptions)
+{
+    // (of the key: one name stands for itself)
+    std::string kernelName;
+    for (const auto& name : kernelNames) kernelName += (kernelName.empty() ? "" : ", ") + name;
     std::lock_guard<std::mutex> lock(mutex_);
     const bool debug = (flags & CompileDebugMode) != 0;
     const bool throwOnError = (flags & CompileThrowOnError) != 0;
@@ -415,7 +426,7 @@ std::optional<KernelFunction> KernelLoader::getKernel(const std::string& kernelN
     }
 
     // (part of the key, not of the command line: a cache filled by one compiler is not taken for the other's)
-    const bool offline = (flags & CompileOffline) != 0 && hasOfflineCompiler() && kernelName.find('<') == std::string::npos;
+    const bool offline = (flags & CompileOffline) != 0 && hasOfflineCompiler() && kernelNames.size() == 1 && kernelName.find('<') == std::string::npos;
     std::vector<std::string> keyOptions = options;
     if (offline) {
         keyOptions.push_back("compiler: " + offlineCompiler().id);
@@ -462,11 +473,12 @@ std::optional<KernelFunction> KernelLoader::getKernel(const std::string& kernelN
                 for (const auto& n : headerNames_) hn.push_back(n.c_str());
                 for (const auto& c : headerContents_) hc.push_back(c.c_str());
                 for (const auto& o : options) opts.push_back(o.c_str());
-                const char* exprs[] = {kernelName.c_str()};
+                std::vector<const char*> exprs;
+                for (const auto& name : kernelNames) exprs.push_back(name.c_str());
                 qmlp_hip_module m = nullptr;
                 char* log = nullptr;
                 int rc = qmlp_hip_module_compile(source.c_str(), "qmlp_generated.hip", hn.data(), hc.data(),
-                                                 static_cast<int>(hn.size()), exprs, 1, opts.data(),
+                                                 static_cast<int>(hn.size()), exprs.data(), static_cast<int>(exprs.size()), opts.data(),
                                                  static_cast<int>(opts.size()), std::getenv("QMLP_OFFLOAD_ARCH"),
                                                  &m, &log);
                 std::string logText = log ? log : "";
@@ -479,24 +491,30 @@ std::optional<KernelFunction> KernelLoader::getKernel(const std::string& kernelN
                 if (!logText.empty()) logger_->debug("compiler log of %s:\n%s", kernelName.c_str(), logText.c_str());
                 ++numCompilations_;
                 entry.module = std::shared_ptr<qmlp_hip_module_s>(m, ModuleDeleter());
-                const char* lowered = nullptr;
-                QMLP_HIP_CALL(qmlp_hip_module_lowered_name(m, kernelName.c_str(), &lowered));
-                entry.lowered[kernelName] = lowered;
+                for (const auto& name : kernelNames) {
+                    const char* lowered = nullptr;
+                    QMLP_HIP_CALL(qmlp_hip_module_lowered_name(m, name.c_str(), &lowered));
+                    entry.lowered[name] = lowered;
+                }
                 if (!fallback) saveToDisk(key, entry);
                 }
             }
             it = modules_.emplace(key, std::move(entry)).first;
         }
-        KernelFunction fun;
-        fun.name_ = kernelName;
-        if (compileOnly) return fun;
-        auto lit = it->second.lowered.find(kernelName);
-        if (lit == it->second.lowered.end()) throw hip_error("cached module lacks the kernel " + kernelName);
-        qmlp_hip_function f = nullptr;
-        QMLP_HIP_CALL(qmlp_hip_module_get_function(it->second.module.get(), lit->second.c_str(), &f));
-        fun.module_ = it->second.module;
-        fun.function_ = f;
-        return fun;
+        std::vector<KernelFunction> functions;
+        for (const auto& name : kernelNames) {
+            functions.emplace_back();
+            KernelFunction& fun = functions.back();
+            fun.name_ = name;
+            if (compileOnly) continue;
+            auto lit = it->second.lowered.find(name);
+            if (lit == it->second.lowered.end()) throw hip_error("cached module lacks the kernel " + name);
+            qmlp_hip_function f = nullptr;
+            QMLP_HIP_CALL(qmlp_hip_module_get_function(it->second.module.get(), lit->second.c_str(), &f));
+            fun.module_ = it->second.module;
+            fun.function_ = f;
+        }
+        return functions;
     } catch (...) {
         if (throwOnError) throw;
         return {};
