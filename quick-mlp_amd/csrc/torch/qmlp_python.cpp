@@ -9,6 +9,7 @@
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <ATen/FuncTorchTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include "qmlp_capi.h"
@@ -140,6 +141,20 @@ at::Tensor createOutput(const at::Tensor& input, int channels)
     return at::empty({input.size(0), channels}, input.options().requires_grad(false));
 }
 
+/**
+ * The nodes below know reverse mode only, and calls below the dispatcher look at the memory of a tensor and at nothing else:
+ * transforms of torch.func and tensors with a tangent are refused, as torch refuses them for functions without rules for them.
+ */
+void refuseOtherModes(at::TensorList tensors)
+{
+    if (const auto& functorch = at::functorch::functorchTLSAccessor()) functorch->checkSupportsCppAutogradFunction();
+    for (const auto& t : tensors) {
+        if (!t.defined() || !t._fw_grad(0).defined()) continue;
+        PyErr_SetString(PyExc_NotImplementedError, "forward-mode AD is not implemented for networks and encodings");
+        throw py::error_already_set();
+    }
+}
+
 at::Tensor inference(const Network_ptr& net, const at::Tensor& input, const at::Tensor& parameters, const std::vector<at::Tensor>& tables)
 {
     try {
@@ -256,6 +271,8 @@ at::Tensor forward(const Network_ptr& net, const at::Tensor& input, const at::Te
     std::vector<at::Tensor> positions(n);   // of encodings without parameters: undefined
     for (size_t i = 0; i < std::min(n, tables.size()); ++i)
         if (net->encodings[i].hasParameters) positions[i] = tables[i];
+    refuseOtherModes({input, parameters});
+    refuseOtherModes(positions);
     auto output = createOutput(input, net->channelsOut);
     at::Tensor p16, memory;
     int contents = 0;
@@ -382,6 +399,7 @@ struct EncodingBackward : torch::autograd::Node
 
 at::Tensor encodeForward(const Encoding_ptr& enc, const at::Tensor& input, const at::Tensor& parameter)
 {
+    refuseOtherModes({input, parameter});
     int flags = 0;
     if (at::GradMode::is_enabled()) {
         if (input.requires_grad()) flags |= QMLP_ENCODING_INPUT_GRADIENTS;

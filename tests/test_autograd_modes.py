@@ -1,0 +1,45 @@
+"""Networks and encodings under what PyTorch offers beside plain reverse mode: refused or recorded, as for any function without
+rules of its own.
+rules of its own."""
+
+import pytest
+import torch
+from torch.autograd import forward_ad
+
+import qmlp
+from helpers import identity_cfg, warm_cache
+
+pytestmark = pytest.mark.gpu
+
+GRID = {"id": "HashGrid", "start_in": 0, "n_in": 3, "n_levels": 4, "n_features_per_level": 2, "log2_hashmap_size": 10, "min_resolution": 4,
+        "max_resolution": 64, "combination_mode": "concat", "bounding_box_min": [0.0] * 3, "bounding_box_size": [1.0] * 3,
+        "parameter_precision": "float"}
+NETWORK = dict(identity_cfg(3, [32, 2], ["relu", "identity"], [True, False]), encodings=[GRID, {"id": "Identity", "start_in": 0, "n_in": 3}])
+
+
+@pytest.fixture
+def modules():
+    warm_cache(NETWORK)
+    network = qmlp.FusedNetwork(json.dumps(NETWORK), weight_dtype=torch.float32)
+    encoding = qmlp.FusedEncoding(json.dumps(GRID))
+    table = torch.nn.Parameter(encoding.create_parameter_tensor())
+    with torch.no_grad():
+        network.encoding_parameters[0].copy_(table)
+    return network, encoding, table
+
+
+def test_tangents_and_function_transforms_are_refused(modules):
+    network, encoding, table = modules
+    x = torch.rand(100, 3, device="cuda")
+    calls = [network, lambda v: encoding(v, table), lambda v: encoding(v, table.detach())]
+    for call in calls:
+        with forward_ad.dual_level():
+            with pytest.raises(NotImplementedError):
+                call(forward_ad.make_dual(x, torch.ones_like(x)))
+            call(x)
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(call)(x[None])
+        with pytest.raises(RuntimeError):
+            torch.func.grad(lambda v: call(v).sum())(x)
+    with forward_ad.dual_level(), pytest.raises(NotImplementedError):
+        encoding(x, forward_ad.make_dual(table.detach(), torch.ones_like(table)))
