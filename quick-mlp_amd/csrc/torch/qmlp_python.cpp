@@ -9,6 +9,7 @@
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/Exceptions.h>
 #include <ATen/FuncTorchTLS.h>
 #include <c10/hip/HIPStream.h>
 
@@ -34,12 +35,37 @@ void check(int rc)
 {
     if (rc != 0) throw Failure{rc, qmlp_last_error()};
 }
+void setError(const Failure& f)
+{
+    py::object cls = py::module_::import("qmlp._lib").attr("QmlpError");
+    PyErr_SetObject(cls.ptr(), cls(f.code, f.message).ptr());
+}
 [[noreturn]] void raise(const Failure& f)
 {
     py::gil_scoped_acquire gil;
-    py::object cls = py::module_::import("qmlp._lib").attr("QmlpError");
-    PyErr_SetObject(cls.ptr(), cls(f.code, f.message).ptr());
+    setError(f);
     throw py::error_already_set();
+}
+/** The exception in flight out of a backward pass: in the form in which the threads of the autograd engine hand on exceptions of Python. */
+[[noreturn]] void raiseFromBackward()
+{
+    auto persist = [] {
+        python_error e;
+        e.persist();
+        throw e;
+    };
+    try {
+        throw;
+    } catch (const Failure& f) {
+        py::gil_scoped_acquire gil;
+        setError(f);
+        persist();
+    } catch (const py::builtin_exception& e) {
+        py::gil_scoped_acquire gil;
+        e.set_error();
+        persist();
+    }
+    throw std::logic_error("unreachable");
 }
 
 qmlp_tensor wrap(const at::Tensor& t)
@@ -214,12 +240,12 @@ struct FusedBackward : torch::autograd::Node
             // well, which is dropped below (bind_network.cpp:277-290)
             for (size_t i = 0; i < n; ++i)
                 if (net->encodings[i].hasParameters) adjTables[i] = at::zeros(unpacked[i].sizes(), unpacked[i].options().dtype(at::kFloat));
-        const auto wrappedTables = wrapAll(*net, unpacked);
-        const qmlp_tensor p = wrap(parameters), in = wrap(x), adjOut = wrap(gradOutput);
-        std::vector<qmlp_tensor> adjEnc(n);
-        for (size_t i = 0; i < n; ++i) adjEnc[i] = wrap(adjTables[i]);
         void* stream = currentStream(x);
         try {
+            const auto wrappedTables = wrapAll(*net, unpacked);
+            const qmlp_tensor p = wrap(parameters), in = wrap(x), adjOut = wrap(gradOutput);
+            std::vector<qmlp_tensor> adjEnc(n);
+            for (size_t i = 0; i < n; ++i) adjEnc[i] = wrap(adjTables[i]);
             std::lock_guard<std::mutex> lock(net->mutex);
             size_t bytes = 0;
             check(qmlp_network_adjoint_memory(net->handle, in.sizes[0], flags, &bytes));
@@ -234,19 +260,24 @@ struct FusedBackward : torch::autograd::Node
                 adjNetwork = overwrite & QMLP_GRADIENTS_NETWORK_WEIGHTS ? at::empty(parameters.sizes(), options) : at::zeros(parameters.sizes(), options);
             }
             const qmlp_tensor adjIn = wrap(adjInput), adjNet = wrap(adjNetwork);
+            struct Unbind   // no dangling gradient bindings, whatever happens
+            {
+                Network& net;
+                bool tables;
+                ~Unbind()
+                {
+                    qmlp_network_set_parameter(net.handle, nullptr, QMLP_GRADIENTS);
+                    for (const auto& e : net.encodings)
+                        if (tables && e.hasParameters) qmlp_encoding_set_parameter(e.handle, nullptr, QMLP_GRADIENTS);
+                }
+            } unbind{*net, (flags & QMLP_GRADIENTS_INPUT_ENCODINGS) != 0};
             if (adjNetwork.defined()) check(qmlp_network_set_parameter(net->handle, &adjNet, QMLP_GRADIENTS));
             for (size_t i = 0; i < n; ++i)
                 if (adjTables[i].defined()) check(qmlp_encoding_set_parameter(net->encodings[i].handle, &adjEnc[i], QMLP_GRADIENTS));
-            const int rc = qmlp_network_adjoint_for(net->handle, &in, &adjOut, flags, overwrite, &adjIn, forwardMemory.data_ptr(), contents,
-                                                    scratch.data_ptr(), stream);
-            const std::string message = rc != 0 ? qmlp_last_error() : "";
-            // no dangling gradient bindings, whatever happened
-            qmlp_network_set_parameter(net->handle, nullptr, QMLP_GRADIENTS);
-            for (size_t i = 0; i < n; ++i)
-                if (adjTables[i].defined()) qmlp_encoding_set_parameter(net->encodings[i].handle, nullptr, QMLP_GRADIENTS);
-            if (rc != 0) throw Failure{rc, message};
-        } catch (const Failure& f) {
-            throw std::runtime_error(f.message);
+            check(qmlp_network_adjoint_for(net->handle, &in, &adjOut, flags, overwrite, &adjIn, forwardMemory.data_ptr(), contents,
+                                           scratch.data_ptr(), stream));
+        } catch (...) {
+            raiseFromBackward();
         }
         if (adjInput.defined() && task_should_compute_output(0)) grads[0] = adjInput;
         if (adjNetwork.defined() && task_should_compute_output(1)) grads[1] = adjNetwork.to(parameterType);
@@ -390,8 +421,8 @@ struct EncodingBackward : torch::autograd::Node
             auto [adjInput, adjParameter] = encodeAdjoint(*enc, x, table, gradOutputs[0].contiguous(), flags);
             if (adjInput.defined() && task_should_compute_output(0)) grads[0] = adjInput;
             if (adjParameter.defined() && task_should_compute_output(1)) grads[1] = adjParameter.to(table.scalar_type());
-        } catch (const Failure& f) {
-            throw std::runtime_error(f.message);
+        } catch (...) {
+            raiseFromBackward();
         }
         return grads;
     }
@@ -427,8 +458,7 @@ PYBIND11_MODULE(_native, m)
         try {
             if (p) std::rethrow_exception(p);
         } catch (const Failure& f) {
-            py::object cls = py::module_::import("qmlp._lib").attr("QmlpError");
-            PyErr_SetObject(cls.ptr(), cls(f.code, f.message).ptr());
+            setError(f);
         }
     });
     py::class_<Network, Network_ptr>(m, "Network")

@@ -1,6 +1,6 @@
 """Networks and encodings under what PyTorch offers beside plain reverse mode: refused or recorded, as for any function without
-rules of its own.
 rules of its own."""
+import json
 
 import pytest
 import torch
@@ -43,3 +43,16 @@ def test_tangents_and_function_transforms_are_refused(modules):
             torch.func.grad(lambda v: call(v).sum())(x)
     with forward_ad.dual_level(), pytest.raises(NotImplementedError):
         encoding(x, forward_ad.make_dual(table.detach(), torch.ones_like(table)))
+
+
+def test_errors_of_a_backward_pass_are_those_of_the_native_library(modules):
+    """Provoked by a hook that hands saved tensors of the wrong shape back: refused before anything is launched."""
+    network, encoding, table = modules
+    x = torch.rand(100, 3, device="cuda", requires_grad=True)
+    for call in (network, lambda v: encoding(v, table)):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t[:, :2] if t.dim() == 2 else t):
+            out = call(x).sum()
+        with pytest.raises(qmlp.QmlpError) as error:
+            out.backward()
+        assert error.value.code != 0
+    call(x).sum().backward()
