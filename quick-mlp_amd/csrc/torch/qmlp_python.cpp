@@ -300,8 +300,11 @@ at::Tensor forward(const Network_ptr& net, const at::Tensor& input, const at::Te
     }
     if (flags == 0) return inference(net, input, parameters, tables);
     std::vector<at::Tensor> positions(n);   // of encodings without parameters: undefined
-    for (size_t i = 0; i < std::min(n, tables.size()); ++i)
-        if (net->encodings[i].hasParameters) positions[i] = tables[i];
+    for (size_t i = 0; i < n; ++i) {
+        if (!net->encodings[i].hasParameters) continue;
+        if (i < tables.size()) positions[i] = tables[i];
+        if (!positions[i].defined()) raise(Failure{2, "encoding " + std::to_string(i) + " has parameters, but none are given"});
+    }
     refuseOtherModes({input, parameters});
     refuseOtherModes(positions);
     auto output = createOutput(input, net->channelsOut);

@@ -254,6 +254,8 @@ class Encoding:
     def forward_with_parameter(self, input, parameter):
         if not self.has_parameters():
             raise RuntimeError("Encoding doesn't have parameters, call the variation of 'forward' without parameters")
+        if parameter is None:
+            raise RuntimeError("Encoding has parameters, but none are given")
         return self._native.forward(input, parameter)
 
     def __getstate__(self):

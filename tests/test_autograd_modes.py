@@ -56,3 +56,16 @@ def test_errors_of_a_backward_pass_are_those_of_the_native_library(modules):
             out.backward()
         assert error.value.code != 0
     call(x).sum().backward()
+
+
+def test_a_differentiable_call_wants_the_parameters_of_every_encoding(modules):
+    """... and does not take those that an earlier call has left bound."""
+    network, encoding, _ = modules
+    x = torch.rand(100, 3, device="cuda", requires_grad=True)
+    table = network.encoding_parameters[0]
+    network._network.forward(x, network.weights, [table, None]).sum().backward()
+    for tables in ([], [None, None]):
+        with pytest.raises(qmlp.QmlpError, match="encoding 0"):
+            network._network.forward(x, network.weights, tables)
+    with pytest.raises(RuntimeError, match="none are given"):
+        encoding._encoding.forward_with_parameter(x, None)
