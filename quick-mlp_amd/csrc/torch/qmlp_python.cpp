@@ -11,6 +11,7 @@
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/Exceptions.h>
 #include <ATen/FuncTorchTLS.h>
+#include <ATen/TracerMode.h>
 #include <c10/hip/HIPStream.h>
 
 #include "qmlp_capi.h"
@@ -202,15 +203,98 @@ at::Tensor inference(const Network_ptr& net, const at::Tensor& input, const at::
     }
 }
 
+/** What a forward pass leaves for its adjoint pass, beside its inputs. */
+struct ForwardPass
+{
+    at::Tensor output, memory;
+    int contents = 0;   // of the memory
+};
+
+/** parameters: in half precision; tables: undefined for encodings without parameters */
+ForwardPass forwardPass(const Network_ptr& net, const at::Tensor& input, const at::Tensor& parameters, const std::vector<at::Tensor>& tables, int flags)
+{
+    ForwardPass pass;
+    pass.output = createOutput(input, net->channelsOut);
+    at::AutoDispatchBelowADInplaceOrView guard;
+    const auto wrappedTables = wrapAll(*net, tables);
+    const qmlp_tensor p = wrap(parameters), in = wrap(input), out = wrap(pass.output);
+    void* stream = currentStream(input);
+    py::gil_scoped_release release;
+    std::lock_guard<std::mutex> lock(net->mutex);
+    size_t bytes = 0;
+    check(qmlp_network_forward_memory(net->handle, in.sizes[0], flags, &bytes));
+    pass.memory = bytesOn(input, bytes);
+    net->bind(p, wrappedTables);
+    check(qmlp_network_forward_for(net->handle, &in, &out, flags, pass.memory.data_ptr(), &pass.contents, stream));
+    return pass;
+}
+
+/** Gradients of the input, the network parameters and the tables, those of parameters in floats; undefined where flags do not ask for them. */
+struct Gradients
+{
+    at::Tensor input, network;
+    std::vector<at::Tensor> tables;
+};
+
+Gradients adjointPass(const Network_ptr& net, const at::Tensor& input, const at::Tensor& parameters, const std::vector<at::Tensor>& tables,
+                      const at::Tensor& memory, int contents, const at::Tensor& adjOutput, int flags)
+{
+    const size_t n = net->encodings.size();
+    // (memory: may have been elsewhere in between, see saved-tensor hooks)
+    TORCH_CHECK(input.is_cuda() && memory.device() == input.device() && memory.is_contiguous(), "saved tensors came back on another device");
+    at::AutoDispatchBelowADInplaceOrView guard;
+    Gradients g;
+    g.tables.resize(n);
+    if (flags & QMLP_GRADIENTS_INPUT_ENCODINGS)
+        // the kernel adds the gradients of every encoding with parameters: a frozen one gets a zero tensor as
+        // well, which the callers drop (bind_network.cpp:277-290)
+        for (size_t i = 0; i < n; ++i)
+            if (net->encodings[i].hasParameters) g.tables[i] = at::zeros(tables.at(i).sizes(), tables[i].options().dtype(at::kFloat));
+    void* stream = currentStream(input);
+    const auto wrappedTables = wrapAll(*net, tables);
+    const qmlp_tensor p = wrap(parameters), in = wrap(input), adjOut = wrap(adjOutput);
+    std::vector<qmlp_tensor> adjEnc(n);
+    for (size_t i = 0; i < n; ++i) adjEnc[i] = wrap(g.tables[i]);
+    std::lock_guard<std::mutex> lock(net->mutex);
+    size_t bytes = 0;
+    check(qmlp_network_adjoint_memory(net->handle, in.sizes[0], flags, &bytes));
+    const at::Tensor scratch = bytesOn(input, bytes);
+    net->bind(p, wrappedTables);
+    // zeroed only where the kernels add to them
+    int overwrite = 0;
+    check(qmlp_network_overwritable_gradients(net->handle, in.sizes[0], flags, nullptr, &overwrite));
+    if (flags & QMLP_GRADIENTS_INPUT) g.input = overwrite & QMLP_GRADIENTS_INPUT ? at::empty_like(input) : at::zeros_like(input);
+    if (flags & QMLP_GRADIENTS_NETWORK_WEIGHTS) {
+        const auto options = parameters.options().dtype(at::kFloat);
+        g.network = overwrite & QMLP_GRADIENTS_NETWORK_WEIGHTS ? at::empty(parameters.sizes(), options) : at::zeros(parameters.sizes(), options);
+    }
+    const qmlp_tensor adjIn = wrap(g.input), adjNet = wrap(g.network);
+    struct Unbind   // no dangling gradient bindings, whatever happens
+    {
+        Network& net;
+        bool tables;
+        ~Unbind()
+        {
+            qmlp_network_set_parameter(net.handle, nullptr, QMLP_GRADIENTS);
+            for (const auto& e : net.encodings)
+                if (tables && e.hasParameters) qmlp_encoding_set_parameter(e.handle, nullptr, QMLP_GRADIENTS);
+        }
+    } unbind{*net, (flags & QMLP_GRADIENTS_INPUT_ENCODINGS) != 0};
+    if (g.network.defined()) check(qmlp_network_set_parameter(net->handle, &adjNet, QMLP_GRADIENTS));
+    for (size_t i = 0; i < n; ++i)
+        if (g.tables[i].defined()) check(qmlp_encoding_set_parameter(net->encodings[i].handle, &adjEnc[i], QMLP_GRADIENTS));
+    check(qmlp_network_adjoint_for(net->handle, &in, &adjOut, flags, overwrite, &adjIn, memory.data_ptr(), contents, scratch.data_ptr(), stream));
+    return g;
+}
+
 /** The backward pass of one forward call: outputs are the gradients of (input, network parameters, tables ...). */
 struct FusedBackward : torch::autograd::Node
 {
     Network_ptr net;
     int flags = 0;
-    SavedVariable input, p16;
+    SavedVariable input, p16, memory;
     std::vector<SavedVariable> tables;
-    SavedVariable memory;   // what the forward pass left for the adjoint pass (may come back at another address: saved-tensor hooks)
-    int contents = 0;       // of it
+    int contents = 0;   // of the memory
     at::ScalarType parameterType = at::kHalf;
 
     std::string name() const override { return "QmlpFusedBackward"; }
@@ -227,65 +311,30 @@ struct FusedBackward : torch::autograd::Node
         const size_t n = net->encodings.size();
         variable_list grads(2 + n);
         if (!gradOutputs[0].defined()) return grads;
-        const at::Tensor x = input.unpack(), parameters = p16.unpack(), forwardMemory = memory.unpack();
-        TORCH_CHECK(x.is_cuda() && forwardMemory.device() == x.device() && forwardMemory.is_contiguous(), "saved tensors came back on another device");
-        std::vector<at::Tensor> unpacked(n), adjTables(n);
+        const at::Tensor x = input.unpack(), parameters = p16.unpack();
+        std::vector<at::Tensor> unpacked(n);
         for (size_t i = 0; i < n; ++i)
             if (net->encodings[i].hasParameters) unpacked[i] = tables[i].unpack();
-        at::AutoDispatchBelowADInplaceOrView guard;
-        const at::Tensor gradOutput = gradOutputs[0].contiguous();
-        at::Tensor adjInput, adjNetwork;
-        if (flags & QMLP_GRADIENTS_INPUT_ENCODINGS)
-            // the kernel adds the gradients of every encoding with parameters: a frozen one gets a zero tensor as
-            // well, which is dropped below (bind_network.cpp:277-290)
-            for (size_t i = 0; i < n; ++i)
-                if (net->encodings[i].hasParameters) adjTables[i] = at::zeros(unpacked[i].sizes(), unpacked[i].options().dtype(at::kFloat));
-        void* stream = currentStream(x);
+        Gradients g;
         try {
-            const auto wrappedTables = wrapAll(*net, unpacked);
-            const qmlp_tensor p = wrap(parameters), in = wrap(x), adjOut = wrap(gradOutput);
-            std::vector<qmlp_tensor> adjEnc(n);
-            for (size_t i = 0; i < n; ++i) adjEnc[i] = wrap(adjTables[i]);
-            std::lock_guard<std::mutex> lock(net->mutex);
-            size_t bytes = 0;
-            check(qmlp_network_adjoint_memory(net->handle, in.sizes[0], flags, &bytes));
-            const at::Tensor scratch = bytesOn(x, bytes);
-            net->bind(p, wrappedTables);
-            // zeroed only where the kernels add to them
-            int overwrite = 0;
-            check(qmlp_network_overwritable_gradients(net->handle, in.sizes[0], flags, nullptr, &overwrite));
-            if (flags & QMLP_GRADIENTS_INPUT) adjInput = overwrite & QMLP_GRADIENTS_INPUT ? at::empty_like(x) : at::zeros_like(x);
-            if (flags & QMLP_GRADIENTS_NETWORK_WEIGHTS) {
-                const auto options = parameters.options().dtype(at::kFloat);
-                adjNetwork = overwrite & QMLP_GRADIENTS_NETWORK_WEIGHTS ? at::empty(parameters.sizes(), options) : at::zeros(parameters.sizes(), options);
-            }
-            const qmlp_tensor adjIn = wrap(adjInput), adjNet = wrap(adjNetwork);
-            struct Unbind   // no dangling gradient bindings, whatever happens
-            {
-                Network& net;
-                bool tables;
-                ~Unbind()
-                {
-                    qmlp_network_set_parameter(net.handle, nullptr, QMLP_GRADIENTS);
-                    for (const auto& e : net.encodings)
-                        if (tables && e.hasParameters) qmlp_encoding_set_parameter(e.handle, nullptr, QMLP_GRADIENTS);
-                }
-            } unbind{*net, (flags & QMLP_GRADIENTS_INPUT_ENCODINGS) != 0};
-            if (adjNetwork.defined()) check(qmlp_network_set_parameter(net->handle, &adjNet, QMLP_GRADIENTS));
-            for (size_t i = 0; i < n; ++i)
-                if (adjTables[i].defined()) check(qmlp_encoding_set_parameter(net->encodings[i].handle, &adjEnc[i], QMLP_GRADIENTS));
-            check(qmlp_network_adjoint_for(net->handle, &in, &adjOut, flags, overwrite, &adjIn, forwardMemory.data_ptr(), contents,
-                                           scratch.data_ptr(), stream));
+            g = adjointPass(net, x, parameters, unpacked, memory.unpack(), contents, gradOutputs[0].contiguous(), flags);
         } catch (...) {
             raiseFromBackward();
         }
-        if (adjInput.defined() && task_should_compute_output(0)) grads[0] = adjInput;
-        if (adjNetwork.defined() && task_should_compute_output(1)) grads[1] = adjNetwork.to(parameterType);
+        at::AutoDispatchBelowADInplaceOrView guard;
+        if (g.input.defined() && task_should_compute_output(0)) grads[0] = g.input;
+        if (g.network.defined() && task_should_compute_output(1)) grads[1] = g.network.to(parameterType);
         for (size_t i = 0; i < n; ++i)
-            if (adjTables[i].defined() && task_should_compute_output(2 + i)) grads[2 + i] = adjTables[i].to(unpacked[i].scalar_type());
+            if (g.tables[i].defined() && task_should_compute_output(2 + i)) grads[2 + i] = g.tables[i].to(unpacked[i].scalar_type());
         return grads;
     }
 };
+
+at::Tensor halves(const at::Tensor& parameters)
+{
+    at::AutoDispatchBelowADInplaceOrView guard;
+    return parameters.scalar_type() == at::kHalf ? parameters : parameters.to(at::kHalf);
+}
 
 /** Differentiable forward pass; gradients flow to every argument that requires them. */
 at::Tensor forward(const Network_ptr& net, const at::Tensor& input, const at::Tensor& parameters, const std::vector<at::Tensor>& tables)
@@ -307,22 +356,10 @@ at::Tensor forward(const Network_ptr& net, const at::Tensor& input, const at::Te
     }
     refuseOtherModes({input, parameters});
     refuseOtherModes(positions);
-    auto output = createOutput(input, net->channelsOut);
-    at::Tensor p16, memory;
-    int contents = 0;
+    const at::Tensor p16 = halves(parameters);
+    ForwardPass pass;
     try {
-        at::AutoDispatchBelowADInplaceOrView guard;
-        p16 = parameters.scalar_type() == at::kHalf ? parameters : parameters.to(at::kHalf);
-        const auto wrappedTables = wrapAll(*net, positions);
-        const qmlp_tensor p = wrap(p16), in = wrap(input), out = wrap(output);
-        void* stream = currentStream(input);
-        py::gil_scoped_release release;
-        std::lock_guard<std::mutex> lock(net->mutex);
-        size_t bytes = 0;
-        check(qmlp_network_forward_memory(net->handle, in.sizes[0], flags, &bytes));
-        memory = bytesOn(input, bytes);
-        net->bind(p, wrappedTables);
-        check(qmlp_network_forward_for(net->handle, &in, &out, flags, memory.data_ptr(), &contents, stream));
+        pass = forwardPass(net, input, p16, positions, flags);
     } catch (const Failure& f) {
         raise(f);
     }
@@ -334,11 +371,11 @@ at::Tensor forward(const Network_ptr& net, const at::Tensor& input, const at::Te
     node->p16 = SavedVariable(p16, false);
     node->tables.reserve(n);
     for (const auto& t : positions) node->tables.emplace_back(t, false);
-    node->memory = SavedVariable(memory, false);
-    node->contents = contents;
+    node->memory = SavedVariable(pass.memory, false);
+    node->contents = pass.contents;
     node->parameterType = parameters.scalar_type();
-    torch::autograd::set_history(output, node);
-    return output;
+    torch::autograd::set_history(pass.output, node);
+    return pass.output;
 }
 
 // ------------------------------------------------------------------------------------------------ standalone encodings
@@ -452,6 +489,14 @@ at::Tensor encodeForward(const Encoding_ptr& enc, const at::Tensor& input, const
 }
 
 at::Tensor tensorOrNone(const py::object& o) { return o.is_none() ? at::Tensor() : o.cast<at::Tensor>(); }
+py::object noneOr(const at::Tensor& t) { return t.defined() ? py::cast(t) : py::none(); }
+
+/**
+ * While torch.jit.trace records, a call goes through the function of the Python package that it can record: of what is done
+ * here it would see the allocation of the output and nothing else.
+ */
+bool recording() { return at::tracer::impl::is_dispatch_enabled(); }
+py::object recorded(const char* function) { return py::module_::import("qmlp.classes").attr(function).attr("apply"); }
 
 } // namespace
 
@@ -476,8 +521,33 @@ PYBIND11_MODULE(_native, m)
              "Binds inference parameters (with the lock held).")
         .def("inference", [](const Network_ptr& net, const at::Tensor& input, const at::Tensor& parameters,
                              const py::list& tables) { return inference(net, input, parameters, tensorsOf(tables)); })
-        .def("forward", [](const Network_ptr& net, const at::Tensor& input, const at::Tensor& parameters,
-                           const py::list& tables) { return forward(net, input, parameters, tensorsOf(tables)); });
+        .def("forward", [](const Network_ptr& net, const at::Tensor& input, const at::Tensor& parameters, const py::list& tables) {
+            if (!recording()) return forward(net, input, parameters, tensorsOf(tables));
+            py::list positions;
+            for (size_t i = 0; i < net->encodings.size(); ++i)
+                positions.append(net->encodings[i].hasParameters && i < tables.size() ? py::object(tables[i]) : py::object(py::none()));
+            return recorded("_RecordedNetwork")(net, input, parameters, *py::tuple(positions)).cast<at::Tensor>();
+        })
+        .def("forward_pass",
+             [](const Network_ptr& net, const at::Tensor& input, const at::Tensor& parameters, const py::list& tables, int flags) {
+                 const auto pass = forwardPass(net, input, parameters, tensorsOf(tables), flags);
+                 return py::make_tuple(pass.output, pass.memory, pass.contents);
+             },
+             "(output, memory, contents) without autograd; parameters: in half precision.")
+        .def("adjoint_pass",
+             [](const Network_ptr& net, const at::Tensor& input, const at::Tensor& parameters, const py::list& tables, const at::Tensor& memory,
+                int contents, const at::Tensor& adjOutput, int flags) {
+                 const auto unwrapped = tensorsOf(tables);
+                 Gradients g;
+                 {
+                     py::gil_scoped_release release;
+                     g = adjointPass(net, input, parameters, unwrapped, memory, contents, adjOutput, flags);
+                 }
+                 py::list adjTables;
+                 for (const auto& t : g.tables) adjTables.append(noneOr(t));
+                 return py::make_tuple(noneOr(g.input), noneOr(g.network), adjTables);
+             },
+             "Gradients (input, parameters, [tables]), those of parameters in floats; None where flags do not ask for them.");
     py::class_<Encoding, Encoding_ptr>(m, "Encoding")
         .def(py::init<uintptr_t, Network_ptr>())   // handle, the network it belongs to (None: it is taken over)
         .def_property_readonly("calls", [](const Encoding_ptr& enc) { return enc->calls.load(); })
@@ -485,6 +555,18 @@ PYBIND11_MODULE(_native, m)
             return encode(enc, input, tensorOrNone(parameter));
         })
         .def("forward", [](const Encoding_ptr& enc, const at::Tensor& input, const py::object& parameter) {
+            if (recording()) return recorded("_RecordedEncoding")(enc, input, parameter).cast<at::Tensor>();
             return encodeForward(enc, input, tensorOrNone(parameter));
-        });
+        })
+        .def("adjoint_pass",
+             [](const Encoding_ptr& enc, const at::Tensor& input, const py::object& parameter, const at::Tensor& adjOutput, int flags) {
+                 const at::Tensor p = tensorOrNone(parameter);
+                 std::pair<at::Tensor, at::Tensor> g;
+                 {
+                     py::gil_scoped_release release;
+                     g = encodeAdjoint(*enc, input, p, adjOutput, flags);
+                 }
+                 return py::make_tuple(noneOr(g.first), noneOr(g.second));
+             },
+             "Gradients (input, parameter), the latter in floats; None where flags do not ask for them.");
 }

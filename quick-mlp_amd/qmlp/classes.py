@@ -110,6 +110,26 @@ class Activation:
 
 
 # ---------------------------------------------------------------------------- encoding
+class _RecordedEncoding(torch.autograd.Function):
+    """A call of an encoding while torch.jit.trace records: what it records, and plays later, is a call of this function.
+    Everywhere else the autograd node in C++ does the same with less work on the host."""
+
+    @staticmethod
+    def forward(ctx, native, input, parameter):
+        ctx.native = native
+        ctx.flags = (1 if ctx.needs_input_grad[1] else 0) | (2 if ctx.needs_input_grad[2] else 0)
+        ctx.save_for_backward(input, parameter)
+        return native.inference(input, parameter)
+
+    @staticmethod
+    def backward(ctx, grad_output):
+        input, parameter = ctx.saved_tensors
+        if ctx.flags == 0:
+            return None, None, None
+        adj_input, adj_parameter = ctx.native.adjoint_pass(input, parameter, grad_output.contiguous(), ctx.flags)
+        return None, adj_input, None if adj_parameter is None else adj_parameter.to(parameter.dtype)
+
+
 class Encoding:
     """One input encoding, standalone (fp32 in, fp32 out)."""
 
@@ -266,6 +286,32 @@ class Encoding:
 
 
 # ---------------------------------------------------------------------------- network
+class _RecordedNetwork(torch.autograd.Function):
+    """As _RecordedEncoding, for networks; tables: None for encodings without parameters."""
+
+    @staticmethod
+    def forward(ctx, native, input, network_parameters, *tables):
+        needs = ctx.needs_input_grad[1:]
+        flags = ((GRADIENTS_INPUT if needs[0] else 0) | (GRADIENTS_NETWORK_WEIGHTS if needs[1] else 0)
+                 | (GRADIENTS_INPUT_ENCODINGS if any(needs[2:]) else 0))
+        if flags == 0:
+            return native.inference(input, network_parameters, list(tables))
+        half = network_parameters.to(torch.float16)
+        output, memory, contents = native.forward_pass(input, half, list(tables), flags)
+        ctx.native, ctx.flags, ctx.contents, ctx.dtype = native, flags, contents, network_parameters.dtype
+        ctx.save_for_backward(input, half, memory, *tables)
+        return output
+
+    @staticmethod
+    def backward(ctx, grad_output):
+        input, half, memory, *tables = ctx.saved_tensors
+        adj_input, adj_network, adj_tables = ctx.native.adjoint_pass(input, half, tables, memory, ctx.contents,
+                                                                     grad_output.contiguous(), ctx.flags)
+        adj_tables = [g.to(t.dtype) if g is not None and ctx.needs_input_grad[3 + i] else None
+                      for i, (g, t) in enumerate(zip(adj_tables, tables))]
+        return (None, adj_input, None if adj_network is None else adj_network.to(ctx.dtype), *adj_tables)
+
+
 class Network:
     """The fused network of a JSON configuration (bind_network.h:16-95)."""
 

@@ -69,3 +69,22 @@ def test_a_differentiable_call_wants_the_parameters_of_every_encoding(modules):
             network._network.forward(x, network.weights, tables)
     with pytest.raises(RuntimeError, match="none are given"):
         encoding._encoding.forward_with_parameter(x, None)
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.filterwarnings("ignore")   # (of the tracer, about Python values)
+def test_traced_modules_call_the_kernels_when_they_are_played(modules, grad):
+    network, encoding, table = modules
+    x = torch.rand(100, 3, device="cuda")
+    with torch.set_grad_enabled(grad):
+        calls = [(network, torch.jit.trace(network, x, check_trace=False), ()),
+                 (encoding, torch.jit.trace(encoding, (x, table), check_trace=False), (table,))]
+    for module, traced, more in calls:
+        for n in (100, 777):
+            x = torch.rand(n, 3, device="cuda", requires_grad=True)
+            want, got = module(x, *more), traced(x, *more)
+            assert torch.equal(got, want) and float(want.abs().max()) > 0
+            leaves = [x, *more, *(p for p in module.parameters() if p.requires_grad)]
+            g = torch.randn_like(want)
+            for a, b in zip(torch.autograd.grad(got, leaves, g), torch.autograd.grad(want, leaves, g)):
+                torch.testing.assert_close(a, b, rtol=0.0, atol=1e-5 * float(b.abs().max()))
