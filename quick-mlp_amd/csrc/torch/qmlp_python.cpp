@@ -300,6 +300,7 @@ struct FusedBackward : torch::autograd::Node
     std::string name() const override { return "QmlpFusedBackward"; }
     void release_variables() override
     {
+        std::lock_guard<std::mutex> lock(mutex_);   // (as generated nodes do: two threads may run backward on one graph)
         input.reset_data();
         p16.reset_data();
         for (auto& t : tables) t.reset_data();
@@ -308,6 +309,7 @@ struct FusedBackward : torch::autograd::Node
 
     variable_list apply(variable_list&& gradOutputs) override
     {
+        std::lock_guard<std::mutex> lock(mutex_);
         const size_t n = net->encodings.size();
         variable_list grads(2 + n);
         if (!gradOutputs[0].defined()) return grads;
@@ -449,11 +451,13 @@ struct EncodingBackward : torch::autograd::Node
     std::string name() const override { return "QmlpEncodingBackward"; }
     void release_variables() override
     {
+        std::lock_guard<std::mutex> lock(mutex_);   // (as generated nodes do: two threads may run backward on one graph)
         input.reset_data();
         parameter.reset_data();
     }
     variable_list apply(variable_list&& gradOutputs) override
     {
+        std::lock_guard<std::mutex> lock(mutex_);
         variable_list grads(2);
         if (!gradOutputs[0].defined()) return grads;
         const at::Tensor x = input.unpack(), table = parameter.unpack();

@@ -1,6 +1,7 @@
 """Networks and encodings under what PyTorch offers beside plain reverse mode: refused or recorded, as for any function without
 rules of its own."""
 import json
+import threading
 
 import pytest
 import torch
@@ -87,4 +88,27 @@ def test_traced_modules_call_the_kernels_when_they_are_played(modules, grad):
             leaves = [x, *more, *(p for p in module.parameters() if p.requires_grad)]
             g = torch.randn_like(want)
             for a, b in zip(torch.autograd.grad(got, leaves, g), torch.autograd.grad(want, leaves, g)):
+                torch.testing.assert_close(a, b, rtol=0.0, atol=1e-5 * float(b.abs().max()))
+
+
+def test_threads_run_backward_on_one_graph(modules):
+    network, encoding, table = modules
+    x = torch.rand(500, 3, device="cuda", requires_grad=True)
+    leaves = {network: [x, network.weights], encoding: [x, table]}
+    for module, call in ((network, network), (encoding, lambda v: encoding(v, table))):
+        out = call(x)
+        g = torch.randn_like(out)
+        want = torch.autograd.grad(out, leaves[module], g, retain_graph=True)
+        results = []
+
+        def run():
+            for i in range(50):
+                results.append(torch.autograd.grad(out, leaves[module], g, retain_graph=True))
+
+        threads = [threading.Thread(target=run) for _ in range(4)]
+        [t.start() for t in threads]
+        [t.join() for t in threads]
+        assert len(results) == 200
+        for got in results:
+            for a, b in zip(got, want):
                 torch.testing.assert_close(a, b, rtol=0.0, atol=1e-5 * float(b.abs().max()))
