@@ -17,6 +17,7 @@
 #include "qmlp_capi.h"
 
 #include <atomic>
+#include <cstdint>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -85,6 +86,7 @@ qmlp_tensor wrap(const at::Tensor& t)
     d.ndim = static_cast<int32_t>(dim);
     const auto sizes = t.sizes(), strides = t.strides();
     for (int i = 0; i < d.ndim; ++i) {
+        if (sizes[i] > INT32_MAX || strides[i] > INT32_MAX) throw py::value_error("sizes and strides of tensors must fit into 32 bits");
         d.sizes[i] = static_cast<int32_t>(sizes[i]);
         d.strides[i] = static_cast<int32_t>(strides[i]);
     }

@@ -35,6 +35,7 @@ qmlp_tensor wrap(const torch::Tensor& t)
     d.data = t.data_ptr();
     d.ndim = static_cast<int32_t>(t.dim());
     for (int i = 0; i < d.ndim; ++i) {
+        TORCH_CHECK(t.size(i) <= INT32_MAX && t.stride(i) <= INT32_MAX, "sizes and strides of tensors must fit into 32 bits");
         d.sizes[i] = static_cast<int32_t>(t.size(i));
         d.strides[i] = static_cast<int32_t>(t.stride(i));
     }

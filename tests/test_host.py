@@ -659,3 +659,14 @@ def test_staging_rows_beyond_the_lds_are_a_configuration_error():
     src = qmlp.Network(json.dumps(mid)).generated_source("backward", 1)
     m = re.search(r"__launch_bounds__\((\d+)\) [^;]*NetworkKernelBackward", src)
     assert m and int(m.group(1)) % 64 == 0 and 64 <= int(m.group(1)) < 1024
+
+
+def test_strides_beyond_32_bits_are_refused():
+    """The descriptors of the C ABI hold 32 bits: a larger stride is an error and not another stride."""
+    net = qmlp.Network(json.dumps(_two_grid_cfg()))
+    count = net.num_network_parameters()
+    net._native.bind(torch.zeros(count, dtype=torch.float16), [])
+    with pytest.raises(ValueError, match="32 bits"):
+        net._native.bind(torch.zeros(1, dtype=torch.float16).as_strided((1, 1), (1 << 32, 1)), [])
+    with pytest.raises(ValueError, match="32 bits"):
+        net._native.bind(torch.zeros(count, dtype=torch.float16), [torch.zeros(1).as_strided((1,), (1 << 31,))])
