@@ -7,12 +7,30 @@
 #include "kernel_loader.h"
 #include "tensor.h"
 
+#include <atomic>
+#include <mutex>
 #include <optional>
 #include <unordered_map>
 #include <random>
 #include <vector>
 
 QUICKMLP_NAMESPACE_BEGIN
+
+/** A function of the specification that is worked out by the first of the threads that ask for it. */
+template <typename T>
+class Once
+{
+    mutable std::once_flag flag_;
+    mutable std::optional<T> value_;
+
+public:
+    template <typename F>
+    const T& operator()(F&& find) const
+    {
+        std::call_once(flag_, [&] { value_ = find(); });
+        return *value_;
+    }
+};
 
 /**
  * A fully fused coordinate MLP: input encodings, linear layers and activations in one
@@ -283,7 +301,7 @@ private:
     };
     const CooperativeLayout& cooperativeLayout() const;
     CooperativeLayout findCooperativeLayout() const;
-    mutable std::optional<CooperativeLayout> cooperativeLayout_;
+    Once<CooperativeLayout> cooperativeLayout_;
     /** Registers of a lane for what the cooperative kernel holds across a tile: gradient tiles, pre-activations, one layer's work. */
     int cooperativeRegisters(int waves, int registerWeight) const;
     /** Slices of partial weight gradients that a batch leaves room for: one per workgroup of the cooperative kernel. */
@@ -314,7 +332,7 @@ private:
      * intermediates, and here stands which memory holds those of how many points. Only a hint: memory that is not listed
      * (moved, or pushed out of the list) has all that an adjoint pass needs, and the grids are gathered from again.
      */
-    int announcedFlags_ = 0;
+    std::atomic<int> announcedFlags_{0};
     std::unordered_map<const void*, int> derivativeMemories_;
     static constexpr size_t MAX_DERIVATIVE_MEMORIES = 256;
     /** What of the intermediates the backward kernel of this mode reads (ForwardContents). */
@@ -326,8 +344,8 @@ private:
     bool recomputesFor(int numel, int flags) const;
     bool canRecompute(int flags, bool sliceGradients) const;
     /** Whether the wavefronts of a workgroup share the grid levels of a tile in the backward kernel for this batch. */
-    bool sharesBackwardTile(int numel, int flags);
-    int sharesBackwardTile_[ADJOINT_MODE_MAX_COMBINATIONS] = {-1, -1, -1, -1, -1, -1, -1, -1};
+    bool sharesBackwardTile(int numel, int flags) const;
+    Once<bool> sharesBackwardTile_[ADJOINT_MODE_MAX_COMBINATIONS];   // size of the batch aside
     static constexpr int SHARED_BACKWARD_MAX_TILES = 256;   // a workgroup per compute unit
     static constexpr int NUM_SHARED_DIMENSIONS = 6;         // of a grid, at most
     /** LDS of such a kernel, and where in it the derivatives of the levels begin. */
@@ -335,7 +353,7 @@ private:
     int sharedTileLdsOffset(int blockSize) const;
     /** Whether the backward kernel itself adds input gradients of an encoding (those of sliced grids come from the kernels behind it). */
     bool differentiatesEncodings(int flags, bool sliceGradients) const;
-    mutable int recomputesKnown_[ADJOINT_MODE_MAX_COMBINATIONS][2];   // canRecompute(), -1: not known yet
+    Once<bool> recomputes_[ADJOINT_MODE_MAX_COMBINATIONS][2];   // canRecompute()
     /**
      * The mode of the backward kernel of a batch: cooperatesFor(), else recomputesFor(), where that kernel also holds its
      * registers: it is loaded on the first call for these flags (it is the kernel that adjoint() will run), and not used
@@ -527,7 +545,7 @@ private:
     int registerVariantTiles(bool store) const;
     /** Wavefronts per workgroup of the SHARED shape, 0 if the network has none. */
     int sharedTileWaves(bool store) const;
-    mutable int sharedTileWaves_[2] = {-1, -1};
+    Once<int> sharedTileWaves_[2];
     static constexpr int SHARED_TILE_MAX_TILES = 448;   // from about 500 on the other shapes are faster, see kernels/network_forward.h
     /** Workgroup size and tiles per wavefront of a shape of the forward kernel. */
     void forwardShape(bool store, int variant, int& blockSize, int& pointsPerLane) const;
@@ -582,7 +600,8 @@ private:
         std::vector<bool> layers;
         bool all = false, wideRegisters = false;
     };
-    mutable std::optional<FusedLayers> fusedLayers_[ADJOINT_MODE_MAX_COMBINATIONS][2];
+    const FusedLayers& fusedLayers(int adjointFlags, bool sliceGradients) const;
+    Once<FusedLayers> fusedLayers_[ADJOINT_MODE_MAX_COMBINATIONS][2];
     /** LDS halves per wavefront of the backward kernel for the tile that Layer::weightGradient transposes. */
     int fusedWeightUpdateTransposeHalves(bool recompute = false) const;
     /** Channels of adjoint pre-activations that the backward kernel stores per point for the weight-update kernels. */

@@ -219,7 +219,6 @@ FusedNetwork::FusedNetwork(const json& cfg, const std::filesystem::path& parent)
     }
     perEntryForwardMemoryBytes_ = offsetFwd * static_cast<int>(sizeof(half));
 
-    for (auto& perFlags : recomputesKnown_) perFlags[0] = perFlags[1] = -1;
     for (auto& perFlags : recomputeVerdict_)
         for (auto& perSlices : perFlags) std::fill(std::begin(perSlices), std::end(perSlices), -1);
     // behind the intermediates: the position derivatives of the grids whose gradients take the slice kernels
@@ -240,9 +239,7 @@ bool FusedNetwork::recomputesFor(int numel, int flags) const
     if (compileOptions_.recomputeIntermediates == 0 || flags <= 0 || flags >= ADJOINT_MODE_MAX_COMBINATIONS) return false;
     if (!(flags & GRADIENTS_NETWORK_WEIGHTS)) return false;
     const bool sliceGradients = useSliceGradients(numel, flags);
-    int& known = recomputesKnown_[flags][sliceGradients ? 1 : 0];
-    if (known < 0) known = canRecompute(flags, sliceGradients) ? 1 : 0;
-    return known == 1;
+    return recomputes_[flags][sliceGradients ? 1 : 0]([&] { return canRecompute(flags, sliceGradients); });
 }
 
 bool FusedNetwork::canRecompute(int flags, bool sliceGradients) const
@@ -292,9 +289,8 @@ bool FusedNetwork::cooperatesFor(int numel, int flags) const
         // them to kernels of their own is behind at every size (64 x 4 hidden layers, 2048 points: 58 against 29 us). With an
         // encoded input to be stored and read, two wavefronts per SIMD that hold all tiles are as fast as the shared
         // ones (16 -> 32 x 3 -> 16 behind a dense 4-D grid, 2^21 points: 568 us both).
-        bool wideRegisters = false;
-        (void)fusedWeightUpdateLayers(flags, useSliceGradients(numel, flags), &wideRegisters);
-        if (fusedLayers_[flags][useSliceGradients(numel, flags) ? 1 : 0]->all && (numel < COOPERATIVE_MIN_BATCH || (!wideRegisters && !cooperativeReadsInputRows()))) return false;
+        const FusedLayers& fused = fusedLayers(flags, useSliceGradients(numel, flags));
+        if (fused.all && (numel < COOPERATIVE_MIN_BATCH || (!fused.wideRegisters && !cooperativeReadsInputRows()))) return false;
     }
     // grids are left to the kernels of the gradient slices, which also differentiate them with respect to the position
     const bool sliceGradients = useSliceGradients(numel, flags);
@@ -308,8 +304,7 @@ bool FusedNetwork::cooperatesFor(int numel, int flags) const
 
 const FusedNetwork::CooperativeLayout& FusedNetwork::cooperativeLayout() const
 {
-    if (!cooperativeLayout_.has_value()) cooperativeLayout_ = findCooperativeLayout();
-    return cooperativeLayout_.value();
+    return cooperativeLayout_([&] { return findCooperativeLayout(); });
 }
 
 FusedNetwork::CooperativeLayout FusedNetwork::findCooperativeLayout() const
@@ -784,17 +779,22 @@ int FusedNetwork::weightUpdateSlices(int numTiles) const
     return std::max(1, std::min(divUp(numTiles, waves), MAX_WEIGHT_UPDATE_SLICES));
 }
 
+const FusedNetwork::FusedLayers& FusedNetwork::fusedLayers(int adjointFlags, bool sliceGradients) const
+{
+    // (the calls of a training loop ask several times each)
+    return fusedLayers_[adjointFlags & (ADJOINT_MODE_MAX_COMBINATIONS - 1)][sliceGradients ? 1 : 0]([&] {
+        FusedLayers fused;
+        fused.layers = findFusedWeightUpdateLayers(adjointFlags, sliceGradients, &fused.wideRegisters);
+        fused.all = std::find(fused.layers.begin(), fused.layers.end(), false) == fused.layers.end();
+        return fused;
+    });
+}
+
 std::vector<bool> FusedNetwork::fusedWeightUpdateLayers(int adjointFlags, bool sliceGradients, bool* wideRegisters) const
 {
-    // (a function of the specification: worked out once, the calls of a training loop ask several times each)
-    auto& known = fusedLayers_[adjointFlags & (ADJOINT_MODE_MAX_COMBINATIONS - 1)][sliceGradients ? 1 : 0];
-    if (!known.has_value()) {
-        known.emplace();
-        known->layers = findFusedWeightUpdateLayers(adjointFlags, sliceGradients, &known->wideRegisters);
-        known->all = std::find(known->layers.begin(), known->layers.end(), false) == known->layers.end();
-    }
-    if (wideRegisters) *wideRegisters = known->wideRegisters;
-    return known->layers;
+    const FusedLayers& fused = fusedLayers(adjointFlags, sliceGradients);
+    if (wideRegisters) *wideRegisters = fused.wideRegisters;
+    return fused.layers;
 }
 
 std::vector<bool> FusedNetwork::findFusedWeightUpdateLayers(int adjointFlags, bool sliceGradients, bool* wideRegisters) const
@@ -1333,21 +1333,19 @@ int FusedNetwork::sharedTileLdsBytes(int flags, int blockSize) const
     return bytes;
 }
 
-bool FusedNetwork::sharesBackwardTile(int numel, int flags)
+bool FusedNetwork::sharesBackwardTile(int numel, int flags) const
 {
     if (divUp(numel, TILE_POINTS) > SHARED_BACKWARD_MAX_TILES || !(flags & (GRADIENTS_INPUT | GRADIENTS_INPUT_ENCODINGS)) || useSliceGradients(numel, flags)) return false;
-    int& known = sharesBackwardTile_[flags];   // (but for the size fixed by the specification)
-    if (known < 0) {
-        known = 0;
-        for (const auto& e : encodings_) known = known || e->sharedAdjointWaves() > 0 ? 1 : 0;
-        if (trainsSortedBatches() || compileOptions_.overwriteBlocksizeBackward > 0) known = 0;
+    return sharesBackwardTile_[flags]([&] {
+        bool shares = false;
+        for (const auto& e : encodings_) shares = shares || e->sharedAdjointWaves() > 0;
+        if (trainsSortedBatches() || compileOptions_.overwriteBlocksizeBackward > 0) return false;
         for (bool fused : fusedWeightUpdateLayers(flags, false))
-            if (fused) known = 0;   // (as many workgroups as slices of partial sums: a fourth of the tiles)
+            if (fused) return false;   // (as many workgroups as slices of partial sums: a fourth of the tiles)
         for (auto placement : weightPlacement(true))
-            if (placement == WEIGHTS_STREAMED) known = 0;
-        if (sharedTileLdsBytes(flags, forwardBlockSize(compileOptions_.overwriteBlocksizeBackward, true)) > MaxSharedMemoryBytes()) known = 0;
-    }
-    return known != 0;
+            if (placement == WEIGHTS_STREAMED) return false;
+        return shares && sharedTileLdsBytes(flags, forwardBlockSize(compileOptions_.overwriteBlocksizeBackward, true)) <= MaxSharedMemoryBytes();
+    });
 }
 
 std::string FusedNetwork::cooperativeBackwardSource(int flags, bool sliceGradients) const
@@ -1618,19 +1616,17 @@ void FusedNetwork::forwardShape(bool store, int variant, int& blockSize, int& po
 
 int FusedNetwork::sharedTileWaves(bool store) const
 {
-    int& known = sharedTileWaves_[store ? 1 : 0];   // (fixed by the specification, asked on every call)
-    if (known >= 0) return known;
-    known = 0;
-    if ((store ? compileOptions_.overwriteBlocksizeForward : compileOptions_.overwriteBlocksizeInference) > 0) return known;   // a pinned shape
-    std::vector<int> ldsW, ldsB;
-    int streamOffset = -1;
-    const int params = ldsLayout(false, ldsW, ldsB, &streamOffset);
-    if (streamOffset >= 0 || params * static_cast<int>(sizeof(half)) + stageBytesPerWave(false) > MaxSharedMemoryBytes()) return known;
-    int levels = 0;
-    for (const auto& e : encodings_)
-        if (e->levelGroups() > 1) levels = std::max(levels, e->numSweptTables());
-    known = levels >= 8 ? 8 : levels >= 4 ? 4 : 0;
-    return known;
+    return sharedTileWaves_[store ? 1 : 0]([&] {   // (asked on every call)
+        if ((store ? compileOptions_.overwriteBlocksizeForward : compileOptions_.overwriteBlocksizeInference) > 0) return 0;   // a pinned shape
+        std::vector<int> ldsW, ldsB;
+        int streamOffset = -1;
+        const int params = ldsLayout(false, ldsW, ldsB, &streamOffset);
+        if (streamOffset >= 0 || params * static_cast<int>(sizeof(half)) + stageBytesPerWave(false) > MaxSharedMemoryBytes()) return 0;
+        int levels = 0;
+        for (const auto& e : encodings_)
+            if (e->levelGroups() > 1) levels = std::max(levels, e->numSweptTables());
+        return levels >= 8 ? 8 : levels >= 4 ? 4 : 0;
+    });
 }
 
 void FusedNetwork::compileForwardKernel(bool store, int variant, bool compileOnly, bool derivatives, bool inputOnly)

@@ -556,6 +556,9 @@ PYBIND11_MODULE(_native, m)
              "Gradients (input, parameters, [tables]), those of parameters in floats; None where flags do not ask for them.");
     py::class_<Encoding, Encoding_ptr>(m, "Encoding")
         .def(py::init<uintptr_t, Network_ptr>())   // handle, the network it belongs to (None: it is taken over)
+        // as a context manager: the lock of the native encoding, of its network if it belongs to one
+        .def("__enter__", [](const Encoding_ptr& enc) { py::gil_scoped_release release; enc->mutex.lock(); })
+        .def("__exit__", [](const Encoding_ptr& enc, const py::args&) { enc->mutex.unlock(); })
         .def_property_readonly("calls", [](const Encoding_ptr& enc) { return enc->calls.load(); })
         .def("inference", [](const Encoding_ptr& enc, const at::Tensor& input, const py::object& parameter) {
             return encode(enc, input, tensorOrNone(parameter));

@@ -199,7 +199,8 @@ class Encoding:
 
     def precompile(self, adjoint_mode=3):
         """Compiles the standalone kernels into the kernel cache (needs no GPU)."""
-        check(lib.qmlp_encoding_precompile(self._handle, int(adjoint_mode)))
+        with self._native:
+            check(lib.qmlp_encoding_precompile(self._handle, int(adjoint_mode)))
 
     def hashgrid_levels(self):
         """[(resolution, hashed, memory_offset, hash_grid_size)] of a HashGrid encoding."""
@@ -217,15 +218,17 @@ class Encoding:
         records of large batches (sums per slice of the table) stand for; 4: the elements behind the
         sums of the column kernel (single dense levels whose batches train sorted by slab)."""
         if input is None:      # compile the kernel of this mode into the kernel cache, nothing runs
-            check(lib.qmlp_encoding_hashgrid_trace(self._handle, None, int(mode), None, None, None))
+            with self._native:
+                check(lib.qmlp_encoding_hashgrid_trace(self._handle, None, int(mode), None, None, None))
             return None
         levels = self.hashgrid_levels()
         dim = int(json.loads(self.to_json())["n_in"])
         n = input.shape[0]
         idx = torch.full((n, len(levels), 1 << dim), -1, dtype=torch.int32, device=input.device)
         w = torch.full((n, len(levels), 1 << dim), float("nan"), dtype=torch.float32, device=input.device)
-        check(lib.qmlp_encoding_hashgrid_trace(self._handle, desc(input), int(mode), idx.data_ptr(), w.data_ptr(),
-                                               current_stream(input.device)))
+        with self._native:
+            check(lib.qmlp_encoding_hashgrid_trace(self._handle, desc(input), int(mode), idx.data_ptr(), w.data_ptr(),
+                                                   current_stream(input.device)))
         return idx, w
 
     def inference(self, input):
@@ -244,8 +247,9 @@ class Encoding:
         if self.has_parameters():
             raise RuntimeError("Encoding has parameters, call the variation of 'adjoint' with parameters")
         adj_input = torch.zeros_like(input)
-        check(lib.qmlp_encoding_adjoint(self._handle, desc(input), desc(adj_output), desc(adj_input),
-                                        current_stream(input.device), None, None, 3))
+        with self._native:
+            check(lib.qmlp_encoding_adjoint(self._handle, desc(input), desc(adj_output), desc(adj_input),
+                                            current_stream(input.device), None, None, 3))
         return adj_input
 
     def adjoint_with_parameter(self, input, parameter_forward, adj_output):
@@ -260,9 +264,10 @@ class Encoding:
         size = ctypes.c_size_t()
         check(lib.qmlp_encoding_adjoint_memory(self._handle, input.shape[0], int(flags), ctypes.byref(size)))
         memory = torch.empty((size.value,), dtype=torch.uint8, device=input.device) if size.value else None
-        check(lib.qmlp_encoding_adjoint_in(self._handle, desc(input), desc(adj_output), desc(adj_input),
-                                           current_stream(input.device), desc(parameter_forward), desc(adj_param),
-                                           int(flags), memory.data_ptr() if size.value else None))
+        with self._native:
+            check(lib.qmlp_encoding_adjoint_in(self._handle, desc(input), desc(adj_output), desc(adj_input),
+                                               current_stream(input.device), desc(parameter_forward), desc(adj_param),
+                                               int(flags), memory.data_ptr() if size.value else None))
         self._bound_inference = None   # as in inference_with_parameter
         return adj_input, adj_param.to(parameter_forward.dtype)
 
@@ -346,7 +351,8 @@ class Network:
         return bool(_lib.get_int(lib.qmlp_network_is_parallel_streams, self._handle))
 
     def set_parallel_streams(self, enabled):
-        check(lib.qmlp_network_set_parallel_streams(self._handle, 1 if enabled else 0))
+        with self._mutex:
+            check(lib.qmlp_network_set_parallel_streams(self._handle, 1 if enabled else 0))
 
     def num_encodings(self):
         if getattr(self, "_num_encodings", None) is None:
@@ -413,15 +419,18 @@ class Network:
         return n.value
 
     def precompile(self, adjoint_flags=7):
-        check(lib.qmlp_network_precompile(self._handle, int(adjoint_flags)))
+        with self._mutex:
+            check(lib.qmlp_network_precompile(self._handle, int(adjoint_flags)))
 
     def prepare(self, num_elements, adjoint_flags=0):
         """Loads the kernels and allocates the workspace that calls on a batch of this size need,
         so that those calls only enqueue kernels (e.g. under graph capture)."""
-        check(lib.qmlp_network_prepare(self._handle, int(num_elements), int(adjoint_flags)))
+        with self._mutex:
+            check(lib.qmlp_network_prepare(self._handle, int(num_elements), int(adjoint_flags)))
 
     def generated_source(self, kind, adjoint_flags=0):
-        return _lib.get_string(lib.qmlp_network_generated_source, self._handle, kind.encode(), int(adjoint_flags))
+        with self._mutex:
+            return _lib.get_string(lib.qmlp_network_generated_source, self._handle, kind.encode(), int(adjoint_flags))
 
     def _set_network_parameters(self, network_parameters, encoding_parameters):
         self._native.bind(network_parameters, list(encoding_parameters))

@@ -670,3 +670,28 @@ def test_strides_beyond_32_bits_are_refused():
         net._native.bind(torch.zeros(1, dtype=torch.float16).as_strided((1, 1), (1 << 32, 1)), [])
     with pytest.raises(ValueError, match="32 bits"):
         net._native.bind(torch.zeros(count, dtype=torch.float16), [torch.zeros(1).as_strided((1,), (1 << 31,))])
+
+
+def test_threads_ask_a_fresh_network_for_its_memory_sizes():
+    """What depends on the specification alone is worked out by the first call: the others wait for it."""
+    import threading
+    cfg = json.loads(json.dumps(bc.CONFIGS[3]["cfg"]))
+    cfg["network"] = [{"n_out": 32, "bias": False, "activation": "relu"}] * 12 + [{"n_out": 1, "bias": False, "activation": "identity"}]
+    qmlp.set_log_level("error")
+
+    def sizes(net):
+        return [f(n, flags) for f in (net.adjoint_memory, net.forward_memory) for n in (1000, 100000) for flags in (2, 6, 7, 3, 1)]
+
+    want = sizes(qmlp.Network(json.dumps(cfg)))
+    for _ in range(30):
+        net, start, got = qmlp.Network(json.dumps(cfg)), threading.Barrier(8), []
+
+        def run():
+            start.wait()
+            got.append(sizes(net))
+
+        threads = [threading.Thread(target=run) for _ in range(8)]
+        [t.start() for t in threads]
+        [t.join() for t in threads]
+        assert got == [want] * 8
+    qmlp.set_log_level("warn")
