@@ -22,9 +22,11 @@
 //   B, coarse to fine: the gradient of a level before inpainting = adjoint of up with respect to the high-res
 //      level + adjoint of down, both formed per quad by gathering, without atomics
 // so a level of P pixels and C channels moves 2C+1 + (2C+2)/4 planes in A and 3C+2 + (5C+6)/4 planes in B.
-// 1 x 4 x 2048 x 2048 floats, finest level: down 21, up 37, A 49, B 68 us (4.9, 4.6, 2.6, 4.1 TB/s of the planes above; a
-// large copy reaches 5.2); the whole forward and adjoint call 428 us (438 with the coarse levels formed again by the adjoint), of which 175 are levels of 1024 x 1024 and larger
-// (9.4 ms with four passes per level through memory, atomics for odd sizes, and memory allocated and released by every call).
+// 1 x 4 x 2048 x 2048 floats, finest level: down 20, up 39, A 50, B 69 us (5.0, 4.3, 2.5, 4.1 TB/s of the planes above; a
+// large copy reaches 5.2), 178 of the 439 us of a forward and adjoint call; 1024 x 1024 takes 53, the levels below it, whose
+// launches and single workgroups wait for latency, the rest. (Coarse levels formed again by the adjoint: 10 us more; four
+// passes per level through memory, atomics for odd sizes, and memory allocated and released by every call: 9.4 ms.) A and B
+// are held to 128 registers for floats, four wavefronts per SIMD: with 129 and 130 they take 57 and 90 us.
 //
 // Follows src_cpp/include/qmlp/kernels/pullpush.cuh:22-303 of the reference. Differences on
 // purpose: no per-thread channel arrays, no atomics (the reference scatters the adjoint of up with atomics and adds
@@ -112,6 +114,27 @@ __device__ __forceinline__ void storePair(T* p, unsigned stride, bool second, co
     }
 }
 
+/** d / n for a sum of masks n, and zero where nothing is known, whatever d is then (NaN or infinite data times a mask of zero). */
+template <typename T>
+__device__ __forceinline__ T quotient(T d, T n)
+{
+    return n > 0 ? d / n : T(0);
+}
+
+/**
+ * The same as a multiplication, for several quotients by one sum in the adjoint, whose terms are products of several factors
+ * anyway. Scaled, as the reciprocal of a sum below 3e-39 has no float.
+ */
+template <typename T>
+struct Reciprocal
+{
+    static constexpr T SCALE = sizeof(T) == 4 ? T(1 << 22) : T(1ll << 52);
+    T inverse;
+    __device__ __forceinline__ Reciprocal() : inverse(0) {}
+    __device__ __forceinline__ explicit Reciprocal(T n) : inverse(n > 0 ? T(1) / (n * SCALE) : T(0)) {}
+    __device__ __forceinline__ T operator()(T d) const { return inverse > 0 ? d * inverse * SCALE : T(0); }
+};
+
 /** down for the low-res pixel (a, e). */
 template <bool PAIRS, typename T>
 __device__ __forceinline__ void downPixel(const PullPushLevel<T>& high, const PullPushLevel<T>& low, int C, int b, int a, int e)
@@ -143,7 +166,6 @@ __device__ __forceinline__ void downPixel(const PullPushLevel<T>& high, const Pu
         }
     *at(low.maskPre, b, 0, a, e) = most;
     *at(low.maskSum, b, 0, a, e) = sum;
-    const T inverse = sum > 0 ? T(1) / sum : T(0);
     constexpr int CHUNK = pullpushChunk<T>();
     for (int c0 = 0; c0 < C; c0 += CHUNK) {
         T d[CHUNK];
@@ -161,7 +183,7 @@ __device__ __forceinline__ void downPixel(const PullPushLevel<T>& high, const Pu
         }
 #pragma unroll
         for (int k = 0; k < CHUNK; ++k)
-            if (c0 + k < C) *at(low.dataPre, b, c0 + k, a, e) = d[k] * inverse;
+            if (c0 + k < C) *at(low.dataPre, b, c0 + k, a, e) = quotient(d[k], sum);
     }
 }
 
@@ -214,7 +236,8 @@ struct Neighbourhood
 template <typename T>
 struct QuadMix
 {
-    T wm[2][2][4], n[2][2], inverse[2][2], weight[2][2];   // (inverse: 1 / n, or zero)
+    T wm[2][2][4], n[2][2], weight[2][2];
+    Reciprocal<T> inverse[2][2];
     __device__ __forceinline__ QuadMix(const Neighbourhood& nb, const T (&maskLow)[3][3])
     {
 #pragma unroll
@@ -233,7 +256,7 @@ struct QuadMix
                     weight[di][dj] += w[k];
                     n[di][dj] += wm[di][dj][k];
                 }
-                inverse[di][dj] = n[di][dj] > 0 ? T(1) / n[di][dj] : T(0);
+                inverse[di][dj] = Reciprocal<T>(n[di][dj]);
             }
     }
     /** The weighted sum of a channel for pixel (di, dj). */
@@ -290,7 +313,7 @@ __device__ __forceinline__ void upQuad(const PullPushLevel<T>& high, const PullP
                 T out[2];
 #pragma unroll
                 for (int dj = 0; dj < 2; ++dj)
-                    out[dj] = m[di][dj] * v[k][di][dj] + (1 - m[di][dj]) * (mix.sum(lowData[k], di, dj) * mix.inverse[di][dj]);
+                    out[dj] = m[di][dj] * v[k][di][dj] + (1 - m[di][dj]) * quotient(mix.sum(lowData[k], di, dj), mix.n[di][dj]);
                 storePair<PAIRS>(at(high.dataPost, b, c0 + k, 2 * a + di, 2 * e), high.dataPost.x, second, out);
             }
         }
@@ -376,13 +399,12 @@ __device__ __forceinline__ void gradientUpTile(const PullPushLevel<T>& high, con
                             for (int k = 0; k < CHUNK; ++k) fill[k][di][dj] = T(0);
                             continue;
                         }
-                        const T passed = (1 - m[di][dj]) * mix.inverse[di][dj];
                         if (c0 == 0) fillN[di][dj] = gm[di][dj] * ((1 - m[di][dj]) / mix.weight[di][dj]);
 #pragma unroll
                         for (int k = 0; k < CHUNK; ++k) {
                             if (c0 + k >= C) continue;
-                            fill[k][di][dj] *= passed;
-                            fillN[di][dj] -= fill[k][di][dj] * (mix.sum(lowData[k], di, dj) * mix.inverse[di][dj]);
+                            fill[k][di][dj] = mix.inverse[di][dj](fill[k][di][dj] * (1 - m[di][dj]));
+                            fillN[di][dj] -= fill[k][di][dj] * mix.inverse[di][dj](mix.sum(lowData[k], di, dj));
                         }
                     }
             }
@@ -424,17 +446,17 @@ __device__ __forceinline__ void gradientQuad(const PullPushLevel<T>& high, const
     // left, which reach into the first row and column of the quad
     const bool oddH = high.H & 1, oddW = high.W & 1;
     bool in[2][2];
-    T inverse[2][2], most[2][2], gradMost[2][2];
+    T most[2][2], gradMost[2][2];
+    Reciprocal<T> sums[2][2];
 #pragma unroll
     for (int wa = 0; wa < 2; ++wa)
 #pragma unroll
         for (int we = 0; we < 2; ++we) {
             const int y = a - wa, x = e - we;
             in[wa][we] = (wa == 0 || oddH) && (we == 0 || oddW) && y >= 0 && x >= 0 && y < low.H && x < low.W;
-            inverse[wa][we] = most[wa][we] = gradMost[wa][we] = T(0);
+            most[wa][we] = gradMost[wa][we] = T(0);
             if (!in[wa][we]) continue;
-            const T sum = *at(low.maskSum, b, 0, y, x);
-            inverse[wa][we] = sum > 0 ? T(1) / sum : T(0);
+            sums[wa][we] = Reciprocal<T>(*at(low.maskSum, b, 0, y, x));
             most[wa][we] = *at(low.maskPre, b, 0, y, x);
             gradMost[wa][we] = *at(low.gradMaskPre, b, 0, y, x);
         }
@@ -474,7 +496,7 @@ __device__ __forceinline__ void gradientQuad(const PullPushLevel<T>& high, const
                 mean[k][wa][we] = grad[k][wa][we] = T(0);
                 if (!in[wa][we]) continue;
                 mean[k][wa][we] = *at(low.dataPre, b, c0 + k, a - wa, e - we);
-                grad[k][wa][we] = *at(low.gradDataPre, b, c0 + k, a - wa, e - we) * inverse[wa][we];
+                grad[k][wa][we] = sums[wa][we](*at(low.gradDataPre, b, c0 + k, a - wa, e - we));
             }
 #pragma unroll
             for (int di = 0; di < 2; ++di) {
@@ -495,7 +517,7 @@ __device__ __forceinline__ void gradientQuad(const PullPushLevel<T>& high, const
 #pragma unroll
                 for (int dj = 0; dj < 2; ++dj) {
                     // dataHigh = m * data + (1 - m) * (n > 0 ? d / n : 0)
-                    gradMask[di][dj] += g[k][di][dj] * (v[k][di][dj] - mix.sum(lowData[k], di, dj) * mix.inverse[di][dj]);
+                    gradMask[di][dj] += g[k][di][dj] * (v[k][di][dj] - mix.inverse[di][dj](mix.sum(lowData[k], di, dj)));
                     T sum = g[k][di][dj];
 #pragma unroll
                     for (int wa = 0; wa <= 1 - di; ++wa)
@@ -605,7 +627,7 @@ __global__ void __launch_bounds__(256) PullPushUpKernel(const PullPushLevel<T> h
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256) PullPushGradientUpKernel(const PullPushLevel<T> high, const PullPushLevel<T> low, int C, int pairs)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 1))) PullPushGradientUpKernel(const PullPushLevel<T> high, const PullPushLevel<T> low, int C, int pairs)
 {
     using namespace pullpush;
     __shared__ T sFill[pullpushChunk<T>() + 1][pullpushTileEntries(TILE_W, TILE_H)];
@@ -616,7 +638,7 @@ __global__ void __launch_bounds__(256) PullPushGradientUpKernel(const PullPushLe
 }
 
 template <typename T, bool ACCUMULATE>
-__global__ void __launch_bounds__(256) PullPushGradientKernel(const PullPushLevel<T> high, const PullPushLevel<T> low, int C, int pairs)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && !ACCUMULATE ? 4 : 1))) PullPushGradientKernel(const PullPushLevel<T> high, const PullPushLevel<T> low, int C, int pairs)
 {
     using namespace pullpush;
     int b, a, e;

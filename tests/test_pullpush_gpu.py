@@ -236,3 +236,37 @@ def test_rows_with_room_behind_an_odd_width():
     np.testing.assert_allclose(view_d.cpu().numpy(), wd, **ADJ_TOL[torch.float64])
     np.testing.assert_allclose(view_m.cpu().numpy(), wm, **ADJ_TOL[torch.float64])
     assert (gd[..., 101] == 7).all() and (gm[..., 101] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("shape", [(1, 3, 64, 96), (2, 2, 65, 97), (1, 5, 200, 201)])
+def test_data_of_unknown_pixels_stays_where_it_is(shape, dtype):
+    """A window without any known pixel has no mean: NaN or infinity inside it reach neither the coarser levels nor the
+    gradients of other pixels, whatever the kernel multiplies them with."""
+    mask, data, adj = make_case(sum(shape), *shape, dtype)
+    mask[:, 24:40, 40:60] = 0
+    mask[:, :5, -5:] = 0
+    print("pullpush unknown", shape, dtype, flush=True)
+    clean, dirty = gpu(data, dtype), gpu(data, dtype)
+    bad = torch.zeros(shape, dtype=torch.bool, device="cuda")
+    for k, (y, x) in enumerate([(28, 44), (33, 51), (34, 52), (30, 47), (1, shape[3] - 2)]):
+        bad[:, k % shape[1], y, x] = True
+    dirty[bad] = torch.tensor([float("nan"), float("inf")], dtype=dtype, device="cuda").repeat(int(bad.sum()))[:int(bad.sum())]
+    clean[bad] = 0
+    m, a = gpu(mask, dtype), gpu(adj, dtype)
+    assert torch.equal(pullpush(m, dirty)[~bad], pullpush(m, clean)[~bad])
+    (gm, gd), (wm, wd) = qpp.pullpush_backward(m, dirty, a), qpp.pullpush_backward(m, clean, a)
+    assert torch.equal(gd, wd)
+    pixel = bad.any(dim=1)
+    assert torch.equal(gm[~pixel], wm[~pixel])
+
+
+def test_masks_near_the_smallest_float():
+    """Masks of 2e-39 weigh as any others: their sums have no reciprocal in floats."""
+    rng = np.random.default_rng(6)
+    mask = np.full((1, 67, 130), 2e-39, np.float32)
+    data = rng.uniform(-1, 1, (1, 2, 67, 130)).astype(np.float32)
+    print("pullpush tiny masks", flush=True)
+    out = pullpush(gpu(mask, torch.float32), gpu(data, torch.float32))
+    # (masks are multiples of 2^-149, of which a sixteenth of 2e-39 has 9e4: weights good to 1e-5)
+    np.testing.assert_allclose(out.cpu().numpy(), ppo.pullpush(mask.astype(np.float64), data.astype(np.float64)), rtol=0, atol=1e-4)
