@@ -396,7 +396,12 @@ void Utils::adjointFractionalPullpush(const Tensor& mask, const Tensor& data, co
     checkLike(adjOutput, data, "adjOutput");
     checkLike(adjData, data, "adjData");
     checkLike(adjMask, mask, "adjMask");
-    if (data.numel() == 0) return;
+    if (data.numel() == 0) {
+        if (accumulate || mask.numel() == 0) return;   // images of no channels: their mask has no influence
+        if (mask.precision() == Tensor::FLOAT) elementwise<float>(COPY_4, adjMask, nullptr, stream);
+        else elementwise<double>(COPY_4, adjMask, nullptr, stream);
+        return;
+    }
     if (data.precision() == Tensor::FLOAT)
         adjoint<float>(mask, data, adjOutput, adjMask, adjData, accumulate, pyramid, pyramidReady, gradients, stream);
     else

@@ -270,3 +270,17 @@ def test_masks_near_the_smallest_float():
     out = pullpush(gpu(mask, torch.float32), gpu(data, torch.float32))
     # (masks are multiples of 2^-149, of which a sixteenth of 2e-39 has 9e4: weights good to 1e-5)
     np.testing.assert_allclose(out.cpu().numpy(), ppo.pullpush(mask.astype(np.float64), data.astype(np.float64)), rtol=0, atol=1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_images_of_no_channels(dtype):
+    """... have a mask, whose gradient is zero."""
+    print("pullpush no channels", dtype, flush=True)
+    mask = torch.ones((2, 6, 5), dtype=dtype, device="cuda").requires_grad_(True)
+    data = torch.zeros((2, 0, 6, 5), dtype=dtype, device="cuda").requires_grad_(True)
+    for _ in range(3):
+        rest = [torch.full_like(mask, 7.0) for _ in range(4)]     # what the allocator hands out next is not zero
+        del rest
+        out = pullpush(mask, data)
+        gm, gd = torch.autograd.grad(out, [mask, data], torch.zeros_like(out))
+        assert out.shape == data.shape and gd.shape == data.shape and (gm == 0).all()
