@@ -38,17 +38,23 @@
 
 QUICKMLP_KERNEL_NAMESPACE_BEGIN
 
-/**
- * A stack of images: entry (b, c, y, x); p == nullptr: absent. As built by the host (src/utils.cpp), which makes sure
- * that the entries of a plane lie within 2^32 of each other: the same plane for a whole workgroup (scalar registers) and
- * one 32-bit offset per lane.
- */
+// The entries of a plane lie within 2^32 of each other and behind the first: the same plane for a whole workgroup (scalar
+// registers) and one 32-bit offset per lane. For other images the host (src/utils.cpp) defines PULLPUSH_WIDE_PLANES.
+#ifdef PULLPUSH_WIDE_PLANES
+typedef int PullPushStride;
+typedef long long PullPushOffset;
+#else
+typedef unsigned PullPushStride;
+typedef unsigned PullPushOffset;
+#endif
+
+/** A stack of images: entry (b, c, y, x); p == nullptr: absent. */
 template <typename T>
 struct PullPushView
 {
     T* p;
     long long b, c;   // strides in entries
-    unsigned y, x;
+    PullPushStride y, x;
 };
 
 /** One level of the pyramid. The views of the coarsest level alias (post = pre, its gradients too). */
@@ -81,7 +87,7 @@ template <> struct Pair<double> { typedef double type __attribute__((ext_vector_
 template <typename T>
 __device__ __forceinline__ T* at(const PullPushView<T>& v, int b, int c, int y, int x)
 {
-    return v.p + (b * v.b + c * v.c) + (static_cast<unsigned>(y) * v.y + static_cast<unsigned>(x) * v.x);
+    return v.p + (b * v.b + c * v.c) + (static_cast<PullPushOffset>(y) * v.y + static_cast<PullPushOffset>(x) * v.x);
 }
 
 /**
@@ -89,7 +95,7 @@ __device__ __forceinline__ T* at(const PullPushView<T>& v, int b, int c, int y, 
  * an odd row is padding that belongs to the image. Otherwise the second is only touched if it exists (v[1] stays as it is).
  */
 template <bool PAIRS, typename T>
-__device__ __forceinline__ void loadPair(const T* p, unsigned stride, bool second, T (&v)[2])
+__device__ __forceinline__ void loadPair(const T* p, PullPushStride stride, bool second, T (&v)[2])
 {
     if constexpr (PAIRS) {
         const typename Pair<T>::type w = *reinterpret_cast<const typename Pair<T>::type*>(p);
@@ -101,7 +107,7 @@ __device__ __forceinline__ void loadPair(const T* p, unsigned stride, bool secon
     }
 }
 template <bool PAIRS, typename T>
-__device__ __forceinline__ void storePair(T* p, unsigned stride, bool second, const T (&v)[2])
+__device__ __forceinline__ void storePair(T* p, PullPushStride stride, bool second, const T (&v)[2])
 {
     if constexpr (PAIRS) {
         typename Pair<T>::type w;
@@ -152,7 +158,7 @@ __device__ __forceinline__ void downPixel(const PullPushLevel<T>& high, const Pu
             loadPair<PAIRS>(p, v.x, true, pair);
             out[i][0] = pair[0];
             out[i][1] = pair[1];
-            if (columns > 2) out[i][2] = p[2 * v.x];
+            if (columns > 2) out[i][2] = p[static_cast<PullPushOffset>(2) * v.x];
         }
     };
     window(high.maskPre, 0, m);
@@ -579,7 +585,7 @@ __device__ __forceinline__ PullPushLevel<T> ldsLevel(T* sLevels, const PullPushT
     l.W = W >> k;
     const unsigned pitch = (l.W + 1) & ~1, plane = l.H * pitch;
     auto take = [&](int channels) {
-        PullPushView<T> v{next, 0, plane, pitch, 1};
+        PullPushView<T> v{next, 0, plane, static_cast<PullPushStride>(pitch), 1};
         next += channels * plane;
         return v;
     };

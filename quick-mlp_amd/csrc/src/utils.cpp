@@ -37,7 +37,11 @@ constexpr int tailFillBytes()
     return planes * (2 * (TH + 2) * (2 * (TILE_W + 2) + 1)) * static_cast<int>(sizeof(T));
 }
 
-std::string pullpushSource() { return KernelLoader::MainFile("qmlp/kernels/pullpush.h"); }
+/** \param wide for images whose planes span 2^32 entries or more, or run backwards (see the header) */
+std::string pullpushSource(bool wide)
+{
+    return (wide ? "#define PULLPUSH_WIDE_PLANES\n" : "") + KernelLoader::MainFile("qmlp/kernels/pullpush.h");
+}
 
 std::string kernelName(int index, const std::string& scalar)
 {
@@ -48,14 +52,14 @@ std::string kernelName(int index, const std::string& scalar)
 
 /** The compiled kernels stay loaded for the life of the process, like the reference's static kernels. */
 template <typename T>
-KernelFunction& pullpushKernel(KernelIndex index)
+KernelFunction& pullpushKernel(KernelIndex index, bool wide = false)
 {
     static std::mutex mutex;
-    static KernelFunction kernels[sizeof(KERNEL_NAMES) / sizeof(KERNEL_NAMES[0])];
+    static KernelFunction kernels[2][sizeof(KERNEL_NAMES) / sizeof(KERNEL_NAMES[0])];
     std::lock_guard<std::mutex> lock(mutex);
-    auto& fun = kernels[index];
+    auto& fun = kernels[wide ? 1 : 0][index];
     if (!fun.defined())
-        fun = QuickMLP::Instance().kernelLoader()->getKernel(kernelName(index, sizeof(T) == 4 ? "float" : "double"), pullpushSource(),
+        fun = QuickMLP::Instance().kernelLoader()->getKernel(kernelName(index, sizeof(T) == 4 ? "float" : "double"), pullpushSource(wide),
                                                              QuickMLP::Instance().getCompileFlags()).value();
     return fun;
 }
@@ -66,7 +70,7 @@ struct View
 {
     T* p = nullptr;
     long long b = 0, c = 0;
-    unsigned y = 0, x = 0;
+    unsigned y = 0, x = 0;   // (the bits of a PullPushStride)
 };
 /** PullPushLevel of kernels/pullpush.h */
 template <typename T>
@@ -85,10 +89,18 @@ View<T> viewOf(const Tensor& t)
     v.c = n == 4 ? t.stride(1) : 0;
     v.y = static_cast<unsigned>(t.stride(n - 2));
     v.x = static_cast<unsigned>(t.stride(n - 1));
-    CHECK_ERROR(t.stride(n - 2) >= 0 && t.stride(n - 1) >= 0
-                    && (t.size(n - 2) - 1ll) * t.stride(n - 2) + (t.size(n - 1) - 1ll) * t.stride(n - 1) < (1ll << 32),
-                "fractionalPullpush: the entries of an image plane must lie within 2^32 of each other");
     return v;
+}
+/** Whether an entry of a plane of some of these images has no 32-bit offset from the first. */
+bool anyWide(std::initializer_list<const Tensor*> images)
+{
+    for (const Tensor* t : images) {
+        const int n = t->ndim();
+        if (t->stride(n - 2) < 0 || t->stride(n - 1) < 0
+            || (t->size(n - 2) - 1ll) * t->stride(n - 2) + (t->size(n - 1) - 1ll) * t->stride(n - 1) >= (1ll << 32))
+            return true;
+    }
+    return false;
 }
 
 bool isCoarsest(int H, int W) { return H <= 1 || W <= 1; }
@@ -188,14 +200,14 @@ std::vector<Level<T>> layout(int B, int C, int H, int W, void* pyramid, void* gr
 
 /** The levels below the last one with launches of its own, one workgroup per image. */
 template <typename T>
-void launchTail(KernelIndex kernel, int B, int C, Level<T> finest, bool gradients, T* kept, stream_t stream)
+void launchTail(KernelIndex kernel, bool wide, int B, int C, Level<T> finest, bool gradients, T* kept, stream_t stream)
 {
     if (isCoarsest(finest.H, finest.W)) return;
     Tail tail = {}, keptTail = {};
     const size_t lds = tailLdsBytes<T>(C, finest.H, finest.W, gradients, &tail);
     int keptEntries = static_cast<int>(tailLdsBytes<T>(C, finest.H, finest.W, false, &keptTail) / sizeof(T));
     void* args[] = {&finest, &C, &tail, &kept, &keptEntries, &keptTail};   // (the last one for the gradients only)
-    pullpushKernel<T>(kernel).launch(static_cast<unsigned>(B), TAIL_BLOCK, static_cast<unsigned>(lds), stream, args);
+    pullpushKernel<T>(kernel, wide).launch(static_cast<unsigned>(B), TAIL_BLOCK, static_cast<unsigned>(lds), stream, args);
 }
 
 /** Whether the pixels (y, 2k) and (y, 2k + 1) of all images of a level can be moved as one aligned pair. */
@@ -211,34 +223,34 @@ bool movesPairs(const Level<T>& level, bool padded)
 
 /** One launch for one level: a workgroup per tile of 32 x 8 items. */
 template <typename T>
-void launchLevel(KernelIndex kernel, int B, int C, int height, int width, const std::vector<Level<T>>& levels, int l, stream_t stream)
+void launchLevel(KernelIndex kernel, bool wide, int B, int C, int height, int width, const std::vector<Level<T>>& levels, int l, stream_t stream)
 {
     Level<T> high = levels[l], low = levels[l + 1];
     int pairs = movesPairs(high, l > 0) ? 1 : 0;
     const long long grid = static_cast<long long>(B) * divUp(height, TILE_H) * divUp(width, TILE_W);
     void* args[] = {&high, &low, &C, &pairs};
-    pullpushKernel<T>(kernel).launch(static_cast<unsigned>(grid), BLOCK, 0, stream, args);
+    pullpushKernel<T>(kernel, wide).launch(static_cast<unsigned>(grid), BLOCK, 0, stream, args);
 }
 
 /** The pyramid down to the coarsest level and the inpainted levels up to levels[1]; with 'finest' up to levels[0]. */
 template <typename T>
-void runForward(const std::vector<Level<T>>& levels, int B, int C, bool finest, T* keptTail, stream_t stream)
+void runForward(const std::vector<Level<T>>& levels, bool wide, int B, int C, bool finest, T* keptTail, stream_t stream)
 {
     const int last = static_cast<int>(levels.size()) - 1;
-    for (int l = 0; l < last; ++l) launchLevel(DOWN, B, C, levels[l + 1].H, levels[l + 1].W, levels, l, stream);
-    launchTail(TAIL, B, C, levels[last], false, keptTail, stream);
+    for (int l = 0; l < last; ++l) launchLevel(DOWN, wide, B, C, levels[l + 1].H, levels[l + 1].W, levels, l, stream);
+    launchTail(TAIL, wide, B, C, levels[last], false, keptTail, stream);
     for (int l = last - 1; l >= (finest ? 0 : 1); --l)
-        launchLevel(UP, B, C, divUp(levels[l].H, 2), divUp(levels[l].W, 2), levels, l, stream);
+        launchLevel(UP, wide, B, C, divUp(levels[l].H, 2), divUp(levels[l].W, 2), levels, l, stream);
 }
 
 template <typename T>
-void runAdjoint(const std::vector<Level<T>>& levels, int B, int C, bool accumulate, T* keptTail, stream_t stream)
+void runAdjoint(const std::vector<Level<T>>& levels, bool wide, int B, int C, bool accumulate, T* keptTail, stream_t stream)
 {
     const int last = static_cast<int>(levels.size()) - 1;
-    for (int l = 0; l < last; ++l) launchLevel(GRADIENT_UP, B, C, levels[l + 1].H, levels[l + 1].W, levels, l, stream);
-    launchTail(last == 0 && accumulate ? GRADIENT_TAIL_ADD : GRADIENT_TAIL, B, C, levels[last], true, keptTail, stream);
+    for (int l = 0; l < last; ++l) launchLevel(GRADIENT_UP, wide, B, C, levels[l + 1].H, levels[l + 1].W, levels, l, stream);
+    launchTail(last == 0 && accumulate ? GRADIENT_TAIL_ADD : GRADIENT_TAIL, wide, B, C, levels[last], true, keptTail, stream);
     for (int l = last - 1; l >= 0; --l)
-        launchLevel(l == 0 && accumulate ? GRADIENT_ADD : GRADIENT, B, C, divUp(levels[l].H, 2), divUp(levels[l].W, 2), levels, l, stream);
+        launchLevel(l == 0 && accumulate ? GRADIENT_ADD : GRADIENT, wide, B, C, divUp(levels[l].H, 2), divUp(levels[l].W, 2), levels, l, stream);
 }
 
 /** dst = src or dst += src for image stacks of any strides; without src: zero. */
@@ -276,7 +288,7 @@ void forward(const Tensor& mask, const Tensor& data, Tensor& output, void* pyram
     levels[0].maskPre = viewOf<T>(mask);
     levels[0].dataPre = viewOf<T>(data);
     levels[0].dataPost = viewOf<T>(output);
-    runForward(levels, B, C, true, keptTail, stream);
+    runForward(levels, anyWide({&mask, &data, &output}), B, C, true, keptTail, stream);
 }
 
 template <typename T>
@@ -293,11 +305,12 @@ void adjoint(const Tensor& mask, const Tensor& data, const Tensor& adjOutput, Te
     auto levels = layout<T>(B, C, H, W, pyramid, gradients, keptTail);
     levels[0].maskPre = viewOf<T>(mask);
     levels[0].dataPre = viewOf<T>(data);
-    if (!pyramidReady) runForward(levels, B, C, false, keptTail, stream);
+    const bool wide = anyWide({&mask, &data, &adjOutput, &adjMask, &adjData});
+    if (!pyramidReady) runForward(levels, wide, B, C, false, keptTail, stream);
     levels[0].gradDataPost = viewOf<T>(adjOutput);
     levels[0].gradMaskPre = viewOf<T>(adjMask);
     levels[0].gradDataPre = viewOf<T>(adjData);
-    runAdjoint(levels, B, C, accumulate, keptTail, stream);
+    runAdjoint(levels, wide, B, C, accumulate, keptTail, stream);
 }
 
 void checkShapes(const Tensor& mask, const Tensor& data)
@@ -339,7 +352,7 @@ void Utils::precompile(Tensor::Precision precision)
     auto kl = QuickMLP::Instance().kernelLoader();
     const int flags = QuickMLP::Instance().getCompileFlags() | KernelLoader::CompileOnly;
     for (size_t i = 0; i < sizeof(KERNEL_NAMES) / sizeof(KERNEL_NAMES[0]); ++i)
-        kl->getKernel(kernelName(static_cast<int>(i), t), pullpushSource(), flags);
+        kl->getKernel(kernelName(static_cast<int>(i), t), pullpushSource(false), flags);
 }
 
 void Utils::pullpushMemory(const Tensor& data, size_t& pyramidBytes, size_t& gradientBytes)

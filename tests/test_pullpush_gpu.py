@@ -284,3 +284,16 @@ def test_images_of_no_channels(dtype):
         out = pullpush(mask, data)
         gm, gd = torch.autograd.grad(out, [mask, data], torch.zeros_like(out))
         assert out.shape == data.shape and gd.shape == data.shape and (gm == 0).all()
+
+
+def test_planes_beyond_32_bit_offsets():
+    """Rows of a view so far apart that the last entry of a plane lies beyond 2^32 of the first."""
+    B, C, H, W, row = 1, 2, 4, 64, (1 << 31) - 64
+    mask, data, adj = make_case(3, B, C, H, W, torch.float32)
+    print("pullpush wide planes", flush=True)
+    m, d, a = (gpu(x, torch.float32) for x in (mask, data, adj))
+    far = torch.empty(((H - 1) * row + C * W,), device="cuda").as_strided((B, C, H, W), (C * W, W, row, 1))   # 26 GB
+    far.copy_(d)
+    assert torch.equal(pullpush(m, far), pullpush(m, d))
+    for got, want in zip(qpp.pullpush_backward(m, far, a), qpp.pullpush_backward(m, d, a)):
+        assert torch.equal(got, want)
