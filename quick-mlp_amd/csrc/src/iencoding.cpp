@@ -268,9 +268,10 @@ void IEncoding::adjointBySlices(const GradientSliceLayout& layout, const Tensor&
     if (!variants[variant].has_value()) variants[variant] = compileRecords(layout, inputGradients, variant, flags).value();
     if (!sk.clear.has_value()) sk.clear = compileSlices(layout, true, flags).value();
     if (!sk.slices.has_value()) {
-        sk.slices = compileSlices(layout, false, flags).value();
+        const KernelFunction slices = compileSlices(layout, false, flags).value();
         sk.items = Tensor(Tensor::FLOAT, {static_cast<int32_t>(layout.items.size() * (sizeof(GradientSlice) / sizeof(float)))});
         QMLP_HIP_CALL(qmlp_hip_memcpy_h2d(sk.items.rawPtr(), layout.items.data(), layout.items.size() * sizeof(layout.items[0]), nullptr));
+        sk.slices = slices;   // (last: what it reads is there, whatever of the above has thrown)
     }
 
     int* cursors = static_cast<int*>(tmpMemory);
