@@ -125,9 +125,11 @@ class FusedNetwork(torch.nn.Module):
         if self._scriptable:
             return self._network.forward(x, self.weights, list(self.encoding_parameters))
         encodings = self.encoding_parameters
-        # (from the list's own dict: its iterator looks every parameter up by name again)
-        tables = list(encodings._parameters.values())
-        if len(tables) != self._num_encodings:
+        # (from the list's own dict, by name: parameters that were replaced stand at its end; the list's iterator takes longer)
+        own = encodings._parameters
+        if len(own) == self._num_encodings:
+            tables = [own[str(i)] for i in range(self._num_encodings)]
+        else:
             tables = list(encodings)
         return self._network._native.forward(x, self.weights, tables)
 

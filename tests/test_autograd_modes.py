@@ -112,3 +112,19 @@ def test_threads_run_backward_on_one_graph(modules):
         for got in results:
             for a, b in zip(got, want):
                 torch.testing.assert_close(a, b, rtol=0.0, atol=1e-5 * float(b.abs().max()))
+
+
+def test_tables_that_were_replaced_keep_their_place(modules):
+    """A table that passes through a parametrization comes back at the end of its list's dict."""
+    cfg = dict(identity_cfg(3, [32, 2], ["relu", "identity"], [True, False]), encodings=[GRID, GRID])
+    warm_cache(cfg)
+    network = qmlp.FusedNetwork(json.dumps(cfg), weight_dtype=torch.float32)
+    for p in network.encoding_parameters:
+        p.data.uniform_(-1, 1)
+    x = torch.rand(200, 3, device="cuda")
+    want = network(x)
+    torch.nn.utils.parametrize.register_parametrization(network.encoding_parameters, "0", torch.nn.Identity())
+    assert torch.equal(network(x), want)
+    torch.nn.utils.parametrize.remove_parametrizations(network.encoding_parameters, "0")
+    assert list(network.encoding_parameters._parameters) == ["1", "0"]
+    assert torch.equal(network(x), want)
