@@ -36,12 +36,12 @@
 // records, such that no sum can overflow: at least 37 bits remain below the largest possible
 // contribution at 2^24 records, and the sums do not depend on the order of the additions. Batches whose
 // adjoints are not finite take the float additions, so that NaN and infinity reach the gradients. Weights
+// are at most one for points inside the box; the records of points outside of it (extrapolated with weights
+// beyond one, or NaN for a NaN coordinate) are added to the gradient tensor by the records kernel itself.
 // The adjoint pass of a standalone encoding gives its adjoints in floats. Its records hold floats (GridGradientLayout),
 // the scale of a sum goes by the records of its work item, and a value that would still lose bits in it (floats span
 // more than 64 bits) goes to the gradient tensor with an atomic: 3 of 10^5 in a batch of normally distributed adjoints
-// (16 levels of 2^19 entries of 2 floats, 2^17 points: 458 us with atomics, 81 + 53 us; 2^14 points 61 -> 51 us). Weights
-// are at most one for points inside the box; the records of points outside of it (extrapolated with weights
-// beyond one, or NaN for a NaN coordinate) are added to the gradient tensor by the records kernel itself.
+// (16 levels of 2^19 entries of 2 floats, 2^17 points: 458 us with atomics, 81 + 53 us; 2^14 points 61 -> 51 us).
 // Two forms that were measured and dropped: a workgroup per slice that tests every point of
 // the batch against its slice and recomputes the hits (the work of a hit falls to one lane of
 // 64, 890 us for 2^18 points and 16 levels), and the same with the hits queued in LDS first (the

@@ -42,7 +42,7 @@ __device__ __forceinline__ void workgroupLdsBarrier()
  * Few large blocks need fewer operand reads, many small ones fewer registers: the split of least
  *   matrix instructions + operand reads + REGISTER_WEIGHT / 8 x registers   (per tile of points and wavefront)
  * with the weight that the host found to leave the registers of the whole kernel within their budget
- * (FusedNetwork::cooperativeRegisterWeight repeats this sum). Blocks may overlap the edge (3 tiles in blocks of 2):
+ * (FusedNetwork::cooperativeRegisters repeats this sum). Blocks may overlap the edge (3 tiles in blocks of 2):
  * those beyond it repeat the last tile and are not stored.
  */
 template <int MT, int KT, int WAVES, int REGISTER_WEIGHT>

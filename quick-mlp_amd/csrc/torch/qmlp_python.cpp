@@ -1,7 +1,7 @@
 // qmlp._native: the calls that a training or rendering loop makes once per batch (FusedNetwork.forward, a standalone
-// encoding, and their backward passes), from Python straight into C++. A call on a small batch is bound by the host: through ctypes and a
-// Python autograd function, inference on 1000 points took 13 us beside a kernel of 3.6 us, and a train step on 513
-// points 148 us beside kernels of 25 us. Everything else of the Python package stays on ctypes.
+// encoding, and their backward passes), from Python straight into C++. A call on a small batch is bound by the host:
+// inference on 1000 points takes 8 us beside a kernel of 3.4 us, a train step on 513 points 60 us beside kernels of 20 us;
+// through ctypes and a Python autograd function they took 13 and 143 us. Everything else of the Python package stays on ctypes.
 //
 // Like the torch custom classes (qmlp_torch.cpp) this is written on the C ABI of libqmlp.so; the autograd node
 // replaces the one of the reference's binding (src_cpp/pytorch-bindings/src/bind_network.cpp:189-319).
