@@ -21,8 +21,9 @@
 //      (adjoint of up with respect to the low-res level; the terms that high-res pixels pass down stay in LDS)
 //   B, coarse to fine: the gradient of a level before inpainting = adjoint of up with respect to the high-res
 //      level + adjoint of down, both formed per quad by gathering, without atomics
-// so a level of P pixels and C channels moves 2C+1 + (2C+2)/4 planes in A and 3C+2 + (5C+6)/4 planes in B.
-// 1 x 4 x 2048 x 2048 floats, finest level: down 20, up 39, A 50, B 69 us (5.0, 4.3, 2.5, 4.1 TB/s of the planes above; a
+// so the finest level of C channels moves C+1 + (2C+2)/4 planes in A and 3C+2 + (3C+4)/4 in B (a coarser one, whose mask has a
+// gradient, one more in each), C+1 + (C+2)/4 in down and 2C+1 + (C+1)/4 in up.
+// 1 x 4 x 2048 x 2048 floats, finest level: down 20, up 39, A 50, B 69 us (5.4, 4.4, 2.5, 4.4 TB/s of the planes above; a
 // large copy reaches 5.2), 178 of the 439 us of a forward and adjoint call; 1024 x 1024 takes 53, the levels below it, whose
 // launches and single workgroups wait for latency, the rest. (Coarse levels formed again by the adjoint: 10 us more; four
 // passes per level through memory, atomics for odd sizes, and memory allocated and released by every call: 9.4 ms.) A and B
