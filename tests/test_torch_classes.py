@@ -13,7 +13,7 @@ import qmlp
 
 try:
     Q = qmlp.load_library()
-except ImportError:      # not built yet (a GPU box only loads what is built; here it takes a minute)
+except ImportError:      # not built yet (compiling takes a minute)
     import subprocess
     subprocess.run(["make", "-C", os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
                                                "quick-mlp_amd", "csrc", "torch")], check=True, capture_output=True)
