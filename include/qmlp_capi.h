@@ -136,6 +136,9 @@ int qmlp_network_overwritable_gradients(qmlp_network_t network, int num_elements
 int qmlp_network_adjoint_overwriting(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* adj_output,
                                      int adjoint_flags, int overwrite, const qmlp_tensor* adj_input,
                                      const void* tmp_memory_forward, void* tmp_memory_adjoint, void* stream);
+/* Whether the two entry points around this one can write the gradients of all encodings, too (QMLP_GRADIENTS_INPUT_ENCODINGS
+ * in `overwrite`). */
+int qmlp_network_overwritable_tables(qmlp_network_t network, int num_elements, int adjoint_flags, int* overwritable);
 /* qmlp_network_adjoint_overwriting on what qmlp_network_forward_for left, with the `contents` that it reported. Where
  * adjoint_flags need more than that, the forward pass runs again into tmp_memory_forward. */
 int qmlp_network_adjoint_for(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* adj_output,
@@ -184,6 +187,10 @@ int qmlp_encoding_adjoint_memory(qmlp_encoding_t encoding, long long points, int
 int qmlp_encoding_adjoint_in(qmlp_encoding_t encoding, const qmlp_tensor* input, const qmlp_tensor* adj_output,
                              const qmlp_tensor* adj_input, void* stream, const qmlp_tensor* parameters_forward,
                              const qmlp_tensor* parameters_gradients, int adjoint_mode, void* memory);
+/* The same where qmlp_encoding_adjoint_memory is not 0: the gradients of the parameters are written, whatever the tensor held. */
+int qmlp_encoding_adjoint_overwriting(qmlp_encoding_t encoding, const qmlp_tensor* input, const qmlp_tensor* adj_output,
+                                      const qmlp_tensor* adj_input, void* stream, const qmlp_tensor* parameters_forward,
+                                      const qmlp_tensor* parameters_gradients, int adjoint_mode, void* memory);
 /* Compiles the standalone kernels (forward, and the adjoint of adjoint_mode if > 0) into the
  * kernel cache without a GPU. No counterpart in the reference, which compiles lazily inside
  * forward()/adjoint() (src_cpp/src/iencoding.cpp:30-43,98-112). */

@@ -255,6 +255,7 @@ private:
         std::string recordsSource;
         int channelOffset = 0;
         CompiledKernel kernel;       // GridGradientSlicesKernel
+        KernelFunction exceptions;   // GridGradientExceptionsKernel
         Tensor items;                // device copy of layout.items
         // For batches that train sorted by grid slab, where the encoding offers it: the kernels of
         // kernels/grid_gradient_columns.h (compiled on first use), which take the place of records and slices
@@ -313,7 +314,7 @@ private:
     bool hasSliceGradients() const;
     /** Bytes per point of adjoint memory for the adjoint of the encoded rows (read by the records kernels); 0 without them. */
     int sliceGradientBytesPerPoint() const;
-    /** Bytes of bucket cursors and records of all encodings with gradient slices for a batch of numel (padded) points. */
+    /** Bytes of the records of all encodings with gradient slices for a batch of numel (padded) points. */
     size_t sliceGradientWorkspaceBytes(long long numel) const;
     /** Whether a batch of numel points with these flags takes the slice kernels. */
     bool useSliceGradients(int numel, int flags) const;
@@ -492,8 +493,8 @@ public:
     void adjoint(const Tensor& input, const Tensor& adjOutput, AdjointModeFlags adjointFlags, Tensor& adjInput,
                  const void* tmpMemoryForward, void* tmpMemoryAdjoint, stream_t stream);
     /**
-     * \param overwrite of GRADIENTS_INPUT and GRADIENTS_NETWORK_WEIGHTS those whose tensor holds nothing yet; only those that
-     *    overwritableGradients() names
+     * \param overwrite those whose tensor holds nothing yet: of GRADIENTS_INPUT and GRADIENTS_NETWORK_WEIGHTS only those that
+     *    overwritableGradients() names, GRADIENTS_INPUT_ENCODINGS only where overwritableTables() says so
      */
     void adjoint(const Tensor& input, const Tensor& adjOutput, AdjointModeFlags adjointFlags, Tensor& adjInput,
                  const void* tmpMemoryForward, void* tmpMemoryAdjoint, stream_t stream, AdjointModeFlags overwrite);
@@ -510,6 +511,8 @@ public:
      * kernel of 4 us in front of a small batch). Depends on neither the memory of the forward pass nor what it holds.
      */
     [[nodiscard]] AdjointModeFlags overwritableGradients(int numel, AdjointModeFlags adjointFlags, const void* tmpMemoryForward = nullptr);
+    /** Whether adjoint() can write the gradients of all encodings instead of adding to them: where the slice kernels sum them. */
+    [[nodiscard]] bool overwritableTables(int numel, AdjointModeFlags adjointFlags) const;
 
     /** For debugging, clears all cached kernels. */
     void clearCachedKernels();

@@ -143,53 +143,85 @@ public:
         int slice;
         int part;
         int parts;
-        int reserved0;
-        int reserved1;
+        int place;
+        int slices;
     };
     /** What the host needs to run the kernels of kernels/grid_gradient.h for an encoding. */
+    /** The temporary memory of the kernels of kernels/grid_gradient.h (mirrors kernel::GridGradientWorkspace). */
+    struct GradientWorkspace
+    {
+        void *records, *places, *exceptions, *largest;
+        int regions, recordsPerRegion, largestCount, reserved;
+    };
     struct GradientSliceLayout
     {
         std::string configType;            // device type of the level table
-        int sliceFloats = 0;               // floats of a full slice (= LDS of the slice kernel / 4)
+        int sliceFloats = 0;               // floats of a full slice
         int recordWords = 0;               // 32-bit words of a record
         int pairs = 0;                     // records per point and level
+        int features = 0;                  // floats of an entry
+        int inputChannels = 0;             // coordinates of a point
         int pointsPerWorkgroup = 0;        // most lanes of a workgroup of the records kernel (a power of two)
         int derivativeBytesPerPoint = 0;   // of kernel::PositionDerivativeLayout: what a training pass may keep for the input gradients
-        /** Dynamic LDS of the records kernel with this many lanes: its records of one level with the slice of each
-         *  (16 bits), and per slice of the level (at most 512) room in the bucket, count and place among the records. */
-        int recordsLdsBytes(int points) const { return points * pairs * (recordWords * 4 + 2) + 512 * 8 + (2 * 512 + 1) * 4 + 64; }
+        /** Dynamic LDS of the records kernel with this many lanes: its records of one level, and per slice of the level (at
+         *  most 512) their number and the place of the first. */
+        int recordsLdsBytes(int points) const { return points * pairs * recordWords * 4 + 2 * (512 + 1) * 4 + 64; }
+        /** Dynamic LDS of the slice kernel: 64-bit sums of a slice and of the entry behind it. */
+        int slicesLdsBytes() const { return (sliceFloats + features) * 8; }
         std::vector<int> slicesPerLevel;
         std::vector<GradientSlice> items;  // one workgroup of the slice kernel each
-        /** Records a bucket of level l holds for a batch of numel points (as in the device code). */
-        long long capacity(int l, long long numel) const { return ((5 * numel * pairs / 4) / slicesPerLevel[l] + 2048) & ~3ll; }
-        long long totalRecords(long long numel) const
-        {
-            long long n = 0;
-            for (size_t l = 0; l < slicesPerLevel.size(); ++l) n += slicesPerLevel[l] * capacity(static_cast<int>(l), numel);
-            return n;
-        }
-        int numBuckets() const
+        int numSlices() const
         {
             int n = 0;
             for (int s : slicesPerLevel) n += s;
             return n;
         }
         /**
-         * Workgroups of the records kernel over which the levels of a point are shared out. The levels of a batch
-         * without input gradients have nothing in common: eight times as many workgroups, each with an eighth of the
-         * chain of sorts (16 levels, records and slices of 2^14 / 2^15 / 2^16 / 2^17 points with 1 group 87 / 99 / 106 / 126 us,
-         * with 4 groups 55 / 61 / 88 / 125 us, with 8 groups 51 / 66 / 89 / 128 us; no difference from there on).
+         * Workgroups of the records kernel over which the levels of a region are shared out; input gradients have one more
+         * of their own.
          */
-        int levelGroups(bool inputGradients) const { return inputGradients ? 1 : std::min(8, static_cast<int>(slicesPerLevel.size())); }
-        static int recordsGrid(int numel, int points, int groups, int fullGrid)
+        int levelGroups() const { return std::min(8, static_cast<int>(slicesPerLevel.size())); }
+        int workgroupsPerRegion(bool inputGradients) const { return levelGroups() + (inputGradients ? 1 : 0); }
+        /** Regions that the records kernel works on at a time (of a large batch every workgroup gets several). */
+        static int regionSlots(long long numel, int points) { return static_cast<int>(std::min<long long>(divUp<long long>(numel, points), 1024)); }
+        /** Workgroups of GridGradientExceptionsKernel. */
+        static int exceptionsGrid(const GradientWorkspace& workspace) { return std::min(workspace.regions, 4096); }
+        /** The parts of the temporary memory for regions of so many points, and its bytes. */
+        GradientWorkspace workspace(void* memory, long long numel, int points, size_t* bytes = nullptr) const
         {
-            return groups * std::min(divUp(numel, points), std::max(1, fullGrid / groups));
+            GradientWorkspace w{};
+            size_t offset = 0;
+            auto take = [&](size_t size) {
+                void* p = memory ? static_cast<char*>(memory) + offset : nullptr;
+                offset += roundUp(size, size_t(256));
+                return p;
+            };
+            w.regions = static_cast<int>(divUp<long long>(numel, points));
+            w.recordsPerRegion = points * pairs;
+            w.largestCount = regionSlots(numel, points) * levelGroups();
+            const size_t levels = slicesPerLevel.size(), records = static_cast<size_t>(w.regions) * w.recordsPerRegion * levels;
+            w.largest = take(static_cast<size_t>(w.largestCount) * sizeof(uint32_t));
+            w.places = take(static_cast<size_t>(w.regions) * (numSlices() + 2 * levels) * sizeof(uint16_t));
+            w.records = take(records * recordWords * sizeof(uint32_t));
+            w.exceptions = take(records * sizeof(uint16_t));
+            if (bytes) *bytes = offset;
+            return w;
         }
-        /** What the records kernel and the slice kernel share: first the fill of the buckets and the largest adjoint, then the records. */
-        size_t cursorBytes() const { return roundUp(static_cast<size_t>(numBuckets() + 1) * sizeof(int), size_t(256)); }
+        /**
+         * Bytes of temporary memory of a batch, whatever the size of its regions. Callers size theirs once and for
+         * long: a quarter more records than the batch has and 2048 per slice, which is more than what lies beside the records takes.
+         */
         size_t workspaceBytes(long long numel) const
         {
-            return cursorBytes() + roundUp(static_cast<size_t>(totalRecords(numel)) * recordWords * sizeof(uint32_t), size_t(256));
+            size_t records = 0;
+            for (int slices : slicesPerLevel) records += static_cast<size_t>(slices) * static_cast<size_t>(((5 * numel * pairs / 4) / slices + 2048) & ~3ll);
+            size_t most = roundUp(static_cast<size_t>(numSlices() + 1) * sizeof(int), size_t(256)) + roundUp(records * recordWords * sizeof(uint32_t), size_t(256));
+            for (int points = pointsPerWorkgroup; points >= std::min(128, pointsPerWorkgroup); points /= 2) {
+                size_t bytes = 0;
+                (void)workspace(nullptr, numel, points, &bytes);
+                most = std::max(most, bytes);
+            }
+            return most;
         }
     };
     /** What the host needs to run the kernels of kernels/grid_gradient_columns.h for an encoding. */
@@ -291,10 +323,12 @@ public:
     /**
      * \param tmpMemory adjointMemory() bytes at a multiple of 256, which belong to this call until its kernels have
      *    run; without them the parameter gradients are scattered with atomics
+     * \param overwriteParameters with tmpMemory, where adjointMemory() is not 0: the parameter gradients are written
+     *    instead of added to
      */
     void adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& adjInput, stream_t stream,
                  const std::optional<const Tensor>& parametersForward,
-                 const std::optional<const Tensor>& parametersGradients, int adjointMode, void* tmpMemory);
+                 const std::optional<const Tensor>& parametersGradients, int adjointMode, void* tmpMemory, bool overwriteParameters = false);
 
     /**
      * Compiles the standalone forward kernel and, for adjointMode > 0, the adjoint kernels of
@@ -318,15 +352,16 @@ private:
     {
         // GridGradientRecordsKernel without / with input gradients, with pointsPerWorkgroup >> i lanes per workgroup
         std::vector<std::optional<KernelFunction>> records[2];
-        std::optional<KernelFunction> clear, slices;
+        std::optional<KernelFunction> slices, exceptions;
         Tensor items;
     };
     SliceKernels sliceKernels_;
     static int recordsVariants(const GradientSliceLayout& layout);
     std::optional<KernelFunction> compileRecords(const GradientSliceLayout& layout, bool inputGradients, int variant, int flags) const;
-    std::optional<KernelFunction> compileSlices(const GradientSliceLayout& layout, bool clear, int flags) const;
+    /** GridGradientSlicesKernel and GridGradientExceptionsKernel */
+    std::vector<KernelFunction> compileSlices(const GradientSliceLayout& layout, int flags) const;
     void adjointBySlices(const GradientSliceLayout& layout, const Tensor& input, const Tensor& adjOutput, Tensor& adjInput, stream_t stream,
-                         int adjointMode, void* tmpMemory, char* parameters);
+                         int adjointMode, void* tmpMemory, char* parameters, bool overwriteParameters);
 };
 typedef std::shared_ptr<IEncoding> IEncoding_ptr;
 

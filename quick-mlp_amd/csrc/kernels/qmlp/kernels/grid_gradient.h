@@ -1,34 +1,38 @@
 // Parameter gradients of a grid encoding without a global atomic per contribution: the
-// contributions are first written as records into buckets, one bucket per slice of the gradient
-// table, and a workgroup per slice then sums its bucket in LDS and adds the slice to the gradient
-// tensor once.
+// contributions are first written as records, sorted by slice of the gradient table, and a
+// workgroup per slice then sums its records in LDS and writes the slice once.
 //
 // Float atomics on device memory complete at about 21e9 requests per second on the whole
-// device wherever the data lives, and a hashed level offers nothing to combine (a batch of
+// device wherever the data lives (16e9 measured for atomics of 4 neighbouring floats, also where all
+// of a level are issued by one die), and a hashed level offers nothing to combine (a batch of
 // random points touches every entry about once). So the scatter of the fused backward kernel
 // (EncodingHashGrid::scatterTile, 4.5 requests per point and level) bounds a train step. Here
 // the backward kernel only stores the adjoint of the encoded rows. Then
-//   GridGradientRecordsKernel  walks over the points, one per lane, level by level: for every
+//   GridGradientRecordsKernel  takes a region of consecutive points, one per lane, level by level: for every
 //       pair of corners that are neighbours in memory it forms a record (the offsets of the two
 //       entries within their slice, their weights, the adjoint of the level's features), sorts the
-//       records of the workgroup by the slice of the gradient table they belong to (a slice is a
-//       run of 8192 or 16 384 floats, whose 64-bit sums take 64 or 128 KiB of LDS) in LDS, reserves
-//       room in the buckets of these slices with one atomic per slice and workgroup, and copies the
-//       sorted records there in runs: all stores of the records are coalesced. An upper entry that
-//       lies in another slice than the lower one is added to the gradient tensor right away. With
-//       INPUT_GRADIENTS the kernel also gathers the entries of all corners and adds the grid's
-//       share of the gradient with respect to the input (what EncodingHashGrid::adjoint computes,
-//       operation by operation): two entries that lie side by side with one load, issued after the
-//       bucket atomics of the level and used at its end, while the barriers in between (ldsBarrier)
-//       wait for LDS only, so the gathers stay in flight over the staging and the copy of the records
-//       (16 levels of a 3-D hash grid, 2^18 points: 203 -> 188 us; without the gathers 117 us). Where the forward
+//       records of the region by the slice of the gradient table they belong to (a slice is a
+//       run of 8192 or 16 384 floats, whose 64-bit sums take 64 or 128 KiB of LDS) in LDS, and copies them
+//       out as they are: the records of a region and level lie without gaps at a place that is known beforehand,
+//       and a row of `places` says where those of each slice begin. (Buckets per slice, in which every workgroup reserved room
+//       with an atomic per slice and level: 25 us of atomics, and a batch of unevenly spread points found them full. 16
+//       levels, 2^18 points with input gradients: 124 -> 82 us.) The levels of a region are shared out over several
+//       workgroups, and the grid's share of the gradient with respect to the input
+//       (what EncodingHashGrid::adjoint computes, operation by operation) is left to one workgroup more per region: from the
+//       entries of all corners, two that lie side by side with one load, or, where the forward
 //       pass kept the derivatives of the features with respect to the position (PositionDerivativeLayout,
-//       INPUT_GRADIENTS == 2), the share is adjoint x derivative from one or two coalesced loads per level
-//       instead (same grid: 126 us);
+//       INPUT_GRADIENTS == 2), as adjoint x derivative from one or two coalesced loads per level. Bound by the memory that
+//       the records are written to: 268 MB of them for 2^18 points, 3.3 TB/s;
 //   GridGradientSlicesKernel   runs one workgroup per work item (level, slice, part of the
-//       bucket): it streams through its records and adds weight * adjoint to the slice in LDS,
-//       then adds the slice to the gradient tensor (with atomics only for a coarse level, whose
-//       few slices receive all records of the level and are shared out over several work items).
+//       regions): it streams through its records, a segment in every region, and adds weight * adjoint to the slice in LDS,
+//       then writes the slice, or adds it to the gradient tensor (with atomics only for a coarse level, whose
+//       few slices receive all records of the level and are shared out over several work items, and for the first entry
+//       of a slice, to which the slice in front adds as well). Bound by the memory that the records come from: without its
+//       LDS additions it takes 76 instead of 79 us (2^18 points; 52 of them are the records, at 5 TB/s, 9 the stores of 50 MB,
+//       and the rest what a work item waits for before its first record). Tensors that hold nothing yet are written: 50 MB that nobody
+//       zeroes first nor reads again (2^18 points: 95 -> 84 us and a fill of 9 us);
+//   GridGradientExceptionsKernel   adds, with atomics, what has no record: the points outside of the box and upper
+//       entries in another slice than the one behind the lower one's.
 // The sums in LDS are 64-bit fixed point, added with integer atomics: ds_add_f32 completes one
 // lane every three cycles on this hardware (0.32 lanes per clock and CU measured, whatever the
 // addresses), ds_add_u64 3.5 lanes per clock. The scale is a power of two chosen per launch from the
@@ -37,17 +41,15 @@
 // contribution at 2^24 records, and the sums do not depend on the order of the additions. Batches whose
 // adjoints are not finite take the float additions, so that NaN and infinity reach the gradients. Weights
 // are at most one for points inside the box; the records of points outside of it (extrapolated with weights
-// beyond one, or NaN for a NaN coordinate) are added to the gradient tensor by the records kernel itself.
+// beyond one, or NaN for a NaN coordinate) are exceptions.
 // The adjoint pass of a standalone encoding gives its adjoints in floats. Its records hold floats (GridGradientLayout),
 // the scale of a sum goes by the records of its work item, and a value that would still lose bits in it (floats span
 // more than 64 bits) goes to the gradient tensor with an atomic: 3 of 10^5 in a batch of normally distributed adjoints
-// (16 levels of 2^19 entries of 2 floats, 2^17 points: 458 us with atomics, 81 + 53 us; 2^14 points 61 -> 51 us).
+// (16 levels of 2^19 entries of 2 floats, 2^17 points: 458 us with atomics, 44 + 49 us; 2^14 points 61 -> 51 us).
 // Two forms that were measured and dropped: a workgroup per slice that tests every point of
 // the batch against its slice and recomputes the hits (the work of a hit falls to one lane of
 // 64, 890 us for 2^18 points and 16 levels), and the same with the hits queued in LDS first (the
 // queued hits gather their point's coordinates and adjoints at random: bound by line requests).
-// A bucket has room for 1.25 times its share of the records of a uniform batch; a record that
-// finds its bucket full is added to the gradient tensor with atomics by the lane that holds it.
 //
 // Replaces, for batches that are large enough, the atomicAdd of
 // src_cpp/include/qmlp/kernels/encoding_hashgrid.cuh:117-166,345-369 of the reference.
@@ -58,7 +60,7 @@
 QUICKMLP_KERNEL_NAMESPACE_BEGIN
 
 /** One work item of GridGradientSlicesKernel: the `floats` elements of the gradient table from
- *  element `first` on (slice `slice` of level `level`), part `part` of `parts` of its bucket. */
+ *  element `first` on (slice `slice` of level `level`), part `part` of `parts` of its regions. */
 struct GridGradientSlice
 {
     int level;
@@ -67,8 +69,28 @@ struct GridGradientSlice
     int slice;
     int part;
     int parts;       // > 1: other work items hold sums for the same slice, all add it with atomics
-    int reserved0;
-    int reserved1;
+    int place;       // of the slice in a row of GridGradientWorkspace::places
+    int slices;      // of the level
+};
+
+/** Every level gets about this many work items of the slice kernel. */
+constexpr int GRID_GRADIENT_ITEMS_PER_LEVEL = 32;
+
+/**
+ * The temporary memory of these kernels. A region is what one workgroup of the records kernel files of POINTS
+ * consecutive points: per level POINTS * PAIRS records, sorted by slice and without gaps.
+ */
+struct GridGradientWorkspace
+{
+    unsigned* records;            // (levels, regions, recordsPerRegion)
+    // (regions, PLACES): per level where the records of each slice begin, how many records there are, how many exceptions
+    unsigned short* places;
+    unsigned short* exceptions;   // (levels, regions, recordsPerRegion): pairs that are left to GridGradientExceptionsKernel
+    unsigned* largest;            // per workgroup the largest magnitude among its adjoints (bits without the sign)
+    int regions;
+    int recordsPerRegion;
+    int largestCount;
+    int reserved;
 };
 
 /**
@@ -166,32 +188,26 @@ struct GridGradientLayout
         return (l + 1 < L ? Cfg::memoryOffset[l + 1] : Cfg::ParameterCount) - Cfg::memoryOffset[l];
     }
     __device__ __host__ static constexpr int numSlices(int l) { return (levelFloats(l) + SLICE_FLOATS - 1) / SLICE_FLOATS; }
-    /** Records a bucket of level l holds for a batch of numel points. */
-    __device__ __host__ static constexpr long long capacity(int l, long long numel)
-    {
-        return ((5 * numel * PAIRS / 4) / numSlices(l) + 2048) & ~3ll;
-    }
-    /** Index of the first bucket of level l. */
-    __device__ __host__ static constexpr int firstBucket(int l)
+    /** Index of the first word of level l in a row of GridGradientWorkspace::places, and the words of a row. */
+    __device__ __host__ static constexpr int firstPlace(int l)
     {
         int n = 0;
-        for (int k = 0; k < l; ++k) n += numSlices(k);
+        for (int k = 0; k < l; ++k) n += numSlices(k) + 2;
         return n;
     }
-    /** Offset in records of the first bucket of level l. */
-    __device__ __host__ static constexpr long long levelOffset(int l, long long numel)
+    static constexpr int PLACES = firstPlace(L);
+
+    /** Levels with few slices are summed by several work items each (as encoding_hashgrid.cpp makes them). */
+    __device__ __host__ static constexpr int parts(int l)
     {
-        long long n = 0;
-        for (int k = 0; k < l; ++k) n += numSlices(k) * capacity(k, numel);
-        return n;
+        return GRID_GRADIENT_ITEMS_PER_LEVEL / numSlices(l) > 1 ? GRID_GRADIENT_ITEMS_PER_LEVEL / numSlices(l) : 1;
     }
 };
 
 /**
  * A workgroup barrier that orders the LDS accesses of the workgroup and nothing else. __syncthreads() also waits for
- * every load from and store to global memory that the wavefront has in flight; the records kernel keeps the gathers
- * of a level's table entries in flight across the barriers of that level's sort, and nothing it writes to global
- * memory is read again before the kernel ends.
+ * every load from and store to global memory that the wavefront has in flight; nothing that the records kernel writes to
+ * global memory is read again before the kernel ends.
  */
 __device__ __forceinline__ void ldsBarrier()
 {
@@ -320,24 +336,12 @@ struct GridGradientRecords
         }
     }
 
-    /** What happens to an upper entry that lies in another slice than its record: the product adds it to the
-     *  gradient tensor right away. */
-    struct AddToTensor
-    {
-        float* __restrict__ gradients;
-        __device__ __forceinline__ void operator()(unsigned element, float weight, const unsigned (&adjWords)[AW]) const
-        {
-#pragma unroll
-            for (int i = 0; i < F; ++i) unsafeAtomicAdd(gradients + element + i, weight * Layout::adjoint(adjWords, i));
-        }
-    };
-
     /**
      * The record of pair c of a point in one level: the offsets of its two entries within the slice of the lower
-     * one, their weights and the adjoint words. Returns the slice (= bucket within the level) that files it.
+     * one, their weights and the adjoint words. Returns the slice within the level that files it.
      * \param otherSlice called with (element of feature 0 in the table, weight, adjWords) for an upper entry that
-     *    lies in another slice (an entry next to a slice boundary; in a hashed level one pair in thousands): the
-     *    record then keeps the lower entry only
+     *    lies in another slice and not right behind this one (in a hashed level of more cells along a coordinate than a
+     *    slice has entries): the record then keeps the lower entry only
      */
     template <int LEVEL, typename OtherSlice>
     __device__ __forceinline__ static int buildRecord(const typename Grid::LevelSetup& s, int c,
@@ -355,7 +359,7 @@ struct GridGradientRecords
         unsigned eH = idxH * F - sliceStart;                     // wraps if the upper entry lies below the slice
         float wH = w * s.f[PD];
         const float wL = w * (1.f - s.f[PD]);
-        if (eH >= static_cast<unsigned>(SLICE_FLOATS)) {
+        if (eH >= static_cast<unsigned>(SLICE_FLOATS + F)) {
             otherSlice(base + idxH * F, wH, adjWords);
             eH = eL;
             wH = 0.f;
@@ -379,47 +383,40 @@ struct GridGradientRecords
         return bucket;
     }
 
-    /** Adds a record to the gradient tensor itself (its bucket was full); grad: element 0 of the record's slice. */
-    __device__ __forceinline__ static void addToTensor(const unsigned (&rec)[RW], float* __restrict__ grad)
-    {
-        float wL, wH;
-        Layout::weights(rec, wL, wH);
-        const unsigned eL = rec[0] & 0xffffu, eH = rec[0] >> 16;
-#pragma unroll
-        for (int i = 0; i < F; ++i) {
-            const float adj = Layout::adjoint(rec + Layout::FIRST_ADJOINT, i);
-            unsafeAtomicAdd(grad + eL + i, wL * adj);
-            if (wH != 0.f) unsafeAtomicAdd(grad + eH + i, wH * adj);
-        }
-    }
-
     /** Feature i of a level among the channels of the encoded rows. */
     template <int LEVEL>
     __device__ __forceinline__ static constexpr int channel(int i) { return CHANNEL_OFFSET + (Cfg::Concat ? LEVEL * F : 0) + i; }
 
-    template <int LEVEL, int INPUT_GRADIENTS>
-    __device__ __forceinline__ static void runLevel(int p, bool valid, long long numel, const float (&pos)[D],
-                                                    const Adjoints& adjEncoded, const param_t& params,
-                                                    unsigned* __restrict__ records, int* __restrict__ cursors,
-                                                    unsigned* sStage, unsigned short* sBucketOf, int* sHist,
-                                                    int* sLocalBase, long long* sGlobalBase, unsigned& maxAdjBits,
-                                                    float (&adjPos)[D], const DerivativeChunk* __restrict__ derivatives)
+    /** What an entry of GridGradientWorkspace::exceptions says: the lane and the pair, and whether the lower entry is in its record. */
+    static constexpr unsigned EXCEPTION_PAIR_SHIFT = 10, EXCEPTION_UPPER_ONLY = 1u << 13;
+    static_assert(POINTS <= 1024 && PAIRS <= 8, "an exception takes 16 bits");
+
+    /**
+     * Files the records of the workgroup's points in one level. sCount: zeros on entry and on return, MAX_SLICES + 1 words.
+     */
+    template <int LEVEL>
+    __device__ __forceinline__ static void runLevel(int p, int numel, int region, const float (&position)[D], const Adjoints& adjEncoded,
+                                                    const GridGradientWorkspace& ws, unsigned* sStage, int* sCount, int* sStart,
+                                                    unsigned& maxAdjBits)
     {
-        constexpr bool hashed = Cfg::hashed[LEVEL];
-        constexpr int PD = hashed ? 0 : D - 1;
-        constexpr unsigned base = static_cast<unsigned>(Cfg::memoryOffset[LEVEL]);
         constexpr int NS = Layout::numSlices(LEVEL);
-        static_assert(NS <= MAX_SLICES, "the slice of a record is kept in the histogram arrays");
-        const int tid = threadIdx.x;
-        for (int b = tid; b < NS; b += POINTS) sHist[b] = 0;
-        ldsBarrier();   // also: the staging area of the previous level has been copied out
+        static_assert(NS <= MAX_SLICES, "the records of a slice are counted in LDS");
+        int tid = threadIdx.x;
+        const long long regionStart = (static_cast<long long>(LEVEL) * ws.regions + region) * (POINTS * PAIRS);
+        // (nothing of a level is worked out, and held in registers, before the one in front of it has ended)
+        float pos[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            pos[d] = position[d];
+            asm volatile("" : "+v"(pos[d]));
+        }
+        asm volatile("" : "+v"(p), "+v"(tid));
+        const bool valid = p < numel;
 
         // my records of this level, in registers, and their places among the workgroup's records of the same slice
         unsigned rec[PAIRS][RW];
         int bucket[PAIRS], rank[PAIRS];
         const typename Grid::LevelSetup s = Grid::setupLevel(LEVEL, pos);
-        detail::HeldFeatures<F, typename Cfg::table_t> held[Grid::NC];
-        (void)held;
         if (valid) {
             unsigned adjWords[AW];
 #pragma unroll
@@ -436,71 +433,45 @@ struct GridGradientRecords
                     maxAdjBits = max(maxAdjBits, bits & 0x7fffu);
                 }
             }
-            if constexpr (INPUT_GRADIENTS == 1 && !DEFER_ENTRIES) {
-                // the entries of all corners, for this grid's share of dL/dinput (a dense 4-D grid with 8 features
-                // holds 64 registers: used at once; held until the end of the level 302 against 275 us)
-                loadHeld<LEVEL>(s, params, held);
-                positionGradient<LEVEL>(p, s, held, adjEncoded, adjPos);
-            }
-#pragma unroll
-            for (int c = 0; c < PAIRS; ++c) {
-                bucket[c] = buildRecord<LEVEL>(s, c, adjWords, rec[c], AddToTensor{params.parametersBackward});
-                // (a level of one slice needs no sorting: every lane has fixed places)
-                rank[c] = NS == 1 ? tid * PAIRS + c : atomicAdd(sHist + bucket[c], 1);
-            }
             // The sums of the slice kernel are fixed point with a scale that counts on weights of at most one, which
             // holds while every fractional position lies in [0, 1]: for every point inside the box. A point outside of
             // it is extrapolated (the fractional position is not clamped) with weights that grow with its distance, a
-            // NaN coordinate gives NaN weights: the records of such a point are added to the gradient tensor right
-            // here, as records are whose bucket is full, and go to the buckets with weights of zero.
+            // NaN coordinate gives NaN weights: the pairs of such a point are exceptions, and their records hold zeros.
             bool inside = true;
 #pragma unroll
             for (int d = 0; d < D; ++d) inside = inside && s.f[d] >= 0.f && s.f[d] <= 1.f;
+            auto except = [&](int c, unsigned which) {
+                const int at = atomicAdd(sCount + NS, 1);
+                ws.exceptions[regionStart + at] = static_cast<unsigned short>(static_cast<unsigned>(tid) | (static_cast<unsigned>(c) << EXCEPTION_PAIR_SHIFT) | which);
+            };
+#pragma unroll
+            for (int c = 0; c < PAIRS; ++c) {
+                bool otherSlice = false;
+                bucket[c] = buildRecord<LEVEL>(s, c, adjWords, rec[c], [&](unsigned, float, const unsigned (&)[AW]) { otherSlice = true; });
+                // (a level of one slice needs no sorting: every lane has fixed places)
+                rank[c] = NS == 1 ? tid * PAIRS + c : atomicAdd(sCount + bucket[c], 1);
+                if (otherSlice && inside) except(c, EXCEPTION_UPPER_ONLY);
+            }
             if (!inside) {
-                // (rare: a loop that recomputes the pairs and reads the adjoints again, so that it costs the points
-                // inside the box neither registers nor code)
-                float* __restrict__ grad = params.parametersBackward + base;
-#pragma unroll 1
-                for (int c = 0; c < PAIRS; ++c) {
-                    unsigned idxL, idxH;
-                    float w;
-                    pairEntries<LEVEL>(s, c, idxL, idxH, w);
-                    const float wL = w * (1.f - s.f[PD]), wH = w * s.f[PD];
-                    // (an upper entry in another slice than the lower one has been added by buildRecord already)
-                    const unsigned sliceStart = idxL * F / SLICE_FLOATS * SLICE_FLOATS;
-                    const bool upperAdded = idxH * F - sliceStart >= static_cast<unsigned>(SLICE_FLOATS);
-#pragma unroll 1
-                    for (int i = 0; i < F; ++i) {
-                        const float adj = static_cast<float>(adjEncoded(p, channel<LEVEL>(i)));
-                        unsafeAtomicAdd(grad + idxL * F + i, wL * adj);
-                        if (!upperAdded) unsafeAtomicAdd(grad + idxH * F + i, wH * adj);
-                    }
-                }
 #pragma unroll
                 for (int c = 0; c < PAIRS; ++c) {
+                    except(c, 0u);
 #pragma unroll
                     for (int v = 1; v < (FLOATS ? 2 + F : 3); ++v) rec[c][v] = 0u;
                 }
             }
-        } else {
-            // lanes beyond the batch: in a level of one slice they fill their fixed places with records that add nothing
-#pragma unroll
-            for (int c = 0; c < PAIRS; ++c) {
-#pragma unroll
-                for (int v = 0; v < RW; ++v) rec[c][v] = 0u;
-                bucket[c] = 0;
-                rank[c] = tid * PAIRS + c;
-            }
         }
-        if (NS == 1 && tid == 0) sHist[0] = POINTS * PAIRS;
-        ldsBarrier();
+        if (NS == 1 && tid == 0) sCount[0] = min(POINTS, numel - (p - tid)) * PAIRS;
+        ldsBarrier();   // also: the staging area of the previous level has been copied out
 
-        // places of the slices in the staging area, and room in their buckets (one atomic per slice)
+        // where the records of each slice begin
         if (tid < 64) {
+            unsigned short* places = ws.places + static_cast<long long>(region) * Layout::PLACES + Layout::firstPlace(LEVEL);
             int running = 0;
+#pragma unroll
             for (int b0 = 0; b0 < NS; b0 += 64) {
                 const int b = b0 + tid;
-                const int n = b < NS ? sHist[b] : 0;
+                const int n = b < NS ? sCount[b] : 0;
                 int inclusive = n;
 #pragma unroll
                 for (int d = 1; d < 64; d *= 2) {
@@ -508,53 +479,33 @@ struct GridGradientRecords
                     if (tid >= d) inclusive += other;
                 }
                 if (b < NS) {
-                    sLocalBase[b] = running + inclusive - n;
-                    sGlobalBase[b] = n > 0 ? static_cast<long long>(atomicAdd(cursors + Layout::firstBucket(LEVEL) + b, n)) : 0;
+                    sStart[b] = running + inclusive - n;
+                    places[b] = static_cast<unsigned short>(running + inclusive - n);
                 }
                 running += __shfl(inclusive, 63, 64);
             }
-            if (tid == 0) sLocalBase[NS] = running;
-        }
-        ldsBarrier();
-
-        if constexpr (INPUT_GRADIENTS == 1 && DEFER_ENTRIES) {
-            // The entries of all corners, for this grid's share of dL/dinput, where they take few registers: loaded
-            // here and used at the end of the level, so that the two steps in between hide their latency (the
-            // barriers order LDS only). Not earlier: the first wavefront waits for its bucket atomics above, and
-            // loads return in the order of their issue.
-            if (valid) loadHeld<LEVEL>(s, params, held);
-        }
-        if (valid || NS == 1) {
-#pragma unroll
-            for (int c = 0; c < PAIRS; ++c) {
-                const int at = sLocalBase[bucket[c]] + rank[c];
-                Layout::storeRecord(sStage + at * RW, rec[c]);
-                sBucketOf[at] = static_cast<unsigned short>(bucket[c]);
+            if (tid == 0) {
+                sStart[NS] = running;
+                places[NS] = static_cast<unsigned short>(running);
+                places[NS + 1] = static_cast<unsigned short>(sCount[NS]);
             }
         }
         ldsBarrier();
 
-        // sorted by slice: consecutive lanes copy consecutive records of a bucket
-        const int total = sLocalBase[NS];
-        const long long capacity = Layout::capacity(LEVEL, numel);
-        unsigned* levelRecords = records + Layout::levelOffset(LEVEL, numel) * RW;
+        for (int b = tid; b <= NS; b += POINTS) sCount[b] = 0;
+        if (valid) {
+#pragma unroll
+            for (int c = 0; c < PAIRS; ++c) Layout::storeRecord(sStage + (sStart[bucket[c]] + rank[c]) * RW, rec[c]);
+        }
+        const int total = sStart[NS];
+        ldsBarrier();
+
+        // sorted by slice: the region as a whole
+        unsigned* __restrict__ records = ws.records + regionStart * RW;
         for (int j = tid; j < total; j += POINTS) {
-            const int b = sBucketOf[j];
-            const long long at = sGlobalBase[b] + (j - sLocalBase[b]);
             unsigned r[RW];
             Layout::loadRecord(sStage + j * RW, r);
-            if (at < capacity) {
-                Layout::storeRecord(levelRecords + (static_cast<long long>(b) * capacity + at) * RW, r);
-            } else {
-                addToTensor(r, params.parametersBackward + base + static_cast<unsigned>(b) * SLICE_FLOATS);
-            }
-        }
-
-        if constexpr (INPUT_GRADIENTS == 1 && DEFER_ENTRIES) {
-            if (valid) positionGradient<LEVEL>(p, s, held, adjEncoded, adjPos);
-        }
-        if constexpr (INPUT_GRADIENTS == 2) {
-            if (valid) positionGradientFromDerivatives<LEVEL>(p, derivatives, adjEncoded, adjPos);
+            Layout::storeRecord(records + j * RW, r);
         }
     }
 
@@ -582,9 +533,6 @@ struct GridGradientRecords
 #pragma unroll
         for (int d = 0; d < D; ++d) adjPos[d] += scale * lvl[d];
     }
-
-    /** Registers worth holding across the sort of a level's records: 64 bytes of table entries per lane. */
-    static constexpr bool DEFER_ENTRIES = Grid::NC * F * static_cast<int>(sizeof(typename Cfg::table_t)) <= 64;
 
     /**
      * This level's share of the gradient with respect to the position, operation by operation as
@@ -631,109 +579,231 @@ struct GridGradientRecords
         for (int d = 0; d < D; ++d) adjPos[d] += scale * lvl[d];
     }
 
+    /** Two workgroups of 1024 lanes per compute unit where the records of a lane leave room for it in 64 registers. */
+    template <int INPUT_GRADIENTS>
+    __device__ __host__ static constexpr int wavesPerSimd() { return PAIRS * RW <= 16 && INPUT_GRADIENTS != 1 ? 8 : POINTS >= 1024 ? 4 : 1; }
+
     /** The levels from LEVEL to END - 1. */
-    template <int LEVEL, int END, int INPUT_GRADIENTS>
-    __device__ __forceinline__ static void runLevels(int p, bool valid, long long numel, const float (&pos)[D],
-                                                     const Adjoints& adjEncoded, const param_t& params,
-                                                     unsigned* __restrict__ records, int* __restrict__ cursors,
-                                                     unsigned* sStage, unsigned short* sBucketOf, int* sHist,
-                                                     int* sLocalBase, long long* sGlobalBase, unsigned& maxAdjBits,
-                                                     float (&adjPos)[D], const DerivativeChunk* __restrict__ derivatives)
+    template <int LEVEL, int END, typename... Args>
+    __device__ __forceinline__ static void runLevels(Args&&... args)
     {
         if constexpr (LEVEL < END) {
-            runLevel<LEVEL, INPUT_GRADIENTS>(p, valid, numel, pos, adjEncoded, params, records, cursors, sStage, sBucketOf, sHist,
-                                             sLocalBase, sGlobalBase, maxAdjBits, adjPos, derivatives);
-            runLevels<LEVEL + 1, END, INPUT_GRADIENTS>(p, valid, numel, pos, adjEncoded, params, records, cursors, sStage, sBucketOf,
-                                                  sHist, sLocalBase, sGlobalBase, maxAdjBits, adjPos, derivatives);
+            runLevel<LEVEL>(args...);
+            runLevels<LEVEL + 1, END>(args...);
         }
     }
 
     /** The levels of one of GROUPS groups. */
-    template <int G, int GROUPS, int INPUT_GRADIENTS, typename... Args>
+    template <int G, int GROUPS, typename... Args>
     __device__ __forceinline__ static void runGroup(int group, Args&&... args)
     {
         if constexpr (G + 1 < GROUPS) {
-            if (group == G) runLevels<Cfg::Levels * G / GROUPS, Cfg::Levels * (G + 1) / GROUPS, INPUT_GRADIENTS>(args...);
-            else runGroup<G + 1, GROUPS, INPUT_GRADIENTS>(group, args...);
+            if (group == G) runLevels<Cfg::Levels * G / GROUPS, Cfg::Levels * (G + 1) / GROUPS>(args...);
+            else runGroup<G + 1, GROUPS>(group, args...);
         } else {
-            runLevels<Cfg::Levels * G / GROUPS, Cfg::Levels, INPUT_GRADIENTS>(args...);
+            runLevels<Cfg::Levels * G / GROUPS, Cfg::Levels>(args...);
+        }
+    }
+
+    /** The gradient of a point with respect to its position: from the entries of all corners or from stored derivatives. */
+    template <int LEVEL, int INPUT_GRADIENTS>
+    __device__ __forceinline__ static void positionGradients(int p, const float (&position)[D], const Adjoints& adjEncoded, const param_t& params,
+                                                             const DerivativeChunk* __restrict__ derivatives, float (&adjPos)[D])
+    {
+        if constexpr (LEVEL < Cfg::Levels) {
+            // (the entries of one level in registers at a time; of the derivatives four)
+            float pos[D];
+#pragma unroll
+            for (int d = 0; d < D; ++d) pos[d] = position[d];
+            if (INPUT_GRADIENTS == 1 || LEVEL % 4 == 0) {
+                asm volatile("" : "+v"(p));
+#pragma unroll
+                for (int d = 0; d < D; ++d) asm volatile("" : "+v"(pos[d]), "+v"(adjPos[d]));
+            }
+            if constexpr (INPUT_GRADIENTS == 2) {
+                positionGradientFromDerivatives<LEVEL>(p, derivatives, adjEncoded, adjPos);
+            } else {
+                const typename Grid::LevelSetup s = Grid::setupLevel(LEVEL, pos);
+                detail::HeldFeatures<F, typename Cfg::table_t> held[Grid::NC];
+                loadHeld<LEVEL>(s, params, held);
+                positionGradient<LEVEL>(p, s, held, adjEncoded, adjPos);
+            }
+            positionGradients<LEVEL + 1, INPUT_GRADIENTS>(p, pos, adjEncoded, params, derivatives, adjPos);
+        }
+    }
+
+    __device__ __forceinline__ static void loadPosition(const Tensor2Read<float>& inputs, int p, const param_t& params, float (&pos)[D])
+    {
+#pragma clang fp contract(off)
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const float in = inputs.data_[static_cast<long long>(p) * inputs.strides_[0] + static_cast<long long>(d + Cfg::Start) * inputs.strides_[1]];
+            pos[d] = (in - params.boundingBoxMin[d]) * params.boundingBoxInvSize[d];
+        }
+    }
+
+    /** Zeroes the elements of the gradient tensor that the slice kernel adds to with atomics; index: of the thread. */
+    template <int LEVEL>
+    __device__ __forceinline__ static void zeroShared(int index, int threads, float* __restrict__ gradients)
+    {
+        if constexpr (LEVEL < Cfg::Levels) {
+            constexpr int SLICES = Layout::numSlices(LEVEL);
+            constexpr bool WHOLE = Layout::parts(LEVEL) > 1;
+            constexpr int COUNT = WHOLE ? Layout::levelFloats(LEVEL) : (SLICES - 1) * F;   // (the first entry of every slice but the first)
+            float* __restrict__ level = gradients + Cfg::memoryOffset[LEVEL];
+            for (int i = index; i < COUNT; i += threads) level[WHOLE ? i : (i / F + 1) * SLICE_FLOATS + i % F] = 0.f;
+            zeroShared<LEVEL + 1>(index, threads, gradients);
+        }
+    }
+
+    /** Adds one entry of GridGradientWorkspace::exceptions to the gradient tensor. */
+    template <int LEVEL>
+    __device__ __forceinline__ static void addException(unsigned exception, int firstPoint, const Tensor2Read<float>& inputs,
+                                                        const Adjoints& adjEncoded, const param_t& params)
+    {
+        constexpr int PD = Cfg::hashed[LEVEL] ? 0 : D - 1;
+        const int p = firstPoint + static_cast<int>(exception & ((1u << EXCEPTION_PAIR_SHIFT) - 1u));
+        const int c = static_cast<int>(exception >> EXCEPTION_PAIR_SHIFT) & 7;
+        float pos[D];
+        loadPosition(inputs, p, params, pos);
+        const typename Grid::LevelSetup s = Grid::setupLevel(LEVEL, pos);
+        unsigned idxL, idxH;
+        float w;
+        pairEntries<LEVEL>(s, c, idxL, idxH, w);
+        const float wL = w * (1.f - s.f[PD]), wH = w * s.f[PD];
+        float* __restrict__ grad = params.parametersBackward + Cfg::memoryOffset[LEVEL];
+#pragma unroll 1
+        for (int i = 0; i < F; ++i) {
+            const float adj = static_cast<float>(adjEncoded(p, channel<LEVEL>(i)));
+            if (!(exception & EXCEPTION_UPPER_ONLY)) unsafeAtomicAdd(grad + idxL * F + i, wL * adj);
+            unsafeAtomicAdd(grad + idxH * F + i, wH * adj);
         }
     }
 };
 
 /**
- * \tparam GROUPS the levels are shared out over so many workgroups (the grid is a multiple of it) where each of them
- *    needs nothing of the others (no input gradients)
+ * \tparam GROUPS the levels are shared out over so many workgroups; with INPUT_GRADIENTS another one computes those
  * \tparam POINTS points (= lanes) of a workgroup; its records of one level are staged in LDS
- * records: room for levelOffset(Levels, layoutNumel) records; cursors: one int per bucket, then one word that
- * receives the largest magnitude among the adjoints (bits without the sign); all zeroed by the caller.
  * \tparam ROW_CHANNELS, CHANNEL_OFFSET where the adjoints of this grid lie, see GridGradientAdjoints
+ * Launched with a multiple of GROUPS (+ 1) workgroups; their number / (GROUPS + 1) * GROUPS is workspace.largestCount.
  */
 template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS, int POINTS, int INPUT_GRADIENTS, int GROUPS>
-__global__ void __launch_bounds__(POINTS) GridGradientRecordsKernel(
+__global__ void __launch_bounds__(POINTS) __attribute__((amdgpu_waves_per_eu(GridGradientRecords<Cfg, ROW_CHANNELS, CHANNEL_OFFSET, SLICE_FLOATS, POINTS>::template wavesPerSimd<INPUT_GRADIENTS>())))
+GridGradientRecordsKernel(
     int numel,
-    int layoutNumel,                          //points the buckets are laid out for (numel rounded up to whole tiles)
     const Tensor2Read<float> inputs,          //shape (numel, Cin)
     const GridGradientAdjoints<ROW_CHANNELS> adjEncoded,
     const HashGridParams<typename Cfg::table_t, Cfg::Dim> params,
-    unsigned* __restrict__ records, int* __restrict__ cursors,
+    const GridGradientWorkspace workspace,
+    int overwrite,                            //the gradient tensor holds nothing yet
     Tensor2RW<float> adjInputs,               //INPUT_GRADIENTS: shape (numel, Cin), this grid's share of dL/dinput is added
+    int overwriteInput,                       //... or written
     const void* __restrict__ derivativesV)    //INPUT_GRADIENTS == 2: the position derivatives of this grid that the forward pass stored
 {
     typedef GridGradientRecords<Cfg, ROW_CHANNELS, CHANNEL_OFFSET, SLICE_FLOATS, POINTS> Impl;
     constexpr int D = Cfg::Dim;
+    constexpr int WORKGROUPS = GROUPS + (INPUT_GRADIENTS != 0 ? 1 : 0);   // of a region
     extern __shared__ __align__(16) unsigned char sMemory[];
-    unsigned* sStage = reinterpret_cast<unsigned*>(sMemory);                               // POINTS * PAIRS records
-    long long* sGlobalBase = reinterpret_cast<long long*>(sStage + POINTS * Impl::PAIRS * Impl::RW);
-    int* sHist = reinterpret_cast<int*>(sGlobalBase + Impl::MAX_SLICES);
-    int* sLocalBase = sHist + Impl::MAX_SLICES;
-    unsigned short* sBucketOf = reinterpret_cast<unsigned short*>(sLocalBase + Impl::MAX_SLICES + 1);
-    unsigned maxAdjBits = 0u;
-    const int group = blockIdx.x % GROUPS;
-    for (int chunk = blockIdx.x / GROUPS * POINTS; chunk < numel; chunk += gridDim.x / GROUPS * POINTS) {
-        const int p = chunk + threadIdx.x;
-        const bool valid = p < numel;
-        float pos[D];
-        {
-#pragma clang fp contract(off)
+    unsigned* sStage = reinterpret_cast<unsigned*>(sMemory);              // POINTS * PAIRS records
+    int* sCount = reinterpret_cast<int*>(sStage + POINTS * Impl::PAIRS * Impl::RW);
+    int* sStart = sCount + Impl::MAX_SLICES + 1;
+    // (by few workgroups: the others only pass by)
+    constexpr int ZEROING = 64;
+    if (overwrite && blockIdx.x < ZEROING)
+        Impl::template zeroShared<0>(blockIdx.x * POINTS + threadIdx.x, min(ZEROING, static_cast<int>(gridDim.x)) * POINTS, params.parametersBackward);
+    // Adjoints in rows: a row holds all levels, so that the groups follow one another and every die finds the rows of its
+    // regions in its L2 again (16 levels, 2^17 points: 44 us, 62 with the groups of a region side by side). Adjoints of
+    // tiles: nothing is shared, and the slice kernel reads what lies in memory region by region faster (2^18 points: 82 and
+    // 84 us, 90 and 95 with the groups one behind the other).
+    const int step = gridDim.x / WORKGROUPS;
+    const int group = Impl::FLOATS ? blockIdx.x / step : blockIdx.x % WORKGROUPS, first = Impl::FLOATS ? blockIdx.x % step : blockIdx.x / WORKGROUPS;
+    if constexpr (INPUT_GRADIENTS != 0) {
+        if (group == GROUPS) {
+            for (int p = first * POINTS + threadIdx.x; p < numel; p += step * POINTS) {
+                float pos[D], adjPos[D];
+                Impl::loadPosition(inputs, p, params, pos);
 #pragma unroll
-            for (int d = 0; d < D; ++d) {
-                const float in = valid ? inputs.data_[static_cast<long long>(p) * inputs.strides_[0]
-                                                      + static_cast<long long>(d + Cfg::Start) * inputs.strides_[1]] : 0.f;
-                pos[d] = (in - params.boundingBoxMin[d]) * params.boundingBoxInvSize[d];
+                for (int d = 0; d < D; ++d) adjPos[d] = 0.f;
+                Impl::template positionGradients<0, INPUT_GRADIENTS>(p, pos, adjEncoded, params,
+                                                                     static_cast<const typename Impl::DerivativeChunk*>(derivativesV), adjPos);
+                // every point belongs to one lane of one workgroup: a plain read-modify-write
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    float* adj = adjInputs.data_ + (static_cast<long long>(p) * adjInputs.strides_[0]
+                                                    + static_cast<long long>(d + Cfg::Start) * adjInputs.strides_[1]);
+                    const float before = overwriteInput ? 0.f : *adj;
+                    *adj = before + adjPos[d] * params.boundingBoxInvSize[d];
+                }
             }
+            return;
         }
-        float adjPos[D];
-#pragma unroll
-        for (int d = 0; d < D; ++d) adjPos[d] = 0.f;
-        Impl::template runGroup<0, GROUPS, INPUT_GRADIENTS>(group, p, valid, layoutNumel, pos, adjEncoded, params,
-                                                     records, cursors, sStage, sBucketOf, sHist, sLocalBase, sGlobalBase, maxAdjBits,
-                                                     adjPos, static_cast<const typename Impl::DerivativeChunk*>(derivativesV));
-        if constexpr (INPUT_GRADIENTS != 0) {
-            // every point belongs to one lane of one workgroup: a plain read-modify-write
-            if (valid) {
-#pragma unroll
-                for (int d = 0; d < D; ++d)
-                    adjInputs.data_[static_cast<long long>(p) * adjInputs.strides_[0]
-                                    + static_cast<long long>(d + Cfg::Start) * adjInputs.strides_[1]] += adjPos[d] * params.boundingBoxInvSize[d];
-            }
-        }
-        ldsBarrier();
     }
-    // the largest adjoint of the workgroup: one LDS word, then one atomic per workgroup
-    if (threadIdx.x == 0) sHist[0] = 0;
+    unsigned maxAdjBits = 0u;
+    for (int b = threadIdx.x; b <= Impl::MAX_SLICES; b += POINTS) sCount[b] = 0;
+    ldsBarrier();
+    for (int region = first; region < workspace.regions; region += step) {
+        const int p = region * POINTS + threadIdx.x;
+        float pos[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) pos[d] = 0.f;
+        if (p < numel) Impl::loadPosition(inputs, p, params, pos);
+        Impl::template runGroup<0, GROUPS>(group, p, numel, region, pos, adjEncoded, workspace, sStage, sCount, sStart, maxAdjBits);
+    }
+    // the largest adjoint of the workgroup
+    if (maxAdjBits != 0u) atomicMax(sCount, static_cast<int>(maxAdjBits));
     __syncthreads();
-    if (maxAdjBits != 0u) atomicMax(sHist, static_cast<int>(maxAdjBits));
-    __syncthreads();
-    if (threadIdx.x == 0 && sHist[0] != 0)
-        atomicMax(cursors + Impl::Layout::firstBucket(Cfg::Levels), sHist[0]);
+    if (threadIdx.x == 0) workspace.largest[first * GROUPS + group] = static_cast<unsigned>(sCount[0]);
 }
 
-/** Zeroes the fill of the buckets and the largest adjoint. */
-__global__ void __launch_bounds__(256) GridGradientClearKernel(int* __restrict__ words, int count)
+template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS, int LEVEL>
+struct GridGradientExceptions
 {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < count) words[i] = 0;
+    typedef GridGradientRecords<Cfg, ROW_CHANNELS, CHANNEL_OFFSET, SLICE_FLOATS, 1024> Records;
+    typedef typename Records::Layout Layout;
+    /** The exceptions of a region from LEVEL on; counts: those of every level in the lanes of the wavefront. */
+    __device__ __forceinline__ static void run(int region, unsigned long long levels, const Tensor2Read<float>& inputs,
+                                               const typename Records::Adjoints& adjEncoded, const typename Records::param_t& params,
+                                               const GridGradientWorkspace& ws)
+    {
+        if constexpr (LEVEL < Cfg::Levels) {
+            if (levels >> (LEVEL % 64) & 1) {
+                const int count = ws.places[static_cast<long long>(region) * Layout::PLACES + Layout::firstPlace(LEVEL) + Layout::numSlices(LEVEL) + 1];
+                const unsigned short* from = ws.exceptions + (static_cast<long long>(LEVEL) * ws.regions + region) * ws.recordsPerRegion;
+                for (int i = threadIdx.x; i < count; i += 64)
+                    Records::template addException<LEVEL>(from[i], region * (ws.recordsPerRegion / Records::PAIRS), inputs, adjEncoded, params);
+            }
+            GridGradientExceptions<Cfg, ROW_CHANNELS, CHANNEL_OFFSET, SLICE_FLOATS, LEVEL + 1>::run(region, levels, inputs, adjEncoded, params, ws);
+        }
+    }
+};
+
+/**
+ * What the records leave out, added to the gradient tensor with atomics behind the slice kernel: one wavefront per region.
+ * Few batches have any: upper entries beyond the end of a slice (in a dense level one pair in thousands), and points
+ * outside of the box. A launch that finds none takes 2 to 3 us.
+ */
+template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS>
+__global__ void __launch_bounds__(64) GridGradientExceptionsKernel(
+    const Tensor2Read<float> inputs, const GridGradientAdjoints<ROW_CHANNELS> adjEncoded,
+    const HashGridParams<typename Cfg::table_t, Cfg::Dim> params, const GridGradientWorkspace workspace)
+{
+    typedef GridGradientExceptions<Cfg, ROW_CHANNELS, CHANNEL_OFFSET, SLICE_FLOATS, 0> Impl;
+    typedef typename Impl::Layout Layout;
+    const int lane = threadIdx.x;
+    for (int region = blockIdx.x; region < workspace.regions; region += gridDim.x) {
+        // (a lane per level; bit l % 64: some level with that remainder has exceptions)
+        bool any = false;
+#pragma unroll
+        for (int l0 = 0; l0 < Cfg::Levels; l0 += 64) {
+            int place = 0;
+#pragma unroll
+            for (int l = l0; l < Cfg::Levels && l < l0 + 64; ++l)
+                if (lane == l - l0) place = Layout::firstPlace(l) + Layout::numSlices(l) + 1;
+            if (lane < Cfg::Levels - l0) any = any || workspace.places[static_cast<long long>(region) * Layout::PLACES + place] != 0;
+        }
+        const unsigned long long levels = __ballot(any);
+        if (levels != 0) Impl::run(region, levels, inputs, adjEncoded, params, workspace);
+    }
 }
 
 template <typename Cfg, int SLICE_FLOATS, int LEVEL>
@@ -771,7 +841,7 @@ struct GridGradientTraceLevels
 
 /**
  * Test aid: for every point (one per lane) and level, the table elements and weights that the records of
- * GridGradientRecords::buildRecord stand for, decoded as the slice kernel decodes them (slice of the bucket +
+ * GridGradientRecords::buildRecord stand for, decoded as the slice kernel decodes them (its slice +
  * 16-bit offset), and the entries the records kernel adds itself because they lie in another slice.
  * Slots as in CornerTrace: level * 2^Dim + 2 * pair (+ 1 for the upper entry).
  */
@@ -812,22 +882,16 @@ struct GridGradientSlices
     static constexpr int RW = Layout::RECORD_WORDS;
     static constexpr int BLOCK = 1024;
 
-    /** v * 2^scaleExponent as a 64-bit integer, rounded towards minus infinity in the low word (|v * 2^scaleExponent| < 2^62). */
-    __device__ __forceinline__ static long long toFixed(float v, int scaleExponent)
+    /**
+     * v * 2^scaleExponent as a 64-bit integer (scale: that power of two; |v * scale| < 2^51), rounded to nearest: the
+     * sum with 1.5 * 2^52 has the integer in the low bits of its mantissa. Three instructions, two of them in double
+     * precision; split into two words in single precision it takes nine.
+     */
+    static constexpr int FIXED_BITS = 51;
+    __device__ __forceinline__ static long long toFixed(float v, double scale)
     {
-        if constexpr (FLOATS) {
-            // by magnitude: no bit of a float of 2^23 units or more is lost
-            const float magnitude = ldexpf(fabsf(v), scaleExponent - 32);
-            const float whole = floorf(magnitude);
-            const long long fixed = (static_cast<long long>(static_cast<int>(whole)) << 32)
-                + static_cast<long long>(static_cast<unsigned>(ldexpf(magnitude - whole, 32)));
-            return v < 0.f ? -fixed : fixed;
-        }
-        const float x = ldexpf(v, scaleExponent - 32);             // in units of 2^32
-        const float hi = floorf(x);
-        // the low bits of a 24-bit mantissa: exact, in [0, 2^32) (a tiny negative x gives hi = -1 and x - hi = 1 after rounding)
-        const float lo = fminf(ldexpf(x - hi, 32), 4294967040.f);
-        return (static_cast<long long>(static_cast<int>(hi)) << 32) + static_cast<long long>(static_cast<unsigned>(lo));
+        const double shifted = __builtin_fma(static_cast<double>(v), scale, 6755399441055744.0);
+        return __builtin_bit_cast(long long, shifted) - 0x4338000000000000ll;
     }
 
     __device__ __forceinline__ static void ldsAddFixed(long long* p, long long v)
@@ -836,155 +900,237 @@ struct GridGradientSlices
         __hip_atomic_fetch_add((lds_u64*)p, static_cast<unsigned long long>(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
 
-    /** Floats span more than the 64 bits of a sum: a value of which the sum would lose bits goes to the gradient tensor. */
-    __device__ __forceinline__ static void addFixedOrSmall(long long* sum, float* __restrict__ gradient, float v, int scaleExponent, float smallest)
+    /** Two workgroups per compute unit where the LDS has room for two. */
+    static constexpr int WAVES_PER_SIMD = SLICE_FLOATS <= 8192 && RW <= 4 ? 8 : 4;
+
+    /** Sums of a slice and of the entry behind it. */
+    static constexpr int SUMS = SLICE_FLOATS + F;
+    /** What the workgroup keeps in LDS beside the sums. */
+    static constexpr int SEGMENTS = BLOCK;      // regions that are looked up together
+    static constexpr int WAVES = BLOCK / 64;
+    static constexpr int SMALL = FLOATS ? 256 : 0;
+    struct Shared
     {
-        if (fabsf(v) >= smallest) ldsAddFixed(sum, toFixed(v, scaleExponent));
-        else if (v != 0.f) unsafeAtomicAdd(gradient, v);
+        unsigned segments[SEGMENTS];            // where the records of the slice begin and end in each region (16 bits each)
+        unsigned largest[WAVES];
+        int records[WAVES];
+        int smallCount;
+        float smallValues[SMALL + 1];
+        unsigned short smallElements[SMALL + 1];
+    };
+
+    /** Where the records of the slice begin and end in a region. */
+    __device__ __forceinline__ static unsigned segmentOf(const GridGradientWorkspace& ws, const GridGradientSlice& item, int region)
+    {
+        const unsigned short* place = ws.places + static_cast<long long>(region) * Layout::PLACES + item.place;
+        return place[0] | (static_cast<unsigned>(place[1]) << 16);
     }
 
-    /** FIXED: 64-bit fixed-point sums (the slice is SLICE_FLOATS long long); else float sums. */
-    template <int LEVEL, bool FIXED>
-    __device__ __forceinline__ static void sumRecords(long long numel, const unsigned* __restrict__ records,
-                                                      const int* __restrict__ cursors, float* __restrict__ gradients,
-                                                      const GridGradientSlice item, long long* sFixed, float* sFloat,
-                                                      int scaleExponent)
+    /**
+     * Calls add(record) for the records of a work item. The records of a slice lie in segments, one per region, of
+     * recordsPerRegion / (slices of the level) records where the points are spread evenly: groups of half as many lanes
+     * (8 to all of them) take a segment each, three records per lane at a time, of several segments. shared.segments holds
+     * the first SEGMENTS regions.
+     */
+    template <typename Add>
+    __device__ __forceinline__ static void forEachRecord(const GridGradientWorkspace& ws, const GridGradientSlice& item, int begin, int end,
+                                                         Shared& shared, const Add& add)
     {
         const int tid = threadIdx.x;
-        const long long capacity = Layout::capacity(LEVEL, numel);
-        const long long filled = min(static_cast<long long>(cursors[Layout::firstBucket(LEVEL) + item.slice]), capacity);
-        const long long begin = filled * item.part / item.parts, end = filled * (item.part + 1) / item.parts;
-        const unsigned* bucket = records + (Layout::levelOffset(LEVEL, numel) + static_cast<long long>(item.slice) * capacity) * RW;
-        constexpr int UNROLL = 4;
-        // (the smallest magnitude of which the fixed-point sums keep all bits of a float)
-        const float smallest = ldexpf(1.f, 23 - scaleExponent);
-        (void)smallest;
-        for (long long j0 = begin + tid; j0 < end; j0 += UNROLL * BLOCK) {
-            unsigned rec[UNROLL][RW];
-#pragma unroll
-            for (int u = 0; u < UNROLL; ++u) {
-                const long long j = j0 + u * BLOCK;
-                if (j < end) {
-                    Layout::loadRecord(bucket + j * RW, rec[u]);
-                } else {
-#pragma unroll
-                    for (int v = 0; v < RW; ++v) rec[u][v] = 0u;
-                }
+        int groupLog2 = 3;
+        while (groupLog2 < 10 && (4 << groupLog2) * item.slices <= ws.recordsPerRegion) ++groupLog2;
+        const int group = tid >> groupLog2, groups = BLOCK >> groupLog2, lanes = 1 << groupLog2, lane = tid & (lanes - 1);
+        constexpr int UNROLL = 2, STEPS = 3;
+        for (int r0 = begin; r0 < end; r0 += SEGMENTS) {
+            const int count = min(SEGMENTS, end - r0);
+            if (r0 != begin) {
+                __syncthreads();   // the segments in front of these have been read
+                if (tid < count) shared.segments[tid] = segmentOf(ws, item, r0 + tid);
+                __syncthreads();
             }
+            const unsigned* first = ws.records + (static_cast<long long>(item.level) * ws.regions + r0) * ws.recordsPerRegion * RW;
+            for (int s0 = group; s0 < count; s0 += UNROLL * groups) {
+                unsigned rec[UNROLL][STEPS][RW];
+                int size[UNROLL];
+                unsigned segment[UNROLL];   // (in words; a thousand regions take less than 2^27)
 #pragma unroll
-            for (int u = 0; u < UNROLL; ++u) {
-                if (j0 + u * BLOCK >= end) continue;
-                const unsigned eL = rec[u][0] & 0xffffu, eH = rec[u][0] >> 16;   // both inside this slice
-                float wL, wH;
-                Layout::weights(rec[u], wL, wH);
+                for (int u = 0; u < UNROLL; ++u) {
+                    const int s = s0 + u * groups;
+                    const unsigned places = s < count ? shared.segments[s] : 0u;
+                    size[u] = static_cast<int>(places >> 16) - static_cast<int>(places & 0xffffu);
+                    segment[u] = (static_cast<unsigned>(s) * static_cast<unsigned>(ws.recordsPerRegion) + (places & 0xffffu)) * RW;
 #pragma unroll
-                for (int step = 0; step < F; ++step) {
-                    // Neighbouring lanes take the features in rotated order: an entry starts at a multiple of
-                    // 8 * F bytes, so lanes that all add feature `step` meet on a few LDS banks (measured on a
-                    // dense grid with 8 features: conflicts 90 % of the LDS cycles of this kernel).
-                    const int i = (F & (F - 1)) == 0 ? ((step + tid) & (F - 1)) : ((step + tid % F) % F);
-                    unsigned word = rec[u][Layout::FIRST_ADJOINT];
-                    const int at = FLOATS ? i : i >> 1;
+                    for (int k = 0; k < STEPS; ++k)
+                        if (lane + k * lanes < size[u]) Layout::loadRecord(first + (segment[u] + static_cast<unsigned>((lane + k * lanes) * RW)), rec[u][k]);
+                }
 #pragma unroll
-                    for (int w = 1; w < Layout::ADJOINT_WORDS; ++w) word = at == w ? rec[u][Layout::FIRST_ADJOINT + w] : word;
-                    const float adj = FLOATS ? __builtin_bit_cast(float, word)
-                        : static_cast<float>(__builtin_bit_cast(f16, static_cast<unsigned short>(word >> (16 * (i & 1)))));
-                    if constexpr (FIXED && FLOATS) {
-                        addFixedOrSmall(sFixed + eL + i, gradients + item.first + eL + i, wL * adj, scaleExponent, smallest);
-                        addFixedOrSmall(sFixed + eH + i, gradients + item.first + eH + i, wH * adj, scaleExponent, smallest);
-                    } else if constexpr (FIXED) {
-                        ldsAddFixed(sFixed + eL + i, toFixed(wL * adj, scaleExponent));
-                        ldsAddFixed(sFixed + eH + i, toFixed(wH * adj, scaleExponent));
-                    } else {
-                        Grid::ldsAdd(sFloat + eL + i, wL * adj);
-                        Grid::ldsAdd(sFloat + eH + i, wH * adj);
+                for (int u = 0; u < UNROLL; ++u) {
+#pragma unroll
+                    for (int k = 0; k < STEPS; ++k)
+                        if (lane + k * lanes < size[u]) add(rec[u][k]);
+                    for (int j = lane + STEPS * lanes; j < size[u]; j += lanes) {   // points that are not spread evenly
+                        Layout::loadRecord(first + (segment[u] + static_cast<unsigned>(j * RW)), rec[u][0]);
+                        add(rec[u][0]);
                     }
                 }
             }
         }
     }
 
-    /**
-     * Terms of at most the largest adjoint that one sum may take. Halves: those of the whole batch, so that a slice
-     * gives the same bits however its bucket is split. Floats need the bits below more: the records of this work item
-     * (the two weights of a record make at most one).
-     */
-    template <int LEVEL>
-    __device__ __forceinline__ static unsigned long long termsOf(long long numel, const int* __restrict__ cursors, const GridGradientSlice item)
-    {
-        if constexpr (FLOATS)
-            return static_cast<unsigned long long>(min(static_cast<long long>(cursors[Layout::firstBucket(LEVEL) + item.slice]),
-                                                       Layout::capacity(LEVEL, numel)) / item.parts + 1);
-        else return static_cast<unsigned long long>(2 * Layout::PAIRS) * static_cast<unsigned long long>(numel);
-    }
-
-    template <int LEVEL>
-    __device__ __forceinline__ static void runLevel(long long numel, const unsigned* __restrict__ records,
-                                                    const int* __restrict__ cursors, float* __restrict__ gradients,
-                                                    const GridGradientSlice item, long long* sSlice)
+    /** Calls term(element, value) for the terms of a record. */
+    template <typename Term>
+    __device__ __forceinline__ static void forEachTerm(const unsigned (&rec)[RW], const Term& term)
     {
         const int tid = threadIdx.x;
-        for (int i = tid; i < item.floats; i += BLOCK) sSlice[i] = 0;
-        __syncthreads();
-        // |adjoint| < 2^maxExponent; a sum has at most 2 * PAIRS * numel terms, each at most that large (weights <= 1)
-        const unsigned maxBits = static_cast<unsigned>(cursors[Layout::firstBucket(Cfg::Levels)]);
-        if (maxBits == 0u) return;   // all adjoints are zero: nothing to add
-        const bool finite = maxBits < (FLOATS ? 0x7f800000u : 0x7c00u);
-        // value < 2^(biased exponent - 14) of halves, 2^(biased exponent - 126) of floats, subnormals included
-        const int maxExponent = FLOATS ? static_cast<int>(maxBits >> 23) - 126 : static_cast<int>(maxBits >> 10) - 14;
-        const int termsLog2 = 64 - __builtin_clzll(termsOf<LEVEL>(numel, cursors, item));
-        const int scaleExponent = 61 - maxExponent - termsLog2;
-        float* sFloat = reinterpret_cast<float*>(sSlice);
-        if (finite) sumRecords<LEVEL, true>(numel, records, cursors, gradients, item, sSlice, sFloat, scaleExponent);
-        else sumRecords<LEVEL, false>(numel, records, cursors, gradients, item, sSlice, sFloat, 0);
-        if constexpr (FLOATS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's atomics have been carried out
-        __syncthreads();
-        // Added to the gradient tensor: with atomics (16 neighbouring floats per request) where other work
-        // items hold sums for the same slice (parts > 1), else this workgroup is the only writer of its
-        // slice in this launch (contributions to entries of other slices were added by the records kernel).
-        float* __restrict__ grad = gradients + item.first;
-        for (int i = tid; i < item.floats; i += BLOCK) {
-            float v;
-            if (finite) {
-                const long long fixed = sSlice[i];
-                v = static_cast<float>(ldexp(static_cast<double>(fixed), -scaleExponent));
-            } else {
-                v = sFloat[i];
-            }
-            if (v != 0.f) {
-                if (item.parts > 1) {
-                    unsafeAtomicAdd(grad + i, v);
-                } else if constexpr (FLOATS) {
-                    // (read behind this workgroup's own atomics: they have ended, but the L1 does not know of them)
-                    grad[i] = __hip_atomic_load(grad + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + v;
-                } else {
-                    grad[i] += v;
-                }
-            }
+        const unsigned eL = rec[0] & 0xffffu, eH = rec[0] >> 16;   // both inside this slice
+        float wL, wH;
+        Layout::weights(rec, wL, wH);
+#pragma unroll
+        for (int step = 0; step < F; ++step) {
+            // Neighbouring lanes take the features in rotated order: an entry starts at a multiple of
+            // 8 * F bytes, so lanes that all add feature `step` meet on a few LDS banks (measured on a
+            // dense grid with 8 features: conflicts 90 % of the LDS cycles of this kernel).
+            const int i = (F & (F - 1)) == 0 ? ((step + tid) & (F - 1)) : ((step + tid % F) % F);
+            unsigned word = rec[Layout::FIRST_ADJOINT];
+            const int at = FLOATS ? i : i >> 1;
+#pragma unroll
+            for (int w = 1; w < Layout::ADJOINT_WORDS; ++w) word = at == w ? rec[Layout::FIRST_ADJOINT + w] : word;
+            const float adj = FLOATS ? __builtin_bit_cast(float, word)
+                : static_cast<float>(__builtin_bit_cast(f16, static_cast<unsigned short>(word >> (16 * (i & 1)))));
+            term(eL + i, wL * adj);
+            term(eH + i, wH * adj);
         }
     }
 
-    template <int LEVEL>
-    __device__ __forceinline__ static void dispatch(long long numel, const unsigned* __restrict__ records,
-                                                    const int* __restrict__ cursors, float* __restrict__ gradients,
-                                                    const GridGradientSlice item, long long* sSlice)
+    /** \param overwrite the elements of the slice are written, whatever is there; those that others add to as well are zero */
+    __device__ __forceinline__ static void run(int numel, const GridGradientWorkspace& ws, float* __restrict__ gradients,
+                                               const GridGradientSlice item, int overwrite, long long* sSlice, Shared& shared)
     {
-        if constexpr (LEVEL < Cfg::Levels) {
-            if (item.level == LEVEL) runLevel<LEVEL>(numel, records, cursors, gradients, item, sSlice);
-            else dispatch<LEVEL + 1>(numel, records, cursors, gradients, item, sSlice);
+        const int tid = threadIdx.x;
+        const int begin = static_cast<int>(static_cast<long long>(ws.regions) * item.part / item.parts);
+        const int end = static_cast<int>(static_cast<long long>(ws.regions) * (item.part + 1) / item.parts);
+        // everything that has to be looked up first, in flight while the sums are zeroed
+        const unsigned segment = tid < min(SEGMENTS, end - begin) ? segmentOf(ws, item, begin + tid) : 0u;
+        unsigned largest = 0u;
+        for (int i = tid; i < ws.largestCount; i += BLOCK) largest = max(largest, ws.largest[i]);
+        const int sums = item.floats < SLICE_FLOATS ? item.floats : SUMS;
+        for (int i = tid; i < sums; i += BLOCK) sSlice[i] = 0;
+        int records = 0;
+        if constexpr (FLOATS) {
+            records = static_cast<int>(segment >> 16) - static_cast<int>(segment & 0xffffu);
+            for (int r = begin + SEGMENTS + tid; r < end; r += BLOCK) {
+                const unsigned s = segmentOf(ws, item, r);
+                records += static_cast<int>(s >> 16) - static_cast<int>(s & 0xffffu);
+            }
+        }
+#pragma unroll
+        for (int d = 32; d > 0; d /= 2) {
+            largest = max(largest, static_cast<unsigned>(__shfl_xor(static_cast<int>(largest), d, 64)));
+            if constexpr (FLOATS) records += __shfl_xor(records, d, 64);
+        }
+        shared.segments[tid] = segment;
+        if (tid % 64 == 0) {
+            shared.largest[tid / 64] = largest;
+            if constexpr (FLOATS) shared.records[tid / 64] = records;
+        }
+        if (tid == 0) shared.smallCount = 0;
+        __syncthreads();
+        unsigned maxBits = 0u;
+        int allRecords = 0;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            maxBits = max(maxBits, shared.largest[w]);
+            if constexpr (FLOATS) allRecords += shared.records[w];
+        }
+        const bool finite = maxBits < (FLOATS ? 0x7f800000u : 0x7c00u);
+        // |adjoint| < 2^maxExponent: 2^(biased exponent - 14) of halves, 2^(biased exponent - 126) of floats, subnormals included
+        const int maxExponent = FLOATS ? static_cast<int>(maxBits >> 23) - 126 : static_cast<int>(maxBits >> 10) - 14;
+        // Terms of at most the largest adjoint (weights <= 1) that one sum may take. Halves: those of the whole batch, so that
+        // a slice gives the same bits however its records are split. Floats need the bits below more: the records of this
+        // work item (the two weights of a record make at most one).
+        const unsigned long long terms = FLOATS ? static_cast<unsigned long long>(allRecords) + 1ull
+                                                : static_cast<unsigned long long>(2 * Layout::PAIRS) * static_cast<unsigned long long>(numel);
+        const int termsLog2 = 64 - __builtin_clzll(terms);
+        const int scaleExponent = min(61 - termsLog2, FIXED_BITS) - maxExponent;
+        const double scale = ldexp(1.0, scaleExponent), unit = ldexp(1.0, -scaleExponent);
+        float* sFloat = reinterpret_cast<float*>(sSlice);
+        // Floats span more than the 64 bits of a sum: a value of which the sum would lose bits is added to the gradient tensor
+        // behind the sums, from a list, or if that is full by another pass over the records.
+        const float smallest = ldexpf(1.f, 23 - scaleExponent);
+        (void)smallest;
+        if (maxBits == 0u) {
+            // all adjoints are zero: nothing to add
+        } else if (finite) {
+            forEachRecord(ws, item, begin, end, shared, [&](const unsigned (&rec)[RW]) {
+                forEachTerm(rec, [&](unsigned element, float v) {
+                    if constexpr (FLOATS) {
+                        if (fabsf(v) < smallest) {
+                            if (v != 0.f) {
+                                const int at = atomicAdd(&shared.smallCount, 1);
+                                if (at < SMALL) {
+                                    shared.smallValues[at] = v;
+                                    shared.smallElements[at] = static_cast<unsigned short>(element);
+                                }
+                            }
+                            return;
+                        }
+                    }
+                    ldsAddFixed(sSlice + element, toFixed(v, scale));
+                });
+            });
+        } else {
+            forEachRecord(ws, item, begin, end, shared, [&](const unsigned (&rec)[RW]) {
+                forEachTerm(rec, [&](unsigned element, float v) { Grid::ldsAdd(sFloat + element, v); });
+            });
+        }
+        __syncthreads();
+        // Added to the gradient tensor: with atomics (16 neighbouring floats per request) where other work
+        // items hold sums for the same slice (parts > 1), and for the first entry of a slice and the one behind it, to
+        // which two slices add; else this workgroup is the only writer of its slice in this launch.
+        float* __restrict__ grad = gradients + item.first;
+        const int firstOwn = item.parts > 1 ? sums : item.slice > 0 ? F : 0;
+        for (int i = tid; i < sums; i += BLOCK) {
+            const float v = finite ? static_cast<float>(static_cast<double>(sSlice[i]) * unit) : sFloat[i];
+            if (i < firstOwn || i >= SLICE_FLOATS) {
+                if (v != 0.f) unsafeAtomicAdd(grad + i, v);
+            } else if (overwrite) {
+                grad[i] = v;
+            } else if (v != 0.f) {
+                grad[i] += v;
+            }
+        }
+        if constexpr (FLOATS) {
+            const int small = shared.smallCount;
+            if (small == 0) return;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's stores have been carried out
+            __syncthreads();
+            if (small <= SMALL) {
+                if (tid < small) unsafeAtomicAdd(grad + shared.smallElements[tid], shared.smallValues[tid]);
+            } else {
+                if (end - begin > SEGMENTS) {
+                    shared.segments[tid] = segment;
+                    __syncthreads();
+                }
+                forEachRecord(ws, item, begin, end, shared, [&](const unsigned (&rec)[RW]) {
+                    forEachTerm(rec, [&](unsigned element, float v) {
+                        if (fabsf(v) < smallest && v != 0.f) unsafeAtomicAdd(grad + element, v);
+                    });
+                });
+            }
         }
     }
 };
 
-/** One workgroup of 1024 lanes per work item; `items` is indexed by the workgroup; SLICE_FLOATS * 8 bytes of dynamic LDS. */
+/** One workgroup of 1024 lanes per work item; `items` is indexed by the workgroup; (SLICE_FLOATS + Features) * 8 bytes of dynamic LDS. */
 template <typename Cfg, int SLICE_FLOATS, bool FLOATS>
-__global__ void __launch_bounds__(1024) GridGradientSlicesKernel(
-    int numel, const unsigned* __restrict__ records, const int* __restrict__ cursors, float* __restrict__ gradients,
-    const GridGradientSlice* __restrict__ items)
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(GridGradientSlices<Cfg, SLICE_FLOATS, FLOATS>::WAVES_PER_SIMD)))
+GridGradientSlicesKernel(
+    int numel, const GridGradientWorkspace workspace, float* __restrict__ gradients, const GridGradientSlice* __restrict__ items, int overwrite)
 {
+    typedef GridGradientSlices<Cfg, SLICE_FLOATS, FLOATS> Impl;
     extern __shared__ __align__(16) unsigned char sMemory[];
-    GridGradientSlices<Cfg, SLICE_FLOATS, FLOATS>::template dispatch<0>(numel, records, cursors, gradients, items[blockIdx.x],
-                                                                reinterpret_cast<long long*>(sMemory));
+    __shared__ typename Impl::Shared shared;
+    Impl::run(numel, workspace, gradients, items[blockIdx.x], overwrite, reinterpret_cast<long long*>(sMemory), shared);
 }
 
 QUICKMLP_KERNEL_NAMESPACE_END

@@ -361,6 +361,13 @@ int qmlp_network_overwritable_gradients(qmlp_network_t network, int num_elements
     QMLP_API_END
 }
 
+int qmlp_network_overwritable_tables(qmlp_network_t network, int num_elements, int adjoint_flags, int* overwritable)
+{
+    QMLP_API_BEGIN
+    *overwritable = network->network->overwritableTables(num_elements, adjoint_flags) ? 1 : 0;
+    QMLP_API_END
+}
+
 int qmlp_network_adjoint_overwriting(qmlp_network_t network, const qmlp_tensor* input, const qmlp_tensor* adj_output,
                                      int adjoint_flags, int overwrite, const qmlp_tensor* adj_input,
                                      const void* tmp_memory_forward, void* tmp_memory_adjoint, void* stream)
@@ -509,6 +516,17 @@ int qmlp_encoding_adjoint_in(qmlp_encoding_t encoding, const qmlp_tensor* input,
     encoding->encoding->adjoint(wrap(input), wrap(adj_output), adjIn, static_cast<stream_t>(stream),
                                 optionalTensor(parameters_forward), optionalTensor(parameters_gradients),
                                 adjoint_mode, memory);
+    QMLP_API_END
+}
+int qmlp_encoding_adjoint_overwriting(qmlp_encoding_t encoding, const qmlp_tensor* input, const qmlp_tensor* adj_output,
+                                      const qmlp_tensor* adj_input, void* stream, const qmlp_tensor* parameters_forward,
+                                      const qmlp_tensor* parameters_gradients, int adjoint_mode, void* memory)
+{
+    QMLP_API_BEGIN
+    Tensor adjIn = wrap(adj_input);
+    encoding->encoding->adjoint(wrap(input), wrap(adj_output), adjIn, static_cast<stream_t>(stream),
+                                optionalTensor(parameters_forward), optionalTensor(parameters_gradients),
+                                adjoint_mode, memory, true);
     QMLP_API_END
 }
 

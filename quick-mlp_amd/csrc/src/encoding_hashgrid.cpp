@@ -333,12 +333,14 @@ bool EncodingHashGrid::gradientSlices(GradientSliceLayout& layout, bool floatAdj
         largestLevel = std::max(largestLevel, (l + 1 < numLevels_ ? layers_[l + 1].memoryOffset : numParameters_) - layers_[l].memoryOffset);
     const int smallSlice = 8192 / numFeaturesPerLevel_ * numFeaturesPerLevel_;
     const int sliceSums = smallSlice > 0 && divUp(largestLevel, smallSlice) <= 512 ? 8192 : 16384;
-    const int entries = std::min(sliceSums, lds / 8) / numFeaturesPerLevel_;
+    const int entries = std::min(sliceSums, lds / 8 - 1024) / numFeaturesPerLevel_;
     if (entries < 64) return false;
     layout = GradientSliceLayout{};
     layout.sliceFloats = entries * numFeaturesPerLevel_;
     layout.configType = "qmlp::kernel::" + configName();
     layout.pairs = std::max(1, (1 << dimension_) / 2);
+    layout.features = numFeaturesPerLevel_;
+    layout.inputChannels = dimension_;
     // as GridGradientLayout::RECORD_WORDS: two 16-bit offsets, two weights, the adjoint halves (or: one weight, products in float),
     // padded to 16 / 32 bytes
     const int usedWords = floatAdjoints ? 2 + numFeaturesPerLevel_ : 3 + (numFeaturesPerLevel_ + 1) / 2;
@@ -360,7 +362,7 @@ bool EncodingHashGrid::gradientSlices(GradientSliceLayout& layout, bool floatAdj
         layout.derivativeBytesPerPoint = chunks <= 2 ? numLevels_ * chunks * 16 : 0;
     }
     if (layout.recordsLdsBytes(points) > lds) return false;
-    // every level gets about this many work items: the bucket of a slice that holds more than its share is split
+    // every level gets about this many work items: those of a slice of a coarse level share out the regions
     constexpr int ITEMS_PER_LEVEL = 32;
     for (int l = 0; l < numLevels_; ++l) {
         const int begin = layers_[l].memoryOffset;
@@ -369,10 +371,12 @@ bool EncodingHashGrid::gradientSlices(GradientSliceLayout& layout, bool floatAdj
         if (count > 512) return false;   // the records kernel keeps a histogram of 512 slices
         layout.slicesPerLevel.push_back(count);
         const int parts = std::max(1, ITEMS_PER_LEVEL / count);
+        // as GridGradientLayout::firstPlace
+        const int firstPlace = layout.numSlices() - count + 2 * l;
         for (int k = 0; k < count; ++k)
             for (int part = 0; part < parts; ++part)
                 layout.items.push_back({l, static_cast<unsigned>(begin + k * layout.sliceFloats),
-                                        std::min(layout.sliceFloats, end - begin - k * layout.sliceFloats), k, part, parts, 0, 0});
+                                        std::min(layout.sliceFloats, end - begin - k * layout.sliceFloats), k, part, parts, firstPlace + k, count});
     }
     return true;
 }

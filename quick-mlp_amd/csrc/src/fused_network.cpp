@@ -1878,14 +1878,18 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
                     if ((flags & GRADIENTS_INPUT) && sk.derivativeOffset >= 0) compileRecordsKernel(sk, flags, v, true, true);
                 }
             sk.kernel.blockSize = 1024;
-            sk.kernel.sharedMemorySize = layout.sliceFloats * static_cast<int>(sizeof(long long));
-            sk.kernel.fun = kl->getKernel(format("qmlp::kernel::GridGradientSlicesKernel<%s, %d, false>", layout.configType.c_str(), layout.sliceFloats),
-                                          source.str(), loaderFlags(compileOnly)).value();
+            sk.kernel.sharedMemorySize = layout.slicesLdsBytes();
+            const auto kernels = kl->getKernels({format("qmlp::kernel::GridGradientSlicesKernel<%s, %d, false>", layout.configType.c_str(), layout.sliceFloats),
+                                                 format("qmlp::kernel::GridGradientExceptionsKernel<%s, %d, %d, %d>", layout.configType.c_str(),
+                                                        layers_[0].channelsIn, offset, layout.sliceFloats)},
+                                                source.str(), loaderFlags(compileOnly));
             if (!compileOnly) {
+                sk.kernel.fun = kernels.at(0);
+                sk.exceptions = kernels.at(1);
                 static_assert(sizeof(IEncoding::GradientSlice) == 32, "eight 32-bit words, as in kernels/grid_gradient.h");
                 sk.items = Tensor(Tensor::FLOAT, {static_cast<int32_t>(layout.items.size() * 8)});
                 QMLP_HIP_CALL(qmlp_hip_memcpy_h2d(sk.items.rawPtr(), layout.items.data(), layout.items.size() * sizeof(layout.items[0]), nullptr));
-                logger->debug("gradient slices of encoding %d: %d buckets, %d work items", sk.encoding, layout.numBuckets(),
+                logger->debug("gradient slices of encoding %d: %d slices, %d work items", sk.encoding, layout.numSlices(),
                               static_cast<int>(layout.items.size()));
             }
             ak.sliceGradients.push_back(std::move(sk));
@@ -1943,7 +1947,7 @@ void FusedNetwork::compileRecordsKernel(SliceGradientKernel& sk, int flags, size
         // (last argument: no input gradients | from gathers of all corners | from the position derivatives of the forward pass)
         format("qmlp::kernel::GridGradientRecordsKernel<%s, %d, %d, %d, %d, %d, %d>", layout.configType.c_str(), layers_[0].channelsIn,
                sk.channelOffset, layout.sliceFloats, points, !(flags & GRADIENTS_INPUT) ? 0 : fromDerivatives ? 2 : 1,
-               layout.levelGroups(flags & GRADIENTS_INPUT)),
+               layout.levelGroups()),
         sk.recordsSource, loaderFlags(compileOnly)).value();
     if (compileOnly) return;
     ck.fullGrid = ck.fun.fullGridSize(ck.blockSize, ck.sharedMemorySize);
@@ -1998,7 +2002,7 @@ const FusedNetwork::CompiledKernel& FusedNetwork::recordsKernelFor(SliceGradient
     // 2^17 points 0.414 / 0.302 / 0.319 / 0.371, 2^16 points 0.290 / 0.233 / 0.215 / 0.244.
     const int computeUnits = KernelFunction::computeUnits();
     size_t variant = 0;
-    const int groups = sk.layout.levelGroups(flags & GRADIENTS_INPUT);
+    const int groups = sk.layout.levelGroups();
     while (variant + 1 < sk.records.size() && groups * divUp(numel, sk.layout.pointsPerWorkgroup >> variant) < computeUnits) ++variant;
     auto& kernels = fromDerivatives ? sk.recordsFromDerivatives : sk.records;
     if (!kernels[variant].has_value()) compileRecordsKernel(sk, flags, variant, false, fromDerivatives);
@@ -2507,11 +2511,24 @@ FusedNetwork::AdjointModeFlags FusedNetwork::overwritableGradients(int numel, Ad
     if (!(adjointFlags & GRADIENTS_INPUT)) return weights;
     // the rows of a batch that trained in sorted order are moved to the caller's tensor, all of them, at the end
     if (sortsTraining(numel)) return weights | GRADIENTS_INPUT;
+    // the records kernel of the only encoding, a grid over all channels of the input
+    if ((adjointFlags & GRADIENTS_INPUT_ENCODINGS) && useSliceGradients(numel, adjointFlags) && encodings_.size() == 1 && slicesOf(*encodings_[0])
+        && slicesOf(*encodings_[0])->inputChannels == channelsIn())
+        return weights | GRADIENTS_INPUT;
     if (backwardMode(numel, adjointFlags) != BACKWARD_COOPERATIVE) return weights;
     // the cooperative kernel: one that reads the input rows writes the channels of its encoding, else all of them
     const bool all = differentiatesEncodings(adjointFlags, useSliceGradients(numel, adjointFlags))
         && (directInputStart() < 0 || (directInputStart() == 0 && encodings_[0]->numOutputChannels() == channelsIn()));
     return all ? weights | GRADIENTS_INPUT : weights;
+}
+
+bool FusedNetwork::overwritableTables(int numel, AdjointModeFlags adjointFlags) const
+{
+    // (a batch that trains in sorted order may sum a grid by columns, which add to its table)
+    if (numel <= 0 || !(adjointFlags & GRADIENTS_INPUT_ENCODINGS) || !useSliceGradients(numel, adjointFlags) || sortsTraining(numel)) return false;
+    for (const auto& e : encodings_)
+        if (e->hasParameters() && !offersSlices(*e)) return false;
+    return true;
 }
 
 void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, AdjointModeFlags adjointFlags,
@@ -2573,7 +2590,8 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
 
     const bool sliceGradients = useSliceGradients(numel, adjointFlags);
     CHECK_ERROR(!sliceGradients || numel < (1 << 27), "batches of 2^27 points or more: set options.slice_gradients to 0");
-    CHECK_ERROR((overwrite & ~overwritableGradients(numel, adjointFlags)) == 0,
+    const AdjointModeFlags overwritable = overwritableGradients(numel, adjointFlags) | (overwritableTables(numel, adjointFlags) ? GRADIENTS_INPUT_ENCODINGS : 0);
+    CHECK_ERROR((overwrite & ~overwritable) == 0,
                 "adjoint() adds to gradients of this batch that it was asked to overwrite");
     const bool overwriteInputGradients = overwrite & GRADIENTS_INPUT;
     CHECK_ERROR(contents >= 0 && contents <= (CONTENTS_DERIVATIVES | CONTENTS_NOTHING) && (contents & CONTENTS_AMOUNT) != CONTENTS_AMOUNT,
@@ -2722,37 +2740,37 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
                         const auto& ck = sk.columns[fromDerivatives ? 1 : 0].value();
                         ck.fun.launch(maxItems, ck.blockSize, ck.sharedMemorySize, stream, args);
                     }
-                    // (the room of this encoding's cursors and records stays where it is for the encodings behind it)
+                    // (the room of this encoding's records stays where it is for the encodings behind it)
                     workspace += layout.workspaceBytes(numel64);
                     continue;
                 }
             }
-            int* cursors = reinterpret_cast<int*>(workspace);
-            const size_t cursorBytes = layout.cursorBytes();
-            uint32_t* records = reinterpret_cast<uint32_t*>(workspace + cursorBytes);
-            workspace += layout.workspaceBytes(numel64);
-            QMLP_HIP_CALL(qmlp_hip_memset_async(cursors, 0, cursorBytes, stream));
+            const CompiledKernel& rk = recordsKernelFor(sk, adjointFlags, numel, derivativesStored && sk.derivativeOffset >= 0);
+            const int points = rk.blockSize;
+            IEncoding::GradientWorkspace regions = layout.workspace(workspace, numel, points);
+            workspace += layout.workspaceBytes(numel64);   // (the layout of the encodings in the memory is that of adjointMemory())
+            int overwriteTables = overwrite & GRADIENTS_INPUT_ENCODINGS ? 1 : 0;
+            int overwriteInput = overwriteInputGradients && !sortedPoints && encodings_.size() == 1 ? 1 : 0;
             std::vector<char> params(1024);
             int n = encodings_[sk.encoding]->fillParameterMemory(params.data(), static_cast<int>(params.size()));
             (void)n;
-            int numelPadded = static_cast<int>(numel64);   // the layout of the buckets is that of adjointMemory()
             {
-                // the records kernel walks over the real points, but lays its buckets out for the padded batch
                 auto adjInputAcc = sortedAdjInput;   // this grid's share of dL/dinput (zeros in it if none is asked for: unused)
-                const bool fromDerivatives = derivativesStored && sk.derivativeOffset >= 0;
                 const void* derivatives = static_cast<const char*>(tmpMemoryForward)
                     + (static_cast<long long>(perEntryForwardMemoryBytes_) + std::max(0ll, sk.derivativeOffset)) * numel64;
-                void* args[] = {&numel, &numelPadded, &inputAcc, &adjEncoded, params.data(), &records, &cursors, &adjInputAcc, &derivatives};
-                const CompiledKernel& rk = recordsKernelFor(sk, adjointFlags, numel, fromDerivatives);
-                rk.fun.launch(layout.recordsGrid(numel, rk.blockSize, layout.levelGroups(adjointFlags & GRADIENTS_INPUT), rk.fullGrid), rk.blockSize, rk.sharedMemorySize, stream, args);
+                void* args[] = {&numel, &inputAcc, &adjEncoded, params.data(), &regions, &overwriteTables, &adjInputAcc, &overwriteInput, &derivatives};
+                rk.fun.launch(layout.workgroupsPerRegion(adjointFlags & GRADIENTS_INPUT) * layout.regionSlots(numel, points), points, rk.sharedMemorySize,
+                              stream, args);
             }
-            const uint32_t* recordsRead = records;
-            const int* cursorsRead = cursors;
-            float* gradients = nullptr;
-            std::memcpy(&gradients, params.data() + sizeof(void*), sizeof(void*));   // HashGridParams: forward table, gradient table, ...
-            const void* items = sk.items.rawPtr();
-            void* args[] = {&numelPadded, &recordsRead, &cursorsRead, &gradients, &items};
-            sk.kernel.fun.launch(static_cast<int>(layout.items.size()), sk.kernel.blockSize, sk.kernel.sharedMemorySize, stream, args);
+            {
+                float* gradients = nullptr;
+                std::memcpy(&gradients, params.data() + sizeof(void*), sizeof(void*));   // HashGridParams: forward table, gradient table, ...
+                const void* items = sk.items.rawPtr();
+                void* args[] = {&numel, &regions, &gradients, &items, &overwriteTables};
+                sk.kernel.fun.launch(static_cast<int>(layout.items.size()), sk.kernel.blockSize, sk.kernel.sharedMemorySize, stream, args);
+            }
+            void* args[] = {&inputAcc, &adjEncoded, params.data(), &regions};
+            sk.exceptions.launch(layout.exceptionsGrid(regions), 64, 0, stream, args);
         }
     }
 

@@ -100,8 +100,7 @@ void IEncoding::precompile(int adjointMode)
         if (sharedAdjointWaves() > 0) kl->getKernel("qmlp::kernel::EncodingAdjointSharedKernel", adjointKernelSource(adjointMode, true), flags);
         if (const auto* layout = (adjointMode & PARAM_GRADIENTS) && hasParameters() ? sliceLayout(true) : nullptr) {
             for (int v = 0; v < recordsVariants(*layout); ++v) compileRecords(*layout, adjointMode & INPUT_GRADIENTS, v, flags);
-            compileSlices(*layout, true, flags);
-            compileSlices(*layout, false, flags);
+            compileSlices(*layout, flags);
         }
     }
 }
@@ -157,7 +156,7 @@ void IEncoding::adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& ad
 
 void IEncoding::adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& adjInput, stream_t stream,
                         const std::optional<const Tensor>& parametersForward,
-                        const std::optional<const Tensor>& parametersGradients, int adjointMode, void* tmpMemory)
+                        const std::optional<const Tensor>& parametersGradients, int adjointMode, void* tmpMemory, bool overwriteParameters)
 {
     CHECK_DIM(input, 2);
     CHECK_DIM(adjOutput, 2);
@@ -179,8 +178,9 @@ void IEncoding::adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& ad
                         || hasParameterTensor(Tensor::GRADIENTS),
                     "Parameter gradients requested, but no gradient tensor is bound or passed");
     }
-    if (numel == 0) return;
     const bool bySlices = tmpMemory != nullptr && adjointMemory(numel, adjointMode) > 0;
+    CHECK_ERROR(bySlices || !overwriteParameters, "adjoint() adds to parameter gradients of this batch that it was asked to overwrite");
+    if (numel == 0) return;
 
     const bool sharedTile = !bySlices && sharedAdjointWaves() > 0 && numel <= SHARED_ADJOINT_MAX_BATCH;
     auto& kernel = sharedTile ? adjointSharedKernel_[adjointMode] : adjointKernel_[adjointMode];
@@ -198,7 +198,7 @@ void IEncoding::adjoint(const Tensor& input, const Tensor& adjOutput, Tensor& ad
     }
 
     if (bySlices) {
-        adjointBySlices(*sliceLayout(true), input, adjOutput, adjInput, stream, adjointMode, tmpMemory, paramBytes.data());
+        adjointBySlices(*sliceLayout(true), input, adjOutput, adjInput, stream, adjointMode, tmpMemory, paramBytes.data(), overwriteParameters);
     } else {
         auto& fun = kernel.value();
         const int block = sharedTile ? sharedAdjointWaves() * 64 : 256;
@@ -237,69 +237,64 @@ std::optional<KernelFunction> IEncoding::compileRecords(const GradientSliceLayou
     source << "\n" << KernelLoader::MainFile("qmlp/kernels/grid_gradient.h");
     return QuickMLP::Instance().kernelLoader()->getKernel(
         format("qmlp::kernel::GridGradientRecordsKernel<%s, 0, 0, %d, %d, %d, %d>", layout.configType.c_str(), layout.sliceFloats,
-               layout.pointsPerWorkgroup >> variant, inputGradients ? 1 : 0, layout.levelGroups(inputGradients)), source.str(), flags);
+               layout.pointsPerWorkgroup >> variant, inputGradients ? 1 : 0, layout.levelGroups()), source.str(), flags);
 }
 
-std::optional<KernelFunction> IEncoding::compileSlices(const GradientSliceLayout& layout, bool clear, int flags) const
+std::vector<KernelFunction> IEncoding::compileSlices(const GradientSliceLayout& layout, int flags) const
 {
     std::stringstream source;
     fillCode(source);
     source << "\n" << KernelLoader::MainFile("qmlp/kernels/grid_gradient.h");
-    return QuickMLP::Instance().kernelLoader()->getKernel(
-        clear ? std::string("qmlp::kernel::GridGradientClearKernel")
-              : format("qmlp::kernel::GridGradientSlicesKernel<%s, %d, true>", layout.configType.c_str(), layout.sliceFloats),
+    return QuickMLP::Instance().kernelLoader()->getKernels(
+        {format("qmlp::kernel::GridGradientSlicesKernel<%s, %d, true>", layout.configType.c_str(), layout.sliceFloats),
+         format("qmlp::kernel::GridGradientExceptionsKernel<%s, 0, 0, %d>", layout.configType.c_str(), layout.sliceFloats)},
         source.str(), flags);
 }
 
 void IEncoding::adjointBySlices(const GradientSliceLayout& layout, const Tensor& input, const Tensor& adjOutput, Tensor& adjInput, stream_t stream,
-                                int adjointMode, void* tmpMemory, char* parameters)
+                                int adjointMode, void* tmpMemory, char* parameters, bool overwriteParameters)
 {
     CHECK_ERROR(reinterpret_cast<uintptr_t>(tmpMemory) % 256 == 0, "The temporary memory must be aligned to 256 bytes");
     auto& sk = sliceKernels_;
     const int flags = QuickMLP::Instance().getCompileFlags();
     int numel = static_cast<int>(input.size(0));
     const bool inputGradients = adjointMode & INPUT_GRADIENTS;
-    const int groups = layout.levelGroups(inputGradients);
+    const int groups = layout.levelGroups();
     // as for the fused networks: as many points per workgroup as keep every compute unit busy
     int variant = 0;
     while (variant + 1 < recordsVariants(layout) && groups * divUp(numel, layout.pointsPerWorkgroup >> variant) < KernelFunction::computeUnits()) ++variant;
     auto& variants = sk.records[inputGradients ? 1 : 0];
     if (variants.empty()) variants.resize(recordsVariants(layout));
     if (!variants[variant].has_value()) variants[variant] = compileRecords(layout, inputGradients, variant, flags).value();
-    if (!sk.clear.has_value()) sk.clear = compileSlices(layout, true, flags).value();
     if (!sk.slices.has_value()) {
-        const KernelFunction slices = compileSlices(layout, false, flags).value();
+        const auto kernels = compileSlices(layout, flags);
         sk.items = Tensor(Tensor::FLOAT, {static_cast<int32_t>(layout.items.size() * (sizeof(GradientSlice) / sizeof(float)))});
         QMLP_HIP_CALL(qmlp_hip_memcpy_h2d(sk.items.rawPtr(), layout.items.data(), layout.items.size() * sizeof(layout.items[0]), nullptr));
-        sk.slices = slices;   // (last: what it reads is there, whatever of the above has thrown)
+        sk.exceptions = kernels.at(1);
+        sk.slices = kernels.at(0);   // (last: what it reads is there, whatever of the above has thrown)
     }
 
-    int* cursors = static_cast<int*>(tmpMemory);
-    uint32_t* records = reinterpret_cast<uint32_t*>(static_cast<char*>(tmpMemory) + layout.cursorBytes());
+    const int points = layout.pointsPerWorkgroup >> variant;
+    GradientWorkspace workspace = layout.workspace(tmpMemory, numel, points);
+    int overwrite = overwriteParameters ? 1 : 0, overwriteInput = 0;
+    auto inputAcc = input.accessor<kernel::Tensor2Read<float>>();
+    auto adjOutputAcc = adjOutput.accessor<kernel::Tensor2Read<float>>();
     {
-        // (a kernel and not a memset, which calls that are captured into a graph would not repeat reliably)
-        int words = layout.numBuckets() + 1;
-        void* args[] = {&cursors, &words};
-        sk.clear.value().launch(divUp(words, 256), 256, 0, stream, args);
-    }
-    {
-        auto inputAcc = input.accessor<kernel::Tensor2Read<float>>();
-        auto adjOutputAcc = adjOutput.accessor<kernel::Tensor2Read<float>>();
         auto adjInputAcc = adjInput.accessor<kernel::Tensor2RW<float>>();
         const void* derivatives = nullptr;
-        void* args[] = {&numel, &numel, &inputAcc, &adjOutputAcc, parameters, &records, &cursors, &adjInputAcc, &derivatives};
-        const int points = layout.pointsPerWorkgroup >> variant;
-        auto& fun = variants[variant].value();
-        const int lds = layout.recordsLdsBytes(points);
-        fun.launch(layout.recordsGrid(numel, points, groups, fun.fullGridSize(points, lds)), points, lds, stream, args);
+        void* args[] = {&numel, &inputAcc, &adjOutputAcc, parameters, &workspace, &overwrite, &adjInputAcc, &overwriteInput, &derivatives};
+        variants[variant].value().launch(layout.workgroupsPerRegion(inputGradients) * layout.regionSlots(numel, points), points,
+                                         layout.recordsLdsBytes(points), stream, args);
     }
-    const uint32_t* recordsRead = records;
-    const int* cursorsRead = cursors;
-    float* gradients = nullptr;
-    std::memcpy(&gradients, parameters + sizeof(void*), sizeof(void*));   // HashGridParams: forward table, gradient table, ...
-    const void* items = sk.items.rawPtr();
-    void* args[] = {&numel, &recordsRead, &cursorsRead, &gradients, &items};
-    sk.slices.value().launch(static_cast<int>(layout.items.size()), 1024, layout.sliceFloats * static_cast<int>(sizeof(long long)), stream, args);
+    {
+        float* gradients = nullptr;
+        std::memcpy(&gradients, parameters + sizeof(void*), sizeof(void*));   // HashGridParams: forward table, gradient table, ...
+        const void* items = sk.items.rawPtr();
+        void* args[] = {&numel, &workspace, &gradients, &items, &overwrite};
+        sk.slices.value().launch(static_cast<int>(layout.items.size()), 1024, layout.slicesLdsBytes(), stream, args);
+    }
+    void* args[] = {&inputAcc, &adjOutputAcc, parameters, &workspace};
+    sk.exceptions.value().launch(layout.exceptionsGrid(workspace), 64, 0, stream, args);
 }
 
 void EncodingHashGrid::corners(const Tensor& input, unsigned* indices, float* weights, stream_t stream, int mode)

@@ -247,11 +247,20 @@ Gradients adjointPass(const Network_ptr& net, const at::Tensor& input, const at:
     at::AutoDispatchBelowADInplaceOrView guard;
     Gradients g;
     g.tables.resize(n);
+    // zeroed only where the kernels add to them
+    int overwriteTables = 0;
+    {
+        std::lock_guard<std::mutex> lock(net->mutex);
+        check(qmlp_network_overwritable_tables(net->handle, wrap(input).sizes[0], flags, &overwriteTables));
+    }
     if (flags & QMLP_GRADIENTS_INPUT_ENCODINGS)
         // the kernel adds the gradients of every encoding with parameters: a frozen one gets a zero tensor as
         // well, which the callers drop (bind_network.cpp:277-290)
         for (size_t i = 0; i < n; ++i)
-            if (net->encodings[i].hasParameters) g.tables[i] = at::zeros(tables.at(i).sizes(), tables[i].options().dtype(at::kFloat));
+            if (net->encodings[i].hasParameters) {
+                const auto options = tables.at(i).options().dtype(at::kFloat);
+                g.tables[i] = overwriteTables ? at::empty(tables[i].sizes(), options) : at::zeros(tables[i].sizes(), options);
+            }
     void* stream = currentStream(input);
     const auto wrappedTables = wrapAll(*net, tables);
     const qmlp_tensor p = wrap(parameters), in = wrap(input), adjOut = wrap(adjOutput);
@@ -262,9 +271,9 @@ Gradients adjointPass(const Network_ptr& net, const at::Tensor& input, const at:
     check(qmlp_network_adjoint_memory(net->handle, in.sizes[0], flags, &bytes));
     const at::Tensor scratch = bytesOn(input, bytes);
     net->bind(p, wrappedTables);
-    // zeroed only where the kernels add to them
     int overwrite = 0;
     check(qmlp_network_overwritable_gradients(net->handle, in.sizes[0], flags, nullptr, &overwrite));
+    if (overwriteTables) overwrite |= QMLP_GRADIENTS_INPUT_ENCODINGS;
     if (flags & QMLP_GRADIENTS_INPUT) g.input = overwrite & QMLP_GRADIENTS_INPUT ? at::empty_like(input) : at::zeros_like(input);
     if (flags & QMLP_GRADIENTS_NETWORK_WEIGHTS) {
         const auto options = parameters.options().dtype(at::kFloat);
@@ -428,19 +437,23 @@ std::pair<at::Tensor, at::Tensor> encodeAdjoint(Encoding& enc, const at::Tensor&
     at::AutoDispatchBelowADInplaceOrView guard;
     // (the native call wants the tensor in any case: without input gradients it is not written)
     at::Tensor adjInput = flags & QMLP_ENCODING_INPUT_GRADIENTS ? at::zeros_like(input) : at::Tensor();
-    at::Tensor adjParameter;
-    if (parameter.defined() && (flags & QMLP_ENCODING_PARAM_GRADIENTS))
-        adjParameter = at::zeros(parameter.sizes(), parameter.options().dtype(at::kFloat));
-    const qmlp_tensor in = wrap(input), adjOut = wrap(adjOutput), adjIn = adjInput.defined() ? wrap(adjInput) : in, par = wrap(parameter),
-                      adjPar = wrap(adjParameter);
     std::lock_guard<std::mutex> lock(enc.mutex);
     ++enc.calls;
     size_t bytes = 0;
-    check(qmlp_encoding_adjoint_memory(enc.handle, in.sizes[0], flags, &bytes));
+    check(qmlp_encoding_adjoint_memory(enc.handle, wrap(input).sizes[0], flags, &bytes));
     at::Tensor memory;
     if (bytes > 0) memory = bytesOn(input, bytes);
-    check(qmlp_encoding_adjoint_in(enc.handle, &in, &adjOut, &adjIn, currentStream(input), parameter.defined() ? &par : nullptr,
-                                   adjParameter.defined() ? &adjPar : nullptr, flags, bytes > 0 ? memory.data_ptr() : nullptr));
+    at::Tensor adjParameter;
+    if (parameter.defined() && (flags & QMLP_ENCODING_PARAM_GRADIENTS)) {
+        // with the memory the table's gradients are written, without it added to
+        const auto options = parameter.options().dtype(at::kFloat);
+        adjParameter = bytes > 0 ? at::empty(parameter.sizes(), options) : at::zeros(parameter.sizes(), options);
+    }
+    const qmlp_tensor in = wrap(input), adjOut = wrap(adjOutput), adjIn = adjInput.defined() ? wrap(adjInput) : in, par = wrap(parameter),
+                      adjPar = wrap(adjParameter);
+    auto* adjoint = bytes > 0 && adjParameter.defined() ? qmlp_encoding_adjoint_overwriting : qmlp_encoding_adjoint_in;
+    check(adjoint(enc.handle, &in, &adjOut, &adjIn, currentStream(input), parameter.defined() ? &par : nullptr,
+                  adjParameter.defined() ? &adjPar : nullptr, flags, bytes > 0 ? memory.data_ptr() : nullptr));
     return {adjInput, adjParameter};
 }
 

@@ -463,6 +463,9 @@ struct NetworkFunction : torch::autograd::Function<NetworkFunction>
             // zeroed only where the kernels add to them
             int overwrite = 0;
             QMLP_CHECK(qmlp_network_overwritable_gradients(net->handle_, static_cast<int>(input.size(0)), flags, nullptr, &overwrite));
+            int overwriteTables = 0;
+            QMLP_CHECK(qmlp_network_overwritable_tables(net->handle_, static_cast<int>(input.size(0)), flags, &overwriteTables));
+            if (overwriteTables) overwrite |= QMLP_GRADIENTS_INPUT_ENCODINGS;
             if (flags & QMLP_GRADIENTS_INPUT) adjInput = overwrite & QMLP_GRADIENTS_INPUT ? torch::empty_like(input) : torch::zeros_like(input);
             if (flags & QMLP_GRADIENTS_NETWORK_WEIGHTS) {
                 const auto options = p16.options().dtype(torch::kFloat32);
@@ -477,7 +480,9 @@ struct NetworkFunction : torch::autograd::Function<NetworkFunction>
                     if (!net->encodingHasParameters(static_cast<int64_t>(i))) continue;
                     int precision = QMLP_FLOAT;
                     QMLP_CHECK(qmlp_encoding_parameter_precision(net->encodingHandle(static_cast<int64_t>(i)), QMLP_GRADIENTS, &precision));
-                    adjEncodings[i] = torch::zeros(encodingParameters[i].sizes(), encodingParameters[i].options().dtype(dtypeOf(precision)));
+                    const auto options = encodingParameters[i].options().dtype(dtypeOf(precision));
+                    adjEncodings[i] = overwriteTables ? torch::empty(encodingParameters[i].sizes(), options)
+                                                      : torch::zeros(encodingParameters[i].sizes(), options);
                     const qmlp_tensor g = wrap(adjEncodings[i]);
                     QMLP_CHECK(qmlp_encoding_set_parameter(net->encodingHandle(static_cast<int64_t>(i)), &g, QMLP_GRADIENTS));
                 }

@@ -80,6 +80,7 @@ _SIGNATURES = {
     "qmlp_network_adjoint_memory": [_vp, _ci, _ci, _P(ctypes.c_size_t)],
     "qmlp_network_adjoint": [_vp, _TD, _TD, _ci, _TD, _vp, _vp, _vp],
     "qmlp_network_overwritable_gradients": [_vp, _ci, _ci, _vp, _pi],
+    "qmlp_network_overwritable_tables": [_vp, _ci, _ci, _pi],
     "qmlp_network_adjoint_overwriting": [_vp, _TD, _TD, _ci, _ci, _TD, _vp, _vp, _vp],
     "qmlp_network_adjoint_for": [_vp, _TD, _TD, _ci, _ci, _TD, _vp, _ci, _vp, _vp],
     "qmlp_network_clear_cached_kernels": [_vp],
@@ -101,6 +102,7 @@ _SIGNATURES = {
     "qmlp_encoding_adjoint": [_vp, _TD, _TD, _TD, _vp, _TD, _TD, _ci],
     "qmlp_encoding_adjoint_memory": [_vp, ctypes.c_longlong, _ci, _P(ctypes.c_size_t)],
     "qmlp_encoding_adjoint_in": [_vp, _TD, _TD, _TD, _vp, _TD, _TD, _ci, _vp],
+    "qmlp_encoding_adjoint_overwriting": [_vp, _TD, _TD, _TD, _vp, _TD, _TD, _ci, _vp],
     "qmlp_encoding_hashgrid_levels": [_vp, _ci, _pi, _pi, _pi, _pi, _pi],
     "qmlp_encoding_hashgrid_corners": [_vp, _TD, _vp, _vp, _vp],
     "qmlp_encoding_hashgrid_trace": [_vp, _TD, _ci, _vp, _vp, _vp],
