@@ -69,7 +69,7 @@ struct PullPushLevel
     PullPushView<T> gradMaskPost, gradDataPost, gradMaskPre, gradDataPre;   // adjoint; the first is absent on the finest level (zero)
 };
 
-constexpr int PULLPUSH_TAIL_BLOCK = 512;
+constexpr int PULLPUSH_TAIL_BLOCK = 1024;
 /** The levels that the kernels for all coarse levels keep in LDS: levels[0] is the one above them. */
 struct PullPushTail
 {
@@ -575,35 +575,335 @@ __device__ __forceinline__ void tileOf(int width, int height, int& b, int& a0, i
 
 /**
  * Level k (> 0) of the coarse levels that one workgroup keeps in LDS, below a level of H x W pixels (sizes are halved, rounding
- * down, and rows start at even entries). The views have no image stride: a workgroup has one image.
+ * down, and rows start at even entries). Read and written as LDS and not through addresses that may lie anywhere.
  */
-template <typename T, bool GRADIENTS>
-__device__ __forceinline__ PullPushLevel<T> ldsLevel(T* sLevels, const PullPushTail& tail, int H, int W, int C, int k)
+template <typename T>
+struct LdsLevel
 {
-    T* next = sLevels + tail.offsets[k];
-    PullPushLevel<T> l;
-    l.H = H >> k;
-    l.W = W >> k;
-    const unsigned pitch = (l.W + 1) & ~1, plane = l.H * pitch;
-    auto take = [&](int channels) {
-        PullPushView<T> v{next, 0, plane, static_cast<PullPushStride>(pitch), 1};
-        next += channels * plane;
-        return v;
-    };
-    l.maskPre = take(1);
-    l.dataPre = take(C);
-    l.maskSum = take(1);
-    const bool coarsest = k == tail.numLevels - 1;   // its own inpainting: nothing changes from before to after
-    l.maskPost = coarsest ? l.maskPre : take(1);
-    l.dataPost = coarsest ? l.dataPre : take(C);
-    if (GRADIENTS) {
-        l.gradMaskPost = take(1);
-        l.gradDataPost = take(C);
-        l.gradMaskPre = coarsest ? l.gradMaskPost : take(1);
-        l.gradDataPre = coarsest ? l.gradDataPost : take(C);
+    typedef __attribute__((address_space(3))) T entry;
+    int H, W, pitch, plane;
+    entry *maskPreP, *dataPreP, *maskSumP, *maskPostP, *dataPostP, *gradMaskPostP, *gradDataPostP, *gradMaskPreP, *gradDataPreP;
+
+    /** \param gradients the gradients of a level lie behind it */
+    __device__ __forceinline__ LdsLevel(entry* levels, const PullPushTail& tail, int finestH, int finestW, int C, int k, bool gradients)
+    {
+        entry* next = levels + tail.offsets[k];
+        H = finestH >> k;
+        W = finestW >> k;
+        pitch = (W + 1) & ~1;
+        plane = H * pitch;
+        auto take = [&](int channels) {
+            entry* p = next;
+            next += channels * plane;
+            return p;
+        };
+        maskPreP = take(1);
+        dataPreP = take(C);
+        maskSumP = take(1);
+        const bool coarsest = k == tail.numLevels - 1;   // its own inpainting: nothing changes from before to after
+        maskPostP = coarsest ? maskPreP : take(1);
+        dataPostP = coarsest ? dataPreP : take(C);
+        gradMaskPostP = gradDataPostP = gradMaskPreP = gradDataPreP = next;
+        if (gradients) {
+            gradMaskPostP = take(1);
+            gradDataPostP = take(C);
+            gradMaskPreP = coarsest ? gradMaskPostP : take(1);
+            gradDataPreP = coarsest ? gradDataPostP : take(C);
+        }
     }
-    return l;
-}
+    __device__ __forceinline__ entry& at(entry* p, int c, int y, int x) const { return p[c * plane + y * pitch + x]; }
+    __device__ __forceinline__ bool hasMaskPost() const { return true; }
+    __device__ __forceinline__ bool hasGradMaskPost() const { return true; }
+    __device__ __forceinline__ entry& maskPre(int y, int x) const { return at(maskPreP, 0, y, x); }
+    __device__ __forceinline__ entry& dataPre(int c, int y, int x) const { return at(dataPreP, c, y, x); }
+    __device__ __forceinline__ entry& maskSum(int y, int x) const { return at(maskSumP, 0, y, x); }
+    __device__ __forceinline__ entry& maskPost(int y, int x) const { return at(maskPostP, 0, y, x); }
+    __device__ __forceinline__ entry& dataPost(int c, int y, int x) const { return at(dataPostP, c, y, x); }
+    __device__ __forceinline__ entry& gradMaskPost(int y, int x) const { return at(gradMaskPostP, 0, y, x); }
+    __device__ __forceinline__ entry& gradDataPost(int c, int y, int x) const { return at(gradDataPostP, c, y, x); }
+    __device__ __forceinline__ entry& gradMaskPre(int y, int x) const { return at(gradMaskPreP, 0, y, x); }
+    __device__ __forceinline__ entry& gradDataPre(int c, int y, int x) const { return at(gradDataPreP, c, y, x); }
+};
+
+/**
+ * The level above them, in global memory: what the steps read of it is copied into LDS first, as it is read several
+ * times and by few lanes (a global load in every round of a step's loop: 64 x 64 pixels 103 us), what they write goes to global memory.
+ */
+template <typename T>
+struct TopLevel
+{
+    typedef typename LdsLevel<T>::entry entry;
+    const PullPushLevel<T>& l;
+    int b, H, W, pitch, plane;
+    entry *maskPreP, *dataPreP, *gradMaskPostP, *gradDataPostP;
+
+    __device__ __forceinline__ static void copy(entry* to, const PullPushView<T>& from, int b, int C, int H, int W, int pitch)
+    {
+        const float inverse = 1.f / static_cast<float>(W);
+        for (int c = 0; c < C; ++c)
+#pragma unroll 4
+            for (int i = threadIdx.x; i < H * W; i += PULLPUSH_TAIL_BLOCK) {
+                const int y = static_cast<int>((static_cast<float>(i) + 0.5f) * inverse);
+                to[(c * H + y) * pitch + (i - y * W)] = *at(from, b, c, y, i - y * W);
+            }
+    }
+    /** All lanes of the workgroup; a barrier is up to the caller. */
+    __device__ __forceinline__ TopLevel(const PullPushLevel<T>& level, int image, entry* top, int C, bool gradients)
+        : l(level), b(image), H(level.H), W(level.W)
+    {
+        pitch = (W + 1) & ~1;
+        plane = H * pitch;
+        maskPreP = top;
+        dataPreP = maskPreP + plane;
+        gradMaskPostP = dataPreP + C * plane;
+        gradDataPostP = gradMaskPostP + plane;
+        copy(maskPreP, l.maskPre, b, 1, H, W, pitch);
+        copy(dataPreP, l.dataPre, b, C, H, W, pitch);
+        if (!gradients) return;
+        if (l.gradMaskPost.p) copy(gradMaskPostP, l.gradMaskPost, b, 1, H, W, pitch);
+        copy(gradDataPostP, l.gradDataPost, b, C, H, W, pitch);
+    }
+    __device__ __forceinline__ bool hasMaskPost() const { return l.maskPost.p != nullptr; }
+    __device__ __forceinline__ bool hasGradMaskPost() const { return l.gradMaskPost.p != nullptr; }
+    __device__ __forceinline__ T maskPre(int y, int x) const { return maskPreP[y * pitch + x]; }
+    __device__ __forceinline__ T dataPre(int c, int y, int x) const { return dataPreP[c * plane + y * pitch + x]; }
+    __device__ __forceinline__ T gradMaskPost(int y, int x) const { return gradMaskPostP[y * pitch + x]; }
+    __device__ __forceinline__ T gradDataPost(int c, int y, int x) const { return gradDataPostP[c * plane + y * pitch + x]; }
+    __device__ __forceinline__ T& maskPost(int y, int x) const { return *at(l.maskPost, b, 0, y, x); }
+    __device__ __forceinline__ T& dataPost(int c, int y, int x) const { return *at(l.dataPost, b, c, y, x); }
+    __device__ __forceinline__ T& gradMaskPre(int y, int x) const { return *at(l.gradMaskPre, b, 0, y, x); }
+    __device__ __forceinline__ T& gradDataPre(int c, int y, int x) const { return *at(l.gradDataPre, b, c, y, x); }
+};
+
+/**
+ * The steps of the coarse levels, by one compute unit: a chain of a few dependent loads and a division per step, and on the larger
+ * levels vector instructions. An item is a pixel with all its channels where that fills the workgroup, on smaller levels 2^n neighbouring
+ * lanes share the channels of a pixel, look the masks up each for itself, and add up what the mask's gradient takes
+ * from all channels with shuffles. (A lane per channel on every level: 39
+ * instead of 32 us for the adjoint of 32 x 32 x 4 floats and below, of which a step of 2 x 2 pixels takes 2 us, one of 32 x 32 up to 5.)
+ */
+template <typename T>
+struct TailSteps
+{
+    typedef typename LdsLevel<T>::entry entry;
+    int C;
+    __device__ __forceinline__ explicit TailSteps(int channels) : C(channels) {}
+
+    /** Lanes per pixel (their logarithm) for so many pixels and channels. */
+    __device__ __forceinline__ static int lanesLog2(int pixels, int channels)
+    {
+        int log2 = 0;
+        while ((1 << log2) < channels && (pixels << (log2 + 1)) <= PULLPUSH_TAIL_BLOCK) ++log2;
+        return log2;
+    }
+    /** Calls item(y, x, lane of the pixel) for rows x W pixels from (y0, x0) on, all lanes of a pixel at the same time. */
+    template <typename Item>
+    __device__ __forceinline__ static void forEach(int y0, int x0, int rows, int W, int log2, const Item& item)
+    {
+        const int items = (rows * W) << log2;
+        const float inverse = 1.f / static_cast<float>(W);
+        for (int i = threadIdx.x; i < items; i += PULLPUSH_TAIL_BLOCK) {
+            const int pixel = i >> log2;
+            const int y = static_cast<int>((static_cast<float>(pixel) + 0.5f) * inverse);   // exact: LDS holds fewer than 2^20 pixels
+            item(y0 + y, x0 + pixel - y * W, i & ((1 << log2) - 1));
+        }
+    }
+    __device__ __forceinline__ static T sumOver(T v, int log2)
+    {
+        for (int d = 1; d < (1 << log2); d *= 2) v += __shfl_xor(v, d, 64);
+        return v;
+    }
+
+    template <typename High>
+    __device__ __forceinline__ void down(const High& high, const LdsLevel<T>& low) const
+    {
+        const int rows = 2 + (high.H & 1), columns = 2 + (high.W & 1);
+        const int log2 = lanesLog2(low.H * low.W, C);
+        forEach(0, 0, low.H, low.W, log2, [&](int a, int e, int lane) {
+            T m[3][3];
+            T sum = 0, most = 0;
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    m[i][j] = T(0);
+                    if (i >= rows || j >= columns) continue;
+                    m[i][j] = high.maskPre(2 * a + i, 2 * e + j);
+                    sum += m[i][j];
+                    most = max(most, m[i][j]);
+                }
+            for (int c = lane; c < C; c += 1 << log2) {
+                T d = 0;
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+                        if (i < rows && j < columns) d += m[i][j] * high.dataPre(c, 2 * a + i, 2 * e + j);
+                low.dataPre(c, a, e) = quotient(d, sum);
+            }
+            if (lane == 0) {
+                low.maskPre(a, e) = most;
+                low.maskSum(a, e) = sum;
+            }
+        });
+    }
+
+    /** The low-res neighbours of high-res pixel (y, x): the own cell, the one in the other row, in the other column, the diagonal one. */
+    struct Mix
+    {
+        int at[4];
+        T wm[4], n, weight;
+        __device__ __forceinline__ Mix(int y, int x, const LdsLevel<T>& low)
+        {
+            const int row = y >> 1, column = x >> 1;
+            const int otherRow = row - 1 + 2 * (y & 1), otherColumn = column - 1 + 2 * (x & 1);
+            const float own = row < low.H ? 0.75f : 0.f, other = otherRow >= 0 && otherRow < low.H ? 0.25f : 0.f;
+            const float ownColumn = column < low.W ? 0.75f : 0.f, otherC = otherColumn >= 0 && otherColumn < low.W ? 0.25f : 0.f;
+            const int a[2] = {min(row, low.H - 1) * low.pitch, min(max(otherRow, 0), low.H - 1) * low.pitch};
+            const int e[2] = {min(column, low.W - 1), min(max(otherColumn, 0), low.W - 1)};
+            const float w[4] = {own * ownColumn, other * ownColumn, own * otherC, other * otherC};
+            n = weight = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                at[k] = a[k & 1] + e[k >> 1];
+                wm[k] = w[k] * low.maskPostP[at[k]];
+                weight += w[k];
+                n += wm[k];
+            }
+        }
+        __device__ __forceinline__ T sum(const LdsLevel<T>& low, int c) const
+        {
+            const entry* data = low.dataPostP + c * low.plane;
+            T d = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) d += wm[k] * data[at[k]];
+            return d;
+        }
+    };
+
+    template <typename High>
+    __device__ __forceinline__ void up(const High& high, const LdsLevel<T>& low) const
+    {
+        const int log2 = lanesLog2(high.H * high.W, C);
+        forEach(0, 0, high.H, high.W, log2, [&](int y, int x, int lane) {
+            const T m = high.maskPre(y, x);
+            const Mix mix(y, x, low);
+            for (int c = lane; c < C; c += 1 << log2)
+                high.dataPost(c, y, x) = m * high.dataPre(c, y, x) + (1 - m) * quotient(mix.sum(low, c), mix.n);
+            if (lane == 0 && high.hasMaskPost()) high.maskPost(y, x) = m + (mix.n > 0 ? (1 - m) * (mix.n / mix.weight) : T(0));
+        });
+    }
+
+    /** Step A (see gradientUpTile). fill: room for fillEntries entries, at least (C + 1) x 4 rows of the high-res level and a border. */
+    template <typename High>
+    __device__ __forceinline__ void gradientUp(const High& high, const LdsLevel<T>& low, entry* fill, int fillEntries) const
+    {
+        const int pitch = high.W + 2;
+        const int stripe = max(1, (fillEntries / ((C + 1) * pitch) - 2) / 2);   // low-res rows that are gathered together
+        for (int a0 = 0; a0 < low.H; a0 += stripe) {
+            const int a1 = min(a0 + stripe, low.H);
+            const int y0 = 2 * a0 - 1, rows = 2 * (a1 - a0) + 2;   // with the border, which passes nothing down
+            const int plane = rows * pitch;
+            const int fillLog2 = lanesLog2(plane, C);
+            forEach(y0, -1, rows, pitch, fillLog2, [&](int y, int x, int lane) {
+                entry* to = fill + ((y - y0) * pitch + x + 1);
+                const bool inside = y >= 0 && y < high.H && x >= 0 && x < high.W;
+                if (!inside) {
+                    for (int c = lane; c <= C; c += 1 << fillLog2) to[c * plane] = T(0);
+                    return;
+                }
+                const T m = high.maskPre(y, x);
+                const Mix mix(y, x, low);
+                const Reciprocal<T> inverse(mix.n);
+                T fromMask = 0;
+                for (int c = lane; c < C; c += 1 << fillLog2) {
+                    const T f = inverse(high.gradDataPost(c, y, x) * (1 - m));
+                    to[c * plane] = f;
+                    fromMask += f * inverse(mix.sum(low, c));
+                }
+                fromMask = sumOver(fromMask, fillLog2);
+                if (lane == 0) to[C * plane] = (high.hasGradMaskPost() ? high.gradMaskPost(y, x) * ((1 - m) / mix.weight) : T(0)) - fromMask;
+            });
+            __syncthreads();
+            const int gatherLog2 = lanesLog2((a1 - a0) * low.W, C + 1);
+            forEach(a0, 0, a1 - a0, low.W, gatherLog2, [&](int a, int e, int lane) {
+                T gradMask = 0;
+                const T mask = low.maskPost(a, e);
+                for (int c = lane; c <= C; c += 1 << gatherLog2) {
+                    const entry* from = fill + (c * plane + 2 * (a - a0) * pitch + 2 * e);
+                    T sum = 0;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float wr = (i == 1 || i == 2) ? 0.75f : 0.25f;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) sum += (wr * ((j == 1 || j == 2) ? 0.75f : 0.25f)) * from[i * pitch + j];
+                    }
+                    if (c == C) {
+                        gradMask += sum;
+                    } else {
+                        gradMask += sum * low.dataPost(c, a, e);
+                        low.gradDataPost(c, a, e) = sum * mask;
+                    }
+                }
+                gradMask = sumOver(gradMask, gatherLog2);
+                if (lane == 0) low.gradMaskPost(a, e) = gradMask;
+            });
+            __syncthreads();
+        }
+    }
+
+    /** Step B (see gradientQuad). \tparam ACCUMULATE add to what is there */
+    template <bool ACCUMULATE, typename High>
+    __device__ __forceinline__ void gradient(const High& high, const LdsLevel<T>& low) const
+    {
+        const bool oddH = high.H & 1, oddW = high.W & 1;
+        const int log2 = lanesLog2(high.H * high.W, C);
+        forEach(0, 0, high.H, high.W, log2, [&](int y, int x, int lane) {
+            const T m = high.maskPre(y, x);
+            const Mix mix(y, x, low);
+            const Reciprocal<T> inverse(mix.n);
+            // the windows that the pixel lies in: of the own cell, and of odd sizes those of the row above and of the column to the left
+            Reciprocal<T> sums[2][2];
+            int window[2][2];
+            bool in[2][2];
+            T gradMask = 0;
+#pragma unroll
+            for (int wa = 0; wa < 2; ++wa)
+#pragma unroll
+                for (int we = 0; we < 2; ++we) {
+                    const int a = (y >> 1) - wa, e = (x >> 1) - we;
+                    in[wa][we] = (wa == 0 || (oddH && !(y & 1))) && (we == 0 || (oddW && !(x & 1))) && a >= 0 && e >= 0 && a < low.H && e < low.W;
+                    window[wa][we] = 0;
+                    if (!in[wa][we]) continue;
+                    window[wa][we] = a * low.pitch + e;
+                    sums[wa][we] = Reciprocal<T>(low.maskSumP[window[wa][we]]);
+                    // the maximum of a window passes its gradient to every pixel that attains it
+                    if (lane == 0 && low.maskPreP[window[wa][we]] == m) gradMask += low.gradMaskPreP[window[wa][we]];
+                }
+            for (int c = lane; c < C; c += 1 << log2) {
+                const T v = high.dataPre(c, y, x), g = high.gradDataPost(c, y, x);
+                T sum = g;
+                gradMask += g * (v - inverse(mix.sum(low, c)));
+#pragma unroll
+                for (int wa = 0; wa < 2; ++wa)
+#pragma unroll
+                    for (int we = 0; we < 2; ++we) {
+                        if (!in[wa][we]) continue;
+                        const T grad = sums[wa][we](low.gradDataPreP[c * low.plane + window[wa][we]]);
+                        sum += grad;
+                        gradMask += grad * (v - low.dataPreP[c * low.plane + window[wa][we]]);
+                    }
+                const T out = m * sum;
+                high.gradDataPre(c, y, x) = ACCUMULATE ? high.gradDataPre(c, y, x) + out : out;
+            }
+            gradMask = sumOver(gradMask, log2);
+            if (lane == 0) {
+                if (high.hasGradMaskPost()) gradMask += high.gradMaskPost(y, x) * (1 - mix.n / mix.weight);
+                high.gradMaskPre(y, x) = ACCUMULATE ? high.gradMaskPre(y, x) + gradMask : gradMask;
+            }
+        });
+    }
+};
 } // namespace pullpush
 
 template <typename T>
@@ -661,66 +961,67 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof
 /**
  * All coarse levels, one workgroup per image: from 'finest' down to the coarsest level and up again (without an output
  * for 'finest' up to the level below it). The levels below 'finest' live in LDS (dynamic, sized by the host); a copy goes
- * to kept, keptEntries per image, for the adjoint.
+ * to kept, keptEntries per image, for the adjoint. 32 x 32 x 4 floats: 12 us, the adjoint 32; with a quad of pixels per
+ * lane and addresses that may lie anywhere 26 and 58.
  */
 template <typename T>
 __global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushTailKernel(const PullPushLevel<T> finest, int C, const PullPushTail tail,
-                                                                           T* __restrict__ kept, int keptEntries)
+                                                                           T* __restrict__ kept, int keptEntries, int topOffset)
 {
     using namespace pullpush;
     extern __shared__ __align__(16) unsigned char sMemory[];
-    T* sLevels = reinterpret_cast<T*>(sMemory);
+    auto* sLevels = (typename LdsLevel<T>::entry*)sMemory;
     const int b = blockIdx.x;
-    auto level = [&](int k) { return k == 0 ? finest : ldsLevel<T, false>(sLevels, tail, finest.H, finest.W, C, k); };
-    for (int k = 0; k + 1 < tail.numLevels; ++k) {
-        const auto high = level(k), low = level(k + 1);
-        for (int i = threadIdx.x; i < low.H * low.W; i += PULLPUSH_TAIL_BLOCK) downPixel<false>(high, low, C, b, i / low.W, i % low.W);
+    const TailSteps<T> steps(C);
+    const TopLevel<T> top(finest, b, sLevels + topOffset, C, false);
+    auto level = [&](int k) { return LdsLevel<T>(sLevels, tail, finest.H, finest.W, C, k, false); };
+    __syncthreads();
+    steps.down(top, level(1));
+    __syncthreads();
+    for (int k = 1; k + 1 < tail.numLevels; ++k) {
+        steps.down(level(k), level(k + 1));
         __syncthreads();
     }
-    for (int k = tail.numLevels - 2; k >= (finest.dataPost.p ? 0 : 1); --k) {
-        const auto high = level(k), low = level(k + 1);
-        const int height = (high.H + 1) / 2, width = (high.W + 1) / 2;
-        for (int i = threadIdx.x; i < height * width; i += PULLPUSH_TAIL_BLOCK) upQuad<false>(high, low, C, b, i / width, i % width);
+    for (int k = tail.numLevels - 2; k >= 1; --k) {
+        steps.up(level(k), level(k + 1));
         __syncthreads();
     }
+    if (finest.dataPost.p) steps.up(top, level(1));
     for (int i = threadIdx.x; i < keptEntries; i += PULLPUSH_TAIL_BLOCK) kept[static_cast<long long>(b) * keptEntries + i] = sLevels[i];
 }
 
-/** The adjoint of all coarse levels, one workgroup per image. ACCUMULATE: 'finest' is the image itself and its gradients are added to. */
+/**
+ * The adjoint of all coarse levels, one workgroup per image. ACCUMULATE: 'finest' is the image itself and its gradients are
+ * added to. Behind the levels lie what is read of 'finest' and the fills of step A, fillEntries of them.
+ */
 template <typename T, bool ACCUMULATE>
 __global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushGradientTailKernel(const PullPushLevel<T> finest, int C, const PullPushTail tail,
                                                                                    const T* __restrict__ kept, int keptEntries,
-                                                                                   const PullPushTail keptTail)
+                                                                                   const PullPushTail keptTail, int topOffset, int fillOffset, int fillEntries)
 {
     using namespace pullpush;
-    constexpr int TW = 32, TH = PULLPUSH_TAIL_BLOCK / TW;
     extern __shared__ __align__(16) unsigned char sMemory[];
-    auto& sFill = *reinterpret_cast<T (*)[pullpushChunk<T>() + 1][pullpushTileEntries(TW, TH)]>(sMemory);
-    T* sLevels = reinterpret_cast<T*>(sMemory + sizeof(sFill));
+    auto* sLevels = (typename LdsLevel<T>::entry*)sMemory;
+    auto* sFill = sLevels + fillOffset;
     const int b = blockIdx.x;
-    auto level = [&](int k) { return k == 0 ? finest : ldsLevel<T, true>(sLevels, tail, finest.H, finest.W, C, k); };
+    const TailSteps<T> steps(C);
+    const TopLevel<T> top(finest, b, sLevels + topOffset, C, true);
+    auto level = [&](int k) { return LdsLevel<T>(sLevels, tail, finest.H, finest.W, C, k, true); };
     // the levels of the forward pass; here the gradients of a level follow behind it
     for (int k = 1; k < tail.numLevels; ++k) {
         const T* from = kept + (static_cast<long long>(b) * keptEntries + keptTail.offsets[k]);
         const int entries = (k + 1 < tail.numLevels ? keptTail.offsets[k + 1] : keptEntries) - keptTail.offsets[k];
+#pragma unroll 4
         for (int i = threadIdx.x; i < entries; i += PULLPUSH_TAIL_BLOCK) sLevels[tail.offsets[k] + i] = from[i];
     }
     __syncthreads();
-    for (int k = 0; k + 1 < tail.numLevels; ++k) {
-        const auto high = level(k), low = level(k + 1);
-        for (int a0 = 0; a0 < low.H; a0 += TH)
-            for (int e0 = 0; e0 < low.W; e0 += TW) gradientUpTile<false, TW, TH>(high, low, C, b, a0, e0, sFill);
+    steps.gradientUp(top, level(1), sFill, fillEntries);
+    for (int k = 1; k + 1 < tail.numLevels; ++k) steps.gradientUp(level(k), level(k + 1), sFill, fillEntries);
+    for (int k = tail.numLevels - 2; k >= 1; --k) {
+        steps.template gradient<false>(level(k), level(k + 1));
         __syncthreads();
     }
-    for (int k = tail.numLevels - 2; k >= 0; --k) {
-        const auto high = level(k), low = level(k + 1);
-        const int height = (high.H + 1) / 2, width = (high.W + 1) / 2;
-        for (int i = threadIdx.x; i < height * width; i += PULLPUSH_TAIL_BLOCK) {
-            if (ACCUMULATE && k == 0) gradientQuad<false, true>(high, low, C, b, i / width, i % width);
-            else gradientQuad<false, false>(high, low, C, b, i / width, i % width);
-        }
-        __syncthreads();
-    }
+    steps.template gradient<ACCUMULATE>(top, level(1));
 }
 
 namespace pullpush

@@ -29,13 +29,10 @@ const char* const KERNEL_NAMES[] = {"PullPushDownKernel<$T>", "PullPushUpKernel<
 enum KernelIndex { DOWN, UP, TAIL, GRADIENT_UP, GRADIENT, GRADIENT_ADD, GRADIENT_TAIL, GRADIENT_TAIL_ADD, ADD_4, COPY_4 };
 
 // as in kernels/pullpush.h
-constexpr int TAIL_BLOCK = 512, TILE_W = 32, TILE_H = 8, BLOCK = 256;
-template <typename T>
-constexpr int tailFillBytes()
-{
-    constexpr int TH = TAIL_BLOCK / TILE_W, planes = (sizeof(T) == 4 ? 4 : 2) + 1;
-    return planes * (2 * (TH + 2) * (2 * (TILE_W + 2) + 1)) * static_cast<int>(sizeof(T));
-}
+constexpr int TAIL_BLOCK = 1024, TILE_W = 32, TILE_H = 8, BLOCK = 256;
+// What the kernel of the coarse levels keeps in LDS beside them for step A, four rows at least: all of 32 x 32 pixels of 4
+// channels of floats with a border.
+constexpr size_t TAIL_FILL_BYTES = 24 * 1024;
 
 /** \param wide for images whose planes span 2^32 entries or more, or run backwards (see the header) */
 std::string pullpushSource(bool wide)
@@ -131,12 +128,20 @@ struct Tail
     int offsets[31];
 };
 
+/** Where the kernel of the coarse levels keeps, in entries, what is read of the level above them and the fills of step A. */
+struct TailLds
+{
+    int topOffset, fillOffset, fillEntries;
+};
+
 /** LDS bytes of the kernel that takes over the coarse levels below an (H, W) level: with the gradients, which need more. */
 template <typename T>
-size_t tailLdsBytes(int C, int H, int W, bool gradients, Tail* tail = nullptr)
+size_t tailLdsBytes(int C, int H, int W, bool gradients, Tail* tail = nullptr, TailLds* lds = nullptr)
 {
     size_t entries = 0;
     int level = 0;
+    const size_t top = static_cast<size_t>(C + 1) * (gradients ? 2 : 1) * static_cast<size_t>(H) * roundUp(W, 2);
+    const size_t fill = std::max(TAIL_FILL_BYTES / sizeof(T), static_cast<size_t>(C + 1) * 4 * (static_cast<size_t>(W) + 2));
     while (!isCoarsest(H, W)) {
         H /= 2;
         W /= 2;
@@ -148,7 +153,8 @@ size_t tailLdsBytes(int C, int H, int W, bool gradients, Tail* tail = nullptr)
         if (gradients) entries += plane * (coarsest ? 1 + C : 2 + 2 * C);
     }
     if (tail) tail->numLevels = level + 1;
-    return entries * sizeof(T) + (gradients ? tailFillBytes<T>() : 0);
+    if (lds) *lds = {static_cast<int>(entries), static_cast<int>(entries + top), static_cast<int>(fill)};
+    return (entries + top + (gradients ? fill : 0)) * sizeof(T);
 }
 
 /**
@@ -192,7 +198,9 @@ std::vector<Level<T>> layout(int B, int C, int H, int W, void* pyramid, void* gr
         levels.push_back(l);
     }
     keptTail = forward.base ? forward.base + forward.entries : nullptr;
-    forward.entries += static_cast<size_t>(B) * (tailLdsBytes<T>(C, H, W, false) / sizeof(T));
+    TailLds tail = {};
+    (void)tailLdsBytes<T>(C, H, W, false, nullptr, &tail);
+    forward.entries += static_cast<size_t>(B) * tail.topOffset;
     if (bytes) *bytes = forward.entries * sizeof(T);
     if (gradientBytes) *gradientBytes = adjoint.entries * sizeof(T);
     return levels;
@@ -204,10 +212,15 @@ void launchTail(KernelIndex kernel, bool wide, int B, int C, Level<T> finest, bo
 {
     if (isCoarsest(finest.H, finest.W)) return;
     Tail tail = {}, keptTail = {};
-    const size_t lds = tailLdsBytes<T>(C, finest.H, finest.W, gradients, &tail);
-    int keptEntries = static_cast<int>(tailLdsBytes<T>(C, finest.H, finest.W, false, &keptTail) / sizeof(T));
-    void* args[] = {&finest, &C, &tail, &kept, &keptEntries, &keptTail};   // (the last one for the gradients only)
-    pullpushKernel<T>(kernel, wide).launch(static_cast<unsigned>(B), TAIL_BLOCK, static_cast<unsigned>(lds), stream, args);
+    TailLds places = {}, keptPlaces = {};
+    const size_t lds = tailLdsBytes<T>(C, finest.H, finest.W, gradients, &tail, &places);
+    (void)tailLdsBytes<T>(C, finest.H, finest.W, false, &keptTail, &keptPlaces);
+    int keptEntries = keptPlaces.topOffset;   // the levels alone
+    std::vector<void*> args = {&finest, &C, &tail, &kept, &keptEntries};
+    if (gradients) args.push_back(&keptTail);
+    args.push_back(&places.topOffset);
+    if (gradients) args.insert(args.end(), {&places.fillOffset, &places.fillEntries});
+    pullpushKernel<T>(kernel, wide).launch(static_cast<unsigned>(B), TAIL_BLOCK, static_cast<unsigned>(lds), stream, args.data());
 }
 
 /** Whether the pixels (y, 2k) and (y, 2k + 1) of all images of a level can be moved as one aligned pair. */
