@@ -258,4 +258,14 @@ struct RowAccessor
     __device__ __forceinline__ T& operator[](int i) const { return p[static_cast<long long>(i) * stride]; }
 };
 
+/**
+ * A workgroup barrier that orders the LDS accesses of the workgroup and nothing else. __syncthreads() also waits for
+ * every load from and store to global memory that the wavefront has in flight: for kernels that read none of what they
+ * write to global memory.
+ */
+__device__ __forceinline__ void ldsBarrier()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 QUICKMLP_KERNEL_NAMESPACE_END

@@ -204,16 +204,6 @@ struct GridGradientLayout
     }
 };
 
-/**
- * A workgroup barrier that orders the LDS accesses of the workgroup and nothing else. __syncthreads() also waits for
- * every load from and store to global memory that the wavefront has in flight; nothing that the records kernel writes to
- * global memory is read again before the kernel ends.
- */
-__device__ __forceinline__ void ldsBarrier()
-{
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS, int POINTS>
 struct GridGradientRecords
 {

@@ -9,9 +9,9 @@
 //          weights 9/16, 3/16, 3/16, 1/16, renormalised by the low-res masks)
 //
 // The coarsest level (a row or a column of pixels) is its own inpainting. Every step is bound by HBM traffic
-// on the fine levels and by latency on the coarse ones (a launch for a level of 64 x 64 pixels takes 5 to 10 us, most of it
-// instructions and operands that arrive for the first time). Hence one launch per level while a level is large, and one
-// launch with a workgroup per image for all levels below, which then fit into LDS (4 channels of float: below 32 x 32).
+// on the fine levels and by latency on the coarse ones (a launch for a level of 64 x 64 pixels takes 5 to 10 us). Hence one
+// launch per level while a level is large, one for several levels below, and one with a workgroup per image for the coarsest, which
+// fit into LDS (4 channels of float: below 32 x 32).
 //
 // The unit of work is the quad: the 2 x 2 high-res pixels of one low-res pixel. Its pixels are moved in pairs
 // (8 or 16 bytes per lane) and share their 3 x 3 low-res neighbours (9 loads instead of 16).
@@ -23,11 +23,11 @@
 //      level + adjoint of down, both formed per quad by gathering, without atomics
 // so the finest level of C channels moves C+1 + (2C+2)/4 planes in A and 3C+2 + (3C+4)/4 in B (a coarser one, whose mask has a
 // gradient, one more in each), C+1 + (C+2)/4 in down and 2C+1 + (C+1)/4 in up.
-// 1 x 4 x 2048 x 2048 floats, finest level: down 20, up 39, A 50, B 69 us (5.4, 4.4, 2.5, 4.4 TB/s of the planes above; a
-// large copy reaches 5.2), 178 of the 439 us of a forward and adjoint call; 1024 x 1024 takes 53, the levels below it, whose
-// launches and single workgroups wait for latency, the rest. (Coarse levels formed again by the adjoint: 10 us more; four
-// passes per level through memory, atomics for odd sizes, and memory allocated and released by every call: 9.4 ms.) A and B
-// are held to 128 registers for floats, four wavefronts per SIMD: with 129 and 130 they take 57 and 90 us.
+// 1 x 4 x 2048 x 2048 floats, finest level: down 21, up 36, A 45, B 70 us (5.2, 4.8, 2.8, 4.3 TB/s of the planes above; a
+// large copy reaches 4.8), 172 of the 352 us of a forward and adjoint call; 1024 x 1024 takes 50, the levels below it, which take several
+// steps per launch (the trees below) or live in one workgroup's LDS, the rest: a step is a chain of 1.5 to 2 us. (A launch per level: 446 us.
+// Coarse levels formed again by the adjoint: 10 us more; four passes per level through memory, atomics for odd sizes, and memory allocated and
+// released by every call: 9.4 ms.) A and B are held to 128 registers for floats, four wavefronts per SIMD.
 //
 // Follows src_cpp/include/qmlp/kernels/pullpush.cuh:22-303 of the reference. Differences on
 // purpose: no per-thread channel arrays, no atomics (the reference scatters the adjoint of up with atomics and adds
@@ -75,6 +75,14 @@ struct PullPushTail
 {
     int numLevels;
     int offsets[31];   // of level k in entries
+};
+/** Consecutive levels, finest first, that one launch walks through, with the tile of the finest that a workgroup takes. */
+constexpr int PULLPUSH_TREE_LEVELS = 6;
+template <typename T>
+struct PullPushTree
+{
+    int count, tile;
+    PullPushLevel<T> levels[PULLPUSH_TREE_LEVELS];
 };
 /** Channels that are in flight together: their loads are issued before the first of them is used. */
 template <typename T> constexpr int pullpushChunk() { return sizeof(T) == 4 ? 4 : 2; }
@@ -194,30 +202,22 @@ __device__ __forceinline__ void downPixel(const PullPushLevel<T>& high, const Pu
     }
 }
 
-/** The low-res neighbourhood of a quad (a, e): rows a-1 .. a+1, columns e-1 .. e+1, clamped into the image;
- *  validity as factors of the bilinear weights. */
+/**
+ * The low-res neighbourhood of a quad (a, e): rows a-1 .. a+1, columns e-1 .. e+1; validity as factors of the bilinear weights.
+ * \tparam INTERIOR all of it lies in the image
+ */
+template <bool INTERIOR = false>
 struct Neighbourhood
 {
-    int row[3], column[3];
     float rowIn[3], columnIn[3];
     __device__ __forceinline__ Neighbourhood(int a, int e, int oH, int oW)
     {
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             const int y = a - 1 + k, x = e - 1 + k;
-            rowIn[k] = y >= 0 && y < oH ? 1.f : 0.f;
-            columnIn[k] = x >= 0 && x < oW ? 1.f : 0.f;
-            row[k] = min(max(y, 0), oH - 1);
-            column[k] = min(max(x, 0), oW - 1);
+            rowIn[k] = INTERIOR || (y >= 0 && y < oH) ? 1.f : 0.f;
+            columnIn[k] = INTERIOR || (x >= 0 && x < oW) ? 1.f : 0.f;
         }
-    }
-    template <typename T>
-    __device__ __forceinline__ void load(const PullPushView<T>& v, int b, int c, T (&out)[3][3]) const
-    {
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j) out[i][j] = *at(v, b, c, row[i], column[j]);
     }
     /** Weights of the own cell, the neighbour in the other row, in the other column, and the diagonal one, for pixel (di, dj) of the quad. */
     __device__ __forceinline__ void weights(int di, int dj, float (&w)[4]) const
@@ -245,7 +245,8 @@ struct QuadMix
 {
     T wm[2][2][4], n[2][2], weight[2][2];
     Reciprocal<T> inverse[2][2];
-    __device__ __forceinline__ QuadMix(const Neighbourhood& nb, const T (&maskLow)[3][3])
+    template <typename Neighbours>
+    __device__ __forceinline__ QuadMix(const Neighbours& nb, const T (&maskLow)[3][3])
     {
 #pragma unroll
         for (int di = 0; di < 2; ++di)
@@ -270,7 +271,7 @@ struct QuadMix
     __device__ __forceinline__ T sum(const T (&low)[3][3], int di, int dj) const
     {
         T v[4];
-        Neighbourhood::pick(low, di, dj, v);
+        Neighbourhood<>::pick(low, di, dj, v);
         T d = 0;
 #pragma unroll
         for (int k = 0; k < 4; ++k) d += wm[di][dj][k] * v[k];
@@ -278,175 +279,250 @@ struct QuadMix
     }
 };
 
-/** up for the quad (a, e) of the high-res level. */
-template <bool PAIRS, typename T>
-__device__ __forceinline__ void upQuad(const PullPushLevel<T>& high, const PullPushLevel<T>& low, int C, int b, int a, int e)
+/**
+ * The low-res pixels that the quads of a workgroup interpolate from, in LDS: QW x QH quads from (a0, e0) on and one more on every
+ * side, clamped into the image. A thread that loads the nine of its quad itself asks the memory pipeline for 45 values (4 channels), at 16
+ * cycles per instruction of a wavefront, and holds their addresses: 2048 x 2048 floats, the way up 39 us in 222 registers, from LDS 36 in
+ * 96, step B 73 and 70.
+ */
+template <typename T, int QW, int QH>
+struct LowTile
 {
-    const Neighbourhood nb(a, e, low.H, low.W);
-    T lowMask[3][3];
-    nb.load(low.maskPost, b, 0, lowMask);
-    const QuadMix<T> mix(nb, lowMask);
-    const bool second = 2 * e + 1 < high.W;
-    T m[2][2];
+    static constexpr int PITCH = QW + 2, ENTRIES = PITCH * (QH + 2), PLANES = pullpushChunk<T>() + 1;
+    typedef T Memory[PLANES][ENTRIES];
+
+    /** All threads of the workgroup; up to CHUNK channels from c0 on, and with the first of them the mask into the last plane. */
+    __device__ __forceinline__ static void stage(Memory& s, const PullPushLevel<T>& low, int C, int b, int c0, int a0, int e0)
+    {
+#pragma unroll 2
+        for (int i = threadIdx.x; i < ENTRIES; i += blockDim.x) {
+            const int a = min(max(a0 - 1 + i / PITCH, 0), low.H - 1), e = min(max(e0 - 1 + i % PITCH, 0), low.W - 1);
+            T v[PLANES];
 #pragma unroll
-    for (int di = 0; di < 2; ++di) {
-        m[di][0] = m[di][1] = T(0);
-        if (2 * a + di >= high.H) continue;
-        loadPair<PAIRS>(at(high.maskPre, b, 0, 2 * a + di, 2 * e), high.maskPre.x, second, m[di]);
-        if (!high.maskPost.p) continue;
-        T out[2];
+            for (int k = 0; k + 1 < PLANES; ++k)
+                if (c0 + k < C) v[k] = *at(low.dataPost, b, c0 + k, a, e);
+            if (c0 == 0) v[PLANES - 1] = *at(low.maskPost, b, 0, a, e);
 #pragma unroll
-        for (int dj = 0; dj < 2; ++dj)
-            out[dj] = m[di][dj] + (mix.n[di][dj] > 0 ? (1 - m[di][dj]) * (mix.n[di][dj] / mix.weight[di][dj]) : T(0));
-        storePair<PAIRS>(at(high.maskPost, b, 0, 2 * a + di, 2 * e), high.maskPost.x, second, out);
+            for (int k = 0; k + 1 < PLANES; ++k)
+                if (c0 + k < C) s[k][i] = v[k];
+            if (c0 == 0) s[PLANES - 1][i] = v[PLANES - 1];
+        }
     }
+    /** The neighbours of quad (la, le) of the tile. */
+    __device__ __forceinline__ static void load(const T (&plane)[ENTRIES], int la, int le, T (&out)[3][3])
+    {
+        const T* p = plane + (la * PITCH + le);
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) out[i][j] = p[i * PITCH + j];
+    }
+};
+
+/** up for the QW x QH quads from (a0, e0) on, a thread each (all threads of the workgroup call this). */
+template <bool PAIRS, int QW, int QH, typename T>
+__device__ __forceinline__ void upQuads(const PullPushLevel<T>& high, const PullPushLevel<T>& low, int C, int b, int a0, int e0,
+                                        typename LowTile<T, QW, QH>::Memory& sLow)
+{
+    typedef LowTile<T, QW, QH> Low;
     constexpr int CHUNK = pullpushChunk<T>();
+    const int la = threadIdx.x / QW, le = threadIdx.x % QW, a = a0 + la, e = e0 + le;
+    const bool mine = 2 * a < high.H && 2 * e < high.W, second = 2 * e + 1 < high.W;
+    T m[2][2];
     for (int c0 = 0; c0 < C; c0 += CHUNK) {
-        T lowData[CHUNK][3][3], v[CHUNK][2][2];
+        T v[CHUNK][2][2];
 #pragma unroll
-        for (int k = 0; k < CHUNK; ++k) {
-            if (c0 + k >= C) continue;
-            nb.load(low.dataPost, b, c0 + k, lowData[k]);
+        for (int di = 0; di < 2; ++di) {
+            if (!mine || 2 * a + di >= high.H) continue;
+            if (c0 == 0) {
+                m[di][0] = m[di][1] = T(0);
+                loadPair<PAIRS>(at(high.maskPre, b, 0, 2 * a + di, 2 * e), high.maskPre.x, second, m[di]);
+            }
 #pragma unroll
-            for (int di = 0; di < 2; ++di)
-                if (2 * a + di < high.H) loadPair<PAIRS>(at(high.dataPre, b, c0 + k, 2 * a + di, 2 * e), high.dataPre.x, second, v[k][di]);
+            for (int k = 0; k < CHUNK; ++k)
+                if (c0 + k < C) loadPair<PAIRS>(at(high.dataPre, b, c0 + k, 2 * a + di, 2 * e), high.dataPre.x, second, v[k][di]);
+        }
+        if (c0 > 0) __syncthreads();   // the channels in front of these have been read
+        Low::stage(sLow, low, C, b, c0, a0, e0);
+        __syncthreads();
+        if (!mine) continue;
+        const Neighbourhood<> nb(a, e, low.H, low.W);
+        T lowMask[3][3];
+        Low::load(sLow[Low::PLANES - 1], la, le, lowMask);
+        const QuadMix<T> mix(nb, lowMask);
+#pragma unroll
+        for (int di = 0; di < 2; ++di) {
+            if (2 * a + di >= high.H || c0 > 0 || !high.maskPost.p) continue;
+            T out[2];
+#pragma unroll
+            for (int dj = 0; dj < 2; ++dj)
+                out[dj] = m[di][dj] + (mix.n[di][dj] > 0 ? (1 - m[di][dj]) * (mix.n[di][dj] / mix.weight[di][dj]) : T(0));
+            storePair<PAIRS>(at(high.maskPost, b, 0, 2 * a + di, 2 * e), high.maskPost.x, second, out);
         }
 #pragma unroll
         for (int k = 0; k < CHUNK; ++k) {
             if (c0 + k >= C) continue;
+            T lowData[3][3];
+            Low::load(sLow[k], la, le, lowData);
 #pragma unroll
             for (int di = 0; di < 2; ++di) {
                 if (2 * a + di >= high.H) continue;
                 T out[2];
 #pragma unroll
                 for (int dj = 0; dj < 2; ++dj)
-                    out[dj] = m[di][dj] * v[k][di][dj] + (1 - m[di][dj]) * quotient(mix.sum(lowData[k], di, dj), mix.n[di][dj]);
+                    out[dj] = m[di][dj] * v[k][di][dj] + (1 - m[di][dj]) * quotient(mix.sum(lowData, di, dj), mix.n[di][dj]);
                 storePair<PAIRS>(at(high.dataPost, b, c0 + k, 2 * a + di, 2 * e), high.dataPost.x, second, out);
             }
         }
     }
 }
 
-constexpr int pullpushTileEntries(int tw, int th) { return 2 * (th + 2) * (2 * (tw + 2) + 1); }   // high-res pixels of a tile with its border
-
-/**
- * Step A for the TW x TH low-res pixels from (a0, e0) on, by a workgroup of TW * TH threads (all of them call this):
- *   gradDataPost_c of the low-res pixel = mask * sum over the 4 x 4 high-res pixels p that interpolate from it of w_p fill_c(p)
- *   gradMaskPost                        = sum of w_p (fillN(p) + sum_c fill_c(p) data_c)
- * with fill_c(p) the gradient of the weighted low-res sum d_c of p and fillN(p) that of its mask sum n. A thread forms these
- * terms for the quads of the tile and a border of one quad (34 x 10 quads for 32 x 8 pixels) and they wait in LDS, a
- * few channels at a time, until the low-res pixels gather them; fillN (the last plane) is summed over the channels there.
- */
-template <bool PAIRS, int TW, int TH, typename T>
-__device__ __forceinline__ void gradientUpTile(const PullPushLevel<T>& high, const PullPushLevel<T>& low, int C, int b, int a0, int e0,
-                                               T (&sFill)[pullpushChunk<T>() + 1][pullpushTileEntries(TW, TH)])
+/** The value of the lane in front (STEP = -1) or behind (1) in a row of 16 lanes; zero where there is none. All lanes of the wavefront. */
+template <int STEP, typename T>
+__device__ __forceinline__ T besides(T v)
 {
-    constexpr int THREADS = TW * TH, QW = TW + 2, QH = TH + 2, QUADS = QW * QH, CHUNK = pullpushChunk<T>();
-    constexpr int STRIDE = 2 * QW + 1;   // entries per row of high-res pixels
-    const int la = threadIdx.x / TW, le = threadIdx.x % TW;
-    const int a = a0 + la, e = e0 + le;
-    const bool mine = a < low.H && e < low.W;
-    auto gather = [&](const T* plane) {
-        T sum = 0;
+    constexpr int CONTROL = STEP < 0 ? 0x111 : 0x101;   // row_shr:1, row_shl:1
+    int words[sizeof(T) / 4];
+    __builtin_memcpy(words, &v, sizeof(T));
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const T* row = plane + (2 * la + 1 + i) * STRIDE + 2 * le + 1;
-            const float wr = (i == 1 || i == 2) ? 0.75f : 0.25f;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) sum += (wr * ((j == 1 || j == 2) ? 0.75f : 0.25f)) * row[j];
-        }
-        return sum;
-    };
-    T lowMask = 0, gradMask = 0;
-    if (mine) lowMask = *at(low.maskPost, b, 0, a, e);
-    for (int c0 = 0; c0 < C; c0 += CHUNK) {
-        __syncthreads();   // what the previous channels (or tile) left has been gathered
-#pragma unroll 1
-        for (int quad = threadIdx.x; quad < QUADS; quad += THREADS) {
-            const int qa = a0 - 1 + quad / QW, qe = e0 - 1 + quad % QW;
-            const int at0 = 2 * (quad / QW) * STRIDE + 2 * (quad % QW);
-            T fill[CHUNK][2][2], fillN[2][2];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                fillN[i >> 1][i & 1] = T(0);
-#pragma unroll
-                for (int k = 0; k < CHUNK; ++k) fill[k][i >> 1][i & 1] = T(0);
-            }
-            if (qa >= 0 && qe >= 0 && 2 * qa < high.H && 2 * qe < high.W) {
-                const Neighbourhood nb(qa, qe, low.H, low.W);
-                const bool second = 2 * qe + 1 < high.W;
-                T masks[3][3], lowData[CHUNK][3][3], m[2][2], gm[2][2];
-                nb.load(low.maskPost, b, 0, masks);
-#pragma unroll
-                for (int di = 0; di < 2; ++di) {
-                    m[di][0] = m[di][1] = T(0);
-                    gm[di][0] = gm[di][1] = T(0);
-                    if (2 * qa + di >= high.H) continue;
-                    loadPair<PAIRS>(at(high.maskPre, b, 0, 2 * qa + di, 2 * qe), high.maskPre.x, second, m[di]);
-                    if (c0 == 0 && high.gradMaskPost.p)
-                        loadPair<PAIRS>(at(high.gradMaskPost, b, 0, 2 * qa + di, 2 * qe), high.gradMaskPost.x, second, gm[di]);
-                }
-#pragma unroll
-                for (int k = 0; k < CHUNK; ++k) {
-                    if (c0 + k >= C) continue;
-                    nb.load(low.dataPost, b, c0 + k, lowData[k]);
-#pragma unroll
-                    for (int di = 0; di < 2; ++di)
-                        if (2 * qa + di < high.H)   // (the gradient: turned into the fill below)
-                            loadPair<PAIRS>(at(high.gradDataPost, b, c0 + k, 2 * qa + di, 2 * qe), high.gradDataPost.x, second, fill[k][di]);
-                }
-                const QuadMix<T> mix(nb, masks);
-#pragma unroll
-                for (int di = 0; di < 2; ++di)
-#pragma unroll
-                    for (int dj = 0; dj < 2; ++dj) {
-                        if (2 * qa + di >= high.H || (dj == 1 && !second)) {
-                            // outside: passes nothing down
-#pragma unroll
-                            for (int k = 0; k < CHUNK; ++k) fill[k][di][dj] = T(0);
-                            continue;
-                        }
-                        if (c0 == 0) fillN[di][dj] = gm[di][dj] * ((1 - m[di][dj]) / mix.weight[di][dj]);
-#pragma unroll
-                        for (int k = 0; k < CHUNK; ++k) {
-                            if (c0 + k >= C) continue;
-                            fill[k][di][dj] = mix.inverse[di][dj](fill[k][di][dj] * (1 - m[di][dj]));
-                            fillN[di][dj] -= fill[k][di][dj] * mix.inverse[di][dj](mix.sum(lowData[k], di, dj));
-                        }
-                    }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int entry = at0 + (i >> 1) * STRIDE + (i & 1);
-#pragma unroll
-                for (int k = 0; k < CHUNK; ++k)
-                    if (c0 + k < C) sFill[k][entry] = fill[k][i >> 1][i & 1];
-                sFill[CHUNK][entry] = (c0 == 0 ? T(0) : sFill[CHUNK][entry]) + fillN[i >> 1][i & 1];
-            }
-        }
-        __syncthreads();
-        if (!mine) continue;
-#pragma unroll
-        for (int k = 0; k < CHUNK; ++k) {
-            if (c0 + k >= C) continue;
-            const T sum = gather(sFill[k]);
-            gradMask += sum * *at(low.dataPost, b, c0 + k, a, e);
-            *at(low.gradDataPost, b, c0 + k, a, e) = sum * lowMask;
-        }
-    }
-    if (mine) *at(low.gradMaskPost, b, 0, a, e) = gradMask + gather(sFill[CHUNK]);
+    for (int i = 0; i < static_cast<int>(sizeof(T) / 4); ++i) words[i] = __builtin_amdgcn_update_dpp(0, words[i], CONTROL, 0xf, 0xf, true);
+    __builtin_memcpy(&v, words, sizeof(T));
+    return v;
 }
 
 /**
- * Step B for the quad (a, e) of the high-res level: the gradients of its pixels before inpainting.
+ * Step A for the TW x TH low-res pixels from (a0, e0) on, by a workgroup of a thread per quad of the tile and a border of one quad (all
+ * of them call this; a row of quads is a row of 16 lanes):
+ *   gradDataPost_c of the low-res pixel = mask * sum over the 4 x 4 high-res pixels p that interpolate from it of w_p fill_c(p)
+ *   gradMaskPost                        = sum of w_p (fillN(p) + sum_c fill_c(p) data_c)
+ * with fill_c(p) the gradient of the weighted low-res sum d_c of p and fillN(p) that of its mask sum n. The weights are
+ * products of 1/4, 3/4, 3/4, 1/4 in both directions: a thread forms the terms of its quad's four pixels and adds up those of
+ * a row with the quads besides it, and what remains of the rows above and below comes through LDS, two values per quad and channel. (All
+ * terms through LDS and 16 of them read per low-res pixel and channel: two per bank and instruction, the same time on 2048 x 2048
+ * floats with the tests for the border taken out of the interior. Bound by its vector instructions, about 700 per quad: 33 of 45 us.)
+ */
+template <bool PAIRS, bool INTERIOR, int TW, int TH, typename T>
+__device__ __forceinline__ void gradientUpTile(const PullPushLevel<T>& high, const PullPushLevel<T>& low, int C, int b, int a0, int e0,
+                                               T (&sRows)[pullpushChunk<T>() + 1][2][(TW + 2) * (TH + 2)],
+                                               typename LowTile<T, TW + 2, TH + 2>::Memory& sLow)
+{
+    typedef LowTile<T, TW + 2, TH + 2> Low;
+    constexpr int QW = TW + 2, CHUNK = pullpushChunk<T>();
+    static_assert(QW == 16, "a row of quads is a row of 16 lanes");
+    const int tid = threadIdx.x, la = tid / QW, le = tid % QW;
+    const int qa = a0 - 1 + la, qe = e0 - 1 + le;   // the quad, and the low-res pixel that it lies in
+    const bool inside = INTERIOR || (qa >= 0 && qe >= 0 && 2 * qa < high.H && 2 * qe < high.W);
+    const bool mine = la >= 1 && la <= TH && le >= 1 && le <= TW && (INTERIOR || (qa < low.H && qe < low.W));
+    const bool second = INTERIOR || 2 * qe + 1 < high.W;
+    bool in[2][2];   // outside: passes nothing down
+#pragma unroll
+    for (int i = 0; i < 4; ++i) in[i >> 1][i & 1] = INTERIOR || (inside && 2 * qa + (i >> 1) < high.H && ((i & 1) == 0 || second));
+    T fillN[2][2], m[2][2], gradMask = 0;
+    // the sum along the rows of the terms of a quad and of those besides it
+    auto along = [&](const T (&f)[2][2], T (&rows)[2]) {
+#pragma unroll
+        for (int di = 0; di < 2; ++di) rows[di] = 0.75f * (f[di][0] + f[di][1]) + 0.25f * (besides<-1>(f[di][1]) + besides<1>(f[di][0]));
+    };
+    auto down = [&](const T (&rows)[2], const T (&other)[2][(TW + 2) * (TH + 2)]) {
+        return 0.75f * (rows[0] + rows[1]) + 0.25f * (other[1][tid - QW] + other[0][tid + QW]);
+    };
+    for (int c0 = 0; c0 < C; c0 += CHUNK) {
+        if (c0 > 0) ldsBarrier();   // what the channels in front of these left has been read
+        Low::stage(sLow, low, C, b, c0, a0 - 1, e0 - 1);
+        ldsBarrier();
+        T fill[CHUNK][2][2], gm[2][2];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            gm[i >> 1][i & 1] = T(0);
+#pragma unroll
+            for (int k = 0; k < CHUNK; ++k) fill[k][i >> 1][i & 1] = T(0);
+        }
+        if (inside) {
+#pragma unroll
+            for (int di = 0; di < 2; ++di) {
+                if (!INTERIOR && 2 * qa + di >= high.H) continue;
+                if (c0 == 0) {
+                    m[di][0] = m[di][1] = T(0);
+                    loadPair<PAIRS>(at(high.maskPre, b, 0, 2 * qa + di, 2 * qe), high.maskPre.x, second, m[di]);
+                    if (high.gradMaskPost.p)
+                        loadPair<PAIRS>(at(high.gradMaskPost, b, 0, 2 * qa + di, 2 * qe), high.gradMaskPost.x, second, gm[di]);
+                }
+#pragma unroll
+                for (int k = 0; k < CHUNK; ++k)   // (the gradient: turned into the fill below)
+                    if (c0 + k < C) loadPair<PAIRS>(at(high.gradDataPost, b, c0 + k, 2 * qa + di, 2 * qe), high.gradDataPost.x, second, fill[k][di]);
+            }
+        }
+        {
+            const Neighbourhood<INTERIOR> nb(qa, qe, low.H, low.W);
+            T masks[3][3];
+            Low::load(sLow[CHUNK], la, le, masks);
+            const QuadMix<T> mix(nb, masks);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int di = i >> 1, dj = i & 1;
+                if (c0 == 0) fillN[di][dj] = high.gradMaskPost.p && in[di][dj] ? gm[di][dj] * ((1 - m[di][dj]) / mix.weight[di][dj]) : T(0);
+            }
+#pragma unroll
+            for (int k = 0; k < CHUNK; ++k) {
+                if (c0 + k >= C) continue;
+                T lowData[3][3];
+                Low::load(sLow[k], la, le, lowData);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int di = i >> 1, dj = i & 1;
+                    const T f = mix.inverse[di][dj](fill[k][di][dj] * (1 - m[di][dj]));
+                    fill[k][di][dj] = in[di][dj] ? f : T(0);
+                    if (in[di][dj]) fillN[di][dj] -= f * mix.inverse[di][dj](mix.sum(lowData, di, dj));
+                }
+            }
+        }
+        T rows[CHUNK + 1][2];
+#pragma unroll
+        for (int k = 0; k < CHUNK; ++k) {
+            if (c0 + k >= C) continue;
+            along(fill[k], rows[k]);
+            sRows[k][0][tid] = rows[k][0];
+            sRows[k][1][tid] = rows[k][1];
+        }
+        const bool last = c0 + CHUNK >= C;
+        if (last) {
+            along(fillN, rows[CHUNK]);
+            sRows[CHUNK][0][tid] = rows[CHUNK][0];
+            sRows[CHUNK][1][tid] = rows[CHUNK][1];
+        }
+        ldsBarrier();
+        if (!mine) continue;
+        const int own = (la + 1) * Low::PITCH + le + 1;
+        const T lowMask = sLow[CHUNK][own];
+#pragma unroll
+        for (int k = 0; k < CHUNK; ++k) {
+            if (c0 + k >= C) continue;
+            const T sum = down(rows[k], sRows[k]);
+            gradMask += sum * sLow[k][own];
+            *at(low.gradDataPost, b, c0 + k, qa, qe) = sum * lowMask;
+        }
+        if (last) *at(low.gradMaskPost, b, 0, qa, qe) = gradMask + down(rows[CHUNK], sRows[CHUNK]);
+    }
+}
+
+/**
+ * Step B for the QW x QH quads from (a0, e0) on: the gradients of their pixels before inpainting, a thread per quad (all threads of
+ * the workgroup call this).
  * \tparam ACCUMULATE add to what is there
  */
-template <bool PAIRS, bool ACCUMULATE, typename T>
-__device__ __forceinline__ void gradientQuad(const PullPushLevel<T>& high, const PullPushLevel<T>& low, int C, int b, int a, int e)
+template <bool PAIRS, bool ACCUMULATE, int QW, int QH, typename T>
+__device__ __forceinline__ void gradientQuads(const PullPushLevel<T>& high, const PullPushLevel<T>& low, int C, int b, int a0, int e0,
+                                              typename LowTile<T, QW, QH>::Memory& sLow)
 {
-    const Neighbourhood nb(a, e, low.H, low.W);
+    typedef LowTile<T, QW, QH> Low;
+    constexpr int STAGED = pullpushChunk<T>();
+    const int la = threadIdx.x / QW, le = threadIdx.x % QW, a = a0 + la, e = e0 + le;
+    const bool mine = 2 * a < high.H && 2 * e < high.W;
+    Low::stage(sLow, low, C, b, 0, a0, e0);
+    __syncthreads();
+    const Neighbourhood<> nb(a, e, low.H, low.W);
     T lowMask[3][3];
-    nb.load(low.maskPost, b, 0, lowMask);
+    Low::load(sLow[STAGED], la, le, lowMask);
     const QuadMix<T> mix(nb, lowMask);
     const bool second = 2 * e + 1 < high.W;
     // the low-res windows the pixels lie in: (a, e), and of odd sizes also those of the row above and the column to the
@@ -460,7 +536,7 @@ __device__ __forceinline__ void gradientQuad(const PullPushLevel<T>& high, const
 #pragma unroll
         for (int we = 0; we < 2; ++we) {
             const int y = a - wa, x = e - we;
-            in[wa][we] = (wa == 0 || oddH) && (we == 0 || oddW) && y >= 0 && x >= 0 && y < low.H && x < low.W;
+            in[wa][we] = mine && (wa == 0 || oddH) && (we == 0 || oddW) && y >= 0 && x >= 0 && y < low.H && x < low.W;
             most[wa][we] = gradMost[wa][we] = T(0);
             if (!in[wa][we]) continue;
             sums[wa][we] = Reciprocal<T>(*at(low.maskSum, b, 0, y, x));
@@ -471,7 +547,7 @@ __device__ __forceinline__ void gradientQuad(const PullPushLevel<T>& high, const
 #pragma unroll
     for (int di = 0; di < 2; ++di) {
         m[di][0] = m[di][1] = gradMask[di][0] = gradMask[di][1] = T(0);
-        if (2 * a + di >= high.H) continue;
+        if (!mine || 2 * a + di >= high.H) continue;
         loadPair<PAIRS>(at(high.maskPre, b, 0, 2 * a + di, 2 * e), high.maskPre.x, second, m[di]);
         T gm[2] = {T(0), T(0)};
         if (high.gradMaskPost.p)
@@ -491,12 +567,18 @@ __device__ __forceinline__ void gradientQuad(const PullPushLevel<T>& high, const
     }
     constexpr int CHUNK = 1;   // (more of them in flight cost more wavefronts than they hide: 2048 x 2048 floats 70 us with one, 98 us with two)
     for (int c0 = 0; c0 < C; c0 += CHUNK) {
+        if (c0 > 0 && c0 % STAGED == 0) {
+            __syncthreads();   // the channels in front of these have been read
+            Low::stage(sLow, low, C, b, c0, a0, e0);
+            __syncthreads();
+        }
+        if (!mine) continue;
         T lowData[CHUNK][3][3], v[CHUNK][2][2], g[CHUNK][2][2], before[CHUNK][2][2];
         T mean[CHUNK][2][2], grad[CHUNK][2][2];   // of the windows
 #pragma unroll
         for (int k = 0; k < CHUNK; ++k) {
             if (c0 + k >= C) continue;
-            nb.load(low.dataPost, b, c0 + k, lowData[k]);
+            Low::load(sLow[(c0 + k) % STAGED], la, le, lowData[k]);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int wa = i >> 1, we = i & 1;
@@ -541,6 +623,7 @@ __device__ __forceinline__ void gradientQuad(const PullPushLevel<T>& high, const
             }
         }
     }
+    if (!mine) return;
 #pragma unroll
     for (int di = 0; di < 2; ++di) {
         if (2 * a + di >= high.H) continue;
@@ -556,21 +639,25 @@ __device__ __forceinline__ void gradientQuad(const PullPushLevel<T>& high, const
 }
 
 constexpr int TILE_W = 32, TILE_H = 8;   // of the kernels with a launch per level: 256 threads
+// ... and of step A: with their border the quads of a tile are as many as there are threads, in rows of 16 lanes (32 x 8 pixels by 256
+// threads were 340 quads, two rounds with the second a third full; 2048 x 2048 floats 51 us, now 45)
+constexpr int UP_TILE_W = 14, UP_TILE_H = 14, UP_THREADS = (UP_TILE_W + 2) * (UP_TILE_H + 2);
 
 /**
  * Tile of this workgroup: a stack of B images of width x height items in tiles of TILE_W x TILE_H. Workgroups go to the 8 XCDs
  * in turn; every XCD gets a run of consecutive tiles, whose borders then meet in its own L2.
  */
+template <int TW = TILE_W, int TH = TILE_H>
 __device__ __forceinline__ void tileOf(int width, int height, int& b, int& a0, int& e0)
 {
     constexpr unsigned XCDS = 8;
     const unsigned xcd = blockIdx.x % XCDS, perXcd = gridDim.x / XCDS, more = gridDim.x % XCDS;
     const unsigned tile = xcd * perXcd + min(xcd, more) + blockIdx.x / XCDS;
-    const unsigned tilesX = (width + TILE_W - 1) / TILE_W, tilesY = (height + TILE_H - 1) / TILE_H;
+    const unsigned tilesX = (width + TW - 1) / TW, tilesY = (height + TH - 1) / TH;
     const unsigned row = tile / tilesX;
-    e0 = static_cast<int>(tile - row * tilesX) * TILE_W;
+    e0 = static_cast<int>(tile - row * tilesX) * TW;
     b = static_cast<int>(row / tilesY);
-    a0 = static_cast<int>(row - b * tilesY) * TILE_H;
+    a0 = static_cast<int>(row - b * tilesY) * TH;
 }
 
 /**
@@ -619,6 +706,8 @@ struct LdsLevel
     __device__ __forceinline__ entry& maskSum(int y, int x) const { return at(maskSumP, 0, y, x); }
     __device__ __forceinline__ entry& maskPost(int y, int x) const { return at(maskPostP, 0, y, x); }
     __device__ __forceinline__ entry& dataPost(int c, int y, int x) const { return at(dataPostP, c, y, x); }
+    __device__ __forceinline__ void setGradMaskPost(int y, int x, T v) const { gradMaskPost(y, x) = v; }
+    __device__ __forceinline__ void setGradDataPost(int c, int y, int x, T v) const { gradDataPost(c, y, x) = v; }
     __device__ __forceinline__ entry& gradMaskPost(int y, int x) const { return at(gradMaskPostP, 0, y, x); }
     __device__ __forceinline__ entry& gradDataPost(int c, int y, int x) const { return at(gradDataPostP, c, y, x); }
     __device__ __forceinline__ entry& gradMaskPre(int y, int x) const { return at(gradMaskPreP, 0, y, x); }
@@ -675,6 +764,161 @@ struct TopLevel
     __device__ __forceinline__ T& gradDataPre(int c, int y, int x) const { return *at(l.gradDataPre, b, c, y, x); }
 };
 
+/** What the steps read of a low-res level in global memory, all planes of which have the same pitch (the workspaces'). */
+template <typename T>
+struct GlobalLow
+{
+    int H, W, pitch;
+    long long plane;
+    const T *maskPreP, *dataPreP, *maskSumP, *maskPostP, *dataPostP, *gradMaskPreP, *gradDataPreP;
+    __device__ __forceinline__ GlobalLow(const PullPushLevel<T>& l, int b)
+        : H(l.H), W(l.W), pitch(static_cast<int>(l.maskPre.y)), plane(l.dataPre.c), maskPreP(l.maskPre.p + b * l.maskPre.b),
+          dataPreP(l.dataPre.p + b * l.dataPre.b), maskSumP(l.maskSum.p + b * l.maskSum.b), maskPostP(l.maskPost.p + b * l.maskPost.b),
+          dataPostP(l.dataPost.p + b * l.dataPost.b), gradMaskPreP(l.gradMaskPre.p + b * l.gradMaskPre.b),
+          gradDataPreP(l.gradDataPre.p + b * l.gradDataPre.b)
+    {
+    }
+    __device__ __forceinline__ T gradMaskPre(int a, int e) const { return gradMaskPreP[a * pitch + e]; }
+    __device__ __forceinline__ T gradDataPre(int c, int a, int e) const { return gradDataPreP[c * plane + a * pitch + e]; }
+};
+
+/** Rows and columns of a level that a workgroup works on. */
+struct PullPushRegion
+{
+    int y0, y1, x0, x1;
+    __device__ __forceinline__ int rows() const { return y1 - y0; }
+    __device__ __forceinline__ int columns() const { return x1 - x0; }
+};
+
+/** C + 1 planes of a region in LDS: of a mask, and of the channels. Zero bytes behind the entries of the region before it. */
+template <typename T>
+struct LdsTile
+{
+    typedef typename LdsLevel<T>::entry entry;
+    entry* p;
+    int y0, x0, pitch, plane;
+    __device__ __forceinline__ LdsTile(entry* memory, const PullPushRegion& r)
+        : p(memory), y0(r.y0), x0(r.x0), pitch(r.columns()), plane(r.rows() * r.columns()) {}
+    __device__ __forceinline__ entry& mask(int y, int x) const { return p[(y - y0) * pitch + (x - x0)]; }
+    __device__ __forceinline__ entry& data(int c, int y, int x) const { return p[(c + 1) * plane + (y - y0) * pitch + (x - x0)]; }
+};
+
+/** What the steps read and write of a high-res level in global memory. */
+template <typename T>
+struct GlobalHigh
+{
+    const PullPushLevel<T>& l;
+    int b, H, W;
+    __device__ __forceinline__ GlobalHigh(const PullPushLevel<T>& level, int image) : l(level), b(image), H(level.H), W(level.W) {}
+    __device__ __forceinline__ bool hasMaskPost() const { return l.maskPost.p != nullptr; }
+    __device__ __forceinline__ bool hasGradMaskPost() const { return l.gradMaskPost.p != nullptr; }
+    __device__ __forceinline__ T maskPre(int y, int x) const { return *at(l.maskPre, b, 0, y, x); }
+    __device__ __forceinline__ T dataPre(int c, int y, int x) const { return *at(l.dataPre, b, c, y, x); }
+    __device__ __forceinline__ T gradMaskPost(int y, int x) const { return *at(l.gradMaskPost, b, 0, y, x); }
+    __device__ __forceinline__ T gradDataPost(int c, int y, int x) const { return *at(l.gradDataPost, b, c, y, x); }
+    __device__ __forceinline__ T& maskPost(int y, int x) const { return *at(l.maskPost, b, 0, y, x); }
+    __device__ __forceinline__ T& dataPost(int c, int y, int x) const { return *at(l.dataPost, b, c, y, x); }
+    __device__ __forceinline__ T& gradMaskPre(int y, int x) const { return *at(l.gradMaskPre, b, 0, y, x); }
+    __device__ __forceinline__ T& gradDataPre(int c, int y, int x) const { return *at(l.gradDataPre, b, c, y, x); }
+};
+/** ... whose gradients before inpainting stay in LDS, and a low-res level with its own there. */
+template <typename T>
+struct GradientTileHigh : GlobalHigh<T>
+{
+    LdsTile<T> tile;
+    __device__ __forceinline__ GradientTileHigh(const PullPushLevel<T>& level, int image, const LdsTile<T>& t) : GlobalHigh<T>(level, image), tile(t) {}
+    __device__ __forceinline__ typename LdsTile<T>::entry& gradMaskPre(int y, int x) const { return tile.mask(y, x); }
+    __device__ __forceinline__ typename LdsTile<T>::entry& gradDataPre(int c, int y, int x) const { return tile.data(c, y, x); }
+};
+template <typename T>
+struct GradientTileLow : GlobalLow<T>
+{
+    LdsTile<T> tile;
+    __device__ __forceinline__ GradientTileLow(const PullPushLevel<T>& level, int image, const LdsTile<T>& t) : GlobalLow<T>(level, image), tile(t) {}
+    __device__ __forceinline__ T gradMaskPre(int a, int e) const { return tile.mask(a, e); }
+    __device__ __forceinline__ T gradDataPre(int c, int a, int e) const { return tile.data(c, a, e); }
+};
+
+/** An inpainted low-res level in LDS, and a high-res level that is inpainted into LDS, into global memory where it is owned, or both. */
+template <typename T>
+struct InpaintedTileLow
+{
+    int H, W, pitch, plane;
+    typename LdsTile<T>::entry *maskPostP, *dataPostP;
+    __device__ __forceinline__ InpaintedTileLow(const PullPushLevel<T>& l, const LdsTile<T>& t)
+        : H(l.H), W(l.W), pitch(t.pitch), plane(t.plane), maskPostP(t.p - (t.y0 * t.pitch + t.x0)), dataPostP(maskPostP + t.plane) {}
+};
+
+/**
+ * Where workgroups of PULLPUSH_TAIL_BLOCK lanes take tiles of the finest of several levels and what the coarser ones below have to
+ * do with them. Sizes in LDS: a region of level k has at most (tile >> k) + TREE_BORDER rows and columns.
+ */
+constexpr int TREE_BORDER = 5;
+__device__ __forceinline__ PullPushRegion treeTile(int H, int W, int tile, int& b)
+{
+    constexpr unsigned XCDS = 8;
+    const unsigned xcd = blockIdx.x % XCDS, perXcd = gridDim.x / XCDS, more = gridDim.x % XCDS;
+    const unsigned index = xcd * perXcd + min(xcd, more) + blockIdx.x / XCDS;
+    const unsigned tilesX = (W + tile - 1) / tile, tilesY = (H + tile - 1) / tile;
+    const unsigned row = index / tilesX;
+    b = static_cast<int>(row / tilesY);
+    const int x0 = static_cast<int>(index - row * tilesX) * tile, y0 = static_cast<int>(row - b * tilesY) * tile;
+    return {y0, min(y0 + tile, H), x0, min(x0 + tile, W)};
+}
+template <typename T>
+__device__ __forceinline__ typename LdsLevel<T>::entry* treeMemory(typename LdsLevel<T>::entry* memory, const PullPushTree<T>& tree, int C, int k)
+{
+    for (int i = 1; i < k; ++i) memory += (C + 1) * ((tree.tile >> i) + TREE_BORDER) * ((tree.tile >> i) + TREE_BORDER);
+    return memory;
+}
+
+/** A high-res level with its pixels before inpainting in LDS. */
+template <typename T>
+struct DownTileHigh
+{
+    int H, W;
+    LdsTile<T> tile;
+    __device__ __forceinline__ DownTileHigh(const PullPushLevel<T>& l, const LdsTile<T>& t) : H(l.H), W(l.W), tile(t) {}
+    __device__ __forceinline__ T maskPre(int y, int x) const { return tile.mask(y, x); }
+    __device__ __forceinline__ T dataPre(int c, int y, int x) const { return tile.data(c, y, x); }
+};
+/** A high-res level with the gradients of its inpainted pixels in LDS, and a low-res one that receives its own there, in global memory where it is owned, or both. */
+template <typename T>
+struct UpTileHigh : GlobalHigh<T>
+{
+    LdsTile<T> tile;
+    __device__ __forceinline__ UpTileHigh(const PullPushLevel<T>& level, int image, const LdsTile<T>& t) : GlobalHigh<T>(level, image), tile(t) {}
+    __device__ __forceinline__ T gradMaskPost(int y, int x) const { return tile.mask(y, x); }
+    __device__ __forceinline__ T gradDataPost(int c, int y, int x) const { return tile.data(c, y, x); }
+};
+template <typename T>
+struct UpTileLow : GlobalLow<T>
+{
+    const PullPushLevel<T>& l;
+    int b;
+    PullPushRegion owned;
+    bool keep;
+    LdsTile<T> tile;
+    __device__ __forceinline__ UpTileLow(const PullPushLevel<T>& level, int image, const PullPushRegion& own, bool keepTile, const LdsTile<T>& t)
+        : GlobalLow<T>(level, image), l(level), b(image), owned(own), keep(keepTile), tile(t) {}
+    __device__ __forceinline__ bool own(int a, int e) const { return a >= owned.y0 && a < owned.y1 && e >= owned.x0 && e < owned.x1; }
+    __device__ __forceinline__ void setGradDataPost(int c, int a, int e, T v) const
+    {
+        if (own(a, e)) *at(l.gradDataPost, b, c, a, e) = v;
+        if (keep) tile.data(c, a, e) = v;
+    }
+    __device__ __forceinline__ void setGradMaskPost(int a, int e, T v) const
+    {
+        if (own(a, e)) *at(l.gradMaskPost, b, 0, a, e) = v;
+        if (keep) tile.mask(a, e) = v;
+    }
+    __device__ __forceinline__ T maskPost(int a, int e) const { return this->maskPostP[a * this->pitch + e]; }
+    __device__ __forceinline__ T dataPost(int c, int a, int e) const { return this->dataPostP[c * this->plane + a * this->pitch + e]; }
+};
+/** Rows (and columns) at most of a region of level k in LDS, of a tree that ends at level 'last' with (tile >> last) of them. */
+__device__ __forceinline__ int treeDownSize(int tile, int last, int k) { return (tile >> k) + (1 << (last - k)) - 1; }
+__device__ __forceinline__ int treeUpSize(int tile, int last, int k) { return (tile >> k) + 2 * ((1 << (last - k)) - 1); }
+
 /**
  * The steps of the coarse levels, by one compute unit: a chain of a few dependent loads and a division per step, and on the larger
  * levels vector instructions. An item is a pixel with all its channels where that fills the workgroup, on smaller levels 2^n neighbouring
@@ -714,18 +958,27 @@ struct TailSteps
         return v;
     }
 
-    template <typename High>
-    __device__ __forceinline__ void down(const High& high, const LdsLevel<T>& low) const
+    /** down for a region of the low-res level: store(c, a, e, value), storeMask(a, e, mask, sum of masks). */
+    template <typename High, typename Store, typename StoreMask>
+    __device__ __forceinline__ void downTo(const High& high, const PullPushRegion& r, const Store& store, const StoreMask& storeMask) const
     {
-        const int rows = 2 + (high.H & 1), columns = 2 + (high.W & 1);
-        const int log2 = lanesLog2(low.H * low.W, C);
-        forEach(0, 0, low.H, low.W, log2, [&](int a, int e, int lane) {
-            T m[3][3];
+        if ((high.H | high.W) & 1) downTo<true>(high, r, store, storeMask);
+        else downTo<false>(high, r, store, storeMask);
+    }
+    /** \tparam ODD some size is odd: windows of three rows or columns */
+    template <bool ODD, typename High, typename Store, typename StoreMask>
+    __device__ __forceinline__ void downTo(const High& high, const PullPushRegion& r, const Store& store, const StoreMask& storeMask) const
+    {
+        constexpr int MOST = ODD ? 3 : 2;
+        const int rows = ODD ? 2 + (high.H & 1) : 2, columns = ODD ? 2 + (high.W & 1) : 2;
+        const int log2 = lanesLog2(r.rows() * r.columns(), C);
+        forEach(r.y0, r.x0, r.rows(), r.columns(), log2, [&](int a, int e, int lane) {
+            T m[MOST][MOST];
             T sum = 0, most = 0;
 #pragma unroll
-            for (int j = 0; j < 3; ++j)
+            for (int j = 0; j < MOST; ++j)
 #pragma unroll
-                for (int i = 0; i < 3; ++i) {
+                for (int i = 0; i < MOST; ++i) {
                     m[i][j] = T(0);
                     if (i >= rows || j >= columns) continue;
                     m[i][j] = high.maskPre(2 * a + i, 2 * e + j);
@@ -735,17 +988,42 @@ struct TailSteps
             for (int c = lane; c < C; c += 1 << log2) {
                 T d = 0;
 #pragma unroll
-                for (int j = 0; j < 3; ++j)
+                for (int j = 0; j < MOST; ++j)
 #pragma unroll
-                    for (int i = 0; i < 3; ++i)
+                    for (int i = 0; i < MOST; ++i)
                         if (i < rows && j < columns) d += m[i][j] * high.dataPre(c, 2 * a + i, 2 * e + j);
-                low.dataPre(c, a, e) = quotient(d, sum);
+                store(c, a, e, quotient(d, sum));
             }
-            if (lane == 0) {
-                low.maskPre(a, e) = most;
-                low.maskSum(a, e) = sum;
-            }
+            if (lane == 0) storeMask(a, e, most, sum);
         });
+    }
+    template <typename High>
+    __device__ __forceinline__ void down(const High& high, const LdsLevel<T>& low) const
+    {
+        downTo(high, PullPushRegion{0, low.H, 0, low.W}, [&](int c, int a, int e, T v) { low.dataPre(c, a, e) = v; },
+               [&](int a, int e, T most, T sum) {
+                   low.maskPre(a, e) = most;
+                   low.maskSum(a, e) = sum;
+               });
+    }
+    /** ... into global memory what is owned, all of it into a tile as well. */
+    template <typename High>
+    __device__ __forceinline__ void downRegion(const High& high, const GlobalHigh<T>& low, const PullPushRegion& r, const PullPushRegion& owned, bool keep,
+                                               const LdsTile<T>& tile) const
+    {
+        auto own = [&](int a, int e) { return a >= owned.y0 && a < owned.y1 && e >= owned.x0 && e < owned.x1; };
+        downTo(high, r,
+               [&](int c, int a, int e, T v) {
+                   if (own(a, e)) *at(low.l.dataPre, low.b, c, a, e) = v;
+                   if (keep) tile.data(c, a, e) = v;
+               },
+               [&](int a, int e, T most, T sum) {
+                   if (own(a, e)) {
+                       *at(low.l.maskPre, low.b, 0, a, e) = most;
+                       *at(low.l.maskSum, low.b, 0, a, e) = sum;
+                   }
+                   if (keep) tile.mask(a, e) = most;
+               });
     }
 
     /** The low-res neighbours of high-res pixel (y, x): the own cell, the one in the other row, in the other column, the diagonal one. */
@@ -753,7 +1031,8 @@ struct TailSteps
     {
         int at[4];
         T wm[4], n, weight;
-        __device__ __forceinline__ Mix(int y, int x, const LdsLevel<T>& low)
+        template <typename Low>
+        __device__ __forceinline__ Mix(int y, int x, const Low& low)
         {
             const int row = y >> 1, column = x >> 1;
             const int otherRow = row - 1 + 2 * (y & 1), otherColumn = column - 1 + 2 * (x & 1);
@@ -771,9 +1050,10 @@ struct TailSteps
                 n += wm[k];
             }
         }
-        __device__ __forceinline__ T sum(const LdsLevel<T>& low, int c) const
+        template <typename Low>
+        __device__ __forceinline__ T sum(const Low& low, int c) const
         {
-            const entry* data = low.dataPostP + c * low.plane;
+            const auto* data = low.dataPostP + c * low.plane;
             T d = 0;
 #pragma unroll
             for (int k = 0; k < 4; ++k) d += wm[k] * data[at[k]];
@@ -794,19 +1074,45 @@ struct TailSteps
         });
     }
 
-    /** Step A (see gradientUpTile). fill: room for fillEntries entries, at least (C + 1) x 4 rows of the high-res level and a border. */
-    template <typename High>
-    __device__ __forceinline__ void gradientUp(const High& high, const LdsLevel<T>& low, entry* fill, int fillEntries) const
+    /** The way up for a region of the high-res level: into global memory what is owned, all of it into a tile as well. */
+    template <typename High, typename Low>
+    __device__ __forceinline__ void upRegion(const High& high, const Low& low, const PullPushRegion& r, const PullPushRegion& owned, bool keep,
+                                             const LdsTile<T>& tile) const
     {
-        const int pitch = high.W + 2;
+        const int log2 = lanesLog2(r.rows() * r.columns(), C);
+        forEach(r.y0, r.x0, r.rows(), r.columns(), log2, [&](int y, int x, int lane) {
+            const bool own = y >= owned.y0 && y < owned.y1 && x >= owned.x0 && x < owned.x1;
+            const T m = high.maskPre(y, x);
+            const Mix mix(y, x, low);
+            for (int c = lane; c < C; c += 1 << log2) {
+                const T v = m * high.dataPre(c, y, x) + (1 - m) * quotient(mix.sum(low, c), mix.n);
+                if (own) high.dataPost(c, y, x) = v;
+                if (keep) tile.data(c, y, x) = v;
+            }
+            if (lane == 0) {
+                const T v = m + (mix.n > 0 ? (1 - m) * (mix.n / mix.weight) : T(0));
+                if (own && high.hasMaskPost()) high.maskPost(y, x) = v;
+                if (keep) tile.mask(y, x) = v;
+            }
+        });
+    }
+
+    /**
+     * Step A (see gradientUpTile) for a region of the low-res level. fill: room for fillEntries entries, at least (C + 1) x 4 rows of the
+     * high-res pixels that it reaches. Ends with a barrier.
+     */
+    template <typename High, typename Low>
+    __device__ __forceinline__ void gradientUp(const High& high, const Low& low, const PullPushRegion& r, entry* fill, int fillEntries) const
+    {
+        const int x0 = 2 * r.x0 - 1, pitch = 2 * r.columns() + 2;
         const int stripe = max(1, (fillEntries / ((C + 1) * pitch) - 2) / 2);   // low-res rows that are gathered together
-        for (int a0 = 0; a0 < low.H; a0 += stripe) {
-            const int a1 = min(a0 + stripe, low.H);
-            const int y0 = 2 * a0 - 1, rows = 2 * (a1 - a0) + 2;   // with the border, which passes nothing down
+        for (int a0 = r.y0; a0 < r.y1; a0 += stripe) {
+            const int a1 = min(a0 + stripe, r.y1);
+            const int y0 = 2 * a0 - 1, rows = 2 * (a1 - a0) + 2;   // (what lies outside of the image passes nothing down)
             const int plane = rows * pitch;
             const int fillLog2 = lanesLog2(plane, C);
-            forEach(y0, -1, rows, pitch, fillLog2, [&](int y, int x, int lane) {
-                entry* to = fill + ((y - y0) * pitch + x + 1);
+            forEach(y0, x0, rows, pitch, fillLog2, [&](int y, int x, int lane) {
+                entry* to = fill + ((y - y0) * pitch + x - x0);
                 const bool inside = y >= 0 && y < high.H && x >= 0 && x < high.W;
                 if (!inside) {
                     for (int c = lane; c <= C; c += 1 << fillLog2) to[c * plane] = T(0);
@@ -824,13 +1130,13 @@ struct TailSteps
                 fromMask = sumOver(fromMask, fillLog2);
                 if (lane == 0) to[C * plane] = (high.hasGradMaskPost() ? high.gradMaskPost(y, x) * ((1 - m) / mix.weight) : T(0)) - fromMask;
             });
-            __syncthreads();
-            const int gatherLog2 = lanesLog2((a1 - a0) * low.W, C + 1);
-            forEach(a0, 0, a1 - a0, low.W, gatherLog2, [&](int a, int e, int lane) {
+            ldsBarrier();
+            const int gatherLog2 = lanesLog2((a1 - a0) * r.columns(), C + 1);
+            forEach(a0, r.x0, a1 - a0, r.columns(), gatherLog2, [&](int a, int e, int lane) {
                 T gradMask = 0;
                 const T mask = low.maskPost(a, e);
                 for (int c = lane; c <= C; c += 1 << gatherLog2) {
-                    const entry* from = fill + (c * plane + 2 * (a - a0) * pitch + 2 * e);
+                    const entry* from = fill + (c * plane + 2 * (a - a0) * pitch + 2 * (e - r.x0));
                     T sum = 0;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
@@ -842,54 +1148,62 @@ struct TailSteps
                         gradMask += sum;
                     } else {
                         gradMask += sum * low.dataPost(c, a, e);
-                        low.gradDataPost(c, a, e) = sum * mask;
+                        low.setGradDataPost(c, a, e, sum * mask);
                     }
                 }
                 gradMask = sumOver(gradMask, gatherLog2);
-                if (lane == 0) low.gradMaskPost(a, e) = gradMask;
+                if (lane == 0) low.setGradMaskPost(a, e, gradMask);
             });
-            __syncthreads();
+            ldsBarrier();
         }
     }
 
-    /** Step B (see gradientQuad). \tparam ACCUMULATE add to what is there */
-    template <bool ACCUMULATE, typename High>
-    __device__ __forceinline__ void gradient(const High& high, const LdsLevel<T>& low) const
+    /** Step B (see gradientQuads) for a region of the high-res level. \tparam ACCUMULATE add to what is there */
+    template <bool ACCUMULATE, typename High, typename Low>
+    __device__ __forceinline__ void gradient(const High& high, const Low& low, const PullPushRegion& r) const
     {
+        if ((high.H | high.W) & 1) gradient<ACCUMULATE, true>(high, low, r);
+        else gradient<ACCUMULATE, false>(high, low, r);
+    }
+    /** \tparam ODD some size is odd: a pixel may lie in several windows */
+    template <bool ACCUMULATE, bool ODD, typename High, typename Low>
+    __device__ __forceinline__ void gradient(const High& high, const Low& low, const PullPushRegion& r) const
+    {
+        constexpr int MOST = ODD ? 2 : 1;
         const bool oddH = high.H & 1, oddW = high.W & 1;
-        const int log2 = lanesLog2(high.H * high.W, C);
-        forEach(0, 0, high.H, high.W, log2, [&](int y, int x, int lane) {
+        const int log2 = lanesLog2(r.rows() * r.columns(), C);
+        forEach(r.y0, r.x0, r.rows(), r.columns(), log2, [&](int y, int x, int lane) {
             const T m = high.maskPre(y, x);
             const Mix mix(y, x, low);
             const Reciprocal<T> inverse(mix.n);
             // the windows that the pixel lies in: of the own cell, and of odd sizes those of the row above and of the column to the left
-            Reciprocal<T> sums[2][2];
-            int window[2][2];
-            bool in[2][2];
+            Reciprocal<T> sums[MOST][MOST];
+            int window[MOST][MOST];
+            bool in[MOST][MOST];
             T gradMask = 0;
 #pragma unroll
-            for (int wa = 0; wa < 2; ++wa)
+            for (int wa = 0; wa < MOST; ++wa)
 #pragma unroll
-                for (int we = 0; we < 2; ++we) {
+                for (int we = 0; we < MOST; ++we) {
                     const int a = (y >> 1) - wa, e = (x >> 1) - we;
-                    in[wa][we] = (wa == 0 || (oddH && !(y & 1))) && (we == 0 || (oddW && !(x & 1))) && a >= 0 && e >= 0 && a < low.H && e < low.W;
+                    in[wa][we] = (wa == 0 || (oddH && !(y & 1))) && (we == 0 || (oddW && !(x & 1))) && (!ODD || (a >= 0 && e >= 0 && a < low.H && e < low.W));
                     window[wa][we] = 0;
                     if (!in[wa][we]) continue;
                     window[wa][we] = a * low.pitch + e;
                     sums[wa][we] = Reciprocal<T>(low.maskSumP[window[wa][we]]);
                     // the maximum of a window passes its gradient to every pixel that attains it
-                    if (lane == 0 && low.maskPreP[window[wa][we]] == m) gradMask += low.gradMaskPreP[window[wa][we]];
+                    if (lane == 0 && low.maskPreP[window[wa][we]] == m) gradMask += low.gradMaskPre(a, e);
                 }
             for (int c = lane; c < C; c += 1 << log2) {
                 const T v = high.dataPre(c, y, x), g = high.gradDataPost(c, y, x);
                 T sum = g;
                 gradMask += g * (v - inverse(mix.sum(low, c)));
 #pragma unroll
-                for (int wa = 0; wa < 2; ++wa)
+                for (int wa = 0; wa < MOST; ++wa)
 #pragma unroll
-                    for (int we = 0; we < 2; ++we) {
+                    for (int we = 0; we < MOST; ++we) {
                         if (!in[wa][we]) continue;
-                        const T grad = sums[wa][we](low.gradDataPreP[c * low.plane + window[wa][we]]);
+                        const T grad = sums[wa][we](low.gradDataPre(c, (y >> 1) - wa, (x >> 1) - we));
                         sum += grad;
                         gradMask += grad * (v - low.dataPreP[c * low.plane + window[wa][we]]);
                     }
@@ -923,39 +1237,37 @@ template <typename T>
 __global__ void __launch_bounds__(256) PullPushUpKernel(const PullPushLevel<T> high, const PullPushLevel<T> low, int C, int pairs)
 {
     using namespace pullpush;
-    int b, a, e;
-    const int height = (high.H + 1) / 2, width = (high.W + 1) / 2;
-    tileOf(width, height, b, a, e);
-    a += threadIdx.x / TILE_W;
-    e += threadIdx.x % TILE_W;
-    if (a >= height || e >= width) return;
-    if (pairs) upQuad<true>(high, low, C, b, a, e);
-    else upQuad<false>(high, low, C, b, a, e);
+    __shared__ typename LowTile<T, TILE_W, TILE_H>::Memory sLow;
+    int b, a0, e0;
+    tileOf((high.W + 1) / 2, (high.H + 1) / 2, b, a0, e0);
+    if (pairs) upQuads<true, TILE_W, TILE_H>(high, low, C, b, a0, e0, sLow);
+    else upQuads<false, TILE_W, TILE_H>(high, low, C, b, a0, e0, sLow);
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 1))) PullPushGradientUpKernel(const PullPushLevel<T> high, const PullPushLevel<T> low, int C, int pairs)
+__global__ void __launch_bounds__(pullpush::UP_THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2))) PullPushGradientUpKernel(const PullPushLevel<T> high, const PullPushLevel<T> low, int C, int pairs)
 {
     using namespace pullpush;
-    __shared__ T sFill[pullpushChunk<T>() + 1][pullpushTileEntries(TILE_W, TILE_H)];
+    __shared__ T sRows[pullpushChunk<T>() + 1][2][UP_THREADS];
+    __shared__ typename LowTile<T, UP_TILE_W + 2, UP_TILE_H + 2>::Memory sLow;
     int b, a0, e0;
-    tileOf(low.W, low.H, b, a0, e0);
-    if (pairs) gradientUpTile<true, TILE_W, TILE_H>(high, low, C, b, a0, e0, sFill);
-    else gradientUpTile<false, TILE_W, TILE_H>(high, low, C, b, a0, e0, sFill);
+    tileOf<UP_TILE_W, UP_TILE_H>(low.W, low.H, b, a0, e0);
+    // all quads of the tile and its border, and their neighbours, lie in the image
+    const bool interior = a0 >= 2 && e0 >= 2 && a0 + UP_TILE_H + 1 < low.H && e0 + UP_TILE_W + 1 < low.W;
+    if (pairs && interior) gradientUpTile<true, true, UP_TILE_W, UP_TILE_H>(high, low, C, b, a0, e0, sRows, sLow);
+    else if (pairs) gradientUpTile<true, false, UP_TILE_W, UP_TILE_H>(high, low, C, b, a0, e0, sRows, sLow);
+    else gradientUpTile<false, false, UP_TILE_W, UP_TILE_H>(high, low, C, b, a0, e0, sRows, sLow);
 }
 
 template <typename T, bool ACCUMULATE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && !ACCUMULATE ? 4 : 1))) PullPushGradientKernel(const PullPushLevel<T> high, const PullPushLevel<T> low, int C, int pairs)
 {
     using namespace pullpush;
-    int b, a, e;
-    const int height = (high.H + 1) / 2, width = (high.W + 1) / 2;
-    tileOf(width, height, b, a, e);
-    a += threadIdx.x / TILE_W;
-    e += threadIdx.x % TILE_W;
-    if (a >= height || e >= width) return;
-    if (pairs) gradientQuad<true, ACCUMULATE>(high, low, C, b, a, e);
-    else gradientQuad<false, ACCUMULATE>(high, low, C, b, a, e);
+    __shared__ typename LowTile<T, TILE_W, TILE_H>::Memory sLow;
+    int b, a0, e0;
+    tileOf((high.W + 1) / 2, (high.H + 1) / 2, b, a0, e0);
+    if (pairs) gradientQuads<true, ACCUMULATE, TILE_W, TILE_H>(high, low, C, b, a0, e0, sLow);
+    else gradientQuads<false, ACCUMULATE, TILE_W, TILE_H>(high, low, C, b, a0, e0, sLow);
 }
 
 /**
@@ -975,16 +1287,16 @@ __global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushTailKernel(const 
     const TailSteps<T> steps(C);
     const TopLevel<T> top(finest, b, sLevels + topOffset, C, false);
     auto level = [&](int k) { return LdsLevel<T>(sLevels, tail, finest.H, finest.W, C, k, false); };
-    __syncthreads();
+    ldsBarrier();
     steps.down(top, level(1));
-    __syncthreads();
+    ldsBarrier();
     for (int k = 1; k + 1 < tail.numLevels; ++k) {
         steps.down(level(k), level(k + 1));
-        __syncthreads();
+        ldsBarrier();
     }
     for (int k = tail.numLevels - 2; k >= 1; --k) {
         steps.up(level(k), level(k + 1));
-        __syncthreads();
+        ldsBarrier();
     }
     if (finest.dataPost.p) steps.up(top, level(1));
     for (int i = threadIdx.x; i < keptEntries; i += PULLPUSH_TAIL_BLOCK) kept[static_cast<long long>(b) * keptEntries + i] = sLevels[i];
@@ -1014,14 +1326,166 @@ __global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushGradientTailKerne
 #pragma unroll 4
         for (int i = threadIdx.x; i < entries; i += PULLPUSH_TAIL_BLOCK) sLevels[tail.offsets[k] + i] = from[i];
     }
-    __syncthreads();
-    steps.gradientUp(top, level(1), sFill, fillEntries);
-    for (int k = 1; k + 1 < tail.numLevels; ++k) steps.gradientUp(level(k), level(k + 1), sFill, fillEntries);
+    ldsBarrier();
+    auto whole = [](const auto& l) { return PullPushRegion{0, l.H, 0, l.W}; };
+    steps.gradientUp(top, level(1), whole(level(1)), sFill, fillEntries);
+    for (int k = 1; k + 1 < tail.numLevels; ++k) steps.gradientUp(level(k), level(k + 1), whole(level(k + 1)), sFill, fillEntries);
     for (int k = tail.numLevels - 2; k >= 1; --k) {
-        steps.template gradient<false>(level(k), level(k + 1));
-        __syncthreads();
+        steps.template gradient<false>(level(k), level(k + 1), whole(level(k)));
+        ldsBarrier();
     }
-    steps.template gradient<ACCUMULATE>(top, level(1));
+    steps.template gradient<ACCUMULATE>(top, level(1), whole(top));
+}
+
+/**
+ * Step B for all levels of a tree but the coarsest, which has its gradients already, in one launch: a workgroup walks from the
+ * coarsest to a tile of the finest level, the gradients of the levels in between stay in its LDS (where sizes are odd, a tile needs a
+ * pixel more of the next coarser level, which neighbours form twice). 64 x 64 to 512 x 512 pixels of 4 floats: 22 us, with a launch
+ * each 45. Bound by the chain of a step, 1.5 to 2 us whatever the size; a level of 1024 x 1024 is better off with a launch of its own (18 us, within the
+ * tree 27).
+ */
+template <typename T>
+__global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushGradientTreeKernel(const PullPushTree<T> tree, int C)
+{
+    using namespace pullpush;
+    extern __shared__ __align__(16) unsigned char sMemory[];
+    auto* sTiles = (typename LdsLevel<T>::entry*)sMemory;
+    const TailSteps<T> steps(C);
+    int b;
+    const int H = tree.levels[0].H, W = tree.levels[0].W;   // halved from level to level, rounding down
+    const PullPushRegion finest = treeTile(H, W, tree.tile, b);
+    auto region = [&](int k) {   // of level k: the windows that the pixels of the level above lie in
+        PullPushRegion r = finest;
+        for (int i = 0; i < k; ++i)
+            r = {max((r.y0 >> 1) - ((H >> i) & 1), 0), min(((r.y1 - 1) >> 1) + 1, H >> (i + 1)), max((r.x0 >> 1) - ((W >> i) & 1), 0),
+                 min(((r.x1 - 1) >> 1) + 1, W >> (i + 1))};
+        return r;
+    };
+    auto tile = [&](int k) { return LdsTile<T>(treeMemory(sTiles, tree, C, k), region(k)); };
+    const int last = tree.count - 2;
+    if (last == 0) {
+        steps.template gradient<false>(GlobalHigh<T>(tree.levels[0], b), GlobalLow<T>(tree.levels[1], b), finest);
+        return;
+    }
+    steps.template gradient<false>(GradientTileHigh<T>(tree.levels[last], b, tile(last)), GlobalLow<T>(tree.levels[last + 1], b), region(last));
+    for (int k = last - 1; k >= 1; --k) {
+        ldsBarrier();
+        steps.template gradient<false>(GradientTileHigh<T>(tree.levels[k], b, tile(k)), GradientTileLow<T>(tree.levels[k + 1], b, tile(k + 1)), region(k));
+    }
+    ldsBarrier();
+    steps.template gradient<false>(GlobalHigh<T>(tree.levels[0], b), GradientTileLow<T>(tree.levels[1], b, tile(1)), finest);
+}
+
+/**
+ * The way up for all levels of a tree but the coarsest, which is inpainted already, in one launch: as above; a tile needs the
+ * neighbours of its pixels on every coarser level, a border that neighbours form twice. 64 x 64 to 512 x 512 pixels of 4 floats: 15 us,
+ * with a launch each 23.
+ */
+template <typename T>
+__global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushUpTreeKernel(const PullPushTree<T> tree, int C)
+{
+    using namespace pullpush;
+    extern __shared__ __align__(16) unsigned char sMemory[];
+    auto* sTiles = (typename LdsLevel<T>::entry*)sMemory;
+    const TailSteps<T> steps(C);
+    int b;
+    const int H = tree.levels[0].H, W = tree.levels[0].W;   // halved from level to level, rounding down
+    const PullPushRegion finest = treeTile(H, W, tree.tile, b);
+    auto region = [&](int k) {
+        PullPushRegion r = finest;
+        for (int i = 0; i < k; ++i)
+            r = {max((r.y0 >> 1) - 1, 0), min(((r.y1 - 1) >> 1) + 2, H >> (i + 1)), max((r.x0 >> 1) - 1, 0), min(((r.x1 - 1) >> 1) + 2, W >> (i + 1))};
+        return r;
+    };
+    auto tile = [&](int k) { return LdsTile<T>(treeMemory(sTiles, tree, C, k), region(k)); };
+    // (what is owned of level k: sizes are halved rounding down, so the tiles cover all of it)
+    auto owned = [&](int k) {
+        return PullPushRegion{finest.y0 >> k, (finest.y0 + tree.tile) >> k, finest.x0 >> k, (finest.x0 + tree.tile) >> k};
+    };
+    const int last = tree.count - 2;
+    for (int k = last; k >= 0; --k) {
+        const bool keep = k > 0;
+        if (k == last) steps.upRegion(GlobalHigh<T>(tree.levels[k], b), GlobalLow<T>(tree.levels[k + 1], b), region(k), owned(k), keep, tile(max(k, 1)));
+        else steps.upRegion(GlobalHigh<T>(tree.levels[k], b), InpaintedTileLow<T>(tree.levels[k + 1], tile(k + 1)), region(k), owned(k), keep, tile(max(k, 1)));
+        ldsBarrier();
+    }
+}
+
+/**
+ * The way down for all levels of a tree but the finest, which is there already, in one launch: a workgroup forms a tile of the
+ * coarsest level and all that it needs of the finer ones (where sizes are odd, windows overlap, and neighbours form a border twice). The
+ * tile is counted in pixels of the finest level. 1024 x 1024 to 32 x 32 pixels of 4 floats: 17 us, with a launch each 24.
+ */
+template <typename T>
+__global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushDownTreeKernel(const PullPushTree<T> tree, int C)
+{
+    using namespace pullpush;
+    extern __shared__ __align__(16) unsigned char sMemory[];
+    auto* sTiles = (typename LdsLevel<T>::entry*)sMemory;
+    const TailSteps<T> steps(C);
+    const int last = tree.count - 1;
+    int b;
+    const int H = tree.levels[0].H, W = tree.levels[0].W;   // halved from level to level, rounding down
+    const PullPushRegion coarsest = treeTile(H >> last, W >> last, tree.tile >> last, b);
+    auto region = [&](int k) {   // of level k: what the windows of the level below cover
+        PullPushRegion r = coarsest;
+        for (int i = last - 1; i >= k; --i)
+            r = {2 * r.y0, min(2 * r.y1 + ((H >> i) & 1), H >> i), 2 * r.x0, min(2 * r.x1 + ((W >> i) & 1), W >> i)};
+        return r;
+    };
+    auto tile = [&](int k) {
+        auto* memory = sTiles;
+        for (int i = 1; i < k; ++i) memory += (C + 1) * treeDownSize(tree.tile, last, i) * treeDownSize(tree.tile, last, i);
+        return LdsTile<T>(memory, region(k));
+    };
+    auto owned = [&](int k) {   // the last tile has what is left over
+        return PullPushRegion{coarsest.y0 << (last - k), coarsest.y1 == H >> last ? H >> k : coarsest.y1 << (last - k), coarsest.x0 << (last - k),
+                              coarsest.x1 == W >> last ? W >> k : coarsest.x1 << (last - k)};
+    };
+    for (int k = 1; k <= last; ++k) {
+        const bool keep = k < last;
+        if (k == 1) steps.downRegion(GlobalHigh<T>(tree.levels[0], b), GlobalHigh<T>(tree.levels[1], b), region(1), owned(1), keep, tile(1));
+        else steps.downRegion(DownTileHigh<T>(tree.levels[k - 1], tile(k - 1)), GlobalHigh<T>(tree.levels[k], b), region(k), owned(k), keep, tile(min(k, last - 1)));
+        ldsBarrier();
+    }
+}
+
+/**
+ * Step A for all levels of a tree but the finest, in one launch: as the way down, where a tile needs a border of one pixel more of the next
+ * finer level. fillOffset: where the fills lie in LDS, behind the tiles. 512 x 512 to 32 x 32 pixels of 4 floats in two
+ * launches of two steps: 23 us, with a launch each 32.
+ */
+template <typename T>
+__global__ void __launch_bounds__(PULLPUSH_TAIL_BLOCK) PullPushGradientUpTreeKernel(const PullPushTree<T> tree, int C, int fillOffset, int fillEntries)
+{
+    using namespace pullpush;
+    extern __shared__ __align__(16) unsigned char sMemory[];
+    auto* sTiles = (typename LdsLevel<T>::entry*)sMemory;
+    const TailSteps<T> steps(C);
+    const int last = tree.count - 1;
+    int b;
+    const int H = tree.levels[0].H, W = tree.levels[0].W;   // halved from level to level, rounding down
+    const PullPushRegion coarsest = treeTile(H >> last, W >> last, tree.tile >> last, b);
+    auto region = [&](int k) {   // of level k: what the gathers of the level below reach
+        PullPushRegion r = coarsest;
+        for (int i = last - 1; i >= k; --i)
+            r = {max(2 * r.y0 - 1, 0), min(2 * r.y1 + 1, H >> i), max(2 * r.x0 - 1, 0), min(2 * r.x1 + 1, W >> i)};
+        return r;
+    };
+    auto tile = [&](int k) {
+        auto* memory = sTiles;
+        for (int i = 1; i < k; ++i) memory += (C + 1) * treeUpSize(tree.tile, last, i) * treeUpSize(tree.tile, last, i);
+        return LdsTile<T>(memory, region(k));
+    };
+    auto owned = [&](int k) {
+        return PullPushRegion{coarsest.y0 << (last - k), coarsest.y1 == H >> last ? H >> k : coarsest.y1 << (last - k), coarsest.x0 << (last - k),
+                              coarsest.x1 == W >> last ? W >> k : coarsest.x1 << (last - k)};
+    };
+    for (int k = 1; k <= last; ++k) {
+        const UpTileLow<T> low(tree.levels[k], b, owned(k), k < last, tile(max(min(k, last - 1), 1)));
+        if (k == 1) steps.gradientUp(GlobalHigh<T>(tree.levels[0], b), low, region(1), sTiles + fillOffset, fillEntries);
+        else steps.gradientUp(UpTileHigh<T>(tree.levels[k - 1], b, tile(k - 1)), low, region(k), sTiles + fillOffset, fillEntries);
+    }
 }
 
 namespace pullpush

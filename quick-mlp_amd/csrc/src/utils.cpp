@@ -21,15 +21,24 @@ const char* scalarName(Tensor::Precision p)
     throw std::runtime_error("fractionalPullpush works on float or double tensors");
 }
 
-const char* const KERNEL_NAMES[] = {"PullPushDownKernel<$T>", "PullPushUpKernel<$T>", "PullPushTailKernel<$T>",
-                                    "PullPushGradientUpKernel<$T>", "PullPushGradientKernel<$T, false>",
-                                    "PullPushGradientKernel<$T, true>", "PullPushGradientTailKernel<$T, false>",
-                                    "PullPushGradientTailKernel<$T, true>", "PullPushAddKernel<$T, 4>",
-                                    "PullPushCopyKernel<$T, 4>"};
-enum KernelIndex { DOWN, UP, TAIL, GRADIENT_UP, GRADIENT, GRADIENT_ADD, GRADIENT_TAIL, GRADIENT_TAIL_ADD, ADD_4, COPY_4 };
+// Kernels on one line share a code object.
+const std::vector<std::vector<const char*>> KERNEL_NAMES = {
+    {"PullPushDownKernel<$T>", "PullPushDownTreeKernel<$T>"},
+    {"PullPushUpKernel<$T>", "PullPushUpTreeKernel<$T>"},
+    {"PullPushTailKernel<$T>"},
+    {"PullPushGradientUpKernel<$T>", "PullPushGradientUpTreeKernel<$T>"},
+    {"PullPushGradientKernel<$T, false>", "PullPushGradientTreeKernel<$T>"},
+    {"PullPushGradientKernel<$T, true>"},
+    {"PullPushGradientTailKernel<$T, false>"},
+    {"PullPushGradientTailKernel<$T, true>"},
+    {"PullPushAddKernel<$T, 4>"},
+    {"PullPushCopyKernel<$T, 4>"}};
+constexpr int SECOND = 16;   // the second kernel of a line
+enum KernelIndex { DOWN, UP, TAIL, GRADIENT_UP, GRADIENT, GRADIENT_ADD, GRADIENT_TAIL, GRADIENT_TAIL_ADD, ADD_4, COPY_4,
+                   DOWN_TREE = DOWN + SECOND, GRADIENT_UP_TREE = GRADIENT_UP + SECOND, UP_TREE = UP + SECOND, GRADIENT_TREE = GRADIENT + SECOND };
 
 // as in kernels/pullpush.h
-constexpr int TAIL_BLOCK = 1024, TILE_W = 32, TILE_H = 8, BLOCK = 256;
+constexpr int TAIL_BLOCK = 1024, TILE_W = 32, TILE_H = 8, BLOCK = 256, UP_TILE_W = 14, UP_TILE_H = 14, UP_THREADS = 256;
 // What the kernel of the coarse levels keeps in LDS beside them for step A, four rows at least: all of 32 x 32 pixels of 4
 // channels of floats with a border.
 constexpr size_t TAIL_FILL_BYTES = 24 * 1024;
@@ -40,11 +49,14 @@ std::string pullpushSource(bool wide)
     return (wide ? "#define PULLPUSH_WIDE_PLANES\n" : "") + KernelLoader::MainFile("qmlp/kernels/pullpush.h");
 }
 
-std::string kernelName(int index, const std::string& scalar)
+std::vector<std::string> kernelNames(size_t line, const std::string& scalar)
 {
-    std::string name = KERNEL_NAMES[index];
-    name.replace(name.find("$T"), 2, scalar);
-    return "qmlp::kernel::" + name;
+    std::vector<std::string> names;
+    for (std::string name : KERNEL_NAMES[line]) {
+        name.replace(name.find("$T"), 2, scalar);
+        names.push_back("qmlp::kernel::" + name);
+    }
+    return names;
 }
 
 /** The compiled kernels stay loaded for the life of the process, like the reference's static kernels. */
@@ -52,13 +64,13 @@ template <typename T>
 KernelFunction& pullpushKernel(KernelIndex index, bool wide = false)
 {
     static std::mutex mutex;
-    static KernelFunction kernels[2][sizeof(KERNEL_NAMES) / sizeof(KERNEL_NAMES[0])];
+    static std::vector<KernelFunction> kernels[2][SECOND];
     std::lock_guard<std::mutex> lock(mutex);
-    auto& fun = kernels[wide ? 1 : 0][index];
-    if (!fun.defined())
-        fun = QuickMLP::Instance().kernelLoader()->getKernel(kernelName(index, sizeof(T) == 4 ? "float" : "double"), pullpushSource(wide),
-                                                             QuickMLP::Instance().getCompileFlags()).value();
-    return fun;
+    auto& line = kernels[wide ? 1 : 0][index % SECOND];
+    if (line.empty())
+        line = QuickMLP::Instance().kernelLoader()->getKernels(kernelNames(index % SECOND, sizeof(T) == 4 ? "float" : "double"), pullpushSource(wide),
+                                                               QuickMLP::Instance().getCompileFlags());
+    return line.at(index / SECOND);
 }
 
 /** PullPushView of kernels/pullpush.h */
@@ -234,15 +246,101 @@ bool movesPairs(const Level<T>& level, bool padded)
     return padded || level.W % 2 == 0;   // the rows of the workspaces end at even entries, the caller's where they end
 }
 
-/** One launch for one level: a workgroup per tile of 32 x 8 items. */
+/** One launch for one level: a workgroup per tile of 32 x 8 items, for step A of 14 x 14. */
 template <typename T>
 void launchLevel(KernelIndex kernel, bool wide, int B, int C, int height, int width, const std::vector<Level<T>>& levels, int l, stream_t stream)
 {
     Level<T> high = levels[l], low = levels[l + 1];
     int pairs = movesPairs(high, l > 0) ? 1 : 0;
-    const long long grid = static_cast<long long>(B) * divUp(height, TILE_H) * divUp(width, TILE_W);
+    const bool up = kernel == GRADIENT_UP;
+    const long long grid = static_cast<long long>(B) * divUp(height, up ? UP_TILE_H : TILE_H) * divUp(width, up ? UP_TILE_W : TILE_W);
     void* args[] = {&high, &low, &C, &pairs};
-    pullpushKernel<T>(kernel, wide).launch(static_cast<unsigned>(grid), BLOCK, 0, stream, args);
+    pullpushKernel<T>(kernel, wide).launch(static_cast<unsigned>(grid), up ? UP_THREADS : BLOCK, 0, stream, args);
+}
+
+// The finest levels that trees take (1 x 4 x 2048 x 2048 floats: step B from 1024 x 1024 on 50 us, from 512 x 512 on 22 + 18; the others alike).
+constexpr int DOWN_TREE_FINEST = 1, UP_TREE_FINEST = 2, GRADIENT_UP_TREE_FINEST = 2, GRADIENT_TREE_FINEST = 2;
+
+constexpr size_t TREE_LDS_BYTES = 72 * 1024;
+constexpr int GRADIENT_UP_TREE_LEVELS = 3;   // a border grows by a pixel per level
+/** PullPushTree of kernels/pullpush.h */
+template <typename T>
+struct Tree
+{
+    static constexpr int LEVELS = 6, BORDER = 5;
+    int count, tile;
+    Level<T> levels[LEVELS];
+};
+
+/**
+ * The steps from the level below levels[from] up to levels[to], several levels per launch. A launch for one of these levels
+ * takes 5 to 11 us whatever its size; of a tree a step takes 2.
+ */
+template <typename T>
+void launchTrees(KernelIndex kernel, int B, int C, const std::vector<Level<T>>& levels, int from, int to, stream_t stream)
+{
+    while (from >= to) {
+        Tree<T> tree = {};
+        const int finest = std::max(to, from + 1 - (Tree<T>::LEVELS - 1));
+        tree.count = from + 1 - finest + 1;
+        for (int k = 0; k < tree.count; ++k) tree.levels[k] = levels[finest + k];
+        auto ldsBytes = [&] {
+            size_t entries = 0;
+            for (int k = 1; k < tree.count - 1; ++k) entries += static_cast<size_t>(C + 1) * ((tree.tile >> k) + Tree<T>::BORDER) * ((tree.tile >> k) + Tree<T>::BORDER);
+            return entries * sizeof(T);
+        };
+        auto workgroups = [&] { return static_cast<long long>(B) * divUp(levels[finest].H, tree.tile) * divUp(levels[finest].W, tree.tile); };
+        // a workgroup on every compute unit, and room for two
+        tree.tile = 64;
+        while (tree.tile > 16 && (workgroups() < KernelFunction::computeUnits() || ldsBytes() > TREE_LDS_BYTES)) tree.tile /= 2;
+        void* args[] = {&tree, &C};
+        pullpushKernel<T>(kernel).launch(static_cast<unsigned>(workgroups()), TAIL_BLOCK, static_cast<unsigned>(ldsBytes()), stream, args);
+        from = finest - 1;
+    }
+}
+
+/**
+ * The steps from levels[from] down to levels[to], several levels per launch.
+ * \param border pixels that a region of a level grows by on its way to the next finer one (2 n + border)
+ */
+template <typename T>
+void launchTreesDown(KernelIndex kernel, int B, int C, const std::vector<Level<T>>& levels, int from, int to, int most, int border, stream_t stream)
+{
+    while (from < to) {
+        Tree<T> tree = {};
+        const bool fills = kernel == GRADIENT_UP_TREE;
+        int last = std::min(to - from, most - 1);
+        auto ldsEntries = [&] {
+            size_t entries = 0;
+            for (int k = 1; k < last; ++k) {
+                const size_t size = (tree.tile >> k) + border * ((1 << (last - k)) - 1);
+                entries += (C + 1) * size * size;
+            }
+            return entries;
+        };
+        auto fillBytes = [&] {   // at least four rows
+            const size_t size = (tree.tile >> 1) + border * ((1 << (last - 1)) - 1);
+            return fills ? std::max(TAIL_FILL_BYTES, static_cast<size_t>(C + 1) * 4 * (2 * size + 2) * sizeof(T)) : size_t(0);
+        };
+        auto workgroups = [&] {
+            const int tile = tree.tile >> last;
+            return static_cast<long long>(B) * divUp(levels[from + last].H, tile) * divUp(levels[from + last].W, tile);
+        };
+        // a workgroup on every compute unit and room for two; of many channels fewer levels
+        for (;; --last) {
+            const int smallest = 1 << (last + 1);   // 2 x 2 pixels of the coarsest level
+            tree.tile = 64;
+            while (tree.tile > smallest && (workgroups() < KernelFunction::computeUnits() || ldsEntries() * sizeof(T) + fillBytes() > TREE_LDS_BYTES)) tree.tile /= 2;
+            if (last == 1 || ldsEntries() * sizeof(T) + fillBytes() <= TREE_LDS_BYTES) break;
+        }
+        const int coarsest = from + last;
+        tree.count = last + 1;
+        for (int k = 0; k <= last; ++k) tree.levels[k] = levels[from + k];
+        int fillOffset = static_cast<int>(ldsEntries()), fillEntries = static_cast<int>(fillBytes() / sizeof(T));
+        void* args[] = {&tree, &C, &fillOffset, &fillEntries};   // (the last two for step A)
+        pullpushKernel<T>(kernel).launch(static_cast<unsigned>(workgroups()), TAIL_BLOCK, static_cast<unsigned>(ldsEntries() * sizeof(T) + fillBytes()), stream, args);
+        from = coarsest;
+    }
 }
 
 /** The pyramid down to the coarsest level and the inpainted levels up to levels[1]; with 'finest' up to levels[0]. */
@@ -250,9 +348,16 @@ template <typename T>
 void runForward(const std::vector<Level<T>>& levels, bool wide, int B, int C, bool finest, T* keptTail, stream_t stream)
 {
     const int last = static_cast<int>(levels.size()) - 1;
-    for (int l = 0; l < last; ++l) launchLevel(DOWN, wide, B, C, levels[l + 1].H, levels[l + 1].W, levels, l, stream);
+    const int single = wide ? last : std::min(last, DOWN_TREE_FINEST);   // levels of a launch each
+    for (int k = 0; k < single; ++k) launchLevel(DOWN, wide, B, C, levels[k + 1].H, levels[k + 1].W, levels, k, stream);
+    launchTreesDown(DOWN_TREE, B, C, levels, single, last, Tree<T>::LEVELS, 1, stream);
     launchTail(TAIL, wide, B, C, levels[last], false, keptTail, stream);
-    for (int l = last - 1; l >= (finest ? 0 : 1); --l)
+    int l = last - 1;
+    if (!wide) {
+        launchTrees(UP_TREE, B, C, levels, l, UP_TREE_FINEST, stream);
+        l = std::min(l, UP_TREE_FINEST - 1);
+    }
+    for (; l >= (finest ? 0 : 1); --l)
         launchLevel(UP, wide, B, C, divUp(levels[l].H, 2), divUp(levels[l].W, 2), levels, l, stream);
 }
 
@@ -260,9 +365,16 @@ template <typename T>
 void runAdjoint(const std::vector<Level<T>>& levels, bool wide, int B, int C, bool accumulate, T* keptTail, stream_t stream)
 {
     const int last = static_cast<int>(levels.size()) - 1;
-    for (int l = 0; l < last; ++l) launchLevel(GRADIENT_UP, wide, B, C, levels[l + 1].H, levels[l + 1].W, levels, l, stream);
+    const int single = wide ? last : std::min(last, GRADIENT_UP_TREE_FINEST);
+    for (int k = 0; k < single; ++k) launchLevel(GRADIENT_UP, wide, B, C, levels[k + 1].H, levels[k + 1].W, levels, k, stream);
+    launchTreesDown(GRADIENT_UP_TREE, B, C, levels, single, last, GRADIENT_UP_TREE_LEVELS, 2, stream);
     launchTail(last == 0 && accumulate ? GRADIENT_TAIL_ADD : GRADIENT_TAIL, wide, B, C, levels[last], true, keptTail, stream);
-    for (int l = last - 1; l >= 0; --l)
+    int l = last - 1;
+    if (!wide) {
+        launchTrees(GRADIENT_TREE, B, C, levels, l, GRADIENT_TREE_FINEST, stream);
+        l = std::min(l, GRADIENT_TREE_FINEST - 1);
+    }
+    for (; l >= 0; --l)
         launchLevel(l == 0 && accumulate ? GRADIENT_ADD : GRADIENT, wide, B, C, divUp(levels[l].H, 2), divUp(levels[l].W, 2), levels, l, stream);
 }
 
@@ -364,8 +476,7 @@ void Utils::precompile(Tensor::Precision precision)
     const std::string t = scalarName(precision);
     auto kl = QuickMLP::Instance().kernelLoader();
     const int flags = QuickMLP::Instance().getCompileFlags() | KernelLoader::CompileOnly;
-    for (size_t i = 0; i < sizeof(KERNEL_NAMES) / sizeof(KERNEL_NAMES[0]); ++i)
-        kl->getKernel(kernelName(static_cast<int>(i), t), pullpushSource(false), flags);
+    for (size_t i = 0; i < KERNEL_NAMES.size(); ++i) kl->getKernels(kernelNames(i, t), pullpushSource(false), flags);
 }
 
 void Utils::pullpushMemory(const Tensor& data, size_t& pyramidBytes, size_t& gradientBytes)
