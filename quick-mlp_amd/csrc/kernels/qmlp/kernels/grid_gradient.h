@@ -878,9 +878,9 @@ struct GridGradientSlices
      * precision; split into two words in single precision it takes nine.
      */
     static constexpr int FIXED_BITS = 51;
-    __device__ __forceinline__ static long long toFixed(float v, double scale)
+    __device__ __forceinline__ static long long toFixed(double v, double scale)
     {
-        const double shifted = __builtin_fma(static_cast<double>(v), scale, 6755399441055744.0);
+        const double shifted = __builtin_fma(v, scale, 6755399441055744.0);
         return __builtin_bit_cast(long long, shifted) - 0x4338000000000000ll;
     }
 

@@ -22,12 +22,15 @@
 //                              whose adjoint is not finite, and points whose cell lies in another slab than
 //                              the sort's slab arithmetic put them (a coordinate within rounding of a slab
 //                              boundary, or on the upper border).
-// Measured on the dense 4-D grid above, 2^21 points: 165 + 7 us where the records and slice kernels take 281 + 154 us.
-// Of the 165 us about 100 are the 268 M additions in LDS (ds_add_u64 retires 4 to 6 lanes per clock and compute
-// unit, whatever feeds it), 37 the input gradients, 30 the rest (largest adjoint, zeroing and writing back the sums).
-// A term is the product of two integers (the adjoint in units chosen from the largest adjoint of the work item, the
-// weight of the corner in units of 2^-22): one v_mad_i64_i32 instead of the nine instructions that split a float
-// product into two words (190 -> 165 us).
+// Measured on the dense 4-D grid above, 2^21 points: 150 + 7 us where the records and slice kernels take 281 + 154 us.
+// The loop over the points is short of two things at once: vector instructions (73 % of the time before the last of the steps
+// below) and 268 M additions in LDS, of which ds_add_u64 takes 6.4 lanes per clock and compute unit
+// (entries at random, features rotated; 4.5 with all addresses at random, 7.7 side by side): 68 us; the input gradients take 32, writing the sums back 8. Hence few instructions per addition: a term
+// is one v_fma_f64 (GridGradientSlices::toFixed) and a subtraction, the corners along the unsorted coordinates lie at constant distances (the
+// addresses of one serve all), features change places two to a register, and a lane's rows are found by adding to a pointer,
+// instead of integer products, an address per addition and a choice among all features: 168 -> 150 us, together with adjoints
+// scanned 8 points per load, and the input gradients' loads one point ahead and as rows of four floats. (Half of the workgroups
+// starting with the input gradients, so that two of a compute unit want different things: no gain.)
 //
 // Replaces, for such batches, the atomicAdd of src_cpp/include/qmlp/kernels/encoding_hashgrid.cuh:117-166,345-369
 // of the reference.
@@ -98,19 +101,19 @@ struct GridGradientColumns
         return (l0 * REGION_NODES + l1) * REST + static_cast<int>(rest);
     }
 
-    /** The position of point p in the unit box, as every kernel of the grid computes it. */
-    __device__ __forceinline__ static void loadPosition(const Tensor2Read<float>& inputs, int p, const param_t& params,
+    /** The position of the point of a row of the inputs in the unit box, as every kernel of the grid computes it. */
+    __device__ __forceinline__ static void loadPosition(const float* __restrict__ row, int stride, const param_t& params,
                                                         bool rowsOfFloat4, float (&pos)[D])
     {
 #pragma clang fp contract(off)
         float in[D];
         if (D == 4 && rowsOfFloat4) {
-            const float4 v = *reinterpret_cast<const float4*>(inputs.data_ + static_cast<long long>(p) * inputs.strides_[0] + Cfg::Start);
+            const float4 v = *reinterpret_cast<const float4*>(row + Cfg::Start);
             in[0] = v.x, in[1 % D] = v.y, in[2 % D] = v.z, in[3 % D] = v.w;
         } else {
 #pragma unroll
             for (int d = 0; d < D; ++d)
-                in[d] = inputs.data_[static_cast<long long>(p) * inputs.strides_[0] + static_cast<long long>(d + Cfg::Start) * inputs.strides_[1]];
+                in[d] = row[static_cast<long long>(d + Cfg::Start) * stride];
         }
 #pragma unroll
         for (int d = 0; d < D; ++d) pos[d] = (in[d] - params.boundingBoxMin[d]) * params.boundingBoxInvSize[d];
@@ -127,6 +130,23 @@ struct GridGradientColumns
         for (int d = 2; d < D; ++d) rest += ((c >> d) & 1) ? s.termH[d] : s.termL[d];
     }
 
+    /** The node indices alone of the corners with bits 0 and 1 of c. */
+    __device__ __forceinline__ static void sortedNode(const typename Grid::LevelSetup& s, int c, int& n0, int& n1)
+    {
+        n0 = static_cast<int>(((c & 1) ? s.termH[0] : s.termL[0]) / stride(0));
+        n1 = static_cast<int>(((c & 2) ? s.termH[1] : s.termL[1]) / stride(1));
+    }
+    /** Entries between neighbours along a coordinate. */
+    __device__ __host__ static constexpr unsigned stride(int d) { return detail::upow(static_cast<unsigned>(R), D - 1 - d); }
+    static_assert(R >= 2 || D == 2, "two nodes along the other coordinates");
+    /** Entries from the node that is the lower one along all other coordinates to that of bits `others` (bit d - 2: upper along d). */
+    __device__ __host__ static constexpr int upperNodes(int others)
+    {
+        unsigned n = 0;
+        for (int d = 2; d < D; ++d) n += ((others >> (d - 2)) & 1) ? stride(d) : 0u;
+        return static_cast<int>(n);
+    }
+
     /** The cell of the point in the two sorted coordinates, as the grid computes it. */
     __device__ __forceinline__ static void cell(const typename Grid::LevelSetup& s, int& c0, int& c1)
     {
@@ -141,6 +161,105 @@ struct GridGradientColumns
 #pragma unroll
         for (int d = 0; d < D; ++d) inside = inside && s.f[d] >= 0.f && s.f[d] <= 1.f;
         return inside;
+    }
+
+    /** The adjoints of a point, two halves to a word. */
+    static constexpr int ADJOINT_WORDS = (F + 1) / 2;
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+    /** Whether none of the halves is NaN or infinite. */
+    template <int N>
+    __device__ __forceinline__ static bool finiteHalves(const unsigned (&words)[N])
+    {
+        u16x2 largest = {0, 0};
+#pragma unroll
+        for (int i = 0; i < N; ++i) largest = __builtin_elementwise_max(largest, __builtin_bit_cast(u16x2, words[i] & 0x7fff7fffu));
+        return largest[0] < 0x7c00u && largest[1] < 0x7c00u;
+    }
+
+    __device__ __forceinline__ static float adjointAt(const unsigned (&words)[ADJOINT_WORDS], int i)
+    {
+        return static_cast<float>(__builtin_bit_cast(f16, static_cast<unsigned short>(words[i / 2] >> (16 * (i % 2)))));
+    }
+
+    /** The feature that a lane takes in a step. */
+    __device__ __forceinline__ static int rotatedFeature(int step, int lane)
+    {
+        return (F & (F - 1)) == 0 ? ((step + lane) & (F - 1)) : ((step + lane % F) % F);
+    }
+    /** The adjoints in the order of rotatedFeature(): a power of two of them is moved by 4, 2 and 1 places, two in a word at a time. */
+    __device__ __forceinline__ static void rotate(const unsigned (&words)[ADJOINT_WORDS], int lane, float (&rotated)[F])
+    {
+        if constexpr ((F & (F - 1)) == 0 && F > 1) {
+            unsigned w[ADJOINT_WORDS];
+#pragma unroll
+            for (int i = 0; i < ADJOINT_WORDS; ++i) w[i] = words[i];
+#pragma unroll
+            for (int places = F / 2; places > 0; places /= 2) {
+                unsigned moved[ADJOINT_WORDS];
+                const unsigned move = (lane & places) ? ~0u : 0u;   // (as bits: selections become a search for an index)
+#pragma unroll
+                for (int i = 0; i < ADJOINT_WORDS; ++i) {
+                    if (places >= 2) moved[i] = (w[(i + places / 2) % ADJOINT_WORDS] & move) | (w[i] & ~move);
+                    else moved[i] = __builtin_amdgcn_alignbit(w[(i + 1) % ADJOINT_WORDS], w[i], (lane & 1) * 16);
+                }
+#pragma unroll
+                for (int i = 0; i < ADJOINT_WORDS; ++i) w[i] = moved[i];
+            }
+#pragma unroll
+            for (int i = 0; i < F; ++i) rotated[i] = adjointAt(w, i);
+        } else {
+#pragma unroll
+            for (int step = 0; step < F; ++step) {
+                const int i = rotatedFeature(step, lane);
+                float a = adjointAt(words, 0);
+#pragma unroll
+                for (int k = 1; k < F; ++k) a = i == k ? adjointAt(words, k) : a;
+                rotated[step] = a;
+            }
+        }
+    }
+
+    /**
+     * The largest magnitude (bits without the sign) among the adjoints of points [begin, end) that are finite; first: the first
+     * of their channels in tile 0. The adjoints of 64 points are F * 128 bytes side by side: a lane takes 8 points of a channel.
+     */
+    template <int ROW_CHANNELS, int BLOCK>
+    __device__ __forceinline__ static unsigned largestAdjoint(const f16* __restrict__ first, int begin, int end, int lane)
+    {
+        typedef unsigned u32x4 __attribute__((ext_vector_type(4), aligned(4)));
+        constexpr int CHUNKS = F * (TILE_POINTS / 8);   // of a tile
+        u16x2 largest = {0, 0};
+        if (begin >= end) return 0u;
+        const int firstTile = begin / TILE_POINTS;
+        const int chunks = ((end - 1) / TILE_POINTS - firstTile + 1) * CHUNKS;
+        constexpr int AHEAD = 10;   // loads of a lane: all 5120 points of an average run of 2^21 points in 31 x 31 slabs
+#pragma unroll 1
+        for (int i0 = lane; i0 < chunks; i0 += AHEAD * BLOCK) {
+            u32x4 v[AHEAD];
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) {
+                const int i = min(i0 + k * BLOCK, chunks - 1);   // (the last one again)
+                v[k] = *reinterpret_cast<const u32x4*>(first + static_cast<long long>(firstTile + i / CHUNKS) * (ROW_CHANNELS * TILE_POINTS)
+                                                       + i % CHUNKS * 8);
+            }
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) {
+                const int i = min(i0 + k * BLOCK, chunks - 1);
+                const int p = (firstTile + i / CHUNKS) * TILE_POINTS + i % (TILE_POINTS / 8) * 8;
+                unsigned words[4] = {v[k][0], v[k][1], v[k][2], v[k][3]};
+                if (p < begin || p + 8 > end || !finiteHalves(words)) {
+                    // others' points, and adjoints that are not finite (their points take the atomics), don't count
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        if (p + j < begin || p + j >= end || ((words[j / 2] >> (16 * (j % 2))) & 0x7c00u) == 0x7c00u)
+                            words[j / 2] &= j % 2 ? 0xffffu : 0xffff0000u;
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) largest = __builtin_elementwise_max(largest, __builtin_bit_cast(u16x2, words[j] & 0x7fff7fffu));
+            }
+        }
+        return max(static_cast<unsigned>(largest[0]), static_cast<unsigned>(largest[1]));
     }
 
     /** The runs of the sorted batch that owner (o0, o1) visits: run r covers the slabs (a0, o1 - 1 | o1), a0 = o0 - 1 + r. */
@@ -228,7 +347,10 @@ __global__ void __launch_bounds__(1024) GridGradientColumnsPlan(
  * Dynamic LDS: GridGradientColumns::LDS_BYTES (the sums of an owner, then the entries of the table around its slab).
  */
 template <typename Cfg, int CPS, int ROW_CHANNELS, int CHANNEL_OFFSET, int INPUT_GRADIENTS, int BLOCK>
-__global__ void __launch_bounds__(BLOCK) GridGradientColumnsKernel(
+__global__ void __launch_bounds__(BLOCK)
+    // two workgroups per compute unit where the features of all corners take at most half of the 128 registers that this leaves
+    __attribute__((amdgpu_waves_per_eu(EncodingHashGrid<Cfg>::NC * Cfg::Features * sizeof(typename Cfg::table_t) <= 256 ? 4 : 1)))
+GridGradientColumnsKernel(
     int numel, const Tensor2Read<float> inputs, const half* __restrict__ adjEncodedH,
     const HashGridParams<typename Cfg::table_t, Cfg::Dim> params, const int* __restrict__ starts, int slabs0, int slabs1,
     const GridGradientColumnItem* __restrict__ items, const int* __restrict__ itemCount, Tensor2RW<float> adjInputs,
@@ -248,10 +370,6 @@ __global__ void __launch_bounds__(BLOCK) GridGradientColumnsKernel(
     const f16* __restrict__ adjEncoded = reinterpret_cast<const f16*>(adjEncodedH);
     const typename Impl::Runs runs = Impl::runsOf(item.owner0, item.owner1, starts, slabs0, slabs1);
 
-    for (int i = tid; i < Impl::LOCAL_FLOATS; i += BLOCK) sSums[i] = 0;
-    if (tid == 0) sMaxBits = 0;
-    __syncthreads();
-
     // this part's share of both runs
     int begin[2], end[2];
 #pragma unroll
@@ -264,22 +382,20 @@ __global__ void __launch_bounds__(BLOCK) GridGradientColumnsKernel(
         end[r] = max(begin[r], min(end[r], numel));
     }
 
+    // rows of four floats that lie side by side: one load
+    const bool rowsOfFloat4 = D == 4 && Cfg::Start % 4 == 0 && inputs.strides_[1] == 1 && inputs.strides_[0] % 4 == 0
+        && reinterpret_cast<unsigned long long>(inputs.data_) % 16 == 0;
+
+    for (int i = tid; i < Impl::LOCAL_FLOATS; i += BLOCK) sSums[i] = 0;
+    if (tid == 0) sMaxBits = 0;
+    __syncthreads();
+
     // the largest adjoint among the points of this work item: the scale of the fixed-point sums
     {
         unsigned maxBits = 0u;
-#pragma unroll
+#pragma unroll 1
         for (int r = 0; r < 2; ++r)
-#pragma unroll 4
-            for (int p = begin[r] + tid; p < end[r]; p += BLOCK) {
-                const f16* adjRow = adjEncoded + static_cast<long long>(p / TILE_POINTS) * (ROW_CHANNELS * TILE_POINTS)
-                    + CHANNEL_OFFSET * TILE_POINTS + (p % TILE_POINTS);
-#pragma unroll
-                for (int i = 0; i < F; ++i) {
-                    // (a point with an adjoint that is not finite takes the atomics, see below)
-                    const unsigned bits = static_cast<unsigned>(__builtin_bit_cast(unsigned short, adjRow[i * TILE_POINTS])) & 0x7fffu;
-                    if (bits < 0x7c00u) maxBits = max(maxBits, bits);
-                }
-            }
+            maxBits = max(maxBits, Impl::template largestAdjoint<ROW_CHANNELS, BLOCK>(adjEncoded + CHANNEL_OFFSET * TILE_POINTS, begin[r], end[r], tid));
         if (maxBits != 0u) atomicMax(&sMaxBits, static_cast<int>(maxBits));
     }
     __syncthreads();
@@ -287,18 +403,11 @@ __global__ void __launch_bounds__(BLOCK) GridGradientColumnsKernel(
     const int maxExponent = static_cast<int>(maxBits >> 10) - 14;   // |adjoint| < 2^maxExponent
     const long long terms = static_cast<long long>(NC) * max(1, (end[0] - begin[0]) + (end[1] - begin[1]));
     const int termsLog2 = 64 - __builtin_clzll(static_cast<unsigned long long>(terms));
-    // A term is the product of two integers: the adjoint in units of 2^-adjointShift (below 2^adjointBits in
-    // magnitude) and the weight of the corner in units of 2^-WEIGHT_BITS (at most one): one multiply-add instruction
-    // per term instead of the nine of a float product split into two words. The sum of all terms that can meet in
-    // one element stays below 2^62.
-    constexpr int WEIGHT_BITS = 22;
-    const int adjointBits = min(30, 62 - WEIGHT_BITS - termsLog2);
-    const int adjointShift = adjointBits - maxExponent;
-    const int scaleExponent = adjointShift + WEIGHT_BITS;
+    // A term is weight x adjoint in units of 2^-scaleExponent, formed in double precision and rounded there; the sum of all
+    // terms that can meet in one element stays below 2^62.
+    const int scaleExponent = min(Fixed::FIXED_BITS, 62 - termsLog2) - maxExponent;
+    const double scale = ldexp(1.0, scaleExponent);
     float* __restrict__ gradients = params.parametersBackward;
-    // rows of four floats that lie side by side: one load
-    const bool rowsOfFloat4 = D == 4 && Cfg::Start % 4 == 0 && inputs.strides_[1] == 1 && inputs.strides_[0] % 4 == 0
-        && reinterpret_cast<unsigned long long>(inputs.data_) % 16 == 0;
 
 #pragma unroll 1
     for (int r = 0; r < 2; ++r) {
@@ -306,67 +415,74 @@ __global__ void __launch_bounds__(BLOCK) GridGradientColumnsKernel(
         // (the position and the adjoints of a lane's next point are loaded before it works on this one: with four
         // wavefronts per SIMD nothing else hides the latency of the loads)
         float nextPos[D];
-        f16 nextAdj[F];
-        auto loadPoint = [&](int q) {
-            Impl::loadPosition(inputs, q, params, rowsOfFloat4, nextPos);
-            const f16* row = adjEncoded + static_cast<long long>(q / TILE_POINTS) * (ROW_CHANNELS * TILE_POINTS)
-                + CHANNEL_OFFSET * TILE_POINTS + (q % TILE_POINTS);
+        unsigned nextAdj[Impl::ADJOINT_WORDS];
+        static_assert(BLOCK % TILE_POINTS == 0, "a lane's points lie at the same place of their tiles");
+        const float* nextRow = inputs.data_ + static_cast<long long>(begin[r] + tid) * inputs.strides_[0];
+        const f16* nextAdjRow = adjEncoded + static_cast<long long>((begin[r] + tid) / TILE_POINTS) * (ROW_CHANNELS * TILE_POINTS)
+            + CHANNEL_OFFSET * TILE_POINTS + (begin[r] + tid) % TILE_POINTS;
+        auto loadPoint = [&]() {
+            Impl::loadPosition(nextRow, inputs.strides_[1], params, rowsOfFloat4, nextPos);
 #pragma unroll
-            for (int i = 0; i < F; ++i) nextAdj[i] = row[i * TILE_POINTS];
+            for (int i = 0; i < Impl::ADJOINT_WORDS; ++i) {
+                f16x2 two = {nextAdjRow[2 * i * TILE_POINTS], f16(0)};
+                if (2 * i + 1 < F) two[1] = nextAdjRow[(2 * i + 1) * TILE_POINTS];
+                nextAdj[i] = __builtin_bit_cast(unsigned, two);
+            }
+            nextRow += static_cast<long long>(BLOCK) * inputs.strides_[0];
+            nextAdjRow += BLOCK * ROW_CHANNELS;
         };
-        if (begin[r] + tid < end[r]) loadPoint(begin[r] + tid);
+        if (begin[r] + tid < end[r]) loadPoint();
 #pragma unroll 1
         for (int p = begin[r] + tid; p < end[r]; p += BLOCK) {
             const int a1 = p < runs.middle[r] ? item.owner1 - 1 : item.owner1;
             const bool home = a0 == item.owner0 && a1 == item.owner1;
             float pos[D];
-            f16 adjHalf[F];
+            unsigned adjWords[Impl::ADJOINT_WORDS];
 #pragma unroll
             for (int d = 0; d < D; ++d) pos[d] = nextPos[d];
 #pragma unroll
-            for (int i = 0; i < F; ++i) adjHalf[i] = nextAdj[i];
-            if (p + BLOCK < end[r]) loadPoint(p + BLOCK);
+            for (int i = 0; i < Impl::ADJOINT_WORDS; ++i) adjWords[i] = nextAdj[i];
+            if (p + BLOCK < end[r]) loadPoint();
             const typename Grid::LevelSetup s = Grid::setupLevel(0, pos);
             int c0, c1;
             Impl::cell(s, c0, c1);
             // Points that do not fit the scheme -- the same verdict in every workgroup that visits the point: outside
             // the box, in a cell of another slab than the sort's, or with an adjoint that is not finite (NaN and
             // infinity have no fixed-point form and reach the gradients through the atomics of the point's home).
-            float adj[F];
-            bool finite = true;
-#pragma unroll
-            for (int i = 0; i < F; ++i) {
-                const f16 h = adjHalf[i];
-                finite = finite && (static_cast<unsigned>(__builtin_bit_cast(unsigned short, h)) & 0x7c00u) != 0x7c00u;
-                adj[i] = static_cast<float>(h);
-            }
-            const bool regular = finite && Impl::insideBox(s) && c0 / CPS == a0 && c1 / CPS == a1;
+            const bool regular = Impl::finiteHalves(adjWords) && Impl::insideBox(s) && c0 / CPS == a0 && c1 / CPS == a1;
             if (!regular && !home) continue;
             if (regular) {
                 if (maxBits != 0u) {
                     // neighbouring lanes take the features in rotated order (an entry starts at a multiple of
                     // 8 F bytes: lanes that all add the same feature would meet on a few LDS banks)
-                    int rotated[F];
+                    float rotatedAdj[F];
+                    Impl::rotate(adjWords, tid, rotatedAdj);
+                    double rotated[F];
 #pragma unroll
-                    for (int step = 0; step < F; ++step) {
-                        const int i = (F & (F - 1)) == 0 ? ((step + tid) & (F - 1)) : ((step + tid % F) % F);
-                        float a = adj[0];
+                    for (int i = 0; i < F; ++i) rotated[i] = static_cast<double>(rotatedAdj[i]);
+                    // The corners of the pairs of sorted coordinates that are this owner's. Along the other
+                    // coordinates the upper one is the next node: on the upper border (both are the last node) the
+                    // pair is taken as the two last, with all of the weight on the upper.
+                    typename Grid::LevelSetup t = s;
+                    unsigned rest = 0u;
 #pragma unroll
-                        for (int k = 1; k < F; ++k) a = i == k ? adj[k] : a;
-                        rotated[step] = static_cast<int>(rintf(ldexpf(a, adjointShift)));
+                    for (int d = 2; d < D; ++d) {
+                        const bool last = s.termL[d] == s.termH[d];
+                        t.f[d] = last ? 1.f : s.f[d];
+                        rest += last ? s.termL[d] - Impl::stride(d) : s.termL[d];
                     }
 #pragma unroll
-                    for (int c = 0; c < NC; ++c) {
+                    for (int sorted = 0; sorted < 4; ++sorted) {
                         int n0, n1;
-                        unsigned rest;
-                        Impl::cornerNode(s, c, n0, n1, rest);
+                        Impl::sortedNode(s, sorted, n0, n1);
                         if (n0 / CPS != item.owner0 || n1 / CPS != item.owner1) continue;
-                        const int w = static_cast<int>(rintf(ldexpf(Grid::cornerWeight(s, c), WEIGHT_BITS)));
                         long long* sums = sSums + Impl::localElement(n0, n1, rest, item.owner0, item.owner1);
 #pragma unroll
-                        for (int step = 0; step < F; ++step) {
-                            const int i = (F & (F - 1)) == 0 ? ((step + tid) & (F - 1)) : ((step + tid % F) % F);
-                            Fixed::ldsAddFixed(sums + i, static_cast<long long>(w) * static_cast<long long>(rotated[step]));
+                        for (int others = 0; others < NC / 4; ++others) {
+                            const double w = static_cast<double>(Grid::cornerWeight(t, sorted | (others << 2))) * scale;
+#pragma unroll
+                            for (int step = 0; step < F; ++step)
+                                Fixed::ldsAddFixed(sums + Impl::rotatedFeature(step, tid) + Impl::upperNodes(others) * F, Fixed::toFixed(rotated[step], w));
                         }
                     }
                 }
@@ -377,7 +493,10 @@ __global__ void __launch_bounds__(BLOCK) GridGradientColumnsKernel(
                     const float w = Grid::cornerWeight(s, c);
                     const unsigned element = Grid::cornerOffset(0, s, c);
 #pragma unroll 1
-                    for (int i = 0; i < F; ++i) unsafeAtomicAdd(gradients + element + i, w * adj[i]);
+                    for (int i = 0; i < F; ++i) {
+                        const unsigned word = adjWords[i / 2] >> (16 * (i % 2));
+                        unsafeAtomicAdd(gradients + element + i, w * static_cast<float>(__builtin_bit_cast(f16, static_cast<unsigned short>(word))));
+                    }
                 }
             }
         }
@@ -405,7 +524,7 @@ __global__ void __launch_bounds__(BLOCK) GridGradientColumnsKernel(
         // derivatives of the forward pass where it kept them; else from the entries of all corners, as the records
         // kernel gathers them -- but out of the LDS, which the sums have left: the entries around one slab are as
         // many bytes as an owner's sums (half tables) and are copied in with coalesced loads once, instead of
-        // 2^D gathers of one entry per point (dense 4-D grid with 8 features, 2^21 points: 96 -> 37 us).
+        // 2^D gathers of one entry per point (dense 4-D grid with 8 features, 2^21 points: 96 -> 32 us).
         const int a0 = item.owner0, a1 = item.owner1;
         if (a0 >= slabs0 || a1 >= slabs1) return;   // an owner of border nodes only: no slab of its own
         const int homeBegin = max(begin[1], min(runs.middle[1], end[1])), homeEnd = end[1];
@@ -431,10 +550,36 @@ __global__ void __launch_bounds__(BLOCK) GridGradientColumnsKernel(
             }
             __syncthreads();
         }
+        const bool gradientRowsOfFloat4 = D == 4 && Cfg::Start % 4 == 0 && adjInputs.strides_[1] == 1 && adjInputs.strides_[0] % 4 == 0
+            && reinterpret_cast<unsigned long long>(adjInputs.data_) % 16 == 0;
+        auto gradientOf = [&](int q, int d) {
+            return adjInputs.data_ + static_cast<long long>(q) * adjInputs.strides_[0] + static_cast<long long>(d + Cfg::Start) * adjInputs.strides_[1];
+        };
+        // (what a point needs is loaded before the lane works on the point in front of it)
+        float nextPos[D], nextGradient[D], nextAdj[F];
+        auto loadPoint = [&](int q) {
+            Impl::loadPosition(inputs.data_ + static_cast<long long>(q) * inputs.strides_[0], inputs.strides_[1], params, rowsOfFloat4, nextPos);
+            if (D == 4 && gradientRowsOfFloat4) {
+                const float4 v = *reinterpret_cast<const float4*>(gradientOf(q, 0));
+                nextGradient[0] = v.x, nextGradient[1 % D] = v.y, nextGradient[2 % D] = v.z, nextGradient[3 % D] = v.w;
+            } else {
+#pragma unroll
+                for (int d = 0; d < D; ++d) nextGradient[d] = *gradientOf(q, d);
+            }
+            if constexpr (INPUT_GRADIENTS == 1) {
+#pragma unroll
+                for (int i = 0; i < F; ++i) nextAdj[i] = static_cast<float>(typename Records::Adjoints{adjEncodedH}(q, CHANNEL_OFFSET + i));
+            }
+        };
+        if (homeBegin + tid < homeEnd) loadPoint(homeBegin + tid);
 #pragma unroll 1
         for (int p = homeBegin + tid; p < homeEnd; p += BLOCK) {
-            float pos[D];
-            Impl::loadPosition(inputs, p, params, rowsOfFloat4, pos);
+            float pos[D], gradient[D], adj[F];
+#pragma unroll
+            for (int d = 0; d < D; ++d) pos[d] = nextPos[d], gradient[d] = nextGradient[d];
+#pragma unroll
+            for (int i = 0; i < F; ++i) adj[i] = INPUT_GRADIENTS == 1 ? nextAdj[i] : 0.f;
+            if (p + BLOCK < homeEnd) loadPoint(p + BLOCK);
             float adjPos[D];
 #pragma unroll
             for (int d = 0; d < D; ++d) adjPos[d] = 0.f;
@@ -463,12 +608,16 @@ __global__ void __launch_bounds__(BLOCK) GridGradientColumnsKernel(
                 } else {
                     Records::template loadHeld<0>(s, params, held);
                 }
-                Records::template positionGradient<0>(p, s, held, typename Records::Adjoints{adjEncodedH}, adjPos);
+                Records::template positionGradient<0>(s, held, adj, adjPos);
             }
 #pragma unroll
-            for (int d = 0; d < D; ++d)
-                adjInputs.data_[static_cast<long long>(p) * adjInputs.strides_[0]
-                                + static_cast<long long>(d + Cfg::Start) * adjInputs.strides_[1]] += adjPos[d] * params.boundingBoxInvSize[d];
+            for (int d = 0; d < D; ++d) gradient[d] += adjPos[d] * params.boundingBoxInvSize[d];
+            if (D == 4 && gradientRowsOfFloat4) {
+                *reinterpret_cast<float4*>(gradientOf(p, 0)) = make_float4(gradient[0], gradient[1 % D], gradient[2 % D], gradient[3 % D]);
+            } else {
+#pragma unroll
+                for (int d = 0; d < D; ++d) *gradientOf(p, d) = gradient[d];
+            }
         }
     }
 }
