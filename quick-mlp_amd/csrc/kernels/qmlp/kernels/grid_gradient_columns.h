@@ -24,13 +24,14 @@
 //                              boundary, or on the upper border).
 // Measured on the dense 4-D grid above, 2^21 points: 150 + 7 us where the records and slice kernels take 281 + 154 us.
 // The loop over the points is short of two things at once: vector instructions (73 % of the time before the last of the steps
-// below) and 268 M additions in LDS, of which ds_add_u64 takes 6.4 lanes per clock and compute unit
-// (entries at random, features rotated; 4.5 with all addresses at random, 7.7 side by side): 68 us; the input gradients take 32, writing the sums back 8. Hence few instructions per addition: a term
-// is one v_fma_f64 (GridGradientSlices::toFixed) and a subtraction, the corners along the unsorted coordinates lie at constant distances (the
-// addresses of one serve all), features change places two to a register, and a lane's rows are found by adding to a pointer,
-// instead of integer products, an address per addition and a choice among all features: 168 -> 150 us, together with adjoints
-// scanned 8 points per load, and the input gradients' loads one point ahead and as rows of four floats. (Half of the workgroups
-// starting with the input gradients, so that two of a compute unit want different things: no gain.)
+// below) and 268 M additions in LDS, of which ds_add_u64 takes 6.4 lanes per clock and compute unit (entries at random,
+// features rotated; 4.5 with all addresses at random, 7.7 side by side): 68 us. The input gradients take 32, writing the
+// sums back 8. Hence few instructions per addition: a term is one v_fma_f64 (GridGradientSlices::toFixed) and a subtraction, the corners
+// along the unsorted coordinates lie at constant distances (the address of one serves all), features change places two to a
+// register, and a lane's rows are found by adding to a pointer, instead of integer products, an address per addition and a
+// choice among all features: 168 -> 150 us, together with adjoints scanned 8 points per load, and the input gradients' loads
+// one point ahead and as rows of four floats. (Half of the workgroups starting with the input gradients, so that two of a
+// compute unit want different things: no gain.)
 //
 // Replaces, for such batches, the atomicAdd of src_cpp/include/qmlp/kernels/encoding_hashgrid.cuh:117-166,345-369
 // of the reference.

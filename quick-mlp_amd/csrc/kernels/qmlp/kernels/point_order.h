@@ -142,21 +142,28 @@ template <int MAX_CHANNELS>
 __device__ __forceinline__ void pointOrderLoadRow(const Tensor2Read<float>& inputs, long long index, int vectorChannels, float (&row)[MAX_CHANNELS])
 {
     const float* src = inputs.data_ + index * inputs.strides_[0];
+    typedef float f32x2a __attribute__((ext_vector_type(2)));
     typedef float f32x3a __attribute__((ext_vector_type(3), aligned(4)));
+    typedef float f32x4a __attribute__((ext_vector_type(4)));
+    // (the branches fill a vector: stores to the array in each of them become one store to an address that depends on the
+    // branch, and the array moves to scratch memory)
+    f32x4a first = {0.f, 0.f, 0.f, 0.f};
     if (MAX_CHANNELS >= 4 && vectorChannels == 4) {
-        const float4 v = *reinterpret_cast<const float4*>(src);
-        row[0] = v.x; row[1] = v.y; row[2 % MAX_CHANNELS] = v.z; row[3 % MAX_CHANNELS] = v.w;
+        first = *reinterpret_cast<const f32x4a*>(src);
     } else if (MAX_CHANNELS >= 3 && vectorChannels == 3) {
         const f32x3a v = *reinterpret_cast<const f32x3a*>(src);
-        row[0] = v[0]; row[1] = v[1]; row[2 % MAX_CHANNELS] = v[2];
+        first = f32x4a{v[0], v[1], v[2], 0.f};
     } else if (MAX_CHANNELS >= 2 && vectorChannels == 2) {
-        const float2 v = *reinterpret_cast<const float2*>(src);
-        row[0] = v.x; row[1] = v.y;
+        const f32x2a v = *reinterpret_cast<const f32x2a*>(src);
+        first = f32x4a{v[0], v[1], 0.f, 0.f};
     } else {
 #pragma unroll
-        for (int c = 0; c < MAX_CHANNELS; ++c)
-            row[c] = c < inputs.sizes_[1] ? src[static_cast<long long>(c) * inputs.strides_[1]] : 0.f;
+        for (int c = 0; c < 4 && c < MAX_CHANNELS; ++c)
+            if (c < inputs.sizes_[1]) first[c] = src[static_cast<long long>(c) * inputs.strides_[1]];
     }
+#pragma unroll
+    for (int c = 0; c < MAX_CHANNELS; ++c)
+        row[c] = c < 4 ? first[c < 4 ? c : 0] : c < inputs.sizes_[1] ? src[static_cast<long long>(c) * inputs.strides_[1]] : 0.f;
 }
 
 /** How the rows of inputs can be loaded as one vector each (pointOrderLoadRow), 0 if they cannot. */
@@ -191,14 +198,21 @@ __device__ __forceinline__ void pointOrderStoreRow(float* __restrict__ sortedInp
     }
 }
 
+/** An entry of the sorted chunk in LDS. */
+template <bool STAGED_ROWS> struct PointOrderEntry { typedef unsigned int type; };
+template <> struct PointOrderEntry<true> { typedef unsigned short type; };
+
 /**
  * The workgroup sorts its chunk by slab in LDS, then walks the sorted chunk with consecutive lanes on
  * consecutive positions, so that the stores of a wavefront fall into a few runs (a scatter straight from the
  * unsorted chunk sent every lane's stores to a line of their own and took 80 us for 2^21 points).
  * Rows of up to four channels are read once, in the order given (consecutive lanes, consecutive rows), and wait
  * in LDS at their sorted place. Reading them a second time in sorted order, as wider rows still are, asks for 64
- * lines per instruction, many of which the chunks of the other workgroups have meanwhile pushed out of the L2:
- * 14 of the 42 us of this kernel for 2^21 rows of 16 bytes (the stores of the rows take 13 us, everything else 14).
+ * lines per instruction, many of which the chunks of the other workgroups have meanwhile pushed out of the L2 (14 us for
+ * 2^21 rows of 16 bytes). Two workgroups share a compute unit, so that one loads while the other stores: 2^21 rows of 16 bytes 27 us,
+ * 700 000 rows 12 us (75 and 25 MB, 2.8 and 2.1 TB/s). With the slab of each sorted point in LDS too, one workgroup had
+ * 94 KiB, and its rows went through scratch memory, because the compiler turned choices among registers into
+ * addresses: 40 and 17 us.
  * \tparam MAX_CHANNELS at least the number of input channels (4, 8, 16)
  */
 template <int MAX_CHANNELS>
@@ -212,57 +226,61 @@ __global__ void __launch_bounds__(POINT_ORDER_BLOCK) PointOrderScatter(
 {
     constexpr int CHUNK = POINT_ORDER_BLOCK * POINT_ORDER_POINTS_PER_THREAD;
     constexpr bool STAGE_ROWS = MAX_CHANNELS <= 4;
-    __shared__ int sStart[POINT_ORDER_MAX_SLABS];        // first position of the chunk's points of a slab in the sorted batch
-    __shared__ int sCount[POINT_ORDER_MAX_SLABS];
-    __shared__ int sLocalStart[POINT_ORDER_MAX_SLABS];   // the same inside the sorted chunk
+    // 78 KiB with staged rows: two workgroups per compute unit
+    __shared__ int sCount[POINT_ORDER_MAX_SLABS];        // points of the chunk per slab; then from a place in the sorted chunk to that in the batch
+    __shared__ unsigned short sLocalStart[POINT_ORDER_MAX_SLABS];   // of a slab in the sorted chunk
     __shared__ int sWaveSum[POINT_ORDER_BLOCK / WAVE_SIZE];
-    __shared__ unsigned int sSorted[CHUNK];              // sorted chunk: slab << 16 | offset of the point in the chunk
+    // sorted chunk: the offset of the point in the chunk (the slab then comes from the row again), or slab << 16 | offset
+    typedef typename PointOrderEntry<STAGE_ROWS>::type entry_t;
+    __shared__ entry_t sSorted[CHUNK];
     __shared__ __align__(16) float sRows[STAGE_ROWS ? CHUNK * MAX_CHANNELS : 4];   // the rows of the sorted chunk
     const int t = threadIdx.x;
-
-    sCount[t] = 0;
-    const int total = totals[t];
-    const int slabStart = pointOrderBlockScan(total, sWaveSum);   // holds a barrier after sCount = 0
-    sStart[t] = slabStart + histogram[blockIdx.x * POINT_ORDER_MAX_SLABS + t];
 
     const int channels = inputs.sizes_[1];
     const int vectorChannels = pointOrderVectorChannels(inputs);
     const long long chunk = static_cast<long long>(blockIdx.x) * CHUNK;
     const int chunkPoints = static_cast<int>(min(static_cast<long long>(CHUNK), numel - chunk));
+    auto slabOf = [&](const float (&row)[MAX_CHANNELS]) {
+        static_assert(MAX_CHANNELS >= 4, "a row in a vector");
+        // (single values that the compiler knows nothing about: a choice among those of an array it makes an index into scratch memory)
+        float v0 = row[0], v1 = row[1], v2 = row[2], v3 = row[3];
+        asm("" : "+v"(v0), "+v"(v1), "+v"(v2), "+v"(v3));
+        return pointOrderSlabOf([&](int c) { return c == 0 ? v0 : c == 1 ? v1 : c == 2 ? v2 : v3; }, key);
+    };
     int slab[POINT_ORDER_POINTS_PER_THREAD], rank[POINT_ORDER_POINTS_PER_THREAD];
     float rows[STAGE_ROWS ? POINT_ORDER_POINTS_PER_THREAD : 1][MAX_CHANNELS] = {};
     (void)rows;
+    if constexpr (STAGE_ROWS) {   // on their way while the totals are scanned
+#pragma unroll
+        for (int k = 0; k < POINT_ORDER_POINTS_PER_THREAD; ++k)
+            if (k * POINT_ORDER_BLOCK + t < chunkPoints) pointOrderLoadRow<MAX_CHANNELS>(inputs, chunk + k * POINT_ORDER_BLOCK + t, vectorChannels, rows[k]);
+    }
+    sCount[t] = 0;
+    const int before = histogram[blockIdx.x * POINT_ORDER_MAX_SLABS + t];
+    const int slabStart = pointOrderBlockScan(totals[t], sWaveSum) + before;   // holds a barrier after sCount = 0
 #pragma unroll
     for (int k = 0; k < POINT_ORDER_POINTS_PER_THREAD; ++k) {
         const int j = k * POINT_ORDER_BLOCK + t;
         slab[k] = 0;
         rank[k] = 0;
         if (j < chunkPoints) {
-            if constexpr (STAGE_ROWS) {
-                pointOrderLoadRow<MAX_CHANNELS>(inputs, chunk + j, vectorChannels, rows[k]);
-                const float (&row)[MAX_CHANNELS] = rows[k];
-                slab[k] = pointOrderSlabOf([&](int c) {
-                    float v = row[0];
-#pragma unroll
-                    for (int i = 1; i < MAX_CHANNELS; ++i) v = c == i ? row[i] : v;
-                    return v;
-                }, key);
-            } else {
-                slab[k] = pointOrderSlab(inputs, chunk + j, key);
-            }
+            if constexpr (STAGE_ROWS) slab[k] = slabOf(rows[k]);
+            else slab[k] = pointOrderSlab(inputs, chunk + j, key);
             rank[k] = atomicAdd(&sCount[slab[k]], 1);
         }
     }
     __syncthreads();
-    sLocalStart[t] = pointOrderBlockScan(sCount[t], sWaveSum);
+    const int localStart = pointOrderBlockScan(sCount[t], sWaveSum);
+    sLocalStart[t] = static_cast<unsigned short>(localStart);   // (4096 only behind the last point)
+    sCount[t] = slabStart - localStart;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < POINT_ORDER_POINTS_PER_THREAD; ++k) {
         const int j = k * POINT_ORDER_BLOCK + t;
         if (j < chunkPoints) {
             const int at = sLocalStart[slab[k]] + rank[k];
-            sSorted[at] = static_cast<unsigned int>(slab[k]) << 16 | static_cast<unsigned int>(j);
-            if (placement) placement[chunk + j] = sStart[slab[k]] + rank[k];
+            sSorted[at] = static_cast<entry_t>(STAGE_ROWS ? j : slab[k] << 16 | j);
+            if (placement) placement[chunk + j] = sCount[slab[k]] + at;
             if constexpr (STAGE_ROWS) {
 #pragma unroll
                 for (int c = 0; c < MAX_CHANNELS; ++c) sRows[at * MAX_CHANNELS + c] = rows[k][c];
@@ -277,7 +295,6 @@ __global__ void __launch_bounds__(POINT_ORDER_BLOCK) PointOrderScatter(
         if (j >= chunkPoints) continue;
         const unsigned int entry = sSorted[j];
         const long long index = chunk + (entry & 0xffffu);
-        const int s = static_cast<int>(entry >> 16);
         float row[MAX_CHANNELS];
         if constexpr (STAGE_ROWS) {
 #pragma unroll
@@ -285,7 +302,8 @@ __global__ void __launch_bounds__(POINT_ORDER_BLOCK) PointOrderScatter(
         } else {
             pointOrderLoadRow<MAX_CHANNELS>(inputs, index, vectorChannels, row);
         }
-        const long long position = sStart[s] + (j - sLocalStart[s]);
+        const int s = STAGE_ROWS ? slabOf(row) : static_cast<int>(entry >> 16);
+        const long long position = sCount[s] + j;
         order[position] = static_cast<int>(index);
         pointOrderStoreRow<MAX_CHANNELS>(sortedInputs, position, channels, vectorChannels, row);
     }
