@@ -2473,7 +2473,7 @@ size_t FusedNetwork::adjointMemoryAsGiven(int numElements, AdjointModeFlags adjo
     // last: transposed copies of the weights the adjoint kernel cannot keep in LDS
     std::vector<long long> transposed;
     bytes += roundUp(transposedWeightLayout(adjointFlags, transposed) * sizeof(half), size_t(16));
-    // last: bucket cursors and records of the gradient slice kernels
+    // last: the records of the gradient slice kernels and where they lie
     if (sliceGradients) bytes = roundUp(bytes, size_t(256)) + sliceGradientWorkspaceBytes(numElements);
     return bytes;
 }
