@@ -210,8 +210,8 @@ int qmlp_encoding_hashgrid_corners(qmlp_encoding_t encoding, const qmlp_tensor* 
  * (needs a bound table, src_cpp/include/qmlp/kernels/encoding_hashgrid.cuh:267-336 is what they
  * replace); mode 2: the entries and weights the gradient scatter of the fused backward kernel
  * adds to (encoding_hashgrid.cuh:345-369; nothing is added); mode 3: the entries and weights that
- * the gradient records of large batches stand for (slice of the record's bucket + 16-bit offsets,
- * and the entries of other slices that the records kernel adds itself; grids that offer gradient
+ * the gradient records of large batches stand for (slice that files the record + 16-bit offsets,
+ * and the entries of other slices that have no record; grids that offer gradient
  * slices only); mode 4: the entries behind the sums of the column kernel of sorted batches (the place of
  * each corner in the LDS of the owner of its node, and back to the table as the kernel writes its sums;
  * single dense levels that offer gradient columns only); mode 0 = qmlp_encoding_hashgrid_corners.

@@ -146,13 +146,13 @@ public:
         int place;
         int slices;
     };
-    /** What the host needs to run the kernels of kernels/grid_gradient.h for an encoding. */
     /** The temporary memory of the kernels of kernels/grid_gradient.h (mirrors kernel::GridGradientWorkspace). */
     struct GradientWorkspace
     {
         void *records, *places, *exceptions, *largest;
         int regions, recordsPerRegion, largestCount, reserved;
     };
+    /** What the host needs to run the kernels of kernels/grid_gradient.h for an encoding. */
     struct GradientSliceLayout
     {
         std::string configType;            // device type of the level table

@@ -815,7 +815,7 @@ struct GridGradientTraceLevels
                 bool other = false;
                 const int bucket = Impl::template buildRecord<LEVEL>(s, c, adjWords, rec,
                     [&](unsigned element, float weight, const Words&) { other = true; otherElement = element; otherWeight = weight; });
-                // (the records of a point outside the box are added by the records kernel itself, entry by entry as decoded here)
+                // (the pairs of a point outside the box are added by GridGradientExceptionsKernel, entry by entry as decoded here)
                 const unsigned sliceStart = static_cast<unsigned>(Cfg::memoryOffset[LEVEL]) + static_cast<unsigned>(bucket) * SLICE_FLOATS;
                 idx[LEVEL * NC + 2 * c] = sliceStart + (rec[0] & 0xffffu);
                 w[LEVEL * NC + 2 * c] = __builtin_bit_cast(float, rec[1]);
@@ -832,7 +832,7 @@ struct GridGradientTraceLevels
 /**
  * Test aid: for every point (one per lane) and level, the table elements and weights that the records of
  * GridGradientRecords::buildRecord stand for, decoded as the slice kernel decodes them (its slice +
- * 16-bit offset), and the entries the records kernel adds itself because they lie in another slice.
+ * 16-bit offset), and the entries that are exceptions because they lie in another slice.
  * Slots as in CornerTrace: level * 2^Dim + 2 * pair (+ 1 for the upper entry).
  */
 template <typename Cfg, int SLICE_FLOATS>
