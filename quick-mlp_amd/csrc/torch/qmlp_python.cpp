@@ -249,11 +249,11 @@ Gradients adjointPass(const Network_ptr& net, const at::Tensor& input, const at:
     g.tables.resize(n);
     // zeroed only where the kernels add to them
     int overwriteTables = 0;
-    {
-        std::lock_guard<std::mutex> lock(net->mutex);
-        check(qmlp_network_overwritable_tables(net->handle, wrap(input).sizes[0], flags, &overwriteTables));
-    }
-    if (flags & QMLP_GRADIENTS_INPUT_ENCODINGS)
+    if (flags & QMLP_GRADIENTS_INPUT_ENCODINGS) {
+        {
+            std::lock_guard<std::mutex> lock(net->mutex);
+            check(qmlp_network_overwritable_tables(net->handle, wrap(input).sizes[0], flags, &overwriteTables));
+        }
         // the kernel adds the gradients of every encoding with parameters: a frozen one gets a zero tensor as
         // well, which the callers drop (bind_network.cpp:277-290)
         for (size_t i = 0; i < n; ++i)
@@ -261,6 +261,7 @@ Gradients adjointPass(const Network_ptr& net, const at::Tensor& input, const at:
                 const auto options = tables.at(i).options().dtype(at::kFloat);
                 g.tables[i] = overwriteTables ? at::empty(tables[i].sizes(), options) : at::zeros(tables[i].sizes(), options);
             }
+    }
     void* stream = currentStream(input);
     const auto wrappedTables = wrapAll(*net, tables);
     const qmlp_tensor p = wrap(parameters), in = wrap(input), adjOut = wrap(adjOutput);

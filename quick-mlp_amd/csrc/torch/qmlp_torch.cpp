@@ -464,7 +464,8 @@ struct NetworkFunction : torch::autograd::Function<NetworkFunction>
             int overwrite = 0;
             QMLP_CHECK(qmlp_network_overwritable_gradients(net->handle_, static_cast<int>(input.size(0)), flags, nullptr, &overwrite));
             int overwriteTables = 0;
-            QMLP_CHECK(qmlp_network_overwritable_tables(net->handle_, static_cast<int>(input.size(0)), flags, &overwriteTables));
+            if (flags & QMLP_GRADIENTS_INPUT_ENCODINGS)
+                QMLP_CHECK(qmlp_network_overwritable_tables(net->handle_, static_cast<int>(input.size(0)), flags, &overwriteTables));
             if (overwriteTables) overwrite |= QMLP_GRADIENTS_INPUT_ENCODINGS;
             if (flags & QMLP_GRADIENTS_INPUT) adjInput = overwrite & QMLP_GRADIENTS_INPUT ? torch::empty_like(input) : torch::zeros_like(input);
             if (flags & QMLP_GRADIENTS_NETWORK_WEIGHTS) {
