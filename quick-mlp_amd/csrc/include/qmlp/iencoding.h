@@ -184,8 +184,16 @@ public:
         int workgroupsPerRegion(bool inputGradients) const { return levelGroups() + (inputGradients ? 1 : 0); }
         /** Regions that the records kernel works on at a time (of a large batch every workgroup gets several). */
         static int regionSlots(long long numel, int points) { return static_cast<int>(std::min<long long>(divUp<long long>(numel, points), 1024)); }
-        /** Workgroups of GridGradientExceptionsKernel. */
-        static int exceptionsGrid(const GradientWorkspace& workspace) { return std::min(workspace.regions, 4096); }
+        /**
+         * Lanes of a workgroup of GridGradientExceptionsKernel, and workgroups: as many as there are parts of lists, at most what the
+         * chip holds, an odd number: lists have a power of two of parts, of which often only the first ones hold anything.
+         */
+        static constexpr int EXCEPTIONS_BLOCK = 256;
+        int exceptionsGrid(const GradientWorkspace& workspace) const
+        {
+            return static_cast<int>(std::min<long long>(static_cast<long long>(workspace.regions) * static_cast<long long>(slicesPerLevel.size())
+                                                            * divUp(workspace.recordsPerRegion, EXCEPTIONS_BLOCK), 1023));
+        }
         /** The parts of the temporary memory for regions of so many points, and its bytes. */
         GradientWorkspace workspace(void* memory, long long numel, int points, size_t* bytes = nullptr) const
         {

@@ -745,54 +745,86 @@ GridGradientRecordsKernel(
     if (threadIdx.x == 0) workspace.largest[first * GROUPS + group] = static_cast<unsigned>(sCount[0]);
 }
 
-template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS, int LEVEL>
+/** Lanes of a workgroup of GridGradientExceptionsKernel. */
+constexpr int GRID_GRADIENT_EXCEPTIONS_BLOCK = 256;
+
+template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS>
 struct GridGradientExceptions
 {
     typedef GridGradientRecords<Cfg, ROW_CHANNELS, CHANNEL_OFFSET, SLICE_FLOATS, 1024> Records;
     typedef typename Records::Layout Layout;
-    /** The exceptions of a region from LEVEL on; counts: those of every level in the lanes of the wavefront. */
-    __device__ __forceinline__ static void run(int region, unsigned long long levels, const Tensor2Read<float>& inputs,
-                                               const typename Records::Adjoints& adjEncoded, const typename Records::param_t& params,
-                                               const GridGradientWorkspace& ws)
+
+    /** Where a row of GridGradientWorkspace::places says how many exceptions a level has. */
+    __device__ __forceinline__ static int placeOfCount(int level)
+    {
+        int place = 0;
+#pragma unroll
+        for (int l = 0; l < Cfg::Levels; ++l)
+            if (level == l) place = Layout::firstPlace(l) + Layout::numSlices(l) + 1;
+        return place;
+    }
+
+    /** Adds an exception of a level. */
+    template <int LEVEL>
+    __device__ __forceinline__ static void add(int level, unsigned exception, int firstPoint, const Tensor2Read<float>& inputs,
+                                               const typename Records::Adjoints& adjEncoded, const typename Records::param_t& params)
     {
         if constexpr (LEVEL < Cfg::Levels) {
-            if (levels >> (LEVEL % 64) & 1) {
-                const int count = ws.places[static_cast<long long>(region) * Layout::PLACES + Layout::firstPlace(LEVEL) + Layout::numSlices(LEVEL) + 1];
-                const unsigned short* from = ws.exceptions + (static_cast<long long>(LEVEL) * ws.regions + region) * ws.recordsPerRegion;
-                for (int i = threadIdx.x; i < count; i += 64)
-                    Records::template addException<LEVEL>(from[i], region * (ws.recordsPerRegion / Records::PAIRS), inputs, adjEncoded, params);
-            }
-            GridGradientExceptions<Cfg, ROW_CHANNELS, CHANNEL_OFFSET, SLICE_FLOATS, LEVEL + 1>::run(region, levels, inputs, adjEncoded, params, ws);
+            if (level == LEVEL) Records::template addException<LEVEL>(exception, firstPoint, inputs, adjEncoded, params);
+            else add<LEVEL + 1>(level, exception, firstPoint, inputs, adjEncoded, params);
         }
     }
 };
 
 /**
- * What the records leave out, added to the gradient tensor with atomics behind the slice kernel: one wavefront per region.
- * Few batches have any: upper entries beyond the end of a slice (in a dense level one pair in thousands), and points
- * outside of the box. A launch that finds none takes 2 to 3 us.
+ * What the records leave out, added to the gradient tensor with atomics behind the slice kernel: the points outside of the box,
+ * and in hashed levels of more cells along a coordinate than a slice has entries upper entries far away. Most batches have
+ * none: every lane looks up the number of exceptions of one list (a region and a level), and a launch that finds none takes 4 us. Lists
+ * are shared out in parts of one exception per lane, neighbouring parts over neighbouring workgroups, as points outside of the box
+ * often lie next to each other in a batch. Bound by the atomics. (A wavefront per region, which walked through its lists alone: 16
+ * levels, 2^17 points, the first 64th of them outside 1332 us for the adjoint pass, the first quarter 1427; shared out 168 and 479, and without points outside 95.)
  */
 template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS>
-__global__ void __launch_bounds__(64) GridGradientExceptionsKernel(
+__global__ void __launch_bounds__(GRID_GRADIENT_EXCEPTIONS_BLOCK) GridGradientExceptionsKernel(
     const Tensor2Read<float> inputs, const GridGradientAdjoints<ROW_CHANNELS> adjEncoded,
     const HashGridParams<typename Cfg::table_t, Cfg::Dim> params, const GridGradientWorkspace workspace)
 {
-    typedef GridGradientExceptions<Cfg, ROW_CHANNELS, CHANNEL_OFFSET, SLICE_FLOATS, 0> Impl;
-    typedef typename Impl::Layout Layout;
-    const int lane = threadIdx.x;
-    for (int region = blockIdx.x; region < workspace.regions; region += gridDim.x) {
-        // (a lane per level; bit l % 64: some level with that remainder has exceptions)
-        bool any = false;
-#pragma unroll
-        for (int l0 = 0; l0 < Cfg::Levels; l0 += 64) {
-            int place = 0;
-#pragma unroll
-            for (int l = l0; l < Cfg::Levels && l < l0 + 64; ++l)
-                if (lane == l - l0) place = Layout::firstPlace(l) + Layout::numSlices(l) + 1;
-            if (lane < Cfg::Levels - l0) any = any || workspace.places[static_cast<long long>(region) * Layout::PLACES + place] != 0;
+    typedef GridGradientExceptions<Cfg, ROW_CHANNELS, CHANNEL_OFFSET, SLICE_FLOATS> Impl;
+    constexpr int BLOCK = GRID_GRADIENT_EXCEPTIONS_BLOCK;
+    __shared__ int sCount[BLOCK];
+    __shared__ unsigned long long sFound[BLOCK / 64];
+    const int tid = threadIdx.x;
+    const unsigned parts = (workspace.recordsPerRegion + BLOCK - 1) / BLOCK;   // of a list
+    const unsigned items = static_cast<unsigned>(workspace.regions) * Cfg::Levels * parts;
+    for (unsigned i0 = 0; blockIdx.x + i0 * gridDim.x < items; i0 += BLOCK) {
+        // the parts of this workgroup: blockIdx.x + (i0 + lane) * gridDim.x
+        const unsigned item = blockIdx.x + (i0 + tid) * gridDim.x;
+        int count = 0;
+        if (item < items) {
+            const unsigned list = item / parts, part = item - list * parts, region = list / Cfg::Levels;
+            count = workspace.places[static_cast<long long>(region) * Impl::Layout::PLACES + Impl::placeOfCount(static_cast<int>(list - region * Cfg::Levels))];
+            count -= static_cast<int>(part * BLOCK);
         }
-        const unsigned long long levels = __ballot(any);
-        if (levels != 0) Impl::run(region, levels, inputs, adjEncoded, params, workspace);
+        const unsigned long long found = __ballot(count > 0);
+        if (tid % 64 == 0) sFound[tid / 64] = found;
+        sCount[tid] = count;
+        __syncthreads();
+        for (int w = 0; w < BLOCK / 64; ++w) {
+            unsigned long long left = sFound[w];
+            while (left != 0) {
+                const int from = w * 64 + __builtin_ctzll(left);
+                left &= left - 1;
+                if (tid >= sCount[from]) continue;
+                const unsigned which = blockIdx.x + (i0 + from) * gridDim.x;
+                const unsigned list = which / parts, part = which - list * parts, region = list / Cfg::Levels;
+                const int level = static_cast<int>(list - region * Cfg::Levels);
+                const unsigned short* exceptions = workspace.exceptions
+                    + (static_cast<long long>(level) * workspace.regions + region) * workspace.recordsPerRegion + part * BLOCK;
+                Impl::template add<0>(level, exceptions[tid], static_cast<int>(region) * (workspace.recordsPerRegion / Impl::Records::PAIRS), inputs,
+                                      adjEncoded, params);
+            }
+        }
+        __syncthreads();   // sFound and sCount have been read
     }
 }
 

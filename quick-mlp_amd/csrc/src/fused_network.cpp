@@ -2770,7 +2770,7 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
                 sk.kernel.fun.launch(static_cast<int>(layout.items.size()), sk.kernel.blockSize, sk.kernel.sharedMemorySize, stream, args);
             }
             void* args[] = {&inputAcc, &adjEncoded, params.data(), &regions};
-            sk.exceptions.launch(layout.exceptionsGrid(regions), 64, 0, stream, args);
+            sk.exceptions.launch(layout.exceptionsGrid(regions), layout.EXCEPTIONS_BLOCK, 0, stream, args);
         }
     }
 

@@ -294,7 +294,7 @@ void IEncoding::adjointBySlices(const GradientSliceLayout& layout, const Tensor&
         sk.slices.value().launch(static_cast<int>(layout.items.size()), 1024, layout.slicesLdsBytes(), stream, args);
     }
     void* args[] = {&inputAcc, &adjOutputAcc, parameters, &workspace};
-    sk.exceptions.value().launch(layout.exceptionsGrid(workspace), 64, 0, stream, args);
+    sk.exceptions.value().launch(layout.exceptionsGrid(workspace), layout.EXCEPTIONS_BLOCK, 0, stream, args);
 }
 
 void EncodingHashGrid::corners(const Tensor& input, unsigned* indices, float* weights, stream_t stream, int mode)
