@@ -933,9 +933,12 @@ struct GridGradientSlices
     static constexpr int SMALL = FLOATS ? 256 : 0;
     struct Shared
     {
-        unsigned segments[SEGMENTS];            // where the records of the slice begin and end in each region (16 bits each)
+        unsigned segments[SEGMENTS];            // where the records of the slice begin and end in each region (16 bits each), or parts of them
+        unsigned short regions[SEGMENTS];       // of these parts, counted from the first region that is looked up
+        int place[SEGMENTS];                    // among all parts, of the first one of each region
         unsigned largest[WAVES];
         int records[WAVES];
+        int longest[WAVES];
         int smallCount;
         float smallValues[SMALL + 1];
         unsigned short smallElements[SMALL + 1];
@@ -948,53 +951,148 @@ struct GridGradientSlices
         return place[0] | (static_cast<unsigned>(place[1]) << 16);
     }
 
+    /** Sum over the lanes in front of this one, of a workgroup; total: over all. All of them call this. */
+    __device__ __forceinline__ static int scan(int tid, int n, int (&waves)[WAVES], int& total)
+    {
+        int inclusive = n;
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const int other = __shfl_up(inclusive, d, 64);
+            if (tid % 64 >= d) inclusive += other;
+        }
+        __syncthreads();
+        if (tid % 64 == 63) waves[tid / 64] = inclusive;
+        __syncthreads();
+        const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+        int before = 0;
+        total = 0;
+#pragma unroll 1
+        for (int w = 0; w < WAVES; ++w) {
+            const int of = __builtin_amdgcn_readfirstlane(waves[w]);
+            if (w < wave) before += of;
+            total += of;
+        }
+        return before + inclusive - n;
+    }
+
+    /** Groups of so many lanes (the logarithm) take the records of a segment: half of what it holds where points are spread evenly, 8 to all. */
+    __device__ __forceinline__ static int groupLog2(const GridGradientWorkspace& ws, const GridGradientSlice& item)
+    {
+        int log2 = 3;
+        while (log2 < 10 && (4 << log2) * item.slices <= ws.recordsPerRegion) ++log2;
+        return log2;
+    }
+    static constexpr int STEPS = 3;   // records per lane of a group at a time
+    static constexpr unsigned LONG_SEGMENTS = 1u << 31;   // beside a magnitude: some segment holds more than twice what a group takes at a time
+
+    /** Whether the longest segment holds more than twice a group's share of all records of a work item. */
+    __device__ __forceinline__ static bool isUneven(const GridGradientWorkspace& ws, const GridGradientSlice& item, int begin, int end, Shared& shared)
+    {
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));   // (nothing of this is worked out, and held in registers, for batches that do not need it)
+        int records = 0, longest = 0;
+        for (int r = begin + tid; r < end; r += BLOCK) {
+            const unsigned s = segmentOf(ws, item, r);
+            const int size = static_cast<int>(s >> 16) - static_cast<int>(s & 0xffffu);
+            records += size;
+            longest = max(longest, size);
+        }
+        int all;
+        (void)scan(tid, records, shared.records, all);
+#pragma unroll
+        for (int d = 32; d > 0; d /= 2) longest = max(longest, __shfl_xor(longest, d, 64));
+        if (tid % 64 == 0) shared.longest[tid / 64] = longest;
+        __syncthreads();
+#pragma unroll 1
+        for (int w = 0; w < WAVES; ++w) longest = max(longest, shared.longest[w]);
+        return static_cast<long long>(__builtin_amdgcn_readfirstlane(longest)) * (BLOCK >> groupLog2(ws, item)) > 2ll * all;
+    }
+
     /**
      * Calls add(record) for the records of a work item. The records of a slice lie in segments, one per region, of
-     * recordsPerRegion / (slices of the level) records where the points are spread evenly: groups of half as many lanes
-     * (8 to all of them) take a segment each, three records per lane at a time, of several segments. shared.segments holds
-     * the first SEGMENTS regions.
+     * recordsPerRegion / (slices of the level) records where the points are spread evenly: groups of lanes take a segment each, STEPS
+     * records per lane, of several segments at a time. Where neighbours in the batch are neighbours in space as well (samples along rays, a
+     * batch in some order) a few segments may hold most records, and the groups that took them would work on alone (`uneven`): segments
+     * are then cut into parts of STEPS records per lane first. (Left to one group: one level of 64^3 nodes x 4 floats, adjoint pass of
+     * 2^17 samples along rays 98 us; cut 33, points at random 31.)
+     * shared.segments holds the first SEGMENTS regions.
      */
     template <typename Add>
     __device__ __forceinline__ static void forEachRecord(const GridGradientWorkspace& ws, const GridGradientSlice& item, int begin, int end,
-                                                         Shared& shared, const Add& add)
+                                                         bool uneven, Shared& shared, const Add& add)
     {
-        const int tid = threadIdx.x;
-        int groupLog2 = 3;
-        while (groupLog2 < 10 && (4 << groupLog2) * item.slices <= ws.recordsPerRegion) ++groupLog2;
-        const int group = tid >> groupLog2, groups = BLOCK >> groupLog2, lanes = 1 << groupLog2, lane = tid & (lanes - 1);
-        constexpr int UNROLL = 2, STEPS = 3;
+        const int log2 = groupLog2(ws, item);
+        if (!uneven) {
+            for (int r0 = begin; r0 < end; r0 += SEGMENTS) {
+                const int count = min(SEGMENTS, end - r0);
+                if (r0 != begin) {
+                    __syncthreads();   // the segments in front of these have been read
+                    if (static_cast<int>(threadIdx.x) < count) shared.segments[threadIdx.x] = segmentOf(ws, item, r0 + threadIdx.x);
+                    __syncthreads();
+                }
+                forEachPart<false>(threadIdx.x, ws, item, r0, count, log2, shared, add);
+            }
+            return;
+        }
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));   // (nothing of this is worked out, and held in registers, for batches that do not need it)
+        const int most = STEPS << log2;
         for (int r0 = begin; r0 < end; r0 += SEGMENTS) {
             const int count = min(SEGMENTS, end - r0);
-            if (r0 != begin) {
-                __syncthreads();   // the segments in front of these have been read
-                if (tid < count) shared.segments[tid] = segmentOf(ws, item, r0 + tid);
-                __syncthreads();
+            int all;
+            {
+                const unsigned segment = tid < count ? segmentOf(ws, item, r0 + tid) : 0u;
+                const int size = static_cast<int>(segment >> 16) - static_cast<int>(segment & 0xffffu);
+                shared.place[tid] = scan(tid, (size + most - 1) / most, shared.records, all);
             }
-            const unsigned* first = ws.records + (static_cast<long long>(item.level) * ws.regions + r0) * ws.recordsPerRegion * RW;
-            for (int s0 = group; s0 < count; s0 += UNROLL * groups) {
-                unsigned rec[UNROLL][STEPS][RW];
-                int size[UNROLL];
-                unsigned segment[UNROLL];   // (in words; a thousand regions take less than 2^27)
-#pragma unroll
-                for (int u = 0; u < UNROLL; ++u) {
-                    const int s = s0 + u * groups;
-                    const unsigned places = s < count ? shared.segments[s] : 0u;
-                    size[u] = static_cast<int>(places >> 16) - static_cast<int>(places & 0xffffu);
-                    segment[u] = (static_cast<unsigned>(s) * static_cast<unsigned>(ws.recordsPerRegion) + (places & 0xffffu)) * RW;
-#pragma unroll
-                    for (int k = 0; k < STEPS; ++k)
-                        if (lane + k * lanes < size[u]) Layout::loadRecord(first + (segment[u] + static_cast<unsigned>((lane + k * lanes) * RW)), rec[u][k]);
+            for (int q0 = 0; q0 < all; q0 += SEGMENTS) {
+                if (q0 > 0) __syncthreads();   // those in front of these have been read
+                const unsigned segment = tid < count ? segmentOf(ws, item, r0 + tid) : 0u;
+                const int place = shared.place[tid] - q0;
+                int at = max(place, 0);
+                for (int j = static_cast<int>(segment & 0xffffu) + (at - place) * most, to = static_cast<int>(segment >> 16); j < to && at < SEGMENTS; j += most, ++at) {
+                    shared.segments[at] = static_cast<unsigned>(j) | (static_cast<unsigned>(min(j + most, to)) << 16);
+                    shared.regions[at] = static_cast<unsigned short>(tid);
                 }
+                __syncthreads();
+                forEachPart<true>(tid, ws, item, r0, min(SEGMENTS, all - q0), log2, shared, add);
+            }
+        }
+    }
+
+    /** ... for so many segments of the regions from r0 on, or parts of them. */
+    template <bool PARTS, typename Add>
+    __device__ __forceinline__ static void forEachPart(int tid, const GridGradientWorkspace& ws, const GridGradientSlice& item, int r0, int count, int log2,
+                                                       const Shared& shared, const Add& add)
+    {
+        constexpr int UNROLL = PARTS ? 1 : 2;
+        const int group = tid >> log2, groups = BLOCK >> log2, lanes = 1 << log2, lane = tid & (lanes - 1);
+        const unsigned* first = ws.records + (static_cast<long long>(item.level) * ws.regions + r0) * ws.recordsPerRegion * RW;
+        for (int s0 = group; s0 < count; s0 += UNROLL * groups) {
+            unsigned rec[UNROLL][STEPS][RW];
+            int size[UNROLL];
+            unsigned segment[UNROLL];   // (in words; a thousand regions take less than 2^27)
 #pragma unroll
-                for (int u = 0; u < UNROLL; ++u) {
+            for (int u = 0; u < UNROLL; ++u) {
+                const int s = s0 + u * groups;
+                const unsigned places = s < count ? shared.segments[s] : 0u;
+                const unsigned region = !PARTS ? static_cast<unsigned>(s) : s < count ? shared.regions[s] : 0u;
+                size[u] = static_cast<int>(places >> 16) - static_cast<int>(places & 0xffffu);
+                segment[u] = (region * static_cast<unsigned>(ws.recordsPerRegion) + (places & 0xffffu)) * RW;
 #pragma unroll
-                    for (int k = 0; k < STEPS; ++k)
-                        if (lane + k * lanes < size[u]) add(rec[u][k]);
-                    for (int j = lane + STEPS * lanes; j < size[u]; j += lanes) {   // points that are not spread evenly
+                for (int k = 0; k < STEPS; ++k)
+                    if (lane + k * lanes < size[u]) Layout::loadRecord(first + (segment[u] + static_cast<unsigned>((lane + k * lanes) * RW)), rec[u][k]);
+            }
+#pragma unroll
+            for (int u = 0; u < UNROLL; ++u) {
+#pragma unroll
+                for (int k = 0; k < STEPS; ++k)
+                    if (lane + k * lanes < size[u]) add(rec[u][k]);
+                if (!PARTS)
+                    for (int j = lane + STEPS * lanes; j < size[u]; j += lanes) {   // somewhat more than on average
                         Layout::loadRecord(first + (segment[u] + static_cast<unsigned>(j * RW)), rec[u][0]);
                         add(rec[u][0]);
                     }
-                }
             }
         }
     }
@@ -1037,14 +1135,16 @@ struct GridGradientSlices
         for (int i = tid; i < ws.largestCount; i += BLOCK) largest = max(largest, ws.largest[i]);
         const int sums = item.floats < SLICE_FLOATS ? item.floats : SUMS;
         for (int i = tid; i < sums; i += BLOCK) sSlice[i] = 0;
-        int records = 0;
-        if constexpr (FLOATS) {
-            records = static_cast<int>(segment >> 16) - static_cast<int>(segment & 0xffffu);
-            for (int r = begin + SEGMENTS + tid; r < end; r += BLOCK) {
-                const unsigned s = segmentOf(ws, item, r);
-                records += static_cast<int>(s >> 16) - static_cast<int>(s & 0xffffu);
-            }
+        int records = static_cast<int>(segment >> 16) - static_cast<int>(segment & 0xffffu);
+        const int most = 2 * STEPS << groupLog2(ws, item);   // twice what a group takes of a segment at a time
+        bool some = records > most;
+        for (int r = begin + SEGMENTS + tid; r < end; r += BLOCK) {
+            const unsigned s = segmentOf(ws, item, r);
+            const int size = static_cast<int>(s >> 16) - static_cast<int>(s & 0xffffu);
+            records += size;
+            some = some || size > most;
         }
+        const bool any = __ballot(some) != 0;
 #pragma unroll
         for (int d = 32; d > 0; d /= 2) {
             largest = max(largest, static_cast<unsigned>(__shfl_xor(static_cast<int>(largest), d, 64)));
@@ -1052,18 +1152,20 @@ struct GridGradientSlices
         }
         shared.segments[tid] = segment;
         if (tid % 64 == 0) {
-            shared.largest[tid / 64] = largest;
+            shared.largest[tid / 64] = largest | (any ? LONG_SEGMENTS : 0u);
             if constexpr (FLOATS) shared.records[tid / 64] = records;
         }
         if (tid == 0) shared.smallCount = 0;
         __syncthreads();
-        unsigned maxBits = 0u;
+        unsigned maxBits = 0u, flags = 0u;
         int allRecords = 0;
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) {
-            maxBits = max(maxBits, shared.largest[w]);
+            maxBits = max(maxBits, shared.largest[w] & ~LONG_SEGMENTS);
+            flags |= shared.largest[w];
             if constexpr (FLOATS) allRecords += shared.records[w];
         }
+        const bool uneven = (__builtin_amdgcn_readfirstlane(flags) & LONG_SEGMENTS) != 0 && isUneven(ws, item, begin, end, shared);
         const bool finite = maxBits < (FLOATS ? 0x7f800000u : 0x7c00u);
         // |adjoint| < 2^maxExponent: 2^(biased exponent - 14) of halves, 2^(biased exponent - 126) of floats, subnormals included
         const int maxExponent = FLOATS ? static_cast<int>(maxBits >> 23) - 126 : static_cast<int>(maxBits >> 10) - 14;
@@ -1083,7 +1185,7 @@ struct GridGradientSlices
         if (maxBits == 0u) {
             // all adjoints are zero: nothing to add
         } else if (finite) {
-            forEachRecord(ws, item, begin, end, shared, [&](const unsigned (&rec)[RW]) {
+            forEachRecord(ws, item, begin, end, uneven, shared, [&](const unsigned (&rec)[RW]) {
                 forEachTerm(rec, [&](unsigned element, float v) {
                     if constexpr (FLOATS) {
                         if (fabsf(v) < smallest) {
@@ -1101,7 +1203,7 @@ struct GridGradientSlices
                 });
             });
         } else {
-            forEachRecord(ws, item, begin, end, shared, [&](const unsigned (&rec)[RW]) {
+            forEachRecord(ws, item, begin, end, uneven, shared, [&](const unsigned (&rec)[RW]) {
                 forEachTerm(rec, [&](unsigned element, float v) { Grid::ldsAdd(sFloat + element, v); });
             });
         }
@@ -1129,11 +1231,10 @@ struct GridGradientSlices
             if (small <= SMALL) {
                 if (tid < small) unsafeAtomicAdd(grad + shared.smallElements[tid], shared.smallValues[tid]);
             } else {
-                if (end - begin > SEGMENTS) {
-                    shared.segments[tid] = segment;
-                    __syncthreads();
-                }
-                forEachRecord(ws, item, begin, end, shared, [&](const unsigned (&rec)[RW]) {
+                // (the segments of the first regions, where others have taken their place)
+                shared.segments[tid] = tid < min(SEGMENTS, end - begin) ? segmentOf(ws, item, begin + tid) : 0u;
+                __syncthreads();
+                forEachRecord(ws, item, begin, end, uneven, shared, [&](const unsigned (&rec)[RW]) {
                     forEachTerm(rec, [&](unsigned element, float v) {
                         if (fabsf(v) < smallest && v != 0.f) unsafeAtomicAdd(grad + element, v);
                     });

@@ -4,6 +4,7 @@ with a run of points outside, whose lists a whole chip has to share."""
 import ctypes
 import json
 
+import numpy as np
 import pytest
 import torch
 
@@ -33,6 +34,27 @@ def adjoint_call(enc, x, table, g, mode=2):
     return run, out
 
 
+def check_sums(enc, cfg, x, g, got):
+    """The table gradients of adjoints g at points x against sums in double precision."""
+    count, dims, features = x.shape[0], cfg["n_in"], cfg["n_features_per_level"]
+    index, weight = enc.hashgrid_corners(x)   # (points, levels, corners)
+    index, weight = index.cpu().numpy(), weight.cpu().numpy().astype(np.float64)
+    adjoints = g.cpu().numpy().astype(np.float64).reshape(count, cfg["n_levels"], features)
+    sums, magnitude, terms = (np.zeros(enc.num_parameters()) for _ in range(3))
+    for f in range(features):   # (on the host: atomics of the whole batch on one entry take minutes)
+        term = (weight * adjoints[:, :, f, None]).reshape(-1)
+        at = (index + f).reshape(-1)
+        sums += np.bincount(at, term, sums.size)
+        magnitude += np.bincount(at, np.abs(term), sums.size)
+        terms += np.bincount(at, minlength=sums.size)
+    # Float additions in any order: each rounds by at most 2^-24 of a running sum that stays below the sum of magnitudes; a term is a
+    # product of at most dims + 1 rounded factors, taken in another order here. Fixed-point sums are finer than 2^-35 of the largest
+    # adjoint each.
+    bound = (terms + 2 * dims + 4) * 2.0 ** -24 * magnitude + terms * 2.0 ** -35 * float(g.abs().max()) + 1e-12
+    error = np.abs(got.cpu().numpy().astype(np.float64) - sums)
+    assert (error <= bound).all(), float((error / bound).max())
+
+
 def outside(x, beyond):
     """The points moved to just behind the upper border of the first coordinate."""
     y = x.clone()
@@ -49,7 +71,7 @@ GRIDS = [grid(8, 2, 13, "float"), grid(9, 3, 14, "half", 2), grid(8, 2, 16, "flo
 def test_against_sums_in_double_precision(cfg, count, kind):
     require_gpu(cfg, (2,))
     enc = qmlp.Encoding(json.dumps(cfg))
-    dims, features = cfg["n_in"], cfg["n_features_per_level"]
+    dims = cfg["n_in"]
     print("exceptions", cfg["max_resolution"], count, kind, flush=True)
     gen = torch.Generator(device="cuda").manual_seed(count)
     x = torch.rand(count, dims, device="cuda", generator=gen)
@@ -59,21 +81,7 @@ def test_against_sums_in_double_precision(cfg, count, kind):
     g = torch.randn(count, enc.num_output_channels(), device="cuda", generator=gen)
     run, got = adjoint_call(enc, x, table, g)
     run()
-    index, weight = enc.hashgrid_corners(x)   # (points, levels, corners)
-    index, weight = index.long(), weight.double()
-    sums = torch.zeros(enc.num_parameters(), dtype=torch.float64, device="cuda")
-    magnitude, terms = torch.zeros_like(sums), torch.zeros_like(sums)
-    for f in range(features):
-        term = weight * g.double().reshape(count, cfg["n_levels"], features)[:, :, f, None]
-        at = (index + f).reshape(-1)
-        sums.index_add_(0, at, term.reshape(-1))
-        magnitude.index_add_(0, at, term.abs().reshape(-1))
-        terms.index_add_(0, at, torch.ones_like(term).reshape(-1))
-    # Float additions in any order: each rounds by at most 2^-24 of a running sum that stays below the sum of magnitudes; a term is a
-    # product of at most dims + 1 rounded factors, taken in another order here. Fixed-point sums are finer than 2^-35 of the largest
-    # adjoint each.
-    bound = (terms + 2 * dims + 4) * 2.0 ** -24 * magnitude + terms * 2.0 ** -35 * float(g.abs().max()) + 1e-12
-    assert bool(((got.double() - sums).abs() <= bound).all()), float(((got.double() - sums).abs() / bound).max())
+    check_sums(enc, cfg, x, g, got)
 
 
 def time_of(run):
