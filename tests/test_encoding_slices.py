@@ -62,7 +62,12 @@ def test_gradients_by_slices(cfg, points):
     _, adj_table = adjoint(enc, inside, table, g * scale, 2, True)
     small = expected.abs() < 1e4
     assert small.any() and torch.equal(expected == 0, adj_table == 0)
-    torch.testing.assert_close(adj_table[small], expected[small], rtol=1e-4, atol=1e-4)
+    # Float additions (the expected sums, and those of coarse levels) come in any order: each rounds with a standard deviation of at
+    # most 2^-24 / sqrt(3) of the running sum, a random walk that ends within the largest of these sums. Two sums of k terms differ
+    # by sqrt(2 k / 3) 2^-24 of that, here by six of these (12 609 terms, sums up to 76: 2.5e-3; 1.9e-4 seen in 20 repetitions).
+    corners = enc.hashgrid_corners(inside)[0]
+    order = 6 * (2 * int(torch.bincount(corners.flatten()).max()) / 3) ** 0.5 * 2.0 ** -24 * float(expected[small].abs().max())
+    torch.testing.assert_close(adj_table[small], expected[small], rtol=1e-4, atol=order)
 
     # NaN and infinity reach the gradients
     g[7, 0], g[points - 1, 1] = float("nan"), float("inf")
