@@ -407,6 +407,7 @@ struct GridGradientRecords
         unsigned rec[PAIRS][RW];
         int bucket[PAIRS], rank[PAIRS];
         const typename Grid::LevelSetup s = Grid::setupLevel(LEVEL, pos);
+        bool filed = valid;
         if (valid) {
             unsigned adjWords[AW];
 #pragma unroll
@@ -426,7 +427,8 @@ struct GridGradientRecords
             // The sums of the slice kernel are fixed point with a scale that counts on weights of at most one, which
             // holds while every fractional position lies in [0, 1]: for every point inside the box. A point outside of
             // it is extrapolated (the fractional position is not clamped) with weights that grow with its distance, a
-            // NaN coordinate gives NaN weights: the pairs of such a point are exceptions, and their records hold zeros.
+            // NaN coordinate gives NaN weights: the pairs of such a point are exceptions and have no records (in a level of one
+            // slice, where every lane has fixed places, records of zeros).
             bool inside = true;
 #pragma unroll
             for (int d = 0; d < D; ++d) inside = inside && s.f[d] >= 0.f && s.f[d] <= 1.f;
@@ -439,9 +441,10 @@ struct GridGradientRecords
                 bool otherSlice = false;
                 bucket[c] = buildRecord<LEVEL>(s, c, adjWords, rec[c], [&](unsigned, float, const unsigned (&)[AW]) { otherSlice = true; });
                 // (a level of one slice needs no sorting: every lane has fixed places)
-                rank[c] = NS == 1 ? tid * PAIRS + c : atomicAdd(sCount + bucket[c], 1);
+                rank[c] = NS == 1 ? tid * PAIRS + c : inside ? atomicAdd(sCount + bucket[c], 1) : 0;
                 if (otherSlice && inside) except(c, EXCEPTION_UPPER_ONLY);
             }
+            filed = NS == 1 || inside;
             if (!inside) {
 #pragma unroll
                 for (int c = 0; c < PAIRS; ++c) {
@@ -483,7 +486,7 @@ struct GridGradientRecords
         ldsBarrier();
 
         for (int b = tid; b <= NS; b += POINTS) sCount[b] = 0;
-        if (valid) {
+        if (filed) {
 #pragma unroll
             for (int c = 0; c < PAIRS; ++c) Layout::storeRecord(sStage + (sStart[bucket[c]] + rank[c]) * RW, rec[c]);
         }
