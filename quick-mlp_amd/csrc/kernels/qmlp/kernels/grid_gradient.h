@@ -156,7 +156,7 @@ struct GridGradientLayout
         }
     }
 
-    /** Records start at multiples of their size from a 16-byte aligned base (LDS or global memory). */
+    /** Records start at multiples of their size from a 16-byte aligned base (LDS or global memory): 16, 8 or 4 bytes at a time. */
     template <typename Pointer>
     __device__ __forceinline__ static void loadRecord(Pointer src, unsigned (&r)[RECORD_WORDS])
     {
@@ -165,6 +165,12 @@ struct GridGradientLayout
             for (int v = 0; v < RECORD_WORDS / 4; ++v) {
                 const uint4 q = reinterpret_cast<const uint4*>(src)[v];
                 r[4 * v] = q.x, r[4 * v + 1] = q.y, r[4 * v + 2] = q.z, r[4 * v + 3] = q.w;
+            }
+        } else if constexpr (RECORD_WORDS % 2 == 0) {
+#pragma unroll
+            for (int v = 0; v < RECORD_WORDS / 2; ++v) {
+                const uint2 q = reinterpret_cast<const uint2*>(src)[v];
+                r[2 * v] = q.x, r[2 * v + 1] = q.y;
             }
         } else {
 #pragma unroll
@@ -177,6 +183,9 @@ struct GridGradientLayout
 #pragma unroll
             for (int v = 0; v < RECORD_WORDS / 4; ++v)
                 reinterpret_cast<uint4*>(dst)[v] = make_uint4(r[4 * v], r[4 * v + 1], r[4 * v + 2], r[4 * v + 3]);
+        } else if constexpr (RECORD_WORDS % 2 == 0) {
+#pragma unroll
+            for (int v = 0; v < RECORD_WORDS / 2; ++v) reinterpret_cast<uint2*>(dst)[v] = make_uint2(r[2 * v], r[2 * v + 1]);
         } else {
 #pragma unroll
             for (int v = 0; v < RECORD_WORDS; ++v) dst[v] = r[v];
@@ -985,8 +994,8 @@ struct GridGradientSlices
         while (log2 < 10 && (4 << log2) * item.slices <= ws.recordsPerRegion) ++log2;
         return log2;
     }
-    static constexpr int STEPS = 3;   // records per lane of a group at a time
-    static constexpr unsigned LONG_SEGMENTS = 1u << 31;   // beside a magnitude: some segment holds more than twice what a group takes at a time
+    static constexpr int STEPS = 3;   // records per lane of a part of a segment
+    static constexpr unsigned LONG_SEGMENTS = 1u << 31;   // beside a magnitude: some segment holds more than twice what a part does
 
     /** Whether the longest segment holds more than twice a group's share of all records of a work item. */
     __device__ __forceinline__ static bool isUneven(const GridGradientWorkspace& ws, const GridGradientSlice& item, int begin, int end, Shared& shared)
@@ -1013,19 +1022,24 @@ struct GridGradientSlices
 
     /**
      * Calls add(record) for the records of a work item. The records of a slice lie in segments, one per region, of
-     * recordsPerRegion / (slices of the level) records where the points are spread evenly: groups of lanes take a segment each, STEPS
-     * records per lane, of several segments at a time. Where neighbours in the batch are neighbours in space as well (samples along rays, a
+     * recordsPerRegion / (slices of the level) records where the points are spread evenly. A group of lanes takes segments as one stream of
+     * records: a lane that is through with one goes on in the group's next, so that every load and every addition is that of whole
+     * wavefronts, and the loads of the next records are under way while these are added. (A segment at a time, three records per lane,
+     * left a third of the additions to lanes without a record, and nothing was under way meanwhile: four levels of halves, 2^20
+     * points 307 us for the adjoint pass, now 266; a dense 4-D grid of 8 features, four records to a segment, 2^19 points 207 and 177; 16
+     * levels, 2^18 points 197 and 187.) Where neighbours in the batch are neighbours in space as well (samples along rays, a
      * batch in some order) a few segments may hold most records, and the groups that took them would work on alone (`uneven`): segments
      * are then cut into parts of STEPS records per lane first. (Left to one group: one level of 64^3 nodes x 4 floats, adjoint pass of
-     * 2^17 samples along rays 98 us; cut 33, points at random 31.)
+     * 2^17 samples along rays 98 us; cut 34, points at random 29.)
      * shared.segments holds the first SEGMENTS regions.
+     * \tparam RARE passes that few batches need, as little code as possible: cut into parts in any case
      */
-    template <typename Add>
+    template <bool RARE, typename Add>
     __device__ __forceinline__ static void forEachRecord(const GridGradientWorkspace& ws, const GridGradientSlice& item, int begin, int end,
                                                          bool uneven, Shared& shared, const Add& add)
     {
         const int log2 = groupLog2(ws, item);
-        if (!uneven) {
+        if (!RARE && !uneven) {
             for (int r0 = begin; r0 < end; r0 += SEGMENTS) {
                 const int count = min(SEGMENTS, end - r0);
                 if (r0 != begin) {
@@ -1033,7 +1047,7 @@ struct GridGradientSlices
                     if (static_cast<int>(threadIdx.x) < count) shared.segments[threadIdx.x] = segmentOf(ws, item, r0 + threadIdx.x);
                     __syncthreads();
                 }
-                forEachPart<false>(threadIdx.x, ws, item, r0, count, log2, shared, add);
+                forEachPart<false, false>(threadIdx.x, ws, item, r0, count, log2, shared, add);
             }
             return;
         }
@@ -1058,45 +1072,65 @@ struct GridGradientSlices
                     shared.regions[at] = static_cast<unsigned short>(tid);
                 }
                 __syncthreads();
-                forEachPart<true>(tid, ws, item, r0, min(SEGMENTS, all - q0), log2, shared, add);
+                forEachPart<true, RARE>(tid, ws, item, r0, min(SEGMENTS, all - q0), log2, shared, add);
             }
         }
     }
 
     /** ... for so many segments of the regions from r0 on, or parts of them. */
-    template <bool PARTS, typename Add>
+    template <bool PARTS, bool RARE, typename Add>
     __device__ __forceinline__ static void forEachPart(int tid, const GridGradientWorkspace& ws, const GridGradientSlice& item, int r0, int count, int log2,
                                                        const Shared& shared, const Add& add)
     {
-        constexpr int UNROLL = PARTS ? 1 : 2;
-        const int group = tid >> log2, groups = BLOCK >> log2, lanes = 1 << log2, lane = tid & (lanes - 1);
+        constexpr int LOADS = RARE ? 1 : 2;
+        const int groups = BLOCK >> log2, lanes = 1 << log2;
         const unsigned* first = ws.records + (static_cast<long long>(item.level) * ws.regions + r0) * ws.recordsPerRegion * RW;
-        for (int s0 = group; s0 < count; s0 += UNROLL * groups) {
-            unsigned rec[UNROLL][STEPS][RW];
-            int size[UNROLL];
-            unsigned segment[UNROLL];   // (in words; a thousand regions take less than 2^27)
+        // this lane is at record `at` of part s, which begins at word `base` (a thousand regions take less than 2^27) and has `size`
+        int s = tid >> log2, at = tid & (lanes - 1), size = 0;
+        unsigned base = 0u;
+        auto look = [&] {
+            const unsigned places = shared.segments[s], region = PARTS ? shared.regions[s] : static_cast<unsigned>(s);
+            size = static_cast<int>(places >> 16) - static_cast<int>(places & 0xffffu);
+            base = (region * static_cast<unsigned>(ws.recordsPerRegion) + (places & 0xffffu)) * RW;
+        };
+        // (loads without a branch around them: only then those of the next records can be in flight while these are added)
+        auto load = [&](unsigned (&rec)[LOADS][RW]) {
+            int loaded = 0;
 #pragma unroll
-            for (int u = 0; u < UNROLL; ++u) {
-                const int s = s0 + u * groups;
-                const unsigned places = s < count ? shared.segments[s] : 0u;
-                const unsigned region = !PARTS ? static_cast<unsigned>(s) : s < count ? shared.regions[s] : 0u;
-                size[u] = static_cast<int>(places >> 16) - static_cast<int>(places & 0xffffu);
-                segment[u] = (region * static_cast<unsigned>(ws.recordsPerRegion) + (places & 0xffffu)) * RW;
-#pragma unroll
-                for (int k = 0; k < STEPS; ++k)
-                    if (lane + k * lanes < size[u]) Layout::loadRecord(first + (segment[u] + static_cast<unsigned>((lane + k * lanes) * RW)), rec[u][k]);
+            for (int u = 0; u < LOADS; ++u) {
+                while (at >= size && s < count) {
+                    at -= size;
+                    s += groups;
+                    if (s < count) look();
+                }
+                Layout::loadRecord(first + (s < count ? base + static_cast<unsigned>(at * RW) : 0u), rec[u]);
+                at += lanes;
+                loaded += s < count ? 1 : 0;
             }
+            return loaded;
+        };
+        auto addAll = [&](const unsigned (&rec)[LOADS][RW], int loaded) {
 #pragma unroll
-            for (int u = 0; u < UNROLL; ++u) {
-#pragma unroll
-                for (int k = 0; k < STEPS; ++k)
-                    if (lane + k * lanes < size[u]) add(rec[u][k]);
-                if (!PARTS)
-                    for (int j = lane + STEPS * lanes; j < size[u]; j += lanes) {   // somewhat more than on average
-                        Layout::loadRecord(first + (segment[u] + static_cast<unsigned>(j * RW)), rec[u][0]);
-                        add(rec[u][0]);
-                    }
+            for (int u = 0; u < LOADS; ++u)
+                if (u < loaded) add(rec[u]);
+        };
+        if (s < count) look();
+        if constexpr (RARE || PARTS) {
+            for (;;) {
+                unsigned rec[LOADS][RW];
+                const int loaded = load(rec);
+                if (loaded == 0) return;
+                addAll(rec, loaded);
             }
+        }
+        unsigned these[LOADS][RW], next[LOADS][RW];
+        int loaded = load(these);
+        while (loaded > 0) {
+            const int more = load(next);
+            addAll(these, loaded);
+            if (more == 0) break;
+            loaded = load(these);
+            addAll(next, more);
         }
     }
 
@@ -1139,7 +1173,7 @@ struct GridGradientSlices
         const int sums = item.floats < SLICE_FLOATS ? item.floats : SUMS;
         for (int i = tid; i < sums; i += BLOCK) sSlice[i] = 0;
         int records = static_cast<int>(segment >> 16) - static_cast<int>(segment & 0xffffu);
-        const int most = 2 * STEPS << groupLog2(ws, item);   // twice what a group takes of a segment at a time
+        const int most = 2 * STEPS << groupLog2(ws, item);   // twice a part of a segment
         bool some = records > most;
         for (int r = begin + SEGMENTS + tid; r < end; r += BLOCK) {
             const unsigned s = segmentOf(ws, item, r);
@@ -1188,7 +1222,7 @@ struct GridGradientSlices
         if (maxBits == 0u) {
             // all adjoints are zero: nothing to add
         } else if (finite) {
-            forEachRecord(ws, item, begin, end, uneven, shared, [&](const unsigned (&rec)[RW]) {
+            forEachRecord<false>(ws, item, begin, end, uneven, shared, [&](const unsigned (&rec)[RW]) {
                 forEachTerm(rec, [&](unsigned element, float v) {
                     if constexpr (FLOATS) {
                         if (fabsf(v) < smallest) {
@@ -1206,7 +1240,7 @@ struct GridGradientSlices
                 });
             });
         } else {
-            forEachRecord(ws, item, begin, end, uneven, shared, [&](const unsigned (&rec)[RW]) {
+            forEachRecord<true>(ws, item, begin, end, uneven, shared, [&](const unsigned (&rec)[RW]) {
                 forEachTerm(rec, [&](unsigned element, float v) { Grid::ldsAdd(sFloat + element, v); });
             });
         }
@@ -1237,7 +1271,7 @@ struct GridGradientSlices
                 // (the segments of the first regions, where others have taken their place)
                 shared.segments[tid] = tid < min(SEGMENTS, end - begin) ? segmentOf(ws, item, begin + tid) : 0u;
                 __syncthreads();
-                forEachRecord(ws, item, begin, end, uneven, shared, [&](const unsigned (&rec)[RW]) {
+                forEachRecord<true>(ws, item, begin, end, uneven, shared, [&](const unsigned (&rec)[RW]) {
                     forEachTerm(rec, [&](unsigned element, float v) {
                         if (fabsf(v) < smallest && v != 0.f) unsafeAtomicAdd(grad + element, v);
                     });

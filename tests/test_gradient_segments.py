@@ -1,5 +1,6 @@
 """Table gradients of batches whose neighbours are neighbours in space (samples along rays, sorted points, one cell): the records of a
-slice then lie in a few long segments, which the slice kernel cuts into parts. Batches of up to a thousand regions and of more, parts
+slice then lie in a few long segments, which the slice kernel cuts into parts; and of points spread evenly, in segments of a few
+records to some dozens. Batches of up to a thousand regions and of more, parts
 that take several rounds, floats too small for the sums, against sums in double precision; and the time of rays."""
 import json
 
@@ -13,11 +14,15 @@ from test_overwritten_tables import grid
 
 pytestmark = pytest.mark.gpu
 
-GRIDS = {"dense": grid(1, 4, -1, "float", 3, (64, 64)), "levels": grid(8, 2, 14, "half", 3, (5, 200)), "wide": grid(1, 8, -1, "float", 4, (20, 20))}
+GRIDS = {"many": grid(1, 8, -1, "half", 4, (32, 32)),   # 512 slices: four records to a segment
+         "dense": grid(1, 4, -1, "float", 3, (64, 64)),
+         "levels": grid(8, 2, 14, "half", 3, (5, 200)), "wide": grid(1, 8, -1, "float", 4, (20, 20))}
 
 
 def points(kind, count, dims, gen):
     x = torch.rand(count, dims, device="cuda", generator=gen)
+    if kind == "even":
+        return x
     if kind == "sorted":
         return x[torch.argsort(x[:, 0])].contiguous()
     if kind == "cell":
@@ -31,8 +36,9 @@ def points(kind, count, dims, gen):
     return (begin + t * (end - begin)).reshape(-1, dims)[:count].contiguous()
 
 
-@pytest.mark.parametrize("name,count", [("dense", 1 << 16), ("dense", (1 << 20) + 12345), ("levels", 70001), ("wide", 150001)])
-@pytest.mark.parametrize("kind", ["rays", "sorted", "cell", "some"])
+@pytest.mark.parametrize("name,count", [("dense", 1 << 16), ("dense", (1 << 20) + 12345), ("levels", 70001), ("levels", 1 << 14),
+                                        ("wide", 150001), ("many", 1 << 16), ("many", 600001)])
+@pytest.mark.parametrize("kind", ["even", "rays", "sorted", "cell", "some"])
 @pytest.mark.parametrize("span", [0, 60])
 def test_against_sums_in_double_precision(name, count, kind, span):
     cfg = GRIDS[name]
