@@ -943,6 +943,7 @@ struct GridGradientSlices
     static constexpr int SEGMENTS = BLOCK;      // regions that are looked up together
     static constexpr int WAVES = BLOCK / 64;
     static constexpr int SMALL = FLOATS ? 256 : 0;
+    static constexpr int MOST_TERMS_WITH_LIST = 3 << 16;   // of a work item; of normally distributed adjoints about a hundred are on the list then
     struct Shared
     {
         unsigned segments[SEGMENTS];            // where the records of the slice begin and end in each region (16 bits each), or parts of them
@@ -1215,10 +1216,21 @@ struct GridGradientSlices
         const int scaleExponent = min(61 - termsLog2, FIXED_BITS) - maxExponent;
         const double scale = ldexp(1.0, scaleExponent), unit = ldexp(1.0, -scaleExponent);
         float* sFloat = reinterpret_cast<float*>(sSlice);
-        // Floats span more than the 64 bits of a sum: a value of which the sum would lose bits is added to the gradient tensor
-        // behind the sums, from a list, or if that is full by another pass over the records.
+        // Floats span more than the 64 bits of a sum: a value of which the sum would lose bits is added to the gradient tensor. Of few
+        // records behind the sums, from a list (or if that is full by another pass over the records); many records have more
+        // of these than a list holds, as each halves the unit of the sums: they are added right away, to what is there or to zeros.
+        // (One level of 64^3 nodes x 4, 2^20 points: a second pass for lists that were full made 64 us of 33.)
         const float smallest = ldexpf(1.f, 23 - scaleExponent);
         (void)smallest;
+        float* __restrict__ grad = gradients + item.first;
+        const int firstOwn = item.parts > 1 ? sums : item.slice > 0 ? F : 0;   // (see below)
+        const bool direct = FLOATS && static_cast<long long>(__builtin_amdgcn_readfirstlane(allRecords)) * (2 * F) > MOST_TERMS_WITH_LIST;
+        if (direct) {
+            if (overwrite)
+                for (int i = firstOwn + tid; i < min(sums, SLICE_FLOATS); i += BLOCK) grad[i] = 0.f;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's stores have been carried out
+            __syncthreads();
+        }
         if (maxBits == 0u) {
             // all adjoints are zero: nothing to add
         } else if (finite) {
@@ -1226,7 +1238,9 @@ struct GridGradientSlices
                 forEachTerm(rec, [&](unsigned element, float v) {
                     if constexpr (FLOATS) {
                         if (fabsf(v) < smallest) {
-                            if (v != 0.f) {
+                            if (v != 0.f && direct) {
+                                unsafeAtomicAdd(grad + element, v);
+                            } else if (v != 0.f) {
                                 const int at = atomicAdd(&shared.smallCount, 1);
                                 if (at < SMALL) {
                                     shared.smallValues[at] = v;
@@ -1244,14 +1258,25 @@ struct GridGradientSlices
                 forEachTerm(rec, [&](unsigned element, float v) { Grid::ldsAdd(sFloat + element, v); });
             });
         }
+        if (direct) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's atomics have been carried out
         __syncthreads();
         // Added to the gradient tensor: with atomics (16 neighbouring floats per request) where other work
         // items hold sums for the same slice (parts > 1), and for the first entry of a slice and the one behind it, to
         // which two slices add; else this workgroup is the only writer of its slice in this launch.
-        float* __restrict__ grad = gradients + item.first;
-        const int firstOwn = item.parts > 1 ? sums : item.slice > 0 ? F : 0;
+        auto sumOf = [&](int i) { return finite ? static_cast<float>(static_cast<double>(sSlice[i]) * unit) : sFloat[i]; };
+        if (direct) {
+#pragma unroll 1
+            for (int i = tid; i < sums; i += BLOCK) {
+                const float v = sumOf(i);
+                if (v == 0.f) continue;
+                if (i < firstOwn || i >= SLICE_FLOATS) unsafeAtomicAdd(grad + i, v);
+                // (read behind this workgroup's own atomics: they have ended, but the L1 does not know of them)
+                else grad[i] = __hip_atomic_load(grad + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + v;
+            }
+            return;
+        }
         for (int i = tid; i < sums; i += BLOCK) {
-            const float v = finite ? static_cast<float>(static_cast<double>(sSlice[i]) * unit) : sFloat[i];
+            const float v = sumOf(i);
             if (i < firstOwn || i >= SLICE_FLOATS) {
                 if (v != 0.f) unsafeAtomicAdd(grad + i, v);
             } else if (overwrite) {

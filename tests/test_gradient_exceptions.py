@@ -17,8 +17,8 @@ from test_overwritten_tables import grid
 pytestmark = pytest.mark.gpu
 
 
-def adjoint_call(enc, x, table, g, mode=2):
-    """A function that runs one adjoint pass by slices, and the table gradients that it writes."""
+def adjoint_call(enc, x, table, g, mode=2, overwrite=True):
+    """A function that runs one adjoint pass by slices, and the table gradients that it writes, or adds to."""
     size = ctypes.c_size_t()
     check(lib.qmlp_encoding_adjoint_memory(enc._handle, x.shape[0], mode, ctypes.byref(size)))
     assert size.value > 0
@@ -29,8 +29,8 @@ def adjoint_call(enc, x, table, g, mode=2):
     stream = current_stream(x.device)
 
     def run(keep=(x, g, table, adj_x, out, memory)):
-        check(lib.qmlp_encoding_adjoint_overwriting(enc._handle, descs[0], descs[1], descs[2], stream, desc(table), desc(out), mode,
-                                                    memory.data_ptr()))
+        call = lib.qmlp_encoding_adjoint_overwriting if overwrite else lib.qmlp_encoding_adjoint_in
+        check(call(enc._handle, descs[0], descs[1], descs[2], stream, desc(table), desc(out), mode, memory.data_ptr()))
     return run, out
 
 

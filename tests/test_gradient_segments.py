@@ -53,6 +53,11 @@ def test_against_sums_in_double_precision(name, count, kind, span):
     run, got = adjoint_call(enc, x, table, g)
     run()
     check_sums(enc, cfg, x, g, got)
+    # added to gradients that are there: as much again (the last rounding is one of those that the bound counts)
+    run, twice = adjoint_call(enc, x, table, g, overwrite=False)
+    twice.copy_(got)
+    run()
+    check_sums(enc, cfg, x, g, twice - got)
 
 
 def test_samples_along_rays_take_as_long_as_points_at_random():
@@ -69,3 +74,20 @@ def test_samples_along_rays_take_as_long_as_points_at_random():
         times.append(time_of(adjoint_call(enc, x, table, g)[0]))
     print("random, rays:", times, flush=True)
     assert times[1] < 2 * times[0]
+
+
+def test_time_grows_with_the_batch():
+    """Floats that are too small for the fixed-point sums of a slice grow with the square of its records: 2^20 points behind a dense 4-D
+    grid of 8 features have more of them than the list of a workgroup holds. Reading all records a second time for these made the pass
+    2.7 times as long as that of half as many points (twice where they are added right away)."""
+    cfg = GRIDS["many"]
+    require_gpu(cfg, (2,))
+    enc = qmlp.Encoding(json.dumps(cfg))
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    table = torch.zeros(enc.num_parameters(), device="cuda", dtype=enc.parameter_dtype())
+    times = []
+    for count in (1 << 19, 1 << 20):
+        x, g = torch.rand(count, 4, device="cuda", generator=gen), torch.randn(count, 8, device="cuda", generator=gen)
+        times.append(time_of(adjoint_call(enc, x, table, g)[0]))
+    print("2^19, 2^20 points:", times, flush=True)
+    assert times[1] < 2.35 * times[0]
