@@ -176,12 +176,16 @@ public:
             for (int s : slicesPerLevel) n += s;
             return n;
         }
-        /**
-         * Workgroups of the records kernel over which the levels of a region are shared out; input gradients have one more
-         * of their own.
-         */
-        int levelGroups() const { return std::min(8, static_cast<int>(slicesPerLevel.size())); }
-        int workgroupsPerRegion(bool inputGradients) const { return levelGroups() + (inputGradients ? 1 : 0); }
+        /** Where the records kernel gets the gradients with respect to the input from: nowhere, the entries of all corners, or what the forward pass kept. */
+        enum InputGradients { NO_INPUT_GRADIENTS = 0, FROM_ENTRIES = 1, FROM_DERIVATIVES = 2 };
+        /** Workgroups of the records kernel over which the levels of a region are shared out, and all that work on a region (as GridGradientRecords::inputGradientsInline). */
+        int levelGroups(InputGradients input) const { return input == FROM_ENTRIES ? 1 : std::min(8, static_cast<int>(slicesPerLevel.size())); }
+        int workgroupsPerRegion(InputGradients input) const
+        {
+            const bool oneLevel = slicesPerLevel.size() == 1;
+            const bool inputsApart = input == FROM_ENTRIES ? oneLevel : input == FROM_DERIVATIVES && !(oneLevel && pairs * recordWords > 16);
+            return levelGroups(input) + (inputsApart ? 1 : 0);
+        }
         /** Regions that the records kernel works on at a time (of a large batch every workgroup gets several). */
         static int regionSlots(long long numel, int points) { return static_cast<int>(std::min<long long>(divUp<long long>(numel, points), 1024)); }
         /**
@@ -195,7 +199,7 @@ public:
                                                             * divUp(workspace.recordsPerRegion, EXCEPTIONS_BLOCK), 1023));
         }
         /** The parts of the temporary memory for regions of so many points, and its bytes. */
-        GradientWorkspace workspace(void* memory, long long numel, int points, size_t* bytes = nullptr) const
+        GradientWorkspace workspace(void* memory, long long numel, int points, InputGradients input, size_t* bytes = nullptr) const
         {
             GradientWorkspace w{};
             size_t offset = 0;
@@ -206,7 +210,7 @@ public:
             };
             w.regions = static_cast<int>(divUp<long long>(numel, points));
             w.recordsPerRegion = points * pairs;
-            w.largestCount = regionSlots(numel, points) * levelGroups();
+            w.largestCount = regionSlots(numel, points) * levelGroups(input);
             const size_t levels = slicesPerLevel.size(), records = static_cast<size_t>(w.regions) * w.recordsPerRegion * levels;
             w.largest = take(static_cast<size_t>(w.largestCount) * sizeof(uint32_t));
             w.places = take(static_cast<size_t>(w.regions) * (numSlices() + 2 * levels) * sizeof(uint16_t));
@@ -226,7 +230,7 @@ public:
             size_t most = roundUp(static_cast<size_t>(numSlices() + 1) * sizeof(int), size_t(256)) + roundUp(records * recordWords * sizeof(uint32_t), size_t(256));
             for (int points = pointsPerWorkgroup; points >= std::min(128, pointsPerWorkgroup); points /= 2) {
                 size_t bytes = 0;
-                (void)workspace(nullptr, numel, points, &bytes);
+                (void)workspace(nullptr, numel, points, NO_INPUT_GRADIENTS, &bytes);   // (of most groups)
                 most = std::max(most, bytes);
             }
             return most;

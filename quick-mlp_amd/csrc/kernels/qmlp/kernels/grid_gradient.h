@@ -17,11 +17,12 @@
 //       and a row of `places` says where those of each slice begin. (Buckets per slice, in which every workgroup reserved room
 //       with an atomic per slice and level: 25 us of atomics, and a batch of unevenly spread points found them full. 16
 //       levels, 2^18 points with input gradients: 124 -> 82 us.) The levels of a region are shared out over several
-//       workgroups, and the grid's share of the gradient with respect to the input
-//       (what EncodingHashGrid::adjoint computes, operation by operation) is left to one workgroup more per region: from the
+//       workgroups. The grid's share of the gradient with respect to the input
+//       (what EncodingHashGrid::adjoint computes, operation by operation) comes from the
 //       entries of all corners, two that lie side by side with one load, or, where the forward
 //       pass kept the derivatives of the features with respect to the position (PositionDerivativeLayout,
-//       INPUT_GRADIENTS == 2), as adjoint x derivative from one or two coalesced loads per level. Bound by the memory that
+//       INPUT_GRADIENTS == 2), as adjoint x derivative from one or two coalesced loads per level; who computes it: see
+//       GridGradientRecords::inputGradientsInline. Bound by the memory that
 //       the records are written to: 268 MB of them for 2^18 points, 3.3 TB/s;
 //   GridGradientSlicesKernel   runs one workgroup per work item (level, slice, part of the
 //       regions): it streams through its records, a segment in every region, and adds weight * adjoint to the slice in LDS,
@@ -390,13 +391,18 @@ struct GridGradientRecords
     static constexpr unsigned EXCEPTION_PAIR_SHIFT = 10, EXCEPTION_UPPER_ONLY = 1u << 13;
     static_assert(POINTS <= 1024 && PAIRS <= 8, "an exception takes 16 bits");
 
+    /** Registers worth holding across the sort of a level's records: 64 bytes of table entries per lane. */
+    static constexpr bool DEFER_ENTRIES = Grid::NC * F * static_cast<int>(sizeof(typename Cfg::table_t)) <= 64;
+
     /**
      * Files the records of the workgroup's points in one level. sCount: zeros on entry and on return, MAX_SLICES + 1 words.
+     * \tparam INPUT_GRADIENTS the level's share of the gradient with respect to the position is added to adjPos
      */
-    template <int LEVEL>
+    template <int LEVEL, int INPUT_GRADIENTS>
     __device__ __forceinline__ static void runLevel(int p, int numel, int region, const float (&position)[D], const Adjoints& adjEncoded,
                                                     const GridGradientWorkspace& ws, unsigned* sStage, int* sCount, int* sStart,
-                                                    unsigned& maxAdjBits)
+                                                    unsigned& maxAdjBits, const param_t& params, const DerivativeChunk* __restrict__ derivatives,
+                                                    float (&adjPos)[D])
     {
         constexpr int NS = Layout::numSlices(LEVEL);
         static_assert(NS <= MAX_SLICES, "the records of a slice are counted in LDS");
@@ -417,7 +423,15 @@ struct GridGradientRecords
         int bucket[PAIRS], rank[PAIRS];
         const typename Grid::LevelSetup s = Grid::setupLevel(LEVEL, pos);
         bool filed = valid;
+        detail::HeldFeatures<F, typename Cfg::table_t> held[Grid::NC];
+        (void)held;
         if (valid) {
+            if constexpr (INPUT_GRADIENTS == 1 && !DEFER_ENTRIES) {
+                // the entries of all corners, for this grid's share of dL/dinput (a dense 4-D grid with 8 features
+                // holds 64 registers: used at once)
+                loadHeld<LEVEL>(s, params, held);
+                positionGradient<LEVEL>(p, s, held, adjEncoded, adjPos);
+            }
             unsigned adjWords[AW];
 #pragma unroll
             for (int i = 0; i < AW; ++i) adjWords[i] = 0u;
@@ -494,6 +508,11 @@ struct GridGradientRecords
         }
         ldsBarrier();
 
+        if constexpr (INPUT_GRADIENTS == 1 && DEFER_ENTRIES) {
+            // The entries of all corners where they take few registers: loaded here and used at the end of the level, so
+            // that the two steps in between hide their latency (the barriers order LDS only).
+            if (valid) loadHeld<LEVEL>(s, params, held);
+        }
         for (int b = tid; b <= NS; b += POINTS) sCount[b] = 0;
         if (filed) {
 #pragma unroll
@@ -508,6 +527,13 @@ struct GridGradientRecords
             unsigned r[RW];
             Layout::loadRecord(sStage + j * RW, r);
             Layout::storeRecord(records + j * RW, r);
+        }
+
+        if constexpr (INPUT_GRADIENTS == 1 && DEFER_ENTRIES) {
+            if (valid) positionGradient<LEVEL>(p, s, held, adjEncoded, adjPos);
+        }
+        if constexpr (INPUT_GRADIENTS == 2) {
+            if (valid) positionGradientFromDerivatives<LEVEL>(p, derivatives, adjEncoded, adjPos);
         }
     }
 
@@ -581,56 +607,89 @@ struct GridGradientRecords
         for (int d = 0; d < D; ++d) adjPos[d] += scale * lvl[d];
     }
 
+    /**
+     * The input gradients that a workgroup computes beside the records that it files (INPUT_GRADIENTS, or 0: left to another
+     * workgroup). The entries of all corners level by level with the records: the wavefronts of the chip then pass through the tables
+     * together, the sort of a level hides the loads, and regions are as small as it takes to fill the chip (adjoint pass of 16 levels of
+     * floats, 2^15 / 2^16 / 2^17 / 2^18 points 89 / 117 / 171 / 313 us; with a workgroup more per region for all of them 177 / 198 / 255 / 475).
+     * One level is left to workgroups of their own (32^4 nodes x 8, 2^18 / 2^19 points 143 / 247 us, within the records kernel 158 / 285), as
+     * are stored derivatives, which are read at the rate of the memory, unless the records take the registers of a second workgroup anyway (64^3 nodes x 4 halves, 2^20 points 152 us
+     * inline and 164 apart; 512^3 cells hashed to 2 halves 139 and 129).
+     */
+    template <int INPUT_GRADIENTS>
+    __device__ __host__ static constexpr int inputGradientsInline()
+    {
+        return INPUT_GRADIENTS == 1 ? (Cfg::Levels > 1 ? 1 : 0) : INPUT_GRADIENTS == 2 ? (Cfg::Levels == 1 && PAIRS * RW > 16 ? 2 : 0) : 0;
+    }
+
     /** Two workgroups of 1024 lanes per compute unit where the records of a lane leave room for it in 64 registers. */
     template <int INPUT_GRADIENTS>
-    __device__ __host__ static constexpr int wavesPerSimd() { return PAIRS * RW <= 16 && INPUT_GRADIENTS != 1 ? 8 : POINTS >= 1024 ? 4 : 1; }
+    __device__ __host__ static constexpr int wavesPerSimd()
+    {
+        return PAIRS * RW <= 16 && INPUT_GRADIENTS != 1 && inputGradientsInline<INPUT_GRADIENTS>() == 0 ? 8 : POINTS >= 1024 ? 4 : 1;
+    }
 
     /** The levels from LEVEL to END - 1. */
-    template <int LEVEL, int END, typename... Args>
+    template <int LEVEL, int END, int INPUT_GRADIENTS, typename... Args>
     __device__ __forceinline__ static void runLevels(Args&&... args)
     {
         if constexpr (LEVEL < END) {
-            runLevel<LEVEL>(args...);
-            runLevels<LEVEL + 1, END>(args...);
+            runLevel<LEVEL, INPUT_GRADIENTS>(args...);
+            runLevels<LEVEL + 1, END, INPUT_GRADIENTS>(args...);
         }
     }
 
     /** The levels of one of GROUPS groups. */
-    template <int G, int GROUPS, typename... Args>
+    template <int G, int GROUPS, int INPUT_GRADIENTS, typename... Args>
     __device__ __forceinline__ static void runGroup(int group, Args&&... args)
     {
         if constexpr (G + 1 < GROUPS) {
-            if (group == G) runLevels<Cfg::Levels * G / GROUPS, Cfg::Levels * (G + 1) / GROUPS>(args...);
-            else runGroup<G + 1, GROUPS>(group, args...);
+            if (group == G) runLevels<Cfg::Levels * G / GROUPS, Cfg::Levels * (G + 1) / GROUPS, INPUT_GRADIENTS>(args...);
+            else runGroup<G + 1, GROUPS, INPUT_GRADIENTS>(group, args...);
         } else {
-            runLevels<Cfg::Levels * G / GROUPS, Cfg::Levels>(args...);
+            runLevels<Cfg::Levels * G / GROUPS, Cfg::Levels, INPUT_GRADIENTS>(args...);
         }
     }
 
-    /** The gradient of a point with respect to its position: from the entries of all corners or from stored derivatives. */
-    template <int LEVEL, int INPUT_GRADIENTS>
-    __device__ __forceinline__ static void positionGradients(int p, const float (&position)[D], const Adjoints& adjEncoded, const param_t& params,
-                                                             const DerivativeChunk* __restrict__ derivatives, float (&adjPos)[D])
+    /** The gradient of a point with respect to its position from stored derivatives. */
+    template <int LEVEL>
+    __device__ __forceinline__ static void positionGradientsFromDerivatives(int p, const Adjoints& adjEncoded,
+                                                                            const DerivativeChunk* __restrict__ derivatives, float (&adjPos)[D])
     {
         if constexpr (LEVEL < Cfg::Levels) {
-            // (the entries of one level in registers at a time; of the derivatives four)
-            float pos[D];
-#pragma unroll
-            for (int d = 0; d < D; ++d) pos[d] = position[d];
-            if (INPUT_GRADIENTS == 1 || LEVEL % 4 == 0) {
+            if (LEVEL % 4 == 0) {   // (those of four levels in registers at a time)
                 asm volatile("" : "+v"(p));
 #pragma unroll
-                for (int d = 0; d < D; ++d) asm volatile("" : "+v"(pos[d]), "+v"(adjPos[d]));
+                for (int d = 0; d < D; ++d) asm volatile("" : "+v"(adjPos[d]));
             }
-            if constexpr (INPUT_GRADIENTS == 2) {
-                positionGradientFromDerivatives<LEVEL>(p, derivatives, adjEncoded, adjPos);
-            } else {
-                const typename Grid::LevelSetup s = Grid::setupLevel(LEVEL, pos);
-                detail::HeldFeatures<F, typename Cfg::table_t> held[Grid::NC];
-                loadHeld<LEVEL>(s, params, held);
-                positionGradient<LEVEL>(p, s, held, adjEncoded, adjPos);
-            }
-            positionGradients<LEVEL + 1, INPUT_GRADIENTS>(p, pos, adjEncoded, params, derivatives, adjPos);
+            positionGradientFromDerivatives<LEVEL>(p, derivatives, adjEncoded, adjPos);
+            positionGradientsFromDerivatives<LEVEL + 1>(p, adjEncoded, derivatives, adjPos);
+        }
+    }
+
+    /** The gradient of a point with respect to its position from the entries of all corners of a grid of one level. */
+    __device__ __forceinline__ static void positionGradientOfOneLevel(int p, const Tensor2Read<float>& inputs, const Adjoints& adjEncoded,
+                                                                      const param_t& params, float (&adjPos)[D])
+    {
+        float pos[D];
+        loadPosition(inputs, p, params, pos);
+        const typename Grid::LevelSetup s = Grid::setupLevel(0, pos);
+        detail::HeldFeatures<F, typename Cfg::table_t> held[Grid::NC];
+        loadHeld<0>(s, params, held);
+        positionGradient<0>(p, s, held, adjEncoded, adjPos);
+    }
+
+    /** Adds adjPos to the gradient with respect to the input of point p, or writes it. */
+    __device__ __forceinline__ static void storeInputGradient(const Tensor2RW<float>& adjInputs, int p, const param_t& params, int overwrite,
+                                                              const float (&adjPos)[D])
+    {
+        // every point belongs to one lane of one workgroup: a plain read-modify-write
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            float* adj = adjInputs.data_ + (static_cast<long long>(p) * adjInputs.strides_[0]
+                                            + static_cast<long long>(d + Cfg::Start) * adjInputs.strides_[1]);
+            const float before = overwrite ? 0.f : *adj;
+            *adj = before + adjPos[d] * params.boundingBoxInvSize[d];
         }
     }
 
@@ -684,10 +743,12 @@ struct GridGradientRecords
 };
 
 /**
- * \tparam GROUPS the levels are shared out over so many workgroups; with INPUT_GRADIENTS another one computes those
+ * \tparam GROUPS the levels are shared out over so many workgroups
+ * \tparam INPUT_GRADIENTS 0: none; 1: from the entries of all corners (of several levels with GROUPS == 1 only); 2: from stored
+ * derivatives; by another workgroup per region, or by those that file the records (GridGradientRecords::inputGradientsInline)
  * \tparam POINTS points (= lanes) of a workgroup; its records of one level are staged in LDS
  * \tparam ROW_CHANNELS, CHANNEL_OFFSET where the adjoints of this grid lie, see GridGradientAdjoints
- * Launched with a multiple of GROUPS (+ 1) workgroups; their number / (GROUPS + 1) * GROUPS is workspace.largestCount.
+ * Launched with a multiple of the workgroups of a region; without those of input gradients they are workspace.largestCount.
  */
 template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS, int POINTS, int INPUT_GRADIENTS, int GROUPS>
 __global__ void __launch_bounds__(POINTS) __attribute__((amdgpu_waves_per_eu(GridGradientRecords<Cfg, ROW_CHANNELS, CHANNEL_OFFSET, SLICE_FLOATS, POINTS>::template wavesPerSimd<INPUT_GRADIENTS>())))
@@ -704,7 +765,8 @@ GridGradientRecordsKernel(
 {
     typedef GridGradientRecords<Cfg, ROW_CHANNELS, CHANNEL_OFFSET, SLICE_FLOATS, POINTS> Impl;
     constexpr int D = Cfg::Dim;
-    constexpr int WORKGROUPS = GROUPS + (INPUT_GRADIENTS != 0 ? 1 : 0);   // of a region
+    constexpr int INLINE = Impl::template inputGradientsInline<INPUT_GRADIENTS>();
+    constexpr int WORKGROUPS = GROUPS + (INPUT_GRADIENTS != INLINE ? 1 : 0);   // of a region
     extern __shared__ __align__(16) unsigned char sMemory[];
     unsigned* sStage = reinterpret_cast<unsigned*>(sMemory);              // POINTS * PAIRS records
     int* sCount = reinterpret_cast<int*>(sStage + POINTS * Impl::PAIRS * Impl::RW);
@@ -719,23 +781,16 @@ GridGradientRecordsKernel(
     // 84 us, 90 and 95 with the groups one behind the other).
     const int step = gridDim.x / WORKGROUPS;
     const int group = Impl::FLOATS ? blockIdx.x / step : blockIdx.x % WORKGROUPS, first = Impl::FLOATS ? blockIdx.x % step : blockIdx.x / WORKGROUPS;
-    if constexpr (INPUT_GRADIENTS != 0) {
+    const auto* derivatives = static_cast<const typename Impl::DerivativeChunk*>(derivativesV);
+    if constexpr (INPUT_GRADIENTS != INLINE) {
         if (group == GROUPS) {
             for (int p = first * POINTS + threadIdx.x; p < numel; p += step * POINTS) {
-                float pos[D], adjPos[D];
-                Impl::loadPosition(inputs, p, params, pos);
+                float adjPos[D];
 #pragma unroll
                 for (int d = 0; d < D; ++d) adjPos[d] = 0.f;
-                Impl::template positionGradients<0, INPUT_GRADIENTS>(p, pos, adjEncoded, params,
-                                                                     static_cast<const typename Impl::DerivativeChunk*>(derivativesV), adjPos);
-                // every point belongs to one lane of one workgroup: a plain read-modify-write
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    float* adj = adjInputs.data_ + (static_cast<long long>(p) * adjInputs.strides_[0]
-                                                    + static_cast<long long>(d + Cfg::Start) * adjInputs.strides_[1]);
-                    const float before = overwriteInput ? 0.f : *adj;
-                    *adj = before + adjPos[d] * params.boundingBoxInvSize[d];
-                }
+                if constexpr (INPUT_GRADIENTS == 2) Impl::template positionGradientsFromDerivatives<0>(p, adjEncoded, derivatives, adjPos);
+                else Impl::positionGradientOfOneLevel(p, inputs, adjEncoded, params, adjPos);
+                Impl::storeInputGradient(adjInputs, p, params, overwriteInput, adjPos);
             }
             return;
         }
@@ -745,11 +800,15 @@ GridGradientRecordsKernel(
     ldsBarrier();
     for (int region = first; region < workspace.regions; region += step) {
         const int p = region * POINTS + threadIdx.x;
-        float pos[D];
+        float pos[D], adjPos[D];
 #pragma unroll
-        for (int d = 0; d < D; ++d) pos[d] = 0.f;
+        for (int d = 0; d < D; ++d) pos[d] = adjPos[d] = 0.f;
         if (p < numel) Impl::loadPosition(inputs, p, params, pos);
-        Impl::template runGroup<0, GROUPS>(group, p, numel, region, pos, adjEncoded, workspace, sStage, sCount, sStart, maxAdjBits);
+        Impl::template runGroup<0, GROUPS, INLINE>(group, p, numel, region, pos, adjEncoded, workspace, sStage, sCount, sStart, maxAdjBits, params,
+                                                   derivatives, adjPos);
+        if constexpr (INLINE != 0) {
+            if (p < numel) Impl::storeInputGradient(adjInputs, p, params, overwriteInput, adjPos);
+        }
     }
     // the largest adjoint of the workgroup
     if (maxAdjBits != 0u) atomicMax(sCount, static_cast<int>(maxAdjBits));

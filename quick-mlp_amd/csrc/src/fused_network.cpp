@@ -1936,6 +1936,15 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
     if (!compileOnly) backwardKernel_[flags][variant][mode] = std::move(ak);
 }
 
+namespace
+{
+IEncoding::GradientSliceLayout::InputGradients inputGradientsFrom(int flags, bool fromDerivatives)
+{
+    typedef IEncoding::GradientSliceLayout Layout;
+    return !(flags & FusedNetwork::GRADIENTS_INPUT) ? Layout::NO_INPUT_GRADIENTS : fromDerivatives ? Layout::FROM_DERIVATIVES : Layout::FROM_ENTRIES;
+}
+}
+
 void FusedNetwork::compileRecordsKernel(SliceGradientKernel& sk, int flags, size_t variant, bool compileOnly, bool fromDerivatives)
 {
     const auto& layout = sk.layout;
@@ -1946,8 +1955,8 @@ void FusedNetwork::compileRecordsKernel(SliceGradientKernel& sk, int flags, size
     ck.fun = QuickMLP::Instance().kernelLoader()->getKernel(
         // (last argument: no input gradients | from gathers of all corners | from the position derivatives of the forward pass)
         format("qmlp::kernel::GridGradientRecordsKernel<%s, %d, %d, %d, %d, %d, %d>", layout.configType.c_str(), layers_[0].channelsIn,
-               sk.channelOffset, layout.sliceFloats, points, !(flags & GRADIENTS_INPUT) ? 0 : fromDerivatives ? 2 : 1,
-               layout.levelGroups()),
+               sk.channelOffset, layout.sliceFloats, points, static_cast<int>(inputGradientsFrom(flags, fromDerivatives)),
+               layout.levelGroups(inputGradientsFrom(flags, fromDerivatives))),
         sk.recordsSource, loaderFlags(compileOnly)).value();
     if (compileOnly) return;
     ck.fullGrid = ck.fun.fullGridSize(ck.blockSize, ck.sharedMemorySize);
@@ -2002,7 +2011,7 @@ const FusedNetwork::CompiledKernel& FusedNetwork::recordsKernelFor(SliceGradient
     // 2^17 points 0.414 / 0.302 / 0.319 / 0.371, 2^16 points 0.290 / 0.233 / 0.215 / 0.244.
     const int computeUnits = KernelFunction::computeUnits();
     size_t variant = 0;
-    const int groups = sk.layout.levelGroups();
+    const int groups = sk.layout.levelGroups(inputGradientsFrom(flags, fromDerivatives));
     while (variant + 1 < sk.records.size() && groups * divUp(numel, sk.layout.pointsPerWorkgroup >> variant) < computeUnits) ++variant;
     auto& kernels = fromDerivatives ? sk.recordsFromDerivatives : sk.records;
     if (!kernels[variant].has_value()) compileRecordsKernel(sk, flags, variant, false, fromDerivatives);
@@ -2745,9 +2754,11 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
                     continue;
                 }
             }
-            const CompiledKernel& rk = recordsKernelFor(sk, adjointFlags, numel, derivativesStored && sk.derivativeOffset >= 0);
+            const bool fromDerivatives = derivativesStored && sk.derivativeOffset >= 0;
+            const CompiledKernel& rk = recordsKernelFor(sk, adjointFlags, numel, fromDerivatives);
             const int points = rk.blockSize;
-            IEncoding::GradientWorkspace regions = layout.workspace(workspace, numel, points);
+            const auto inputFrom = inputGradientsFrom(adjointFlags, fromDerivatives);
+            IEncoding::GradientWorkspace regions = layout.workspace(workspace, numel, points, inputFrom);
             workspace += layout.workspaceBytes(numel64);   // (the layout of the encodings in the memory is that of adjointMemory())
             int overwriteTables = overwrite & GRADIENTS_INPUT_ENCODINGS ? 1 : 0;
             int overwriteInput = overwriteInputGradients && !sortedPoints && encodings_.size() == 1 ? 1 : 0;
@@ -2759,8 +2770,7 @@ void FusedNetwork::adjoint(const Tensor& input, const Tensor& adjOutput, Adjoint
                 const void* derivatives = static_cast<const char*>(tmpMemoryForward)
                     + (static_cast<long long>(perEntryForwardMemoryBytes_) + std::max(0ll, sk.derivativeOffset)) * numel64;
                 void* args[] = {&numel, &inputAcc, &adjEncoded, params.data(), &regions, &overwriteTables, &adjInputAcc, &overwriteInput, &derivatives};
-                rk.fun.launch(layout.workgroupsPerRegion(adjointFlags & GRADIENTS_INPUT) * layout.regionSlots(numel, points), points, rk.sharedMemorySize,
-                              stream, args);
+                rk.fun.launch(layout.workgroupsPerRegion(inputFrom) * layout.regionSlots(numel, points), points, rk.sharedMemorySize, stream, args);
             }
             {
                 float* gradients = nullptr;

@@ -237,7 +237,8 @@ std::optional<KernelFunction> IEncoding::compileRecords(const GradientSliceLayou
     source << "\n" << KernelLoader::MainFile("qmlp/kernels/grid_gradient.h");
     return QuickMLP::Instance().kernelLoader()->getKernel(
         format("qmlp::kernel::GridGradientRecordsKernel<%s, 0, 0, %d, %d, %d, %d>", layout.configType.c_str(), layout.sliceFloats,
-               layout.pointsPerWorkgroup >> variant, inputGradients ? 1 : 0, layout.levelGroups()), source.str(), flags);
+               layout.pointsPerWorkgroup >> variant, inputGradients ? 1 : 0, layout.levelGroups(inputGradients ? GradientSliceLayout::FROM_ENTRIES : GradientSliceLayout::NO_INPUT_GRADIENTS)),
+        source.str(), flags);
 }
 
 std::vector<KernelFunction> IEncoding::compileSlices(const GradientSliceLayout& layout, int flags) const
@@ -259,7 +260,8 @@ void IEncoding::adjointBySlices(const GradientSliceLayout& layout, const Tensor&
     const int flags = QuickMLP::Instance().getCompileFlags();
     int numel = static_cast<int>(input.size(0));
     const bool inputGradients = adjointMode & INPUT_GRADIENTS;
-    const int groups = layout.levelGroups();
+    const auto inputFrom = inputGradients ? GradientSliceLayout::FROM_ENTRIES : GradientSliceLayout::NO_INPUT_GRADIENTS;
+    const int groups = layout.levelGroups(inputFrom);
     // as for the fused networks: as many points per workgroup as keep every compute unit busy
     int variant = 0;
     while (variant + 1 < recordsVariants(layout) && groups * divUp(numel, layout.pointsPerWorkgroup >> variant) < KernelFunction::computeUnits()) ++variant;
@@ -275,7 +277,7 @@ void IEncoding::adjointBySlices(const GradientSliceLayout& layout, const Tensor&
     }
 
     const int points = layout.pointsPerWorkgroup >> variant;
-    GradientWorkspace workspace = layout.workspace(tmpMemory, numel, points);
+    GradientWorkspace workspace = layout.workspace(tmpMemory, numel, points, inputFrom);
     int overwrite = overwriteParameters ? 1 : 0, overwriteInput = 0;
     auto inputAcc = input.accessor<kernel::Tensor2Read<float>>();
     auto adjOutputAcc = adjOutput.accessor<kernel::Tensor2Read<float>>();
@@ -283,7 +285,7 @@ void IEncoding::adjointBySlices(const GradientSliceLayout& layout, const Tensor&
         auto adjInputAcc = adjInput.accessor<kernel::Tensor2RW<float>>();
         const void* derivatives = nullptr;
         void* args[] = {&numel, &inputAcc, &adjOutputAcc, parameters, &workspace, &overwrite, &adjInputAcc, &overwriteInput, &derivatives};
-        variants[variant].value().launch(layout.workgroupsPerRegion(inputGradients) * layout.regionSlots(numel, points), points,
+        variants[variant].value().launch(layout.workgroupsPerRegion(inputFrom) * layout.regionSlots(numel, points), points,
                                          layout.recordsLdsBytes(points), stream, args);
     }
     {

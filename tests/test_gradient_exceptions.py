@@ -17,14 +17,14 @@ from test_overwritten_tables import grid
 pytestmark = pytest.mark.gpu
 
 
-def adjoint_call(enc, x, table, g, mode=2, overwrite=True):
+def adjoint_call(enc, x, table, g, mode=2, overwrite=True, adj_x=None):
     """A function that runs one adjoint pass by slices, and the table gradients that it writes, or adds to."""
     size = ctypes.c_size_t()
     check(lib.qmlp_encoding_adjoint_memory(enc._handle, x.shape[0], mode, ctypes.byref(size)))
     assert size.value > 0
     memory = torch.empty(size.value, dtype=torch.uint8, device="cuda")
     out = torch.full((enc.num_parameters(),), float("nan"), device="cuda")
-    adj_x = torch.zeros_like(x)
+    adj_x = torch.zeros_like(x) if adj_x is None else adj_x
     descs = [desc(x), desc(g), desc(adj_x)]
     stream = current_stream(x.device)
 
