@@ -186,8 +186,15 @@ public:
             const bool inputsApart = input == FROM_ENTRIES ? oneLevel : input == FROM_DERIVATIVES && !(oneLevel && pairs * recordWords > 16);
             return levelGroups(input) + (inputsApart ? 1 : 0);
         }
-        /** Regions that the records kernel works on at a time (of a large batch every workgroup gets several). */
-        static int regionSlots(long long numel, int points) { return static_cast<int>(std::min<long long>(divUp<long long>(numel, points), 1024)); }
+        /**
+         * Regions that the records kernel works on at a time (of a large batch every workgroup gets several): a multiple of the dies,
+         * so that the groups of a region run on the same one (see GridGradientRecordsKernel).
+         */
+        static int regionSlots(long long numel, int points)
+        {
+            constexpr int DIES = 8;
+            return static_cast<int>(roundUp(std::min<long long>(divUp<long long>(numel, points), 1024), static_cast<long long>(DIES)));
+        }
         /**
          * Lanes of a workgroup of GridGradientExceptionsKernel, and workgroups: as many as there are parts of lists, at most what the
          * chip holds, an odd number: lists have a power of two of parts, of which often only the first ones hold anything.

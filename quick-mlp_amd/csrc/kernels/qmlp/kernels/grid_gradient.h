@@ -776,7 +776,8 @@ GridGradientRecordsKernel(
     if (overwrite && blockIdx.x < ZEROING)
         Impl::template zeroShared<0>(blockIdx.x * POINTS + threadIdx.x, min(ZEROING, static_cast<int>(gridDim.x)) * POINTS, params.parametersBackward);
     // Adjoints in rows: a row holds all levels, so that the groups follow one another and every die finds the rows of its
-    // regions in its L2 again (16 levels, 2^17 points: 44 us, 62 with the groups of a region side by side). Adjoints of
+    // regions in its L2 again (16 levels, 2^17 points: 44 us, 62 with the groups of a region side by side), which takes as many
+    // workgroups to a group as is a multiple of the dies (2^17 + 64 points, adjoint pass: 90 us, 115 with 129 workgroups). Adjoints of
     // tiles: nothing is shared, and the slice kernel reads what lies in memory region by region faster (2^18 points: 82 and
     // 84 us, 90 and 95 with the groups one behind the other).
     const int step = gridDim.x / WORKGROUPS;

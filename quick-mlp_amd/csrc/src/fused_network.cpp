@@ -2007,8 +2007,10 @@ const FusedNetwork::CompiledKernel& FusedNetwork::recordsKernelFor(SliceGradient
 {
     // The table entries that a workgroup gathers for the input gradients and the records it writes pass through
     // one compute unit's memory pipeline: a batch that fills fewer workgroups than there are compute units leaves
-    // the rest of the chip idle. Measured on a 16-level hash grid (train step, ms; 1024 / 512 / 256 / 128 points):
-    // 2^17 points 0.414 / 0.302 / 0.319 / 0.371, 2^16 points 0.290 / 0.233 / 0.215 / 0.244.
+    // the rest of the chip idle. Smaller regions than that have shorter segments, which the slice kernel pays for. Adjoint pass
+    // behind 16 levels of halves (us; 1024 / 512 / 256 / 128 points per workgroup), input gradients from entries (one group):
+    // 2^15 points 155 / 109 / 90 / 88, 2^16 158 / 116 / 106 / 109, 2^17 170 / 142 / 142 / 161, 2^18 251 / 257 / 287 / 332; without
+    // input gradients (eight groups): 2^15 51 / 51 / 53 / 55, 2^16 61 / 61 / 67 / 75, 2^18 168 / 176 / 193 / 220.
     const int computeUnits = KernelFunction::computeUnits();
     size_t variant = 0;
     const int groups = sk.layout.levelGroups(inputGradientsFrom(flags, fromDerivatives));
