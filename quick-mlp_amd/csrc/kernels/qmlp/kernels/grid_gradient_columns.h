@@ -221,6 +221,8 @@ struct GridGradientColumns
         }
     }
 
+    template <int N> struct Constant { static constexpr int value = N; };
+
     /**
      * The largest magnitude (bits without the sign) among the adjoints of points [begin, end) that are finite; first: the first
      * of their channels in tile 0. The adjoints of 64 points are F * 128 bytes side by side: a lane takes 8 points of a channel.
@@ -234,18 +236,22 @@ struct GridGradientColumns
         if (begin >= end) return 0u;
         const int firstTile = begin / TILE_POINTS;
         const int chunks = ((end - 1) / TILE_POINTS - firstTile + 1) * CHUNKS;
-        constexpr int AHEAD = 10;   // loads of a lane: all 5120 points of an average run of 2^21 points in 31 x 31 slabs
-#pragma unroll 1
-        for (int i0 = lane; i0 < chunks; i0 += AHEAD * BLOCK) {
+        // GUARDED: without what lies behind the last chunk for a whole wavefront
+        auto scan = [&](int i0, auto ahead, auto guarded) {
+            constexpr int AHEAD = decltype(ahead)::value;
+            constexpr bool GUARDED = decltype(guarded)::value != 0;
+            const int wave0 = __builtin_amdgcn_readfirstlane(i0);
             u32x4 v[AHEAD];
 #pragma unroll
             for (int k = 0; k < AHEAD; ++k) {
+                if (GUARDED && wave0 + k * BLOCK >= chunks) continue;
                 const int i = min(i0 + k * BLOCK, chunks - 1);   // (the last one again)
                 v[k] = *reinterpret_cast<const u32x4*>(first + static_cast<long long>(firstTile + i / CHUNKS) * (ROW_CHANNELS * TILE_POINTS)
                                                        + i % CHUNKS * 8);
             }
 #pragma unroll
             for (int k = 0; k < AHEAD; ++k) {
+                if (GUARDED && wave0 + k * BLOCK >= chunks) continue;
                 const int i = min(i0 + k * BLOCK, chunks - 1);
                 const int p = (firstTile + i / CHUNKS) * TILE_POINTS + i % (TILE_POINTS / 8) * 8;
                 unsigned words[4] = {v[k][0], v[k][1], v[k][2], v[k][3]};
@@ -259,7 +265,16 @@ struct GridGradientColumns
 #pragma unroll
                 for (int j = 0; j < 4; ++j) largest = __builtin_elementwise_max(largest, __builtin_bit_cast(u16x2, words[j] & 0x7fff7fffu));
             }
-        }
+        };
+        // So many loads of a lane at a time while a run has more than half of them for it (2^21 points of 8 features in 31 x 31 slabs: ten on
+        // average; fewer features have fewer, and need the registers for more wavefronts), then up to half, and none for wavefronts that the
+        // run does not reach: the workgroups of 2^20 points in 32 x 32 slabs have one or two (128^3 nodes x 2: the kernel 34 us, 58 with
+        // ten whatever the run).
+        constexpr int MANY = F >= 8 ? 10 : 4;
+        int from = 0;
+#pragma unroll 1
+        for (; chunks - from > MANY / 2 * BLOCK; from += MANY * BLOCK) scan(from + lane, Constant<MANY>{}, Constant<0>{});
+        if (from < chunks) scan(from + lane, Constant<MANY / 2>{}, Constant<1>{});
         return max(static_cast<unsigned>(largest[0]), static_cast<unsigned>(largest[1]));
     }
 
