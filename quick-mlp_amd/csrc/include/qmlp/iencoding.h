@@ -4,6 +4,7 @@
 #include "json.h"
 #include "kernel_loader.h"
 #include "tensor.h"
+#include <qmlp/kernels/grid_gradient_items.h>
 #include <qmlp/kernels/point_order_key.h>
 
 #include <functional>
@@ -199,7 +200,7 @@ public:
          * Lanes of a workgroup of GridGradientExceptionsKernel, and workgroups: as many as there are parts of lists, at most what the
          * chip holds, an odd number: lists have a power of two of parts, of which often only the first ones hold anything.
          */
-        static constexpr int EXCEPTIONS_BLOCK = 256;
+        static constexpr int EXCEPTIONS_BLOCK = kernel::GRID_GRADIENT_EXCEPTIONS_BLOCK;
         int exceptionsGrid(const GradientWorkspace& workspace) const
         {
             return static_cast<int>(std::min<long long>(static_cast<long long>(workspace.regions) * static_cast<long long>(slicesPerLevel.size())

@@ -57,6 +57,7 @@
 
 #include <qmlp/kernels/common.h>
 #include <qmlp/kernels/encoding_hashgrid.h>
+#include <qmlp/kernels/grid_gradient_items.h>
 
 QUICKMLP_KERNEL_NAMESPACE_BEGIN
 
@@ -73,9 +74,6 @@ struct GridGradientSlice
     int place;       // of the slice in a row of GridGradientWorkspace::places
     int slices;      // of the level
 };
-
-/** Every level gets about this many work items of the slice kernel. */
-constexpr int GRID_GRADIENT_ITEMS_PER_LEVEL = 32;
 
 /**
  * The temporary memory of these kernels. A region is what one workgroup of the records kernel files of POINTS
@@ -207,11 +205,8 @@ struct GridGradientLayout
     }
     static constexpr int PLACES = firstPlace(L);
 
-    /** Levels with few slices are summed by several work items each (as encoding_hashgrid.cpp makes them). */
-    __device__ __host__ static constexpr int parts(int l)
-    {
-        return GRID_GRADIENT_ITEMS_PER_LEVEL / numSlices(l) > 1 ? GRID_GRADIENT_ITEMS_PER_LEVEL / numSlices(l) : 1;
-    }
+    /** Levels with few slices are summed by several work items each. */
+    __device__ __host__ static constexpr int parts(int l) { return gridGradientParts(numSlices(l)); }
 };
 
 template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS, int POINTS>
@@ -816,9 +811,6 @@ GridGradientRecordsKernel(
     __syncthreads();
     if (threadIdx.x == 0) workspace.largest[first * GROUPS + group] = static_cast<unsigned>(sCount[0]);
 }
-
-/** Lanes of a workgroup of GridGradientExceptionsKernel. */
-constexpr int GRID_GRADIENT_EXCEPTIONS_BLOCK = 256;
 
 template <typename Cfg, int ROW_CHANNELS, int CHANNEL_OFFSET, int SLICE_FLOATS>
 struct GridGradientExceptions

@@ -362,15 +362,13 @@ bool EncodingHashGrid::gradientSlices(GradientSliceLayout& layout, bool floatAdj
         layout.derivativeBytesPerPoint = chunks <= 2 ? numLevels_ * chunks * 16 : 0;
     }
     if (layout.recordsLdsBytes(points) > lds) return false;
-    // every level gets about this many work items: those of a slice of a coarse level share out the regions
-    constexpr int ITEMS_PER_LEVEL = 32;
     for (int l = 0; l < numLevels_; ++l) {
         const int begin = layers_[l].memoryOffset;
         const int end = l + 1 < numLevels_ ? layers_[l + 1].memoryOffset : numParameters_;
         const int count = divUp(end - begin, layout.sliceFloats);
         if (count > 512) return false;   // the records kernel keeps a histogram of 512 slices
         layout.slicesPerLevel.push_back(count);
-        const int parts = std::max(1, ITEMS_PER_LEVEL / count);
+        const int parts = kernel::gridGradientParts(count);   // those of a slice of a coarse level share out the regions
         // as GridGradientLayout::firstPlace
         const int firstPlace = layout.numSlices() - count + 2 * l;
         for (int k = 0; k < count; ++k)
