@@ -227,15 +227,10 @@ public:
             if (bytes) *bytes = offset;
             return w;
         }
-        /**
-         * Bytes of temporary memory of a batch, whatever the size of its regions. Callers size theirs once and for
-         * long: a quarter more records than the batch has and 2048 per slice, which is more than what lies beside the records takes.
-         */
+        /** Bytes of temporary memory of a batch, whatever the size of its regions and the number of its groups. */
         size_t workspaceBytes(long long numel) const
         {
-            size_t records = 0;
-            for (int slices : slicesPerLevel) records += static_cast<size_t>(slices) * static_cast<size_t>(((5 * numel * pairs / 4) / slices + 2048) & ~3ll);
-            size_t most = roundUp(static_cast<size_t>(numSlices() + 1) * sizeof(int), size_t(256)) + roundUp(records * recordWords * sizeof(uint32_t), size_t(256));
+            size_t most = 0;
             for (int points = pointsPerWorkgroup; points >= std::min(128, pointsPerWorkgroup); points /= 2) {
                 size_t bytes = 0;
                 (void)workspace(nullptr, numel, points, NO_INPUT_GRADIENTS, &bytes);   // (of most groups)

@@ -258,7 +258,11 @@ void launchLevel(KernelIndex kernel, bool wide, int B, int C, int height, int wi
     pullpushKernel<T>(kernel, wide).launch(static_cast<unsigned>(grid), up ? UP_THREADS : BLOCK, 0, stream, args);
 }
 
-// The finest levels that trees take (1 x 4 x 2048 x 2048 floats: step B from 1024 x 1024 on 50 us, from 512 x 512 on 22 + 18; the others alike).
+// The finest levels that trees take, counted from the image. Forward and adjoint of one image of 4 channels of floats, with steps B, A and the
+// way up from level 1 | 2 | 3 on in trees: 512 x 512 117 | 128 | 145 us, 1024 x 1024 164 | 169 | 182, 777 x 1001 247 | 189 | 188, 2048 x 2048
+// 374 | 353 | 357, 4096 x 4096 1250 | 1081 | 1025; 8 images of 3 x 256 x 256 126 | 122 | 121. A large level with a launch of its own is better
+// off (1024 x 1024 pixels, step B 18 us, within a tree 27), a small one costs 5 to 11 us, and odd sizes, whose tiles need borders, suffer
+// most from large trees: level 2 never loses much.
 constexpr int DOWN_TREE_FINEST = 1, UP_TREE_FINEST = 2, GRADIENT_UP_TREE_FINEST = 2, GRADIENT_TREE_FINEST = 2;
 
 constexpr size_t TREE_LDS_BYTES = 72 * 1024;

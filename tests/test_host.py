@@ -190,17 +190,24 @@ def test_temporary_memory_sizes():
             assert net.adjoint_memory(n, 5) == 0
     # From 2^15 points on (a grid of 16 levels; from 2^16 for grids of fewer than 8 levels) the grid gradients are
     # summed slice by slice: the adjoint of the encoded rows
-    # (32 halves per point) joins the adjoint pre-activations, and behind everything else come the
-    # bucket cursors and the records (4 words each; per level, slices x (1.25 x share + 2048) of them:
-    # the table of a level holds 8192 .. 1 048 576 floats, a slice 8192).
+    # (32 halves per point) joins the adjoint pre-activations, and behind everything else comes what the records kernel leaves, for any
+    # size of the regions of a workgroup (1024 to 128 points): the largest adjoint of each of its workgroups (8 groups of levels), 16-bit
+    # places of the slices in a region with two counts per level, the records (4 pairs of corners, 4 words each) and 16 bits for every
+    # record that is an exception instead (the table of a level holds 8192 .. 1 048 576 floats, a slice 8192).
+    up = lambda b: -(-b // 256) * 256
     n = 1 << 18
     floats = [8192, 24334, 71874, 221184, 686000] + [1 << 20] * 11
-    slices_per_level = [-(-f // 8192) for f in floats]
-    records = sum(s * (((5 * n * 4 // 4) // s + 2048) & ~3) for s in slices_per_level)
-    cursors = -(-(sum(slices_per_level) + 1) * 4 // 256) * 256
+    places = sum(-(-f // 8192) for f in floats) + 2 * 16
+
+    def region_bytes(points):
+        regions = -(-n // points)
+        workgroups = 8 * (-(-min(regions, 1024) // 8) * 8)
+        records = regions * points * 4 * 16
+        return up(workgroups * 4) + up(regions * places * 2) + up(records * 16) + up(records * 2)
+    most = max(region_bytes(points) for points in (1024, 512, 256, 128))
     base = 2 * 32 * n + 512 * n_params * 4       # (all weight gradients are summed in the backward kernel)
-    assert net.adjoint_memory(n, 7) == -(-base // 256) * 256 + cursors + -(-records * 16 // 256) * 256
-    assert net.adjoint_memory(n, 4) == 2 * 32 * n + cursors + -(-records * 16 // 256) * 256
+    assert net.adjoint_memory(n, 7) == up(base) + most
+    assert net.adjoint_memory(n, 4) == 2 * 32 * n + most
     assert net.adjoint_memory((1 << 15) - 64, 5) == 0 and net.adjoint_memory(1 << 15, 5) > 0
     few_levels = qmlp.Network(json.dumps(bc.CONFIGS[5]["cfg"]))
     assert few_levels.adjoint_memory((1 << 16) - 64, 4) == 0 and few_levels.adjoint_memory(1 << 16, 4) > 0
