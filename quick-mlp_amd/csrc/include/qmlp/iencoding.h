@@ -290,9 +290,9 @@ public:
      * point grow with the number of levels, the fixed work of the slice kernels with the size of the table: a train
      * step of a network behind a 16-level hash grid of halves at 2^12 / 2^13 / 2^14 / 2^15 points 71 / 86 / 119 / 192 us with
      * atomics, 84 / 76 / 90 / 103 us by slices (with input gradients 99 / 103 / 139 / 234 and 98 / 99 / 97 / 110 us, of which
-     * the host's path is 90: no reason to go below 2^14); the adjoint pass of that grid alone at 2^13 / 2^14 / 2^15 points
-     * 32 / 60 / 117 us with atomics, and by slices, when their records still went to buckets, 46 / 51 / 66 us (with input
-     * gradients 41 / 72 / 152 and 91 / 96 / 112 us).
+     * the host's path is 90: no reason to go below 2^14); the adjoint pass of that grid alone, of floats, at 2^13 / 2^14 / 2^15 / 2^16
+     * points 31 / 60 / 117 / 229 us with atomics and - / 46 / 51 / 61 by slices, with input gradients 43 / 76 / 157 / 279 and
+     * - / 75 / 88 / 118 us.
      * \param manyLevelsMinBatch from which size on grids of 8 levels or more take the slices
      */
     static constexpr int SLICE_GRADIENTS_MIN_BATCH = 1 << 16;

@@ -16,7 +16,7 @@
 //       out as they are: the records of a region and level lie without gaps at a place that is known beforehand,
 //       and a row of `places` says where those of each slice begin. (Buckets per slice, in which every workgroup reserved room
 //       with an atomic per slice and level: 25 us of atomics, and a batch of unevenly spread points found them full. 16
-//       levels, 2^18 points with input gradients: 124 -> 82 us.) The levels of a region are shared out over several
+//       levels, 2^18 points with input gradients from derivatives: 124 -> 82 us.) The levels of a region are shared out over several
 //       workgroups. The grid's share of the gradient with respect to the input
 //       (what EncodingHashGrid::adjoint computes, operation by operation) comes from the
 //       entries of all corners, two that lie side by side with one load, or, where the forward
@@ -28,25 +28,25 @@
 //       regions): it streams through its records, a segment in every region, and adds weight * adjoint to the slice in LDS,
 //       then writes the slice, or adds it to the gradient tensor (with atomics only for a coarse level, whose
 //       few slices receive all records of the level and are shared out over several work items, and for the first entry
-//       of a slice, to which the slice in front adds as well). Bound by the memory that the records come from: without its
-//       LDS additions it takes 76 instead of 79 us (2^18 points; 52 of them are the records, at 5 TB/s, 9 the stores of 50 MB,
-//       and the rest what a work item waits for before its first record). Tensors that hold nothing yet are written: 50 MB that nobody
-//       zeroes first nor reads again (2^18 points: 95 -> 84 us and a fill of 9 us);
-//   GridGradientExceptionsKernel   adds, with atomics, what has no record: the points outside of the box and upper
+//       of a slice, to which the slice in front adds as well). Bound by the memory that the records come from and by its additions in
+//       turn: 2^18 points 76 us (52 of them for the records alone, at 5 TB/s, 9 for the stores of 50 MB); one level of 64^3 nodes x 4
+//       floats, 2^20 points 33 us on half of the compute units, 25 without the additions. Tensors that hold nothing yet are written:
+//       50 MB that nobody zeroes first nor reads again;
+//   GridGradientExceptionsKernel   adds, with atomics, what has no record: the points outside of the box and, in hashed levels, upper
 //       entries in another slice than the one behind the lower one's.
 // The sums in LDS are 64-bit fixed point, added with integer atomics: ds_add_f32 completes one
 // lane every three cycles on this hardware (0.32 lanes per clock and CU measured, whatever the
 // addresses), ds_add_u64 3.5 lanes per clock. The scale is a power of two chosen per launch from the
 // largest adjoint of the batch (which the records kernel finds on its way) and the number of
-// records, such that no sum can overflow: at least 37 bits remain below the largest possible
+// records, such that no sum can overflow: at least 35 bits remain below the largest possible
 // contribution at 2^24 records, and the sums do not depend on the order of the additions. Batches whose
 // adjoints are not finite take the float additions, so that NaN and infinity reach the gradients. Weights
-// are at most one for points inside the box; the records of points outside of it (extrapolated with weights
+// are at most one for points inside the box; the pairs of points outside of it (extrapolated with weights
 // beyond one, or NaN for a NaN coordinate) are exceptions.
 // The adjoint pass of a standalone encoding gives its adjoints in floats. Its records hold floats (GridGradientLayout),
 // the scale of a sum goes by the records of its work item, and a value that would still lose bits in it (floats span
 // more than 64 bits) goes to the gradient tensor with an atomic: 3 of 10^5 in a batch of normally distributed adjoints
-// (16 levels of 2^19 entries of 2 floats, 2^17 points: 458 us with atomics, 44 + 49 us; 2^14 points 61 -> 51 us).
+// (16 levels of 2^19 entries of 2 floats, 2^17 points: 458 us with atomics, 44 + 45 us; 2^14 points 60 -> 46 us).
 // Two forms that were measured and dropped: a workgroup per slice that tests every point of
 // the batch against its slice and recomputes the hits (the work of a hit falls to one lane of
 // 64, 890 us for 2^18 points and 16 levels), and the same with the hits queued in LDS first (the

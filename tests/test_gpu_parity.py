@@ -325,9 +325,8 @@ def test_grid_indices_are_bit_exact(spec):
     along the last coordinate, hashed pairs idx / idx^1) and the lane-group gradient scatter of
     the backward pass (mode 2) -- as sets per point and level, bit for bit, with their weights.
     Mode 3, for grids of up to four dimensions: what the gradient records of large batches stand
-    for (kernels/grid_gradient.h: the slice of the record's bucket plus the two 16-bit offsets
-    as the slice kernel decodes them, and the entries of other slices that the records kernel adds
-    itself). Mode 4, for single dense levels whose batches are sorted by slab: the elements behind the sums
+    for (kernels/grid_gradient.h: the slice that files the record plus the two 16-bit offsets
+    as the slice kernel decodes them, and the entries of other slices that are exceptions). Mode 4, for single dense levels whose batches are sorted by slab: the elements behind the sums
     of the column kernel (kernels/grid_gradient_columns.h: the place in the LDS of the owner of the corner's
     node, and back to the table as the kernel writes its sums)."""
     import json
@@ -538,12 +537,12 @@ def test_grid_gradients_summed_by_slices_match_the_atomic_scatter_and_the_oracle
     sz = np.array([1.0] + grid["bounding_box_size"], np.float32)
     probe = qmlp.Encoding(json.dumps(grid))
     probe.set_parameter(torch.zeros(probe.num_parameters(), device="cuda", dtype=probe.parameter_dtype()))
-    # one round of every slice workgroup; many rounds and a ragged last tile; all points in one small
-    # region (the records of a level then fall into one or two buckets, which overflow: the rest is added
-    # to the gradient tensor by the records kernel itself). The records kernel runs with fewer points per
-    # workgroup for batches that would not give every compute unit a workgroup of the largest size: of the sizes
-    # 1024 / 512 / 256 / 128 these batches take the last, the third and (140001 points) the second.
-    sizes = [(3000, False), (70001, False), (70001, True)] + ([(140001, False)] if d == 3 else [])
+    # A few segments of every slice workgroup; many and a ragged last tile; all points in one small region (all records of a level
+    # lie in the segments of one or two slices). The records kernel runs with fewer points per workgroup for batches that would not
+    # give every compute unit a workgroup of the largest size. Behind 4, 6 or 7 levels, which are shared out over as many workgroups, 3000 /
+    # 16 500 / 35 000 / 70 001 points take 128 / 256 / 512 / 1024 points per workgroup, with stored derivatives as without input gradients; input
+    # gradients from entries have one group: 70 001 points take 256, 140 001 points 512.
+    sizes = [(3000, False), (16500, False), (35000, False), (70001, False), (70001, True)] + ([(140001, False)] if d == 3 else [])
     for N, clustered in sizes:
         u = rng.uniform(-0.05, 1.05, (N, n_in)) if not clustered else 0.37 + 2e-3 * rng.uniform(0, 1, (N, n_in))
         X = (lo + sz * u).astype(np.float32)
@@ -580,8 +579,8 @@ def test_grid_gradients_summed_by_slices_match_the_atomic_scatter_and_the_oracle
                 assert_close(got[1]["adj_x"] / sx, ref["adj_x"] / sx, "input gradients from stored derivatives vs fp32 oracle")
     # Points several box widths outside are extrapolated with weights far above one (the reference does not clamp the
     # fractional position either; 3 widths outside a level of resolution 128: |w| up to 5e7 in 3-D), while the
-    # fixed-point sums of the slice kernel count on weights of at most one: the records kernel adds such records to
-    # the gradient tensor itself. The corners of such a point coincide at the border of the grid, so an entry
+    # fixed-point sums of the slice kernel count on weights of at most one: the exceptions kernel adds such points to
+    # the gradient tensor. The corners of such a point coincide at the border of the grid, so an entry
     # receives huge terms of both signs that cancel to the adjoint itself, and float additions leave rounding noise
     # of the size of |w| x 2^-24 x |adjoint| there in either mode: the entries that these points touch stay at that
     # level, all other entries agree as usual. A NaN coordinate gives NaN weights: the gradients of the entries it

@@ -27,3 +27,20 @@ def test_trees_against_oracle(shape, dtype):
     wm, wd = ppo.pullpush_adjoint(m64, d64, a64)
     np.testing.assert_allclose(gd.cpu().numpy().astype(np.float64), wd, **ADJ_TOL[dtype])
     np.testing.assert_allclose(gm.cpu().numpy().astype(np.float64), wm, **ADJ_TOL[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("shape", [(26, 2, 259, 517), (100, 1, 259, 517), (90, 1, 515, 261), (40, 3, 300, 400)])
+def test_large_tiles_against_small_ones(shape, dtype):
+    """Many images fill the chip with tiles of 32 and 64 pixels, a single one with tiles of 16: the same pixels, of odd sizes and even ones.
+    (Single images against the oracle: above.)"""
+    print("pullpush tiles", shape, dtype, flush=True)
+    mask, data, adj = (gpu(x, dtype) for x in make_case(sum(shape), *shape, dtype))
+    out = pullpush(mask, data)
+    gm, gd = qpp.pullpush_backward(mask, data, adj)
+    for i in (0, 7, shape[0] - 1):
+        one = slice(i, i + 1)
+        torch.testing.assert_close(out[one], pullpush(mask[one].contiguous(), data[one].contiguous()), **FWD_TOL[dtype])
+        om, od = qpp.pullpush_backward(mask[one].contiguous(), data[one].contiguous(), adj[one].contiguous())
+        torch.testing.assert_close(gd[one], od, **ADJ_TOL[dtype])
+        torch.testing.assert_close(gm[one], om, **ADJ_TOL[dtype])
