@@ -1135,7 +1135,9 @@ struct GridGradientSlices
     __device__ __forceinline__ static void forEachPart(int tid, const GridGradientWorkspace& ws, const GridGradientSlice& item, int r0, int count, int log2,
                                                        const Shared& shared, const Add& add)
     {
-        constexpr int LOADS = RARE ? 1 : 2;
+        // (records of a lane under way while as many are added: of wide ones fewer keep the memory busy; dense 4-D grid of 8 features, 40 B,
+        // 2^20 points 349 us for the adjoint pass with one, 368 with two; 4 levels of 16 B, 2^20 points 275 and 266)
+        constexpr int LOADS = RARE || RW > 4 ? 1 : 2;
         const int groups = BLOCK >> log2, lanes = 1 << log2;
         const unsigned* first = ws.records + (static_cast<long long>(item.level) * ws.regions + r0) * ws.recordsPerRegion * RW;
         // this lane is at record `at` of part s, which begins at word `base` (a thousand regions take less than 2^27) and has `size`
