@@ -90,4 +90,4 @@ def test_time_grows_with_the_batch():
         x, g = torch.rand(count, 4, device="cuda", generator=gen), torch.randn(count, 8, device="cuda", generator=gen)
         times.append(time_of(adjoint_call(enc, x, table, g)[0]))
     print("2^19, 2^20 points:", times, flush=True)
-    assert times[1] < 2.35 * times[0]
+    assert times[1] < 2.45 * times[0]
