@@ -16,6 +16,7 @@ typedef _Float16 f16;
 typedef f16 f16x2 __attribute__((ext_vector_type(2)));
 typedef f16 f16x4 __attribute__((ext_vector_type(4)));
 typedef f16 f16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -161,6 +162,22 @@ struct HasPackedAdjoint<Act, decltype(void(Act::adjoint4(f16x4{}, f16x4{})))>
     static constexpr bool value = true;
 };
 
+/**
+ * Detects activations whose adjoint follows from their output, `static f16x4 adjointOfOutput4(f16x4 y, f16x4 adjz, u32x2 mask)`:
+ * y the output for x, mask as for activationAdjointMasked. Kernels that run the layers again keep the output of such a layer
+ * in the place of its pre-activation.
+ */
+template <typename Act, typename = void>
+struct HasAdjointOfOutput
+{
+    static constexpr bool value = false;
+};
+template <typename Act>
+struct HasAdjointOfOutput<Act, decltype(void(Act::adjointOfOutput4(f16x4{}, f16x4{}, u32x2{})))>
+{
+    static constexpr bool value = true;
+};
+
 /** Detects composites with one activation per channel (forwardAt / adjointAt with a channel). */
 template <typename Act, typename = void>
 struct IsPerChannel
@@ -199,6 +216,34 @@ __device__ __forceinline__ f16x4 activationAdjointChannels(f16x4 x, f16x4 adjz, 
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = fromHalf(activationAdjointChannel<Act>(toHalf(x[i]), toHalf(adjz[i]), channel0 + i));
         return o;
+    }
+}
+
+/**
+ * Adjoint of 4 values that belong to the consecutive channels channel0 .. channel0+3 of a point, zero where mask has no bits (16
+ * per value, all or none: points outside of the batch), whatever the activation makes of a zero adjoint.
+ */
+template <typename Act>
+__device__ __forceinline__ f16x4 activationAdjointMasked(f16x4 x, f16x4 adjz, int channel0, u32x2 mask)
+{
+    if constexpr (HasAdjointOfOutput<Act>::value) {
+        return Act::adjointOfOutput4(Act::forward4(x), adjz, mask);
+    } else {
+        return __builtin_bit_cast(f16x4, __builtin_bit_cast(u32x2, activationAdjointChannels<Act>(x, adjz, channel0)) & mask);
+    }
+}
+
+/** The same for 4 points of one channel. */
+template <typename Act>
+__device__ __forceinline__ f16x4 activationAdjointMaskedPoints(f16x4 x, f16x4 adjz, int channel, u32x2 mask)
+{
+    if constexpr (HasAdjointOfOutput<Act>::value) {
+        return Act::adjointOfOutput4(Act::forward4(x), adjz, mask);
+    } else {
+        f16x4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = fromHalf(activationAdjointChannel<Act>(toHalf(x[i]), toHalf(adjz[i]), channel));
+        return __builtin_bit_cast(f16x4, __builtin_bit_cast(u32x2, o) & mask);
     }
 }
 

@@ -232,7 +232,7 @@ struct Layer
      * forward<false> that also hands out the pre-activations, in the layout in which forward<true> stores them and
      * adjoint reads them (lane: channels 16m + 4g + i of the points 4r + nt): the adjoint kernel of a network whose
      * training pass kept the encoded input only runs the layers again (the same operations: the same bits) instead
-     * of reading 2 C_out bytes per point and layer back from memory.
+     * of reading 2 C_out bytes per point and layer back from memory. (pre is the output where the adjoint follows from it.)
      */
     __device__ __forceinline__ static void forwardKeep(const f16* __restrict__ w, const f16* __restrict__ bias,
                                                        const f16x4 (&x)[NT][KT], f16x4 (&pre)[NT][MT], f16x4 (&y)[NT][MT], int lane)
@@ -265,6 +265,7 @@ struct Layer
             for (int nt = 0; nt < NT; ++nt) {
                 pre[nt][m] = toF16(acc[nt]);
                 y[nt][m] = activationForwardChannels<Activation>(pre[nt][m], 16 * m + 4 * g);
+                if constexpr (HasAdjointOfOutput<Activation>::value) pre[nt][m] = y[nt][m];
             }
         }
     }
@@ -287,18 +288,17 @@ struct Layer
                                                    f16* __restrict__ dpreTile, int validMask, int lane)
     {
         const int g = lane >> 4, r = lane & 15;
+        const u32x2 mask = {((validMask & 1) ? 0xffffu : 0u) | ((validMask & 2) ? 0xffff0000u : 0u),
+                            ((validMask & 4) ? 0xffffu : 0u) | ((validMask & 8) ? 0xffff0000u : 0u)};
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const f16x4 pre = *reinterpret_cast<const f16x4*>(preTile + (16 * m + 4 * g + i) * TILE_POINTS + 4 * r);
-                f16x4 d;
+                const f16x4 d = activationAdjointMaskedPoints<Activation>(pre, f16x4{dy[0][m][i], dy[1][m][i], dy[2][m][i], dy[3][m][i]},
+                                                                          16 * m + 4 * g + i, mask);
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    const half a = activationAdjointChannel<Activation>(toHalf(pre[nt]), toHalf(dy[nt][m][i]), 16 * m + 4 * g + i);
-                    d[nt] = ((validMask >> nt) & 1) ? fromHalf(a) : static_cast<f16>(0);
-                    dy[nt][m][i] = d[nt];
-                }
+                for (int nt = 0; nt < NT; ++nt) dy[nt][m][i] = d[nt];
                 if (STORE_DPRE && (!GUARDED || dpreTile != nullptr))
                     *reinterpret_cast<f16x4*>(dpreTile + (16 * m + 4 * g + i) * DPRE_STRIDE + 4 * r) = d;
             }
@@ -326,7 +326,7 @@ struct Layer
     }
 
     /**
-     * adjoint<true, COMPUTE_DX, false, false, T_STRIDE> with the pre-activations in registers (forwardKeep) instead of
+     * adjoint<true, COMPUTE_DX, false, false, T_STRIDE> with what forwardKeep kept in registers instead of pre-activations
      * in memory: the adjoint pre-activations go to the wavefront's LDS tile for weightGradient.
      */
     template <bool COMPUTE_DX>
@@ -337,14 +337,14 @@ struct Layer
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                f16x4 d;
+            for (int nt = 0; nt < NT; ++nt) {
+                const unsigned valid = ((validMask >> nt) & 1) ? ~0u : 0u;
+                if constexpr (HasAdjointOfOutput<Activation>::value) dy[nt][m] = Activation::adjointOfOutput4(pre[nt][m], dy[nt][m], u32x2{valid, valid});
+                else dy[nt][m] = activationAdjointMasked<Activation>(pre[nt][m], dy[nt][m], 16 * m + 4 * g, u32x2{valid, valid});
+            }
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    const half a = activationAdjointChannel<Activation>(toHalf(pre[nt][m][i]), toHalf(dy[nt][m][i]), 16 * m + 4 * g + i);
-                    d[nt] = ((validMask >> nt) & 1) ? fromHalf(a) : static_cast<f16>(0);
-                    dy[nt][m][i] = d[nt];
-                }
+            for (int i = 0; i < 4; ++i) {
+                const f16x4 d = {dy[0][m][i], dy[1][m][i], dy[2][m][i], dy[3][m][i]};
                 *reinterpret_cast<f16x4*>(dpreTile + (16 * m + 4 * g + i) * (TILE_POINTS + 8) + 4 * r) = d;
             }
         }
@@ -402,7 +402,7 @@ struct Layer
      * the registers of a wavefront; replaces network_weight_update_block.cuh:356-494 of the reference).
      * \param sTile T_HALVES halves of LDS of this wavefront: the adjoint pre-activations (zero for points outside the batch)
      * \param inTile CIN rows of IN_STRIDE halves (64 points each): the input of the layer before InputActivation, as
-     *        the forward kernel stored it, or (IN_STRIDE = T_STRIDE) as stageInput put it into LDS
+     *        the forward kernel stored it, or (IN_STRIDE = T_STRIDE) what forwardKeep kept, as stageInput put it into LDS
      */
     template <typename InputActivation, int IN_STRIDE = TILE_POINTS>
     __device__ __forceinline__ static void weightGradient(const f16* sTile, const f16* __restrict__ inTile,
@@ -421,7 +421,9 @@ struct Layer
             for (int k = 0; k < KT; ++k) {
                 const int channel = 16 * k + r;
                 const f16x8 raw = *reinterpret_cast<const f16x8*>(inTile + channel * IN_STRIDE + 32 * kb + 8 * g);
-                b[k] = activationForwardChannel<InputActivation>(raw, channel);
+                // (what forwardKeep kept may be the output itself)
+                if constexpr (IN_STRIDE == T_STRIDE && HasAdjointOfOutput<InputActivation>::value) b[k] = raw;
+                else b[k] = activationForwardChannel<InputActivation>(raw, channel);
             }
 #pragma unroll
             for (int m = 0; m < MT; ++m) {

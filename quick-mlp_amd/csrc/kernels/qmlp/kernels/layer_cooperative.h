@@ -130,43 +130,51 @@ struct CooperativeLayer
         }
     }
 
-    /** The activation of the layer. */
-    __device__ __forceinline__ static void activate(const output_t& pre, output_t& y, int lane)
+    // The activation's adjoint follows from its output: kept (output_t pre) is the output then, else the pre-activation.
+    static constexpr bool KEEPS_OUTPUT = HasAdjointOfOutput<Activation>::value;
+
+    /** The activation of the layer: y, and in pre what the adjoint needs. */
+    __device__ __forceinline__ static void activate(output_t& pre, output_t& y, int lane)
     {
         const int g = lane >> 4;
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int nt = 0; nt < COOP_NT; ++nt) y[nt][m] = activationForwardChannels<Activation>(pre[nt][m], 16 * m + 4 * g);
+            for (int nt = 0; nt < COOP_NT; ++nt) {
+                y[nt][m] = activationForwardChannels<Activation>(pre[nt][m], 16 * m + 4 * g);
+                if constexpr (KEEPS_OUTPUT) pre[nt][m] = y[nt][m];
+            }
     }
 
     /** dy: from the adjoint of the output to that of the pre-activation, into the rows of this wavefront. valid: all bits set for
-     *  a point of the batch; zero: no gradient (whatever the activation makes of a zero adjoint). */
-    __device__ __forceinline__ static void adjointActivation(const output_t& pre, output_t& dy, f16* rows, const unsigned (&valid)[COOP_NT], int lane)
+     *  a point of the batch; zero: no gradient (whatever the activation makes of a zero adjoint). kept: pre after activate. */
+    __device__ __forceinline__ static void adjointActivation(const output_t& kept, output_t& dy, f16* rows, const unsigned (&valid)[COOP_NT], int lane)
     {
         const int g = lane >> 4, r = lane & 15;
 #pragma unroll
         for (int nt = 0; nt < COOP_NT; ++nt)
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
-                typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-                const f16x4 d = activationAdjointChannels<Activation>(pre[nt][m], dy[nt][m], 16 * m + 4 * g);
-                dy[nt][m] = __builtin_bit_cast(f16x4, __builtin_bit_cast(u32x2, d) & u32x2{valid[nt], valid[nt]});
+                const u32x2 mask = {valid[nt], valid[nt]};
+                if constexpr (KEEPS_OUTPUT) dy[nt][m] = Activation::adjointOfOutput4(kept[nt][m], dy[nt][m], mask);
+                else dy[nt][m] = activationAdjointMasked<Activation>(kept[nt][m], dy[nt][m], 16 * m + 4 * g, mask);
                 *reinterpret_cast<f16x4*>(rows + (16 * nt + r) * D_STRIDE + 16 * m + 4 * g) = dy[nt][m];
             }
     }
 
-    /** The input of the layer, InputActivation applied, into the rows of this wavefront. */
+    /** The input of the layer, from what the layer of InputActivation in front kept, into the rows of this wavefront. */
     template <typename InputActivation>
-    __device__ __forceinline__ static void stageInput(const input_t& x, f16* rows, int lane)
+    __device__ __forceinline__ static void stageInput(const input_t& kept, f16* rows, int lane)
     {
         const int g = lane >> 4, r = lane & 15;
 #pragma unroll
         for (int t = 0; t < KT; ++t) {
 #pragma unroll
-            for (int nt = 0; nt < COOP_NT; ++nt)
-                *reinterpret_cast<f16x4*>(rows + X_OFFSET + (16 * nt + r) * X_STRIDE + 16 * t + 4 * g)
-                    = activationForwardChannels<InputActivation>(x[nt][t], 16 * t + 4 * g);
+            for (int nt = 0; nt < COOP_NT; ++nt) {
+                f16x4 x = kept[nt][t];
+                if constexpr (!HasAdjointOfOutput<InputActivation>::value) x = activationForwardChannels<InputActivation>(x, 16 * t + 4 * g);
+                *reinterpret_cast<f16x4*>(rows + X_OFFSET + (16 * nt + r) * X_STRIDE + 16 * t + 4 * g) = x;
+            }
         }
     }
 

@@ -36,13 +36,25 @@ static std::string packedForward(const std::string& forward)
 static std::string packedAdjoint(const std::string& adjoint)
 {
     const std::string a = withoutSpaces(adjoint);
-    if (a == "adjx=__hgt(x,hZERO())?adjz:hZERO()")
-        // ReLU: one where x is positive (as integers: neither NaN, which the maximum removed, nor -0), times the bits of adjz
-        return "        typedef short s16x4 __attribute__((ext_vector_type(4)));\n"
-               "        const s16x4 p = __builtin_bit_cast(s16x4, __builtin_elementwise_max(x, f16x4{0, 0, 0, 0}));\n"
-               "        const s16x4 one = __builtin_elementwise_min(__builtin_elementwise_max(p, s16x4{0, 0, 0, 0}), s16x4{1, 1, 1, 1});\n"
-               "        return __builtin_bit_cast(f16x4, __builtin_bit_cast(s16x4, adjz) * one);\n";
     if (a == "adjx=adjz") return "        return adjz;\n";
+    return "";
+}
+
+/** Members for snippets whose adjoint follows from the output (HasAdjointOfOutput in kernels/common.h). */
+static std::string adjointOfOutput(const std::string& forward, const std::string& adjoint)
+{
+    if (withoutSpaces(forward) == "z=__hgt(x,hZERO())?x:hZERO()" && withoutSpaces(adjoint) == "adjx=__hgt(x,hZERO())?adjz:hZERO()")
+        // ReLU: y = v_pk_max_f16(x, 0) is neither NaN nor -0, as an integer its minimum with one is one where x is positive (with
+        // the mask's zero: zero), times the bits of adjz. Two packed instructions for two values; the empty statements keep
+        // the compiler from seeing comparisons in them, of which it makes three instructions for each value.
+        return "    static __device__ __forceinline__ f16x4 adjointOfOutput4(f16x4 y, f16x4 adjz, u32x2 mask) {\n"
+               "        typedef short s16x4 __attribute__((ext_vector_type(4)));\n"
+               "        s16x4 p = __builtin_bit_cast(s16x4, y);\n"
+               "        asm(\"\" : \"+v\"(p));\n"
+               "        s16x4 one = __builtin_elementwise_min(p, __builtin_bit_cast(s16x4, mask & u32x2{0x00010001u, 0x00010001u}));\n"
+               "        asm(\"\" : \"+v\"(one));\n"
+               "        return __builtin_bit_cast(f16x4, __builtin_bit_cast(s16x4, adjz) * one);\n"
+               "    }\n";
     return "";
 }
 
@@ -73,6 +85,7 @@ struct %s
     const std::string packedAdj = packedAdjoint(adjoint);
     if (!packedAdj.empty())
         packed += "    static __device__ __forceinline__ f16x4 adjoint4(f16x4 x, f16x4 adjz) {\n" + packedAdj + "    }\n";
+    packed += adjointOfOutput(forward, adjoint);
     return format(TEMPLATE, id.c_str(), forward.c_str(), adjoint.c_str(), packed.c_str());
 }
 

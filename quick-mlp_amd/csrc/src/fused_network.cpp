@@ -1373,7 +1373,8 @@ std::string FusedNetwork::cooperativeBackwardSource(int flags, bool sliceGradien
         call << "        Layer" << i << "::output_t pre" << i << ";\n        Layer" << i << "::forward(sParams + " << ldsW[i] << ", "
              << (l.useBias ? "sParams + " + std::to_string(ldsB[i]) : std::string("nullptr")) << ", " << (i == 0 ? std::string("x0") : "act" + std::to_string(i))
              << ", pre" << i << ", " << lane << ");\n";
-        if (i + 1 < L) call << "        Layer" << i << "::output_t act" << (i + 1) << ";\n        Layer" << i << "::activate(pre" << i << ", act" << (i + 1) << ", lane);\n";
+        call << "        Layer" << i << "::output_t act" << (i + 1) << ";\n        Layer" << i << "::activate(pre" << i << ", act" << (i + 1) << ", lane);\n";
+        if (i + 1 == L) call << "        (void)act" << L << ";\n";
         store << "    Layer" << i << "::storeWeightGradient(sums" << i << ", reinterpret_cast<float*>(sMemory),\n        partialGradients + (static_cast<long long>(blockIdx.x) * NUM_PARAMETERS + "
               << l.weightsStart << "), partialGradients + (static_cast<long long>(blockIdx.x) * NUM_PARAMETERS + " << (l.useBias ? l.biasStart : 0)
               << "), partialSlices, NUM_PARAMETERS, wave, lane);\n";
