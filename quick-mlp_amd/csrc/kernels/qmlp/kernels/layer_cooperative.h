@@ -203,23 +203,20 @@ struct CooperativeLayer
         }
     }
 
-    /** Gradient tiles of this wavefront; column m of the bias tile holds the sums of its m-th tile of output channels. */
+    /** Gradient tiles of this wavefront. */
     struct Sums
     {
         f32x4 w[MO][KI];
-        f32x4 b;
-        __device__ __forceinline__ void zero()
-        {
-            zeroTiles(w);
-            b = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
+        __device__ __forceinline__ void zero() { zeroTiles(w); }
     };
 
     /**
      * Adds the points of all wavefronts to the tiles of this one. rows: the rows of wavefront 0, those of wavefront i
-     * start i * rowsPerWave halves further.
+     * start i * rowsPerWave halves further. bias: tiles that all layers share, column FIRST_COLUMN + m (16 to a tile) holds the
+     * sums of this wavefront's m-th tile of output channels.
      */
-    __device__ __forceinline__ static void weightGradient(const f16* rows, int rowsPerWave, Sums& sums, int wave, int lane)
+    template <int FIRST_COLUMN, int BIAS_TILES>
+    __device__ __forceinline__ static void weightGradient(const f16* rows, int rowsPerWave, Sums& sums, f32x4 (&bias)[BIAS_TILES], int wave, int lane)
     {
         const int g = lane >> 4, i = lane & 15;
         const int wm = wave % Share::M, wk = (wave / Share::M) % Share::K, wp = wave / (Share::M * Share::K);
@@ -243,7 +240,8 @@ struct CooperativeLayer
 #pragma unroll
                 for (int k = 0; k < KI; ++k) sums.w[m][k] = mfma32(a, b[k], sums.w[m][k]);
                 if constexpr (BIAS) {
-                    if (wk == 0) sums.b = mfma32(a, i == m ? ones : zeros, sums.b);
+                    f32x4& tile = bias[(FIRST_COLUMN + m) / 16];
+                    if (wk == 0) tile = mfma32(a, i == (FIRST_COLUMN + m) % 16 ? ones : zeros, tile);
                 }
             }
         }
@@ -253,7 +251,8 @@ struct CooperativeLayer
      * After the last tile: the workgroup's sums into slice blockIdx.x of the partial gradients, slices beyond the grid
      * zeroed (as Layer::storeWeightGradient). sAcc: (MT * KT * 256 + COUT) floats. All threads call this.
      */
-    __device__ __forceinline__ static void storeWeightGradient(const Sums& sums, float* sAcc, float* __restrict__ partialWeights,
+    template <int FIRST_COLUMN, int BIAS_TILES>
+    __device__ __forceinline__ static void storeWeightGradient(const Sums& sums, const f32x4 (&bias)[BIAS_TILES], float* sAcc, float* __restrict__ partialWeights,
                                                                float* __restrict__ partialBias, int numSlices, int sliceStride, int wave, int lane)
     {
         const int g = lane >> 4, r = lane & 15;
@@ -274,11 +273,14 @@ struct CooperativeLayer
                     }
                 }
             if constexpr (BIAS) {
-                if (wk == 0 && r < MO && wm * MO + r < MT) {
+#pragma unroll
+                for (int m = 0; m < MO; ++m) {
+                    if (wk != 0 || r != (FIRST_COLUMN + m) % 16 || wm * MO + m >= MT) continue;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        float* target = sBias + 16 * (wm * MO + r) + 4 * g + i;
-                        *target = p == 0 ? sums.b[i] : *target + sums.b[i];
+                        const float sum = bias[(FIRST_COLUMN + m) / 16][i];
+                        float* target = sBias + 16 * (wm * MO + m) + 4 * g + i;
+                        *target = p == 0 ? sum : *target + sum;
                     }
                 }
             }

@@ -8,9 +8,12 @@
 // (layer_cooperative.h), two workgroup barriers per layer. For the adjoint of the encoded input: the input gradients
 // of identity encodings are added here, those of grids are left to the kernels behind this one.
 //
-// 64 -> 64 x 4 -> 4, 10^6 points: 139 us, 541 vector and 144 matrix instructions per 32 points and SIMD of 4 and 16 cycles, which
-// hardly overlap on a SIMD (152 us with 957: the adjoint of ReLU as comparisons, and its output computed three times).
-// 4 -> 128 -> 64 -> 48 -> 4 with sines, 2^20 points: 300 us, 43 % and 14 %; its 232 bytes of spills are 240 of the 310 MB it moves.
+// 64 -> 64 x 4 -> 4, 10^6 points: 125 us, 541 vector and 144 matrix instructions per 32 points of 4 and 16 cycles, which hardly
+// overlap on a SIMD (half of the time), while the LDS is busy for 0.6 of it (152 us with 957 vector instructions: the adjoint of
+// ReLU as comparisons, and its output computed three times). 4 -> 128 -> 64 -> 48 -> 4 with sines, 2^20 points: 225 us, vector
+// instructions 0.57 and matrix instructions 0.2 of the time (300 us while it spilled 232 bytes per lane). Slower or the same:
+// one wavefront per SIMD with all gradient tiles and no barriers (+25 %), or with 64 points (+20 %); fewer vector
+// instructions (outputs of the sines kept, masks left out of full tiles: nothing, at 100 bytes of spills the first).
 //
 // Replaces, like network_backward.h, NetworkKernelBackward of the reference
 // (src_cpp/include/qmlp/kernels/network_backward.cuh:33-114) and its weight update
