@@ -8,12 +8,13 @@
 // (layer_cooperative.h), two workgroup barriers per layer. For the adjoint of the encoded input: the input gradients
 // of identity encodings are added here, those of grids are left to the kernels behind this one.
 //
-// 64 -> 64 x 4 -> 4, 10^6 points: 125 us, 541 vector and 144 matrix instructions per 32 points of 4 and 16 cycles, which hardly
-// overlap on a SIMD (half of the time), while the LDS is busy for 0.6 of it (152 us with 957 vector instructions: the adjoint of
-// ReLU as comparisons, and its output computed three times). 4 -> 128 -> 64 -> 48 -> 4 with sines, 2^20 points: 225 us, vector
-// instructions 0.57 and matrix instructions 0.2 of the time (300 us while it spilled 232 bytes per lane). Slower or the same:
-// one wavefront per SIMD with all gradient tiles and no barriers (+25 %), or with 64 points (+20 %); fewer vector
-// instructions (outputs of the sines kept, masks left out of full tiles: nothing, at 100 bytes of spills the first).
+// 64 -> 64 x 4 -> 4, 10^6 points: 110 us, 541 vector and 144 matrix instructions per 32 points of 4 and 16 cycles, which hardly
+// overlap on a SIMD, while the LDS is busy for 0.6 of the time (152 us with 957 vector instructions, the adjoint of ReLU as
+// comparisons and its output computed three times; 125 with the rows of a tile waited for one after the other). 4 -> 128 -> 64
+// -> 48 -> 4 with sines, 2^20 points: 210 us, vector instructions 0.6 and matrix instructions 0.2 of the time (300 us while it spilled
+// 232 bytes per lane, 225 with the rows waited for). Slower or the same: one wavefront per SIMD with all gradient tiles
+// and no barriers (+25 %), or with 64 points (+20 %); fewer vector instructions (outputs of the sines kept or the first layer's pre-activations
+// formed again by matrix instructions, masks left out of full tiles: 0 to 2 %); other paddings of the rows; other orders between the barriers.
 //
 // Replaces, like network_backward.h, NetworkKernelBackward of the reference
 // (src_cpp/include/qmlp/kernels/network_backward.cuh:33-114) and its weight update
@@ -90,10 +91,91 @@ $$DECLARE_WEIGHT_GRADIENTS$$
     const int actualChannelsOut = adjOutputs.sizes_[1];
     const bool adjOutputRowsOfFloat4 = actualChannelsOut % 4 == 0 && adjOutputs.strides_[1] == 1 && adjOutputs.strides_[0] % 4 == 0
         && reinterpret_cast<unsigned long long>(adjOutputs.data_) % 16 == 0;
-    const bool inputRowsOfFloat4 = DIRECT_INPUT && DIRECT_INPUT_START % 4 == 0 && inputs.strides_[1] == 1 && inputs.strides_[0] % 4 == 0
-        && reinterpret_cast<unsigned long long>(inputs.data_) % 16 == 0;
+    const bool inputRowsOfFloat4 = DIRECT_INPUT && DIRECT_INPUT_START % 4 == 0 && ENCODED_CHANNELS % 4 == 0 && inputs.strides_[1] == 1
+        && inputs.strides_[0] % 4 == 0 && reinterpret_cast<unsigned long long>(inputs.data_) % 16 == 0;
     (void)inputRowsOfFloat4;
     const int numGroups = (numel + WAVES * COOP_POINTS - 1) / (WAVES * COOP_POINTS);
+
+    // What a wavefront reads of its 32 points: dL/dy and the input rows, or the encoded input as the forward kernel stored it
+    // (channel-major tiles of 64 points, zero outside the batch). Asked for a group of tiles ahead, and without a branch
+    // around any load but what is the same for the whole launch: behind branches for lanes every load was waited for
+    // before the next was asked for, six times the latency of the memory per tile. Lanes without a point or
+    // a channel read another one's, which takeRows leaves out.
+    f32x4 dyAhead[COOP_NT][MTL];
+    f32x4 inputAhead[DIRECT_INPUT ? COOP_NT : 1][DIRECT_INPUT ? KT0 : 1];
+    f16x2 encodedAhead[DIRECT_INPUT ? 1 : KT0][4];
+    (void)inputAhead; (void)encodedAhead;
+    auto loadRows = [&](int group) {
+        const int ahead = (group < numGroups ? group : numGroups - 1) * WAVES + wave;
+        int point[COOP_NT];
+#pragma unroll
+        for (int nt = 0; nt < COOP_NT; ++nt) point[nt] = min(ahead * COOP_POINTS + 2 * r + nt, numel - 1);
+        auto loadAdjoints = [&](const int (&rows)[COOP_NT]) {
+            if (adjOutputRowsOfFloat4) {
+#pragma unroll
+                for (int nt = 0; nt < COOP_NT; ++nt)
+#pragma unroll
+                    for (int m = 0; m < MTL; ++m)
+                        dyAhead[nt][m] = *reinterpret_cast<const f32x4*>(adjOutputs.data_ + static_cast<long long>(rows[nt]) * adjOutputs.strides_[0]
+                                                                         + min(16 * m + 4 * g, actualChannelsOut - 4));
+            } else {
+#pragma unroll
+                for (int nt = 0; nt < COOP_NT; ++nt)
+#pragma unroll
+                    for (int m = 0; m < MTL; ++m)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            dyAhead[nt][m][i] = adjOutputs.data_[static_cast<long long>(rows[nt]) * adjOutputs.strides_[0]
+                                                                 + static_cast<long long>(min(16 * m + 4 * g + i, actualChannelsOut - 1)) * adjOutputs.strides_[1]];
+            }
+        };
+        // (twice, and the order waited for at once: merged, the way without an order would wait wherever the other one might have to)
+        if (adjOutputOrder) {
+            int rows[COOP_NT];
+#pragma unroll
+            for (int nt = 0; nt < COOP_NT; ++nt) rows[nt] = adjOutputOrder[point[nt]];
+#pragma unroll
+            for (int nt = 0; nt < COOP_NT; ++nt) asm volatile("" : "+v"(rows[nt]));
+            loadAdjoints(rows);
+        } else {
+            loadAdjoints(point);
+        }
+        if constexpr (DIRECT_INPUT) {
+            if (inputRowsOfFloat4) {
+#pragma unroll
+                for (int nt = 0; nt < COOP_NT; ++nt)
+#pragma unroll
+                    for (int t = 0; t < KT0; ++t)
+                        inputAhead[nt][t] = *reinterpret_cast<const f32x4*>(inputs.data_ + static_cast<long long>(point[nt]) * inputs.strides_[0] + DIRECT_INPUT_START
+                                                                            + min(16 * t + 4 * g, ENCODED_CHANNELS - 4));
+            } else {
+#pragma unroll
+                for (int nt = 0; nt < COOP_NT; ++nt)
+#pragma unroll
+                    for (int t = 0; t < KT0; ++t)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            inputAhead[nt][t][i] = inputs.data_[static_cast<long long>(point[nt]) * inputs.strides_[0]
+                                                                + static_cast<long long>(DIRECT_INPUT_START + min(16 * t + 4 * g + i, ENCODED_CHANNELS - 1)) * inputs.strides_[1]];
+            }
+        } else {
+            const int tileAhead = ahead >> 1;
+            const f16* encTile = forwardTmpMemory + static_cast<long long>(tileAhead < numTiles ? tileAhead : numTiles - 1) * (CHANNELS_IN * TILE_POINTS)
+                + (ahead & 1) * COOP_POINTS + 2 * r;
+#pragma unroll
+            for (int t = 0; t < KT0; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) encodedAhead[t][i] = *reinterpret_cast<const f16x2*>(encTile + (16 * t + 4 * g + i) * TILE_POINTS);
+        }
+    };
+    // (fp32 -> fp16, zero outside batch / real channels)
+    auto takeChannels = [&](f32x4 v, bool pv, int c, int channels) {
+        f16x4 out = toF16(v);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[i] = pv && c + i < channels ? out[i] : static_cast<f16>(0);
+        return out;
+    };
+    loadRows(blockIdx.x);
     for (int group = blockIdx.x; group < numGroups; group += gridDim.x)
     {
         const int half32 = group * WAVES + wave;               // this wavefront's 32 points
@@ -104,54 +186,22 @@ $$DECLARE_WEIGHT_GRADIENTS$$
         f16x4 x0[COOP_NT][KT0];
 #pragma unroll
         for (int nt = 0; nt < COOP_NT; ++nt) {
-            const int p = point0 + nt;
-            const bool pv = p < numel;
+            const bool pv = point0 + nt < numel;
             valid[nt] = pv ? ~0u : 0u;
-            // dL/dy -> accumulator layout (fp32 -> fp16), zero outside batch / real channels
-            const long long adjRow = pv ? (adjOutputOrder ? adjOutputOrder[p] : p) : 0;
-            const float* row = adjOutputs.data_ + adjRow * adjOutputs.strides_[0];
 #pragma unroll
-            for (int m = 0; m < MTL; ++m) {
-                const int c = 16 * m + 4 * g;
-                f32x4 v = {0.f, 0.f, 0.f, 0.f};
-                if (adjOutputRowsOfFloat4) {
-                    if (pv && c < actualChannelsOut) v = *reinterpret_cast<const f32x4*>(row + c);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (pv && c + i < actualChannelsOut) v[i] = row[static_cast<long long>(c + i) * adjOutputs.strides_[1]];
-                }
-                dyOut[nt][m] = toF16(v);
-            }
+            for (int m = 0; m < MTL; ++m) dyOut[nt][m] = takeChannels(dyAhead[nt][m], pv, 16 * m + 4 * g, actualChannelsOut);
             if constexpr (DIRECT_INPUT) {
-                const float* in = inputs.data_ + static_cast<long long>(pv ? p : 0) * inputs.strides_[0]
-                    + static_cast<long long>(DIRECT_INPUT_START) * inputs.strides_[1];
 #pragma unroll
-                for (int t = 0; t < KT0; ++t) {
-                    const int c = 16 * t + 4 * g;
-                    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-                    if (16 * t + 15 < ENCODED_CHANNELS && inputRowsOfFloat4) {
-                        if (pv) v = *reinterpret_cast<const f32x4*>(in + c);
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            if (pv && c + i < ENCODED_CHANNELS) v[i] = in[static_cast<long long>(c + i) * inputs.strides_[1]];
-                    }
-                    x0[nt][t] = toF16(v);
-                }
+                for (int t = 0; t < KT0; ++t) x0[nt][t] = takeChannels(inputAhead[nt][t], pv, 16 * t + 4 * g, ENCODED_CHANNELS);
             }
         }
         if constexpr (!DIRECT_INPUT) {
-            // as the forward kernel stored it: channel-major tiles of 64 points, zero outside the batch
-            const f16* encTile = forwardTmpMemory + static_cast<long long>(tile < numTiles ? tile : numTiles - 1) * (CHANNELS_IN * TILE_POINTS)
-                + (half32 & 1) * COOP_POINTS + 2 * r;
 #pragma unroll
             for (int t = 0; t < KT0; ++t)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const f16x2 v = *reinterpret_cast<const f16x2*>(encTile + (16 * t + 4 * g + i) * TILE_POINTS);
-                    x0[0][t][i] = v[0];
-                    x0[1][t][i] = v[1];
+                    x0[0][t][i] = encodedAhead[t][i][0];
+                    x0[1][t][i] = encodedAhead[t][i][1];
                 }
         }
 

@@ -381,10 +381,12 @@ int FusedNetwork::cooperativeRegisters(int waves, int registerWeight) const
 
 int FusedNetwork::cooperativeSlices(int numTiles) const
 {
-    // One per workgroup: two of them per compute unit, up to four where a lane holds so little that more wavefronts find room.
+    // One per workgroup: two of them per compute unit, up to four where a lane holds so little that more wavefronts find room
+    // (16 -> 64 x 2 -> 4, 10^6 points, forward and backward: 88 us with three, 95 with two).
     const CooperativeLayout& layout = cooperativeLayout();
     const int waves = layout.blockSize / WARP_SIZE;
-    const int perComputeUnit = cooperativeRegisters(waves, layout.registerWeight) <= 100 ? 4 : 2;
+    const int registers = cooperativeRegisters(waves, layout.registerWeight);
+    const int perComputeUnit = registers <= 100 ? 4 : registers <= 120 ? 3 : 2;
     return std::max(1, std::min(divUp(2 * numTiles, waves), perComputeUnit * (MAX_WEIGHT_UPDATE_SLICES / 2)));
 }
 
@@ -1396,6 +1398,8 @@ std::string FusedNetwork::cooperativeBackwardSource(int flags, bool sliceGradien
                  << ">(pre" << (i - 1) << ", sRows, " << lane << ");\n";
         else
             call << "        Layer0::template stageInput<activations::passthrough_>(x0, sRows, " << lane << ");\n";
+        // (where the registers of the layers behind are free again)
+        if (i == 0) call << "        loadRows(group + gridDim.x);\n";
         call << "        workgroupLdsBarrier();\n        Layer" << i << "::template weightGradient<BIAS_COLUMN" << i << ">(sRowsAll, ROWS_PER_WAVE, sums" << i << ", biasSums, wave, "
              << lane << ");\n        workgroupLdsBarrier();\n        Layer" << i << "::input_t dx" << i << ";\n";
         // (behind the barrier: while the gradient tiles are formed the adjoint of the output is held, not the wider one of an input,
@@ -1767,9 +1771,11 @@ void FusedNetwork::compileBackwardKernel(int flags, bool sliceGradients, bool co
         ak.outputOrder = true;
         ak.fusedLayers.assign(layers_.size(), true);
         ak.fusedWeightUpdate = true;
-        // a kernel of many registers like those below: left to the offline compiler where there is one
+        // A kernel of many registers like those below: left to the offline compiler where there is one, whose scheduler then does not
+        // move LDS accesses together (64 x 4 hidden layers 159 -> 156 us, 4 -> 128 -> 64 -> 48 -> 4 299 -> 292, forward and backward).
         const int offlineFlags = loaderFlags(compileOnly) | KernelLoader::CompileOffline;
-        ak.adjoint.fun = kl->getKernel("qmlp::kernel::NetworkKernelBackwardCooperative", cooperativeBackwardSource(flags, sliceGradients), offlineFlags).value();
+        ak.adjoint.fun = kl->getKernel("qmlp::kernel::NetworkKernelBackwardCooperative", cooperativeBackwardSource(flags, sliceGradients), offlineFlags,
+                                       {"-mllvm", "-misched-cluster=0"}).value();
     } else {
     ak.adjoint.blockSize = forwardBlockSize(compileOptions_.overwriteBlocksizeBackward, true);
     {
