@@ -152,57 +152,65 @@ $$ZERO_LDS_GRADIENTS$$
     // Kernels that run the layers again read little per tile: dL/dy and the encoded input of this wavefront's next tile
     // are asked for one tile ahead, behind the order of a sorted batch (the row of dL/dy) that is asked for two ahead. A
     // wavefront's tiles follow each other with nothing else to hide the latency of three dependent loads (12 -> 16 -> 32 x 3
-    // -> 2 with a grid, 2^21 points: 154 -> 131 us).
+    // -> 2 with a grid, 2^21 points: 154 -> 92 us; 112 while the rows of a tile were waited for one after the other).
     constexpr bool LOADS_AHEAD = $$RECOMPUTES$$ && MTL == 1 && KT0 <= 2 && !HAS_STREAMED_LAYERS;
     const int firstTile = static_cast<int>(blockIdx.x) * WAVES + wave, tileStep = static_cast<int>(gridDim.x) * WAVES;
     (void)firstTile; (void)tileStep;
+    // No branch around a load but what is the same for the whole launch: behind branches for lanes every load was waited for before the next
+    // was asked for. Lanes without a point or a channel read another one's, which is left out below.
 #if $$HAS_OUTPUT_ORDER$$
     // a batch that trains in sorted order: the rows of dL/dy of this wavefront's next tile, asked for one tile ahead
     int adjRowAhead[NT];
     auto loadRows = [&](int tile) {
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int p = tile * TILE_POINTS + 4 * r + nt;
-            adjRowAhead[nt] = p < numel ? (adjOutputOrder ? adjOutputOrder[p] : p) : 0;
+        for (int nt = 0; nt < NT; ++nt) adjRowAhead[nt] = min(tile * TILE_POINTS + 4 * r + nt, numel - 1);
+        if (adjOutputOrder) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) adjRowAhead[nt] = adjOutputOrder[adjRowAhead[nt]];
         }
     };
     loadRows(firstTile < numTiles ? firstTile : numTiles - 1);
 #endif
-    float4 dyAhead[NT];
+    f32x4 dyAhead[NT][MTL];
+    auto loadAdjoints = [&](int tile) {
+        const float* row[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+#if $$HAS_OUTPUT_ORDER$$
+            const long long adjRow = adjRowAhead[nt];
+#else
+            const long long adjRow = min(tile * TILE_POINTS + 4 * r + nt, numel - 1);
+#endif
+            row[nt] = adjOutputs.data_ + adjRow * adjOutputs.strides_[0];
+        }
+        (void)tile;
+        if (adjOutputRowsOfFloat4) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int m = 0; m < MTL; ++m) dyAhead[nt][m] = *reinterpret_cast<const f32x4*>(row[nt] + min(16 * m + 4 * g, actualChannelsOut - 4));
+        } else if (MTL == 1 && adjOutputRowsOfFloat2) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const f32x2 two = *reinterpret_cast<const f32x2*>(row[nt]);
+                dyAhead[nt][0] = __builtin_shufflevector(two, two, 0, 1, -1, -1);   // (nobody looks at the others)
+            }
+        } else {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int m = 0; m < MTL; ++m)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        dyAhead[nt][m][i] = row[nt][static_cast<long long>(min(16 * m + 4 * g + i, actualChannelsOut - 1)) * adjOutputs.strides_[1]];
+        }
+    };
     f16x4 encodedAhead[LOADS_AHEAD ? KT0 : 1][4];
-    (void)dyAhead; (void)encodedAhead;
+    (void)encodedAhead;
     auto loadAhead = [&](int tile) {
         const int last = numTiles - 1;
         const int t0 = tile < last ? tile : last;   // (behind the last tile nobody looks at what is loaded)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int p = t0 * TILE_POINTS + 4 * r + nt;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (p < numel) {
-#if $$HAS_OUTPUT_ORDER$$
-                const long long adjRow = adjRowAhead[nt];
-#else
-                const long long adjRow = p;
-#endif
-                const float* row = adjOutputs.data_ + adjRow * adjOutputs.strides_[0];
-                if (adjOutputRowsOfFloat4) {
-                    if (4 * g < actualChannelsOut) v = *reinterpret_cast<const float4*>(row + 4 * g);
-                } else if (adjOutputRowsOfFloat2) {
-                    if (g == 0) {
-                        const float2 two = *reinterpret_cast<const float2*>(row);
-                        v.x = two.x, v.y = two.y;
-                    }
-                } else {
-                    const int c = 4 * g;
-                    const long long stride = adjOutputs.strides_[1];
-                    if (c < actualChannelsOut) v.x = row[c * stride];
-                    if (c + 1 < actualChannelsOut) v.y = row[(c + 1) * stride];
-                    if (c + 2 < actualChannelsOut) v.z = row[(c + 2) * stride];
-                    if (c + 3 < actualChannelsOut) v.w = row[(c + 3) * stride];
-                }
-            }
-            dyAhead[nt] = v;
-        }
+        loadAdjoints(t0);
 #if $$HAS_OUTPUT_ORDER$$
         loadRows(t0 + tileStep < last ? t0 + tileStep : last);
 #endif
@@ -225,61 +233,22 @@ $$ZERO_LDS_GRADIENTS$$
         // dL/dy -> accumulator layout (fp32 -> fp16), zero outside batch / real channels
         f16x4 dyOut[NT][MTL];
         int validMask = 0;
+        if constexpr (!LOADS_AHEAD) {
+            loadAdjoints(tileRead);
+#if $$HAS_OUTPUT_ORDER$$
+            loadRows(tileRead + tileStep < numTiles ? tileRead + tileStep : numTiles - 1);
+#endif
+        }
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            const int p = tile * TILE_POINTS + 4 * r + nt;
-            const bool pv = p < numel;
+            const bool pv = tile * TILE_POINTS + 4 * r + nt < numel;
             validMask |= pv ? (1 << nt) : 0;
-            if constexpr (LOADS_AHEAD) {
-                dyOut[nt][0][0] = static_cast<f16>(dyAhead[nt].x);
-                dyOut[nt][0][1] = static_cast<f16>(dyAhead[nt].y);
-                dyOut[nt][0][2] = static_cast<f16>(dyAhead[nt].z);
-                dyOut[nt][0][3] = static_cast<f16>(dyAhead[nt].w);
-                continue;
-            }
-#if $$HAS_OUTPUT_ORDER$$
-            const long long adjRow = adjRowAhead[nt];
-            {
-                const long long ahead = static_cast<long long>(p) + static_cast<long long>(gridDim.x) * (WAVES * TILE_POINTS);
-                adjRowAhead[nt] = (adjOutputOrder && ahead < numel) ? adjOutputOrder[ahead] : static_cast<int>(ahead < numel ? ahead : 0);
-            }
-#else
-            const long long adjRow = p;
-#endif
-            if (adjOutputRowsOfFloat2 || adjOutputRowsOfFloat4) {
-                // channels side by side in memory: four per load (a lane holds channels
-                // 16m+4g .. +3 of its points), a row of two channels as one 8-byte load
-                const float* row = adjOutputs.data_ + adjRow * adjOutputs.strides_[0];
 #pragma unroll
-                for (int m = 0; m < MTL; ++m) {
+            for (int m = 0; m < MTL; ++m) {
+                dyOut[nt][m] = toF16(dyAhead[nt][m]);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) dyOut[nt][m][i] = static_cast<f16>(0);
-                    const int c = 16 * m + 4 * g;
-                    if (adjOutputRowsOfFloat4 && pv && c < actualChannelsOut) {
-                        const float4 v = *reinterpret_cast<const float4*>(row + c);
-                        dyOut[nt][m][0] = static_cast<f16>(v.x);
-                        dyOut[nt][m][1] = static_cast<f16>(v.y);
-                        dyOut[nt][m][2] = static_cast<f16>(v.z);
-                        dyOut[nt][m][3] = static_cast<f16>(v.w);
-                    }
-                }
-                if (!adjOutputRowsOfFloat4 && pv && g == 0) {
-                    const float2 v = *reinterpret_cast<const float2*>(row);
-                    dyOut[nt][0][0] = static_cast<f16>(v.x);
-                    dyOut[nt][0][1] = static_cast<f16>(v.y);
-                }
-            } else {
-#pragma unroll
-                for (int m = 0; m < MTL; ++m)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int c = 16 * m + 4 * g + i;
-                        float v = 0.f;
-                        if (pv && c < actualChannelsOut)
-                            v = adjOutputs.data_[adjRow * adjOutputs.strides_[0]
-                                                 + static_cast<long long>(c) * adjOutputs.strides_[1]];
-                        dyOut[nt][m][i] = static_cast<f16>(v);
-                    }
+                for (int i = 0; i < 4; ++i)
+                    if (!pv || 16 * m + 4 * g + i >= actualChannelsOut) dyOut[nt][m][i] = static_cast<f16>(0);
             }
         }
 
@@ -355,19 +324,21 @@ $$CALL_ENCODINGS$$
                         // the channels of a row side by side: four per load and store. Kept to
                         // kernels without a grid scatter: in front of the gradient atomics of a grid
                         // no gain was measurable.
+                        float4 before[NUM_INPUTS / 4 > 0 ? NUM_INPUTS / 4 : 1];
+#pragma unroll
+                        for (int i = 0; i + 3 < NUM_INPUTS; i += 4) before[i / 4] = *reinterpret_cast<const float4*>(adjRow + i);
 #pragma unroll
                         for (int i = 0; i + 3 < NUM_INPUTS; i += 4) {
-                            float4 v = *reinterpret_cast<float4*>(adjRow + i);
-                            v.x += adjEncodingInput[i];
-                            v.y += adjEncodingInput[i + 1];
-                            v.z += adjEncodingInput[i + 2];
-                            v.w += adjEncodingInput[i + 3];
-                            *reinterpret_cast<float4*>(adjRow + i) = v;
+                            const float4 v = before[i / 4];
+                            *reinterpret_cast<float4*>(adjRow + i) = make_float4(v.x + adjEncodingInput[i], v.y + adjEncodingInput[i + 1],
+                                                                                v.z + adjEncodingInput[i + 2], v.w + adjEncodingInput[i + 3]);
                         }
                     } else {
+                        float before[NUM_INPUTS];
 #pragma unroll
-                        for (int i = 0; i < NUM_INPUTS; ++i)
-                            adjRow[static_cast<long long>(i) * adjInputs.strides_[1]] += adjEncodingInput[i];
+                        for (int i = 0; i < NUM_INPUTS; ++i) before[i] = adjRow[static_cast<long long>(i) * adjInputs.strides_[1]];
+#pragma unroll
+                        for (int i = 0; i < NUM_INPUTS; ++i) adjRow[static_cast<long long>(i) * adjInputs.strides_[1]] = before[i] + adjEncodingInput[i];
                     }
                 }
             }

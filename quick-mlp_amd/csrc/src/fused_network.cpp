@@ -1221,7 +1221,9 @@ std::string FusedNetwork::backwardSource(int flags, int blockSize, bool sliceGra
                     << "                    const f16x4 v = LOADS_AHEAD ? encodedAhead[LOADS_AHEAD ? t : 0][i]\n"
                     << "                        : *reinterpret_cast<const f16x4*>(encTile + (16 * t + 4 * g + i) * TILE_POINTS + 4 * r);\n"
                     << "#pragma unroll\n                    for (int nt = 0; nt < NT; ++nt) x0Kept[nt][t][i] = v[nt];\n                }\n        }\n"
-                    << "        if constexpr (LOADS_AHEAD) loadAhead(tile + tileStep);\n";
+                    // (what the loads of the tile in front brought is taken over first: behind the new ones it would be waited for together with them)
+                    << "        if constexpr (LOADS_AHEAD) {\n            materialize(x0Kept);\n            materialize(dyOut);\n"
+                    << "            __builtin_amdgcn_sched_barrier(0);\n            loadAhead(tile + tileStep);\n        }\n";
             for (int i = 0; i < L; ++i) {
                 const auto& l = layers_[i];
                 const std::string in = i == 0 ? std::string("x0Kept") : "act" + std::to_string(i);
