@@ -559,7 +559,10 @@ private:
      * how many of them that launch should take (whole steps of a large shape first; the caller
      * asks again for the rest).
      */
-    const CompiledKernel& forwardKernelFor(bool store, int numTiles, int* launchTiles = nullptr, bool noAlloc = false, bool derivatives = false, bool inputOnly = false);
+    const CompiledKernel& forwardKernelFor(bool store, int numTiles, int* launchTiles = nullptr, bool noAlloc = false, bool derivatives = false, bool inputOnly = false,
+                                           bool sorted = false);
+    /** Tables that a forward kernel goes through one after the other (most of an encoding's). */
+    int sweptTables() const;
     /** Points per launch of a forward kernel: the whole batch, or two passes of the grid for networks that gather. */
     int gatherChunkPoints(const CompiledKernel& ck) const;
     /** inference (store = false) or forward with stored intermediates, in one or several launches. */

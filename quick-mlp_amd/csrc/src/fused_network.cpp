@@ -1674,8 +1674,15 @@ void FusedNetwork::compileForwardKernel(bool store, int variant, bool compileOnl
     slot = std::move(ck);
 }
 
+int FusedNetwork::sweptTables() const
+{
+    int tables = 0;
+    for (const auto& e : encodings_) tables = std::max(tables, e->numSweptTables());
+    return tables;
+}
+
 const FusedNetwork::CompiledKernel& FusedNetwork::forwardKernelFor(bool store, int numTiles, int* launchTiles, bool noAlloc, bool derivatives,
-                                                                  bool inputOnly)
+                                                                  bool inputOnly, bool sorted)
 {
     derivatives = derivatives && store;
     inputOnly = inputOnly && store;
@@ -1694,6 +1701,28 @@ const FusedNetwork::CompiledKernel& FusedNetwork::forwardKernelFor(bool store, i
         int blockSize = 0, pointsPerLane = 1;
         forwardShape(store, VARIANT_DEFAULT, blockSize, pointsPerLane);
         if (pointsPerLane == 1) return loaded(VARIANT_DEFAULT);   // no gathers, or a pinned shape: one kernel
+    }
+    const int overwrite = store ? compileOptions_.overwriteBlocksizeForward : compileOptions_.overwriteBlocksizeInference;
+    if (sweptTables() < 2 && compileOptions_.pointsPerLane <= 0 && overwrite <= 0) {
+        // One table: there are no levels to sweep through together, and a tile per wavefront leaves room for more wavefronts and has no
+        // steps (256^2 nodes x 4, 300 007 / 700 001 / 2^21 points: 10 / 17 / 41 us, with the rule below 16 / 23 / 51; 512^3 cells hashed to 2^19
+        // entries x 2: 14 / 24 / 60 and 20 / 32 / 69). But the points of a slab of a sorted batch share lines: there the kernel of four tiles per
+        // wavefront takes a sixth less per point in whole steps (32^4 nodes x 8, 2^20 / 2^21 points 73 / 123 us, with one tile 84 / 139; 700 001
+        // points 83 and 64). A launch more costs what 1900 of its tiles take.
+        if (sorted && hasLargeVariant(store)) {
+            int blockSize = 0, pointsPerLane = 1;
+            forwardShape(store, VARIANT_LARGE, blockSize, pointsPerLane);
+            const long long step = static_cast<long long>(KernelFunction::computeUnits()) * (blockSize / WARP_SIZE) * pointsPerLane;
+            const long long steps = numTiles / step;
+            const double narrow = 1.2 * numTiles, large = static_cast<double>(divUp<long long>(numTiles, step) * step);
+            const double both = static_cast<double>(steps * step) + 1.2 * static_cast<double>(numTiles - steps * step) + 1900;
+            if (large <= narrow && (large <= both || steps == 0)) return loaded(VARIANT_LARGE);
+            if (steps > 0 && both < narrow) {
+                if (launchTiles) *launchTiles = static_cast<int>(steps * step);
+                return loaded(VARIANT_LARGE);
+            }
+        }
+        return loaded(VARIANT_NARROW);
     }
     // Kernels that take more tiles per wave are faster per point, but the time grows in steps
     // of one workgroup per compute unit, whether all compute units have one or not. Measured on
@@ -1750,7 +1779,7 @@ const FusedNetwork::CompiledKernel& FusedNetwork::forwardKernelFor(bool store, i
         QuickMLP::Instance().getLogger()->debug("the forward kernel with rows in registers spills %d bytes per lane, not used",
                                                 forwardKernels_[s][best].value().fun.scratchBytes());
         registerShapeSpills_[s] = true;
-        return forwardKernelFor(store, numTiles, launchTiles, noAlloc, derivatives, inputOnly);
+        return forwardKernelFor(store, numTiles, launchTiles, noAlloc, derivatives, inputOnly, sorted);
     }
     return forwardKernels_[s][best].value();
 }
@@ -2113,9 +2142,7 @@ int FusedNetwork::gatherChunkPoints(const CompiledKernel& ck) const
     // at 2^20. Batches of a network that gathers are therefore cut into launches of two
     // passes each; a launch boundary brings the workgroups back in step. A single table (cfg5)
     // has nothing to compete with and stays in one launch (two launches cost 3 % there).
-    int tables = 0;
-    for (const auto& e : encodings_) tables = std::max(tables, e->numSweptTables());
-    if (tables < 2) return std::numeric_limits<int>::max();
+    if (sweptTables() < 2) return std::numeric_limits<int>::max();
     const long long pass = static_cast<long long>(KernelFunction::computeUnits()) * (ck.blockSize / WARP_SIZE) * ck.pointsPerLane * TILE_POINTS;
     return static_cast<int>(std::min<long long>(2 * pass, std::numeric_limits<int>::max()));
 }
@@ -2199,7 +2226,7 @@ void FusedNetwork::launchForward(bool store, const Tensor& input, Tensor& output
         // the kernel shape for what is left; a network that gathers gets at most two steps of it per launch
         int launchTiles = 0;
         const auto& ck = forwardKernelFor(store, static_cast<int>(divUp<long long>(numel - start, TILE_POINTS)), &launchTiles, noAlloc, derivatives,
-                                          inputOnly);
+                                          inputOnly, sorted);
         int count = static_cast<int>(std::min<long long>(
             {static_cast<long long>(gatherChunkPoints(ck)), static_cast<long long>(launchTiles) * TILE_POINTS, numel - start}));
         auto inputAcc = inputAll;
@@ -2250,18 +2277,20 @@ void FusedNetwork::prepare(int numel, int adjointFlags)
     // the forward kernels that launchForward() takes for the pieces of a batch of this size
     // ([0]: inference, [1]: forward passes that store all intermediates, [2]: that store the encoded input only)
     if (adjointFlags > 0) announcedFlags_ = adjointFlags;
+    kernel::PointOrderKey key{};
+    const bool orders = pointOrderFor(numel, key);
     const int forwardKinds = adjointFlags <= 0 ? 1 : contentsFor(backwardMode(numel, adjointFlags)) == CONTENTS_ENCODED_INPUT ? 3 : 2;
     for (int store = 0; store < forwardKinds; ++store)
         for (long long start = 0; start < numel;) {
             int launchTiles = 0;
             const auto& ck = forwardKernelFor(store > 0, static_cast<int>(divUp<long long>(numel - start, TILE_POINTS)), &launchTiles, false,
-                                              store > 0 && storesDerivatives(numel, adjointFlags), store > 1);
+                                              store > 0 && storesDerivatives(numel, adjointFlags), store > 1,
+                                              store > 0 ? sortsTraining(numel) : orders);
             start += std::min<long long>({static_cast<long long>(gatherChunkPoints(ck)), static_cast<long long>(launchTiles) * TILE_POINTS,
                                           numel - start});
         }
     // the sort of a batch that is evaluated slab by slab: kernels, workspace, and the static buffer of inferenceNoAlloc()
-    kernel::PointOrderKey key{};
-    if (pointOrderFor(numel, key)) {
+    if (orders) {
         loadPointOrderKernels(adjointFlags > 0 && sortsTraining(numel));
         constexpr long long SLABS = 1024, CHUNK = 4 * 1024;   // as in sortPoints()
         const long long words = (divUp<long long>(numel, CHUNK) + 1) * SLABS + static_cast<long long>(numel) * (channelsIn_ + 1);
