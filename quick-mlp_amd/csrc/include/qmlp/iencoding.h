@@ -165,8 +165,8 @@ public:
         int pointsPerWorkgroup = 0;        // most lanes of a workgroup of the records kernel (a power of two)
         int derivativeBytesPerPoint = 0;   // of kernel::PositionDerivativeLayout: what a training pass may keep for the input gradients
         /** Dynamic LDS of the records kernel with this many lanes: its records of one level, and per slice of the level (at
-         *  most 512) their number and the place of the first. */
-        int recordsLdsBytes(int points) const { return points * pairs * recordWords * 4 + 2 * (512 + 1) * 4 + 64; }
+         *  most 512) their number, that of the next level and the place of the first. */
+        int recordsLdsBytes(int points) const { return points * pairs * recordWords * 4 + 3 * (512 + 1) * 4 + 64; }
         /** Dynamic LDS of the slice kernel: 64-bit sums of a slice and of the entry behind it. */
         int slicesLdsBytes() const { return (sliceFloats + features) * 8; }
         std::vector<int> slicesPerLevel;

@@ -303,6 +303,18 @@ struct RowAccessor
     __device__ __forceinline__ T& operator[](int i) const { return p[static_cast<long long>(i) * stride]; }
 };
 
+/** Sum over the lanes of the wavefront up to this one: six additions that take their operands from other lanes' registers. All lanes call this. */
+__device__ __forceinline__ int waveInclusiveScan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1, 2, 4, 8 (rows of 16 lanes; zero from outside)
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 /**
  * A workgroup barrier that orders the LDS accesses of the workgroup and nothing else. __syncthreads() also waits for
  * every load from and store to global memory that the wavefront has in flight: for kernels that read none of what they

@@ -16,14 +16,14 @@
 //       out as they are: the records of a region and level lie without gaps at a place that is known beforehand,
 //       and a row of `places` says where those of each slice begin. (Buckets per slice, in which every workgroup reserved room
 //       with an atomic per slice and level: 25 us of atomics, and a batch of unevenly spread points found them full. 16
-//       levels, 2^18 points with input gradients from derivatives: 124 -> 82 us.) The levels of a region are shared out over several
+//       levels, 2^18 points with input gradients from derivatives: 124 -> 82 us, 80 with two barriers per level instead of three.) The levels of a region are shared out over several
 //       workgroups. The grid's share of the gradient with respect to the input
 //       (what EncodingHashGrid::adjoint computes, operation by operation) comes from the
 //       entries of all corners, two that lie side by side with one load, or, where the forward
 //       pass kept the derivatives of the features with respect to the position (PositionDerivativeLayout,
 //       INPUT_GRADIENTS == 2), as adjoint x derivative from one or two coalesced loads per level; who computes it: see
 //       GridGradientRecords::inputGradientsInline. Bound by the memory that
-//       the records are written to: 268 MB of them for 2^18 points, 3.3 TB/s;
+//       the records are written to: 268 MB of them for 2^18 points, with what it reads 400 MB at 5 TB/s, what a copy reaches;
 //   GridGradientSlicesKernel   runs one workgroup per work item (level, slice, part of the
 //       regions): it streams through its records, a segment in every region, and adds weight * adjoint to the slice in LDS,
 //       then writes the slice, or adds it to the gradient tensor (with atomics only for a coarse level, whose
@@ -389,13 +389,22 @@ struct GridGradientRecords
     /** Registers worth holding across the sort of a level's records: 64 bytes of table entries per lane. */
     static constexpr bool DEFER_ENTRIES = Grid::NC * F * static_cast<int>(sizeof(typename Cfg::table_t)) <= 64;
 
+    /** Most slices of a level of the grid. */
+    __device__ __host__ static constexpr int mostSlices()
+    {
+        int most = 1;
+        for (int l = 0; l < Cfg::Levels; ++l) most = Layout::numSlices(l) > most ? Layout::numSlices(l) : most;
+        return most;
+    }
+
     /**
-     * Files the records of the workgroup's points in one level. sCount: zeros on entry and on return, MAX_SLICES + 1 words.
+     * Files the records of the workgroup's points in one level. sCount: zeros on entry and on return, MAX_SLICES + 1 words, as many in
+     * sOther: every level counts in the one that the level in front of it did not use, which is zeroed meanwhile.
      * \tparam INPUT_GRADIENTS the level's share of the gradient with respect to the position is added to adjPos
      */
     template <int LEVEL, int INPUT_GRADIENTS>
     __device__ __forceinline__ static void runLevel(int p, int numel, int region, const float (&position)[D], const Adjoints& adjEncoded,
-                                                    const GridGradientWorkspace& ws, unsigned* sStage, int* sCount, int* sStart,
+                                                    const GridGradientWorkspace& ws, unsigned* sStage, int*& sCount, int*& sOther, int* sStart,
                                                     unsigned& maxAdjBits, const param_t& params, const DerivativeChunk* __restrict__ derivatives,
                                                     float (&adjPos)[D])
     {
@@ -475,46 +484,47 @@ struct GridGradientRecords
         if (NS == 1 && tid == 0) sCount[0] = min(POINTS, numel - (p - tid)) * PAIRS;
         ldsBarrier();   // also: the staging area of the previous level has been copied out
 
-        // where the records of each slice begin
-        if (tid < 64) {
+        // Where the records of each slice begin: every wavefront adds the counts up for itself (all of them write the same values), which
+        // takes less than a barrier behind one of them that does it for all (16 levels, 2^18 / 2^17 floats / 2^15 points: 83 -> 80.5,
+        // 44.3 -> 42.5, 13.3 -> 12.8 us).
+        {
             unsigned short* places = ws.places + static_cast<long long>(region) * Layout::PLACES + Layout::firstPlace(LEVEL);
+            const int waveLane = tid % 64;
             int running = 0;
 #pragma unroll
             for (int b0 = 0; b0 < NS; b0 += 64) {
-                const int b = b0 + tid;
+                const int b = b0 + waveLane;
                 const int n = b < NS ? sCount[b] : 0;
-                int inclusive = n;
-#pragma unroll
-                for (int d = 1; d < 64; d *= 2) {
-                    const int other = __shfl_up(inclusive, d, 64);
-                    if (tid >= d) inclusive += other;
-                }
+                const int inclusive = waveInclusiveScan(n);
                 if (b < NS) {
                     sStart[b] = running + inclusive - n;
-                    places[b] = static_cast<unsigned short>(running + inclusive - n);
+                    if (tid < 64) places[b] = static_cast<unsigned short>(running + inclusive - n);
                 }
-                running += __shfl(inclusive, 63, 64);
+                running += __builtin_amdgcn_readlane(inclusive, 63);
             }
+            if (waveLane == 0) sStart[NS] = running;
             if (tid == 0) {
-                sStart[NS] = running;
                 places[NS] = static_cast<unsigned short>(running);
                 places[NS + 1] = static_cast<unsigned short>(sCount[NS]);
             }
+            waveLdsSync();
         }
-        ldsBarrier();
 
         if constexpr (INPUT_GRADIENTS == 1 && DEFER_ENTRIES) {
             // The entries of all corners where they take few registers: loaded here and used at the end of the level, so
             // that the two steps in between hide their latency (the barriers order LDS only).
             if (valid) loadHeld<LEVEL>(s, params, held);
         }
-        for (int b = tid; b <= NS; b += POINTS) sCount[b] = 0;
+        for (int b = tid; b <= mostSlices(); b += POINTS) sOther[b] = 0;
         if (filed) {
 #pragma unroll
             for (int c = 0; c < PAIRS; ++c) Layout::storeRecord(sStage + (sStart[bucket[c]] + rank[c]) * RW, rec[c]);
         }
         const int total = sStart[NS];
         ldsBarrier();
+        int* const counted = sCount;
+        sCount = sOther;
+        sOther = counted;
 
         // sorted by slice: the region as a whole
         unsigned* __restrict__ records = ws.records + regionStart * RW;
@@ -765,7 +775,8 @@ GridGradientRecordsKernel(
     extern __shared__ __align__(16) unsigned char sMemory[];
     unsigned* sStage = reinterpret_cast<unsigned*>(sMemory);              // POINTS * PAIRS records
     int* sCount = reinterpret_cast<int*>(sStage + POINTS * Impl::PAIRS * Impl::RW);
-    int* sStart = sCount + Impl::MAX_SLICES + 1;
+    int* sOther = sCount + Impl::MAX_SLICES + 1;
+    int* sStart = sOther + Impl::MAX_SLICES + 1;
     // (by few workgroups: the others only pass by)
     constexpr int ZEROING = 64;
     if (overwrite && blockIdx.x < ZEROING)
@@ -792,7 +803,7 @@ GridGradientRecordsKernel(
         }
     }
     unsigned maxAdjBits = 0u;
-    for (int b = threadIdx.x; b <= Impl::MAX_SLICES; b += POINTS) sCount[b] = 0;
+    for (int b = threadIdx.x; b <= Impl::MAX_SLICES; b += POINTS) sCount[b] = sOther[b] = 0;
     ldsBarrier();
     for (int region = first; region < workspace.regions; region += step) {
         const int p = region * POINTS + threadIdx.x;
@@ -800,8 +811,8 @@ GridGradientRecordsKernel(
 #pragma unroll
         for (int d = 0; d < D; ++d) pos[d] = adjPos[d] = 0.f;
         if (p < numel) Impl::loadPosition(inputs, p, params, pos);
-        Impl::template runGroup<0, GROUPS, INLINE>(group, p, numel, region, pos, adjEncoded, workspace, sStage, sCount, sStart, maxAdjBits, params,
-                                                   derivatives, adjPos);
+        Impl::template runGroup<0, GROUPS, INLINE>(group, p, numel, region, pos, adjEncoded, workspace, sStage, sCount, sOther, sStart,
+                                                   maxAdjBits, params, derivatives, adjPos);
         if constexpr (INLINE != 0) {
             if (p < numel) Impl::storeInputGradient(adjInputs, p, params, overwriteInput, adjPos);
         }
