@@ -382,11 +382,13 @@ int FusedNetwork::cooperativeRegisters(int waves, int registerWeight) const
 int FusedNetwork::cooperativeSlices(int numTiles) const
 {
     // One per workgroup: two of them per compute unit, up to four where a lane holds so little that more wavefronts find room
-    // (16 -> 64 x 2 -> 4, 10^6 points, forward and backward: 88 us with three, 95 with two).
+    // (16 -> 64 x 2 -> 4, 10^6 points, forward and backward: 88 us with three, 95 with two). Behind tables two or four: the pass is
+    // bound by the kernels of the tables, and a third slice per compute unit would only be more temporary memory.
     const CooperativeLayout& layout = cooperativeLayout();
     const int waves = layout.blockSize / WARP_SIZE;
     const int registers = cooperativeRegisters(waves, layout.registerWeight);
-    const int perComputeUnit = registers <= 100 ? 4 : registers <= 120 ? 3 : 2;
+    const bool tables = std::any_of(encodings_.begin(), encodings_.end(), [](const auto& e) { return e->hasParameters(); });
+    const int perComputeUnit = registers <= 100 ? 4 : registers <= 120 && !tables ? 3 : 2;
     return std::max(1, std::min(divUp(2 * numTiles, waves), perComputeUnit * (MAX_WEIGHT_UPDATE_SLICES / 2)));
 }
 
