@@ -75,6 +75,7 @@ public:
     [[nodiscard]] bool gradientSlices(GradientSliceLayout& layout, bool floatAdjoints) const override;
     [[nodiscard]] bool gradientColumns(const kernel::PointOrderKey& key, GradientColumnLayout& layout) const override;
     [[nodiscard]] int levelGroups() const override;
+    [[nodiscard]] std::vector<int> levelTiles() const override;
     [[nodiscard]] int numSweptTables() const override { return numLevels_; }
     [[nodiscard]] int gatherRegistersPerPoint() const override;
     [[nodiscard]] bool pointOrderKey(kernel::PointOrderKey& key, long long numPoints = 0) const override;

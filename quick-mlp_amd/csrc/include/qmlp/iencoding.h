@@ -4,6 +4,7 @@
 #include "json.h"
 #include "kernel_loader.h"
 #include "tensor.h"
+#include <qmlp/kernels/encoding_level_shares.h>
 #include <qmlp/kernels/grid_gradient_items.h>
 #include <qmlp/kernels/point_order_key.h>
 
@@ -124,6 +125,9 @@ public:
 
     /** Workgroups of the standalone forward kernel that may share out the levels of a point (device function forwardGroup; 1: forward). */
     [[nodiscard]] virtual int levelGroups() const { return 1; }
+
+    /** Tiles of each level that a wavefront of EncodingLevelsKernel takes; empty: no such kernel. */
+    [[nodiscard]] virtual std::vector<int> levelTiles() const { return {}; }
 
     /** Grids of many levels whose tile-wide adjoint the wavefronts of a workgroup may share by levels (device function
      *  adjointShared, for as many features as scatterTile() takes); 0 or the number of wavefronts. */
@@ -358,6 +362,10 @@ private:
     std::string adjointKernelSource(int adjointMode, bool sharedTile = false) const;
     std::optional<KernelFunction> adjointSharedKernel_[AdjointMode::ALL_GRADIENTS + 1];
     std::optional<KernelFunction> forwardKernel_[2];   // [1]: by groups of levels
+    /** Whether forward() takes EncodingLevelsKernel. */
+    bool forwardByLevels(const Tensor& input, const Tensor& output) const;
+    std::vector<KernelFunction> compileForwardByLevels(int flags) const;
+    std::vector<KernelFunction> forwardByLevels_;      // EncodingLevelsKernel, EncodingRowsKernel
     // Where the kernel without groups is the faster one, see EncodingForwardKernel.
     static constexpr long long FORWARD_WHOLE_ROWS_MIN_BATCH = 3 << 14;
     std::optional<KernelFunction> adjointKernel_[AdjointMode::ALL_GRADIENTS + 1];

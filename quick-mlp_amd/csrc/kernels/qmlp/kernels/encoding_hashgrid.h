@@ -582,6 +582,19 @@ struct EncodingHashGrid
         }
     }
 
+    /** The features of one level (the same for the whole wavefront). */
+    template <int LEVEL = 0, typename I>
+    __device__ __forceinline__ static void featuresOfLevel(int level, const I& input, const param_t& params, float (&feat)[F])
+    {
+        if (LEVEL + 1 == L || level == LEVEL) {
+            float pos[D];
+            unitPosition(input, params, pos);
+            gatherLevel(LEVEL, pos, params.parametersForward, feat);
+        } else if constexpr (LEVEL + 1 < L) {
+            featuresOfLevel<LEVEL + 1>(level, input, params, feat);
+        }
+    }
+
     /** What corner c of a level adds to the derivative of the loss with respect to the position in cells. */
     __device__ __forceinline__ static void addCornerDerivative(int l, const LevelSetup& s, int c, const float (&adjFeat)[F],
                                                                const param_t& params, float (&lvl)[D])

@@ -4,6 +4,7 @@
 
 #include <qmlp/kernels/common.h>
 #include <qmlp/kernels/arrays.h>
+#include <qmlp/kernels/encoding_level_shares.h>
 
 $$INCLUDES$$
 
@@ -53,6 +54,90 @@ __global__ void __launch_bounds__(256) EncodingForwardKernel(
         }
     }
 }
+
+#if $$BY_LEVELS$$
+/**
+ * Larger batches of grids of many levels, rows without gaps: the dies share out the levels (encoding_level_shares.h), so that a
+ * level's table is brought into the L2 of one die, or two, instead of all eight. Workgroups go to the dies in turn. A wavefront takes one
+ * level of 64 points; the values of a tile of 64 points lie level by level where its rows will be, for EncodingRowsKernel.
+ * 16 levels of 2^19 entries of 2 floats, 2^16 / 2^17 / 2^18 / 2^20 points: 37 / 64 / 116 / 437 us with EncodingRowsKernel,
+ * EncodingForwardKernel 42 / 70 / 182 / 771 (of 2 halves 29 / 49 / 95 / 364 and 35 / 49 / 132 / 568; which of them:
+ * IEncoding::forwardByLevels). Bound by the lines of 128 bytes that the L1s get from the L2, 64 to 68 per point.
+ */
+__global__ void __launch_bounds__(256) EncodingLevelsKernel(
+    long long numel,
+    const Tensor2Read<float> inputs,  //shape (numel, Cin)
+    float* __restrict__ outputs       //(numel, Cout) without gaps
+    $$ENCODING_PARAMETERS$$)
+{
+    typedef $$ENCODING$$ Encoding;
+    constexpr int L = Encoding::L, F = Encoding::F;
+    static_assert(ENCODING_LEVEL_WAVES == 256 / WAVE_SIZE, "a workgroup");
+    constexpr int TILES[L] = {$$LEVEL_TILES$$};   // of a wavefront
+    const int lane = threadIdx.x % WAVE_SIZE;
+    const int tiles = static_cast<int>((numel + TILE_POINTS - 1) / TILE_POINTS);
+    int left = blockIdx.x % ENCODING_DIES * (gridDim.x / ENCODING_DIES) + blockIdx.x / ENCODING_DIES, level = -1, perWave = 1;
+#pragma unroll
+    for (int l = 0; l < L; ++l) {
+        const int workgroups = (tiles + TILES[l] * ENCODING_LEVEL_WAVES - 1) / (TILES[l] * ENCODING_LEVEL_WAVES);
+        if (level < 0) {
+            if (left < workgroups) {
+                level = l;
+                perWave = TILES[l];
+            } else {
+                left -= workgroups;
+            }
+        }
+    }
+    if (level < 0) return;
+    const int first = left * perWave * ENCODING_LEVEL_WAVES + threadIdx.x / WAVE_SIZE;
+    for (int i = 0; i < perWave; ++i) {
+        const int tile = first + i * ENCODING_LEVEL_WAVES;
+        if (tile >= tiles) return;
+        const long long begin = static_cast<long long>(tile) * TILE_POINTS;
+        const int points = static_cast<int>(min(numel - begin, static_cast<long long>(TILE_POINTS)));
+        if (lane >= points) return;   // (of the last tile)
+        const StridedArray<const float> encodingInput{inputs.data_ + (begin + lane) * inputs.strides_[0], inputs.strides_[1]};
+        float features[F];
+        Encoding::featuresOfLevel(level, encodingInput, cEncoding, features);
+        float* target = outputs + begin * (L * F) + (level * points + lane) * F;
+#pragma unroll
+        for (int c = 0; c < F; ++c) target[c] = features[c];
+    }
+}
+
+/** The values of EncodingLevelsKernel, tile by tile, into rows in their place. A wavefront reads a tile before it writes it. */
+__global__ void __launch_bounds__(TILE_POINTS) EncodingRowsKernel(long long numel, float* outputs)
+{
+    typedef $$ENCODING$$ Encoding;
+    constexpr int L = Encoding::L, F = Encoding::F, CHANNELS = L * F, PITCH = CHANNELS | 1;
+    static_assert(CHANNELS <= ENCODING_ROWS_MAX_CHANNELS, "LDS of a workgroup");
+    __shared__ float rows[TILE_POINTS * PITCH];
+    const int lane = threadIdx.x;
+    const long long tileBase = blockIdx.x * static_cast<long long>(TILE_POINTS);
+    const int points = static_cast<int>(min(numel - tileBase, static_cast<long long>(TILE_POINTS)));
+    float* tile = outputs + tileBase * CHANNELS;
+    if (lane < points) {
+        float values[CHANNELS];
+#pragma unroll
+        for (int l = 0; l < L; ++l)
+#pragma unroll
+            for (int i = 0; i < F; ++i) values[l * F + i] = tile[(l * points + lane) * F + i];
+#pragma unroll
+        for (int c = 0; c < CHANNELS; ++c) rows[lane * PITCH + c] = values[c];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if constexpr (CHANNELS % 4 == 0) {
+        typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+        for (int i = lane; i < points * (CHANNELS / 4); i += WAVE_SIZE) {
+            const float* from = rows + i / (CHANNELS / 4) * PITCH + i % (CHANNELS / 4) * 4;
+            *reinterpret_cast<f32x4u*>(tile + 4 * i) = f32x4u{from[0], from[1], from[2], from[3]};
+        }
+    } else {
+        for (int i = lane; i < points * CHANNELS; i += WAVE_SIZE) tile[i] = rows[i / CHANNELS * PITCH + i % CHANNELS];
+    }
+}
+#endif
 
 #if $$SHARED_TILE$$
 // Small batches of grids of many levels: the wavefronts of a workgroup share the levels of 64 points, which one wavefront

@@ -303,6 +303,18 @@ int EncodingHashGrid::levelGroups() const
     return combinationMode_ == LayerCombinationMode::CONCAT ? std::min(8, numLevels_) : 1;
 }
 
+std::vector<int> EncodingHashGrid::levelTiles() const
+{
+    std::vector<int> tiles;
+    if (levelGroups() != kernel::ENCODING_DIES) return tiles;
+    const int entryBytes = parameterPrecision_ == Tensor::HALF ? 2 : 4;
+    for (int l = 0; l < numLevels_; ++l) {
+        const int end = l + 1 < numLevels_ ? layers_[l + 1].memoryOffset : numParameters_;
+        tiles.push_back(kernel::encodingLevelTiles(static_cast<long long>(end - layers_[l].memoryOffset) * entryBytes));
+    }
+    return tiles;
+}
+
 int EncodingHashGrid::ldsGradientFloats(int maxBytes, int& levels) const
 {
     levels = 0;

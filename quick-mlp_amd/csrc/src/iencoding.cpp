@@ -8,6 +8,7 @@
 
 #include <cctype>
 #include <cstring>
+#include <mutex>
 
 QUICKMLP_NAMESPACE_BEGIN
 
@@ -22,7 +23,7 @@ struct ArgPack
 
 std::string standaloneSource(const IEncoding& e, const std::string& callForward, const std::string& callAdjoint,
                              const std::string& callCorners = "", const std::string& callScatter = "",
-                             const std::string& callTraceGather = "", const std::string& callTraceScatter = "", int groups = 1, bool sharedTile = false)
+                             const std::string& callTraceGather = "", const std::string& callTraceScatter = "", int groups = 1, bool sharedTile = false, bool byLevels = false)
 {
     auto kl = QuickMLP::Instance().kernelLoader();
     std::string codeTemplate = kl->findFile("qmlp/kernels/encoding_kernels.h").value();
@@ -33,6 +34,13 @@ std::string standaloneSource(const IEncoding& e, const std::string& callForward,
     replaceAll(codeTemplate, "$$ENCODING_PARAMETERS$$",
                e.hasParameters() ? ", const " + e.parameterName() + " cEncoding" : std::string());
     replaceAll(codeTemplate, "$$SHARED_TILE$$", sharedTile ? "1" : "0");
+    replaceAll(codeTemplate, "$$BY_LEVELS$$", byLevels ? "1" : "0");
+    if (byLevels) {
+        std::string tiles;
+        for (int perWave : e.levelTiles()) tiles += (tiles.empty() ? "" : ", ") + std::to_string(perWave);
+        replaceAll(codeTemplate, "$$ENCODING$$", e.qualifiedName());
+        replaceAll(codeTemplate, "$$LEVEL_TILES$$", tiles);
+    }
     // the channels of a group of levels (EncodingForwardKernel)
     const std::string levels = std::to_string(e.numOutputChannels() / e.channelsWrittenTogether());
     const std::string features = std::to_string(e.channelsWrittenTogether());
@@ -60,6 +68,12 @@ std::string IEncoding::forwardKernelSource(int groups) const
     if (hasParameters()) call << ", cEncoding";
     call << ");\n";
     return standaloneSource(*this, call.str(), "", "", "", "", "", groups);
+}
+
+std::vector<KernelFunction> IEncoding::compileForwardByLevels(int flags) const
+{
+    return QuickMLP::Instance().kernelLoader()->getKernels({"qmlp::kernel::EncodingLevelsKernel", "qmlp::kernel::EncodingRowsKernel"},
+                                                           standaloneSource(*this, "", "", "", "", "", "", 1, false, true), flags);
 }
 
 std::string IEncoding::adjointKernelSource(int adjointMode, bool sharedTile) const
@@ -94,6 +108,7 @@ void IEncoding::precompile(int adjointMode)
     const int flags = QuickMLP::Instance().getCompileFlags() | KernelLoader::CompileOnly;
     kl->getKernel("qmlp::kernel::EncodingForwardKernel", forwardKernelSource(1), flags);
     if (levelGroups() > 1) kl->getKernel("qmlp::kernel::EncodingForwardKernel", forwardKernelSource(levelGroups()), flags);
+    if (!levelTiles().empty() && numOutputChannels() <= kernel::ENCODING_ROWS_MAX_CHANNELS) compileForwardByLevels(flags);
     if (adjointMode > 0) {
         CHECK_ERROR(adjointMode <= ALL_GRADIENTS, "Illegal adjoint mode");
         kl->getKernel("qmlp::kernel::EncodingAdjointKernel", adjointKernelSource(adjointMode), flags);
@@ -103,6 +118,34 @@ void IEncoding::precompile(int adjointMode)
             compileSlices(*layout, flags);
         }
     }
+}
+
+bool IEncoding::forwardByLevels(const Tensor& input, const Tensor& output) const
+{
+    const long long numel = input.size(0);
+    if (levelTiles().empty() || numOutputChannels() > kernel::ENCODING_ROWS_MAX_CHANNELS) return false;
+    // Tables that one die's L2 (4 MB) would have to take turns with, and batches that make up for a second kernel. Whole rows -> by levels,
+    // us, for grids of 8 to 32 levels and 20 to 90 MB of tables:
+    //   2^14 / 2^15 points   13 -> 17 / 23 -> 24 (16 levels of 2^19 entries of 2 floats, 50 MB; of 2 halves 10 -> 14 / 17 -> 20)
+    //   3 2^14, 2^16         37 -> 30, 42 -> 37 (halves 32 -> 25, 35 -> 29; the others 1.04 to 1.5 times as fast)
+    //   7 2^14 to 2^17       69 -> 63, in a training step 67 -> 67 (halves 49 -> 49, 25 MB 51 -> 56): the kernel of whole rows fills
+    //                        the chip exactly once, and its wavefronts walk through the levels together
+    //   80 000 to 7 2^14     72 -> 50 (98 304; halves 55 -> 39)
+    //   3 2^16               126 -> 90 (halves 78 -> 72)
+    //   2^18 / 2^20          182 -> 116 / 771 -> 437 (halves 132 -> 95 / 568 -> 364; the others 1.02 to 1.8 / 1.15 to 2.1 times as fast)
+    // One feature per level: 52 -> 39 at 3 2^14 points, but 73 -> 81 at 3 2^16. Tables of 13 MB at 2^17 points: 44 -> 56.
+    constexpr long long MIN_TABLE_BYTES = 20 << 20;
+    const long long tableBytes = static_cast<long long>(parameterCount()) * (parameterPrecision(Tensor::INFERENCE) == Tensor::HALF ? 2 : 4);
+    if (numel < FORWARD_WHOLE_ROWS_MIN_BATCH || tableBytes < MIN_TABLE_BYTES) return false;
+    if (channelsWrittenTogether() < 2 && numel < (1 << 18)) return false;
+    if (numel > (7 << 14) && numel <= (1 << 17)) return false;
+    if (numel * numOutputChannels() >= (1ll << 32)) return false;   // (lanes of a launch)
+    // Rows without gaps, which hold other points' values between the two kernels: not those that a caller reads the positions from.
+    if (output.size(1) != numOutputChannels() || output.strides()[0] != numOutputChannels()) return false;
+    const char* rows = static_cast<const char*>(output.rawPtr());
+    const char* positions = static_cast<const char*>(input.rawPtr());
+    const long long span = (numel - 1) * input.strides()[0] + (input.size(1) - 1) * input.strides()[1] + 1;
+    return positions + span * sizeof(float) <= rows || rows + numel * numOutputChannels() * sizeof(float) <= positions;
 }
 
 void IEncoding::forward(const Tensor& input, Tensor& output, stream_t stream,
@@ -122,12 +165,17 @@ void IEncoding::forward(const Tensor& input, Tensor& output, stream_t stream,
                     "The encoding has parameters, but no inference tensor is bound or passed");
     if (numel == 0) return;
 
+    const bool byLevels = forwardByLevels(input, output);
     const int groups = numel < FORWARD_WHOLE_ROWS_MIN_BATCH ? levelGroups() : 1;
     auto& kernel = forwardKernel_[groups > 1 ? 1 : 0];
-    if (!kernel.has_value())
+    if (byLevels) {
+        static std::mutex mutex;
+        std::lock_guard<std::mutex> lock(mutex);
+        if (forwardByLevels_.empty()) forwardByLevels_ = compileForwardByLevels(QuickMLP::Instance().getCompileFlags());
+    } else if (!kernel.has_value()) {
         kernel = QuickMLP::Instance().kernelLoader()->getKernel(
             "qmlp::kernel::EncodingForwardKernel", forwardKernelSource(groups), QuickMLP::Instance().getCompileFlags()).value();
-    auto& fun = kernel.value();
+    }
 
     std::vector<char> paramBytes(4096);
     if (hasParameters()) {
@@ -137,12 +185,24 @@ void IEncoding::forward(const Tensor& input, Tensor& output, stream_t stream,
     }
 
     const int block = 256;
-    const int grid = groups * static_cast<int>(std::min<long long>(divUp<long long>(numel, block), std::max(1, fun.fullGridSize(block, 0) / groups)));
     auto inputAcc = input.accessor<kernel::Tensor2Read<float>>();
     auto outputAcc = output.accessor<kernel::Tensor2RW<float>>();
-    std::vector<void*> args = {&numel, &inputAcc, &outputAcc};
-    if (hasParameters()) args.push_back(paramBytes.data());
-    fun.launch(grid, block, 0, stream, args.data());
+    if (byLevels) {
+        const long long tiles = divUp<long long>(numel, 64);
+        long long workgroups = 0;
+        for (int perWave : levelTiles()) workgroups += divUp<long long>(tiles, perWave * kernel::ENCODING_LEVEL_WAVES);
+        const long long perDie = divUp<long long>(workgroups, kernel::ENCODING_DIES);
+        float* rows = outputAcc.data_;
+        std::vector<void*> levelArgs = {&numel, &inputAcc, &rows, paramBytes.data()}, rowArgs = {&numel, &rows};
+        forwardByLevels_[0].launch(static_cast<int>(kernel::ENCODING_DIES * perDie), block, 0, stream, levelArgs.data());
+        forwardByLevels_[1].launch(static_cast<int>(tiles), 64, 0, stream, rowArgs.data());
+    } else {
+        auto& fun = kernel.value();
+        const int grid = groups * static_cast<int>(std::min<long long>(divUp<long long>(numel, block), std::max(1, fun.fullGridSize(block, 0) / groups)));
+        std::vector<void*> args = {&numel, &inputAcc, &outputAcc};
+        if (hasParameters()) args.push_back(paramBytes.data());
+        fun.launch(grid, block, 0, stream, args.data());
+    }
 
     if (hasParameters() && parametersForward.has_value()) setParameter({}, Tensor::INFERENCE);
 }

@@ -86,3 +86,27 @@ def test_forward_by_groups_of_levels_gives_the_same_bits(cfg):
     whole = enc.inference_with_parameter(x, table)
     for points in (1, 63, 65, 257, 5000, (3 << 14) - 1):
         assert torch.equal(enc.inference_with_parameter(x[:points], table), whole[:points]), points
+
+
+@pytest.mark.parametrize("levels, features, precision", [(11, 4, "half"), (16, 2, "half"), (9, 3, "float"), (24, 1, "float"), (16, 8, "half")])
+def test_forward_by_levels_gives_the_same_bits(levels, features, precision):
+    # tables of 20 to 60 MB: the dies share out the levels of larger batches. Rows with gaps, and positions in the rows' memory, take the
+    # kernel of whole rows.
+    cfg = json.loads(grid(levels, features, 19, precision))
+    cfg["max_resolution"] = 2000
+    require_gpu(cfg, (2, 3))
+    enc = qmlp.Encoding(json.dumps(cfg))
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    channels = enc.num_output_channels()
+    table = (torch.rand(enc.num_parameters(), device="cuda", generator=gen) - 0.5).to(enc.parameter_dtype())
+    for points in ((3 << 14) - 1, 3 << 14, 50001, (7 << 14) + 1, (1 << 17) + 63, (1 << 18) + 65):
+        x = torch.rand(points, 4, device="cuda", generator=gen) * 1.2 - 0.1
+        padded = torch.zeros(points, channels + 1, device="cuda")
+        check(lib.qmlp_encoding_forward(enc._handle, desc(x), desc(padded), current_stream(x.device), desc(table)))
+        assert torch.equal(enc.inference_with_parameter(x, table), padded[:, :channels]), points
+        if channels > 62 or points < 3 << 14:
+            continue   # (rows that are written as they come, and in pieces)
+        shared = torch.empty(points, channels, device="cuda")
+        shared[:, :3] = x[:, :3]
+        check(lib.qmlp_encoding_forward(enc._handle, desc(shared[:, :3]), desc(shared), current_stream(x.device), desc(table)))
+        assert torch.equal(shared, padded[:, :channels]), points
