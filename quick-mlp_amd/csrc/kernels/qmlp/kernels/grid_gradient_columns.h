@@ -306,7 +306,8 @@ struct GridGradientColumns
 
 /**
  * totals: points per slab (slabs0 * slabs1 <= 1024 values, as PointOrderScan leaves them). Writes starts
- * (slabs + 1 values), the work items and their number. One workgroup of 1024 threads.
+ * (slabs + 1 values), the work items and their number. One workgroup of 1024 threads, as long as its chain of steps: 5.3 us, 7 with items
+ * counted by an atomic in LDS, a lane at a time, and sums over the lanes by way of LDS.
  */
 template <typename Cfg, int CPS>
 __global__ void __launch_bounds__(1024) GridGradientColumnsPlan(
@@ -315,43 +316,41 @@ __global__ void __launch_bounds__(1024) GridGradientColumnsPlan(
 {
     typedef GridGradientColumns<Cfg, CPS> Impl;
     __shared__ int sScan[GRID_GRADIENT_COLUMNS_MAX_SLABS + 1];
-    __shared__ int sItems;
+    __shared__ int sWave[16];
     const int tid = threadIdx.x;
     const int slabs = slabs0 * slabs1;
-    // exclusive scan of the totals
-    const int mine = tid < slabs ? totals[tid] : 0;
-    int inclusive = mine;
-#pragma unroll
-    for (int d = 1; d < 64; d *= 2) {
-        const int other = __shfl_up(inclusive, d, 64);
-        if ((tid & 63) >= d) inclusive += other;
-    }
-    if ((tid & 63) == 63) sScan[tid / 64] = inclusive;   // wave totals
-    if (tid == 0) sItems = 0;
-    __syncthreads();
-    int before = 0;
-    for (int w = 0; w < tid / 64; ++w) before += sScan[w];
-    __syncthreads();
-    sScan[tid] = before + inclusive - mine;
-    if (tid == 1023) sScan[1024] = before + inclusive;
+    const int lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    // the values of the lanes in front of this one, and those of all lanes
+    auto scan = [&](int value, int& all) {
+        const int inclusive = waveInclusiveScan(value);
+        __syncthreads();   // (sWave of the scan before)
+        if (lane == 63) sWave[wave] = inclusive;
+        __syncthreads();
+        const int sums = waveInclusiveScan(lane < 16 ? sWave[lane] : 0);
+        all = __builtin_amdgcn_readlane(sums, 15);
+        return (wave > 0 ? __builtin_amdgcn_readlane(sums, wave - 1) : 0) + inclusive - value;
+    };
+    int points;
+    sScan[tid] = scan(tid < slabs ? totals[tid] : 0, points);
+    if (tid == 1023) sScan[1024] = points;
     __syncthreads();
     if (tid < slabs) starts[tid] = sScan[tid];
     if (tid == 0) starts[slabs] = numel;
-    // work items
-    for (int o = tid; o < Impl::OWNERS * Impl::OWNERS; o += 1024) {
-        const int o0 = o / Impl::OWNERS, o1 = o % Impl::OWNERS;
+    // work items, in the order of the owners
+    int itemsBefore = 0;
+    for (int first = 0; first < Impl::OWNERS * Impl::OWNERS; first += 1024) {
+        const int o = first + tid, o0 = o / Impl::OWNERS, o1 = o % Impl::OWNERS;
         // (the starts are read from LDS: the global copy is not visible to the whole workgroup yet; the totals
         // beyond the last slab are zero, so sScan[slabs] is the number of all points)
-        const typename Impl::Runs runs = Impl::runsOf(o0, o1, sScan, slabs0, slabs1);
-        const int points = runs.points();
-        if (points == 0) continue;
-        const int parts = (points + GRID_GRADIENT_COLUMNS_PART_POINTS - 1) / GRID_GRADIENT_COLUMNS_PART_POINTS;
-        const int at = atomicAdd(&sItems, parts);
+        const int visited = o < Impl::OWNERS * Impl::OWNERS ? Impl::runsOf(o0, o1, sScan, slabs0, slabs1).points() : 0;
+        const int parts = (visited + GRID_GRADIENT_COLUMNS_PART_POINTS - 1) / GRID_GRADIENT_COLUMNS_PART_POINTS;
+        int all;
+        const int at = itemsBefore + scan(parts, all);
         for (int part = 0; part < parts; ++part)
             if (at + part < maxItems) items[at + part] = GridGradientColumnItem{o0, o1, part, parts};
+        itemsBefore += all;
     }
-    __syncthreads();
-    if (tid == 0) *itemCount = min(sItems, maxItems);
+    if (tid == 0) *itemCount = min(itemsBefore, maxItems);
 }
 
 /**

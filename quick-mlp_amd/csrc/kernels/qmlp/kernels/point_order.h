@@ -23,6 +23,17 @@ constexpr int POINT_ORDER_BLOCK = 1024;
 constexpr int POINT_ORDER_POINTS_PER_THREAD = 4;    // a workgroup's chunk: 4096 points (offsets in it take 12 bits)
 constexpr int POINT_ORDER_SCAN_SLABS = 16;          // slabs per workgroup of PointOrderScan
 
+/**
+ * The chunk of this workgroup. Workgroups go to the 8 dies in turn; a die takes consecutive chunks, whose points of a slab lie side by
+ * side in the sorted batch: what is read or written of a line by several of them meets in its L2.
+ */
+__device__ __forceinline__ unsigned pointOrderChunk()
+{
+    constexpr unsigned DIES = 8;
+    const unsigned die = blockIdx.x % DIES;
+    return die * (gridDim.x / DIES) + min(die, gridDim.x % DIES) + blockIdx.x / DIES;
+}
+
 /** Slab of one coordinate value, clamped to the box (the comparisons are false for NaN, which then lands in slab 0). */
 __device__ __forceinline__ int pointOrderSlab1(float value, float lo, float scale, int slabs)
 {
@@ -83,36 +94,51 @@ __global__ void __launch_bounds__(POINT_ORDER_BLOCK) PointOrderCount(
 /**
  * histogram[w][slab] becomes the number of points of the slab in the chunks before w,
  * totals[slab] their number in all chunks. A workgroup takes POINT_ORDER_SCAN_SLABS slabs; 64 groups of
- * its threads take a 64th of the chunks each: sum, exchange through LDS, running sum. (64 workgroups: with
- * 16 workgroups of 64 slabs the pass took 8 us for 256 chunks and 13 us for 512.)
+ * its threads take a 64th of the chunks each: sum, exchange through LDS (a wavefront adds up a slab's), running sum; a thread's first chunks
+ * stay in its registers in between. All loads of a batch are asked for without a branch for the lane, behind which each would be
+ * waited for (512 chunks 6.7 -> 5.2 us, 147 chunks 4.9 -> 3.2). (64 workgroups: with 16 workgroups of 64 slabs the pass took 8 us for 256
+ * chunks and 13 us for 512.)
  */
 __global__ void __launch_bounds__(POINT_ORDER_BLOCK) PointOrderScan(int chunks, int* __restrict__ histogram, int* __restrict__ totals)
 {
     constexpr int GROUPS = POINT_ORDER_BLOCK / POINT_ORDER_SCAN_SLABS;
     constexpr int BATCH = 8;   // loads in flight
-    __shared__ int sPartial[GROUPS][POINT_ORDER_SCAN_SLABS];
+    static_assert(GROUPS == WAVE_SIZE && POINT_ORDER_BLOCK / WAVE_SIZE == POINT_ORDER_SCAN_SLABS, "a wavefront per slab, a lane per group");
+    __shared__ int sPartial[POINT_ORDER_SCAN_SLABS][GROUPS + 1];
     const int local = threadIdx.x % POINT_ORDER_SCAN_SLABS, group = threadIdx.x / POINT_ORDER_SCAN_SLABS;
-    const int slab = blockIdx.x * POINT_ORDER_SCAN_SLABS + local;
+    int* const counts = histogram + blockIdx.x * POINT_ORDER_SCAN_SLABS + local;
     const int perGroup = (chunks + GROUPS - 1) / GROUPS;
     const int begin = min(group * perGroup, chunks), end = min(begin + perGroup, chunks);
-    int sum = 0;
-    for (int w0 = begin; w0 < end; w0 += BATCH) {
+    int v[BATCH], sum = 0;
+    auto load = [&](int w0) {
 #pragma unroll
-        for (int j = 0; j < BATCH; ++j)
-            if (w0 + j < end) sum += histogram[(w0 + j) * POINT_ORDER_MAX_SLABS + slab];
+        for (int j = 0; j < BATCH; ++j) v[j] = counts[min(w0 + j, chunks - 1) * POINT_ORDER_MAX_SLABS];
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) v[j] = w0 + j < end ? v[j] : 0;
+    };
+    for (int w0 = begin + BATCH; w0 < end; w0 += BATCH) {
+        load(w0);
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) sum += v[j];
     }
-    sPartial[group][local] = sum;
-    __syncthreads();
-    int running = 0;
-    for (int q = 0; q < group; ++q) running += sPartial[q][local];
-    if (group == GROUPS - 1) totals[slab] = running + sum;
-    for (int w0 = begin; w0 < end; w0 += BATCH) {
-        int v[BATCH];
+    load(begin);   // (last: they are still held below)
 #pragma unroll
-        for (int j = 0; j < BATCH; ++j) v[j] = w0 + j < end ? histogram[(w0 + j) * POINT_ORDER_MAX_SLABS + slab] : 0;
+    for (int j = 0; j < BATCH; ++j) sum += v[j];
+    sPartial[local][group] = sum;
+    __syncthreads();
+    {
+        const int slab = threadIdx.x / WAVE_SIZE, lane = threadIdx.x % WAVE_SIZE;
+        const int own = sPartial[slab][lane], inclusive = waveInclusiveScan(own);
+        sPartial[slab][lane] = inclusive - own;
+        if (lane == WAVE_SIZE - 1) totals[blockIdx.x * POINT_ORDER_SCAN_SLABS + slab] = inclusive;
+    }
+    __syncthreads();
+    int running = sPartial[local][group];
+    for (int w0 = begin; w0 < end; w0 += BATCH) {
+        if (w0 > begin) load(w0);
 #pragma unroll
         for (int j = 0; j < BATCH; ++j) {
-            if (w0 + j < end) histogram[(w0 + j) * POINT_ORDER_MAX_SLABS + slab] = running;
+            if (w0 + j < end) counts[(w0 + j) * POINT_ORDER_MAX_SLABS] = running;
             running += v[j];
         }
     }
@@ -121,52 +147,65 @@ __global__ void __launch_bounds__(POINT_ORDER_BLOCK) PointOrderScan(int chunks, 
 /** Exclusive scan over the POINT_ORDER_MAX_SLABS values held one per thread of the workgroup. */
 __device__ __forceinline__ int pointOrderBlockScan(int value, int* sWaveSum)
 {
-    const int lane = threadIdx.x % WAVE_SIZE, wave = threadIdx.x / WAVE_SIZE;
-    int inclusive = value;
-#pragma unroll
-    for (int d = 1; d < WAVE_SIZE; d *= 2) {
-        const int other = __shfl_up(inclusive, d, WAVE_SIZE);
-        if (lane >= d) inclusive += other;
-    }
+    constexpr int WAVES = POINT_ORDER_MAX_SLABS / WAVE_SIZE;
+    static_assert(WAVES <= WAVE_SIZE, "a lane per wavefront");
+    const int lane = threadIdx.x % WAVE_SIZE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+    const int inclusive = waveInclusiveScan(value);
     __syncthreads();   // sWaveSum may still be read from a previous scan
     if (lane == WAVE_SIZE - 1) sWaveSum[wave] = inclusive;
     __syncthreads();
-    int before = 0;
-    for (int w = 0; w < wave; ++w) before += sWaveSum[w];
-    return before + inclusive - value;
+    const int sums = waveInclusiveScan(lane < WAVES ? sWaveSum[lane] : 0);
+    return (wave > 0 ? __builtin_amdgcn_readlane(sums, wave - 1) : 0) + inclusive - value;
 }
 
-/** The channels of one input row; one load of 8, 12 or 16 bytes where the layout allows it (vectorChannels > 0:
- *  rows of that many channels with unit stride between them, aligned to the vector). */
-template <int MAX_CHANNELS>
-__device__ __forceinline__ void pointOrderLoadRow(const Tensor2Read<float>& inputs, long long index, int vectorChannels, float (&row)[MAX_CHANNELS])
+/** The channels of N input rows, all of them asked for before the first is waited for; one load of 8, 12 or 16 bytes where the layout allows it
+ *  (vectorChannels > 0: rows of that many channels with unit stride between them, aligned to the vector). index(k): the row, one that is there. */
+template <int MAX_CHANNELS, int N, typename Index>
+__device__ __forceinline__ void pointOrderLoadRows(const Tensor2Read<float>& inputs, const Index& index, int vectorChannels, float (&rows)[N][MAX_CHANNELS])
 {
-    const float* src = inputs.data_ + index * inputs.strides_[0];
     typedef float f32x2a __attribute__((ext_vector_type(2)));
     typedef float f32x3a __attribute__((ext_vector_type(3), aligned(4)));
     typedef float f32x4a __attribute__((ext_vector_type(4)));
-    // (the branches fill a vector: stores to the array in each of them become one store to an address that depends on the
+    const float* src[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) src[k] = inputs.data_ + index(k) * inputs.strides_[0];
+    // (the branches fill vectors: stores to the array in each of them become one store to an address that depends on the
     // branch, and the array moves to scratch memory)
-    f32x4a first = {0.f, 0.f, 0.f, 0.f};
+    f32x4a first[N] = {};
     if (MAX_CHANNELS >= 4 && vectorChannels == 4) {
-        first = *reinterpret_cast<const f32x4a*>(src);
+#pragma unroll
+        for (int k = 0; k < N; ++k) first[k] = *reinterpret_cast<const f32x4a*>(src[k]);
     } else if (MAX_CHANNELS >= 3 && vectorChannels == 3) {
-        const f32x3a v = *reinterpret_cast<const f32x3a*>(src);
-        first = f32x4a{v[0], v[1], v[2], 0.f};
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const f32x3a v = *reinterpret_cast<const f32x3a*>(src[k]);
+            first[k] = f32x4a{v[0], v[1], v[2], 0.f};
+        }
     } else if (MAX_CHANNELS >= 2 && vectorChannels == 2) {
-        const f32x2a v = *reinterpret_cast<const f32x2a*>(src);
-        first = f32x4a{v[0], v[1], 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const f32x2a v = *reinterpret_cast<const f32x2a*>(src[k]);
+            first[k] = f32x4a{v[0], v[1], 0.f, 0.f};
+        }
     } else {
 #pragma unroll
         for (int c = 0; c < 4 && c < MAX_CHANNELS; ++c)
-            if (c < inputs.sizes_[1]) first[c] = src[static_cast<long long>(c) * inputs.strides_[1]];
+            if (c < inputs.sizes_[1]) {
+#pragma unroll
+                for (int k = 0; k < N; ++k) first[k][c] = src[k][static_cast<long long>(c) * inputs.strides_[1]];
+            }
     }
 #pragma unroll
-    for (int c = 0; c < MAX_CHANNELS; ++c)
-        row[c] = c < 4 ? first[c < 4 ? c : 0] : c < inputs.sizes_[1] ? src[static_cast<long long>(c) * inputs.strides_[1]] : 0.f;
+    for (int k = 0; k < N; ++k)
+#pragma unroll
+        for (int c = 0; c < 4 && c < MAX_CHANNELS; ++c) rows[k][c] = first[k][c];
+#pragma unroll
+    for (int c = 4; c < MAX_CHANNELS; ++c)
+#pragma unroll
+        for (int k = 0; k < N; ++k) rows[k][c] = c < inputs.sizes_[1] ? src[k][static_cast<long long>(c) * inputs.strides_[1]] : 0.f;
 }
 
-/** How the rows of inputs can be loaded as one vector each (pointOrderLoadRow), 0 if they cannot. */
+/** How the rows of inputs can be loaded as one vector each (pointOrderLoadRows), 0 if they cannot. */
 __device__ __forceinline__ int pointOrderVectorChannels(const Tensor2Read<float>& inputs)
 {
     const int channels = inputs.sizes_[1];
@@ -209,8 +248,9 @@ template <> struct PointOrderEntry<true> { typedef unsigned short type; };
  * Rows of up to four channels are read once, in the order given (consecutive lanes, consecutive rows), and wait
  * in LDS at their sorted place. Reading them a second time in sorted order, as wider rows still are, asks for 64
  * lines per instruction, many of which the chunks of the other workgroups have meanwhile pushed out of the L2 (14 us for
- * 2^21 rows of 16 bytes). Two workgroups share a compute unit, so that one loads while the other stores: 2^21 rows of 16 bytes 27 us,
- * 700 000 rows 12 us (75 and 25 MB, 2.8 and 2.1 TB/s). With the slab of each sorted point in LDS too, one workgroup had
+ * 2^21 rows of 16 bytes). Two workgroups share a compute unit, so that one loads while the other stores. Bound by the lines that are written
+ * in part: a chunk has four rows for a slab, and the chunk behind it the next four of the same line (pointOrderChunk: 2^21 rows of 16 bytes
+ * 27 -> 21 us, 10^6 rows 15 -> 13, 700 000 rows 11; 75 MB at 3.5 TB/s). With the slab of each sorted point in LDS too, one workgroup had
  * 94 KiB, and its rows went through scratch memory, because the compiler turned choices among registers into
  * addresses: 40 and 17 us.
  * \tparam MAX_CHANNELS at least the number of input channels (4, 8, 16)
@@ -238,7 +278,8 @@ __global__ void __launch_bounds__(POINT_ORDER_BLOCK) PointOrderScatter(
 
     const int channels = inputs.sizes_[1];
     const int vectorChannels = pointOrderVectorChannels(inputs);
-    const long long chunk = static_cast<long long>(blockIdx.x) * CHUNK;
+    const unsigned chunkIndex = pointOrderChunk();
+    const long long chunk = static_cast<long long>(chunkIndex) * CHUNK;
     const int chunkPoints = static_cast<int>(min(static_cast<long long>(CHUNK), numel - chunk));
     auto slabOf = [&](const float (&row)[MAX_CHANNELS]) {
         static_assert(MAX_CHANNELS >= 4, "a row in a vector");
@@ -247,22 +288,21 @@ __global__ void __launch_bounds__(POINT_ORDER_BLOCK) PointOrderScatter(
         asm("" : "+v"(v0), "+v"(v1), "+v"(v2), "+v"(v3));
         return pointOrderSlabOf([&](int c) { return c == 0 ? v0 : c == 1 ? v1 : c == 2 ? v2 : v3; }, key);
     };
-    int slab[POINT_ORDER_POINTS_PER_THREAD], rank[POINT_ORDER_POINTS_PER_THREAD];
-    float rows[STAGE_ROWS ? POINT_ORDER_POINTS_PER_THREAD : 1][MAX_CHANNELS] = {};
+    constexpr int N = POINT_ORDER_POINTS_PER_THREAD;
+    int slab[N], rank[N];
+    float rows[STAGE_ROWS ? N : 1][MAX_CHANNELS] = {};
     (void)rows;
-    if constexpr (STAGE_ROWS) {   // on their way while the totals are scanned
-#pragma unroll
-        for (int k = 0; k < POINT_ORDER_POINTS_PER_THREAD; ++k)
-            if (k * POINT_ORDER_BLOCK + t < chunkPoints) pointOrderLoadRow<MAX_CHANNELS>(inputs, chunk + k * POINT_ORDER_BLOCK + t, vectorChannels, rows[k]);
-    }
+    const int before = histogram[chunkIndex * POINT_ORDER_MAX_SLABS + t], total = totals[t];
+    // (lanes behind the last point: that one again)
+    if constexpr (STAGE_ROWS)
+        pointOrderLoadRows<MAX_CHANNELS>(inputs, [&](int k) { return chunk + min(k * POINT_ORDER_BLOCK + t, chunkPoints - 1); }, vectorChannels, rows);
     sCount[t] = 0;
-    const int before = histogram[blockIdx.x * POINT_ORDER_MAX_SLABS + t];
-    const int slabStart = pointOrderBlockScan(totals[t], sWaveSum) + before;   // holds a barrier after sCount = 0
+    const int slabStart = pointOrderBlockScan(total, sWaveSum) + before;   // holds a barrier after sCount = 0
 #pragma unroll
-    for (int k = 0; k < POINT_ORDER_POINTS_PER_THREAD; ++k) {
-        const int j = k * POINT_ORDER_BLOCK + t;
+    for (int k = 0; k < N; ++k) {
         slab[k] = 0;
         rank[k] = 0;
+        const int j = k * POINT_ORDER_BLOCK + t;
         if (j < chunkPoints) {
             if constexpr (STAGE_ROWS) slab[k] = slabOf(rows[k]);
             else slab[k] = pointOrderSlab(inputs, chunk + j, key);
@@ -289,23 +329,36 @@ __global__ void __launch_bounds__(POINT_ORDER_BLOCK) PointOrderScatter(
     }
     __syncthreads();
 
-#pragma unroll 4
-    for (int k = 0; k < POINT_ORDER_POINTS_PER_THREAD; ++k) {
-        const int j = k * POINT_ORDER_BLOCK + t;
-        if (j >= chunkPoints) continue;
-        const unsigned int entry = sSorted[j];
-        const long long index = chunk + (entry & 0xffffu);
-        float row[MAX_CHANNELS];
-        if constexpr (STAGE_ROWS) {
+    if constexpr (STAGE_ROWS) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const int j = k * POINT_ORDER_BLOCK + t;
+            if (j >= chunkPoints) continue;
+            float row[MAX_CHANNELS];
 #pragma unroll
             for (int c = 0; c < MAX_CHANNELS; ++c) row[c] = sRows[j * MAX_CHANNELS + c];
-        } else {
-            pointOrderLoadRow<MAX_CHANNELS>(inputs, index, vectorChannels, row);
+            const long long position = sCount[slabOf(row)] + j;
+            order[position] = static_cast<int>(chunk + sSorted[j]);
+            pointOrderStoreRow<MAX_CHANNELS>(sortedInputs, position, channels, vectorChannels, row);
         }
-        const int s = STAGE_ROWS ? slabOf(row) : static_cast<int>(entry >> 16);
-        const long long position = sCount[s] + j;
-        order[position] = static_cast<int>(index);
-        pointOrderStoreRow<MAX_CHANNELS>(sortedInputs, position, channels, vectorChannels, row);
+    } else {
+        // (two rows of up to 16 channels in flight)
+        constexpr int AHEAD = 2;
+#pragma unroll 1
+        for (int k0 = 0; k0 < N; k0 += AHEAD) {
+            float row[AHEAD][MAX_CHANNELS];
+            auto entryOf = [&](int k) -> unsigned { return sSorted[min((k0 + k) * POINT_ORDER_BLOCK + t, chunkPoints - 1)]; };
+            pointOrderLoadRows<MAX_CHANNELS>(inputs, [&](int k) { return chunk + (entryOf(k) & 0xffffu); }, vectorChannels, row);
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) {
+                const int j = (k0 + k) * POINT_ORDER_BLOCK + t;
+                if (j >= chunkPoints) continue;
+                const unsigned entry = entryOf(k);
+                const long long position = sCount[entry >> 16] + j;
+                order[position] = static_cast<int>(chunk + (entry & 0xffffu));
+                pointOrderStoreRow<MAX_CHANNELS>(sortedInputs, position, channels, vectorChannels, row[k]);
+            }
+        }
     }
 }
 
@@ -314,7 +367,8 @@ __global__ void __launch_bounds__(POINT_ORDER_BLOCK) PointOrderScatter(
  * (src dense), or written to it. The rows of dst are walked in their own order, so the read-modify-write is coalesced
  * and only the reads of src are scattered (2^21 rows of 16 bytes: 76 us as a scatter through `order`, whose rows of 16
  * bytes each cost a line read and a line written). Rows of 16 bytes move as one load and one store, four rows of a lane
- * in flight (43 us with a lane per element, 28 us so, written and not added to).
+ * in flight (43 us with a lane per element, 27 us so, written and not added to). Bound by the lines of src: a chunk's rows of a slab are
+ * half a line, and the rest of it belongs to the chunks beside it, which the same die therefore takes (22 us; 10^6 rows 13 -> 10).
  */
 __global__ void __launch_bounds__(POINT_ORDER_BLOCK) PointOrderGatherAddRows(
     long long elements, int channels, const float* __restrict__ src, const int* __restrict__ placement, Tensor2RW<float> dst, int overwrite)
@@ -323,21 +377,22 @@ __global__ void __launch_bounds__(POINT_ORDER_BLOCK) PointOrderGatherAddRows(
         && reinterpret_cast<unsigned long long>(src) % 16 == 0) {
         constexpr int ROWS = 4;
         const long long rows = elements / 4;
-        for (long long first = static_cast<long long>(blockIdx.x) * (ROWS * POINT_ORDER_BLOCK) + threadIdx.x; first < rows;
+        for (long long first = static_cast<long long>(pointOrderChunk()) * (ROWS * POINT_ORDER_BLOCK) + threadIdx.x; first < rows;
              first += static_cast<long long>(gridDim.x) * (ROWS * POINT_ORDER_BLOCK)) {
+            // (lanes behind the last row: that one again)
             int from[ROWS];
             float4 v[ROWS], old[ROWS];
 #pragma unroll
-            for (int k = 0; k < ROWS; ++k) {
-                const long long row = first + k * POINT_ORDER_BLOCK;
-                from[k] = row < rows ? placement[row] : 0;
-            }
+            for (int k = 0; k < ROWS; ++k) from[k] = placement[min(first + k * POINT_ORDER_BLOCK, rows - 1)];
 #pragma unroll
             for (int k = 0; k < ROWS; ++k) {
                 v[k] = reinterpret_cast<const float4*>(src)[from[k]];
-                const long long row = first + k * POINT_ORDER_BLOCK;
                 old[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (!overwrite && row < rows) old[k] = *reinterpret_cast<const float4*>(dst.data_ + row * dst.strides_[0]);
+            }
+            if (!overwrite) {
+#pragma unroll
+                for (int k = 0; k < ROWS; ++k)
+                    old[k] = *reinterpret_cast<const float4*>(dst.data_ + min(first + k * POINT_ORDER_BLOCK, rows - 1) * dst.strides_[0]);
             }
 #pragma unroll
             for (int k = 0; k < ROWS; ++k) {

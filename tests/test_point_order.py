@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from helpers import require_gpu, warm_cache
-from test_gpu_parity import Case, random_parameters
+from test_gpu_parity import FLAG_ENC, FLAG_INPUT, Case, random_parameters
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +50,32 @@ def test_sorted_rows_of_all_layouts_give_the_bits_of_the_order_given(dims, chann
                 a, b = outputs(layout)
                 assert torch.equal(torch.nan_to_num(a, nan=7.0), torch.nan_to_num(b, nan=7.0)), (points, layout.stride())
     assert float(a[torch.isfinite(a)].abs().max()) > 0.01
+
+
+# chunks of 4096 points: 8 dies share them out, of 512 and more a thread of the scan adds up more than it holds
+@pytest.mark.parametrize("chunks", [7, 9, 37, 517])
+def test_batches_of_many_chunks_give_the_bits_of_the_order_given(chunks):
+    require_gpu()
+    points = chunks * 4096 - 1001
+    base = {"num_inputs": 4, "num_outputs": 2, "activation_specification": ["qmlp/builtin-activations.json"],
+            "encodings": [{"id": "HashGrid", "start_in": 0, "n_in": 3, "n_levels": 1, "n_features_per_level": 2, "log2_hashmap_size": -1,
+                           "min_resolution": 128, "max_resolution": 128, "combination_mode": "concat", "bounding_box_min": [0.0] * 3,
+                           "bounding_box_size": [1.0] * 3, "parameter_precision": "half"}],
+            "network": [{"n_out": 2, "bias": False, "activation": "identity"}]}
+    specs = [dict(base, options={"sort_points": mode, "slice_gradients": 1}) for mode in (1, 0)]
+    warm_cache(*specs)
+    rng = np.random.default_rng(chunks)
+    x = rng.uniform(0, 1, (points, 4)).astype(np.float32)
+    adj = rng.uniform(-1, 1, (points, 2)).astype(np.float32)
+    results = []
+    for spec in specs:
+        case = Case(spec)
+        if not results:
+            parameters = random_parameters(case.oracle, rng)
+            table = rng.uniform(-1, 1, case.oracle.encodings[0][1].n_params)
+        case.set_parameters(parameters)
+        case.set_table(0, table)
+        out = case.net.inference(torch.from_numpy(x).cuda(), case.params, case.encoding_parameters())
+        results.append((out, case.gpu_train(x, adj, FLAG_ENC | FLAG_INPUT)["adj_x"]))
+    assert torch.equal(results[0][0], results[1][0])
+    assert np.array_equal(results[0][1], results[1][1]) and np.abs(results[0][1]).max() > 0.01
