@@ -1708,16 +1708,18 @@ const FusedNetwork::CompiledKernel& FusedNetwork::forwardKernelFor(bool store, i
     if (sweptTables() < 2 && compileOptions_.pointsPerLane <= 0 && overwrite <= 0) {
         // One table: there are no levels to sweep through together, and a tile per wavefront leaves room for more wavefronts and has no
         // steps (256^2 nodes x 4, 300 007 / 700 001 / 2^21 points: 10 / 17 / 41 us, with the rule below 16 / 23 / 51; 512^3 cells hashed to 2^19
-        // entries x 2: 14 / 24 / 60 and 20 / 32 / 69). But the points of a slab of a sorted batch share lines: there the kernel of four tiles per
-        // wavefront takes a sixth less per point in whole steps (32^4 nodes x 8, 2^20 / 2^21 points 73 / 123 us, with one tile 84 / 139; 700 001
-        // points 83 and 64). A launch more costs what 1900 of its tiles take.
-        if (sorted && hasLargeVariant(store)) {
+        // entries x 2: 14 / 24 / 60 and 20 / 32 / 69). But the points of a slab of a sorted batch share lines: training passes of many
+        // points, whose lanes hold what they store as well, take a twentieth less per point with four tiles per wavefront in whole steps, behind
+        // a longer start (32^4 nodes x 8, forward and backward of 2^20 / 1 500 007 / 2^21 / 2^22 points 242 / 319 / 410 / 787 us, with one tile 238 /
+        // 316 / 416 / 799; inference 68 / 95 / 112 / 207 and 63 / 80 / 107 / 199). A launch more costs what 1900 of its tiles take.
+        if (sorted && store && hasLargeVariant(store)) {
             int blockSize = 0, pointsPerLane = 1;
             forwardShape(store, VARIANT_LARGE, blockSize, pointsPerLane);
             const long long step = static_cast<long long>(KernelFunction::computeUnits()) * (blockSize / WARP_SIZE) * pointsPerLane;
             const long long steps = numTiles / step;
-            const double narrow = 1.2 * numTiles, large = static_cast<double>(divUp<long long>(numTiles, step) * step);
-            const double both = static_cast<double>(steps * step) + 1.2 * static_cast<double>(numTiles - steps * step) + 1900;
+            constexpr double PER_TILE = 1.055, START = 1300;
+            const double narrow = PER_TILE * numTiles, large = START + static_cast<double>(divUp<long long>(numTiles, step) * step);
+            const double both = START + static_cast<double>(steps * step) + PER_TILE * static_cast<double>(numTiles - steps * step) + 1900;
             if (large <= narrow && (large <= both || steps == 0)) return loaded(VARIANT_LARGE);
             if (steps > 0 && both < narrow) {
                 if (launchTiles) *launchTiles = static_cast<int>(steps * step);

@@ -1,4 +1,4 @@
-"""Networks behind a grid of one table take one tile per wavefront, and four for whole steps of a batch in slab order
+"""Networks behind a grid of one table take one tile per wavefront, and four for whole steps of a training pass in slab order
 (FusedNetwork::forwardKernelFor): batches on both sides of the steps, cut into two launches, and small ones."""
 import numpy as np
 import pytest
@@ -21,7 +21,7 @@ def configuration(dim, features, resolution, log2, options):
 
 # ordered by slab from 2^19 points on; a table that stays in the L2, never ordered; hashed entries
 @pytest.mark.parametrize("dim,features,resolution,log2,sizes", [
-    (4, 8, 32, -1, (1, 65, 300007, 1 << 19, (1 << 19) + 1, 700001, (1 << 20) + 30011)),
+    (4, 8, 32, -1, (1, 65, 300007, 1 << 19, (1 << 19) + 1, 700001, (1 << 20) + 30011, 1 << 21, (1 << 22) + 6403)),
     (2, 4, 64, -1, (1, 4097, 300007, 1 << 19)), (3, 2, 128, 12, (63, 70001, 600011))])
 def test_shapes_give_the_bits_of_one_tile_per_wavefront(dim, features, resolution, log2, sizes):
     free, pinned = configuration(dim, features, resolution, log2, {}), configuration(dim, features, resolution, log2, {"points_per_lane": 1, "sort_points": 0})
