@@ -18,6 +18,11 @@ static std::string withoutSpaces(const std::string& s)
     return o;
 }
 
+// CELU: max(x, 0) + (exp(min(x, 0)) - 1), whose adjoint is that exponential times adjz: the bits of the snippets (one of the two terms is a
+// zero, or the exponential one; a NaN stays in the minimum), without a comparison and a choice for every value.
+static constexpr const char* CELU_FORWARD = "z=__hgt(x,hZERO())?x:__hsub(hexp(x),__float2half(1.0f))";
+static constexpr const char* CELU_ADJOINT = "adjx=__hgt(x,hZERO())?adjz:__hmul(adjz,hexp(x))";
+
 /**
  * Packed form of snippets that are recognised literally (after removing white space): the
  * kernels apply it to four values at once (two packed instructions) instead of calling the
@@ -28,6 +33,7 @@ static std::string packedForward(const std::string& forward)
     const std::string f = withoutSpaces(forward);
     if (f == "z=__hgt(x,hZERO())?x:hZERO()")   // ReLU: v_pk_max_f16 (NaN -> 0 like the comparison)
         return "        return __builtin_elementwise_max(x, f16x4{0, 0, 0, 0});\n";
+    if (f == CELU_FORWARD) return "        return __builtin_elementwise_max(x, f16x4{0, 0, 0, 0}) + (exponentialOfNegative(x) - f16x4{1, 1, 1, 1});\n";
     if (f == "z=x") return "        return x;\n";
     return "";
 }
@@ -36,6 +42,7 @@ static std::string packedForward(const std::string& forward)
 static std::string packedAdjoint(const std::string& adjoint)
 {
     const std::string a = withoutSpaces(adjoint);
+    if (a == CELU_ADJOINT) return "        return adjz * exponentialOfNegative(x);\n";
     if (a == "adjx=adjz") return "        return adjz;\n";
     return "";
 }
