@@ -233,22 +233,62 @@ $$ZERO_LDS_GRADIENTS$$
         // dL/dy -> accumulator layout (fp32 -> fp16), zero outside batch / real channels
         f16x4 dyOut[NT][MTL];
         int validMask = 0;
-        if constexpr (!LOADS_AHEAD) {
-            loadAdjoints(tileRead);
+        if constexpr (LOADS_AHEAD) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const bool pv = tile * TILE_POINTS + 4 * r + nt < numel;
+                validMask |= pv ? (1 << nt) : 0;
+#pragma unroll
+                for (int m = 0; m < MTL; ++m) {
+                    dyOut[nt][m] = toF16(dyAhead[nt][m]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (!pv || 16 * m + 4 * g + i >= actualChannelsOut) dyOut[nt][m][i] = static_cast<f16>(0);
+                }
+            }
+        } else {
+            // (a point after the other, behind its own branch: by way of the arrays of the loads ahead, which then lie in scratch memory, the kernel
+            // of 30 000 points behind 32^4 nodes x 8 took 35 us, 30 so)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const int p = tile * TILE_POINTS + 4 * r + nt;
+                const bool pv = p < numel;
+                validMask |= pv ? (1 << nt) : 0;
 #if $$HAS_OUTPUT_ORDER$$
-            loadRows(tileRead + tileStep < numTiles ? tileRead + tileStep : numTiles - 1);
+                const long long adjRow = adjRowAhead[nt];
+                {
+                    const long long ahead = static_cast<long long>(p) + static_cast<long long>(tileStep) * TILE_POINTS;
+                    adjRowAhead[nt] = (adjOutputOrder && ahead < numel) ? adjOutputOrder[ahead] : static_cast<int>(ahead < numel ? ahead : 0);
+                }
+#else
+                const long long adjRow = p;
 #endif
-        }
+                const float* row = adjOutputs.data_ + adjRow * adjOutputs.strides_[0];
+                if (adjOutputRowsOfFloat2 || adjOutputRowsOfFloat4) {
+                    // channels side by side in memory: four per load (a lane holds channels
+                    // 16m+4g .. +3 of its points), a row of two channels as one 8-byte load
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const bool pv = tile * TILE_POINTS + 4 * r + nt < numel;
-            validMask |= pv ? (1 << nt) : 0;
+                    for (int m = 0; m < MTL; ++m) {
+                        dyOut[nt][m] = f16x4{0, 0, 0, 0};
+                        const int c = 16 * m + 4 * g;
+                        if (adjOutputRowsOfFloat4 && pv && c < actualChannelsOut) dyOut[nt][m] = toF16(*reinterpret_cast<const f32x4*>(row + c));
+                    }
+                    if (!adjOutputRowsOfFloat4 && pv && g == 0) {
+                        const f32x2 two = *reinterpret_cast<const f32x2*>(row);
+                        dyOut[nt][0][0] = static_cast<f16>(two[0]);
+                        dyOut[nt][0][1] = static_cast<f16>(two[1]);
+                    }
+                } else {
 #pragma unroll
-            for (int m = 0; m < MTL; ++m) {
-                dyOut[nt][m] = toF16(dyAhead[nt][m]);
+                    for (int m = 0; m < MTL; ++m)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (!pv || 16 * m + 4 * g + i >= actualChannelsOut) dyOut[nt][m][i] = static_cast<f16>(0);
+                        for (int i = 0; i < 4; ++i) {
+                            const int c = 16 * m + 4 * g + i;
+                            float v = 0.f;
+                            if (pv && c < actualChannelsOut) v = row[static_cast<long long>(c) * adjOutputs.strides_[1]];
+                            dyOut[nt][m][i] = static_cast<f16>(v);
+                        }
+                }
             }
         }
 
