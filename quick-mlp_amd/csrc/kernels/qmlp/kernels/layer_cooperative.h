@@ -203,20 +203,25 @@ struct CooperativeLayer
         }
     }
 
-    /** Gradient tiles of this wavefront. */
+    /** Gradient tiles of this wavefront; column m of the bias tile holds the sums of its m-th tile of output channels. (A tile that
+     *  several layers share saves registers, but its other columns are multiplied by zero: an infinite adjoint in one layer
+     *  makes sums of the others NaN.) */
     struct Sums
     {
         f32x4 w[MO][KI];
-        __device__ __forceinline__ void zero() { zeroTiles(w); }
+        f32x4 b;
+        __device__ __forceinline__ void zero()
+        {
+            zeroTiles(w);
+            b = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
     };
 
     /**
      * Adds the points of all wavefronts to the tiles of this one. rows: the rows of wavefront 0, those of wavefront i
-     * start i * rowsPerWave halves further. bias: tiles that all layers share, column FIRST_COLUMN + m (16 to a tile) holds the
-     * sums of this wavefront's m-th tile of output channels.
+     * start i * rowsPerWave halves further.
      */
-    template <int FIRST_COLUMN, int BIAS_TILES>
-    __device__ __forceinline__ static void weightGradient(const f16* rows, int rowsPerWave, Sums& sums, f32x4 (&bias)[BIAS_TILES], int wave, int lane)
+    __device__ __forceinline__ static void weightGradient(const f16* rows, int rowsPerWave, Sums& sums, int wave, int lane)
     {
         const int g = lane >> 4, i = lane & 15;
         const int wm = wave % Share::M, wk = (wave / Share::M) % Share::K, wp = wave / (Share::M * Share::K);
@@ -240,8 +245,9 @@ struct CooperativeLayer
 #pragma unroll
                 for (int k = 0; k < KI; ++k) sums.w[m][k] = mfma32(a, b[k], sums.w[m][k]);
                 if constexpr (BIAS) {
-                    f32x4& tile = bias[(FIRST_COLUMN + m) / 16];
-                    if (wk == 0) tile = mfma32(a, i == (FIRST_COLUMN + m) % 16 ? ones : zeros, tile);
+                    if (p % Share::K == wk) {   // (one of the wavefronts that read these rows)
+                        sums.b = mfma32(a, MO == 1 || i == m ? ones : zeros, sums.b);
+                    }
                 }
             }
         }
@@ -249,10 +255,9 @@ struct CooperativeLayer
 
     /**
      * After the last tile: the workgroup's sums into slice blockIdx.x of the partial gradients, slices beyond the grid
-     * zeroed (as Layer::storeWeightGradient). sAcc: (MT * KT * 256 + COUT) floats. All threads call this.
+     * zeroed (as Layer::storeWeightGradient). sAcc: (MT * KT * 256 + WAVES * COUT) floats. All threads call this.
      */
-    template <int FIRST_COLUMN, int BIAS_TILES>
-    __device__ __forceinline__ static void storeWeightGradient(const Sums& sums, const f32x4 (&bias)[BIAS_TILES], float* sAcc, float* __restrict__ partialWeights,
+    __device__ __forceinline__ static void storeWeightGradient(const Sums& sums, float* sAcc, float* __restrict__ partialWeights,
                                                                float* __restrict__ partialBias, int numSlices, int sliceStride, int wave, int lane)
     {
         const int g = lane >> 4, r = lane & 15;
@@ -272,23 +277,22 @@ struct CooperativeLayer
                         *target = p == 0 ? sums.w[m][k][i] : *target + sums.w[m][k][i];
                     }
                 }
-            if constexpr (BIAS) {
+        }
+        if constexpr (BIAS) {
+            if (r < MO && wm * MO + r < MT) {
 #pragma unroll
-                for (int m = 0; m < MO; ++m) {
-                    if (wk != 0 || r != (FIRST_COLUMN + m) % 16 || wm * MO + m >= MT) continue;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float sum = bias[(FIRST_COLUMN + m) / 16][i];
-                        float* target = sBias + 16 * (wm * MO + m) + 4 * g + i;
-                        *target = p == 0 ? sum : *target + sum;
-                    }
-                }
+                for (int i = 0; i < 4; ++i) sBias[(wp * Share::K + wk) * COUT + 16 * (wm * MO + r) + 4 * g + i] = sums.b[i];
             }
         }
         __syncthreads();
         for (int e = threadIdx.x; e < COUT * CIN; e += blockDim.x) partialWeights[e] = sAcc[e];
         if constexpr (BIAS) {
-            for (int e = threadIdx.x; e < COUT; e += blockDim.x) partialBias[e] = sBias[e];
+            for (int e = threadIdx.x; e < COUT; e += blockDim.x) {
+                float sum = sBias[e];
+#pragma unroll
+                for (int s = 1; s < Share::P * Share::K; ++s) sum += sBias[s * COUT + e];
+                partialBias[e] = sum;
+            }
         }
         for (int slice = blockIdx.x + gridDim.x; slice < numSlices; slice += gridDim.x) {
             const long long offset = static_cast<long long>(slice - static_cast<int>(blockIdx.x)) * sliceStride;

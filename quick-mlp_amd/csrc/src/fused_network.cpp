@@ -314,12 +314,10 @@ FusedNetwork::CooperativeLayout FusedNetwork::findCooperativeLayout() const
     constexpr int PAD = 4, POINTS = 32;
     CooperativeLayout c;
     c.biasOffsets.assign(layers_.size(), 0);
-    int sums = 0;
     for (const auto& l : layers_) {
         c.weightOffsets.push_back(c.paramHalves);
         c.paramHalves += l.channelsOut * (l.channelsIn + PAD);
         c.rowsPerWave = std::max(c.rowsPerWave, POINTS * (l.channelsOut + PAD + l.channelsIn + PAD));
-        sums = std::max(sums, l.channelsOut * (l.channelsIn + 1) * static_cast<int>(sizeof(float)));
     }
     for (size_t i = 0; i < layers_.size(); ++i) {
         if (!layers_[i].useBias) continue;
@@ -338,7 +336,9 @@ FusedNetwork::CooperativeLayout FusedNetwork::findCooperativeLayout() const
                                     {8, lds, 225, ""},
                                     {4, lds, 420, "__attribute__((amdgpu_waves_per_eu(1, 1)))"}};
     for (const auto& candidate : candidates) {
-        const int bytes = std::max(sums, (c.paramHalves + candidate.waves * c.rowsPerWave) * static_cast<int>(sizeof(half)));
+        int bytes = (c.paramHalves + candidate.waves * c.rowsPerWave) * static_cast<int>(sizeof(half));
+        for (const auto& l : layers_)   // after the last tile: the sums of a layer, a row of bias sums per wavefront
+            bytes = std::max(bytes, l.channelsOut * (l.channelsIn + (l.useBias ? candidate.waves : 0)) * static_cast<int>(sizeof(float)));
         if (bytes > candidate.ldsLimit) continue;
         for (int weight : {8, 16}) {
             const int registers = cooperativeRegisters(candidate.waves, weight);
@@ -357,10 +357,10 @@ FusedNetwork::CooperativeLayout FusedNetwork::findCooperativeLayout() const
 
 int FusedNetwork::cooperativeRegisters(int waves, int registerWeight) const
 {
-    int tiles = 0, biasColumns = 0, kept = layers_[0].channelsIn / MATRIX_SIZE, work = 0;
+    int tiles = 0, kept = layers_[0].channelsIn / MATRIX_SIZE, work = 0;
     for (const auto& l : layers_) {
         const int mt = l.channelsOut / MATRIX_SIZE, kt = l.channelsIn / MATRIX_SIZE;
-        int best = std::numeric_limits<int>::max(), own = 0, ownOut = 0;
+        int best = std::numeric_limits<int>::max(), own = 0;
         for (int m = 1; m <= waves; m *= 2)   // TileShare::split
             for (int k = 1; m * k <= waves; k *= 2) {
                 const int mo = divUp(mt, m), ki = divUp(kt, k);
@@ -368,15 +368,13 @@ int FusedNetwork::cooperativeRegisters(int waves, int registerWeight) const
                 if (cost < best) {
                     best = cost;
                     own = mo * ki;
-                    ownOut = mo;
                 }
             }
-        tiles += own;
-        if (l.useBias) biasColumns += ownOut;
+        tiles += own + (l.useBias ? 1 : 0);
         kept += mt;
         work = std::max(work, mt + 2 * kt);   // adjoint, input and its adjoint of a layer
     }
-    return 4 * (tiles + divUp(biasColumns, 16) + kept + work);   // a tile of sums: 4 registers; 16 channels of 2 x 16 points in half precision: 4
+    return 4 * (tiles + kept + work);   // a tile of sums: 4 registers; 16 channels of 2 x 16 points in half precision: 4
 }
 
 int FusedNetwork::cooperativeSlices(int numTiles) const
@@ -1369,8 +1367,6 @@ std::string FusedNetwork::cooperativeBackwardSource(int flags, bool sliceGradien
     const int weight = layout.registerWeight;
     const std::string lane = layout.opaqueLanes ? "opaqueLane(lane)" : "lane";
     std::stringstream stage, declare, call, store;
-    // bias sums: a column of 16 per tile of output channels and wavefront, side by side in the tiles that the layers share
-    std::string firstColumn = "0";
     for (int i = 0; i < L; ++i) {
         const auto& l = layers_[i];
         stage << "    typedef CooperativeLayer<" << l.channelsIn << ", " << l.channelsOut << ", " << (l.useBias ? "true" : "false")
@@ -1379,19 +1375,16 @@ std::string FusedNetwork::cooperativeBackwardSource(int flags, bool sliceGradien
         if (l.useBias)
             stage << "    for (int i = threadIdx.x; i < " << l.channelsOut << "; i += blockDim.x) sParams[" << ldsB[i] << " + i] = networkParameters["
                   << l.biasStart << " + i];\n";
-        declare << "    Layer" << i << "::Sums sums" << i << ";\n    sums" << i << ".zero();\n    constexpr int BIAS_COLUMN" << i << " = " << firstColumn << ";\n";
-        if (l.useBias) firstColumn = "BIAS_COLUMN" + std::to_string(i) + " + Layer" + std::to_string(i) + "::MO";
-        else firstColumn = "BIAS_COLUMN" + std::to_string(i);
+        declare << "    Layer" << i << "::Sums sums" << i << ";\n    sums" << i << ".zero();\n";
         call << "        Layer" << i << "::output_t pre" << i << ";\n        Layer" << i << "::forward(sParams + " << ldsW[i] << ", "
              << (l.useBias ? "sParams + " + std::to_string(ldsB[i]) : std::string("nullptr")) << ", " << (i == 0 ? std::string("x0") : "act" + std::to_string(i))
              << ", pre" << i << ", " << lane << ");\n";
         call << "        Layer" << i << "::output_t act" << (i + 1) << ";\n        Layer" << i << "::activate(pre" << i << ", act" << (i + 1) << ", lane);\n";
         if (i + 1 == L) call << "        (void)act" << L << ";\n";
-        store << "    Layer" << i << "::template storeWeightGradient<BIAS_COLUMN" << i << ">(sums" << i << ", biasSums, reinterpret_cast<float*>(sMemory),\n        partialGradients + (static_cast<long long>(blockIdx.x) * NUM_PARAMETERS + "
+        store << "    Layer" << i << "::storeWeightGradient(sums" << i << ", reinterpret_cast<float*>(sMemory),\n        partialGradients + (static_cast<long long>(blockIdx.x) * NUM_PARAMETERS + "
               << l.weightsStart << "), partialGradients + (static_cast<long long>(blockIdx.x) * NUM_PARAMETERS + " << (l.useBias ? l.biasStart : 0)
               << "), partialSlices, NUM_PARAMETERS, wave, lane);\n";
     }
-    declare << "    constexpr int BIAS_COLUMNS = " << firstColumn << ";\n    f32x4 biasSums[BIAS_COLUMNS > 16 ? (BIAS_COLUMNS + 15) / 16 : 1];\n    zeroTiles(biasSums);\n";
     const bool needsEncodingAdjoint = hasInputGradients || hasEncodingGradients;
     for (int i = L - 1; i >= 0; --i) {
         const std::string dy = i == L - 1 ? std::string("dyOut") : "dx" + std::to_string(i + 1);
@@ -1404,7 +1397,7 @@ std::string FusedNetwork::cooperativeBackwardSource(int flags, bool sliceGradien
             call << "        Layer0::template stageInput<activations::passthrough_>(x0, sRows, " << lane << ");\n";
         // (where the registers of the layers behind are free again)
         if (i == 0) call << "        loadRows(group + gridDim.x);\n";
-        call << "        workgroupLdsBarrier();\n        Layer" << i << "::template weightGradient<BIAS_COLUMN" << i << ">(sRowsAll, ROWS_PER_WAVE, sums" << i << ", biasSums, wave, "
+        call << "        workgroupLdsBarrier();\n        Layer" << i << "::weightGradient(sRowsAll, ROWS_PER_WAVE, sums" << i << ", wave, "
              << lane << ");\n        workgroupLdsBarrier();\n        Layer" << i << "::input_t dx" << i << ";\n";
         // (behind the barrier: while the gradient tiles are formed the adjoint of the output is held, not the wider one of an input,
         // and what follows each barrier has vector, matrix and LDS instructions to mix; 64 x 4 hidden layers, 10^6 points, forward
