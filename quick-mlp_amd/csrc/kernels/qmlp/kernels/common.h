@@ -244,22 +244,6 @@ __device__ __forceinline__ f16x4 activationAdjointMasked(f16x4 x, f16x4 adjz, in
     }
 }
 
-/** The same for 4 points of one channel. */
-template <typename Act>
-__device__ __forceinline__ f16x4 activationAdjointMaskedPoints(f16x4 x, f16x4 adjz, int channel, u32x2 mask)
-{
-    if constexpr (HasAdjointOfOutput<Act>::value) {
-        return Act::adjointOfOutput4(Act::forward4(x), adjz, mask);
-    } else if constexpr (HasPackedAdjoint<Act>::value) {
-        return __builtin_bit_cast(f16x4, __builtin_bit_cast(u32x2, Act::adjoint4(x, adjz)) & mask);
-    } else {
-        f16x4 o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = fromHalf(activationAdjointChannel<Act>(toHalf(x[i]), toHalf(adjz[i]), channel));
-        return __builtin_bit_cast(f16x4, __builtin_bit_cast(u32x2, o) & mask);
-    }
-}
-
 template <typename Act>
 __device__ __forceinline__ f16x4 activationForward(f16x4 v)
 {
