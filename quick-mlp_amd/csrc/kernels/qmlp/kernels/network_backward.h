@@ -364,21 +364,30 @@ $$CALL_ENCODINGS$$
                         // the channels of a row side by side: four per load and store. Kept to
                         // kernels without a grid scatter: in front of the gradient atomics of a grid
                         // no gain was measurable.
-                        float4 before[NUM_INPUTS / 4 > 0 ? NUM_INPUTS / 4 : 1];
+                        // What a row holds is read before any of it is written, 16 channels at a time: all of a wide row took the registers of the
+                        // layers (128 -> 64 -> 64 -> 64: 1320 bytes of scratch, forward and backward of 300 000 points 430 -> 500 us).
 #pragma unroll
-                        for (int i = 0; i + 3 < NUM_INPUTS; i += 4) before[i / 4] = *reinterpret_cast<const float4*>(adjRow + i);
+                        for (int first = 0; first < NUM_INPUTS; first += 16) {
+                            float4 before[4];
 #pragma unroll
-                        for (int i = 0; i + 3 < NUM_INPUTS; i += 4) {
-                            const float4 v = before[i / 4];
-                            *reinterpret_cast<float4*>(adjRow + i) = make_float4(v.x + adjEncodingInput[i], v.y + adjEncodingInput[i + 1],
-                                                                                v.z + adjEncodingInput[i + 2], v.w + adjEncodingInput[i + 3]);
+                            for (int i = first; i < first + 16 && i + 3 < NUM_INPUTS; i += 4) before[(i - first) / 4] = *reinterpret_cast<const float4*>(adjRow + i);
+#pragma unroll
+                            for (int i = first; i < first + 16 && i + 3 < NUM_INPUTS; i += 4) {
+                                const float4 v = before[(i - first) / 4];
+                                *reinterpret_cast<float4*>(adjRow + i) = make_float4(v.x + adjEncodingInput[i], v.y + adjEncodingInput[i + 1],
+                                                                                    v.z + adjEncodingInput[i + 2], v.w + adjEncodingInput[i + 3]);
+                            }
                         }
                     } else {
-                        float before[NUM_INPUTS];
 #pragma unroll
-                        for (int i = 0; i < NUM_INPUTS; ++i) before[i] = adjRow[static_cast<long long>(i) * adjInputs.strides_[1]];
+                        for (int first = 0; first < NUM_INPUTS; first += 16) {
+                            float before[16];
 #pragma unroll
-                        for (int i = 0; i < NUM_INPUTS; ++i) adjRow[static_cast<long long>(i) * adjInputs.strides_[1]] = before[i] + adjEncodingInput[i];
+                            for (int i = first; i < first + 16 && i < NUM_INPUTS; ++i) before[i - first] = adjRow[static_cast<long long>(i) * adjInputs.strides_[1]];
+#pragma unroll
+                            for (int i = first; i < first + 16 && i < NUM_INPUTS; ++i)
+                                adjRow[static_cast<long long>(i) * adjInputs.strides_[1]] = before[i - first] + adjEncodingInput[i];
+                        }
                     }
                 }
             }

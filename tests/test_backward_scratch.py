@@ -24,6 +24,8 @@ CASES = [
     (identity_cfg(16, [64] * 4 + [4], ["relu"] * 4 + ["identity"], [False] * 5), FLAG_INPUT | FLAG_WEIGHTS),
     (identity_cfg(16, [64] * 4 + [4], ["sine"] * 4 + ["identity"], [True] * 5), FLAG_INPUT | FLAG_WEIGHTS),
     (dense_grid_cfg(), FLAG_ENC),
+    # input gradients of wide rows, added to what the rows hold
+    (identity_cfg(128, [64, 64, 64], ["sine", "sine", "identity"], [False] * 3), FLAG_INPUT | FLAG_WEIGHTS),
 ]
 
 
