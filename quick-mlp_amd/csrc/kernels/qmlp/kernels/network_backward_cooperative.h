@@ -100,7 +100,7 @@ $$DECLARE_WEIGHT_GRADIENTS$$
     // (channel-major tiles of 64 points, zero outside the batch). Asked for a group of tiles ahead, and without a branch
     // around any load but what is the same for the whole launch: behind branches for lanes every load was waited for
     // before the next was asked for, six times the latency of the memory per tile. Lanes without a point or
-    // a channel read another one's, which takeRows leaves out.
+    // a channel read another one's, which takeChannels leaves out.
     f32x4 dyAhead[COOP_NT][MTL];
     f32x4 inputAhead[DIRECT_INPUT ? COOP_NT : 1][DIRECT_INPUT ? KT0 : 1];
     f16x2 encodedAhead[DIRECT_INPUT ? 1 : KT0][4];

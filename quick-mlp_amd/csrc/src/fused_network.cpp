@@ -1537,7 +1537,8 @@ std::string FusedNetwork::generatedSource(const std::string& kind, int adjointFl
     if (kind == "backward_resources" || kind == "backward_slices_resources") {
         // what the loaded backward kernel takes (needs a device): for tests of the register budget
         const bool slices = kind == "backward_slices_resources";
-        // ("recompute": the kernel of a batch of that kind runs the layers again instead of reading their intermediates)
+        // ("recompute": the kernel of a batch of that kind runs the layers again instead of reading their intermediates; "cooperative": it is the
+        // cooperative one, which networks whose option asks for it have at every size)
         // (of batches below COOPERATIVE_MIN_BATCH points)
         const int numel = slices ? COOPERATIVE_MIN_BATCH - 1 : 1;
         BackwardMode mode = BACKWARD_STORED;
@@ -1545,9 +1546,9 @@ std::string FusedNetwork::generatedSource(const std::string& kind, int adjointFl
         const bool recompute = mode == BACKWARD_RECOMPUTED;
         compileBackwardKernel(adjointFlags, slices, false, mode);
         const auto& ak = backwardKernel_[adjointFlags][slices ? 1 : 0][mode].value();
-        return format("{\"block\": %d, \"lds_bytes\": %d, \"registers\": %d, \"scratch_bytes\": %d, \"full_grid\": %d, \"recompute\": %s}",
+        return format("{\"block\": %d, \"lds_bytes\": %d, \"registers\": %d, \"scratch_bytes\": %d, \"full_grid\": %d, \"recompute\": %s, \"cooperative\": %s}",
                       ak.adjoint.blockSize, ak.adjoint.sharedMemorySize, ak.adjoint.fun.numVgprs(), ak.adjoint.fun.scratchBytes(),
-                      ak.adjoint.fullGrid, recompute ? "true" : "false");
+                      ak.adjoint.fullGrid, recompute ? "true" : "false", mode == BACKWARD_COOPERATIVE ? "true" : "false");
     }
     throw std::runtime_error("unknown kernel kind '" + kind + "'");
 }
