@@ -909,6 +909,8 @@ std::string FusedNetwork::forwardSource(int blockSize, int pointsPerLane, bool r
     replaceAll(code, "$$REGISTER_STAGING$$", registerStaging ? "true" : "false");
     replaceAll(code, "$$SHARED_TILE$$", sharedTile ? "true" : "false");
     replaceAll(code, "$$DIRECT_INPUT_START$$", std::to_string(directInputStart()));
+    kernel::PointOrderKey key{};
+    replaceAll(code, "$$SORTED_BATCHES$$", pointOrderFor(1 << 30, key) ? "true" : "false");
     replaceAll(code, "$$KERNEL_ATTRIBUTES$$", kernelAttributes(blockSize));
     // rows in registers are indexed by the tile: that loop has to be unrolled
     replaceAll(code, "$$TILE_LOOP_PRAGMA$$", registerStaging ? "#pragma unroll" : "#pragma unroll 1");
