@@ -565,6 +565,8 @@ private:
                                            bool sorted = false);
     /** Tables that a forward kernel goes through one after the other (most of an encoding's). */
     int sweptTables() const;
+    /** Whether some grid's entries are lines that several wavefronts of one tile each take from one another. */
+    bool gathersWideEntries() const;
     /** Points per launch of a forward kernel: the whole batch, or two passes of the grid for networks that gather. */
     int gatherChunkPoints(const CompiledKernel& ck) const;
     /** inference (store = false) or forward with stored intermediates, in one or several launches. */

@@ -1,6 +1,7 @@
 #include <qmlp/fused_network.h>
 #include <qmlp/device_code.h>
 
+#include <qmlp/encoding_hashgrid.h>
 #include <qmlp/encoding_identity.h>
 #include <qmlp/qmlp.h>
 
@@ -1527,6 +1528,23 @@ std::string FusedNetwork::generatedSource(const std::string& kind, int adjointFl
         ss << "]";
         return ss.str();
     }
+    if (kind == "inference_launches" || kind == "forward_launches") {
+        // which shapes a batch of this many points (in the place of the flags) is launched with (needs a device; loads the kernels)
+        std::stringstream ss;
+        kernel::PointOrderKey key{};
+        const bool store = kind == "forward_launches";
+        const int numel = adjointFlags;
+        for (long long start = 0; start < numel;) {
+            int launchTiles = 0;
+            const auto& ck = forwardKernelFor(store, static_cast<int>(divUp<long long>(numel - start, TILE_POINTS)), &launchTiles, false, false, false,
+                                              store ? sortsTraining(numel) : pointOrderFor(numel, key));
+            ss << (start ? ", " : "[") << "{\"tiles\": " << launchTiles << ", \"block\": " << ck.blockSize << ", \"tiles_per_wave\": " << ck.pointsPerLane
+               << ", \"scratch_bytes\": " << ck.fun.scratchBytes() << "}";
+            start += static_cast<long long>(launchTiles) * TILE_POINTS;
+        }
+        ss << (numel > 0 ? "]" : "[]");
+        return ss.str();
+    }
     // the shape with the encoded rows in registers, whether or not the network would get it
     if (kind == "forward_registers") return forwardSource(2 * DEFAULT_BLOCK_SIZE, std::min(8, 256 / layers_[0].channelsIn), true);
     if (kind == "backward") return backwardSource(adjointFlags, forwardBlockSize(compileOptions_.overwriteBlocksizeBackward, true));
@@ -1679,6 +1697,18 @@ int FusedNetwork::sweptTables() const
     return tables;
 }
 
+bool FusedNetwork::gathersWideEntries() const
+{
+    // Eight corners of 64 bytes: a wavefront more loses what the lines of its points bring to the L1 (64^3 nodes x 16 floats, inference of 100 003 /
+    // 300 007 / 700 001 / 2^20 points 16 / 39 / 71 / 87 us, with a tile per wavefront 19 / 41 / 87 / 80; 128^3 21 / 48 / 100 / 134 and 20 / 46 / 99 / 143;
+    // four corners, 256^2 nodes, 13 / 26 / 51 / 61 and 13 / 18 / 43 / 53; sixteen, 24^4 nodes, 32 / 78 / 140 / 188 and 31 / 72 / 96 / 135).
+    for (const auto& e : encodings_) {
+        const auto* grid = dynamic_cast<const EncodingHashGrid*>(e.get());
+        if (grid && grid->ndim() == 3 && grid->channelsWrittenTogether() * (grid->parameterPrecision(Tensor::INFERENCE) == Tensor::HALF ? 2 : 4) >= 64) return true;
+    }
+    return false;
+}
+
 const FusedNetwork::CompiledKernel& FusedNetwork::forwardKernelFor(bool store, int numTiles, int* launchTiles, bool noAlloc, bool derivatives,
                                                                   bool inputOnly, bool sorted)
 {
@@ -1701,13 +1731,16 @@ const FusedNetwork::CompiledKernel& FusedNetwork::forwardKernelFor(bool store, i
         if (pointsPerLane == 1) return loaded(VARIANT_DEFAULT);   // no gathers, or a pinned shape: one kernel
     }
     const int overwrite = store ? compileOptions_.overwriteBlocksizeForward : compileOptions_.overwriteBlocksizeInference;
-    if (sweptTables() < 2 && compileOptions_.pointsPerLane <= 0 && overwrite <= 0) {
-        // One table: there are no levels to sweep through together, and a tile per wavefront leaves room for more wavefronts and has no
-        // steps (256^2 nodes x 4, 300 007 / 700 001 / 2^21 points: 10 / 17 / 41 us, with the rule below 16 / 23 / 51; 512^3 cells hashed to 2^19
-        // entries x 2: 14 / 24 / 60 and 20 / 32 / 69). But the points of a slab of a sorted batch share lines: training passes of many
-        // points, whose lanes hold what they store as well, take a twentieth less per point with four tiles per wavefront in whole steps, behind
-        // a longer start (32^4 nodes x 8, forward and backward of 2^20 / 1 500 007 / 2^21 / 2^22 points 242 / 319 / 410 / 787 us, with one tile 238 /
-        // 316 / 416 / 799; inference 68 / 95 / 112 / 207 and 63 / 80 / 107 / 199). A launch more costs what 1900 of its tiles take.
+    if (sweptTables() < 2 && !gathersWideEntries() && compileOptions_.pointsPerLane <= 0 && overwrite <= 0) {
+        // No levels that wavefronts sweep through together: a tile per wavefront leaves room for more wavefronts and has no steps. Inference of 300 007 /
+        // 700 001 / 2^20 points, and with the rule below: 256^2 nodes x 4 10 / 17 / 26 us and 16 / 23 / 31; 32^4 nodes x 8 41 / 48 / 63 and 48 / 82 / 84;
+        // two grids of 256^2 x 4 14 / 19 / 26 and 18 / 25 / 31; the latter in front of 128-wide layers the same to 3 %. Rays that march through grids of
+        // 16 and 8 levels and of 64^3 nodes (LineIntegration), 300 007 points: 12.4, 6.8 and 0.35 ms and 15.9, 8.6 and 0.49.
+        // But the points of a slab of a sorted batch share lines: training passes of many points, whose lanes hold what they store as well, take a
+        // twentieth less per point with four tiles per wavefront in whole steps, behind a longer start (forward and backward of 2^20 / 1 500 007 / 2^21 /
+        // 2^22 points: 32^4 nodes x 8 203 / 279 / 352 / 658 us, with one tile 203 / 281 / 362 / 685; x 4 159 / 196 / 268 / 532 and 159 / 197 / 279 / 545; x 8
+        // floats 401 / 544 / 715 / 1548 and 400 / 546 / 731 / 1630; 160^3 x 2 129 / 185 / 224 / 434 and 129 / 187 / 230 / 448; 128^3 x 8 663 / 892 / 1217 / 2326
+        // and 665 / 889 / 1255 / 2394). A launch more costs what 1900 of its tiles take. Not where that kernel spills (24^4 x 16: 509 us for 2^21 points, 435).
         if (sorted && store && hasLargeVariant(store)) {
             int blockSize = 0, pointsPerLane = 1;
             forwardShape(store, VARIANT_LARGE, blockSize, pointsPerLane);
@@ -1716,9 +1749,9 @@ const FusedNetwork::CompiledKernel& FusedNetwork::forwardKernelFor(bool store, i
             constexpr double PER_TILE = 1.055, START = 1300;
             const double narrow = PER_TILE * numTiles, large = START + static_cast<double>(divUp<long long>(numTiles, step) * step);
             const double both = START + static_cast<double>(steps * step) + PER_TILE * static_cast<double>(numTiles - steps * step) + 1900;
-            if (large <= narrow && (large <= both || steps == 0)) return loaded(VARIANT_LARGE);
-            if (steps > 0 && both < narrow) {
-                if (launchTiles) *launchTiles = static_cast<int>(steps * step);
+            const bool whole = large <= narrow && (large <= both || steps == 0), first = !whole && steps > 0 && both < narrow;
+            if ((whole || first) && loaded(VARIANT_LARGE).fun.scratchBytes() == 0) {
+                if (first && launchTiles) *launchTiles = static_cast<int>(steps * step);
                 return loaded(VARIANT_LARGE);
             }
         }
