@@ -195,6 +195,9 @@ int qmlp_encoding_adjoint_overwriting(qmlp_encoding_t encoding, const qmlp_tenso
  * kernel cache without a GPU. No counterpart in the reference, which compiles lazily inside
  * forward()/adjoint() (src_cpp/src/iencoding.cpp:30-43,98-112). */
 int qmlp_encoding_precompile(qmlp_encoding_t encoding, int adjoint_mode);
+/* Name of the kernel that forward() takes for these tensors (diagnostics and tests; needs a device); free with
+ * qmlp_free_string(). */
+int qmlp_encoding_forward_kernel(qmlp_encoding_t encoding, const qmlp_tensor* input, const qmlp_tensor* output, char** name);
 /* HashGrid only: level table as the reference computes it in
  * src_cpp/src/encoding_hashgrid.cpp:63-96. Arrays hold `capacity` entries. */
 int qmlp_encoding_hashgrid_levels(qmlp_encoding_t encoding, int capacity, int* num_levels, int* memory_offset,

@@ -357,6 +357,9 @@ public:
      */
     void precompile(int adjointMode = AdjointMode::ALL_GRADIENTS);
 
+    /** The kernel that forward() takes for these tensors (diagnostics and tests; needs a device). */
+    [[nodiscard]] std::string forwardKernelName(const Tensor& input, const Tensor& output) const;
+
 private:
     std::string forwardKernelSource(int groups) const;
     std::string adjointKernelSource(int adjointMode, bool sharedTile = false) const;

@@ -494,6 +494,13 @@ int qmlp_encoding_forward(qmlp_encoding_t encoding, const qmlp_tensor* input, co
     QMLP_API_END
 }
 
+int qmlp_encoding_forward_kernel(qmlp_encoding_t encoding, const qmlp_tensor* input, const qmlp_tensor* output, char** name)
+{
+    QMLP_API_BEGIN
+    *name = dupString(encoding->encoding->forwardKernelName(wrap(input), wrap(output)));
+    QMLP_API_END
+}
+
 int qmlp_encoding_adjoint(qmlp_encoding_t encoding, const qmlp_tensor* input, const qmlp_tensor* adj_output,
                           const qmlp_tensor* adj_input, void* stream, const qmlp_tensor* parameters_forward,
                           const qmlp_tensor* parameters_gradients, int adjoint_mode)

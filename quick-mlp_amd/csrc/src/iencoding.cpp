@@ -123,29 +123,43 @@ void IEncoding::precompile(int adjointMode)
 bool IEncoding::forwardByLevels(const Tensor& input, const Tensor& output) const
 {
     const long long numel = input.size(0);
-    if (levelTiles().empty() || numOutputChannels() > kernel::ENCODING_ROWS_MAX_CHANNELS) return false;
-    // Tables that one die's L2 (4 MB) would have to take turns with, and batches that make up for a second kernel. Whole rows -> by levels,
-    // us, for grids of 8 to 32 levels and 20 to 90 MB of tables:
+    const std::vector<int> levels = levelTiles();
+    if (levels.empty() || numOutputChannels() > kernel::ENCODING_ROWS_MAX_CHANNELS) return false;
+    // Tables that one die's L2 (4 MB) would have to take turns with, and batches that make up for a second kernel. The time of the kernel of whole
+    // rows grows in steps of a workgroup of 256 points per compute unit (2^16 points of 256), and just before the end of the first two its
+    // wavefronts walk through the levels together. Whole rows -> by levels, us:
     //   2^14 / 2^15 points   13 -> 17 / 23 -> 24 (16 levels of 2^19 entries of 2 floats, 50 MB; of 2 halves 10 -> 14 / 17 -> 20)
-    //   3 2^14, 2^16         37 -> 30, 42 -> 37 (halves 32 -> 25, 35 -> 29; the others 1.04 to 1.5 times as fast)
-    //   7 2^14 to 2^17       69 -> 63, in a training step 67 -> 67 (halves 49 -> 49, 25 MB 51 -> 56): the kernel of whole rows fills
-    //                        the chip exactly once, and its wavefronts walk through the levels together
-    //   80 000 to 7 2^14     72 -> 50 (98 304; halves 55 -> 39)
-    //   3 2^16               126 -> 90 (halves 78 -> 72)
-    //   2^18 / 2^20          182 -> 116 / 771 -> 437 (halves 132 -> 95 / 568 -> 364; the others 1.02 to 1.8 / 1.15 to 2.1 times as fast)
-    // One feature per level: 52 -> 39 at 3 2^14 points, but 73 -> 81 at 3 2^16. Tables of 13 MB at 2^17 points: 44 -> 56.
-    constexpr long long MIN_TABLE_BYTES = 20 << 20;
+    //   3 2^14, 2^16         37 -> 30, 42 -> 37 (halves 33 -> 25, 35 -> 29), but with 128 bytes or more per point and level 62 -> 68 (16 levels of
+    //                        8 halves, 2^16), 53 -> 58 (12 of 8 floats), 42 -> 48 (4-D, 12 of 2 floats)
+    //   9 2^13, 7 2^14       66 -> 40, 72 -> 57 (halves 53 -> 32, 52 -> 43; 16 of 8 halves 105 -> 84, 117 -> 111)
+    //   15 2^13, 2^17        72 -> 60, 70 -> 63, in a training step 67 -> 67 (halves 50 -> 46, 49 -> 49, 12 levels 45 -> 44, 45 -> 47; 4-D 86 -> 83, 81 -> 88)
+    //   2^18 / 2^20          183 -> 116 / 776 -> 434 (halves 133 -> 95 / 569 -> 361; 16 of 8 halves 265 -> 236 / 1139 -> 949)
+    // One feature per level: 66 -> 48 at 3 2^15 points, but 78 -> 86 at 3 2^16. Tables of 13 MB at 2^17 points: 44 -> 56. Eight levels, one per die, of
+    // which the coarse ones are done first: 2^16 / 2^17 / 2^18 points 25 -> 29 / 39 -> 50 / 78 -> 90 (of 2 floats), 45 -> 59 / 92 -> 109 / 189 -> 211 (8
+    // floats), 26 -> 32 / 41 -> 54 / 97 -> 97 (4 halves); ten 27 -> 22 / 38 -> 38 / 71 -> 70 (2 halves).
+    constexpr long long MIN_TABLE_BYTES = 20 << 20, POINTS_PER_WORKGROUP = 256;
+    constexpr int MIN_LEVELS = 10, WIDE_BYTES = 128;
     const long long tableBytes = static_cast<long long>(parameterCount()) * (parameterPrecision(Tensor::INFERENCE) == Tensor::HALF ? 2 : 4);
-    if (numel < FORWARD_WHOLE_ROWS_MIN_BATCH || tableBytes < MIN_TABLE_BYTES) return false;
-    if (channelsWrittenTogether() < 2 && numel < (1 << 18)) return false;
-    if (numel > (7 << 14) && numel <= (1 << 17)) return false;
+    if (static_cast<int>(levels.size()) < MIN_LEVELS || numel < FORWARD_WHOLE_ROWS_MIN_BATCH || tableBytes < MIN_TABLE_BYTES) return false;
+    const long long step = POINTS_PER_WORKGROUP * KernelFunction::computeUnits();
+    if (numel <= step && 4 * gatherRegistersPerPoint() >= WIDE_BYTES) return false;
+    if (4 * numel > 7 * step && numel <= 2 * step) return false;
+    if (channelsWrittenTogether() < 2 && numel < 4 * step) return false;
     if (numel * numOutputChannels() >= (1ll << 32)) return false;   // (lanes of a launch)
     // Rows without gaps, which hold other points' values between the two kernels: not those that a caller reads the positions from.
     if (output.size(1) != numOutputChannels() || output.strides()[0] != numOutputChannels()) return false;
-    const char* rows = static_cast<const char*>(output.rawPtr());
-    const char* positions = static_cast<const char*>(input.rawPtr());
-    const long long span = (numel - 1) * input.strides()[0] + (input.size(1) - 1) * input.strides()[1] + 1;
-    return positions + span * sizeof(float) <= rows || rows + numel * numOutputChannels() * sizeof(float) <= positions;
+    const float* rows = static_cast<const float*>(output.rawPtr());
+    const float *first = static_cast<const float*>(input.rawPtr()), *last = first;
+    for (int d = 0; d < 2; ++d) {
+        const long long extent = (input.size(d) - 1ll) * input.strides()[d];
+        (extent < 0 ? first : last) += extent;
+    }
+    return last < rows || rows + numel * numOutputChannels() <= first;
+}
+
+std::string IEncoding::forwardKernelName(const Tensor& input, const Tensor& output) const
+{
+    return forwardByLevels(input, output) ? "EncodingLevelsKernel" : "EncodingForwardKernel";
 }
 
 void IEncoding::forward(const Tensor& input, Tensor& output, stream_t stream,

@@ -107,6 +107,7 @@ _SIGNATURES = {
     "qmlp_encoding_hashgrid_corners": [_vp, _TD, _vp, _vp, _vp],
     "qmlp_encoding_hashgrid_trace": [_vp, _TD, _ci, _vp, _vp, _vp],
     "qmlp_encoding_precompile": [_vp, _ci],
+    "qmlp_encoding_forward_kernel": [_vp, _TD, _TD, _pstr],
     "qmlp_activation_create": [ctypes.c_char_p, _P(_vp)],
     "qmlp_activation_destroy": [_vp],
     "qmlp_activation_to_json": [_vp, _pstr],
