@@ -380,9 +380,10 @@ int FusedNetwork::cooperativeRegisters(int waves, int registerWeight) const
 
 int FusedNetwork::cooperativeSlices(int numTiles) const
 {
-    // One per workgroup: two of them per compute unit, up to four where a lane holds so little that more wavefronts find room
-    // (16 -> 64 x 2 -> 4, 10^6 points, forward and backward: 88 us with three, 95 with two). Behind tables two or four: the pass is
-    // bound by the kernels of the tables, and a third slice per compute unit would only be more temporary memory.
+    // One per workgroup: two of them per compute unit, three or four where a lane holds so little that more wavefronts find room (16 -> 64 x 2 -> 4,
+    // 10^6 points, forward and backward: 88 us with three, 95 with two). A slice more per compute unit is 256 times the weights more of temporary
+    // memory for batches of more than 2^16 points, 12.6 -> 18.9 MB for that network. Behind tables two or four: the pass is bound by the kernels of
+    // the tables, which a third would not make faster.
     const CooperativeLayout& layout = cooperativeLayout();
     const int waves = layout.blockSize / WARP_SIZE;
     const int registers = cooperativeRegisters(waves, layout.registerWeight);
