@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
+#include <qmlp/kernels/dies.h>
 #include <qmlp/kernels/tensor.h>
 
 #define QUICKMLP_KERNEL_NAMESPACE ::qmlp::kernel

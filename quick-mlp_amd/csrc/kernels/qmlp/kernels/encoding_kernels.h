@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(256) EncodingLevelsKernel(
     constexpr int TILES[L] = {$$LEVEL_TILES$$};   // of a wavefront
     const int lane = threadIdx.x % WAVE_SIZE;
     const int tiles = static_cast<int>((numel + TILE_POINTS - 1) / TILE_POINTS);
-    int left = blockIdx.x % ENCODING_DIES * (gridDim.x / ENCODING_DIES) + blockIdx.x / ENCODING_DIES, level = -1, perWave = 1;
+    int left = blockIdx.x % DIES * (gridDim.x / DIES) + blockIdx.x / DIES, level = -1, perWave = 1;
 #pragma unroll
     for (int l = 0; l < L; ++l) {
         const int workgroups = (tiles + TILES[l] * ENCODING_LEVEL_WAVES - 1) / (TILES[l] * ENCODING_LEVEL_WAVES);

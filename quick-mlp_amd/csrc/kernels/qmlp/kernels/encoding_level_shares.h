@@ -1,9 +1,9 @@
 #pragma once
 // How EncodingLevelsKernel shares out the levels of a grid; also included by the host, which sizes its grid.
 
-namespace qmlp { namespace kernel {
+#include <qmlp/kernels/dies.h>
 
-constexpr int ENCODING_DIES = 8;
+namespace qmlp { namespace kernel {
 
 /** Tiles of 64 points of a level whose table takes so many bytes that a wavefront of EncodingLevelsKernel takes, such that workgroups cost
  *  the same: the L1 holds up to 32 KB of a table, and much of 256 KB (16 levels of halves, 2^20 points: a microsecond for 16^3 nodes, 4 to

@@ -31,12 +31,6 @@ __device__ __forceinline__ f16x4 readTransposed(const f16* p)
     return __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p)));
 }
 
-/** Workgroup barrier that waits for this wavefront's LDS accesses only: loads and stores of global memory stay in flight. */
-__device__ __forceinline__ void workgroupLdsBarrier()
-{
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 /**
  * How the WAVES wavefronts of a workgroup share MT x KT gradient tiles: M x K blocks of tiles, and P shares of the points.
  * Few large blocks need fewer operand reads, many small ones fewer registers: the split of least

@@ -117,15 +117,15 @@ $$STAGE_PARAMETERS$$
     // the regions of the temporary memory are laid out for the whole batch
     const long long numel64 = static_cast<long long>(tmpNumTiles) * TILE_POINTS;
     (void)numel64;
-    // A sorted batch: workgroups go to the 8 dies in turn, and a die takes consecutive groups of tiles, whose entries of the table then lie in its
+    // A sorted batch: workgroups go to the dies in turn, and a die takes consecutive groups of tiles, whose entries of the table then lie in its
     // own L2 alone (32^4 nodes x 8, 16 MB: 700 001 points 43 -> 33 us, in a training step of 2^21 points 112 -> 103).
     // Compiled into the kernels of such networks only: inference of 64 to 5000 points behind a hash grid 6 to 11 us, 0.1 more with it.
     int tileFirst = blockIdx.x * GROUP_TILES, tileStep = gridDim.x * GROUP_TILES, tileEnd = numTiles;
-    if (SORTED_BATCHES && pointOrder && gridDim.x % 8 == 0) {
-        const int die = blockIdx.x % 8, groups = (numTiles + GROUP_TILES - 1) / GROUP_TILES;
-        tileFirst = (groups * die / 8 + blockIdx.x / 8) * GROUP_TILES;
-        tileEnd = min(numTiles, groups * (die + 1) / 8 * GROUP_TILES);
-        tileStep /= 8;
+    if (SORTED_BATCHES && pointOrder && gridDim.x % DIES == 0) {
+        const int die = blockIdx.x % DIES, groups = (numTiles + GROUP_TILES - 1) / GROUP_TILES;
+        tileFirst = (groups * die / DIES + blockIdx.x / DIES) * GROUP_TILES;
+        tileEnd = min(numTiles, groups * (die + 1) / DIES * GROUP_TILES);
+        tileStep /= DIES;
     }
     for (int tileBase = tileFirst; tileBase < tileEnd; tileBase += tileStep)
     {

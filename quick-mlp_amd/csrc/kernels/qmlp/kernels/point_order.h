@@ -29,9 +29,9 @@ constexpr int POINT_ORDER_SCAN_SLABS = 16;          // slabs per workgroup of Po
  */
 __device__ __forceinline__ unsigned pointOrderChunk()
 {
-    constexpr unsigned DIES = 8;
-    const unsigned die = blockIdx.x % DIES;
-    return die * (gridDim.x / DIES) + min(die, gridDim.x % DIES) + blockIdx.x / DIES;
+    constexpr unsigned dies = DIES;
+    const unsigned die = blockIdx.x % dies;
+    return die * (gridDim.x / dies) + min(die, gridDim.x % dies) + blockIdx.x / dies;
 }
 
 /** Slab of one coordinate value, clamped to the box (the comparisons are false for NaN, which then lands in slab 0). */

@@ -306,7 +306,7 @@ int EncodingHashGrid::levelGroups() const
 std::vector<int> EncodingHashGrid::levelTiles() const
 {
     std::vector<int> tiles;
-    if (levelGroups() != kernel::ENCODING_DIES) return tiles;
+    if (levelGroups() != kernel::DIES) return tiles;
     const int entryBytes = parameterPrecision_ == Tensor::HALF ? 2 : 4;
     for (int l = 0; l < numLevels_; ++l) {
         const int end = l + 1 < numLevels_ ? layers_[l + 1].memoryOffset : numParameters_;

@@ -1401,8 +1401,8 @@ std::string FusedNetwork::cooperativeBackwardSource(int flags, bool sliceGradien
             call << "        Layer0::template stageInput<activations::passthrough_>(x0, sRows, " << lane << ");\n";
         // (where the registers of the layers behind are free again)
         if (i == 0) call << "        loadRows(group + gridDim.x);\n";
-        call << "        workgroupLdsBarrier();\n        Layer" << i << "::weightGradient(sRowsAll, ROWS_PER_WAVE, sums" << i << ", wave, "
-             << lane << ");\n        workgroupLdsBarrier();\n        Layer" << i << "::input_t dx" << i << ";\n";
+        call << "        ldsBarrier();\n        Layer" << i << "::weightGradient(sRowsAll, ROWS_PER_WAVE, sums" << i << ", wave, "
+             << lane << ");\n        ldsBarrier();\n        Layer" << i << "::input_t dx" << i << ";\n";
         // (behind the barrier: while the gradient tiles are formed the adjoint of the output is held, not the wider one of an input,
         // and what follows each barrier has vector, matrix and LDS instructions to mix; 64 x 4 hidden layers, 10^6 points, forward
         // and backward, 172 -> 158 us, 4 -> 128 -> 64 -> 48 -> 4 357 -> 309)

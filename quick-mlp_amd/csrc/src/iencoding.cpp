@@ -205,10 +205,10 @@ void IEncoding::forward(const Tensor& input, Tensor& output, stream_t stream,
         const long long tiles = divUp<long long>(numel, 64);
         long long workgroups = 0;
         for (int perWave : levelTiles()) workgroups += divUp<long long>(tiles, perWave * kernel::ENCODING_LEVEL_WAVES);
-        const long long perDie = divUp<long long>(workgroups, kernel::ENCODING_DIES);
+        const long long perDie = divUp<long long>(workgroups, kernel::DIES);
         float* rows = outputAcc.data_;
         std::vector<void*> levelArgs = {&numel, &inputAcc, &rows, paramBytes.data()}, rowArgs = {&numel, &rows};
-        forwardByLevels_[0].launch(static_cast<int>(kernel::ENCODING_DIES * perDie), block, 0, stream, levelArgs.data());
+        forwardByLevels_[0].launch(static_cast<int>(kernel::DIES * perDie), block, 0, stream, levelArgs.data());
         forwardByLevels_[1].launch(static_cast<int>(tiles), 64, 0, stream, rowArgs.data());
     } else {
         auto& fun = kernel.value();
