@@ -8,11 +8,11 @@
 // (layer_cooperative.h), two workgroup barriers per layer. For the adjoint of the encoded input: the input gradients
 // of identity encodings are added here, those of grids are left to the kernels behind this one.
 //
-// 64 -> 64 x 4 -> 4, 10^6 points: 110 us, 541 vector and 144 matrix instructions per 32 points of 4 and 16 cycles, which hardly
-// overlap on a SIMD, while the LDS is busy for 0.6 of the time (152 us with 957 vector instructions, the adjoint of ReLU as
-// comparisons and its output computed three times; 125 with the rows of a tile waited for one after the other). 4 -> 128 -> 64
-// -> 48 -> 4 with sines, 2^20 points: 210 us, vector instructions 0.6 and matrix instructions 0.2 of the time (300 us while it spilled
-// 232 bytes per lane, 225 with the rows waited for). Slower or the same: one wavefront per SIMD with all gradient tiles
+// 16 -> 64 x 4 -> 4, 10^6 points: 128 us under the profiler (154 with the adjoint of ReLU as comparisons, its output computed three times and the rows of a
+// tile waited for one after the other). 683 vector instructions per 32 points, 172 of them matrix products: a SIMD issues the former for 27 % of the
+// time and has its matrix cores busy for 27 %, which hardly overlap, the LDS is at work for half of it (conflicts 15 %), wavefronts wait
+// for a third of theirs, and 173 MB of memory traffic make 1.4 TB/s. 4 -> 128 -> 64 -> 48 -> 4 with sines, 2^20 points: 231 us (302 while it spilled
+// 232 bytes per lane), vector instructions 52 %, matrix cores 18 %, LDS 34 %. Slower or the same: one wavefront per SIMD with all gradient tiles
 // and no barriers (+25 %), or with 64 points (+20 %); fewer vector instructions (outputs of the sines kept or the first layer's pre-activations
 // formed again by matrix instructions, masks left out of full tiles: 0 to 2 %); other paddings of the rows; other orders between the barriers.
 //
